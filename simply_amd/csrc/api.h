@@ -240,6 +240,11 @@ struct Sections {
 int gemm_generic(const void* A, int a_dtype, int64_t lda, const void* W, const void* W2, int w_dtype, void* C,
                  int c_dtype, int64_t ldc, int M, int N, int K, int epi, int act, float cap, int packed,
                  hipStream_t stream);
+// 32-bit operands and result, row-major, rows a multiple of 16 bytes: the f32 matrix instructions.  A row's sums run in an
+// order that N and the other rows have no part in.
+bool gemm_f32_takes(int M, int N, int K, int64_t lda, const void* A, const void* W, const void* W2);
+int gemm_f32(const float* A, int64_t lda, const float* W, const float* W2, float* C, int64_t ldc, int M, int N, int K, int epi,
+             int act, float cap, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // x = act(x) in place, row by row (the separate kernel behind products whose kernels have no such epilogue)
 int apply_activation(void* x, int dtype, int64_t stride, int M, int N, int act, hipStream_t stream);
 bool gemm_skinny_takes(int M, int N, int K, int64_t lda, const void* A, const void* W, const void* W2);

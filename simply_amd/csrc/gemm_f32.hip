@@ -1,0 +1,411 @@
+// C[M, N] = epilogue(A[M, K] . W[N, K]^T) in 32 bits on the matrix cores: v_mfma_f32_16x16x4_f32, whose products and sums
+// are IEEE single precision.  Row-major float operands whose rows are multiples of 16 bytes; everything else of the 32-bit
+// path goes to gemm_generic.hip.
+//
+// Every output element is summed in one order whatever M is, so a row's result does not depend on which other rows are in
+// the batch: K is cut into at most eight segments of the same length, a multiple of 32 (the length depends on K alone); a
+// segment is summed by one chain of instructions in increasing blocks of 16 (of a block, k = j, 4 + j, 8 + j, 12 + j
+// together for j = 0 .. 3), and the segments' sums are added in increasing order.  Three ways of running that:
+//
+//   few rows    (M <= 16) a workgroup owns 16 rows of W, a wave a segment of them: bound by reading W once.  Loads bring
+//               whole 128-byte pieces of rows, four stages of 32 columns of K ahead in registers; the operand order is made
+//               on the way through LDS (each wave its own part, no barrier in the loop; 16-byte pieces permuted by row, so
+//               that neither side has bank conflicts).
+//   tiles       a workgroup of four waves owns 128 x 128 or 64 x 64 outputs and walks through all segments, adding a
+//               segment's sum to its total at the segment's end: bound by the f32 matrix rate.
+//   cut tiles   the same tiles, a workgroup per segment (gridDim.z); a sum kernel adds the segments' planes: where the
+//               tiles alone leave CUs idle.
+//
+// Measured, weights from HBM, against the vector-ALU kernel that took these products before (64 x 64 tiles and a thread's
+// 4 x 4 outputs whatever M, so that few rows read W with the workgroups of one row of tiles, one 16-column stage at a time):
+//   (N, K)                4 rows             509 rows
+//   (2304, 9216)          23 us for 959      215 us for 1,450 (100 TFLOP/s of 157)
+//   (2304, 2048)          7.1 for 213        63 for 315
+//   (4096, 2304)          10 for 243         101 for 383
+//   (9216 gated, 2304)    45 for 458         395 for 1,026
+//   (256000, 2304)        408 for 1,556 (5.8 TB/s)
+#include "api.h"
+#include "common.h"
+
+namespace sa {
+namespace f32 {
+
+typedef __attribute__((ext_vector_type(4))) float floatx4;
+
+constexpr int kSegments = 8;
+constexpr int BK = 32;         // columns of K of a stage: a row of a tile is 128 bytes
+constexpr int kPieces = BK / 4;
+
+struct Args {
+  const float* A;
+  const float* W;
+  const float* W2;
+  float* C;
+  int64_t lda, ldc;
+  int M, N, K;
+  int seg;      // length of a segment
+  int act;
+  float cap;
+};
+
+// Where the 16-byte piece p of row r lies in a tile of rows of 128 bytes (in floats).
+__device__ __forceinline__ int piece_at(int r, int p) { return r * BK + ((p ^ (r & 7)) * 4); }
+
+template <int EPI>
+__device__ __forceinline__ float finish(const Args& a, float x, float y) {
+  if (EPI == 1) return gated_product_exact(a.act, a.cap, x, y);
+  if (EPI == 2) return a.cap * tanhf(x / a.cap);
+  return x;
+}
+
+__device__ __forceinline__ void store4(const Args& a, int m, int n, floatx4 v) {
+  float* dst = a.C + static_cast<size_t>(m) * a.ldc + n;
+  if (n + 3 < a.N && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+    *reinterpret_cast<floatx4*>(dst) = v;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < a.N) dst[r] = v[r];
+  }
+}
+
+// blockDim: a wave per segment.  AROWS: rows of A that are read (8 or 16).
+template <int EPI, int AROWS>
+__global__ __launch_bounds__(64 * kSegments) void gemm_f32_few_kernel(Args a) {
+  constexpr int NW = EPI == 1 ? 2 : 1, AP = AROWS / 8, D = 4;
+  constexpr int kWaveFloats = (NW * 16 + AROWS) * BK;
+  __shared__ __align__(16) float lds[kSegments * kWaveFloats];
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int n0 = blockIdx.x * 16, r = lane / kPieces, p = lane % kPieces, c = lane % 16, g = lane / 16;
+  float* w_s = lds + wave * kWaveFloats;
+  float* a_s = w_s + NW * 16 * BK;
+  const int k0 = wave * a.seg;
+  const int ns = ((a.K - k0 < a.seg ? a.K - k0 : a.seg) + BK - 1) / BK;
+  const float* wp[NW][2];
+  const float* ap[AP];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int n = n0 + 8 * i + r;
+    const size_t at = static_cast<size_t>(n < a.N ? n : a.N - 1) * a.K;
+    wp[0][i] = a.W + at;
+    if (NW == 2) wp[NW - 1][i] = a.W2 + at;
+  }
+#pragma unroll
+  for (int i = 0; i < AP; ++i) {
+    const int m = 8 * i + r;
+    ap[i] = a.A + static_cast<size_t>(m < a.M ? m : a.M - 1) * a.lda;
+  }
+  floatx4 wv[D][NW][2], av[D][AP];
+  auto load = [&](floatx4 (&w)[NW][2], floatx4 (&x)[AP], int s) __attribute__((always_inline)) {
+    // (behind the segment's last stage: that one again; columns behind K: column 0, replaced by zeros below)
+    int k = k0 + (s < ns ? s : ns - 1) * BK + p * 4;
+    k = k < a.K ? k : 0;
+#pragma unroll
+    for (int v = 0; v < NW; ++v)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) w[v][i] = *reinterpret_cast<const floatx4*>(wp[v][i] + k);
+#pragma unroll
+    for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const floatx4*>(ap[i] + k);
+  };
+  floatx4 acc[NW];
+#pragma unroll
+  for (int v = 0; v < NW; ++v) acc[v] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto to_lds = [&](const floatx4 (&w)[NW][2], const floatx4 (&x)[AP], int s) __attribute__((always_inline)) {
+    const bool ok = k0 + s * BK + p * 4 < a.K;
+    const floatx4 zero{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int v = 0; v < NW; ++v)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<floatx4*>(w_s + v * 16 * BK + piece_at(8 * i + r, p)) = ok ? w[v][i] : zero;
+#pragma unroll
+    for (int i = 0; i < AP; ++i) *reinterpret_cast<floatx4*>(a_s + piece_at(8 * i + r, p)) = ok ? x[i] : zero;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto multiply = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < BK / 16; ++b) {
+      const floatx4 x = *reinterpret_cast<const floatx4*>(a_s + piece_at(c % AROWS, b * 4 + g));
+#pragma unroll
+      for (int v = 0; v < NW; ++v) {
+        const floatx4 w = *reinterpret_cast<const floatx4*>(w_s + v * 16 * BK + piece_at(c, b * 4 + g));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], acc[v], 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(wv[d], av[d], d);
+  int s = 0;
+  for (; s + D <= ns; s += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      to_lds(wv[d], av[d], s + d);
+      load(wv[d], av[d], s + d + D);
+      multiply();
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D - 1; ++d)
+    if (s + d < ns) {   // (uniform over the wave; the loads are there)
+      to_lds(wv[d], av[d], s + d);
+      multiply();
+    }
+  __syncthreads();
+  floatx4* sums = reinterpret_cast<floatx4*>(lds);
+#pragma unroll
+  for (int v = 0; v < NW; ++v) sums[(wave * NW + v) * kWave + lane] = acc[v];
+  __syncthreads();
+  if (wave != 0) return;
+  const int nseg = blockDim.x / kWave;
+  floatx4 t[NW];
+#pragma unroll
+  for (int v = 0; v < NW; ++v) t[v] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int z = 0; z < nseg; ++z)
+#pragma unroll
+    for (int v = 0; v < NW; ++v) t[v] += sums[(z * NW + v) * kWave + lane];
+  if (c >= a.M) return;
+  floatx4 y;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = finish<EPI>(a, t[0][i], t[NW - 1][i]);
+  if (n0 + 4 * g < a.N) store4(a, c, n0 + 4 * g, y);
+}
+
+// TM: blocks of 16 rows and of 16 weight rows of a wave; four waves, two by two.  With the gated epilogue half of a wave's
+// weight rows are the gate's and half the other factor's of the same outputs.  PLANES: this workgroup's segment alone, its
+// sums to planes [segment][M][columns] (gated: all the gate's columns, then the other factor's).
+template <int EPI, int TM, bool PLANES>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(Args a, float* __restrict__ planes) {
+  constexpr int ROWS = 2 * TM * 16;                 // rows of A, and rows of W, of a tile
+  constexpr int LOADS = ROWS * kPieces / 256;
+  constexpr int COLS = EPI == 1 ? ROWS / 2 : ROWS;  // outputs across
+  constexpr int WT = EPI == 1 ? TM / 2 : TM;        // blocks of outputs across of a wave
+  __shared__ __align__(16) float a_s[2][ROWS * BK];
+  __shared__ __align__(16) float w_s[2][ROWS * BK];
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave % 2, wn = wave / 2, c = lane % 16, g = lane / 16;
+  const int m0 = blockIdx.y * ROWS, n0 = blockIdx.x * COLS;
+  const int k0 = PLANES ? blockIdx.z * a.seg : 0;
+  const int k1 = PLANES && k0 + a.seg < a.K ? k0 + a.seg : a.K;
+  const int ns = (k1 - k0 + BK - 1) / BK, per_segment = a.seg / BK;
+  const int r = tid / kPieces, p = tid % kPieces;   // 32 rows at a time
+  const float* ap[LOADS];
+  const float* wp[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = i * 32 + r;
+    const int m = m0 + row < a.M ? m0 + row : a.M - 1;
+    ap[i] = a.A + static_cast<size_t>(m) * a.lda;
+    int n = n0 + row;
+    const float* w = a.W;
+    if (EPI == 1) {   // of a wave's TM * 16 rows the first half belongs to the gate
+      const int in_wave = row % (TM * 16);
+      n = n0 + row / (TM * 16) * (WT * 16) + in_wave % (WT * 16);
+      if (in_wave >= WT * 16) w = a.W2;
+    }
+    wp[i] = w + static_cast<size_t>(n < a.N ? n : a.N - 1) * a.K;
+  }
+  floatx4 av[LOADS], wv[LOADS];
+  auto load = [&](int s) __attribute__((always_inline)) {
+    int k = k0 + (s < ns ? s : ns - 1) * BK + p * 4;
+    k = k < a.K ? k : 0;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      av[i] = *reinterpret_cast<const floatx4*>(ap[i] + k);
+      wv[i] = *reinterpret_cast<const floatx4*>(wp[i] + k);
+    }
+  };
+  auto to_lds = [&](int s, int buf) __attribute__((always_inline)) {
+    const bool ok = k0 + s * BK + p * 4 < a.K;
+    const floatx4 zero{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      *reinterpret_cast<floatx4*>(&a_s[buf][piece_at(i * 32 + r, p)]) = ok ? av[i] : zero;
+      *reinterpret_cast<floatx4*>(&w_s[buf][piece_at(i * 32 + r, p)]) = ok ? wv[i] : zero;
+    }
+  };
+  floatx4 acc[TM][TM], total[PLANES ? 1 : TM][TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (!PLANES) total[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+  load(0);
+  to_lds(0, 0);
+  __syncthreads();
+  int left = per_segment;
+  for (int s = 0; s < ns; ++s) {
+    const int buf = s & 1;
+    load(s + 1);
+#pragma unroll
+    for (int b = 0; b < BK / 16; ++b) {
+      floatx4 x[TM], w[TM];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        x[i] = *reinterpret_cast<const floatx4*>(&a_s[buf][piece_at((wm * TM + i) * 16 + c, b * 4 + g)]);
+        w[i] = *reinterpret_cast<const floatx4*>(&w_s[buf][piece_at((wn * TM + i) * 16 + c, b * 4 + g)]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int t = 0; t < TM; ++t)
+            acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][j], x[i][j], acc[i][t], 0, 0, 0);
+    }
+    if (!PLANES && (--left == 0 || s + 1 == ns)) {
+      left = per_segment;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int t = 0; t < TM; ++t) {
+          total[i][t] += acc[i][t];
+          acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    // (the other buffer's last readers passed the barrier of the stage before)
+    if (s + 1 < ns) to_lds(s + 1, buf ^ 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + (wm * TM + i) * 16 + c;
+    if (m >= a.M) continue;
+    if (PLANES) {
+      const int64_t width = EPI == 1 ? 2 * static_cast<int64_t>(a.N) : a.N;
+      Args b = a;
+      b.C = planes + static_cast<size_t>(blockIdx.z) * a.M * width;
+      b.ldc = width;
+#pragma unroll
+      for (int t = 0; t < TM; ++t) {
+        const int n = n0 + (wn * WT + t % WT) * 16 + 4 * g;
+        Args to = b;
+        if (EPI == 1 && t >= WT) to.C += a.N;
+        if (n < a.N) store4(to, m, n, acc[i][t]);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < WT; ++t) {
+        const int n = n0 + (wn * WT + t) * 16 + 4 * g;
+        floatx4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = finish<EPI>(a, total[PLANES ? 0 : i][t][e], total[PLANES ? 0 : i][EPI == 1 ? t + WT : t][e]);
+        if (n < a.N) store4(a, m, n, y);
+      }
+    }
+  }
+}
+
+// C = epilogue(sum of the segments' planes, in order), V columns a thread.
+template <int EPI, int V>
+__global__ __launch_bounds__(256) void gemm_f32_sum_kernel(Args a, const float* __restrict__ planes, int nseg) {
+  const size_t width = EPI == 1 ? 2 * static_cast<size_t>(a.N) : a.N, plane = static_cast<size_t>(a.M) * width;
+  const size_t per_row = a.N / V, all = per_row * a.M;
+  for (size_t e = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; e < all; e += static_cast<size_t>(gridDim.x) * blockDim.x) {
+    const size_t m = e / per_row, n = e % per_row * V;
+    const float* at = planes + m * width + n;
+    float x[V], y[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) x[i] = y[i] = 0.f;
+    float px[kSegments][V], py[EPI == 1 ? kSegments : 1][V];
+#pragma unroll
+    for (int z = 0; z < kSegments; ++z) {   // (planes behind the last: the last again, not added)
+      const float* from = at + static_cast<size_t>(z < nseg ? z : nseg - 1) * plane;
+      if constexpr (V == 4) {
+        *reinterpret_cast<floatx4*>(px[z]) = *reinterpret_cast<const floatx4*>(from);
+        if constexpr (EPI == 1) *reinterpret_cast<floatx4*>(py[z]) = *reinterpret_cast<const floatx4*>(from + a.N);
+      } else {
+        px[z][0] = from[0];
+        if constexpr (EPI == 1) py[z][0] = from[a.N];
+      }
+    }
+#pragma unroll
+    for (int z = 0; z < kSegments; ++z)
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        if (z < nseg) x[i] += px[z][i];
+        if constexpr (EPI == 1)
+          if (z < nseg) y[i] += py[z][i];
+      }
+    float* dst = a.C + m * a.ldc + n;
+    if constexpr (V == 4) {
+      *reinterpret_cast<floatx4*>(dst) = floatx4{finish<EPI>(a, x[0], y[0]), finish<EPI>(a, x[1], y[1]),
+                                                 finish<EPI>(a, x[2], y[2]), finish<EPI>(a, x[3], y[3])};
+    } else {
+      dst[0] = finish<EPI>(a, x[0], y[0]);
+    }
+  }
+}
+
+template <int EPI>
+static void launch_tiles(const Args& a, int tm, int nseg, float* planes, hipStream_t stream) {
+  const int rows = 32 * tm, cols = EPI == 1 ? rows / 2 : rows;
+  const dim3 grid((a.N + cols - 1) / cols, (a.M + rows - 1) / rows, planes != nullptr ? nseg : 1);
+  if (planes == nullptr) {
+    if (tm == 4) gemm_f32_tile_kernel<EPI, 4, false><<<grid, 256, 0, stream>>>(a, nullptr);
+    else gemm_f32_tile_kernel<EPI, 2, false><<<grid, 256, 0, stream>>>(a, nullptr);
+    return;
+  }
+  if (tm == 4) gemm_f32_tile_kernel<EPI, 4, true><<<grid, 256, 0, stream>>>(a, planes);
+  else gemm_f32_tile_kernel<EPI, 2, true><<<grid, 256, 0, stream>>>(a, planes);
+  const bool by_four = a.N % 4 == 0 && a.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15u) == 0;
+  const size_t all = static_cast<size_t>(a.M) * (a.N / (by_four ? 4 : 1));
+  const int blocks = static_cast<int>((all + 255) / 256 > 4096 ? 4096 : (all + 255) / 256);
+  if (by_four) gemm_f32_sum_kernel<EPI, 4><<<blocks, 256, 0, stream>>>(a, planes, nseg);
+  else gemm_f32_sum_kernel<EPI, 1><<<blocks, 256, 0, stream>>>(a, planes, nseg);
+}
+
+template <int EPI>
+static void launch(const Args& a, int nseg, float* workspace, size_t workspace_bytes, hipStream_t stream) {
+  if (a.M <= 16) {
+    const int blocks = (a.N + 15) / 16;
+    if (a.M <= 8) gemm_f32_few_kernel<EPI, 8><<<blocks, 64 * nseg, 0, stream>>>(a);
+    else gemm_f32_few_kernel<EPI, 16><<<blocks, 64 * nseg, 0, stream>>>(a);
+    return;
+  }
+  // The tile and whether K is cut over workgroups: rounds over the 256 CUs times a tile's products at the share of a CU's
+  // 614 GFLOP/s that the tile reaches, and for cut tiles the planes written and read at 4 TB/s and one launch more.
+  const double NW = EPI == 1 ? 2.0 * a.N : a.N;
+  const size_t plane_bytes = static_cast<size_t>(nseg) * a.M * static_cast<size_t>(NW) * sizeof(float);
+  int best_tm = 4;
+  bool best_cut = false;
+  double best = 1e30;
+  for (int tm = 4; tm >= 2; tm -= 2) {
+    const double rows = 32.0 * tm, tiles = ceil(a.M / rows) * ceil(NW / rows);
+    const double tile_us = 2.0 * rows * rows * a.K / (0.614e6 * (tm == 4 ? 0.85 : 0.7));
+    for (int cut = 0; cut < 2; ++cut) {
+      if (cut && (nseg == 1 || workspace == nullptr || plane_bytes > workspace_bytes)) continue;
+      const double us = cut ? ceil(tiles * nseg / 256.0) * tile_us / nseg + 2.0 * plane_bytes / 4e6 + 5.0
+                            : ceil(tiles / 256.0) * tile_us;
+      if (us < best) best = us, best_tm = tm, best_cut = cut != 0;
+    }
+  }
+  launch_tiles<EPI>(a, best_tm, nseg, best_cut ? workspace : nullptr, stream);
+}
+
+}  // namespace f32
+
+bool gemm_f32_takes(int M, int N, int K, int64_t lda, const void* A, const void* W, const void* W2) {
+  auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+  return M >= 1 && K % 4 == 0 && lda % 4 == 0 && aligned(A) && aligned(W) && aligned(W2) && N <= (1 << 30) / 16 &&
+         (M + 63) / 64 <= 65535;   // (tiles of rows are the grid's second index)
+}
+
+int gemm_f32(const float* A, int64_t lda, const float* W, const float* W2, float* C, int64_t ldc, int M, int N, int K, int epi,
+             int act, float cap, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  f32::Args a;
+  a.A = A, a.W = W, a.W2 = W2, a.C = C, a.lda = lda, a.ldc = ldc, a.M = M, a.N = N, a.K = K, a.act = act, a.cap = cap;
+  a.seg = (K + f32::kSegments * f32::BK - 1) / (f32::kSegments * f32::BK) * f32::BK;
+  const int nseg = (K + a.seg - 1) / a.seg;
+  float* ws = static_cast<float*>(workspace);
+  if (epi == kEpilogueGated) f32::launch<1>(a, nseg, ws, workspace_bytes, stream);
+  else if (epi == kEpilogueSoftCap) f32::launch<2>(a, nseg, ws, workspace_bytes, stream);
+  else f32::launch<0>(a, nseg, ws, workspace_bytes, stream);
+  return check_launch("gemm_f32");
+}
+
+}  // namespace sa

@@ -2,8 +2,8 @@
 // both element types, on the vector ALU in 32-bit (products and sums in float,
 // no reduced-precision matrix mode).  Each output element is summed over k in
 // increasing order whatever M is, so a row's result does not depend on which
-// other rows are in the batch.  This is the kernel of the 32-bit path and the
-// fallback of the bfloat16 path for shapes that the MFMA kernels refuse.
+// other rows are in the batch.  This is the fallback
+// of both paths for operands that the matrix-core kernels refuse (sizes, alignment).
 #include "api.h"
 #include "common.h"
 

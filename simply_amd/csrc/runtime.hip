@@ -107,6 +107,9 @@ static int gemm_routed(const void* A, int a_dtype, int64_t lda, const void* W, c
     rc = gemm_skinny(A, lda, W, W2, C, c_dtype, ldc, M, N, K, epilogue, act, cap, packed, shape, stream, sec);
   else if (kernel == 3)
     rc = gemm_tiled(A, lda, W, C, c_dtype, ldc, M, N, K, epilogue, act, cap, shape, workspace, ws_bytes, stream, sec);
+  else if (algo == 0 && !packed && a_dtype == kF32 && w_dtype == kF32 && c_dtype == kF32 && gemm_f32_takes(M, N, K, lda, A, W, W2))
+    rc = gemm_f32(static_cast<const float*>(A), lda, static_cast<const float*>(W), static_cast<const float*>(W2),
+                  static_cast<float*>(C), ldc, M, N, K, epilogue, act, cap, workspace, ws_bytes, stream);
   else
     rc = gemm_generic(A, a_dtype, lda, W, W2, w_dtype, C, c_dtype, ldc, M, N, K, epilogue, act, cap, packed, stream);
   if (rc == 0 && activated) rc = apply_activation(C, c_dtype, ldc, M, N, activated - 1, stream);
