@@ -3,7 +3,7 @@
 // path goes to gemm_generic.hip.
 //
 // Every output element is summed in one order whatever M is, so a row's result does not depend on which other rows are in
-// the batch: K is cut into at most eight segments of the same length, a multiple of 32 (the length depends on K alone); a
+// the batch: K is cut into at most eight segments of the same length, a multiple of 16 (the length depends on K alone); a
 // segment is summed by one chain of instructions in increasing blocks of 16 (of a block, k = j, 4 + j, 8 + j, 12 + j
 // together for j = 0 .. 3), and the segments' sums are added in increasing order.  Three ways of running that:
 //
@@ -43,7 +43,7 @@ struct Args {
   float* C;
   int64_t lda, ldc;
   int M, N, K;
-  int seg;      // length of a segment
+  int seg;      // length of a segment, a multiple of 16
   int act;
   float cap;
 };
@@ -80,7 +80,8 @@ __global__ __launch_bounds__(64 * kSegments) void gemm_f32_few_kernel(Args a) {
   float* w_s = lds + wave * kWaveFloats;
   float* a_s = w_s + NW * 16 * BK;
   const int k0 = wave * a.seg;
-  const int ns = ((a.K - k0 < a.seg ? a.K - k0 : a.seg) + BK - 1) / BK;
+  const int k1 = a.K - k0 < a.seg ? a.K : k0 + a.seg;
+  const int ns = (k1 - k0 + BK - 1) / BK;
   const float* wp[NW][2];
   const float* ap[AP];
 #pragma unroll
@@ -97,9 +98,9 @@ __global__ __launch_bounds__(64 * kSegments) void gemm_f32_few_kernel(Args a) {
   }
   floatx4 wv[D][NW][2], av[D][AP];
   auto load = [&](floatx4 (&w)[NW][2], floatx4 (&x)[AP], int s) __attribute__((always_inline)) {
-    // (behind the segment's last stage: that one again; columns behind K: column 0, replaced by zeros below)
+    // (behind the segment's last stage: that one again; columns behind its end: its first ones, replaced by zeros below)
     int k = k0 + (s < ns ? s : ns - 1) * BK + p * 4;
-    k = k < a.K ? k : 0;
+    k = k < k1 ? k : k0;
 #pragma unroll
     for (int v = 0; v < NW; ++v)
 #pragma unroll
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(64 * kSegments) void gemm_f32_few_kernel(Args a) {
 #pragma unroll
   for (int v = 0; v < NW; ++v) acc[v] = floatx4{0.f, 0.f, 0.f, 0.f};
   auto to_lds = [&](const floatx4 (&w)[NW][2], const floatx4 (&x)[AP], int s) __attribute__((always_inline)) {
-    const bool ok = k0 + s * BK + p * 4 < a.K;
+    const bool ok = k0 + s * BK + p * 4 < k1;
     const floatx4 zero{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < NW; ++v)
@@ -189,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(Args a, float* __
   const int m0 = blockIdx.y * ROWS, n0 = blockIdx.x * COLS;
   const int k0 = PLANES ? blockIdx.z * a.seg : 0;
   const int k1 = PLANES && k0 + a.seg < a.K ? k0 + a.seg : a.K;
-  const int ns = (k1 - k0 + BK - 1) / BK, per_segment = a.seg / BK;
+  const int ns = (k1 - k0 + BK - 1) / BK, per_segment = a.seg / 16;
   const int r = tid / kPieces, p = tid % kPieces;   // 32 rows at a time
   const float* ap[LOADS];
   const float* wp[LOADS];
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(Args a, float* __
   floatx4 av[LOADS], wv[LOADS];
   auto load = [&](int s) __attribute__((always_inline)) {
     int k = k0 + (s < ns ? s : ns - 1) * BK + p * 4;
-    k = k < a.K ? k : 0;
+    k = k < k1 ? k : k0;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       av[i] = *reinterpret_cast<const floatx4*>(ap[i] + k);
@@ -218,7 +219,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(Args a, float* __
     }
   };
   auto to_lds = [&](int s, int buf) __attribute__((always_inline)) {
-    const bool ok = k0 + s * BK + p * 4 < a.K;
+    const bool ok = k0 + s * BK + p * 4 < k1;
     const floatx4 zero{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
@@ -256,16 +257,17 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(Args a, float* __
 #pragma unroll
           for (int t = 0; t < TM; ++t)
             acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][j], x[i][j], acc[i][t], 0, 0, 0);
-    }
-    if (!PLANES && (--left == 0 || s + 1 == ns)) {
-      left = per_segment;
+      // a segment ends behind any block of 16; blocks behind K's end are zeros
+      if (!PLANES && (--left == 0 || (s + 1 == ns && b + 1 == BK / 16))) {
+        left = per_segment;
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int t = 0; t < TM; ++t) {
-          total[i][t] += acc[i][t];
-          acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
+          for (int t = 0; t < TM; ++t) {
+            total[i][t] += acc[i][t];
+            acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
     }
     // (the other buffer's last readers passed the barrier of the stage before)
     if (s + 1 < ns) to_lds(s + 1, buf ^ 1);
@@ -399,7 +401,7 @@ int gemm_f32(const float* A, int64_t lda, const float* W, const float* W2, float
              int act, float cap, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   f32::Args a;
   a.A = A, a.W = W, a.W2 = W2, a.C = C, a.lda = lda, a.ldc = ldc, a.M = M, a.N = N, a.K = K, a.act = act, a.cap = cap;
-  a.seg = (K + f32::kSegments * f32::BK - 1) / (f32::kSegments * f32::BK) * f32::BK;
+  a.seg = (K + f32::kSegments * 16 - 1) / (f32::kSegments * 16) * 16;
   const int nseg = (K + a.seg - 1) / a.seg;
   float* ws = static_cast<float*>(workspace);
   if (epi == kEpilogueGated) f32::launch<1>(a, nseg, ws, workspace_bytes, stream);
