@@ -159,6 +159,13 @@ int sa_paged_attention(const void* q, int dtype, int64_t q_stride, const void* k
                        const int* block_table, int table_stride, const int* token_seq, const int* positions, void* out,
                        int64_t out_stride, int T, int H, int Kh, int hd, int page_size, int window, float soft_cap,
                        int algo, hipStream_t stream);
+// Attention of units (seq_meta's layout; at most 16 rows, heads of a key head times tokens, each) in 32 bits on the matrix
+// cores; sinks (float [H]) may be null.  sa_paged_attention_f32_takes: which sizes.
+int sa_paged_attention_f32_takes(int H, int Kh, int hd, int page_size, int64_t q_stride, const void* q);
+int sa_paged_attention_f32(const float* q, int64_t q_stride, const float* k_pages, const float* v_pages, const int* block_table,
+                           int table_stride, const int* units, int unit_begin, int unit_count, float* out, int64_t out_stride,
+                           int H, int Kh, int hd, int page_size, int window, float soft_cap, float scale, const float* sinks,
+                           int max_kv_len, int max_q_len, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
 // The same attention for requests seq_begin .. seq_begin + seq_count - 1 of seq_meta (int32 [S, 4]: block-table
 // row, index of the request's first token in this step, number of its tokens, position of its first token), each

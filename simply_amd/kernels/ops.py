@@ -677,6 +677,43 @@ def decode_attention_takes(q: torch.Tensor, k_pages: torch.Tensor, num_heads: in
         int(num_heads), int(Kh), int(hd), int(page_size), int(max_q_len), q.stride(0), _ptr(q)))
 
 
+def attention_f32_takes(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, num_heads: int) -> bool:
+    """Whether `paged_attention_f32` takes these sizes."""
+    _, Kh, page_size, hd = k_pages.shape
+    return q.dtype == torch.float32 and q.is_cuda and v_pages.shape[2] == hd and bool(
+        _lib.load().sa_paged_attention_f32_takes(int(num_heads), int(Kh), int(hd), int(page_size), q.stride(0), _ptr(q)))
+
+
+def paged_attention_f32(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,
+                        units: torch.Tensor, unit_begin: int, unit_count: int, num_heads: int, *, window: int | None,
+                        soft_cap: float | None, max_kv_len: int, max_q_len: int, out: torch.Tensor, scale: float = 1.0,
+                        sinks: torch.Tensor | None = None) -> torch.Tensor:
+    """Attention in 32 bits on the matrix cores: rows unit_begin .. unit_begin + unit_count - 1 of `units` (seq_meta's
+    layout), each of at most 16 query rows (heads per key head times tokens).  A token's result depends on nothing but
+    its position and its keys.  sinks: float32 [H], as for `paged_attention_sink`."""
+    _dev(q, k_pages, v_pages, block_table, units, out, sinks)
+    q_stride, out_stride = _rows(q, "paged_attention_f32: q"), _rows(out, "paged_attention_f32: out")
+    if any(t.dtype != torch.float32 for t in (q, out)):
+        raise KernelError("paged_attention_f32: float32 only")
+    _check_pages(k_pages, v_pages, q.dtype, "paged_attention_f32")
+    _, Kh, page_size, hd = k_pages.shape
+    if block_table.dim() != 2 or block_table.dtype != torch.int32 or block_table.stride(1) != 1:
+        raise KernelError("paged_attention_f32: block_table must be int32 [sequences, blocks]")
+    if units.dtype != torch.int32 or units.dim() != 2 or units.shape[1] != 4 or not units.is_contiguous() \
+            or unit_begin < 0 or unit_begin + unit_count > units.shape[0]:
+        raise KernelError("paged_attention_f32: units must be int32 [U, 4] covering the requested range")
+    if out.shape[0] != q.shape[0] or out.shape[1] != num_heads * hd or q.shape[1] < num_heads * hd:
+        raise KernelError("paged_attention_f32: bad output or query rows")
+    if sinks is not None and (sinks.dtype != torch.float32 or sinks.numel() != num_heads or not sinks.is_contiguous()):
+        raise KernelError("paged_attention_f32: sinks must be contiguous float32, one per query head")
+    ws = _workspace(q.device)
+    _lib.call("sa_paged_attention_f32", _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
+              block_table.stride(0), _ptr(units), unit_begin, unit_count, _ptr(out), out_stride, num_heads, Kh, hd, page_size,
+              int(window or 0), float(soft_cap or 0.0), float(scale), _ptr(sinks), int(max_kv_len), int(max_q_len), _ptr(ws),
+              ws.numel(), _stream())
+    return out
+
+
 def _attention_units(entry: str, q, k_pages, v_pages, block_table, seq_meta, begin, count, num_heads, window, soft_cap,
                      max_kv_len, max_q_len, out, num_splits, sinks=None, slopes=None):
     _dev(q, k_pages, v_pages, block_table, seq_meta, out, sinks, slopes)

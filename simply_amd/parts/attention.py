@@ -92,6 +92,11 @@ class PagedAttention(Mixer):
             if many:
                 ops.paged_attention_prefill(qkv, cache.k_pages, cache.v_pages, group.block_table, units, few, many, H,
                                             **kw)
+        elif ops.attention_f32_takes(qkv, cache.k_pages, cache.v_pages, H):
+            units, few, many, max_q = ctx.attention_units(16 // (H // K))
+            ops.paged_attention_f32(qkv, cache.k_pages, cache.v_pages, group.block_table, units, 0, few + many, H,
+                                    window=self.window, soft_cap=self.soft_cap, max_kv_len=ctx.max_kv_len, max_q_len=max_q,
+                                    out=o)
         else:
             ops.paged_attention(qkv, cache.k_pages, cache.v_pages, group.block_table, ctx.token_seq, ctx.positions, H,
                                 window=self.window, soft_cap=self.soft_cap, out=o)
@@ -208,6 +213,12 @@ class SinkAttention(Mixer):
             if many:
                 ops.paged_attention_prefill(proj, cache.k_pages, cache.v_pages, group.block_table, units, few, many, H,
                                             **kw)
+        elif ops.attention_f32_takes(proj, cache.k_pages, cache.v_pages, H):
+            o = torch.empty((proj.shape[0], H * dv), dtype=proj.dtype, device=proj.device)
+            units, few, many, max_q = ctx.attention_units(16 // (H // K))
+            ops.paged_attention_f32(proj, cache.k_pages, cache.v_pages, group.block_table, units, 0, few + many, H,
+                                    window=self.window, soft_cap=None, max_kv_len=ctx.max_kv_len, max_q_len=max_q, out=o,
+                                    scale=self.scale, sinks=self.sink_f32)
         else:
             o = ops.paged_attention_sink(proj, cache.k_pages, cache.v_pages, group.block_table, ctx.token_seq,
                                          ctx.positions, H, scale=self.scale, sinks=self.sink, window=self.window)

@@ -54,3 +54,91 @@ def test_products_keep_special_values():
         assert torch.isnan(got[:, 7]).all()
         rest = torch.cat([got[:, :7], got[:, 8:]], 1)
         assert torch.isinf(rest[1]).all() and torch.isfinite(rest[torch.arange(M) != 1]).all()
+
+
+def attention_64(q, kp, vp, table, slot, positions, H, window, cap, scale, sinks):
+    """q [T, H, hd] of one request at `positions`, its keys and values gathered from the pages: 64 bits."""
+    from torch_ops import stored_keys_as_rows
+
+    kp = stored_keys_as_rows(kp)
+    _, Kh, P, hd = kp.shape
+    n = int(positions[-1]) + 1
+    at = torch.arange(n, device="cuda")
+    pages = table[slot, at // P].long().clamp_min(0)
+    k, v = kp[pages, :, at % P].double(), vp[pages, :, :, at % P].double()      # [n, Kh, hd]
+    k, v = (x.repeat_interleave(H // Kh, 1) for x in (k, v))
+    s = torch.einsum("thd,nhd->htn", q.double(), k) * scale
+    if cap:
+        s = cap * torch.tanh(s / cap)
+    d = positions[:, None] - at[None]
+    seen = (d >= 0) & (d < (window or n))
+    s = s.masked_fill(~seen, float("-inf"))
+    if sinks is not None:
+        s = torch.cat([s, sinks.double()[:, None, None].expand(H, len(positions), 1)], 2)
+    p = torch.softmax(s, -1)[..., :n]
+    return torch.einsum("htn,nhd->thd", p, torch.where(torch.isnan(v), torch.zeros_like(v), v))
+
+
+@pytest.mark.parametrize("H,Kh,hd,P,window,cap,sink", [
+    (8, 4, 256, 16, None, 50.0, False), (8, 4, 256, 16, 300, 50.0, False), (4, 4, 64, 32, 17, None, True),
+    (6, 2, 128, 16, None, None, True), (16, 1, 64, 48, 64, 30.0, False)])
+def test_attention(H, Kh, hd, P, window, cap, sink):
+    """Portions and single tokens around the ends of chunks (64) and ranges (256) of keys, a workgroup per range and one
+    that walks through them.  Bounds: the scores' sums of hd products and the weighted values' sums, each (n + 8) eps of
+    the sums of magnitudes, which unit normal entries keep below 1e-5 of the largest value."""
+    from simply_amd.kernels import ops
+    from test_gpu_kernels import paged_setup
+
+    lens = [1, 63, 64, 65, 256, 257, 700, 1100]
+    kp, vp, table = paged_setup(torch.float32, len(lens), H, Kh, hd, P, lens, 31)
+    if window:   # pages that no query of the step sees are another's by now
+        first = max(lens) - 150 - window
+        table[len(lens) - 1, :max(first, 0) // P] = -1
+    portions = [(s, max(0, n - (1 if s < 4 else 150)), n) for s, n in enumerate(lens)]
+    T = sum(b - a for _, a, b in portions)
+    q = draw((T, H * hd + 32), 32, 0.5)[:, :H * hd]
+    sinks = draw((H,), 33) if sink else None
+    G = H // Kh
+    kw = dict(window=window, soft_cap=cap, scale=0.7, sinks=sinks, max_kv_len=max(lens))
+    out = torch.zeros(T, H * hd, device="cuda")
+    per = 16 // G
+    units, row = [], 0
+    for s, a, b in portions:
+        units += [(s, row + i, min(per, b - a - i), a + i) for i in range(0, b - a, per)]
+        row += b - a
+    dev = torch.tensor(units, dtype=torch.int32).cuda()
+    assert ops.attention_f32_takes(q, kp, vp, H)
+    ops.paged_attention_f32(q, kp, vp, table, dev, 0, len(units), H, max_q_len=per, out=out, **kw)
+    row = 0
+    for s, a, b in portions:
+        want = attention_64(q[row:row + b - a].reshape(-1, H, hd), kp, vp, table, s, torch.arange(a, b, device="cuda"), H, window,
+                            cap, 0.7, sinks)
+        err = (out[row:row + b - a].double().reshape(want.shape) - want).abs().max()
+        assert err <= 1e-5 * want.abs().max(), (s, float(err), float(want.abs().max()))
+        row += b - a
+    # one token at a time, a few units to a launch: the same bits
+    single = [(s, r + i, 1, p + i) for s, r, n, p in units for i in range(n)]
+    one = torch.zeros_like(out)
+    dev = torch.tensor(single, dtype=torch.int32).cuda()
+    for i in range(0, len(single), 100):
+        ops.paged_attention_f32(q, kp, vp, table, dev, i, min(100, len(single) - i), H, max_q_len=1, out=one, **kw)
+    assert torch.equal(one, out)
+
+
+def test_attention_keeps_special_values():
+    """Values that are not finite reach the queries that see them and no others of the same unit."""
+    from simply_amd.kernels import ops
+    from test_gpu_kernels import paged_setup
+
+    H, Kh, hd, P, n, window = 2, 1, 64, 16, 40, 12
+    kp, vp, table = paged_setup(torch.float32, 1, H, Kh, hd, P, [n], 41)
+    at = 27
+    vp[table[0, at // P].long(), 0, 5, at % P] = float("inf")
+    q = draw((8, H * hd), 42)
+    for first in (20, 24, 32):   # the key becomes visible within the unit, or leaves its window
+        units = torch.tensor([[0, 0, 8, first]], dtype=torch.int32).cuda()
+        out = torch.empty(8, H * hd, device="cuda")
+        ops.paged_attention_f32(q, kp, vp, table, units, 0, 1, H, window=window, soft_cap=None, max_kv_len=n, max_q_len=8, out=out)
+        sees = torch.tensor([first + i >= at and first + i - window < at for i in range(8)], device="cuda")
+        bad = ~torch.isfinite(out.view(8, H, hd))
+        assert torch.equal(bad[:, :, 5], sees[:, None].expand(8, H)) and not bad[:, :, :5].any() and not bad[:, :, 6:].any()

@@ -230,6 +230,10 @@ def decode_attention_takes(q, k_pages, num_heads, max_q_len):
     return False
 
 
+def attention_f32_takes(q, k_pages, v_pages, num_heads):
+    return False
+
+
 def paged_attention_sink(q, k_pages, v_pages, block_table, token_seq, positions, num_heads, *, scale=1.0, sinks=None,
                          window=None, soft_cap=None, out=None, slopes=None):
     T = q.shape[0]
