@@ -438,6 +438,15 @@ int sa_delta_inputs_few(const void* x, int x_dtype, int64_t x_stride, const void
 int sa_delta_rule(const float* qkv, int C, int G, int dk, int dv, const float* gates, int H, float* state,
                   int64_t state_stride, const int* seq_meta, int num_seqs, float* out, hipStream_t stream);
 
+// sa_delta_rule for requests that bring portions, 64 tokens at a time on the matrix cores (32-bit): rows first_row ..
+// first_row + rows - 1 of the step hold the requests' tokens, request by request in seq_meta's order, at most max_q_len of
+// each.  The workspace holds what is computed ahead of the state; sa_delta_chunks_takes: key sizes up to 128 in multiples of
+// 4, rows of qkv and of the state in multiples of 4, and room for at least one piece more than requests.
+int sa_delta_chunks_takes(int C, int G, int H, int dk, int dv, int64_t state_stride, int num_seqs, int64_t workspace_bytes);
+int sa_delta_chunks(const float* qkv, int C, int G, int dk, int dv, const float* gates, int H, float* state,
+                    int64_t state_stride, const int* seq_meta, int num_seqs, int first_row, int rows, int max_q_len, float* out,
+                    void* workspace, int64_t workspace_bytes, hipStream_t stream);
+
 // sa_paged_attention_decode and sa_paged_attention_prefill for softmax sums that hold one more term per query head,
 // exp(sinks[h]) (float32 [H]; null: none), without a value, and with slopes (float32 [H]; null: none): slopes[h] times
 // the distance between query and key is taken off the score.

@@ -1,0 +1,408 @@
+// The gated delta rule of delta_rule.hip for portions of prompts, on the matrix cores: 64 tokens (a piece) at a time.  With
+// L_i the sum of the decays' logarithms up to token i of a piece and S the state in front of it, the rule's
+//
+//   S_i = g_i S_(i-1) + k_i u_i^T,   u_i = beta_i (v_i - g_i S_(i-1)^T k_i),   o_i = S_i^T q_i
+//
+// is a system with a unit lower triangular matrix, A_ij = beta_i exp(L_i - L_j) (k_i . k_j) for j < i:
+//
+//   (I + A) U = diag(beta) V - diag(beta_i exp(L_i)) K S     =>   U = U0 - W S,
+//   (I + A) [W | U0] = [diag(beta_i exp(L_i)) K | diag(beta) V]
+//   o_i = exp(L_i) S^T q_i + sum_(j <= i) P_ij u_j,          P_ij = exp(L_i - L_j) (q_i . k_j)
+//   S  <- exp(L_64) S + sum_j exp(L_64 - L_j) k_j u_j^T
+//
+// (the form that is known from chunked linear recurrences as the WY representation of a product of rank-one updates).
+//
+//   delta_pieces_kernel   everything that does not need the state, a workgroup per piece and head: the products of keys and
+//                         queries, the solution W, U0 by blocks of 16 rows (the blocks on the diagonal inverted by
+//                         substitution, the others by products), and all operands of the second kernel, scaled, in the
+//                         order in which its matrix instructions take them, into the workspace
+//   delta_state_kernel    the walk through the pieces, a workgroup of four waves per head and 16 value columns
+//
+// Everything is 32-bit: products are v_mfma_f32_16x16x4_f32, sums of logarithms 64-bit.  A 16 x 16 result holds rows
+// 4 g + r (g = lane / 16) and column lane % 16; an operand of step r holds k = 4 g + r, so that a result is the next
+// product's right operand as it lies in registers (U0 - W S, then P U and K^T U), and left operands are 16 bytes a lane.
+// In delta_state_kernel wave w owns tokens 16 w .. 16 w + 15 of a piece for W S, Q S and P U, and a quarter of the key
+// channels of the state, kept in registers and, for the other waves, in LDS.  The next piece's operands are asked for while
+// this one is worked through.  Bound by the matrix instructions that a wave issues one after the other (about 110 of 32
+// clocks a piece) and two barriers a piece, on as many CUs as there are heads times blocks of 16 columns.
+//
+// Measured at 2,048 tokens of 16 heads over 8, sizes 128: 45 us for the pieces and 98 for the walk, where delta_rule.hip takes
+// 629 token by token.
+#include "api.h"
+#include "attention_common.h"
+
+namespace sa {
+namespace delta {
+
+constexpr int kTokens = 64, kBlocks = kTokens / 16;
+constexpr int kBlock = 256;   // floats of a 16 x 16 block
+
+// A piece's operands in the workspace (floats), for NT blocks of 16 key channels and CB blocks of 16 value columns.
+struct Layout {
+  int w, q, kt, p, u0, decay, words;
+};
+__host__ __device__ constexpr Layout layout(int nt, int cb) {
+  Layout l{};
+  l.w = 0;                             // [token block][channel block]
+  l.q = l.w + kBlocks * nt * kBlock;   // likewise
+  l.kt = l.q + kBlocks * nt * kBlock;  // [channel block][token block]
+  l.p = l.kt + kBlocks * nt * kBlock;  // [token block][token block]
+  l.u0 = l.p + kBlocks * kBlocks * kBlock;   // [column block][token block]
+  l.decay = l.u0 + cb * kBlocks * kBlock;    // exp(L_64)
+  l.words = l.decay + 64;
+  return l;
+}
+
+struct Args {
+  const float* qkv;     // [T, C]: q heads, k heads (G of them each), values
+  const float* gates;   // [T, 2 H]: beta, decay
+  float* state;         // per slot and head [dv][dk]
+  float* out;           // [T, H * dv]
+  float* pieces;
+  const int* seq_meta;
+  int64_t state_stride;
+  int C, G, H, dk, dv, row0, row1;   // the rows of the step that this launch is about
+};
+
+struct Span {
+  int slot, first, count, piece0;
+};
+// The part of a request that lies in the launch's rows; its pieces are numbered from piece0 on, no two requests' alike.
+__device__ __forceinline__ Span span_of(const Args& a, int seq) {
+  const int* meta = a.seq_meta + 4 * seq;
+  const int lo = meta[1] > a.row0 ? meta[1] : a.row0, end = meta[1] + meta[2], hi = end < a.row1 ? end : a.row1;
+  Span s;
+  s.slot = meta[0];
+  s.first = lo;
+  s.count = hi - lo;
+  s.piece0 = (lo - a.row0) / kTokens + seq;
+  return s;
+}
+
+__device__ __forceinline__ floatx4 mul4(floatx4 a, floatx4 b, floatx4 c) {   // four steps: 16 channels or tokens
+#pragma unroll
+  for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
+  return c;
+}
+
+template <int NT>
+__global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
+  constexpr int ROW = NT * 16 + 4, AROW = kTokens + 4, QUADS = NT * 4;
+  __shared__ __align__(16) float k_s[kTokens * ROW];
+  __shared__ __align__(16) float q_s[kTokens * ROW];   // rows of q; then A, then its diagonal blocks' inverses beside it
+  __shared__ double cum_s[kTokens];
+  __shared__ float beta_s[kTokens], in_s[kTokens], out_s[kTokens];   // beta, exp(L_i), exp(L_64 - L_i)
+  static_assert(kTokens * ROW >= kTokens * AROW || NT < 4, "A lies where q lay");
+  const Span sp = span_of(a, blockIdx.z);
+  const int t0 = blockIdx.x * kTokens;
+  if (t0 >= sp.count) return;   // (uniform)
+  const int left = sp.count - t0 < kTokens ? sp.count - t0 : kTokens;
+  const int h = blockIdx.y, tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
+  const int qk = h / (a.H / a.G), row0 = sp.first + t0;
+  const Layout lay = layout(NT, (a.dv + 15) / 16);
+  float* dst = a.pieces + (static_cast<size_t>(sp.piece0 + blockIdx.x) * a.H + h) * lay.words;
+
+  // rows of q and k (tokens behind the last, channels behind the last: zeros)
+#pragma unroll
+  for (int i = 0; i < kTokens * QUADS / 256; ++i) {
+    const int idx = tid + i * 256, j = idx / QUADS, d = idx % QUADS * 4;
+    floatx4 kv{0.f, 0.f, 0.f, 0.f}, qv{0.f, 0.f, 0.f, 0.f};
+    if (j < left && d < a.dk) {
+      const float* row = a.qkv + static_cast<size_t>(row0 + j) * a.C;
+      qv = *reinterpret_cast<const floatx4*>(row + qk * a.dk + d);
+      kv = *reinterpret_cast<const floatx4*>(row + (a.G + qk) * a.dk + d);
+    }
+    *reinterpret_cast<floatx4*>(&k_s[j * ROW + d]) = kv;
+    *reinterpret_cast<floatx4*>(&q_s[j * ROW + d]) = qv;
+  }
+  if (wave == 0) {
+    const bool live = lane < left;
+    const float* gr = a.gates + static_cast<size_t>(row0 + (live ? lane : 0)) * 2 * a.H + h;
+    const float beta = live ? gr[0] : 0.f, decay = live ? gr[a.H] : 1.f;
+    // (a decay of zero: a logarithm whose exponential is zero, so that differences stay defined)
+    double cum = decay > 0.f ? log(static_cast<double>(decay)) : decay == 0.f ? -1e4 : static_cast<double>(decay) * NAN;
+#pragma unroll
+    for (int by = 1; by < kWave; by *= 2) {
+      const double up = __shfl_up(cum, by, kWave);
+      if (lane >= by) cum += up;
+    }
+    const double end = __shfl(cum, kWave - 1, kWave);
+    cum_s[lane] = cum;
+    beta_s[lane] = beta;
+    in_s[lane] = expf(static_cast<float>(cum));
+    out_s[lane] = expf(static_cast<float>(end - cum));
+    if (lane == 0) dst[lay.decay] = expf(static_cast<float>(end));
+  }
+  __syncthreads();
+
+  // products of rows: P as [key token 4 g + r, query token c], which is the left operand's order, for key blocks b <= wave;
+  // k . k as [token 4 g + r, earlier token c], to become A
+  floatx4 kk[kBlocks];
+  const double cum_c = cum_s[wave * 16 + c];
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) {
+    kk[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (b <= wave) {   // (uniform over the wave)
+      floatx4 qk_b{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const floatx4 kb = *reinterpret_cast<const floatx4*>(&k_s[(b * 16 + c) * ROW + n * 16 + g * 4]);
+        const floatx4 kw = *reinterpret_cast<const floatx4*>(&k_s[(wave * 16 + c) * ROW + n * 16 + g * 4]);
+        const floatx4 qw = *reinterpret_cast<const floatx4*>(&q_s[(wave * 16 + c) * ROW + n * 16 + g * 4]);
+        qk_b = mul4(kb, qw, qk_b);
+        kk[b] = mul4(kw, kb, kk[b]);
+      }
+      floatx4 p;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = b * 16 + g * 4 + r, i = wave * 16 + c;
+        p[r] = j <= i ? qk_b[r] * expf(static_cast<float>(cum_c - cum_s[j])) : 0.f;
+      }
+      *reinterpret_cast<floatx4*>(dst + lay.p + (wave * kBlocks + b) * kBlock + lane * 4) = p;
+    }
+  }
+  // the queries times exp(L_i), and the keys times exp(L_64 - L_j), turned
+  {
+    const float e = in_s[wave * 16 + c];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const floatx4 q = *reinterpret_cast<const floatx4*>(&q_s[(wave * 16 + c) * ROW + n * 16 + g * 4]);
+      *reinterpret_cast<floatx4*>(dst + lay.q + (wave * NT + n) * kBlock + lane * 4) = floatx4{q[0] * e, q[1] * e, q[2] * e, q[3] * e};
+      floatx4 kt;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) kt[r] = k_s[(wave * 16 + g * 4 + r) * ROW + n * 16 + c] * out_s[wave * 16 + g * 4 + r];
+      *reinterpret_cast<floatx4*>(dst + lay.kt + (n * kBlocks + wave) * kBlock + lane * 4) = kt;
+    }
+  }
+  __syncthreads();   // (q has been read)
+  float* a_s = q_s;
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) {
+    if (b <= wave) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = wave * 16 + g * 4 + r, j = b * 16 + c;
+        a_s[i * AROW + j] = j < i ? kk[b][r] * beta_s[i] * expf(static_cast<float>(cum_s[i] - cum_s[j])) : 0.f;
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  // the inverse of the wave's diagonal block: lane c solves for column c (the four groups of lanes alike)
+  {
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float s[4] = {i == c ? 1.f : 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j4 = 0; j4 < (i + 3) / 4; ++j4) {
+        const floatx4 row = *reinterpret_cast<const floatx4*>(&a_s[(wave * 16 + i) * AROW + wave * 16 + j4 * 4]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (j4 * 4 + e < i) s[e] = fmaf(-row[e], x[j4 * 4 + e], s[e]);
+      }
+      x[i] = (s[0] + s[1]) + (s[2] + s[3]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // into the block's own place (its entries have been read)
+    if (g == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) a_s[(wave * 16 + i) * AROW + wave * 16 + c] = x[i];
+    }
+  }
+  __syncthreads();
+  // W and U0, 16 columns at a time: channels first, then value columns
+  const int cb = (a.dv + 15) / 16;
+  for (int n = wave; n < NT + cb; n += 4) {
+    floatx4 x[kBlocks];
+    const int col = (n - NT) * 16 + c;
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+      floatx4 acc;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = b * 16 + g * 4 + r;
+        if (n < NT) acc[r] = k_s[i * ROW + n * 16 + c] * (beta_s[i] * in_s[i]);
+        else acc[r] = (i < left && col < a.dv) ? a.qkv[static_cast<size_t>(row0 + i) * a.C + 2 * a.G * a.dk + h * a.dv + col] * beta_s[i] : 0.f;
+      }
+#pragma unroll
+      for (int e = 0; e < b; ++e) {
+        floatx4 m = *reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + e * 16 + g * 4]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m[r] = -m[r];
+        acc = mul4(m, x[e], acc);
+      }
+      const floatx4 inv = *reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + b * 16 + g * 4]);
+      x[b] = mul4(inv, acc, floatx4{0.f, 0.f, 0.f, 0.f});
+    }
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+      if (n < NT) {   // as a left operand: [token c][channels 4 g ..]; this lane has channel c of tokens 4 g + r
+        float* to = dst + lay.w + (b * NT + n) * kBlock + (c / 4) * 64 + c % 4;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) to[(g * 4 + r) * 4] = x[b][r];
+      } else {
+        *reinterpret_cast<floatx4*>(dst + lay.u0 + ((n - NT) * kBlocks + b) * kBlock + lane * 4) = x[b];
+      }
+    }
+  }
+}
+
+template <int NT>
+__global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
+  constexpr int NW = NT / 4;   // blocks of key channels whose state a wave holds
+  __shared__ __align__(16) floatx4 s_s[2][NT * kWave];
+  __shared__ __align__(16) floatx4 u_s[kBlocks * kWave];
+  const Span sp = span_of(a, blockIdx.z);
+  if (sp.count <= 0) return;
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
+  const int col = blockIdx.y * 16 + c;
+  const bool col_ok = col < a.dv;
+  const Layout lay = layout(NT, (a.dv + 15) / 16);
+  const float* src = a.pieces + (static_cast<size_t>(sp.piece0) * a.H + h) * lay.words;
+  const size_t step = static_cast<size_t>(a.H) * lay.words;
+  float* S = a.state + static_cast<size_t>(sp.slot) * a.state_stride + static_cast<size_t>(h) * a.dk * a.dv;
+  floatx4 s[NW];
+#pragma unroll
+  for (int n = 0; n < NW; ++n) {
+    const int d = (wave * NW + n) * 16 + g * 4;
+    s[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (col_ok && d < a.dk) s[n] = *reinterpret_cast<const floatx4*>(S + static_cast<size_t>(col) * a.dk + d);
+    s_s[0][(wave * NW + n) * kWave + lane] = s[n];
+  }
+  // a piece's operands, asked for a piece ahead
+  floatx4 w[NT], q[NT], kt[NW][kBlocks], p[kBlocks], u0;
+  float all;
+  auto fetch_state = [&](const float* from) __attribute__((always_inline)) {   // what U and the state behind the piece need
+#pragma unroll
+    for (int n = 0; n < NT; ++n) w[n] = *reinterpret_cast<const floatx4*>(from + lay.w + (wave * NT + n) * kBlock + lane * 4);
+    u0 = *reinterpret_cast<const floatx4*>(from + lay.u0 + (blockIdx.y * kBlocks + wave) * kBlock + lane * 4);
+  };
+  auto fetch_rest = [&](const float* from) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) q[n] = *reinterpret_cast<const floatx4*>(from + lay.q + (wave * NT + n) * kBlock + lane * 4);
+#pragma unroll
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b)
+        kt[n][b] = *reinterpret_cast<const floatx4*>(from + lay.kt + ((wave * NW + n) * kBlocks + b) * kBlock + lane * 4);
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {   // (blocks behind the wave's own: the own one again, not used)
+      const int at = b < wave ? b : wave;
+      p[b] = *reinterpret_cast<const floatx4*>(from + lay.p + (wave * kBlocks + at) * kBlock + lane * 4);
+    }
+    all = from[lay.decay];
+  };
+  fetch_state(src);
+  fetch_rest(src);
+  int now = 0;
+  for (int t0 = 0; t0 < sp.count; t0 += kTokens, now ^= 1) {
+    const float* next = t0 + kTokens < sp.count ? src + step : src;   // (behind the last piece: that one again, for nothing)
+    __syncthreads();   // the state in front of the piece is there
+    floatx4 st[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) st[n] = s_s[now][n * kWave + lane];
+    floatx4 x{0.f, 0.f, 0.f, 0.f}, y{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NT; n += 2) {
+      x = mul4(w[n], st[n], x);
+      y = mul4(w[n + 1], st[n + 1], y);
+    }
+    floatx4 u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = u0[r] - (x[r] + y[r]);
+    u_s[wave * kWave + lane] = u;
+    fetch_state(next);
+    floatx4 o{0.f, 0.f, 0.f, 0.f}, o2{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NT; n += 2) {
+      o = mul4(q[n], st[n], o);
+      o2 = mul4(q[n + 1], st[n + 1], o2);
+    }
+    __syncthreads();
+    floatx4 ub[kBlocks];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) ub[b] = u_s[b * kWave + lane];
+#pragma unroll
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[n][r] *= all;
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+      for (int n = 0; n < NW; ++n) s[n] = mul4(kt[n][b], ub[b], s[n]);
+#pragma unroll
+    for (int n = 0; n < NW; ++n) s_s[now ^ 1][(wave * NW + n) * kWave + lane] = s[n];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+      if (b <= wave) o = mul4(p[b], ub[b], o);   // (uniform over the wave)
+    fetch_rest(next);
+    if (col_ok) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = t0 + wave * 16 + g * 4 + r;
+        if (t < sp.count) a.out[static_cast<size_t>(sp.first + t) * (static_cast<size_t>(a.H) * a.dv) + static_cast<size_t>(h) * a.dv + col] = o[r] + o2[r];
+      }
+    }
+    src = next;
+  }
+#pragma unroll
+  for (int n = 0; n < NW; ++n) {
+    const int d = (wave * NW + n) * 16 + g * 4;
+    if (col_ok && d < a.dk) *reinterpret_cast<floatx4*>(S + static_cast<size_t>(col) * a.dk + d) = s[n];
+  }
+}
+
+}  // namespace delta
+}  // namespace sa
+
+using namespace sa;
+
+static int64_t delta_piece_bytes(int H, int dk, int dv) {
+  return static_cast<int64_t>(H) * delta::layout(dk <= 64 ? 4 : 8, (dv + 15) / 16).words * static_cast<int64_t>(sizeof(float));
+}
+
+extern "C" int sa_delta_chunks_takes(int C, int G, int H, int dk, int dv, int64_t state_stride, int num_seqs, int64_t workspace_bytes) {
+  return G > 0 && H > 0 && H % G == 0 && H <= 65535 && dk > 0 && dk <= 128 && dk % 4 == 0 && dv > 0 && dv <= 16 * 65535 &&
+         C % 4 == 0 && state_stride % 4 == 0 && num_seqs > 0 && num_seqs <= 65535 &&
+         (num_seqs + 1) * delta_piece_bytes(H, dk, dv) <= workspace_bytes;
+}
+
+extern "C" int sa_delta_chunks(const float* qkv, int C, int G, int dk, int dv, const float* gates, int H, float* state,
+                               int64_t state_stride, const int* seq_meta, int num_seqs, int first_row, int rows, int max_q_len,
+                               float* out, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+  if (num_seqs == 0 || rows == 0) return 0;
+  SA_REQUIRE(num_seqs > 0 && G > 0 && H > 0 && H % G == 0 && dk > 0 && dv > 0 && C >= 2 * G * dk + H * dv && first_row >= 0 &&
+                 rows > 0 && max_q_len > 0,
+             "delta_chunks: bad sizes S=%d C=%d G=%d H=%d dk=%d dv=%d", num_seqs, C, G, H, dk, dv);
+  SA_REQUIRE(qkv != nullptr && gates != nullptr && state != nullptr && seq_meta != nullptr && out != nullptr && workspace != nullptr &&
+                 reinterpret_cast<uintptr_t>(qkv) % 16 == 0 && reinterpret_cast<uintptr_t>(state) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
+             "delta_chunks: a null or unaligned pointer");
+  SA_REQUIRE(state_stride >= static_cast<int64_t>(H) * dk * dv, "delta_chunks: the state rows are too short");
+  SA_REQUIRE(sa_delta_chunks_takes(C, G, H, dk, dv, state_stride, num_seqs, workspace_bytes),
+             "delta_chunks: does not take keys of %d and values of %d, %d requests", dk, dv, num_seqs);
+  delta::Args a;
+  a.qkv = qkv, a.gates = gates, a.state = state, a.out = out, a.pieces = static_cast<float*>(workspace), a.seq_meta = seq_meta;
+  a.state_stride = state_stride, a.C = C, a.G = G, a.H = H, a.dk = dk, a.dv = dv;
+  // as many rows at a time as the workspace has room for: R rows are at most R / 64 + num_seqs pieces
+  const int64_t room = (workspace_bytes / delta_piece_bytes(H, dk, dv) - num_seqs) * delta::kTokens;
+  const int span = static_cast<int>(room < rows ? room : rows);
+  for (int r = 0; r < rows; r += span) {
+    a.row0 = first_row + r;
+    a.row1 = first_row + (r + span < rows ? r + span : rows);
+    const int longest = a.row1 - a.row0 < max_q_len ? a.row1 - a.row0 : max_q_len;
+    const dim3 pieces((longest + delta::kTokens - 1) / delta::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
+    if (dk <= 64) {
+      delta::delta_pieces_kernel<4><<<pieces, 256, 0, stream>>>(a);
+      delta::delta_state_kernel<4><<<walk, 256, 0, stream>>>(a);
+    } else {
+      delta::delta_pieces_kernel<8><<<pieces, 256, 0, stream>>>(a);
+      delta::delta_state_kernel<8><<<walk, 256, 0, stream>>>(a);
+    }
+  }
+  return check_launch("delta_chunks");
+}

@@ -84,6 +84,8 @@ _SIGNATURES = {
     "sa_delta_inputs_few_takes": [_I, _I],
     "sa_delta_prepare": [_P, _I, _I, _I, _I, _P, _I, _L, _P, _P, _I, _I, _P, _P],
     "sa_delta_rule": [_P, _I, _I, _I, _I, _P, _I, _P, _L, _P, _I, _P, _P],
+    "sa_delta_chunks_takes": [_I, _I, _I, _I, _I, _L, _I, _L],
+    "sa_delta_chunks": [_P, _I, _I, _I, _I, _P, _I, _P, _L, _P, _I, _I, _I, _I, _P, _P, _L, _P],
     "sa_embed_sum": [_P, _P, _P, _I, _I, _P, _I, _I, _P, _I, _L, _L, _L, _P, _L, _P, _I, _I, _P, _I, _P],
     "sa_token_gate": [_P, _I, _L, _P, _P, _I, _L, _I, _I, _I, _I, _P],
     "sa_bias_add": [_P, _I, _L, _P, _I, _I, _I, _P],

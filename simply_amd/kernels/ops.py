@@ -1389,25 +1389,53 @@ def delta_inputs(x: torch.Tensor, taps: torch.Tensor, tails: torch.Tensor, ab: t
     return qkv, gates
 
 
+def _delta_checks(name, qkv, gates, state, seq_meta, num_seqs, H, G, dk, dv, out) -> torch.Tensor:
+    _dev(qkv, gates, state, seq_meta, out)
+    T, C = qkv.shape
+    if qkv.dtype != torch.float32 or not qkv.is_contiguous() or C < 2 * G * dk + H * dv:
+        raise KernelError(f"{name}: qkv must be contiguous float32 [T, >= 2 G dk + H dv]")
+    if gates.dtype != torch.float32 or tuple(gates.shape) != (T, 2 * H) or not gates.is_contiguous():
+        raise KernelError(f"{name}: gates must be contiguous float32 [T, 2 H]")
+    if state.dtype != torch.float32 or state.dim() != 2 or state.stride(1) != 1 or state.shape[1] < H * dk * dv:
+        raise KernelError(f"{name}: the state must be float32 [slots, >= H * dk * dv]")
+    _seq_meta(seq_meta, num_seqs, name)
+    if out is None:
+        out = torch.empty((T, H * dv), dtype=torch.float32, device=qkv.device)
+    if out.dtype != torch.float32 or tuple(out.shape) != (T, H * dv) or not out.is_contiguous():
+        raise KernelError(f"{name}: out must be contiguous float32 [T, H * dv]")
+    return out
+
+
 def delta_rule(qkv: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, seq_meta: torch.Tensor, num_seqs: int,
-               num_heads: int, num_qk_heads: int, key_dim: int, value_dim: int) -> torch.Tensor:
+               num_heads: int, num_qk_heads: int, key_dim: int, value_dim: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """The gated delta rule along each request's tokens, from and into state [slots, >= H * dk * dv] float32 (per
     slot and head the matrix S [dk, dv], stored column by column: [H][dv][dk]).  qkv float32 [T, C] as `delta_prepare` left it, gates [T, 2 H].  Returns float32 [T, H * dv]."""
-    _dev(qkv, gates, state, seq_meta)
-    T, C = qkv.shape
     H, G, dk, dv = num_heads, num_qk_heads, key_dim, value_dim
-    if qkv.dtype != torch.float32 or not qkv.is_contiguous() or C < 2 * G * dk + H * dv:
-        raise KernelError("delta_rule: qkv must be contiguous float32 [T, >= 2 G dk + H dv]")
-    if gates.dtype != torch.float32 or tuple(gates.shape) != (T, 2 * H) or not gates.is_contiguous():
-        raise KernelError("delta_rule: gates must be contiguous float32 [T, 2 H]")
-    if state.dtype != torch.float32 or state.dim() != 2 or state.stride(1) != 1 or state.shape[1] < H * dk * dv:
-        raise KernelError("delta_rule: the state must be float32 [slots, >= H * dk * dv]")
-    if seq_meta.dtype != torch.int32 or seq_meta.dim() != 2 or seq_meta.shape[1] != 4 or not seq_meta.is_contiguous() \
-            or seq_meta.shape[0] < num_seqs:
-        raise KernelError("delta_rule: seq_meta must be int32 [S, 4]")
-    out = torch.empty((T, H * dv), dtype=torch.float32, device=qkv.device)
-    _lib.call("sa_delta_rule", _ptr(qkv), C, G, dk, dv, _ptr(gates), H, _ptr(state), state.stride(0), _ptr(seq_meta),
+    out = _delta_checks("delta_rule", qkv, gates, state, seq_meta, num_seqs, H, G, dk, dv, out)
+    _lib.call("sa_delta_rule", _ptr(qkv), qkv.shape[1], G, dk, dv, _ptr(gates), H, _ptr(state), state.stride(0), _ptr(seq_meta),
               int(num_seqs), _ptr(out), _stream())
+    return out
+
+
+def delta_chunks_takes(qkv: torch.Tensor, state: torch.Tensor, num_seqs: int, num_heads: int, num_qk_heads: int, key_dim: int,
+                       value_dim: int) -> bool:
+    """Whether `delta_chunks` takes these sizes (key sizes up to 128 and rows in multiples of 4, aligned)."""
+    return qkv.is_cuda and state.data_ptr() % 16 == 0 and qkv.data_ptr() % 16 == 0 and bool(_lib.load().sa_delta_chunks_takes(
+        qkv.shape[1], int(num_qk_heads), int(num_heads), int(key_dim), int(value_dim), state.stride(0), int(num_seqs),
+        WORKSPACE_BYTES))
+
+
+def delta_chunks(qkv: torch.Tensor, gates: torch.Tensor, state: torch.Tensor, seq_meta: torch.Tensor, num_seqs: int,
+                 first_row: int, max_q_len: int, num_heads: int, num_qk_heads: int, key_dim: int, value_dim: int,
+                 out: torch.Tensor) -> torch.Tensor:
+    """`delta_rule` for requests that bring portions of prompts, 64 tokens at a time on the matrix cores: seq_meta's first
+    num_seqs rows, whose tokens are the step's rows from first_row on."""
+    H, G, dk, dv = num_heads, num_qk_heads, key_dim, value_dim
+    out = _delta_checks("delta_chunks", qkv, gates, state, seq_meta, num_seqs, H, G, dk, dv, out)
+    T, C = qkv.shape
+    ws = _workspace(qkv.device)
+    _lib.call("sa_delta_chunks", _ptr(qkv), C, G, dk, dv, _ptr(gates), H, _ptr(state), state.stride(0), _ptr(seq_meta),
+              int(num_seqs), int(first_row), T - int(first_row), int(max_q_len), _ptr(out), _ptr(ws), ws.numel(), _stream())
     return out
 
 

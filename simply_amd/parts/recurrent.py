@@ -23,6 +23,9 @@ from .base import Mixer, ParamSpec, StateNeed, as_product_weight
 
 @MIXERS.register("gated_delta")
 class GatedDelta(Mixer):
+    #: tokens of a request in a step from which the recurrence is worked through in pieces
+    PIECES_FROM = 96
+
     def __init__(self, hidden_size: int, num_heads: int, num_qk_heads: int, key_dim: int, value_dim: int,
                  conv_taps: int, norm_eps: float):
         if num_heads % num_qk_heads:
@@ -70,7 +73,21 @@ class GatedDelta(Mixer):
         state, tails = cache.state[:, :self.state_words], cache.state[:, self.state_words:]
         qkv, gates = ops.delta_inputs(proj[:, :C], self.taps, tails, ab, self.a_log, self.dt_bias, ctx.seq_meta,
                                       ctx.num_seqs, ctx.max_q_len, H, G, dk)
-        o = ops.delta_rule(qkv, gates, state, ctx.seq_meta, ctx.num_seqs, H, G, dk, dv)
+        # Requests with few tokens go through the recurrence token by token, portions of prompts of a bfloat16 run in pieces
+        # on the matrix cores where these take the sizes (2,048 tokens of 16 heads of 128: 629 against 143 us; one token
+        # after the other takes 0.3 us each, the pieces' two kernels 25 us and 0.5 to 3 a piece: even at about 96 tokens of one
+        # request, at 32 to 64 of eight).  A 32-bit run, whose
+        # results do not depend on how the tokens are cut into steps, stays with the rule token by token.
+        o = torch.empty((x.shape[0], H * dv), dtype=torch.float32, device=x.device)
+        short = ctx.num_seqs
+        if ctx.dtype == torch.bfloat16 and ctx.max_q_len >= self.PIECES_FROM:
+            few, rows = ctx.short_requests(self.PIECES_FROM - 1)
+            if ops.delta_chunks_takes(qkv, state, ctx.num_seqs - few, H, G, dk, dv):
+                short = few
+                ops.delta_chunks(qkv, gates, state, ctx.seq_meta[short:], ctx.num_seqs - short, rows, ctx.max_q_len, H, G, dk,
+                                 dv, out=o)
+        if short:
+            ops.delta_rule(qkv, gates, state, ctx.seq_meta, short, H, G, dk, dv, out=o)
         z = ops.gated_heads(o, proj[:, C:C + H * dv], H, dv, kind=ops.GATE_SILU, weight=self.norm, eps=self.norm_eps,
                             out_dtype=ctx.dtype)
         return ops.gemm(z, self.o_proj)

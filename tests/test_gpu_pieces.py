@@ -1,0 +1,75 @@
+"""Recurrences worked through in pieces of tokens on the matrix cores, against their token-by-token definition in 64 bits:
+pieces that are full, short, alone and many; sizes that fill no block; decays near one, near zero, zero and one."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def uniform(shape, seed, lo=0.0, hi=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return torch.rand(shape, generator=g) * (hi - lo) + lo
+
+
+def normal(shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed))
+
+
+def delta_64(qkv, gates, state, meta, H, G, dk, dv):
+    """The definition, token by token."""
+    T = qkv.shape[0]
+    out, state = torch.zeros(T, H, dv, dtype=torch.float64), state.double().clone()
+    q, k, v = (t.reshape(T, -1, d).double() for t, d in zip(qkv[:, :2 * G * dk + H * dv].split([G * dk, G * dk, H * dv], 1), (dk, dk, dv)))
+    q, k = (t.repeat_interleave(H // G, 1) for t in (q, k))
+    beta, decay = gates.double().split(H, 1)
+    for slot, first, count, _ in meta:
+        S = state[slot, :H * dk * dv].reshape(H, dv, dk).transpose(1, 2).clone()
+        for t in range(first, first + count):
+            S = decay[t][:, None, None] * S
+            u = beta[t][:, None] * (v[t] - (k[t][:, :, None] * S).sum(1))
+            S = S + k[t][:, :, None] * u[:, None, :]
+            out[t] = (q[t][:, :, None] * S).sum(1)
+        state[slot, :H * dk * dv] = S.transpose(1, 2).reshape(-1)
+    return out.reshape(T, H * dv), state
+
+
+@pytest.mark.parametrize("H,G,dk,dv,kind", [(2, 1, 128, 128, "slow"), (4, 4, 64, 64, "fast"), (3, 1, 20, 24, "ends"),
+                                            (2, 2, 100, 130, "slow"), (2, 1, 128, 40, "alike"), (1, 1, 4, 3, "fast")])
+def test_delta_rule(H, G, dk, dv, kind):
+    """The kernel's error against 64 bits stays within three times that of the token-by-token kernel (both are sums of 32-bit
+    products in another order; three for the exponentials and the substitution) and below 1e-5 of the largest result."""
+    from simply_amd.kernels import ops
+
+    counts, before = [1, 15, 64, 65, 130, 200], 3
+    T = before + sum(counts)
+    meta, row = [], before
+    for i, n in enumerate(counts):
+        meta.append((5 - i if i else 6, row, n, 0))
+        row += n
+    C = 2 * G * dk + H * dv
+    C += -C % 4
+    qkv = normal((T, C), 51)
+    heads = qkv[:, :2 * G * dk].reshape(T, 2 * G, dk)
+    if kind == "alike":   # keys that nearly repeat, taken whole: what the triangular system is hardest on
+        heads[:, G:] = heads[:1, G:] + 0.05 * heads[:, G:]
+    heads = heads / heads.square().sum(-1, keepdim=True).sqrt()
+    heads[:, :G] *= dk ** -0.5
+    qkv[:, :2 * G * dk] = heads.reshape(T, -1)
+    beta = uniform((T, H), 52) if kind != "alike" else uniform((T, H), 52, 0.95, 1.0)
+    decay = {"slow": 1.0 - 0.01 * uniform((T, H), 53), "fast": uniform((T, H), 53), "alike": torch.ones(T, H),
+             "ends": torch.randint(0, 2, (T, H), generator=torch.Generator().manual_seed(53)).float()}[kind]
+    gates = torch.cat([beta, decay], 1).contiguous()
+    state = torch.cat([normal((7, H * dk * dv), 54), torch.zeros(7, 4 + -(H * dk * dv) % 4)], 1)
+    want, want_state = delta_64(qkv, gates, state, meta, H, G, dk, dv)
+    dev_meta = torch.tensor(meta, dtype=torch.int32).cuda()
+    args = (qkv.cuda(), gates.cuda())
+    s1, s2 = state.cuda(), state.cuda()
+    one = ops.delta_rule(*args, s1, dev_meta, len(meta), H, G, dk, dv)
+    out = torch.zeros(T, H * dv, device="cuda")
+    assert ops.delta_chunks_takes(args[0], s2, len(meta), H, G, dk, dv)
+    ops.delta_chunks(*args, s2, dev_meta, len(meta), before, max(counts), H, G, dk, dv, out=out)
+    assert not out[:before].any()
+    for got, ref, plain in ((out[before:], want[before:], one[before:]), (s2, want_state, s1)):
+        err, base, top = ((x.double().cpu() - ref).abs().max() for x in (got, plain, torch.zeros_like(got)))
+        print(kind, float(err / top), float(base / top))
+        assert err <= 3 * base and err <= 1e-5 * top, (float(err), float(base), float(top))

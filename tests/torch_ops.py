@@ -22,7 +22,7 @@ STAND_INS = ("embed", "rmsnorm", "add_rmsnorm", "rope_cache_write", "rope", "gat
              "paged_attention_maps", "attention_maps_units_takes", "norm_rope_cache_write", "short_conv",
              "head_product", "rglru_scan", "attention_inputs", "route_choice", "token_shift", "low_rank_decay",
              "concat_rows", "gemm_sections", "streams", "ssm_inputs", "gated_group_norm",
-             "state_chunks_takes", "state_chunks")
+             "state_chunks_takes", "state_chunks", "attention_f32_takes", "delta_chunks_takes", "delta_chunks")
 
 EPILOGUE_NONE, EPILOGUE_GATED_GELU, EPILOGUE_SOFT_CAP = 0, 1, 2
 ALGO_AUTO, ALGO_GENERIC, ALGO_SKINNY, ALGO_TILED = 0, 1, 2, 3
@@ -368,10 +368,20 @@ def delta_inputs(x, taps, tails, ab, a_log, dt_bias, seq_meta, num_seqs, max_q_l
     return qkv, delta_prepare(qkv, ab, a_log, dt_bias, num_heads, num_qk_heads, key_dim)
 
 
-def delta_rule(qkv, gates, state, seq_meta, num_seqs, num_heads, num_qk_heads, key_dim, value_dim):
+def delta_chunks_takes(qkv, state, num_seqs, num_heads, num_qk_heads, key_dim, value_dim):
+    return True
+
+
+def delta_chunks(qkv, gates, state, seq_meta, num_seqs, first_row, max_q_len, num_heads, num_qk_heads, key_dim, value_dim, out):
+    assert num_seqs > 0 and int(seq_meta[0, 1]) == first_row and int(seq_meta[:num_seqs, 2].sum()) == len(qkv) - first_row
+    return delta_rule(qkv, gates, state, seq_meta, num_seqs, num_heads, num_qk_heads, key_dim, value_dim, out)
+
+
+def delta_rule(qkv, gates, state, seq_meta, num_seqs, num_heads, num_qk_heads, key_dim, value_dim, out=None):
     T, C = qkv.shape
     H, G, dk, dv = num_heads, num_qk_heads, key_dim, value_dim
-    out = torch.empty((T, H * dv), dtype=torch.float32, device=qkv.device)
+    if out is None:
+        out = torch.empty((T, H * dv), dtype=torch.float32, device=qkv.device)
     x, gt = _f(qkv), _f(gates)
     for slot, first, count, _ in seq_meta[:num_seqs].tolist():
         S = _f(state[slot, :H * dk * dv]).reshape(H, dv, dk).transpose(1, 2).clone()   # stored column by column
