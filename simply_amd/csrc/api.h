@@ -497,6 +497,16 @@ int sa_linear_state(const void* proj, int dtype, int64_t proj_stride, int q_at, 
                     const void* bonus, int bonus_dtype, const void* skip, int skip_dtype, int H, int key_heads, int dk, int dv,
                     int ones, float* state, int64_t state_stride, const int* seq_meta, int num_seqs, float* out,
                     hipStream_t stream);
+// sa_linear_state with scalar = 0, ones = 0 and a bfloat16 proj for requests that bring portions, 64 tokens at a time on the
+// matrix cores (linear_chunks.hip): rows first_row .. first_row + rows - 1 of the step hold the requests' tokens, request by
+// request in seq_meta's order, at most max_q_len of each.  The workspace holds what is computed ahead of the state.
+// sa_linear_chunks_takes: key sizes up to 128 and columns and rows in multiples of 4, room for one piece more than requests.
+int sa_linear_chunks_takes(int H, int dk, int dv, int q_at, int k_at, int64_t proj_stride, int64_t gates_stride,
+                           int64_t state_stride, int num_seqs, int64_t workspace_bytes);
+int sa_linear_chunks(const void* proj, int64_t proj_stride, int q_at, int k_at, int v_at, float q_mult, const float* gates,
+                     int64_t gates_stride, const void* gate_bias, int bias_dtype, float tau, const void* bonus, int bonus_dtype,
+                     int H, int dk, int dv, float* state, int64_t state_stride, const int* seq_meta, int num_seqs, int first_row,
+                     int rows, int max_q_len, float* out, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 // sa_linear_state with scalar = 1, ones = 0, q_mult = 1 for requests that bring many tokens, 64 at a time on the matrix cores
 // (state_chunks.hip).  gates [T, >= 3 H]: decays, input factors, the decays' logarithms (the first are not read).
 // sa_state_chunks_takes: key sizes up to 128 in multiples of 8, value sizes in multiples of 4, columns and rows of proj in

@@ -1,0 +1,392 @@
+// The recurrence of linear_state.hip with a decay per key channel, for portions of prompts of bfloat16 runs, on the matrix
+// cores: 64 tokens (a piece) at a time.  With S the state in front of a piece and D_(a..b) the product of the decays of
+// tokens a .. b, channel by channel,
+//
+//   o_i = (D_(1..i-1) q_i)^T S + sum_(j < i) M_ij v_j + ((bonus q_i) . k_i) v_i,   M_ij = sum_d q_i k_j D_(j+1..i-1)
+//   S  <- D_(1..64) S + sum_j (D_(j+1..64) k_j) v_j^T
+//
+// (without a bonus a token reads the state behind it: D_(1..i), M_ij with D_(j+1..i) and M_ii = q_i . k_i).  No logarithms
+// and no quotients of decays: products of decays between two tokens are taken as such, so that a decay of zero, or many
+// small ones, do no harm.  Within a block of 16 tokens a lane holds a key and carries it from token to token, multiplied by
+// their decays (16 lanes: the block's tokens; four groups of lanes: channels 16 n + 4 g + r); what it has become at the
+// block's end is what later blocks see of it, and a query multiplied by the decays in front of it in its block, then by whole
+// blocks', meets those keys in matrix products.
+//
+//   linear_pieces_kernel   everything that does not need the state, a workgroup per piece and head: M and the scaled queries,
+//                          keys and values, in the order in which the second kernel's instructions take them
+//   linear_walk_kernel     the walk through the pieces, a workgroup of four waves per head and 16 value columns, as
+//                          delta_state_kernel does it (delta_chunks.hip), with one barrier a piece
+//
+// Sums and products are 32-bit (v_mfma_f32_16x16x4_f32).  The first kernel is bound by a wave's vector instructions (16
+// steps of 96 multiplications and the operands' reads from LDS), the second by its matrix instructions one after the other.
+//
+// Measured at 2,048 tokens of 16 heads of 128: 33 us for the pieces and 73 for the walk, where linear_state.hip takes 703
+// token by token.
+#include "api.h"
+#include "attention_common.h"
+
+namespace sa {
+namespace linear {
+
+constexpr int kTokens = 64, kBlocks = kTokens / 16;
+constexpr int kBlock = 256;   // floats of a 16 x 16 block
+
+// A piece's operands in the workspace (floats), for NT blocks of 16 key channels and CB blocks of 16 value columns.
+struct Layout {
+  int q, kt, p, v, all, words;
+};
+__host__ __device__ constexpr Layout layout(int nt, int cb) {
+  Layout l{};
+  l.q = 0;                              // [token block][channel block]
+  l.kt = l.q + kBlocks * nt * kBlock;   // [channel block][token block]
+  l.p = l.kt + kBlocks * nt * kBlock;   // [token block][token block]
+  l.v = l.p + kBlocks * kBlocks * kBlock;   // [column block][token block]
+  l.all = l.v + cb * kBlocks * kBlock;      // [16 nt] the decays of the whole piece
+  l.words = l.all + 16 * nt;
+  return l;
+}
+
+struct Args {
+  const bf16* proj;
+  const float* gates;   // [T, >= H dk]: decays, or z where inv_tau > 0
+  const void* gate_bias;
+  const void* bonus;
+  float* state;         // per slot and head [dv][dk]
+  float* out;           // [T, H * dv]
+  float* pieces;
+  const int* seq_meta;
+  int64_t proj_stride, gates_stride, state_stride;
+  float q_mult, inv_tau;
+  int q_at, k_at, v_at, H, dk, dv, bias_dtype, bonus_dtype, row0, row1;
+};
+
+struct Span {
+  int slot, first, count, piece0;
+};
+// The part of a request that lies in the launch's rows; its pieces are numbered from piece0 on, no two requests' alike.
+__device__ __forceinline__ Span span_of(const Args& a, int seq) {
+  const int* meta = a.seq_meta + 4 * seq;
+  const int lo = meta[1] > a.row0 ? meta[1] : a.row0, end = meta[1] + meta[2], hi = end < a.row1 ? end : a.row1;
+  Span s;
+  s.slot = meta[0];
+  s.first = lo;
+  s.count = hi - lo;
+  s.piece0 = (lo - a.row0) / kTokens + seq;
+  return s;
+}
+
+__device__ __forceinline__ floatx4 mul4(floatx4 a, floatx4 b, floatx4 c) {   // four steps: 16 channels or tokens
+#pragma unroll
+  for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
+  return c;
+}
+__device__ __forceinline__ floatx4 to_float4(uint2 v) {   // four bfloat16
+  return floatx4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                 __uint_as_float(v.y & 0xffff0000u)};
+}
+
+template <int NT, bool BONUS>
+__global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
+  constexpr int QUADS = NT * 4, AROW = NT * 16 + 4, QROW = NT * 16 + 8;
+  __shared__ __align__(16) float a_s[kTokens * AROW];   // decays; then the keys as later blocks see them, [block][channel block][lane]
+  __shared__ __align__(16) bf16 q_s[kTokens * QROW];
+  __shared__ __align__(16) bf16 k_s[kTokens * QROW];
+  __shared__ __align__(16) float blk_s[kBlocks][NT * 16];   // a block's decays, multiplied
+  const Span sp = span_of(a, blockIdx.z);
+  const int t0 = blockIdx.x * kTokens;
+  if (t0 >= sp.count) return;   // (uniform)
+  const int left = sp.count - t0 < kTokens ? sp.count - t0 : kTokens;
+  const int h = blockIdx.y, tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
+  const int row0 = sp.first + t0, cb = (a.dv + 15) / 16;
+  const Layout lay = layout(NT, cb);
+  float* dst = a.pieces + (static_cast<size_t>(sp.piece0 + blockIdx.x) * a.H + h) * lay.words;
+
+  // rows of q, k and the decays (tokens behind the last: nothing, decays of one; channels behind the last: zeros)
+#pragma unroll
+  for (int i = 0; i < kTokens * QUADS / 256; ++i) {
+    const int idx = tid + i * 256, j = idx / QUADS, d = idx % QUADS * 4;
+    const bool ok = j < left && d < a.dk;
+    uint2 qv{0, 0}, kv{0, 0};
+    floatx4 av{1.f, 1.f, 1.f, 1.f};
+    if (ok) {
+      const bf16* row = a.proj + static_cast<size_t>(row0 + j) * a.proj_stride + h * a.dk + d;
+      qv = *reinterpret_cast<const uint2*>(row + a.q_at);
+      kv = *reinterpret_cast<const uint2*>(row + a.k_at);
+      av = *reinterpret_cast<const floatx4*>(a.gates + static_cast<size_t>(row0 + j) * a.gates_stride + h * a.dk + d);
+      if (a.inv_tau > 0.f) {   // a = sigmoid(z + bias)^(1 / tau)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float z = av[e] + (a.gate_bias != nullptr ? load_f(a.gate_bias, a.bias_dtype, h * a.dk + d + e) : 0.f);
+          av[e] = __expf((fminf(z, 0.f) - __logf(1.f + __expf(-fabsf(z)))) * a.inv_tau);
+        }
+      }
+    }
+    *reinterpret_cast<uint2*>(&q_s[j * QROW + d]) = qv;
+    *reinterpret_cast<uint2*>(&k_s[j * QROW + d]) = kv;
+    *reinterpret_cast<floatx4*>(&a_s[j * AROW + d]) = av;
+  }
+  __syncthreads();
+  // values of the wave's tokens, as the right operand
+  for (int n = 0; n < cb; ++n) {
+    const int col = n * 16 + c;
+    floatx4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = wave * 16 + g * 4 + r;
+      v[r] = j < left && col < a.dv ? to_float(a.proj[static_cast<size_t>(row0 + j) * a.proj_stride + a.v_at + h * a.dv + col]) : 0.f;
+    }
+    *reinterpret_cast<floatx4*>(dst + lay.v + (n * kBlocks + wave) * kBlock + lane * 4) = v;
+  }
+  // the block of 16 tokens on the diagonal: lane c has query c (qp, times the decays in front of it in the block) and key c
+  // (kw, times the decays behind it so far); step i brings token i's decays and its query to all lanes' keys
+  floatx4 qp[NT], kw[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    qp[n] = to_float4(*reinterpret_cast<const uint2*>(&q_s[(wave * 16 + c) * QROW + n * 16 + g * 4])) * a.q_mult;
+    kw[n] = to_float4(*reinterpret_cast<const uint2*>(&k_s[(wave * 16 + c) * QROW + n * 16 + g * 4]));
+  }
+  float own = 0.f;   // M_cc, by the lane's channels
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float x = qp[n][r] * kw[n][r];
+      const int d = n * 16 + g * 4 + r;
+      if (BONUS) x *= d < a.dk ? load_f(a.bonus, a.bonus_dtype, static_cast<size_t>(h) * a.dk + d) : 0.f;
+      own += x;
+    }
+  own = sum_over_row_lanes(own);
+  float m_c[4] = {0.f, 0.f, 0.f, 0.f};   // M[query 4 g + r][key c] of the block
+#pragma unroll 1
+  for (int i4 = 0; i4 < 4; ++i4) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = i4 * 4 + e;
+      floatx4 av[NT];
+      float s = 0.f;
+      const float* ap = &a_s[(wave * 16 + i) * AROW + g * 4];
+      const bf16* qi = &q_s[(wave * 16 + i) * QROW + g * 4];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) av[n] = *reinterpret_cast<const floatx4*>(ap + n * 16);
+      if (!BONUS && c < i) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) kw[n] *= av[n];
+      }
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const floatx4 q = to_float4(*reinterpret_cast<const uint2*>(qi + n * 16));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s = fmaf(q[r], kw[n][r], s);
+      }
+      if (BONUS && c < i) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) kw[n] *= av[n];
+      }
+      if (BONUS ? i < c : i <= c) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) qp[n] *= av[n];
+      }
+      s = sum_over_row_lanes(s) * a.q_mult;
+      s = c < i ? s : c == i ? own : 0.f;
+      if (g == i4) m_c[e] = s;
+    }
+  }
+  // the block's M, turned: as the left operand lane (query c, group g) has keys 4 g .. 4 g + 3
+  {
+    float* to = dst + lay.p + (wave * kBlocks + wave) * kBlock + (c / 4) * 64 + c % 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) to[(g * 4 + e) * 4] = m_c[e];
+  }
+  // the block's decays, channel by channel
+#pragma unroll
+  for (int d = lane; d < NT * 16; d += kWave) {
+    float x = 1.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x *= a_s[(wave * 16 + j) * AROW + d];
+    blk_s[wave][d] = x;
+  }
+  __syncthreads();   // (the decays have been read)
+  floatx4* key_s = reinterpret_cast<floatx4*>(a_s);
+  static_assert(kBlocks * NT * kWave * 16 <= kTokens * AROW * 4, "the keys lie where the decays lay");
+#pragma unroll
+  for (int n = 0; n < NT; ++n) key_s[(wave * NT + n) * kWave + lane] = kw[n];
+  __syncthreads();
+  // keys of earlier blocks, from the nearest on; the queries take a block's decays on the way
+#pragma unroll 1
+  for (int b = wave - 1; b >= 0; --b) {
+    floatx4 x{0.f, 0.f, 0.f, 0.f}, y{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NT; n += 2) {
+      x = mul4(key_s[(b * NT + n) * kWave + lane], qp[n], x);
+      y = mul4(key_s[(b * NT + n + 1) * kWave + lane], qp[n + 1], y);
+    }
+    *reinterpret_cast<floatx4*>(dst + lay.p + (wave * kBlocks + b) * kBlock + lane * 4) = x + y;   // [key 4 g + r][query c]
+#pragma unroll
+    for (int n = 0; n < NT; ++n) qp[n] *= *reinterpret_cast<const floatx4*>(&blk_s[b][n * 16 + g * 4]);
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) *reinterpret_cast<floatx4*>(dst + lay.q + (wave * NT + n) * kBlock + lane * 4) = qp[n];
+  // the wave's keys times the decays of the blocks behind, turned: [channel c][tokens 4 g ..]
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    float f = 1.f;
+    for (int b = wave + 1; b < kBlocks; ++b) f *= blk_s[b][n * 16 + c];
+    floatx4 kt;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) kt[r] = a_s[((wave * NT + n) * kWave + (c / 4) * 16 + g * 4 + r) * 4 + c % 4] * f;
+    *reinterpret_cast<floatx4*>(dst + lay.kt + (n * kBlocks + wave) * kBlock + lane * 4) = kt;
+  }
+  if (tid < NT * 16) dst[lay.all + tid] = blk_s[0][tid] * blk_s[1][tid] * blk_s[2][tid] * blk_s[3][tid];
+}
+
+template <int NT>
+__global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
+  constexpr int NW = NT / 4;   // blocks of key channels whose state a wave holds
+  __shared__ __align__(16) floatx4 s_s[2][NT * kWave];
+  const Span sp = span_of(a, blockIdx.z);
+  if (sp.count <= 0) return;
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
+  const int col = blockIdx.y * 16 + c;
+  const bool col_ok = col < a.dv;
+  const Layout lay = layout(NT, (a.dv + 15) / 16);
+  const float* src = a.pieces + (static_cast<size_t>(sp.piece0) * a.H + h) * lay.words;
+  const size_t step = static_cast<size_t>(a.H) * lay.words;
+  float* S = a.state + static_cast<size_t>(sp.slot) * a.state_stride + static_cast<size_t>(h) * a.dk * a.dv;
+  floatx4 s[NW];
+#pragma unroll
+  for (int n = 0; n < NW; ++n) {
+    const int d = (wave * NW + n) * 16 + g * 4;
+    s[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (col_ok && d < a.dk) s[n] = *reinterpret_cast<const floatx4*>(S + static_cast<size_t>(col) * a.dk + d);
+    s_s[0][(wave * NW + n) * kWave + lane] = s[n];
+  }
+  // a piece's operands, asked for a piece ahead
+  floatx4 q[NT], kt[NW][kBlocks], p[kBlocks], v[kBlocks], all[NW];
+  auto fetch_state = [&](const float* from) __attribute__((always_inline)) {   // what the state behind the piece needs
+#pragma unroll
+    for (int n = 0; n < NW; ++n) {
+      all[n] = *reinterpret_cast<const floatx4*>(from + lay.all + (wave * NW + n) * 16 + g * 4);
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b)
+        kt[n][b] = *reinterpret_cast<const floatx4*>(from + lay.kt + ((wave * NW + n) * kBlocks + b) * kBlock + lane * 4);
+    }
+  };
+  auto fetch_rest = [&](const float* from) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) q[n] = *reinterpret_cast<const floatx4*>(from + lay.q + (wave * NT + n) * kBlock + lane * 4);
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+      v[b] = *reinterpret_cast<const floatx4*>(from + lay.v + (blockIdx.y * kBlocks + b) * kBlock + lane * 4);
+      const int at = b < wave ? b : wave;   // (blocks behind the wave's own: the own one again, not used)
+      p[b] = *reinterpret_cast<const floatx4*>(from + lay.p + (wave * kBlocks + at) * kBlock + lane * 4);
+    }
+  };
+  fetch_state(src);
+  fetch_rest(src);
+  int now = 0;
+  for (int t0 = 0; t0 < sp.count; t0 += kTokens, now ^= 1) {
+    const float* next = t0 + kTokens < sp.count ? src + step : src;   // (behind the last piece: that one again, for nothing)
+    __syncthreads();   // the state in front of the piece is there
+    floatx4 st[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) st[n] = s_s[now][n * kWave + lane];
+    // the state behind the piece, for the others to read
+#pragma unroll
+    for (int n = 0; n < NW; ++n) s[n] *= all[n];
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+      for (int n = 0; n < NW; ++n) s[n] = mul4(kt[n][b], v[b], s[n]);
+#pragma unroll
+    for (int n = 0; n < NW; ++n) s_s[now ^ 1][(wave * NW + n) * kWave + lane] = s[n];
+    fetch_state(next);
+    floatx4 o{0.f, 0.f, 0.f, 0.f}, o2{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NT; n += 2) {
+      o = mul4(q[n], st[n], o);
+      o2 = mul4(q[n + 1], st[n + 1], o2);
+    }
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+      if (b <= wave) o = mul4(p[b], v[b], o);   // (uniform over the wave)
+    fetch_rest(next);
+    if (col_ok) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = t0 + wave * 16 + g * 4 + r;
+        if (t < sp.count) a.out[static_cast<size_t>(sp.first + t) * (static_cast<size_t>(a.H) * a.dv) + static_cast<size_t>(h) * a.dv + col] = o[r] + o2[r];
+      }
+    }
+    src = next;
+  }
+#pragma unroll
+  for (int n = 0; n < NW; ++n) {
+    const int d = (wave * NW + n) * 16 + g * 4;
+    if (col_ok && d < a.dk) *reinterpret_cast<floatx4*>(S + static_cast<size_t>(col) * a.dk + d) = s[n];
+  }
+}
+
+}  // namespace linear
+}  // namespace sa
+
+using namespace sa;
+
+static int64_t linear_piece_bytes(int H, int dk, int dv) {
+  return static_cast<int64_t>(H) * linear::layout(dk <= 64 ? 4 : 8, (dv + 15) / 16).words * static_cast<int64_t>(sizeof(float));
+}
+
+extern "C" int sa_linear_chunks_takes(int H, int dk, int dv, int q_at, int k_at, int64_t proj_stride, int64_t gates_stride,
+                                      int64_t state_stride, int num_seqs, int64_t workspace_bytes) {
+  return H > 0 && H <= 65535 && dk > 0 && dk <= 128 && dk % 4 == 0 && dv > 0 && dv <= 16 * 65535 && q_at % 4 == 0 &&
+         k_at % 4 == 0 && proj_stride % 4 == 0 && gates_stride % 4 == 0 && state_stride % 4 == 0 && num_seqs > 0 &&
+         num_seqs <= 65535 && (num_seqs + 1) * linear_piece_bytes(H, dk, dv) <= workspace_bytes;
+}
+
+extern "C" int sa_linear_chunks(const void* proj, int64_t proj_stride, int q_at, int k_at, int v_at, float q_mult,
+                                const float* gates, int64_t gates_stride, const void* gate_bias, int bias_dtype, float tau,
+                                const void* bonus, int bonus_dtype, int H, int dk, int dv, float* state, int64_t state_stride,
+                                const int* seq_meta, int num_seqs, int first_row, int rows, int max_q_len, float* out,
+                                void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+  if (num_seqs == 0 || rows == 0) return 0;
+  SA_REQUIRE(num_seqs > 0 && H > 0 && dk > 0 && dv > 0 && first_row >= 0 && rows > 0 && max_q_len > 0 && tau >= 0.f,
+             "linear_chunks: bad sizes S=%d H=%d dk=%d dv=%d", num_seqs, H, dk, dv);
+  SA_REQUIRE(proj != nullptr && gates != nullptr && state != nullptr && seq_meta != nullptr && out != nullptr && workspace != nullptr &&
+                 reinterpret_cast<uintptr_t>(proj) % 8 == 0 && reinterpret_cast<uintptr_t>(gates) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(state) % 16 == 0 && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
+             "linear_chunks: a null or unaligned pointer");
+  SA_REQUIRE(q_at >= 0 && k_at >= 0 && v_at >= 0 && proj_stride >= q_at + static_cast<int64_t>(H) * dk &&
+                 proj_stride >= k_at + static_cast<int64_t>(H) * dk && proj_stride >= v_at + static_cast<int64_t>(H) * dv &&
+                 gates_stride >= static_cast<int64_t>(H) * dk && state_stride >= static_cast<int64_t>(H) * dk * dv,
+             "linear_chunks: rows of the projection, the gates or the state are too short");
+  SA_REQUIRE((gate_bias == nullptr || bias_dtype == kF32 || bias_dtype == kBF16) &&
+                 (bonus == nullptr || bonus_dtype == kF32 || bonus_dtype == kBF16) && (bonus == nullptr || tau == 0.f),
+             "linear_chunks: unknown dtype, or a bonus with tau");
+  SA_REQUIRE(sa_linear_chunks_takes(H, dk, dv, q_at, k_at, proj_stride, gates_stride, state_stride, num_seqs, workspace_bytes),
+             "linear_chunks: does not take keys of %d and values of %d, %d requests", dk, dv, num_seqs);
+  linear::Args a;
+  a.proj = static_cast<const bf16*>(proj), a.gates = gates, a.gate_bias = gate_bias, a.bonus = bonus, a.state = state, a.out = out;
+  a.pieces = static_cast<float*>(workspace), a.seq_meta = seq_meta, a.proj_stride = proj_stride, a.gates_stride = gates_stride;
+  a.state_stride = state_stride, a.q_mult = q_mult, a.inv_tau = tau > 0.f ? 1.f / tau : 0.f, a.q_at = q_at, a.k_at = k_at;
+  a.v_at = v_at, a.H = H, a.dk = dk, a.dv = dv, a.bias_dtype = bias_dtype, a.bonus_dtype = bonus_dtype;
+  // as many rows at a time as the workspace has room for: R rows are at most R / 64 + num_seqs pieces
+  const int64_t room = (workspace_bytes / linear_piece_bytes(H, dk, dv) - num_seqs) * linear::kTokens;
+  const int span = static_cast<int>(room < rows ? room : rows);
+  for (int r = 0; r < rows; r += span) {
+    a.row0 = first_row + r;
+    a.row1 = first_row + (r + span < rows ? r + span : rows);
+    const int longest = a.row1 - a.row0 < max_q_len ? a.row1 - a.row0 : max_q_len;
+    const dim3 pieces((longest + linear::kTokens - 1) / linear::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
+#define SA_LINEAR(NT)                                                                              \
+  do {                                                                                             \
+    if (bonus != nullptr) linear::linear_pieces_kernel<NT, true><<<pieces, 256, 0, stream>>>(a);   \
+    else linear::linear_pieces_kernel<NT, false><<<pieces, 256, 0, stream>>>(a);                   \
+    linear::linear_walk_kernel<NT><<<walk, 256, 0, stream>>>(a);                                   \
+  } while (0)
+    if (dk <= 64) SA_LINEAR(4);
+    else SA_LINEAR(8);
+#undef SA_LINEAR
+  }
+  return check_launch("linear_chunks");
+}

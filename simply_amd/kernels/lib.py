@@ -93,6 +93,9 @@ _SIGNATURES = {
     "sa_exp_gates": [_P, _L, _P, _I, _F, _I, _P, _L, _P, _I, _P, _P],
     "sa_linear_state": [_P, _I, _L, _I, _I, _I, _F, _P, _L, _P, _I, _F, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P, _L, _P, _I,
                         _P, _P],
+    "sa_linear_chunks_takes": [_I, _I, _I, _I, _I, _L, _L, _L, _I, _L],
+    "sa_linear_chunks": [_P, _L, _I, _I, _I, _F, _P, _L, _P, _I, _F, _P, _I, _I, _I, _I, _P, _L, _P, _I, _I, _I, _I, _P, _P, _L,
+                         _P],
     "sa_normalized_readout": [_P, _P, _L, _P, _I, _L, _P, _I, _F, _P, _I, _L, _I, _I, _I, _P],
     "sa_route": [_P, _L, _I, _I, _I, _F, _P, _P, _P],
     "sa_expert_sort": [_P, _I, _I, _I, _P, _P, _I, _P],

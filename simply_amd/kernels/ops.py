@@ -1675,6 +1675,43 @@ def linear_state(proj: torch.Tensor, q_at: int, k_at: int, v_at: int, q_mult: fl
     return out
 
 
+def linear_chunks_takes(proj: torch.Tensor, q_at: int, k_at: int, gates: torch.Tensor, state: torch.Tensor, num_seqs: int,
+                        num_heads: int, key_dim: int, value_dim: int) -> bool:
+    """Whether `linear_chunks` takes these sizes (bfloat16; key sizes up to 128, columns and rows in multiples of 4)."""
+    return proj.is_cuda and proj.dtype == torch.bfloat16 and proj.data_ptr() % 8 == 0 and gates.data_ptr() % 16 == 0 \
+        and state.data_ptr() % 16 == 0 and bool(_lib.load().sa_linear_chunks_takes(
+            int(num_heads), int(key_dim), int(value_dim), int(q_at), int(k_at), proj.stride(0), gates.stride(0), state.stride(0),
+            int(num_seqs), WORKSPACE_BYTES))
+
+
+def linear_chunks(proj: torch.Tensor, q_at: int, k_at: int, v_at: int, q_mult: float, gates: torch.Tensor, num_heads: int,
+                  key_dim: int, value_dim: int, state: torch.Tensor, seq_meta: torch.Tensor, num_seqs: int, first_row: int,
+                  max_q_len: int, *, decay_bias: torch.Tensor | None = None, tau: float | None = None,
+                  bonus: torch.Tensor | None = None, out: torch.Tensor) -> torch.Tensor:
+    """`linear_state` with a decay per key channel (not scalar, no normalizer) for requests that bring portions of prompts,
+    64 tokens at a time on the matrix cores: seq_meta's first num_seqs rows, whose tokens are the step's rows from
+    first_row on."""
+    _dev(proj, gates, state, seq_meta, decay_bias, bonus, out)
+    T, H, dk, dv = proj.shape[0], int(num_heads), int(key_dim), int(value_dim)
+    if proj.dtype != torch.bfloat16 or gates.dtype != torch.float32 or gates.shape[0] != T:
+        raise KernelError("linear_chunks: proj must be bfloat16, gates float32 with one row per token")
+    if state.dtype != torch.float32 or state.dim() != 2 or state.stride(1) != 1 or state.shape[1] < H * dk * dv:
+        raise KernelError("linear_chunks: the state must be float32 [slots, >= H * dk * dv]")
+    _seq_meta(seq_meta, num_seqs, "linear_chunks")
+    if any(v is not None and (v.numel() != H * dk or not v.is_contiguous()) for v in (decay_bias, bonus)) \
+            or (decay_bias is not None and tau is None) or (tau is not None and tau <= 0):
+        raise KernelError("linear_chunks: a bias (with a positive tau) or a bonus has one entry per head and key channel")
+    if out.dtype != torch.float32 or tuple(out.shape) != (T, H * dv) or not out.is_contiguous():
+        raise KernelError("linear_chunks: out must be contiguous float32 [T, H * dv]")
+    ws = _workspace(proj.device)
+    _lib.call("sa_linear_chunks", _ptr(proj), _rows(proj, "linear_chunks: proj"), int(q_at), int(k_at), int(v_at), float(q_mult),
+              _ptr(gates), _rows(gates, "linear_chunks: gates"), _ptr(decay_bias),
+              _code(decay_bias) if decay_bias is not None else 0, float(tau or 0.0), _ptr(bonus),
+              _code(bonus) if bonus is not None else 0, H, dk, dv, _ptr(state), state.stride(0), _ptr(seq_meta), int(num_seqs),
+              int(first_row), T - int(first_row), int(max_q_len), _ptr(out), _ptr(ws), ws.numel(), _stream())
+    return out
+
+
 def state_chunks_takes(proj: torch.Tensor, q_at: int, k_at: int, v_at: int, key_dim: int, value_dim: int,
                        state: torch.Tensor) -> bool:
     """Whether `state_chunks` takes these sizes (key sizes up to 128 in multiples of 8, value sizes in multiples of 4, aligned

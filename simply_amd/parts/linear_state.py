@@ -27,6 +27,27 @@ from ..registry import MIXERS
 from .base import Mixer, ParamSpec, StateNeed, as_product_weight, project
 
 
+#: tokens of a request in a step from which a recurrence with decays per channel is worked through in pieces: one request's 65
+#: tokens take 24 us in pieces and 21 one by one, 96 take 25 and 28 (eight requests': 35 and 30, 36 and 41; 16 heads of 128)
+PIECES_FROM = 80
+
+
+def channel_decay_state(proj, columns, q_mult, gates, H, dk, dv, state, ctx, **kw):
+    """`ops.linear_state` with a decay per key channel.  Requests with few tokens go through the recurrence token by token,
+    portions of prompts of a bfloat16 run in pieces on the matrix cores where these take the sizes."""
+    out = torch.empty((proj.shape[0], H * dv), dtype=torch.float32, device=proj.device)
+    short = ctx.num_seqs
+    if ctx.max_q_len >= PIECES_FROM and proj.dtype == torch.bfloat16:
+        few, rows = ctx.short_requests(PIECES_FROM - 1)
+        if ops.linear_chunks_takes(proj, columns[0], columns[1], gates, state, ctx.num_seqs - few, H, dk, dv):
+            short = few
+            ops.linear_chunks(proj, *columns, q_mult, gates, H, dk, dv, state, ctx.seq_meta[short:], ctx.num_seqs - short, rows,
+                              ctx.max_q_len, out=out, **kw)
+    if short:
+        ops.linear_state(proj, *columns, q_mult, gates, False, H, dk, dv, False, state, ctx.seq_meta, short, out=out, **kw)
+    return out
+
+
 @MIXERS.register("gated_linear_attention")
 class GatedLinearAttention(Mixer):
     #: the mixer's input enters one product only: for a few rows the norm in front of it runs in that product's kernel
@@ -73,8 +94,8 @@ class GatedLinearAttention(Mixer):
         # the decay's second factor is a product of its own, kept in 32-bit; sigmoid(. + bias)^(1 / tau) is computed
         # where the recurrence stages its tiles
         z = ops.gemm(proj[:, u_at:u_at + R], self.decay_out, out_dtype=torch.float32)
-        o = ops.linear_state(proj, 0, C, 2 * C, dk ** -0.5, z, False, H, dk, dv, False, cache.state, ctx.seq_meta,
-                             ctx.num_seqs, decay_bias=self.decay_bias, tau=self.tau)
+        o = channel_decay_state(proj, (0, C, 2 * C), dk ** -0.5, z, H, dk, dv, cache.state, ctx, decay_bias=self.decay_bias,
+                                tau=self.tau)
         z = ops.gated_heads(o, proj[:, g_at:g_at + H * dv], H, dv, kind=ops.GATE_SILU, weight=self.norm,
                             eps=self.norm_eps, out_dtype=ctx.dtype)
         return ops.gemm(z, self.o_proj)

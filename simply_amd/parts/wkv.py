@@ -16,6 +16,7 @@ import torch
 from ..kernels import ops
 from ..registry import MIXERS
 from .base import Mixer, ParamSpec, StateNeed, as_product_weight
+from .linear_state import channel_decay_state
 
 
 @MIXERS.register("wkv")
@@ -65,8 +66,7 @@ class WKV(Mixer):
         else:
             proj, low = ops.gemm_sections(mixes[:, :4 * D], self.in_proj), ops.gemm(mixes[:, 4 * D:], self.decay_in)
         decay = ops.low_rank_decay(low, self.decay_out, self.decay_base)
-        o = ops.linear_state(proj, 0, C, 2 * C, 1.0, decay, False, H, d, d, False, cache.state, ctx.seq_meta, ctx.num_seqs,
-                             bonus=self.bonus)
+        o = channel_decay_state(proj, (0, C, 2 * C), 1.0, decay, H, d, d, cache.state, ctx, bonus=self.bonus)
         z = ops.gated_heads(o, proj[:, 3 * C:4 * C], H, d, kind=ops.GATE_SILU, weight=self.norm, eps=self.norm_eps,
                             out_dtype=ctx.dtype)
         return ops.gemm(z, self.o_proj)

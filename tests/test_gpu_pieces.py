@@ -73,3 +73,68 @@ def test_delta_rule(H, G, dk, dv, kind):
         err, base, top = ((x.double().cpu() - ref).abs().max() for x in (got, plain, torch.zeros_like(got)))
         print(kind, float(err / top), float(base / top))
         assert err <= 3 * base and err <= 1e-5 * top, (float(err), float(base), float(top))
+
+
+def linear_64(p, at, q_mult, decay, bonus, state, meta, H, dk, dv):
+    out, state = torch.zeros(len(p), H, dv, dtype=torch.float64), state.double().clone()
+    q, k, v = (p[:, a:a + H * d].double().reshape(-1, H, d) for a, d in zip(at, (dk, dk, dv)))
+    a = decay.double().reshape(-1, H, dk)
+    for slot, first, count, _ in meta:
+        S = state[slot, :H * dk * dv].reshape(H, dv, dk).transpose(1, 2).clone()
+        for t in range(first, first + count):
+            kv = k[t][:, :, None] * v[t][:, None, :]
+            behind = a[t][:, :, None] * S + kv
+            read = behind if bonus is None else S + bonus.double().reshape(H, dk, 1) * kv
+            out[t], S = (q[t][:, :, None] * q_mult * read).sum(1), behind
+        state[slot, :H * dk * dv] = S.transpose(1, 2).reshape(-1)
+    return out.reshape(len(p), H * dv), state
+
+
+@pytest.mark.parametrize("H,dk,dv,kind,bonus", [(2, 128, 128, "slow", True), (4, 64, 64, "fast", False), (3, 20, 24, "ends", True),
+                                                (2, 100, 130, "spread", False), (1, 4, 3, "fast", True),
+                                                (2, 128, 40, "spread", True)])
+def test_channel_decays(H, dk, dv, kind, bonus):
+    """As above: within three times the error of the kernel that goes token by token, and below 1e-5 of the largest result."""
+    from simply_amd.kernels import ops
+
+    counts, before = [1, 15, 64, 65, 130, 200], 3
+    T = before + sum(counts)
+    meta, row = [], before
+    for i, n in enumerate(counts):
+        meta.append((5 - i if i else 6, row, n, 0))
+        row += n
+    at = (4, 4 + H * dk + 8, 13 + 2 * H * dk)
+    proj = normal((T, at[2] + H * dv + -(at[2] + H * dv) % 4), 61).bfloat16()
+    decay = {"slow": 1.0 - 0.01 * uniform((T, H * dk), 62), "fast": uniform((T, H * dk), 62),
+             "spread": torch.exp(-torch.exp(uniform((T, H * dk), 62, -8.0, 4.0))),
+             "ends": torch.randint(0, 2, (T, H * dk), generator=torch.Generator().manual_seed(62)).float()}[kind]
+    u = normal((H * dk,), 63) if bonus else None
+    q_mult = 1.0 if bonus else dk ** -0.5
+    state = torch.cat([normal((7, H * dk * dv), 64), torch.zeros(7, 4 + -(H * dk * dv) % 4)], 1)
+    want, want_state = linear_64(proj, at, q_mult, decay, u, state, meta, H, dk, dv)
+    dev_meta, dev_u = torch.tensor(meta, dtype=torch.int32).cuda(), u.cuda() if bonus else None
+    s1, s2, p, g = state.cuda(), state.cuda(), proj.cuda(), decay.cuda()
+    one = ops.linear_state(p, *at, q_mult, g, False, H, dk, dv, False, s1, dev_meta, len(meta), bonus=dev_u)
+    out = torch.zeros(T, H * dv, device="cuda")
+    assert ops.linear_chunks_takes(p, at[0], at[1], g, s2, len(meta), H, dk, dv)
+    ops.linear_chunks(p, *at, q_mult, g, H, dk, dv, s2, dev_meta, len(meta), before, max(counts), bonus=dev_u, out=out)
+    assert not out[:before].any()
+    for got, ref, plain in ((out[before:], want[before:], one[before:]), (s2, want_state, s1)):
+        err, base, top = ((x.double().cpu() - ref).abs().max() for x in (got, plain, torch.zeros_like(got)))
+        print(kind, float(err / top), float(base / top))
+        assert err <= 3 * base and err <= 1e-5 * top, (float(err), float(base), float(top))
+
+
+def test_decays_from_their_logits():
+    """a = sigmoid(z + bias)^(1 / tau) is computed as the token-by-token kernel does it: results agree to 32-bit rounding."""
+    from simply_amd.kernels import ops
+
+    H, dk, dv, T = 2, 64, 32, 150
+    proj, z = normal((T, 2 * H * dk + H * dv), 71).bfloat16().cuda(), normal((T, H * dk), 72).cuda()
+    bias, meta = normal((H * dk,), 73).bfloat16().cuda(), torch.tensor([[0, 0, T, 0]], dtype=torch.int32).cuda()
+    at, kw = (0, H * dk, 2 * H * dk), dict(decay_bias=bias, tau=16.0)
+    s1, s2 = torch.zeros(1, H * dk * dv).cuda(), torch.zeros(1, H * dk * dv).cuda()
+    want = ops.linear_state(proj, *at, 0.125, z, False, H, dk, dv, False, s1, meta, 1, **kw)
+    got = ops.linear_chunks(proj, *at, 0.125, z, H, dk, dv, s2, meta, 1, 0, T, out=torch.zeros_like(want), **kw)
+    for x, y in ((got, want), (s2, s1)):
+        assert (x - y).abs().max() <= 1e-5 * y.abs().max()

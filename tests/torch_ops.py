@@ -22,7 +22,8 @@ STAND_INS = ("embed", "rmsnorm", "add_rmsnorm", "rope_cache_write", "rope", "gat
              "paged_attention_maps", "attention_maps_units_takes", "norm_rope_cache_write", "short_conv",
              "head_product", "rglru_scan", "attention_inputs", "route_choice", "token_shift", "low_rank_decay",
              "concat_rows", "gemm_sections", "streams", "ssm_inputs", "gated_group_norm",
-             "state_chunks_takes", "state_chunks", "attention_f32_takes", "delta_chunks_takes", "delta_chunks")
+             "state_chunks_takes", "state_chunks", "attention_f32_takes", "delta_chunks_takes", "delta_chunks",
+             "linear_chunks_takes", "linear_chunks")
 
 EPILOGUE_NONE, EPILOGUE_GATED_GELU, EPILOGUE_SOFT_CAP = 0, 1, 2
 ALGO_AUTO, ALGO_GENERIC, ALGO_SKINNY, ALGO_TILED = 0, 1, 2, 3
@@ -608,6 +609,17 @@ def linear_state(proj, q_at, k_at, v_at, q_mult, gates, scalar, num_heads, key_d
             if into is not None:
                 into[first:first + count] = out[first:first + count].to(torch.float32)
     return out.to(torch.float32) if into is None else into
+
+
+def linear_chunks_takes(proj, q_at, k_at, gates, state, num_seqs, num_heads, key_dim, value_dim):
+    return True
+
+
+def linear_chunks(proj, q_at, k_at, v_at, q_mult, gates, num_heads, key_dim, value_dim, state, seq_meta, num_seqs, first_row,
+                  max_q_len, *, decay_bias=None, tau=None, bonus=None, out):
+    assert num_seqs > 0 and int(seq_meta[0, 1]) == first_row and int(seq_meta[:num_seqs, 2].sum()) == len(proj) - first_row
+    return linear_state(proj, q_at, k_at, v_at, q_mult, gates, False, num_heads, key_dim, value_dim, False, state, seq_meta,
+                        num_seqs, decay_bias=decay_bias, tau=tau, bonus=bonus, out=out)
 
 
 def state_chunks_takes(proj, q_at, k_at, v_at, key_dim, value_dim, state):
