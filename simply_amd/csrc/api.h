@@ -261,6 +261,12 @@ bool gemm_skinny_takes(int M, int N, int K, int64_t lda, const void* A, const vo
 double gemm_skinny_predict_us(int M, int N, int K, int epi);
 double gemm_tiled_predict_us(int M, int N, int K, int epi);
 double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes);
+// The experts' products on the wide kernel (plan, sorted: of the sort kernel with tiles of tile_rows rows, 64 or 128).
+bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t ldc, const void* A, const void* W, const void* W2,
+                            const void* C, int tile_rows);
+int gemm_wide_routed(const void* A, int64_t lda, const void* W, const void* W2, void* C, float* y, int64_t ldc, int tiles, int N,
+                     int K, int tile_rows, const int* plan, const int* sorted, int by_token, int top, int act, float limit,
+                     hipStream_t stream);
 int gemm_skinny(const void* A, int64_t lda, const void* W, const void* W2, void* C, int c_dtype, int64_t ldc, int M,
                 int N, int K, int epi, int act, float cap, int packed, int shape, hipStream_t stream, Sections sec = {});
 bool paged_attention_decode_takes(int H, int Kh, int hd, int page_size, int max_q_len, int64_t q_stride, const void* q);
@@ -573,9 +579,11 @@ int sa_route(const float* logits, int64_t stride, int T, int E, int top, float s
 int sa_route_choice(const float* logits, int64_t stride, int T, int E, int top, float scale, const void* bias,
                     int bias_dtype, const void* correction, int corr_dtype, int groups, int keep, int softmax, int group_best, float renorm, int* experts,
                     float* weights, hipStream_t stream);
-// The most tiles of tile_rows (16 or 64) rows of one expert that P pairs over E experts make.
+// The rows of a tile (16, 64 or 128) that suit P pairs over E experts, D -> F -> D, whose inputs' rows lie at a.
+int sa_expert_tile_rows(int P, int E, int D, int F, int dtype, int64_t a_stride, const void* a);
+// The most tiles of tile_rows rows of one expert that P pairs over E experts make.
 int sa_expert_tiles_max(int P, int E, int tile_rows);
-// sorted [P]: the pairs by expert; plan [1 + 2 * sa_expert_tiles_max(P, E, tile_rows)]: the tiles.
+// sorted [P]: the pairs by expert; plan [1 + 3 * sa_expert_tiles_max(P, E, tile_rows)]: the tiles.
 int sa_expert_sort(const int* experts, int P, int E, int tile_rows, int* sorted, int* plan, int plan_words,
                    hipStream_t stream);
 // w2 given: out[row] = act(a . w1[e]^T) * (a . w2[e]^T) in a's type (or another rule of activations.h, with its limit); else out[row] = a . w1[e]^T in 32-bit, or, with

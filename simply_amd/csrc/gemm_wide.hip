@@ -63,12 +63,23 @@ __device__ __forceinline__ void load_to_lds(const bf16* base, uint32_t offset, u
                : "memory");
 }
 
+// Products of routed experts (ROUTED): row tile blockIdx.y is tile y of the sort kernel's plan (from plan[1 + 3 y] on: its
+// expert, its first row in the sorted order, its rows), row m of it is row `sorted[first + m] / top` of A (by_token) or
+// row first + m; W holds the experts' weights one behind the other, and w2, with the gated epilogue, the other factor's.
+// EPI 0 and 1 write row first + m of C, EPI 4 the 32-bit product to row `sorted[first + m]` of `partials`.
+struct Routed {
+  const int* plan;
+  const int* sorted;
+  const bf16* w2;
+  int by_token, top;
+};
+
 // WM x WN: 16 x 16 tiles of a wave (rows of A x rows of W); WAVES_M x (WAVES / WAVES_M) waves.
-template <int WM, int WN, int WAVES_M, int EPI, int NSTAGE, int WAVES>
+template <int WM, int WN, int WAVES_M, int EPI, int NSTAGE, int WAVES, bool ROUTED = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __restrict__ A, int64_t lda,
                                                         const bf16* __restrict__ W, bf16* __restrict__ C, int64_t ldc,
                                                         int M, int N, int K, int chunks, int act, float limit,
-                                                        float* __restrict__ partials, Sections sec) {
+                                                        float* __restrict__ partials, Sections sec, Routed rt) {
   constexpr int WAVES_N = WAVES / WAVES_M;
   constexpr int MT = WAVES_M * WM, NT = WAVES_N * WN;  // 16-row tiles of A and of W per workgroup
   constexpr int BM = MT * 16;
@@ -87,7 +98,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
   // Which tile: workgroups go to the eight XCDs in turn, each with an L2 of its own; the numbering is turned round
   // so that an XCD gets a contiguous share of the tiles, and within it tiles go in columns eight wide, rows first.
   int bx = blockIdx.x, by = blockIdx.y;
-  {
+  int row_first = 0, tile_rows = M;   // (ROUTED: the tile's rows)
+  if (ROUTED) {
+    // (no turning round: how many tiles there are is known on the device only, and a tile's neighbours in x, which share
+    // its rows, go to the XCDs in turn, so that an XCD meets the same weights again in the expert's next tile)
+    if (by >= rt.plan[0]) return;
+    row_first = rt.plan[2 + 3 * by], tile_rows = rt.plan[3 + 3 * by];
+    const size_t expert = static_cast<size_t>(rt.plan[1 + 3 * by]) * ((N + 15) / 16) * chunks * 512;
+    W += expert;
+    if (EPI == 1) rt.w2 += expert;
+  } else {
     const int nx = gridDim.x, ny = gridDim.y, total = nx * ny;
     int l = bx + nx * by;
     if (total % 8 == 0) l = (l % 8) * (total / 8) + l / 8;
@@ -108,7 +128,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
   const int slab0 = static_cast<int>(static_cast<int64_t>(blockIdx.z) * slabs_all / gridDim.z);
   const int slabs = static_cast<int>(static_cast<int64_t>(blockIdx.z + 1) * slabs_all / gridDim.z) - slab0;
   A += static_cast<size_t>(slab0) * BK;
-  const int m_base = by * BM;
+  const int m_base = ROUTED ? 0 : by * BM;
   const int NW = EPI == 1 ? 2 * ((N + 15) / 16) * 16 : N;
   // several products at once: which section this workgroup is in, its columns of A, its rows of W
   int first_tile = 0, NL = NW;   // the section's first 16-row tile of W and the end of its rows
@@ -135,14 +155,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
   for (int i = 0; i < APW; ++i) {
     const int r = half_mine * 8 + lane / 8;  // row of the tile
     const int m = m_base + (tile_mine + (WAVES / 2) * i) * 16 + r;
-    a_off[i] = (static_cast<uint32_t>(m < M ? m : M - 1) * static_cast<uint32_t>(lda) + ((lane % 8) ^ (r / 2)) * 8) * 2;
+    int from = m < tile_rows ? m : tile_rows - 1;
+    if (ROUTED) from = rt.by_token ? rt.sorted[row_first + from] / rt.top : row_first + from;
+    a_off[i] = (static_cast<uint32_t>(from) * static_cast<uint32_t>(lda) + ((lane % 8) ^ (r / 2)) * 8) * 2;
   }
   const bf16* w_from[WPW];  // the same for the whole wave
 #pragma unroll
   for (int i = 0; i < WPW; ++i) {
     const int nt = nt_base + tile_mine + (WAVES / 2) * i;
     const int clamped = __builtin_amdgcn_readfirstlane(nt < ntiles ? nt : ntiles - 1);
-    w_from[i] = W + (static_cast<size_t>(clamped) * chunks + half_mine) * 512 + static_cast<size_t>(slab0) * 1024;
+    // (routed gated products: the two factors' tiles alternate here, but lie in weights of their own)
+    const bf16* from = ROUTED && EPI == 1 && clamped % 2 ? rt.w2 : W;
+    const int at = ROUTED && EPI == 1 ? clamped / 2 : clamped;
+    w_from[i] = from + (static_cast<size_t>(at) * chunks + half_mine) * 512 + static_cast<size_t>(slab0) * 1024;
   }
   // load n (of LOADS) of slab `slab` into buffer `buf`
   constexpr int LOADS = APW + WPW;
@@ -272,7 +297,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
     const int m = m_base + (wm * WM + i) * 16 + row;
-    if (m >= M) continue;
+    if (m >= tile_rows) continue;
+    if (EPI == 4) {
+      float* y_row = partials + static_cast<size_t>(rt.sorted[row_first + m]) * ldc;
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        const int n = (nt_base + wn * WN + j) * 16 + quad * 4;
+        if (n < NL) *reinterpret_cast<floatx4*>(y_row + n) = acc[i][j];
+      }
+      continue;
+    }
     if (EPI == 3) {  // this workgroup's share of the sum, as it is
       float* p_row = partials + (static_cast<size_t>(blockIdx.z) * M + m) * N;
 #pragma unroll
@@ -282,7 +316,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
       }
       continue;
     }
-    bf16* c_row = C + static_cast<size_t>(m) * ldc;
+    bf16* c_row = C + static_cast<size_t>(row_first + m) * ldc;
     constexpr int OUT = EPI == 1 ? WN / 2 : WN;
 #pragma unroll
     for (int j = 0; j < OUT; ++j) {
@@ -317,16 +351,61 @@ static void launch(const bf16* A, int64_t lda, const bf16* W, bf16* C, int64_t l
   const dim3 grid(whole * ((sec.n_step + BNW - 1) / BNW) + (NW - whole * sec.n_step + BNW - 1) / BNW, (M + BM - 1) / BM, ks);
   if (epi == 1)
     gemm_wide_kernel<WM, WN, WAVES_M, 1, NSTAGE, WAVES><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32,
-                                                                                         act, limit, nullptr, sec);
+                                                                                         act, limit, nullptr, sec, Routed{});
   else if (raw)
     gemm_wide_kernel<WM, WN, WAVES_M, 3, NSTAGE, WAVES><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32,
-                                                                                         act, limit, partials, sec);
+                                                                                         act, limit, partials, sec, Routed{});
   else
     gemm_wide_kernel<WM, WN, WAVES_M, 0, NSTAGE, WAVES><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32,
-                                                                                         act, limit, nullptr, sec);
+                                                                                         act, limit, nullptr, sec, Routed{});
+}
+
+template <int WM, int WN, int WAVES_M, int NSTAGE, int WAVES>
+static void launch_routed(const bf16* A, int64_t lda, const bf16* W, const Routed& rt, bf16* C, float* y, int64_t ldc, int tiles,
+                          int rows, int N, int K, int act, float limit, hipStream_t stream) {
+  constexpr int BNW = (WAVES / WAVES_M) * WN * 16;
+  const int NW = rt.w2 != nullptr ? 2 * ((N + 15) / 16) * 16 : N;
+  const dim3 grid((NW + BNW - 1) / BNW, tiles);
+  if (rt.w2 != nullptr)
+    gemm_wide_kernel<WM, WN, WAVES_M, 1, NSTAGE, WAVES, true><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, rows, N, K, K / 32,
+                                                                                               act, limit, nullptr, Sections{}, rt);
+  else if (y != nullptr)
+    gemm_wide_kernel<WM, WN, WAVES_M, 4, NSTAGE, WAVES, true><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, rows, N, K, K / 32,
+                                                                                               0, 0.f, y, Sections{}, rt);
+  else
+    gemm_wide_kernel<WM, WN, WAVES_M, 0, NSTAGE, WAVES, true><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, rows, N, K, K / 32,
+                                                                                               act, limit, nullptr, Sections{}, rt);
 }
 
 }  // namespace wide
+
+// Products of routed experts on this kernel's tiles: 64 rows of an expert x 128 weight rows with three buffers, or 128 x 192
+// with two (tile_rows); workgroups of four waves, two a CU.  Gate and up together with down of 16 experts, in microseconds:
+//   2,048 x 2,048, rows an expert   16: 72   32: 75   96: 103 / 94   128: 117 / 148   256: 184 / 199   512: 332 / 339 (64 / 128)
+//   4,096 x 3,584                   16: 271  32: 270  96: 352 / 342  128: 420 / 396   256: 636 / 586   512: 1,107 / 1,035
+// (the kernel of routed.hip for 64 rows, which took these products before: 327 at 256 rows of 2,048 x 2,048).  Also tried for
+// 64 rows: eight waves with six buffers (212 at 256 rows), 64 x 256 (199), four waves across (184).
+bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t ldc, const void* A, const void* W, const void* W2,
+                            const void* C, int tile_rows) {
+  auto aligned = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
+  return (tile_rows == 64 || tile_rows == 128) && K % wide::BK == 0 && N % 4 == 0 && lda % 8 == 0 && ldc % 4 == 0 && aligned(A, 16) &&
+         aligned(W, 16) && aligned(W2, 16) && aligned(C, 16) && a_rows * lda < (int64_t{1} << 31);
+}
+
+// act: the gated rule, or with one weight and a bfloat16 result 1 + the activation.  y (and no C): the 32-bit product, a row
+// per pair.
+int gemm_wide_routed(const void* A, int64_t lda, const void* W, const void* W2, void* C, float* y, int64_t ldc, int tiles, int N,
+                     int K, int tile_rows, const int* plan, const int* sorted, int by_token, int top, int act, float limit,
+                     hipStream_t stream) {
+  wide::Routed rt;
+  rt.plan = plan, rt.sorted = sorted, rt.w2 = static_cast<const bf16*>(W2), rt.by_token = by_token, rt.top = top;
+  const bf16* a = static_cast<const bf16*>(A);
+  const bf16* w = static_cast<const bf16*>(W);
+  bf16* c = static_cast<bf16*>(C);
+  if (tile_rows == 128) wide::launch_routed<4, 6, 2, 2, 4>(a, lda, w, rt, c, y, ldc, tiles, tile_rows, N, K, act, limit, stream);
+  else wide::launch_routed<2, 4, 2, 3, 4>(a, lda, w, rt, c, y, ldc, tiles, tile_rows, N, K, act, limit, stream);
+  return check_launch("gemm_wide_routed");
+}
 
 bool gemm_wide_takes(int M, int N, int K, int64_t lda, int64_t ldc, const void* A, const void* W, const void* W2,
                      const void* C, int c_dtype, int epi, int packed) {

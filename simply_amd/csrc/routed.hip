@@ -16,7 +16,8 @@
 namespace sa {
 
 constexpr int kRouteSlots = 8;    // experts per lane: up to 512 experts
-constexpr int kTileRowsMax = 64;  // rows of a tile: 16 (one MFMA operand) or 64 (four, which share the weights' operands)
+constexpr int kTileRowsMax = 64;  // rows of a tile: 16 (one MFMA operand) or 64 (four, which share the weights' operands),
+constexpr int kTileRowsWide = 128;   // or 128, for the wide product kernel alone
 
 // A wave per token.  scores = softmax(logits); `top` times the largest score that is left (of equal ones the lowest
 // index); weight = score * scale.
@@ -184,8 +185,8 @@ __global__ __launch_bounds__(kWave) void route_choice_kernel(const float* __rest
   for (int r = lane; r < top; r += kWave) weights[static_cast<size_t>(t) * top + r] = choice_s[r] / by * scale;
 }
 
-// One workgroup.  plan: [0] number of tiles; [1 .. 1 + 2 * max_tiles): per tile its expert and its first row in the
-// sorted order with the number of its rows packed as first * 128 + rows.  sorted [P]: pair indices by expert.
+// One workgroup.  plan: [0] number of tiles; [1 .. 1 + 3 * max_tiles): per tile its expert, its first row in the sorted order
+// and the number of its rows.  sorted [P]: pair indices by expert.
 __global__ __launch_bounds__(1024) void sort_kernel(const int* __restrict__ experts, int P, int E,
                                                     int* __restrict__ sorted, int* __restrict__ plan, int max_tiles,
                                                     int kTileRows) {
@@ -217,8 +218,9 @@ __global__ __launch_bounds__(1024) void sort_kernel(const int* __restrict__ expe
       const int n = tiles[e] + i;
       if (n >= max_tiles) break;
       const int rows = counts[e] - i * kTileRows < kTileRows ? counts[e] - i * kTileRows : kTileRows;
-      plan[1 + 2 * n] = e;
-      plan[2 + 2 * n] = (offsets[e] + i * kTileRows) * 128 + rows;
+      plan[1 + 3 * n] = e;
+      plan[2 + 3 * n] = offsets[e] + i * kTileRows;
+      plan[3 + 3 * n] = rows;
     }
   }
   __syncthreads();
@@ -247,8 +249,7 @@ __global__ __launch_bounds__(256) void expert_product_kernel(
   // activate (without a second weight): out[row] = act(a . w1[e]^T) in a's type instead of the 32-bit product
   const int tile = blockIdx.x;
   if (tile >= plan[0]) return;
-  const int e = plan[1 + 2 * tile], packed = plan[2 + 2 * tile];
-  const int row0 = packed / 128, rows = packed % 128;
+  const int e = plan[1 + 3 * tile], row0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int n0 = (blockIdx.y * 4 + wave) * 16;
   if (n0 >= N) return;
@@ -370,8 +371,7 @@ __global__ __launch_bounds__(256) void expert_product_rows64_kernel(
   __shared__ int pair_of[kTileRowsMax];
   const int tile = blockIdx.x;
   if (tile >= plan[0]) return;
-  const int e = plan[1 + 2 * tile], packed = plan[2 + 2 * tile];
-  const int row0 = packed / 128, rows = packed % 128;
+  const int e = plan[1 + 3 * tile], row0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int r = lane % 16, kq = lane / 16;
   const int n0 = (blockIdx.y * 4 + wave) * 32;
@@ -526,13 +526,28 @@ extern "C" int sa_expert_tiles_max(int P, int E, int tile_rows) {
   return (P + tile_rows - 1) / tile_rows + (E < P ? E : P);
 }
 
+extern "C" int sa_expert_tile_rows(int P, int E, int D, int F, int dtype, int64_t a_stride, const void* a) {
+  alignas(16) static const char aligned_stand_in[16] = {};   // (weights and results are whole tensors)
+  const void* p = aligned_stand_in;
+  const bool wide = dtype == kBF16 && gemm_wide_routed_takes(F, D, a_stride, P, F, a, p, p, p, kTileRowsWide) &&
+                    gemm_wide_routed_takes(D, F, F, P, D, p, p, nullptr, p, kTileRowsWide);
+  // Rows that an expert gets on average: from 12 on some need a second tile of 16, which reads the weights again (2,048 x
+  // 2,048, 16 experts: 8 rows 63 us with tiles of 16 and 72 with the wide kernel's 64; 16 rows 105 and 72); the kernel of 64
+  // rows here is ahead from 32 on.
+  if (P < (wide ? 12 : 32) * static_cast<int64_t>(E)) return 16;
+  // Tiles of 128 rows where they fill up and an expert's gate and up are more than the L2s hold (4 MiB an XCD), so that every
+  // tile of rows fetches them again (figures: gemm_wide_routed).
+  return wide && P >= 96 * static_cast<int64_t>(E) && 4.0 * D * F > 32.0 * (1 << 20) ? kTileRowsWide : kTileRowsMax;
+}
+
 extern "C" int sa_expert_sort(const int* experts, int P, int E, int tile_rows, int* sorted, int* plan, int plan_words,
                               hipStream_t stream) {
   if (P == 0) return 0;
-  SA_REQUIRE(tile_rows == 16 || tile_rows == kTileRowsMax, "expert_sort: tiles of 16 or %d rows", kTileRowsMax);
+  SA_REQUIRE(tile_rows == 16 || tile_rows == kTileRowsMax || tile_rows == kTileRowsWide, "expert_sort: tiles of 16, %d or %d rows",
+             kTileRowsMax, kTileRowsWide);
   const int max_tiles = sa_expert_tiles_max(P, E, tile_rows);
   SA_REQUIRE(P > 0 && E > 0 && E <= 4096 && P < (1 << 26), "expert_sort: bad sizes P=%d E=%d", P, E);
-  SA_REQUIRE(plan_words >= 1 + 2 * max_tiles, "expert_sort: the plan needs %d words", 1 + 2 * max_tiles);
+  SA_REQUIRE(plan_words >= 1 + 3 * max_tiles, "expert_sort: the plan needs %d words", 1 + 3 * max_tiles);
   SA_REQUIRE(experts != nullptr && sorted != nullptr && plan != nullptr, "expert_sort: a null pointer");
   const int threads = P >= 1024 ? 1024 : ((P + kWave - 1) / kWave) * kWave;
   sort_kernel<<<1, threads, (4 * E + 2) * sizeof(int), stream>>>(experts, P, E, sorted, plan, max_tiles, tile_rows);
@@ -552,7 +567,8 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
   SA_REQUIRE(act >= 0 && act < (w2 != nullptr ? kNumGatedRules : kNumActivations), "expert_product: unknown activation %d", act);
   SA_REQUIRE(act != kActClampedGlu || limit > 0.f, "expert_product: the clamped gated product needs a positive limit");
   SA_REQUIRE(dtype == kF32 || dtype == kBF16, "expert_product: unknown dtype %d", dtype);
-  SA_REQUIRE(tile_rows == 16 || tile_rows == kTileRowsMax, "expert_product: tiles of 16 or %d rows", kTileRowsMax);
+  SA_REQUIRE(tile_rows == 16 || tile_rows == kTileRowsMax || tile_rows == kTileRowsWide,
+             "expert_product: tiles of 16, %d or %d rows", kTileRowsMax, kTileRowsWide);
   const dim3 grid(sa_expert_tiles_max(P, E, tile_rows), (N + 63) / 64);
   SA_REQUIRE(grid.y <= 65535, "expert_product: too many columns");
   const bool gated = w2 != nullptr;
@@ -561,6 +577,15 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
                                                              static_cast<const T*>(w1), static_cast<const T*>(w2), N,  \
                                                              K, sorted, plan, act, limit, out, out_stride, out_by_pair, \
                                                              activate)
+  // Tiles of 64 and 128 rows go to the wide product kernel where it takes the operands; the others to the kernel of 64 rows here.
+  const bool by_wide = dtype == kBF16 && tile_rows != 16 && ((gated || activate) ? !out_by_pair : out_by_pair != 0) &&
+                       gemm_wide_routed_takes(N, K, a_stride, a_by_token ? (P + top - 1) / top : P, out_stride, a, w1, w2, out, tile_rows);
+  SA_REQUIRE(by_wide || tile_rows != kTileRowsWide, "expert_product: tiles of %d rows need aligned bfloat16 operands, K in multiples of 64",
+             kTileRowsWide);
+  if (by_wide)
+    return gemm_wide_routed(a, a_stride, w1, w2, gated || activate ? out : nullptr,
+                            gated || activate ? nullptr : static_cast<float*>(out), out_stride, grid.x, N, K, tile_rows, plan, sorted,
+                            a_by_token, top, gated ? act : activate ? act + 1 : 0, limit, stream);
   if (dtype == kBF16) {
     if (tile_rows == 16) {
       if (gated) SA_EXPERT(bf16, true, 1);

@@ -1975,11 +1975,11 @@ def routed_experts(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor
     limit = _gate_limit(activation, limit)
     P = T * top
     dev = x.device
-    # tiles of 64 rows share the weights' operands between four sub-tiles: for steps that bring an expert many rows
-    tile_rows = 64 if P >= 32 * E else 16
+    # tiles of 64 or 128 rows share the weights' operands between their rows: for steps that bring an expert many
+    tile_rows = _lib.load().sa_expert_tile_rows(P, E, D, F, _code(x), _rows(x, "routed_experts: x"), _ptr(x))
     max_tiles = _lib.load().sa_expert_tiles_max(P, E, tile_rows)
     sorted_ = torch.empty(P, dtype=torch.int32, device=dev)
-    plan = torch.empty(1 + 2 * max_tiles, dtype=torch.int32, device=dev)
+    plan = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=dev)
     _lib.call("sa_expert_sort", _ptr(experts), P, E, tile_rows, _ptr(sorted_), _ptr(plan), plan.numel(), _stream())
     h = torch.empty((P, F), dtype=x.dtype, device=dev)
     first, second = (gate_w.data, up_w.data) if gate_w is not None else (up_w.data, None)
