@@ -237,22 +237,22 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 __device__ __forceinline__ bf16x8 load8(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
 // h[row, f] = act(x[token] . Wg[e, f]) * (x[token] . Wu[e, f]); GATED false: y[pair, n] = h[row] . Wd[e, n].
-// A workgroup of four waves takes one tile of rows and 64 columns (a wave 16 of them, for all RT sub-tiles of 16 rows).
+// A workgroup of one wave takes one tile of rows and 16 columns (for all RT sub-tiles of 16 rows): nothing is shared between
+// waves, and small workgroups even out over the CUs, of which the few experts that a decode step reads would give some two or
+// three workgroups of four waves and others none.
 // bfloat16: the weights are tiled ([E][N / 16][K / 32][64][8], see the product kernels), a wave's operands are one
 // 16-byte load a lane (rows that are not 16-byte aligned are read element by element); 32-bit: row-major weights
 // [E][N][K], a lane per (row, column) of the tile in turn.
 template <typename T, bool GATED, int RT>
-__global__ __launch_bounds__(256) void expert_product_kernel(
+__global__ __launch_bounds__(kWave) void expert_product_kernel(
     const T* __restrict__ a, int64_t a_stride, int a_by_token, int top, const T* __restrict__ w1, const T* __restrict__ w2,
     int N, int K, const int* __restrict__ sorted, const int* __restrict__ plan, int act, float limit,
     void* __restrict__ out, int64_t out_stride, int out_by_pair, int activate) {
   // activate (without a second weight): out[row] = act(a . w1[e]^T) in a's type instead of the 32-bit product
-  const int tile = blockIdx.x;
+  const int tile = blockIdx.y;
   if (tile >= plan[0]) return;
   const int e = plan[1 + 3 * tile], row0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int n0 = (blockIdx.y * 4 + wave) * 16;
-  if (n0 >= N) return;
+  const int lane = threadIdx.x, n0 = blockIdx.x * 16;
   if constexpr (sizeof(T) == 2) {
     const int Nt = (N + 15) / 16, Kt = (K + 31) / 32;
     const int r = lane % 16, kq = lane / 16;
@@ -271,25 +271,45 @@ __global__ __launch_bounds__(256) void expert_product_kernel(
     floatx4 accg[RT], accu[RT];
 #pragma unroll
     for (int s = 0; s < RT; ++s) accg[s] = accu[s] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // Whole k tiles of aligned rows, four at a time: their loads are all asked for before the first product (few
-    // waves run on a SIMD here, so a wave covers its own waits), the products in the order of k.
+    // Whole k tiles of aligned rows: two sets of four, so that one set's loads are under way while the other is multiplied.
+    // Loads behind the last tile ask for it again; the products go in the order of k.  (Weights of 16 experts of 2,048 x 2,048
+    // from HBM, top 2, gate and up + down: 8 tokens 43.3 + 26.8 us with one set and workgroups of four waves, 37.0 + 22.8 with
+    // one set, 45.1 + 26.9 with two sets, 33.7 + 18.0 with two sets and one wave, 5.1 TB/s; 1 token 17.6 + 11.5 and 9.4 + 7.6;
+    // 64 tokens 50.5 + 29.3 and 52.8 + 29.7.  Sets of eight: 34.1 + 18.4.)
     int kt = 0;
     if (aligned && RT == 1) {
       const bf16* src = reinterpret_cast<const bf16*>(arow[0]) + kq * 8;
       constexpr int kAhead = 4;
-      for (; kt + kAhead <= K / 32; kt += kAhead) {
-        bf16x8 gv[kAhead], uv[kAhead], av[kAhead];
+      const int whole = K / 32;
+      bf16x8 gv[2][kAhead], uv[2][kAhead], av[2][kAhead];
+      auto load = [&](int set, int from) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kAhead; ++i) {
-          gv[i] = load8(g + static_cast<size_t>(kt + i) * 512);
-          if constexpr (GATED) uv[i] = load8(u + static_cast<size_t>(kt + i) * 512);
-          av[i] = load8(src + (kt + i) * 32);
+          const int at = from + i < whole ? from + i : whole - 1;
+          gv[set][i] = load8(g + static_cast<size_t>(at) * 512);
+          if constexpr (GATED) uv[set][i] = load8(u + static_cast<size_t>(at) * 512);
+          av[set][i] = load8(src + at * 32);
+        }
+      };
+      auto multiply = [&](int set, int i) __attribute__((always_inline)) {
+        accg[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gv[set][i], av[set][i], accg[0], 0, 0, 0);
+        if constexpr (GATED) accu[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(uv[set][i], av[set][i], accu[0], 0, 0, 0);
+      };
+      if (whole > 0) {
+        load(0, 0);
+        load(1, kAhead);
+        for (; kt + 2 * kAhead <= whole; kt += 2 * kAhead) {
+#pragma unroll
+          for (int set = 0; set < 2; ++set) {
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) multiply(set, i);
+            load(set, kt + (2 + set) * kAhead);
+          }
         }
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-          accg[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gv[i], av[i], accg[0], 0, 0, 0);
-          if constexpr (GATED) accu[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(uv[i], av[i], accu[0], 0, 0, 0);
-        }
+        for (int i = 0; i < 2 * kAhead; ++i)
+          if (kt + i < whole) multiply(i / kAhead, i % kAhead);   // (uniform)
+        kt = whole;
       }
     }
     for (; kt < Kt; ++kt) {
@@ -569,11 +589,11 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
   SA_REQUIRE(dtype == kF32 || dtype == kBF16, "expert_product: unknown dtype %d", dtype);
   SA_REQUIRE(tile_rows == 16 || tile_rows == kTileRowsMax || tile_rows == kTileRowsWide,
              "expert_product: tiles of 16, %d or %d rows", kTileRowsMax, kTileRowsWide);
-  const dim3 grid(sa_expert_tiles_max(P, E, tile_rows), (N + 63) / 64);
-  SA_REQUIRE(grid.y <= 65535, "expert_product: too many columns");
+  const int tiles = sa_expert_tiles_max(P, E, tile_rows);
+  SA_REQUIRE(tiles <= 65535, "expert_product: too many tiles");
   const bool gated = w2 != nullptr;
 #define SA_EXPERT(T, G, RT)                                                                                            \
-  expert_product_kernel<T, G, RT><<<grid, 256, 0, stream>>>(static_cast<const T*>(a), a_stride, a_by_token, top,        \
+  expert_product_kernel<T, G, RT><<<dim3((N + 15) / 16, tiles), kWave, 0, stream>>>(static_cast<const T*>(a), a_stride, a_by_token, top,        \
                                                              static_cast<const T*>(w1), static_cast<const T*>(w2), N,  \
                                                              K, sorted, plan, act, limit, out, out_stride, out_by_pair, \
                                                              activate)
@@ -584,14 +604,14 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
              kTileRowsWide);
   if (by_wide)
     return gemm_wide_routed(a, a_stride, w1, w2, gated || activate ? out : nullptr,
-                            gated || activate ? nullptr : static_cast<float*>(out), out_stride, grid.x, N, K, tile_rows, plan, sorted,
+                            gated || activate ? nullptr : static_cast<float*>(out), out_stride, tiles, N, K, tile_rows, plan, sorted,
                             a_by_token, top, gated ? act : activate ? act + 1 : 0, limit, stream);
   if (dtype == kBF16) {
     if (tile_rows == 16) {
       if (gated) SA_EXPERT(bf16, true, 1);
       else SA_EXPERT(bf16, false, 1);
     } else {
-      const dim3 wide(grid.x, (N + 127) / 128);
+      const dim3 wide(tiles, (N + 127) / 128);
       if (gated)
         expert_product_rows64_kernel<true><<<wide, 256, 0, stream>>>(
             static_cast<const bf16*>(a), a_stride, a_by_token, top, static_cast<const bf16*>(w1),
