@@ -38,3 +38,29 @@ def test_sum_and_norms(D, dtype):
         want = h.double() + 0.7 * y.double() / (y.double().square().mean(1, keepdim=True) + 1e-5).sqrt() * w.double()
         assert ((got_h.double() - want).abs() <= (D / 256 + 20) * 2.0 ** -24 * 25).all()
         assert ((out.double() - want).abs() <= (step + (D / 256 + 20) * 2.0 ** -24) * 30).all()
+
+
+@pytest.mark.parametrize("H,I,O,tail,gates", [(3, 128, 512, 64, None), (2, 512, 128, 0, "outputs"), (4, 32, 20, 4, "heads"),
+                                              (2, 96, 68, 0, "outputs"), (1, 192, 16, 32, None), (2, 40, 36, 0, None)])
+def test_head_products(H, I, O, tail, gates):
+    """Tokens around the tiles of 16 and 64, heads apart from each other (the last case: inputs that the matrix cores do not
+    take).  Sums of I bfloat16 products in 32 bits, rounded once; and a token's result does not depend on the others."""
+    from simply_amd.kernels import ops
+
+    w = draw((H, O, I), 1, torch.bfloat16)
+    for T in (1, 16, 17, 64, 65, 150):
+        x = draw((T, H * (I + tail + 8) + 16), 2, torch.bfloat16)[:, 8:]
+        gate = None if gates is None else draw((T, (H if gates == "heads" else H * O) + 8), 3, torch.bfloat16)[:, 8:]
+        got = ops.head_product(x, w, in_stride=I + tail + 8, tail=tail, gate=gate)
+        rows = torch.stack([x[:, h * (I + tail + 8):h * (I + tail + 8) + I + tail] for h in range(H)], 1).double()
+        want = torch.einsum("thi,hoi->tho", rows[:, :, :I], w.double())
+        size = torch.einsum("thi,hoi->tho", rows[:, :, :I].abs(), w.double().abs())
+        if gates is not None:
+            g = torch.sigmoid(gate.double()).reshape(T, H, -1)
+            want, size = want * g, size * g
+        got = got.double().reshape(T, H, O + tail)
+        assert ((got[:, :, :O] - want).abs() <= 2.0 ** -8 * want.abs() + (I + 8) * 2.0 ** -24 * size).all(), T
+        assert torch.equal(got[:, :, O:], rows[:, :, I:])
+        if T > 1 and I % 32 == 0:
+            alone = ops.head_product(x[T - 1:], w, in_stride=I + tail + 8, tail=tail, gate=None if gate is None else gate[T - 1:])
+            assert torch.equal(alone.double().reshape(H, -1), got[T - 1])
