@@ -339,6 +339,17 @@ int sa_paged_attention_maps_units(const void* q, int64_t q_stride, const void* k
                                   float eps, float mult, int max_kv_len, int max_q_len, void* workspace,
                                   size_t workspace_bytes, hipStream_t stream);
 
+// The same with one map for units in groups of one request each, whose rows share the keys in LDS
+// (csrc/attention_groups.hip).
+int sa_paged_attention_groups_size();
+int sa_paged_attention_groups_takes(int H, int Kh, int hd, int hd_v, int page_size, int64_t q_stride, const void* q);
+int sa_paged_attention_groups_pays(int unit_count, int H, int Kh, int window, int max_kv_len, int max_q_len);
+int sa_paged_attention_groups(const void* q, int64_t q_stride, const void* k_pages, const void* v_pages,
+                              const int* block_table, int table_stride, const int* units, int unit_begin, int unit_count,
+                              void* out, int64_t out_stride, int H, int Kh, int hd, int hd_v, int page_size, int window,
+                              float scale, int max_kv_len, int max_q_len, void* workspace, size_t workspace_bytes,
+                              hipStream_t stream);
+
 // residual += mult * norm(y; w) (w null: + mult * y; y null: nothing is added), then, if out is not null, out = the
 // residual in out's type: the sum of a block that norms what a part returns, and the hand-over to a next part that
 // has no norm in front of it.  The norm is y / sqrt(mean(y^2) + eps) * (w + plus_one).

@@ -894,14 +894,21 @@ def attention_maps_units_takes(q: torch.Tensor, k_pages: torch.Tensor, v_pages: 
                                                                 int(v_pages.shape[2]), int(page_size), q.stride(0), _ptr(q)))
 
 
+def attention_group_size() -> int:
+    """How many consecutive units of a request `paged_attention_maps_units` can take as one group."""
+    return int(_lib.load().sa_paged_attention_groups_size())
+
+
 def paged_attention_maps_units(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,
                                units: torch.Tensor, unit_begin: int, unit_count: int, num_heads: int, *, scale: float,
                                maps: int = 1, window: int | None = None,
                                differential: "tuple[float, float, float] | None" = None, max_kv_len: int, max_q_len: int,
-                               out: torch.Tensor | None = None) -> torch.Tensor:
+                               out: torch.Tensor | None = None, grouped: int = 0) -> torch.Tensor:
     """`paged_attention_maps` in bfloat16 on the matrix cores, over the units [unit_begin, unit_begin + unit_count) of
     `units` (int32 [U, 4]: slot, first row, tokens, first position; at most 16 // attention_maps_heads_per_unit tokens
-    each).  Two maps come with their differential combination.  Returns [T, H * dv] (rows of no unit are not written)."""
+    each).  Two maps come with their differential combination.  Returns [T, H * dv] (rows of no unit are not written).
+    grouped: the last so many units come in groups of `attention_group_size` that belong to one request each (empty
+    units where its tokens end); many of them, of sizes that the kernel for groups takes, share their keys in LDS."""
     _dev(q, k_pages, v_pages, block_table, units, out)
     q_stride = _rows(q, "paged_attention_maps_units: q")
     if not attention_maps_units_takes(q, k_pages, v_pages, num_heads, maps):
@@ -927,6 +934,16 @@ def paged_attention_maps_units(q: torch.Tensor, k_pages: torch.Tensor, v_pages: 
     out_stride = _rows(out, "paged_attention_maps_units: out")
     lam, eps, mult = differential if differential is not None else (0.0, 0.0, 1.0)
     ws = _workspace(q.device)
+    lib = _lib.load()
+    if grouped and maps == 1 and out_stride % 4 == 0 and out.data_ptr() % 8 == 0 and \
+            lib.sa_paged_attention_groups_takes(int(num_heads), Kh, row, dv, page_size, q_stride, _ptr(q)) and \
+            lib.sa_paged_attention_groups_pays(int(grouped), int(num_heads), Kh, int(window or 0), int(max_kv_len), int(max_q_len)):
+        unit_count -= grouped
+        for at in range(0, int(grouped), 32768):
+            _lib.call("sa_paged_attention_groups", _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
+                      block_table.stride(0), _ptr(units), int(unit_begin) + int(unit_count) + at,
+                      min(32768, int(grouped) - at), _ptr(out), out_stride, int(num_heads), Kh, row, dv, page_size,
+                      int(window or 0), float(scale), int(max_kv_len), int(max_q_len), _ptr(ws), ws.numel(), _stream())
     for at in range(0, int(unit_count), 32768):   # (a launch takes that many units)
         _lib.call("sa_paged_attention_maps_units", _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
                   block_table.stride(0), _ptr(units), int(unit_begin) + at, min(32768, int(unit_count) - at), _ptr(out),

@@ -124,11 +124,13 @@ class LatentAttention(Mixer):
                                       k_rot_at=R, slot_mapping=group.slot_mapping, k_pages=cache.k_pages,
                                       v_pages=cache.v_pages, key_values=R)
         if ops.attention_maps_units_takes(qa, cache.k_pages, cache.v_pages, H):
-            # bfloat16 at sizes that the matrix cores take: units of 16 rows (heads times tokens), keys cut into ranges
-            units, few, many, max_q = ctx.attention_units(16 // ops.attention_maps_heads_per_unit(H, 1))
+            # bfloat16 at sizes that the matrix cores take: units of 16 rows (heads times tokens), keys cut into ranges;
+            # a prompt's units come in groups that share the keys
+            units, few, many, max_q = ctx.attention_units(16 // ops.attention_maps_heads_per_unit(H, 1),
+                                                          ops.attention_group_size())
             o = ops.paged_attention_maps_units(qa, cache.k_pages, cache.v_pages, group.block_table, units, 0, few + many,
                                                H, scale=self.scale, window=self.window, max_kv_len=ctx.max_kv_len,
-                                               max_q_len=max_q)
+                                               max_q_len=max_q, grouped=many)
         else:
             o = ops.paged_attention_maps(qa, cache.k_pages, cache.v_pages, group.block_table, ctx.token_seq,
                                          ctx.positions, H, scale=self.scale, window=self.window)     # [T, H * R]
