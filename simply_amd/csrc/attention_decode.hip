@@ -37,13 +37,14 @@ __device__ inline float fast_tanh(float x) {
   return 1.f - 2.f / (e + 1.f);
 }
 
-// NDC = head size / 32
+// A workgroup's work on tiles [tb, te) (absolute, of 32 keys) of the unit (request of `sm`, key head kh).  The result goes
+// to `out`, or, if `partial` is not null, unnormalised to 16 rows there.  NDC = head size / 32.
 template <int NDC>
-__global__ __launch_bounds__(256) void paged_attention_decode_kernel(
+__device__ __forceinline__ void decode_piece(
     const bf16* __restrict__ q, int64_t q_stride, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
-    const int* __restrict__ block_table, int table_stride, const SeqMeta* __restrict__ seq_meta, int seq_begin,
+    const int* __restrict__ block_table, int table_stride, const SeqMeta sm, int kh, int tb, int te,
     bf16* __restrict__ out, int64_t out_stride, int Kh, int G, int page_size, int window, float soft_cap,
-    float* __restrict__ workspace, const float* __restrict__ sinks, const float* __restrict__ slopes) {
+    float* __restrict__ partial, const float* __restrict__ sinks, const float* __restrict__ slopes) {
   // sinks (or null): one logit per query head that joins the softmax's sum and has no value
   // slopes (or null): per query head, what a score loses for every position between the query and the key
   constexpr int HD = NDC * 32;
@@ -55,8 +56,6 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // the same for the whole wave: kept in a scalar register
   const int r = lane % 16, grp = lane / 16;
-  const int split = blockIdx.x, num_splits = gridDim.x, kh = blockIdx.y, seq = seq_begin + blockIdx.z;
-  const SeqMeta sm = seq_meta[seq];
   const int rows = G * sm.q_len;  // <= 16
   const int* table = block_table + static_cast<size_t>(sm.slot) * table_stride;
 
@@ -68,12 +67,6 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
   const int lo = (window > 0 && sm.pos0 - window + 1 > 0) ? sm.pos0 - window + 1 : 0;
   const int lo_r = (window > 0 && pos_r - window + 1 > 0) ? pos_r - window + 1 : 0;
   const float slope_r = slopes != nullptr ? slopes[kh * G + g] : 0.f;
-
-  // tiles of 32 keys aligned to absolute positions; this workgroup's share, then this wave's
-  const int tile0 = lo / kTile, tile1 = (hi + kTile - 1) / kTile;
-  const int ntiles = tile1 - tile0;
-  const int tb = tile0 + static_cast<int>(static_cast<int64_t>(ntiles) * split / num_splits);
-  const int te = tile0 + static_cast<int>(static_cast<int64_t>(ntiles) * (split + 1) / num_splits);
 
   // Where every sub-tile of 16 keys of the range lies is looked up once per pass, into LDS, so that the loop below
   // has no load whose address depends on another load.  (A sub-tile lies within one page: page_size is a multiple
@@ -296,11 +289,8 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
   __syncthreads();
   if (wave == 0) take(0);
 
-  const int KS = num_splits;
-  const size_t row_words = HD + kRowExtra;  // output, maximum, sum
-  const size_t unit = (static_cast<size_t>(blockIdx.z) * Kh + kh);
   if (wave == 0 && row_ok) {
-    if (KS == 1) {
+    if (partial == nullptr) {
       bf16* op = out + static_cast<size_t>(sm.q_start + qi) * out_stride + static_cast<size_t>(kh * G + g) * HD;
       const float inv = 1.f / (sinks != nullptr ? l_run + __expf(sinks[kh * G + g] - m_run) : l_run);
 #pragma unroll
@@ -308,7 +298,7 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
 #pragma unroll
         for (int v = 0; v < 4; ++v) op[db * 16 + 4 * grp + v] = float_to_bf16(acc[db][v] * inv);
     } else {
-      float* wp = workspace + ((unit * KS + split) * 16 + r) * row_words;
+      float* wp = partial + r * (HD + kRowExtra);  // output, maximum, sum
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -321,13 +311,140 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
   }
 }
 
+// The tiles of 32 keys, aligned to absolute positions, that the rows of a request see: [*first, *first + result).
+__device__ inline int request_tiles(const SeqMeta& m, int window, int* first) {
+  const int lo = (window > 0 && m.pos0 - window + 1 > 0) ? m.pos0 - window + 1 : 0;
+  *first = lo / kTile;
+  return m.q_len > 0 ? (m.pos0 + m.q_len + kTile - 1) / kTile - lo / kTile : 0;
+}
+
+// One workgroup per (range of keys, key head, request): every request's keys are cut into gridDim.x ranges.
+template <int NDC>
+__global__ __launch_bounds__(256) void paged_attention_decode_kernel(
+    const bf16* __restrict__ q, int64_t q_stride, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
+    const int* __restrict__ block_table, int table_stride, const SeqMeta* __restrict__ seq_meta, int seq_begin,
+    bf16* __restrict__ out, int64_t out_stride, int Kh, int G, int page_size, int window, float soft_cap,
+    float* __restrict__ workspace, const float* __restrict__ sinks, const float* __restrict__ slopes) {
+  const int split = blockIdx.x, num_splits = gridDim.x, kh = blockIdx.y;
+  const SeqMeta sm = seq_meta[seq_begin + blockIdx.z];
+  int tile0;
+  const int ntiles = request_tiles(sm, window, &tile0);
+  const int tb = tile0 + static_cast<int>(static_cast<int64_t>(ntiles) * split / num_splits);
+  const int te = tile0 + static_cast<int>(static_cast<int64_t>(ntiles) * (split + 1) / num_splits);
+  const size_t unit = static_cast<size_t>(blockIdx.z) * Kh + kh;
+  decode_piece<NDC>(q, q_stride, k_pages, v_pages, block_table, table_stride, sm, kh, tb, te, out, out_stride, Kh, G,
+                    page_size, window, soft_cap,
+                    num_splits == 1 ? nullptr : workspace + (unit * num_splits + split) * 16 * (NDC * 32 + kRowExtra),
+                    sinks, slopes);
+}
+
+// Ranges of about equal size, whatever the requests' lengths: the workgroups read them and cut the keys of every (request,
+// key head) into as many ranges as it takes for ranges of at most `share` tiles, with the smallest `share` (between bounds,
+// by halving) for which the ranges are no more than the workgroups.  A workgroup takes one range.  A range that is not all
+// of its request's keys leaves its result in slot w of the workspace; first_count[unit] are the workgroup of a unit's first
+// range and how many it has.  Bound by reading the keys, as above.
+// Measured (head size 256, lengths spread evenly over their logarithm): 64 requests of 129 to 8,191 keys over 8 key heads
+// 243 -> 211 us, 24 of them 178 -> 100; 40 over 4 key heads 169 -> 83; 8 34 -> 28.  Lengths that are alike are better off
+// with the kernel above (33 requests of 4,096 keys over 4 key heads: 117 us there, 157 here, two ranges for each).
+// A number per lane combined over the wave, and the sum over the lanes up to each, on the vector unit (shuffles go through
+// LDS: with them the ranges were found 3 to 10 us a launch later).
+template <typename Op>
+__device__ __forceinline__ int over_wave(int n, Op op) {
+  n = op(n, __builtin_amdgcn_mov_dpp(n, 0x128, 0xf, 0xf, true));   // rotations within 16 lanes
+  n = op(n, __builtin_amdgcn_mov_dpp(n, 0x124, 0xf, 0xf, true));
+  n = op(n, __builtin_amdgcn_mov_dpp(n, 0x122, 0xf, 0xf, true));
+  n = op(n, __builtin_amdgcn_mov_dpp(n, 0x121, 0xf, 0xf, true));
+  return op(op(__builtin_amdgcn_readlane(n, 0), __builtin_amdgcn_readlane(n, 16)),
+            op(__builtin_amdgcn_readlane(n, 32), __builtin_amdgcn_readlane(n, 48)));
+}
+__device__ __forceinline__ int sum_up_to(int n, int lane) {
+  n += __builtin_amdgcn_update_dpp(0, n, 0x111, 0xf, 0xf, true);   // shifts within 16 lanes, zeros from outside
+  n += __builtin_amdgcn_update_dpp(0, n, 0x112, 0xf, 0xf, true);
+  n += __builtin_amdgcn_update_dpp(0, n, 0x114, 0xf, 0xf, true);
+  n += __builtin_amdgcn_update_dpp(0, n, 0x118, 0xf, 0xf, true);
+  const int a = __builtin_amdgcn_readlane(n, 15), b = a + __builtin_amdgcn_readlane(n, 31),
+            c = b + __builtin_amdgcn_readlane(n, 47);
+  return n + (lane < 16 ? 0 : lane < 32 ? a : lane < 48 ? b : c);
+}
+
+template <int NDC>
+__global__ __launch_bounds__(256) void paged_attention_decode_shares_kernel(
+    const bf16* __restrict__ q, int64_t q_stride, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
+    const int* __restrict__ block_table, int table_stride, const SeqMeta* __restrict__ seq_meta, int seq_begin, int seq_count,
+    bf16* __restrict__ out, int64_t out_stride, int Kh, int G, int page_size, int window, float soft_cap,
+    float* __restrict__ workspace, const float* __restrict__ sinks, const float* __restrict__ slopes, int least,
+    int2* __restrict__ first_count) {
+  const int lane = threadIdx.x % kWave, w = blockIdx.x, workgroups = gridDim.x;   // (every wave looks for itself)
+  // this lane's request of the first 64 (further ones are read again where they are needed)
+  SeqMeta mine{0, 0, 0, 0};
+  if (lane < seq_count) mine = seq_meta[seq_begin + lane];
+  auto tiles_of = [&](int at) __attribute__((always_inline)) {
+    int first;
+    if (at == 0) return request_tiles(mine, window, &first);
+    return at + lane < seq_count ? request_tiles(seq_meta[seq_begin + at + lane], window, &first) : 0;
+  };
+  auto sum_over = [&](auto f) __attribute__((always_inline)) {   // of a number per request, from its tiles
+    int n = f(tiles_of(0));
+    for (int at = kWave; at < seq_count; at += kWave) n += f(tiles_of(at));
+    return over_wave(n, [](int a, int b) { return a + b; }) * Kh;
+  };
+  const int total = sum_over([](int t) { return t; });
+  int share = max((total + workgroups - 1) / workgroups, least);
+  const int units = seq_count * Kh;
+  auto ranges_of = [&](int size) __attribute__((always_inline)) {
+    return sum_over([&](int t) { return (t + size - 1) / size; });
+  };
+  int longest = tiles_of(0);
+  for (int at = kWave; at < seq_count; at += kWave) longest = max(longest, tiles_of(at));
+  longest = over_wave(longest, [](int a, int b) { return max(a, b); });
+  if (ranges_of(share) > workgroups) {
+    // two sizes that are large enough: as many ranges for every unit, or one to spare for every unit (units < workgroups)
+    const int each = workgroups / units;
+    int enough = min((longest + each - 1) / each, (total + workgroups - units - 1) / (workgroups - units));
+    int small = share;
+#pragma unroll 1
+    for (int n = 0; n < 6 && enough - small > small / 16 + 1; ++n) {
+      const int half = (small + enough) / 2;
+      if (ranges_of(half) > workgroups) small = half;
+      else enough = half;
+    }
+    share = enough;
+  }
+  // this workgroup's range
+  for (int at = 0, before = 0; at < seq_count; at += kWave) {
+    const int n = (tiles_of(at) + share - 1) / share;
+    const int upto = sum_up_to(n, lane);   // ranges of the requests up to this lane's, per head
+    const uint64_t beyond = __builtin_amdgcn_ballot_w64((before + upto) * Kh > w);
+    if (beyond == 0) {
+      before += __builtin_amdgcn_readlane(upto, kWave - 1);
+      continue;
+    }
+    const int l = __builtin_ctzll(beyond), count = __builtin_amdgcn_readlane(n, l);
+    const int in = w - (before + __builtin_amdgcn_readlane(upto, l) - count) * Kh;
+    const int kh = __builtin_amdgcn_readfirstlane(in / count), split = in - kh * count;
+    SeqMeta sm{__builtin_amdgcn_readlane(mine.slot, l), __builtin_amdgcn_readlane(mine.q_start, l),
+               __builtin_amdgcn_readlane(mine.q_len, l), __builtin_amdgcn_readlane(mine.pos0, l)};
+    if (at > 0) sm = seq_meta[seq_begin + at + l];
+    int tile0;
+    const int tiles = request_tiles(sm, window, &tile0);
+    const int tb = tile0 + static_cast<int>(static_cast<int64_t>(tiles) * split / count);
+    const int te = tile0 + static_cast<int>(static_cast<int64_t>(tiles) * (split + 1) / count);
+    if (split == 0 && threadIdx.x == 0) first_count[(at + l) * Kh + kh] = int2{w, count};
+    decode_piece<NDC>(q, q_stride, k_pages, v_pages, block_table, table_stride, sm, kh, tb, te, out, out_stride, Kh, G,
+                      page_size, window, soft_cap,
+                      count == 1 ? nullptr : workspace + static_cast<size_t>(w) * 16 * (NDC * 32 + kRowExtra), sinks, slopes);
+    return;
+  }
+}
+
 // Adds up the key ranges of each (request, head, row), in their order: one workgroup per row, one thread per
 // output dimension; the ranges' weights exp(m_y - max) are computed once into LDS.
 __global__ __launch_bounds__(256) void paged_attention_merge_kernel(const float* __restrict__ workspace, int KS, int HD,
                                                                     const SeqMeta* __restrict__ seq_meta, int seq_begin,
                                                                     bf16* __restrict__ out, int64_t out_stride, int Kh,
                                                                     int G, int chunk_tiles, int group, int window,
-                                                                    const float* __restrict__ sinks) {
+                                                                    const float* __restrict__ sinks,
+                                                                    const int2* __restrict__ first_count) {
   __shared__ float w_s[kMaxSplits];
   __shared__ float scratch[16];
   __shared__ float4 part_s[256];
@@ -343,6 +460,12 @@ __global__ __launch_bounds__(256) void paged_attention_merge_kernel(const float*
     group_keys(seq_meta, seq_begin + z / group * group, group, window, &lo, &hi, &slot);
     KS = key_chunks(lo, hi, chunk_tiles);
     if (KS <= 1) return;
+  }
+  if (first_count != nullptr) {  // ranges of about equal size: the unit's first, and how many
+    const int2 fc = first_count[unit];
+    KS = fc.y;
+    if (KS <= 1) return;
+    base = workspace + (static_cast<size_t>(fc.x) * 16 + orow) * row_words;
   }
   const float my = tid < KS ? base[tid * stride + HD] : -INFINITY;
   const float ly = tid < KS ? base[tid * stride + HD + 1] : 0.f;
@@ -420,7 +543,8 @@ static int decode_max_tiles(int window, int max_kv_len) {
   return (span + kTile - 1) / kTile + 1;
 }
 
-// Into how many ranges the keys of each request are cut (num_splits > 0 asks for that many).
+// Into how many ranges the keys of each request are cut (num_splits > 0 asks for that many; < 0: the lengths differ widely,
+// which paged_attention_decode answers with ranges of equal size where it can).
 int paged_attention_decode_ranges(int seq_count, int Kh, int window, int max_kv_len, int num_splits) {
   const int units = seq_count * Kh;
   const int max_tiles = decode_max_tiles(window, max_kv_len);
@@ -454,18 +578,41 @@ int paged_attention_decode(const void* q, int64_t q_stride, const void* k_pages,
   if (seq_count == 0) return 0;
   const int G = H / Kh;
   const int units = seq_count * Kh;
-  int KS = paged_attention_decode_ranges(seq_count, Kh, window, max_kv_len, num_splits);
-  const size_t per_split = static_cast<size_t>(units) * 16 * (hd + kRowExtra) * sizeof(float);
-  while (KS > 1 && (workspace == nullptr || per_split * KS > workspace_bytes)) --KS;
-  // (ranges of more than kMaxRangeSubTiles sub-tiles, which a small workspace or a caller's own num_splits may
-  // leave, take several passes inside the kernel)
-  const dim3 grid(KS, Kh, seq_count);
   const bf16* qp = static_cast<const bf16*>(q);
   const bf16* kp = static_cast<const bf16*>(k_pages);
   const bf16* vp = static_cast<const bf16*>(v_pages);
   const SeqMeta* sm = reinterpret_cast<const SeqMeta*>(seq_meta);
   bf16* op = static_cast<bf16*>(out);
   float* ws = static_cast<float*>(workspace);
+  // Requests whose lengths differ widely (num_splits < 0; the callers' rule stands at StepContext.decode_splits), where
+  // the longest has 1,500 keys or more: ranges of about equal size, as many as one for every unit and one for every CU
+  // (384 and 512 instead of 256 on top measured alike, 1,024 up to 15 % slower), of 16 tiles at least.
+  const int max_tiles = decode_max_tiles(window, max_kv_len);
+  if (num_splits < 0 && seq_count > 1 && max_tiles >= 48) {
+    const int workgroups = units + 256, least = max_tiles / 64 > 16 ? max_tiles / 64 : 16;
+    const size_t index_bytes = (static_cast<size_t>(units) * sizeof(int2) + 255) / 256 * 256;
+    const size_t slots = static_cast<size_t>(workgroups) * 16 * (hd + kRowExtra) * sizeof(float);
+    if (workspace != nullptr && index_bytes + slots <= workspace_bytes) {
+      int2* first_count = static_cast<int2*>(workspace);
+      float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + index_bytes);
+#define SA_LAUNCH(NDC)                                                                                                  paged_attention_decode_shares_kernel<NDC><<<workgroups, 256, 0, stream>>>(                                                qp, q_stride, kp, vp, block_table, table_stride, sm, seq_begin, seq_count, op, out_stride, Kh, G, page_size, window,       soft_cap, partial, sinks, slopes, least, first_count)
+      if (hd == 64) SA_LAUNCH(2);
+      else if (hd == 128) SA_LAUNCH(4);
+      else SA_LAUNCH(8);
+#undef SA_LAUNCH
+      if (check_launch("paged_attention_decode_shares")) return 1;
+      const int max_rows = G * max_q_len < 16 ? G * max_q_len : 16;
+      paged_attention_merge_kernel<<<dim3(Kh, seq_count, max_rows), 256, 0, stream>>>(
+          partial, workgroups, hd, sm, seq_begin, op, out_stride, Kh, G, 0, 1, window, sinks, first_count);
+      return check_launch("paged_attention_merge");
+    }
+  }
+  int KS = paged_attention_decode_ranges(seq_count, Kh, window, max_kv_len, num_splits);
+  const size_t per_split = static_cast<size_t>(units) * 16 * (hd + kRowExtra) * sizeof(float);
+  while (KS > 1 && (workspace == nullptr || per_split * KS > workspace_bytes)) --KS;
+  // (ranges of more than kMaxRangeSubTiles sub-tiles, which a small workspace or a caller's own num_splits may
+  // leave, take several passes inside the kernel)
+  const dim3 grid(KS, Kh, seq_count);
 #define SA_LAUNCH(NDC)                                                                                              \
   paged_attention_decode_kernel<NDC><<<grid, 256, 0, stream>>>(qp, q_stride, kp, vp, block_table, table_stride, sm, \
                                                                seq_begin, op, out_stride, Kh, G, page_size, window,  \
@@ -599,7 +746,7 @@ int attention_merge_ranges(const float* workspace, int num_ranges, int hd, const
   }
   // one workgroup per row: rows beyond the longest unit's are not launched
   paged_attention_merge_kernel<<<dim3(Kh, unit_count, max_rows), 256, 0, stream>>>(
-      workspace, num_ranges, hd, units, unit_begin, out, out_stride, Kh, G, chunk_tiles, group, window, sinks);
+      workspace, num_ranges, hd, units, unit_begin, out, out_stride, Kh, G, chunk_tiles, group, window, sinks, nullptr);
   return check_launch("paged_attention_merge");
 }
 

@@ -17,6 +17,7 @@ import torch
 from ..cache import CacheManager, pages_for_memory
 from ..config import EngineConfig
 from ..models import DecoderModel
+from ..parts.base import PagedKVNeed
 from .context import GroupStep, StepContext
 
 
@@ -76,10 +77,13 @@ class Executor:
         self._extra_dev = torch.empty(self._extra_words, dtype=torch.int32, device=self.device) if self._on_gpu else None
         self._extra_copied = torch.cuda.Event() if self._on_gpu else None
         self._extra_used = 0
-        # decode-only steps (one token per request) are captured once per number of requests and order of magnitude
-        # of the context (the attention kernels choose their cut of the keys when they are recorded) and replayed
+        # decode-only steps (one token per request) are captured once per number of requests, order of magnitude of the
+        # context and whether the requests' lengths differ widely (the attention kernels choose their cut of the keys when
+        # they are recorded) and replayed
         self._graphs: dict[tuple, torch.cuda.CUDAGraph] = {}
         self._graph_pool = None
+        parts = [n for need, _ in needs for n in getattr(need, "parts", (need,))]
+        self._kv_kinds = sorted({(n.window or 0, n.num_kv_heads) for n in parts if isinstance(n, PagedKVNeed)})
         # where every recorded step writes its logits, [batch_size, vocab] float32: made at the first such step
         self._graph_logits: torch.Tensor | None = None
         # several decode steps in a row without the host (decode_many): what was drawn in each, and the step count
@@ -123,7 +127,7 @@ class Executor:
         first step with a new key runs eagerly (kernels choose their plans, scratch buffers get allocated) and is
         this call's result; the recording that follows executes nothing (a mixer that keeps a state of its own would
         otherwise advance it twice)."""
-        key = (T, self._context_bucket(ctx))
+        key = (T, self._context_bucket(ctx), self._splits(ctx))
         ctx.kv_bound = 1 << key[1]
         out = self._shared_logits()[:T]
         graph = self._graphs.get(key)
@@ -157,6 +161,11 @@ class Executor:
         `ahead` further steps in a row, every run of steps) whose longest context stays within 2 ** bucket keys, and
         its kernels are planned for that many (`StepContext.kv_bound`)."""
         return max(ctx.max_kv_len + ahead - 1, 0).bit_length()
+
+    def _splits(self, ctx: StepContext) -> tuple[int, ...]:
+        """How the attention layers of a decode-only step cut the keys (`StepContext.decode_splits`): a recorded step serves
+        steps whose layers would choose alike."""
+        return tuple(ctx.decode_splits(window, ctx.num_seqs, heads) for window, heads in self._kv_kinds)
 
     # ------------------------------------------------------------------ the step
     def step(self, entries: Sequence[StepEntry]) -> torch.Tensor | None:
@@ -241,7 +250,8 @@ class Executor:
                 ops.decode_slots(dev[cap:cap + T], dev[2 * cap:2 * cap + T], table, self.cache.page_size, slots)
 
         ops.fill_(counter, 0)
-        key = ("many", B, self._context_bucket(ctx, num_steps - 1), max_steps, id(sampler), sampler.modes)
+        key = ("many", B, self._context_bucket(ctx, num_steps - 1), max_steps, id(sampler), sampler.modes,
+               self._splits(ctx))
         ctx.kv_bound = 1 << key[2]
         graph = self._graphs.get(key)
         launched = 0

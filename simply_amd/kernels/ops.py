@@ -759,7 +759,8 @@ def paged_attention_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torc
     """Attention of requests seq_begin .. seq_begin + seq_count - 1 of seq_meta, each with few tokens
     ((heads per key head) * tokens <= 16).  q and out are the whole step's rows.  sinks: float32 [H], one more term
     exp(sinks[h]) in every softmax sum, without a value.  slopes: float32 [H], slopes[h] times the distance between
-    query and key is taken off the scores."""
+    query and key is taken off the scores.  num_splits: into how many ranges each request's keys are cut; 0: chosen for
+    lengths that are much alike; -1: for lengths that differ widely (`StepContext.decode_splits`)."""
     return _attention_units("sa_paged_attention_decode", q, k_pages, v_pages, block_table, seq_meta, seq_begin,
                             seq_count, num_heads, window, soft_cap, max_kv_len, max_q_len, out, num_splits, sinks, slopes)
 

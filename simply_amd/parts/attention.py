@@ -88,7 +88,8 @@ class PagedAttention(Mixer):
             units, few, many, max_q = ctx.attention_units(16 // (H // K), ops.prefill_units_per_group())
             kw = dict(window=self.window, soft_cap=self.soft_cap, max_kv_len=ctx.max_kv_len, max_q_len=max_q, out=o)
             if few:
-                ops.paged_attention_decode(qkv, cache.k_pages, cache.v_pages, group.block_table, units, 0, few, H, **kw)
+                ops.paged_attention_decode(qkv, cache.k_pages, cache.v_pages, group.block_table, units, 0, few, H,
+                                           num_splits=ctx.decode_splits(self.window, few, K), **kw)
             if many:
                 ops.paged_attention_prefill(qkv, cache.k_pages, cache.v_pages, group.block_table, units, few, many, H,
                                             **kw)
@@ -209,7 +210,8 @@ class SinkAttention(Mixer):
             kw = dict(window=self.window, soft_cap=None, max_kv_len=ctx.max_kv_len, max_q_len=max_q, out=o,
                       sinks=self.sink_f32)
             if few:
-                ops.paged_attention_decode(proj, cache.k_pages, cache.v_pages, group.block_table, units, 0, few, H, **kw)
+                ops.paged_attention_decode(proj, cache.k_pages, cache.v_pages, group.block_table, units, 0, few, H,
+                                           num_splits=ctx.decode_splits(self.window, few, K), **kw)
             if many:
                 ops.paged_attention_prefill(proj, cache.k_pages, cache.v_pages, group.block_table, units, few, many, H,
                                             **kw)

@@ -216,7 +216,8 @@ class GatedAttention(Mixer):
             kw = dict(window=self.window, soft_cap=None, max_kv_len=ctx.max_kv_len, max_q_len=max_q, out=o,
                       sinks=self.sinks, slopes=self.slopes)
             if few:
-                ops.paged_attention_decode(q, pages.k_pages, pages.v_pages, group.block_table, units, 0, few, H, **kw)
+                ops.paged_attention_decode(q, pages.k_pages, pages.v_pages, group.block_table, units, 0, few, H,
+                                           num_splits=ctx.decode_splits(self.window, few, K), **kw)
             if many:
                 ops.paged_attention_prefill(q, pages.k_pages, pages.v_pages, group.block_table, units, few, many, H, **kw)
         elif self.sinks is None and self.slopes is None and \
