@@ -64,3 +64,54 @@ def test_head_products(H, I, O, tail, gates):
         if T > 1 and I % 32 == 0:
             alone = ops.head_product(x[T - 1:], w, in_stride=I + tail + 8, tail=tail, gate=None if gate is None else gate[T - 1:])
             assert torch.equal(alone.double().reshape(H, -1), got[T - 1])
+
+
+@pytest.mark.parametrize("H,size,dtype,weight,offset", [
+    (3, 128, torch.float32, "shared", 0), (5, 32, torch.bfloat16, "own", 0), (1, 512, torch.bfloat16, None, 0),
+    (7, 64, torch.float32, "own 32", 0), (2, 256, torch.bfloat16, "shared 32", 0), (3, 128, torch.float32, "shared", 3), (3, 96, torch.bfloat16, "own", 0)])
+def test_gated_heads(H, size, dtype, weight, offset):
+    """Heads in pieces of eight entries, and the sizes and alignments that are left to a wave a head (the last two): a norm's
+    sum of squares is off by (size / 64 + 8) steps of 2^-24 at most, the rest by a few; the result is rounded once."""
+    from simply_amd.kernels import ops
+
+    w = None
+    if weight is not None:
+        w = draw((size * (H if "own" in weight else 1),), 2, torch.float32 if "32" in weight else torch.bfloat16, 1.0)
+    for T in (1, 5, 67):
+        x, g = draw((T, H * size + 8), 3, dtype)[:, offset:offset + H * size], draw((T, H * size + 16), 4, torch.bfloat16)[:, 8:8 + H * size]
+        for kind in (0, 1):
+            got = ops.gated_heads(x, g, H, size, kind=kind, weight=w, eps=1e-5, out_dtype=torch.bfloat16).double()
+            v = x.double().reshape(T, H, size)
+            if w is not None:
+                v = v / (v.square().mean(2, keepdim=True) + 1e-5).sqrt() * w.double().reshape(-1, size)
+            gd = g.double().reshape(T, H, size)
+            want = (v * torch.sigmoid(gd) * (gd if kind == 1 else 1.0)).reshape(T, -1)
+            assert ((got - want).abs() <= (2.0 ** -8 + (size / 64 + 24) * 2.0 ** -24) * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("D,dtype,out_dtype,gated,offset", [
+    (2048, torch.bfloat16, torch.bfloat16, True, 0), (1028, torch.float32, torch.float32, False, 0), (4, torch.bfloat16, torch.float32, True, 0),
+    (100, torch.float32, torch.bfloat16, True, 0), (64, None, torch.bfloat16, False, 0), (1030, torch.bfloat16, torch.bfloat16, True, 0),
+    (64, torch.bfloat16, torch.bfloat16, False, 2)])
+def test_expert_combine(D, dtype, out_dtype, gated, offset):
+    """Four entries a thread, and the widths and alignments that are left to one (the last two): top products and two sums
+    in 32 bits, rounded once."""
+    from simply_amd.kernels import lib, ops
+
+    for T, top in ((1, 1), (3, 4), (70, 9)):
+        y, weights = draw((T * top, D), 1), draw((T, top), 2).abs()
+        shared = None if dtype is None else draw((T, D + 8), 3, dtype)[:, offset:offset + D]
+        gate = draw((T, 3), 4)[:, 1:2] if gated else None
+        out = torch.empty((T, D), dtype=out_dtype, device="cuda")
+        code = lambda t: 0 if t is None else ops._code(t)
+        lib.call("sa_expert_combine", y.data_ptr(), weights.data_ptr(), top, None if shared is None else shared.data_ptr(), code(shared),
+                 0 if shared is None else shared.stride(0), None if gate is None else gate.data_ptr(), 3, out.data_ptr(), code(out), D, T, D,
+                 ops._stream())
+        got = out.double()
+        terms = y.double().reshape(T, top, D) * weights.double()[:, :, None]
+        extra = torch.zeros(T, D, dtype=torch.float64, device="cuda") if shared is None else shared.double()
+        if gate is not None:
+            extra = extra * torch.sigmoid(gate.double())
+        step = 2.0 ** -24 if out_dtype == torch.float32 else 2.0 ** -8
+        room = terms.abs().sum(1) + extra.abs()
+        assert ((got - terms.sum(1) - extra).abs() <= step * (terms.sum(1) + extra).abs() + (top + 12) * 2.0 ** -23 * room).all()
