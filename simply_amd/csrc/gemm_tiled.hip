@@ -383,6 +383,15 @@ int gemm_tiled(const void* A, int64_t lda, const void* W, void* C, int c_dtype, 
     // at 256 rows of the 2B down projection 9 cuts (38 us) instead of 36 (54 us); at 64 rows nothing changes
     const int by_traffic = static_cast<int>((static_cast<int64_t>(NW) * K * 2) / (2 * static_cast<int64_t>(M) * NW * 4));
     if (ks > by_traffic) ks = by_traffic < 2 ? 2 : by_traffic;
+    if (M > 64 && M > NW) {
+      // many rows of few outputs (a router, gates): bound by reading the rows, by a workgroup per 64 of them: K is cut until
+      // there is a workgroup per CU, with the partial tiles at half the rows' and weights' bytes
+      const int row_tiles = (M + 63) / 64 * tiles;
+      const int by_rows = static_cast<int>((static_cast<int64_t>(NW) + M) * K * 2 / (2 * static_cast<int64_t>(M) * NW * 4));
+      const int cuts = min(min(256 / row_tiles, stages / 4), by_rows);
+      // (K = 2,048: 2,047 rows of 16 outputs 17.7 -> 10.5 us, of 64 18.2 -> 12.2, of 128 18.7 -> 14.7; 513 rows of 16 17.2 -> 9.7)
+      if (cuts > ks) ks = cuts;
+    }
   }
   if (ks > stages) ks = stages;
   if (ks < 1) ks = 1;

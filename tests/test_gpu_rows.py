@@ -115,3 +115,16 @@ def test_expert_combine(D, dtype, out_dtype, gated, offset):
         step = 2.0 ** -24 if out_dtype == torch.float32 else 2.0 ** -8
         room = terms.abs().sum(1) + extra.abs()
         assert ((got - terms.sum(1) - extra).abs() <= step * (terms.sum(1) + extra).abs() + (top + 12) * 2.0 ** -23 * room).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 16, 256), (65, 64, 2048), (130, 4, 1000), (300, 256, 2048), (1025, 32, 4096), (2047, 16, 2048),
+                                   (2047, 128, 520), (9000, 16, 1024), (17000, 8, 512)])
+def test_narrow_products(M, N, K):
+    """Many rows of few outputs, the inner dimension cut or not: sums of K bfloat16 products in 32 bits."""
+    from simply_amd.kernels import ops
+    from simply_amd.parts.base import as_product_weight
+
+    x, w = draw((M, K + 8), 1, torch.bfloat16)[:, :K], draw((N, K), 2, torch.bfloat16)
+    got = ops.gemm(x, as_product_weight(w), out_dtype=torch.float32).double()
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    assert ((got - want).abs() <= (K / 32 + 16) * 2.0 ** -24 * size).all()
