@@ -397,10 +397,13 @@ __global__ __launch_bounds__(256) void paged_attention_decode_shares_kernel(
   int longest = tiles_of(0);
   for (int at = kWave; at < seq_count; at += kWave) longest = max(longest, tiles_of(at));
   longest = over_wave(longest, [](int a, int b) { return max(a, b); });
+  // (no more ranges for a unit than the second kernel adds up, also where a caller understates the longest request)
+  share = max(share, (longest + kMaxSplits - 1) / kMaxSplits);
   if (ranges_of(share) > workgroups) {
     // two sizes that are large enough: as many ranges for every unit, or one to spare for every unit (units < workgroups)
     const int each = workgroups / units;
     int enough = min((longest + each - 1) / each, (total + workgroups - units - 1) / (workgroups - units));
+    enough = max(enough, share);
     int small = share;
 #pragma unroll 1
     for (int n = 0; n < 6 && enough - small > small / 16 + 1; ++n) {

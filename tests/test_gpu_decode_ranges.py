@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
     (8, 2, 128, 16, None, 1, "sinks", [1 + (i * 37) % 90 for i in range(150)] + [3000, 1, 2600]),
     (6, 2, 64, 48, 1900, 2, "slopes", [2000, 5, 0, 1700, 0, 300] * 12),
     (16, 1, 64, 16, None, 1, "", [4097, 1]),
+    (1, 1, 64, 16, None, 1, "understated", [140000, 40]),   # more tiles than ranges that are added up, of the least size
 ])
 def test_decode_uneven(H, K, hd, page, window, q_len, extra, lens):
     """Probabilities are rounded to bfloat16 before the values and the result once more, 2^-8 each; 2^-11 of the terms more
@@ -56,7 +57,7 @@ def test_decode_uneven(H, K, hd, page, window, q_len, extra, lens):
     results = []
     for _ in range(2):
         out = torch.full((T, H * hd), float("nan"), dtype=torch.bfloat16, device="cuda")
-        ops.paged_attention_decode(qd, kp, vp, table, meta, 0, len(lens), H, window=window, soft_cap=None, max_kv_len=max(lens),
+        ops.paged_attention_decode(qd, kp, vp, table, meta, 0, len(lens), H, window=window, soft_cap=None, max_kv_len=1600 if extra == "understated" else max(lens),
                                    max_q_len=q_len, out=out, num_splits=-1, sinks=sinks, slopes=slopes)
         results.append(out.double().cpu().reshape(T, H, hd))
     assert torch.equal(*results)
