@@ -29,13 +29,12 @@
 // Measured at 2,048 tokens of 16 heads over 8, sizes 128: 45 us for the pieces and 98 for the walk, where delta_rule.hip takes
 // 629 token by token.
 #include "api.h"
-#include "attention_common.h"
+#include "chunks.h"
 
 namespace sa {
 namespace delta {
 
-constexpr int kTokens = 64, kBlocks = kTokens / 16;
-constexpr int kBlock = 256;   // floats of a 16 x 16 block
+using namespace chunks;
 
 // A piece's operands in the workspace (floats), for NT blocks of 16 key channels and CB blocks of 16 value columns.
 struct Layout {
@@ -64,27 +63,6 @@ struct Args {
   int C, G, H, dk, dv, row0, row1;   // the rows of the step that this launch is about
 };
 
-struct Span {
-  int slot, first, count, piece0;
-};
-// The part of a request that lies in the launch's rows; its pieces are numbered from piece0 on, no two requests' alike.
-__device__ __forceinline__ Span span_of(const Args& a, int seq) {
-  const int* meta = a.seq_meta + 4 * seq;
-  const int lo = meta[1] > a.row0 ? meta[1] : a.row0, end = meta[1] + meta[2], hi = end < a.row1 ? end : a.row1;
-  Span s;
-  s.slot = meta[0];
-  s.first = lo;
-  s.count = hi - lo;
-  s.piece0 = (lo - a.row0) / kTokens + seq;
-  return s;
-}
-
-__device__ __forceinline__ floatx4 mul4(floatx4 a, floatx4 b, floatx4 c) {   // four steps: 16 channels or tokens
-#pragma unroll
-  for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
-  return c;
-}
-
 template <int NT>
 __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
   constexpr int ROW = NT * 16 + 4, AROW = kTokens + 4, QUADS = NT * 4;
@@ -93,7 +71,7 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
   __shared__ double cum_s[kTokens];
   __shared__ float beta_s[kTokens], in_s[kTokens], out_s[kTokens];   // beta, exp(L_i), exp(L_64 - L_i)
   static_assert(kTokens * ROW >= kTokens * AROW || NT < 4, "A lies where q lay");
-  const Span sp = span_of(a, blockIdx.z);
+  const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
   const int t0 = blockIdx.x * kTokens;
   if (t0 >= sp.count) return;   // (uniform)
   const int left = sp.count - t0 < kTokens ? sp.count - t0 : kTokens;
@@ -255,7 +233,7 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
   constexpr int NW = NT / 4;   // blocks of key channels whose state a wave holds
   __shared__ __align__(16) floatx4 s_s[2][NT * kWave];
   __shared__ __align__(16) floatx4 u_s[kBlocks * kWave];
-  const Span sp = span_of(a, blockIdx.z);
+  const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
   if (sp.count <= 0) return;
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
@@ -389,13 +367,13 @@ extern "C" int sa_delta_chunks(const float* qkv, int C, int G, int dk, int dv, c
   a.qkv = qkv, a.gates = gates, a.state = state, a.out = out, a.pieces = static_cast<float*>(workspace), a.seq_meta = seq_meta;
   a.state_stride = state_stride, a.C = C, a.G = G, a.H = H, a.dk = dk, a.dv = dv;
   // as many rows at a time as the workspace has room for: R rows are at most R / 64 + num_seqs pieces
-  const int64_t room = (workspace_bytes / delta_piece_bytes(H, dk, dv) - num_seqs) * delta::kTokens;
+  const int64_t room = (workspace_bytes / delta_piece_bytes(H, dk, dv) - num_seqs) * chunks::kTokens;
   const int span = static_cast<int>(room < rows ? room : rows);
   for (int r = 0; r < rows; r += span) {
     a.row0 = first_row + r;
     a.row1 = first_row + (r + span < rows ? r + span : rows);
     const int longest = a.row1 - a.row0 < max_q_len ? a.row1 - a.row0 : max_q_len;
-    const dim3 pieces((longest + delta::kTokens - 1) / delta::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
+    const dim3 pieces((longest + chunks::kTokens - 1) / chunks::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
     if (dk <= 64) {
       delta::delta_pieces_kernel<4><<<pieces, 256, 0, stream>>>(a);
       delta::delta_state_kernel<4><<<walk, 256, 0, stream>>>(a);

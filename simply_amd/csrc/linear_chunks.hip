@@ -23,13 +23,12 @@
 // Measured at 2,048 tokens of 16 heads of 128: 33 us for the pieces and 73 for the walk, where linear_state.hip takes 703
 // token by token.
 #include "api.h"
-#include "attention_common.h"
+#include "chunks.h"
 
 namespace sa {
 namespace linear {
 
-constexpr int kTokens = 64, kBlocks = kTokens / 16;
-constexpr int kBlock = 256;   // floats of a 16 x 16 block
+using namespace chunks;
 
 // A piece's operands in the workspace (floats), for NT blocks of 16 key channels and CB blocks of 16 value columns.
 struct Layout {
@@ -60,26 +59,6 @@ struct Args {
   int q_at, k_at, v_at, H, dk, dv, bias_dtype, bonus_dtype, row0, row1;
 };
 
-struct Span {
-  int slot, first, count, piece0;
-};
-// The part of a request that lies in the launch's rows; its pieces are numbered from piece0 on, no two requests' alike.
-__device__ __forceinline__ Span span_of(const Args& a, int seq) {
-  const int* meta = a.seq_meta + 4 * seq;
-  const int lo = meta[1] > a.row0 ? meta[1] : a.row0, end = meta[1] + meta[2], hi = end < a.row1 ? end : a.row1;
-  Span s;
-  s.slot = meta[0];
-  s.first = lo;
-  s.count = hi - lo;
-  s.piece0 = (lo - a.row0) / kTokens + seq;
-  return s;
-}
-
-__device__ __forceinline__ floatx4 mul4(floatx4 a, floatx4 b, floatx4 c) {   // four steps: 16 channels or tokens
-#pragma unroll
-  for (int r = 0; r < 4; ++r) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
-  return c;
-}
 __device__ __forceinline__ floatx4 to_float4(uint2 v) {   // four bfloat16
   return floatx4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
                  __uint_as_float(v.y & 0xffff0000u)};
@@ -92,7 +71,7 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
   __shared__ __align__(16) bf16 q_s[kTokens * QROW];
   __shared__ __align__(16) bf16 k_s[kTokens * QROW];
   __shared__ __align__(16) float blk_s[kBlocks][NT * 16];   // a block's decays, multiplied
-  const Span sp = span_of(a, blockIdx.z);
+  const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
   const int t0 = blockIdx.x * kTokens;
   if (t0 >= sp.count) return;   // (uniform)
   const int left = sp.count - t0 < kTokens ? sp.count - t0 : kTokens;
@@ -244,7 +223,7 @@ template <int NT>
 __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
   constexpr int NW = NT / 4;   // blocks of key channels whose state a wave holds
   __shared__ __align__(16) floatx4 s_s[2][NT * kWave];
-  const Span sp = span_of(a, blockIdx.z);
+  const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
   if (sp.count <= 0) return;
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
@@ -263,7 +242,7 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
     s_s[0][(wave * NW + n) * kWave + lane] = s[n];
   }
   // a piece's operands, asked for a piece ahead
-  floatx4 q[NT], kt[NW][kBlocks], p[kBlocks], v[kBlocks], all[NW];
+  floatx4 q[NT], kt[NW][kBlocks], p[kBlocks], v[kBlocks], v_own, all[NW];   // (p: blocks in front of the wave's own, and that)
   auto fetch_state = [&](const float* from) __attribute__((always_inline)) {   // what the state behind the piece needs
 #pragma unroll
     for (int n = 0; n < NW; ++n) {
@@ -279,9 +258,10 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) {
       v[b] = *reinterpret_cast<const floatx4*>(from + lay.v + (blockIdx.y * kBlocks + b) * kBlock + lane * 4);
-      const int at = b < wave ? b : wave;   // (blocks behind the wave's own: the own one again, not used)
+      const int at = b < wave ? b : wave;   // (the last: the wave's own; others behind it: that again, not used)
       p[b] = *reinterpret_cast<const floatx4*>(from + lay.p + (wave * kBlocks + at) * kBlock + lane * 4);
     }
+    v_own = *reinterpret_cast<const floatx4*>(from + lay.v + (blockIdx.y * kBlocks + wave) * kBlock + lane * 4);
   };
   fetch_state(src);
   fetch_rest(src);
@@ -309,8 +289,9 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
       o2 = mul4(q[n + 1], st[n + 1], o2);
     }
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b)
-      if (b <= wave) o = mul4(p[b], v[b], o);   // (uniform over the wave)
+    for (int b = 0; b < kBlocks - 1; ++b)
+      if (b < wave) o = mul4(p[b], v[b], o);   // (uniform over the wave)
+    o = lower_mul4(p[kBlocks - 1], v_own, o, lane);
     fetch_rest(next);
     if (col_ok) {
 #pragma unroll
@@ -371,13 +352,13 @@ extern "C" int sa_linear_chunks(const void* proj, int64_t proj_stride, int q_at,
   a.state_stride = state_stride, a.q_mult = q_mult, a.inv_tau = tau > 0.f ? 1.f / tau : 0.f, a.q_at = q_at, a.k_at = k_at;
   a.v_at = v_at, a.H = H, a.dk = dk, a.dv = dv, a.bias_dtype = bias_dtype, a.bonus_dtype = bonus_dtype;
   // as many rows at a time as the workspace has room for: R rows are at most R / 64 + num_seqs pieces
-  const int64_t room = (workspace_bytes / linear_piece_bytes(H, dk, dv) - num_seqs) * linear::kTokens;
+  const int64_t room = (workspace_bytes / linear_piece_bytes(H, dk, dv) - num_seqs) * chunks::kTokens;
   const int span = static_cast<int>(room < rows ? room : rows);
   for (int r = 0; r < rows; r += span) {
     a.row0 = first_row + r;
     a.row1 = first_row + (r + span < rows ? r + span : rows);
     const int longest = a.row1 - a.row0 < max_q_len ? a.row1 - a.row0 : max_q_len;
-    const dim3 pieces((longest + linear::kTokens - 1) / linear::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
+    const dim3 pieces((longest + chunks::kTokens - 1) / chunks::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
 #define SA_LINEAR(NT)                                                                              \
   do {                                                                                             \
     if (bonus != nullptr) linear::linear_pieces_kernel<NT, true><<<pieces, 256, 0, stream>>>(a);   \

@@ -138,3 +138,38 @@ def test_decays_from_their_logits():
     got = ops.linear_chunks(proj, *at, 0.125, z, H, dk, dv, s2, meta, 1, 0, T, out=torch.zeros_like(want), **kw)
     for x, y in ((got, want), (s2, s1)):
         assert (x - y).abs().max() <= 1e-5 * y.abs().max()
+
+
+def special_values(run, T, H, dv, value_at, meta, token, bad):
+    """`run(values)` -> (out, state).  A value of head 1, column 2 of `token` that is not finite changes that column of that
+    head of its own request from `token` on, where nothing is finite any more, and no other bit."""
+    (want, _), (got, state) = run(None), run((token, value_at + 1 * dv + 2, bad))
+    _, first, count, _ = next(m for m in meta if m[1] <= token < m[1] + m[2])
+    hit = torch.zeros(T, H, dv, dtype=torch.bool, device="cuda")
+    hit[token:first + count, 1, 2] = True
+    got, want = got.view(T, H, dv), want.view(T, H, dv)
+    assert torch.isfinite(want).all() and not torch.isfinite(got[hit]).any()
+    assert torch.equal(got[~hit], want[~hit])
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("token", [3, 3 + 40, 3 + 47, 3 + 100 + 79, 3 + 100 + 129])
+@pytest.mark.parametrize("bonus", [True, False])
+def test_channel_decays_keep_special_values(bad, token, bonus):
+    """A value that is not finite reaches its own and later tokens of its request alone, wherever in a piece it stands."""
+    from simply_amd.kernels import ops
+
+    H, dk, dv, meta = 2, 64, 24, [(0, 3, 100, 0), (1, 103, 130, 0)]
+    T, at = 233, (0, 2 * 64, 4 * 64)
+    proj = normal((T, 4 * 64 + H * dv), 81).bfloat16()
+    gates, u = uniform((T, H * dk), 82, 0.5, 1.0).cuda(), normal((H * dk,), 83).cuda() if bonus else None
+
+    def run(change):
+        p, state, out = proj.clone(), normal((2, H * dk * dv), 84).cuda(), torch.zeros(T, H * dv, device="cuda")
+        if change:
+            p[change[0], change[1]] = change[2]
+        ops.linear_chunks(p.cuda(), *at, 1.0, gates, H, dk, dv, state, torch.tensor(meta, dtype=torch.int32).cuda(), 2, 3, 130,
+                          bonus=u, out=out)
+        return out, state
+
+    special_values(run, T, H, dv, at[2], meta, token, bad)
