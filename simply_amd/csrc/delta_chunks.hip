@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
         acc = mul4(m, x[e], acc);
       }
       const floatx4 inv = *reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + b * 16 + g * 4]);
-      x[b] = mul4(inv, acc, floatx4{0.f, 0.f, 0.f, 0.f});
+      x[b] = lower_mul4(inv, acc, floatx4{0.f, 0.f, 0.f, 0.f}, lane);
     }
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) {
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
     s_s[0][(wave * NW + n) * kWave + lane] = s[n];
   }
   // a piece's operands, asked for a piece ahead
-  floatx4 w[NT], q[NT], kt[NW][kBlocks], p[kBlocks], u0;
+  floatx4 w[NT], q[NT], kt[NW][kBlocks], p[kBlocks], u0;   // (p: blocks in front of the wave's own, and that)
   float all;
   auto fetch_state = [&](const float* from) __attribute__((always_inline)) {   // what U and the state behind the piece need
 #pragma unroll
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
       for (int b = 0; b < kBlocks; ++b)
         kt[n][b] = *reinterpret_cast<const floatx4*>(from + lay.kt + ((wave * NW + n) * kBlocks + b) * kBlock + lane * 4);
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b) {   // (blocks behind the wave's own: the own one again, not used)
+    for (int b = 0; b < kBlocks; ++b) {   // (the last: the wave's own; others behind it: that again, not used)
       const int at = b < wave ? b : wave;
       p[b] = *reinterpret_cast<const floatx4*>(from + lay.p + (wave * kBlocks + at) * kBlock + lane * 4);
     }
@@ -315,8 +315,9 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
 #pragma unroll
     for (int n = 0; n < NW; ++n) s_s[now ^ 1][(wave * NW + n) * kWave + lane] = s[n];
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b)
-      if (b <= wave) o = mul4(p[b], ub[b], o);   // (uniform over the wave)
+    for (int b = 0; b < kBlocks - 1; ++b)
+      if (b < wave) o = mul4(p[b], ub[b], o);   // (uniform over the wave)
+    o = lower_mul4(p[kBlocks - 1], u, o, lane);
     fetch_rest(next);
     if (col_ok) {
 #pragma unroll

@@ -173,3 +173,32 @@ def test_channel_decays_keep_special_values(bad, token, bonus):
         return out, state
 
     special_values(run, T, H, dv, at[2], meta, token, bad)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("token", [3, 3 + 40, 3 + 47, 3 + 100 + 79, 3 + 100 + 129])
+def test_delta_rule_keeps_special_values(bad, token):
+    """As above; and a key that is not finite leaves nothing finite behind itself in its head and changes nothing before."""
+    from simply_amd.kernels import ops
+
+    H, dk, dv, meta = 2, 64, 24, [(0, 3, 100, 0), (1, 103, 130, 0)]
+    T, C = 233, 2 * H * 64 + H * 24
+    qkv = normal((T, C), 91)
+    heads = qkv[:, :2 * H * dk].reshape(T, 2 * H, dk)
+    qkv[:, :2 * H * dk] = (heads / heads.square().sum(-1, keepdim=True).sqrt()).reshape(T, -1)
+    gates = torch.cat([uniform((T, H), 92), uniform((T, H), 93, 0.9, 1.0)], 1).cuda()
+
+    def run(change):
+        x, state, out = qkv.clone(), normal((2, H * dk * dv), 94).cuda(), torch.zeros(T, H * dv, device="cuda")
+        if change:
+            x[change[0], change[1]] = change[2]
+        ops.delta_chunks(x.cuda(), gates, state, torch.tensor(meta, dtype=torch.int32).cuda(), 2, 3, 130, H, H, dk, dv, out=out)
+        return out, state
+
+    special_values(run, T, H, dv, 2 * H * dk, meta, token, bad)
+    (want, _), (got, _) = run(None), run((token, (H + 1) * dk + 5, bad))
+    _, first, count, _ = next(m for m in meta if m[1] <= token < m[1] + m[2])
+    hit = torch.zeros(T, H, dv, dtype=torch.bool, device="cuda")
+    hit[token:first + count, 1] = True
+    got, want = got.view(T, H, dv), want.view(T, H, dv)
+    assert not torch.isfinite(got[hit]).any() and torch.equal(got[~hit], want[~hit])
