@@ -32,6 +32,16 @@ __device__ __forceinline__ floatx4 mul4(floatx4 a, floatx4 b, floatx4 c) {   // 
   return c;
 }
 
+// The chains' sums, by halves.
+template <int N>
+__device__ __forceinline__ floatx4 sum_of(floatx4 (&x)[N]) {
+#pragma unroll
+  for (int n = N / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) x[i] += x[i + n];
+  return x[0];
+}
+
 // acc + m . b for a lower triangular m: the diagonal block of a product over earlier tokens.  A product with a zero carries an
 // entry of b that is not finite into every row; such entries are left out of the product, and added one at a time to the rows
 // at and behind their own.

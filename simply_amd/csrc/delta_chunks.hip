@@ -26,8 +26,13 @@
 // this one is worked through.  Bound by the matrix instructions that a wave issues one after the other (about 110 of 32
 // clocks a piece) and two barriers a piece, on as many CUs as there are heads times blocks of 16 columns.
 //
-// Measured at 2,048 tokens of 16 heads over 8, sizes 128: 45 us for the pieces and 98 for the walk, where delta_rule.hip takes
-// 629 token by token.
+// Long chains of matrix instructions round at the size of the sum with every product, so sums run in several short chains, the
+// state's increment and the entries on the diagonal by themselves.  The error against 64 bits is then that of delta_rule.hip
+// (results 0.6 to 1.05 times, the state 0.4 to 0.7 times, 511 to 2,048 tokens); with one or two chains each results were off
+// by up to twice as much.
+//
+// Measured at 2,048 tokens of 16 heads over 8, sizes 128: 41 us for the pieces and 98 for the walk (38 and 89 with one or two
+// chains), where delta_rule.hip takes 629 token by token.
 #include "api.h"
 #include "chunks.h"
 
@@ -38,17 +43,18 @@ using namespace chunks;
 
 // A piece's operands in the workspace (floats), for NT blocks of 16 key channels and CB blocks of 16 value columns.
 struct Layout {
-  int w, q, kt, p, u0, decay, words;
+  int w, q, kt, p, u0, decay, own, words;
 };
 __host__ __device__ constexpr Layout layout(int nt, int cb) {
   Layout l{};
   l.w = 0;                             // [token block][channel block]
   l.q = l.w + kBlocks * nt * kBlock;   // likewise
   l.kt = l.q + kBlocks * nt * kBlock;  // [channel block][token block]
-  l.p = l.kt + kBlocks * nt * kBlock;  // [token block][token block]
+  l.p = l.kt + kBlocks * nt * kBlock;  // [token block][token block], without the diagonal
   l.u0 = l.p + kBlocks * kBlocks * kBlock;   // [column block][token block]
   l.decay = l.u0 + cb * kBlocks * kBlock;    // exp(L_64)
-  l.words = l.decay + 64;
+  l.own = l.decay + 64;                      // the diagonal of P
+  l.words = l.own + kTokens;
   return l;
 }
 
@@ -62,6 +68,12 @@ struct Args {
   int64_t state_stride;
   int C, G, H, dk, dv, row0, row1;   // the rows of the step that this launch is about
 };
+
+// exp(x) for x <= 0; what 32 bits do not hold of x goes in as a factor (a rounding of x alone would be |x| of them of exp(x)).
+__device__ __forceinline__ float decay_between(double x) {
+  const float hi = static_cast<float>(x), e = expf(hi);
+  return fmaf(e, static_cast<float>(x - static_cast<double>(hi)), e);
+}
 
 template <int NT>
 __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
@@ -108,9 +120,9 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
     const double end = __shfl(cum, kWave - 1, kWave);
     cum_s[lane] = cum;
     beta_s[lane] = beta;
-    in_s[lane] = expf(static_cast<float>(cum));
-    out_s[lane] = expf(static_cast<float>(end - cum));
-    if (lane == 0) dst[lay.decay] = expf(static_cast<float>(end));
+    in_s[lane] = decay_between(cum);
+    out_s[lane] = decay_between(end - cum);
+    if (lane == 0) dst[lay.decay] = decay_between(end);
   }
   __syncthreads();
 
@@ -122,20 +134,23 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
   for (int b = 0; b < kBlocks; ++b) {
     kk[b] = floatx4{0.f, 0.f, 0.f, 0.f};
     if (b <= wave) {   // (uniform over the wave)
-      floatx4 qk_b{0.f, 0.f, 0.f, 0.f};
+      floatx4 qk_b[NT], kk_b[NT];   // (a chain of products for each 16 channels)
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const floatx4 kb = *reinterpret_cast<const floatx4*>(&k_s[(b * 16 + c) * ROW + n * 16 + g * 4]);
         const floatx4 kw = *reinterpret_cast<const floatx4*>(&k_s[(wave * 16 + c) * ROW + n * 16 + g * 4]);
         const floatx4 qw = *reinterpret_cast<const floatx4*>(&q_s[(wave * 16 + c) * ROW + n * 16 + g * 4]);
-        qk_b = mul4(kb, qw, qk_b);
-        kk[b] = mul4(kw, kb, kk[b]);
+        qk_b[n] = mul4(kb, qw, kk[b]);
+        kk_b[n] = mul4(kw, kb, kk[b]);
       }
+      const floatx4 qk_all = sum_of(qk_b);
+      kk[b] = sum_of(kk_b);
       floatx4 p;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int j = b * 16 + g * 4 + r, i = wave * 16 + c;
-        p[r] = j <= i ? qk_b[r] * expf(static_cast<float>(cum_c - cum_s[j])) : 0.f;
+        p[r] = j < i ? qk_all[r] * decay_between(cum_c - cum_s[j]) : 0.f;
+        if (j == i) dst[lay.own + i] = qk_all[r];
       }
       *reinterpret_cast<floatx4*>(dst + lay.p + (wave * kBlocks + b) * kBlock + lane * 4) = p;
     }
@@ -161,7 +176,7 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = wave * 16 + g * 4 + r, j = b * 16 + c;
-        a_s[i * AROW + j] = j < i ? kk[b][r] * beta_s[i] * expf(static_cast<float>(cum_s[i] - cum_s[j])) : 0.f;
+        a_s[i * AROW + j] = j < i ? kk[b][r] * beta_s[i] * decay_between(cum_s[i] - cum_s[j]) : 0.f;
       }
     }
   }
@@ -184,10 +199,11 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    // into the block's own place (its entries have been read)
+    // into the block's own place (its entries have been read), without the ones on the diagonal: a sum of 16 products that
+    // holds the large one rounds at its size 16 times
     if (g == 0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) a_s[(wave * 16 + i) * AROW + wave * 16 + c] = x[i];
+      for (int i = 0; i < 16; ++i) a_s[(wave * 16 + i) * AROW + wave * 16 + c] = i == c ? 0.f : x[i];
     }
   }
   __syncthreads();
@@ -205,15 +221,13 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
         if (n < NT) acc[r] = k_s[i * ROW + n * 16 + c] * (beta_s[i] * in_s[i]);
         else acc[r] = (i < left && col < a.dv) ? a.qkv[static_cast<size_t>(row0 + i) * a.C + 2 * a.G * a.dk + h * a.dv + col] * beta_s[i] : 0.f;
       }
+      floatx4 less[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int e = 0; e < b; ++e) {
-        floatx4 m = *reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + e * 16 + g * 4]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) m[r] = -m[r];
-        acc = mul4(m, x[e], acc);
-      }
+      for (int e = 0; e < b; ++e)
+        less[e % 2] = mul4(*reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + e * 16 + g * 4]), x[e], less[e % 2]);
+      acc -= less[0] + less[1];
       const floatx4 inv = *reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + b * 16 + g * 4]);
-      x[b] = lower_mul4(inv, acc, floatx4{0.f, 0.f, 0.f, 0.f}, lane);
+      x[b] = acc + lower_mul4(inv, acc, floatx4{0.f, 0.f, 0.f, 0.f}, lane);
     }
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) {
@@ -252,7 +266,7 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
     s_s[0][(wave * NW + n) * kWave + lane] = s[n];
   }
   // a piece's operands, asked for a piece ahead
-  floatx4 w[NT], q[NT], kt[NW][kBlocks], p[kBlocks], u0;   // (p: blocks in front of the wave's own, and that)
+  floatx4 w[NT], q[NT], kt[NW][kBlocks], p[kBlocks], u0, own;   // (p: blocks in front of the wave's own, and that)
   float all;
   auto fetch_state = [&](const float* from) __attribute__((always_inline)) {   // what U and the state behind the piece need
 #pragma unroll
@@ -272,6 +286,7 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
       const int at = b < wave ? b : wave;
       p[b] = *reinterpret_cast<const floatx4*>(from + lay.p + (wave * kBlocks + at) * kBlock + lane * 4);
     }
+    own = *reinterpret_cast<const floatx4*>(from + lay.own + wave * 16 + g * 4);
     all = from[lay.decay];
   };
   fetch_state(src);
@@ -283,47 +298,53 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
     floatx4 st[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) st[n] = s_s[now][n * kWave + lane];
-    floatx4 x{0.f, 0.f, 0.f, 0.f}, y{0.f, 0.f, 0.f, 0.f};
+    // (sums in four chains, and the state's increment by itself: 64 products added to the state one by one would round it
+    // 64 times)
+    floatx4 x[4], o[4], o2[kBlocks], more[2][NW];
 #pragma unroll
-    for (int n = 0; n < NT; n += 2) {
-      x = mul4(w[n], st[n], x);
-      y = mul4(w[n + 1], st[n + 1], y);
-    }
-    floatx4 u;
+    for (int i = 0; i < 4; ++i) x[i] = o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) u[r] = u0[r] - (x[r] + y[r]);
+    for (int b = 0; b < kBlocks; ++b) o2[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NT; n += 4)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = mul4(w[n + i], st[n + i], x[i]);
+    const floatx4 u = u0 - sum_of(x);
     u_s[wave * kWave + lane] = u;
     fetch_state(next);
-    floatx4 o{0.f, 0.f, 0.f, 0.f}, o2{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int n = 0; n < NT; n += 2) {
-      o = mul4(q[n], st[n], o);
-      o2 = mul4(q[n + 1], st[n + 1], o2);
-    }
+    for (int n = 0; n < NT; n += 4)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = mul4(q[n + i], st[n + i], o[i]);
     __syncthreads();
     floatx4 ub[kBlocks];
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) ub[b] = u_s[b * kWave + lane];
 #pragma unroll
-    for (int n = 0; n < NW; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[n][r] *= all;
+    for (int n = 0; n < NW; ++n) more[0][n] = more[1][n] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
-      for (int n = 0; n < NW; ++n) s[n] = mul4(kt[n][b], ub[b], s[n]);
+      for (int n = 0; n < NW; ++n) more[b % 2][n] = mul4(kt[n][b], ub[b], more[b % 2][n]);
+#pragma unroll
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[n][r] = fmaf(s[n][r], all, more[0][n][r] + more[1][n][r]);
 #pragma unroll
     for (int n = 0; n < NW; ++n) s_s[now ^ 1][(wave * NW + n) * kWave + lane] = s[n];
 #pragma unroll
     for (int b = 0; b < kBlocks - 1; ++b)
-      if (b < wave) o = mul4(p[b], ub[b], o);   // (uniform over the wave)
-    o = lower_mul4(p[kBlocks - 1], u, o, lane);
+      if (b < wave) o2[b] = mul4(p[b], ub[b], o2[b]);   // (uniform over the wave)
+    o2[kBlocks - 1] = lower_mul4(p[kBlocks - 1], u, o2[kBlocks - 1], lane);
+    floatx4 result = sum_of(o) + sum_of(o2);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) result[r] = fmaf(own[r], u[r], result[r]);
     fetch_rest(next);
     if (col_ok) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = t0 + wave * 16 + g * 4 + r;
-        if (t < sp.count) a.out[static_cast<size_t>(sp.first + t) * (static_cast<size_t>(a.H) * a.dv) + static_cast<size_t>(h) * a.dv + col] = o[r] + o2[r];
+        if (t < sp.count) a.out[static_cast<size_t>(sp.first + t) * (static_cast<size_t>(a.H) * a.dv) + static_cast<size_t>(h) * a.dv + col] = result[r];
       }
     }
     src = next;

@@ -20,8 +20,11 @@
 // Sums and products are 32-bit (v_mfma_f32_16x16x4_f32).  The first kernel is bound by a wave's vector instructions (16
 // steps of 96 multiplications and the operands' reads from LDS), the second by its matrix instructions one after the other.
 //
-// Measured at 2,048 tokens of 16 heads of 128: 33 us for the pieces and 73 for the walk, where linear_state.hip takes 703
-// token by token.
+// As in delta_chunks.hip sums run in several short chains: results are 0.9 to 1.0 times as far from 64 bits as those of
+// linear_state.hip, the state 0.8 to 0.95 times (500 to 2,047 tokens; 1.2 to 1.3 times with one or two chains each).
+//
+// Measured at 2,048 tokens of 16 heads of 128: 31 us for the pieces and 74 for the walk (30 and 67 with one or two chains and
+// without the look at values that are not finite), where linear_state.hip takes 703 token by token.
 #include "api.h"
 #include "chunks.h"
 
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
     qp[n] = to_float4(*reinterpret_cast<const uint2*>(&q_s[(wave * 16 + c) * QROW + n * 16 + g * 4])) * a.q_mult;
     kw[n] = to_float4(*reinterpret_cast<const uint2*>(&k_s[(wave * 16 + c) * QROW + n * 16 + g * 4]));
   }
-  float own = 0.f;   // M_cc, by the lane's channels
+  floatx4 own_r{0.f, 0.f, 0.f, 0.f};   // M_cc, by the lane's channels
 #pragma unroll
   for (int n = 0; n < NT; ++n)
 #pragma unroll
@@ -133,17 +136,16 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
       float x = qp[n][r] * kw[n][r];
       const int d = n * 16 + g * 4 + r;
       if (BONUS) x *= d < a.dk ? load_f(a.bonus, a.bonus_dtype, static_cast<size_t>(h) * a.dk + d) : 0.f;
-      own += x;
+      own_r[r] += x;
     }
-  own = sum_over_row_lanes(own);
+  const float own = sum_over_row_lanes((own_r[0] + own_r[1]) + (own_r[2] + own_r[3]));
   float m_c[4] = {0.f, 0.f, 0.f, 0.f};   // M[query 4 g + r][key c] of the block
 #pragma unroll 1
   for (int i4 = 0; i4 < 4; ++i4) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = i4 * 4 + e;
-      floatx4 av[NT];
-      float s = 0.f;
+      floatx4 av[NT], s_r{0.f, 0.f, 0.f, 0.f};
       const float* ap = &a_s[(wave * 16 + i) * AROW + g * 4];
       const bf16* qi = &q_s[(wave * 16 + i) * QROW + g * 4];
 #pragma unroll
@@ -156,7 +158,7 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
       for (int n = 0; n < NT; ++n) {
         const floatx4 q = to_float4(*reinterpret_cast<const uint2*>(qi + n * 16));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s = fmaf(q[r], kw[n][r], s);
+        for (int r = 0; r < 4; ++r) s_r[r] = fmaf(q[r], kw[n][r], s_r[r]);
       }
       if (BONUS && c < i) {
 #pragma unroll
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
 #pragma unroll
         for (int n = 0; n < NT; ++n) qp[n] *= av[n];
       }
-      s = sum_over_row_lanes(s) * a.q_mult;
+      float s = sum_over_row_lanes((s_r[0] + s_r[1]) + (s_r[2] + s_r[3])) * a.q_mult;
       s = c < i ? s : c == i ? own : 0.f;
       if (g == i4) m_c[e] = s;
     }
@@ -194,13 +196,10 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
   // keys of earlier blocks, from the nearest on; the queries take a block's decays on the way
 #pragma unroll 1
   for (int b = wave - 1; b >= 0; --b) {
-    floatx4 x{0.f, 0.f, 0.f, 0.f}, y{0.f, 0.f, 0.f, 0.f};
+    floatx4 x[NT];   // (a chain of products for each 16 channels)
 #pragma unroll
-    for (int n = 0; n < NT; n += 2) {
-      x = mul4(key_s[(b * NT + n) * kWave + lane], qp[n], x);
-      y = mul4(key_s[(b * NT + n + 1) * kWave + lane], qp[n + 1], y);
-    }
-    *reinterpret_cast<floatx4*>(dst + lay.p + (wave * kBlocks + b) * kBlock + lane * 4) = x + y;   // [key 4 g + r][query c]
+    for (int n = 0; n < NT; ++n) x[n] = mul4(key_s[(b * NT + n) * kWave + lane], qp[n], floatx4{0.f, 0.f, 0.f, 0.f});
+    *reinterpret_cast<floatx4*>(dst + lay.p + (wave * kBlocks + b) * kBlock + lane * 4) = sum_of(x);   // [key 4 g + r][query c]
 #pragma unroll
     for (int n = 0; n < NT; ++n) qp[n] *= *reinterpret_cast<const floatx4*>(&blk_s[b][n * 16 + g * 4]);
   }
@@ -273,31 +272,40 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
 #pragma unroll
     for (int n = 0; n < NT; ++n) st[n] = s_s[now][n * kWave + lane];
     // the state behind the piece, for the others to read
+    floatx4 more[NW];   // (summed by itself: 64 products added to the state one by one would round it 64 times)
 #pragma unroll
-    for (int n = 0; n < NW; ++n) s[n] *= all[n];
+    for (int n = 0; n < NW; ++n) more[n] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
-      for (int n = 0; n < NW; ++n) s[n] = mul4(kt[n][b], v[b], s[n]);
+      for (int n = 0; n < NW; ++n) more[n] = mul4(kt[n][b], v[b], more[n]);
+#pragma unroll
+    for (int n = 0; n < NW; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[n][r] = fmaf(s[n][r], all[n][r], more[n][r]);
 #pragma unroll
     for (int n = 0; n < NW; ++n) s_s[now ^ 1][(wave * NW + n) * kWave + lane] = s[n];
     fetch_state(next);
-    floatx4 o{0.f, 0.f, 0.f, 0.f}, o2{0.f, 0.f, 0.f, 0.f};
+    floatx4 o[4], o2[kBlocks];
 #pragma unroll
-    for (int n = 0; n < NT; n += 2) {
-      o = mul4(q[n], st[n], o);
-      o2 = mul4(q[n + 1], st[n + 1], o2);
-    }
+    for (int i = 0; i < 4; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) o2[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NT; n += 4)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = mul4(q[n + i], st[n + i], o[i]);
 #pragma unroll
     for (int b = 0; b < kBlocks - 1; ++b)
-      if (b < wave) o = mul4(p[b], v[b], o);   // (uniform over the wave)
-    o = lower_mul4(p[kBlocks - 1], v_own, o, lane);
+      if (b < wave) o2[b] = mul4(p[b], v[b], o2[b]);   // (uniform over the wave)
+    o2[kBlocks - 1] = lower_mul4(p[kBlocks - 1], v_own, o2[kBlocks - 1], lane);
+    const floatx4 result = sum_of(o) + sum_of(o2);
     fetch_rest(next);
     if (col_ok) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = t0 + wave * 16 + g * 4 + r;
-        if (t < sp.count) a.out[static_cast<size_t>(sp.first + t) * (static_cast<size_t>(a.H) * a.dv) + static_cast<size_t>(h) * a.dv + col] = o[r] + o2[r];
+        if (t < sp.count) a.out[static_cast<size_t>(sp.first + t) * (static_cast<size_t>(a.H) * a.dv) + static_cast<size_t>(h) * a.dv + col] = result[r];
       }
     }
     src = next;
