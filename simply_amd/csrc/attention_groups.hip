@@ -92,6 +92,15 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
   int lo_g, hi_g, slot = 0;
   if (!group_keys(units, u0, kUnits, window, &lo_g, &hi_g, &slot)) return;   // no rows at all
   lo_g = __builtin_amdgcn_readfirstlane(lo_g), hi_g = __builtin_amdgcn_readfirstlane(hi_g);
+  // where the first unit's keys end and where the last one's begin: every unit sees the keys between whole
+  int hi_first = hi_g, lo_last_unit = lo_g;
+  for (int w = 0; w < kUnits; ++w) {
+    const SeqMeta m = units[u0 + w];
+    if (m.q_len <= 0) continue;
+    hi_first = min(hi_first, m.pos0 + m.q_len);
+    if (window > 0) lo_last_unit = max(lo_last_unit, m.pos0 - window + 1);
+  }
+  hi_first = __builtin_amdgcn_readfirstlane(hi_first), lo_last_unit = __builtin_amdgcn_readfirstlane(lo_last_unit);
   const int tile0 = lo_g / kTile, tile1 = (hi_g + kTile - 1) / kTile;
   const int num_chunks = key_chunks(lo_g, hi_g, sh.chunk_tiles);
   if (split >= num_chunks) return;   // (the same for the whole workgroup)
@@ -214,15 +223,45 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
           for (int v = 0; v < 4; ++v) acc[w][j][v] *= alpha[w];
     }
     const int key0 = tile * kTile;
-    if (key0 + kTile > hi_g || key0 < lo_g) {   // keys that no row may use (unwritten, given back) count as 0
+    if (__builtin_expect(key0 + kTile <= hi_first && key0 >= lo_last_unit, 1)) return;
+    // keys that no row may use (unwritten, given back) count as 0
+    constexpr uint32_t kExponents = 0x7f807f80u;
+    typedef __attribute__((ext_vector_type(4))) uint32_t Pairs;   // of neighbouring keys
+    auto between = [&](int lo, int hi) __attribute__((always_inline)) {
+      Pairs m;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = key0 + grp * 8 + 2 * i;
+        m[i] = (key >= lo && key < hi ? 0xffffu : 0u) | (key + 1 >= lo && key + 1 < hi ? 0xffff0000u : 0u);
+      }
+      return m;
+    };
+    const Pairs used = between(lo_g, hi_g);
+    bool odd = false;
+#pragma unroll
+    for (int j = 0; j < VPW; ++j) {
+      const Pairs v = __builtin_bit_cast(Pairs, vf[j]) & used;
+      vf[j] = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t e = v[i] & kExponents;
+        odd |= (e & 0xffffu) == (kExponents & 0xffffu) || e >> 16 == kExponents >> 16;
+      }
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) == 0, 1)) return;
+    // Keys that some units see and others do not, with values that are not finite, which a probability of zero does not
+    // take out: each unit's products here, without the keys that it does not see, and none later.
+#pragma unroll
+    for (int w = 0; w < kUnits; ++w) {
+      const SeqMeta m = units[u0 + w];
+      const Pairs seen = between(window > 0 ? m.pos0 - window + 1 : 0, m.pos0 + m.q_len);
 #pragma unroll
       for (int j = 0; j < VPW; ++j)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = key0 + grp * 8 + e;
-          if (key >= hi_g || key < lo_g) vf[j][e] = to_bf16_raw(0.f);
-        }
+        acc[w][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, __builtin_bit_cast(Pairs, vf[j]) & seen),
+                                                            pf[w], acc[w][j], 0, 0, 0);
     }
+#pragma unroll
+    for (int j = 0; j < VPW; ++j) vf[j] = bf16x8{};
   };
   auto second = [&](int from, int to) __attribute__((always_inline)) {
 #pragma unroll

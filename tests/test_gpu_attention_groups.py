@@ -76,3 +76,36 @@ def test_groups(H, K, hd, hv, page, window, cases):
     assert (error <= (2.0 ** -8 + 2.0 ** -12) * room[3:] + 2.0 ** -8 * want[3:].abs()).all(), (error / room[3:]).max()
     again = run().double().cpu().reshape(T, H, hv)
     assert torch.equal(again, got)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("H,hd,hv,window,at", [(16, 576, 512, None, 41), (16, 192, 128, None, 701), (16, 288, 256, 50, 63),
+                                               (8, 160, 128, 33, 96), (4, 128, 128, None, 100)])
+def test_groups_keep_special_values(H, hd, hv, window, at, bad):
+    """A value that is not finite reaches the rows that see its key (rows of a unit together) and changes no bit of others."""
+    from simply_amd.kernels import lib as _lib, ops
+
+    g, T, page = torch.Generator().manual_seed(17), 703, 16
+    gs, per = ops.attention_group_size(), 16 // ops.attention_maps_heads_per_unit(H, 1)
+    pages = -(-T // page)
+    table = torch.arange(pages, dtype=torch.int32)[None].cuda()
+    k_pages = torch.randn(pages, 1, page, hd, generator=g).bfloat16().cuda()
+    v_pages = torch.randn(pages, 1, hv, page, generator=g).bfloat16().cuda()
+    q = torch.randn(T, H * hd, generator=g).bfloat16().cuda()
+    count = -(-(-(-T // per)) // gs) * gs
+    units = torch.tensor([(0, min(u * per, T), min(T - min(u * per, T), per), min(u * per, T)) for u in range(count)],
+                         dtype=torch.int32).cuda()
+    assert _lib.load().sa_paged_attention_groups_pays(count, H, 1, window or 0, T, per)
+    run = lambda: ops.paged_attention_maps_units(q, k_pages, v_pages, table, units, 0, count, H, scale=hd ** -0.5, window=window,
+                                                 max_kv_len=T, max_q_len=per, grouped=count).reshape(T, H, hv)
+    want = run()
+    entry = hv - 19
+    v_pages[at // page, 0, entry, at % page] = bad
+    got = run()
+    row = torch.arange(T, device="cuda")
+    sees = (row >= at) & ((row - at) < (window or T))
+    of_unit = ((row // per * per + per - 1).clamp(max=T - 1) >= at) & (row // per * per - at < (window or T))
+    assert not torch.isfinite(got[sees][:, :, entry]).any()
+    same = torch.ones(T, H, hv, dtype=torch.bool, device="cuda")
+    same[of_unit, :, entry] = False
+    assert torch.isfinite(want).all() and torch.equal(got[same], want[same])
