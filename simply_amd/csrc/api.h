@@ -179,6 +179,9 @@ int sa_paged_attention_decode(const void* q, int64_t q_stride, const void* k_pag
                               int seq_count, void* out, int64_t out_stride, int H, int Kh, int hd, int page_size,
                               int window, float soft_cap, int max_kv_len, int max_q_len, int num_splits,
                               void* workspace, int64_t workspace_bytes, hipStream_t stream);
+// Whether sa_paged_attention_decode has a way of its own for requests whose lengths differ widely (num_splits < 0) at these
+// numbers; where it has none, num_splits < 0 is the same as 0.
+int sa_paged_attention_decode_evens(int seq_count, int window, int max_kv_len);
 
 // sa_paged_attention_decode for callers that cannot allocate device memory (code under HIP graph capture, tight
 // serving loops, harnesses that forbid hipMalloc): the same kernels, the same result, but the partial results of

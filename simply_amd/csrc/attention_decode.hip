@@ -546,6 +546,15 @@ static int decode_max_tiles(int window, int max_kv_len) {
   return (span + kTile - 1) / kTile + 1;
 }
 
+}  // namespace sa
+
+// Whether a launch over so many requests, whose keys max_kv_len bounds, has a way of its own for lengths that differ widely.
+extern "C" int sa_paged_attention_decode_evens(int seq_count, int window, int max_kv_len) {
+  return seq_count > 1 && sa::decode_max_tiles(window, max_kv_len) >= 48;
+}
+
+namespace sa {
+
 // Into how many ranges the keys of each request are cut (num_splits > 0 asks for that many; < 0: the lengths differ widely,
 // which paged_attention_decode answers with ranges of equal size where it can).
 int paged_attention_decode_ranges(int seq_count, int Kh, int window, int max_kv_len, int num_splits) {
@@ -590,8 +599,8 @@ int paged_attention_decode(const void* q, int64_t q_stride, const void* k_pages,
   // Requests whose lengths differ widely (num_splits < 0; the callers' rule stands at StepContext.decode_splits), where
   // the longest has 1,500 keys or more: ranges of about equal size, as many as one for every unit and one for every CU
   // (384 and 512 instead of 256 on top measured alike, 1,024 up to 15 % slower), of 16 tiles at least.
-  const int max_tiles = decode_max_tiles(window, max_kv_len);
-  if (num_splits < 0 && seq_count > 1 && max_tiles >= 48) {
+  if (num_splits < 0 && sa_paged_attention_decode_evens(seq_count, window, max_kv_len)) {
+    const int max_tiles = decode_max_tiles(window, max_kv_len);
     const int workgroups = units + 256, least = max_tiles / 64 > 16 ? max_tiles / 64 : 16;
     const size_t index_bytes = (static_cast<size_t>(units) * sizeof(int2) + 255) / 256 * 256;
     const size_t slots = static_cast<size_t>(workgroups) * 16 * (hd + kRowExtra) * sizeof(float);

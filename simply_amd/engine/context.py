@@ -44,6 +44,8 @@ class StepContext:
     #: set for a step whose launches are recorded and replayed for later steps: the most keys that any step that
     #: replays them may have (kernels size their plans by `max_kv_len`, which is then this bound)
     kv_bound: int = 0
+    #: (window, key heads) of the layers that asked for `decode_splits`
+    splits_asked: set = dataclasses.field(default_factory=set)
     #: brings an integer array that a part makes for the step to the device without waiting for the device (the
     #: executor's pinned block); None: a plain copy
     to_device: Callable[[np.ndarray], torch.Tensor] | None = None
@@ -64,21 +66,26 @@ class StepContext:
 
     def decode_splits(self, window: int | None, count: int, kv_heads: int) -> int:
         """`num_splits` for `paged_attention_decode` over the first `count` requests: -1 if their lengths differ so widely
-        that cutting each into as many ranges leaves much of the GPU waiting for the longest, else 0: what the ranges
-        hold, counted in ranges of the longest.  A launch of more than 128 (request, key head) has one range for each, one
-        of fewer about 256 in all.  (Key heads x requests as long as the longest, us whole and in ranges of equal size: of
-        more than 128, 39 of them 169 and 83, 67 187 and 128, 123 135 and 123 or 243 and 211, 136 57 and 64, 145 76 and 84; of
-        fewer, 47 178 and 100, 70 34 and 28, 75 34 and 29, 99 17 and 25, 112 37 and 34, 115 37 and 46.)"""
-        if count < 2:
-            return 0
-        key = ("splits", window, count, kv_heads)
+        that cutting each into as many ranges leaves much of the GPU waiting for the longest, else 0 (also where the launch
+        has but one way): what the ranges hold, counted in ranges of the longest.  A launch of more than 128 (request, key
+        head) has one range for each, one of fewer about 256 in all.  (Key heads x requests as long as the longest, us whole
+        and in ranges of equal size: of more than 128, 39 of them 169 and 83, 47 178 and 100, 67 187 and 128, 123 135 and 123
+        or 243 and 211, 136 57 and 64, 145 76 and 84; of fewer, 70 34 and 28, 75 34 and 29, 99 17 and 25, 112 37 and 34, 115
+        37 and 46.)"""
+        self.splits_asked.add((window or 0, kv_heads))
+        key = ("splits", window or 0, count, kv_heads)
         if key not in self._units:
-            seen = np.add(self.seq_starts[:count], self.q_lens[:count])
-            if window:
-                seen = np.minimum(seen, window)
-            alike = int(seen.sum()) / max(int(seen.max()), 1)   # requests as long as the longest that hold as many keys
-            units = count * kv_heads
-            self._units[key] = -1 if (alike * kv_heads < 130 if units > 128 else 256 * alike < 80 * count) else 0
+            from ..kernels import ops
+
+            splits = 0
+            if count > 1 and ops.decode_evens(count, window, self.max_kv_len):
+                seen = np.add(self.seq_starts[:count], self.q_lens[:count])
+                if window:
+                    seen = np.minimum(seen, window)
+                alike = int(seen.sum()) / max(int(seen.max()), 1)   # requests as long as the longest that hold as many keys
+                units = count * kv_heads
+                splits = -1 if (alike * kv_heads < 130 if units > 128 else 256 * alike < 80 * count) else 0
+            self._units[key] = splits
         return self._units[key]
 
     def short_requests(self, max_tokens: int) -> tuple[int, int]:

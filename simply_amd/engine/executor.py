@@ -17,7 +17,6 @@ import torch
 from ..cache import CacheManager, pages_for_memory
 from ..config import EngineConfig
 from ..models import DecoderModel
-from ..parts.base import PagedKVNeed
 from .context import GroupStep, StepContext
 
 
@@ -78,12 +77,11 @@ class Executor:
         self._extra_copied = torch.cuda.Event() if self._on_gpu else None
         self._extra_used = 0
         # decode-only steps (one token per request) are captured once per number of requests, order of magnitude of the
-        # context and whether the requests' lengths differ widely (the attention kernels choose their cut of the keys when
-        # they are recorded) and replayed
+        # context and, where a kernel asks for it, whether the requests' lengths differ widely (the attention kernels choose
+        # their cut of the keys when they are recorded) and replayed
         self._graphs: dict[tuple, torch.cuda.CUDAGraph] = {}
         self._graph_pool = None
-        parts = [n for need, _ in needs for n in getattr(need, "parts", (need,))]
-        self._kv_kinds = sorted({(n.window or 0, n.num_kv_heads) for n in parts if isinstance(n, PagedKVNeed)})
+        self._split_kinds: tuple[tuple[int, int], ...] = ()   # of the layers that ask how to cut the keys (`_splits`)
         # where every recorded step writes its logits, [batch_size, vocab] float32: made at the first such step
         self._graph_logits: torch.Tensor | None = None
         # several decode steps in a row without the host (decode_many): what was drawn in each, and the step count
@@ -127,14 +125,16 @@ class Executor:
         first step with a new key runs eagerly (kernels choose their plans, scratch buffers get allocated) and is
         this call's result; the recording that follows executes nothing (a mixer that keeps a state of its own would
         otherwise advance it twice)."""
-        key = (T, self._context_bucket(ctx), self._splits(ctx))
-        ctx.kv_bound = 1 << key[1]
+        bucket = self._context_bucket(ctx)
+        ctx.kv_bound = 1 << bucket
+        key = (T, bucket, self._splits(ctx))
         out = self._shared_logits()[:T]
         graph = self._graphs.get(key)
         if graph is not None:
             graph.replay()
             return out
         logits = self.model.forward(self._dev[:T], ctx, self.cache.views, logit_rows, logits_out=out)
+        key = (T, bucket, self._splits(ctx))   # (a first step has shown which layers ask)
         self._graphs[key] = self._record(
             lambda: self.model.forward(self._dev[:T], ctx, self.cache.views, logit_rows, logits_out=out))
         return logits
@@ -164,8 +164,10 @@ class Executor:
 
     def _splits(self, ctx: StepContext) -> tuple[int, ...]:
         """How the attention layers of a decode-only step cut the keys (`StepContext.decode_splits`): a recorded step serves
-        steps whose layers would choose alike."""
-        return tuple(ctx.decode_splits(window, ctx.num_seqs, heads) for window, heads in self._kv_kinds)
+        steps whose layers would choose alike.  Layers whose kernels have no such choice do not ask, and take no part."""
+        if not ctx.splits_asked.issubset(self._split_kinds):
+            self._split_kinds = tuple(sorted(ctx.splits_asked.union(self._split_kinds)))
+        return tuple(ctx.decode_splits(window, ctx.num_seqs, heads) for window, heads in self._split_kinds)
 
     # ------------------------------------------------------------------ the step
     def step(self, entries: Sequence[StepEntry]) -> torch.Tensor | None:
@@ -250,15 +252,15 @@ class Executor:
                 ops.decode_slots(dev[cap:cap + T], dev[2 * cap:2 * cap + T], table, self.cache.page_size, slots)
 
         ops.fill_(counter, 0)
-        key = ("many", B, self._context_bucket(ctx, num_steps - 1), max_steps, id(sampler), sampler.modes,
-               self._splits(ctx))
-        ctx.kv_bound = 1 << key[2]
-        graph = self._graphs.get(key)
+        bucket = self._context_bucket(ctx, num_steps - 1)
+        ctx.kv_bound = 1 << bucket
+        key = ("many", B, bucket, max_steps, id(sampler), sampler.modes)
+        graph = self._graphs.get((*key, self._splits(ctx)))
         launched = 0
         if graph is None:
             one_step()   # once eagerly (it counts as the first step), then recorded
             launched = 1
-            graph = self._graphs[key] = self._record(one_step)
+            graph = self._graphs[(*key, self._splits(ctx))] = self._record(one_step)
         if on_step is None:
             lookahead = chunk = num_steps
         if self._side_stream is None:

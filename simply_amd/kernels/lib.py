@@ -159,6 +159,8 @@ def load() -> ctypes.CDLL:
         lib.sa_gemm_plan.restype = c_int
         lib.sa_expert_tiles_max.argtypes = [_I, _I, _I]
         lib.sa_expert_tiles_max.restype = c_int
+        lib.sa_paged_attention_decode_evens.argtypes = [_I, _I, _I]
+        lib.sa_paged_attention_decode_evens.restype = c_int
         lib.sa_expert_tile_rows.argtypes = [_I, _I, _I, _I, _I, _L, _P]
         lib.sa_expert_tile_rows.restype = c_int
         lib.sa_philox4x32_10.argtypes = [_P, _P, _P]

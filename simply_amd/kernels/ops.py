@@ -677,6 +677,12 @@ def decode_attention_takes(q: torch.Tensor, k_pages: torch.Tensor, num_heads: in
         int(num_heads), int(Kh), int(hd), int(page_size), int(max_q_len), q.stride(0), _ptr(q)))
 
 
+def decode_evens(seq_count: int, window: int | None, max_kv_len: int) -> bool:
+    """Whether `paged_attention_decode` has a way of its own for so many requests whose lengths differ widely
+    (num_splits = -1); where it has none, -1 is the same as 0."""
+    return bool(_lib.load().sa_paged_attention_decode_evens(int(seq_count), int(window or 0), int(max_kv_len)))
+
+
 def attention_f32_takes(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, num_heads: int) -> bool:
     """Whether `paged_attention_f32` takes these sizes."""
     _, Kh, page_size, hd = k_pages.shape

@@ -63,3 +63,43 @@ def test_decode_uneven(H, K, hd, page, window, q_len, extra, lens):
     assert torch.equal(*results)
     error = (results[0] - want).abs()
     assert (error <= (2.0 ** -8 + 2.0 ** -11) * room + 2.0 ** -8 * want.abs()).all(), (error / room).max()
+
+
+def test_recorded_steps_follow_the_lengths(tmp_path, monkeypatch):
+    """A recorded step that cuts keys into ranges of equal size reads the lengths when it is replayed: 20 decode steps across
+    2,560 keys, from where on the longest request has a sixth range (its 81st tile of 32 keys), then requests of like lengths,
+    which have a recording of their own, then the first ones' again.  The same bits as without recordings."""
+    import tiny
+    from simply_amd.config import EngineConfig
+    from simply_amd.engine import Executor, StepEntry
+    from simply_amd.engine.loading import load_model
+
+    d = dict(tiny.TINY_D, max_position_embeddings=4096, layer_types=["full_attention", "sliding_attention", "full_attention"])
+    folder = tiny.write_config_model(d, str(tmp_path / "m"), seed=9, dtype=torch.bfloat16, std=0.15)
+
+    def decode(graphs):
+        model, _ = load_model(folder, torch.bfloat16, "cuda:0")
+        ex = Executor(model, EngineConfig(activation_dtype="bfloat16", batch_size=7, max_seq_len=4096, max_num_issue_tokens=2048,
+                                          total_num_pages=1300, device="cuda:0", use_graphs=graphs))
+        out = []
+        for lens, steps in (([2550] + [20] * 6, 20), ([2550] * 7, 3), ([2555] + [20] * 6, 3)):
+            for i, n in enumerate(lens):
+                ex.add_request(i)
+                t = tiny.random_tokens(n, d["vocab_size"], i)
+                for a in range(0, n, 2048):
+                    ex.step([StepEntry(i, t[a:a + 2048])])
+            for k in range(steps):
+                out.append(ex.step([StepEntry(i, [7 * k + i], [0]) for i in range(7)]).clone())
+            for i in range(7):
+                ex.finish_request(i)
+        return torch.stack(out), ex
+
+    from simply_amd.kernels import ops
+
+    asked, plain = [], ops.paged_attention_decode
+    monkeypatch.setattr(ops, "paged_attention_decode", lambda *a, **kw: (asked.append(kw.get("num_splits")), plain(*a, **kw))[1])
+    want, _ = decode(False)
+    assert -1 in asked and 0 in asked
+    got, ex = decode(True)
+    assert torch.equal(got, want) and torch.isfinite(want).all()
+    assert len(ex._graphs) == 2 and {k[-1] for k in ex._graphs} == {(-1, 0), (0, 0)}, list(ex._graphs)
