@@ -361,32 +361,47 @@ static void launch_tiles(const Args& a, int tm, int nseg, float* planes, hipStre
   else gemm_f32_sum_kernel<EPI, 1><<<blocks, 256, 0, stream>>>(a, planes, nseg);
 }
 
+struct Plan {
+  int tile_rows;   // 64 or 128; 16: few rows
+  bool cut;
+};
+// The tile and whether K is cut over workgroups: rounds over the 256 CUs times a tile's products at the share of a CU's
+// 614 GFLOP/s that the tile reaches, and for cut tiles the planes written and read at 4 TB/s and one launch more.
+static Plan plan_for(int M, int N, int K, bool gated, int nseg, size_t workspace_bytes) {
+  Plan best{16, false};
+  if (M <= 16) return best;
+  const double NW = gated ? 2.0 * N : N;
+  const size_t plane_bytes = static_cast<size_t>(nseg) * M * static_cast<size_t>(NW) * sizeof(float);
+  double best_us = 1e30;
+  for (int tile_rows = 128; tile_rows >= 64; tile_rows /= 2) {
+    const double rows = tile_rows, tiles = ceil(M / rows) * ceil(NW / rows);
+    const double tile_us = 2.0 * rows * rows * K / (0.614e6 * (tile_rows == 128 ? 0.85 : 0.7));
+    for (int cut = 0; cut < 2; ++cut) {
+      if (cut && (nseg == 1 || plane_bytes > workspace_bytes)) continue;
+      const double us = cut ? ceil(tiles * nseg / 256.0) * tile_us / nseg + 2.0 * plane_bytes / 4e6 + 5.0
+                            : ceil(tiles / 256.0) * tile_us;
+      if (us < best_us) best_us = us, best = Plan{tile_rows, cut != 0};
+    }
+  }
+  return best;
+}
+
+// Segments of K, and their length.
+static int segments(int K, int* length) {
+  *length = (K + kSegments * 16 - 1) / (kSegments * 16) * 16;
+  return (K + *length - 1) / *length;
+}
+
 template <int EPI>
 static void launch(const Args& a, int nseg, float* workspace, size_t workspace_bytes, hipStream_t stream) {
-  if (a.M <= 16) {
+  const Plan plan = plan_for(a.M, a.N, a.K, EPI == 1, nseg, workspace != nullptr ? workspace_bytes : 0);
+  if (plan.tile_rows == 16) {
     const int blocks = (a.N + 15) / 16;
     if (a.M <= 8) gemm_f32_few_kernel<EPI, 8><<<blocks, 64 * nseg, 0, stream>>>(a);
     else gemm_f32_few_kernel<EPI, 16><<<blocks, 64 * nseg, 0, stream>>>(a);
     return;
   }
-  // The tile and whether K is cut over workgroups: rounds over the 256 CUs times a tile's products at the share of a CU's
-  // 614 GFLOP/s that the tile reaches, and for cut tiles the planes written and read at 4 TB/s and one launch more.
-  const double NW = EPI == 1 ? 2.0 * a.N : a.N;
-  const size_t plane_bytes = static_cast<size_t>(nseg) * a.M * static_cast<size_t>(NW) * sizeof(float);
-  int best_tm = 4;
-  bool best_cut = false;
-  double best = 1e30;
-  for (int tm = 4; tm >= 2; tm -= 2) {
-    const double rows = 32.0 * tm, tiles = ceil(a.M / rows) * ceil(NW / rows);
-    const double tile_us = 2.0 * rows * rows * a.K / (0.614e6 * (tm == 4 ? 0.85 : 0.7));
-    for (int cut = 0; cut < 2; ++cut) {
-      if (cut && (nseg == 1 || workspace == nullptr || plane_bytes > workspace_bytes)) continue;
-      const double us = cut ? ceil(tiles * nseg / 256.0) * tile_us / nseg + 2.0 * plane_bytes / 4e6 + 5.0
-                            : ceil(tiles / 256.0) * tile_us;
-      if (us < best) best = us, best_tm = tm, best_cut = cut != 0;
-    }
-  }
-  launch_tiles<EPI>(a, best_tm, nseg, best_cut ? workspace : nullptr, stream);
+  launch_tiles<EPI>(a, plan.tile_rows / 32, nseg, plan.cut ? workspace : nullptr, stream);
 }
 
 }  // namespace f32
@@ -401,8 +416,7 @@ int gemm_f32(const float* A, int64_t lda, const float* W, const float* W2, float
              int act, float cap, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   f32::Args a;
   a.A = A, a.W = W, a.W2 = W2, a.C = C, a.lda = lda, a.ldc = ldc, a.M = M, a.N = N, a.K = K, a.act = act, a.cap = cap;
-  a.seg = (K + f32::kSegments * 16 - 1) / (f32::kSegments * 16) * 16;
-  const int nseg = (K + a.seg - 1) / a.seg;
+  const int nseg = f32::segments(K, &a.seg);
   float* ws = static_cast<float*>(workspace);
   if (epi == kEpilogueGated) f32::launch<1>(a, nseg, ws, workspace_bytes, stream);
   else if (epi == kEpilogueSoftCap) f32::launch<2>(a, nseg, ws, workspace_bytes, stream);
@@ -411,3 +425,12 @@ int gemm_f32(const float* A, int64_t lda, const float* W, const float* W2, float
 }
 
 }  // namespace sa
+
+// Which way M rows go: 16 (few rows), or a tile's rows (64 or 128), plus 1000 where K is cut over workgroups.
+extern "C" int sa_gemm_f32_plan(int M, int N, int K, int gated, int64_t workspace_bytes) {
+  if (M < 1 || N < 1 || K < 1) return 0;
+  int length;
+  const int nseg = sa::f32::segments(K, &length);
+  const sa::f32::Plan plan = sa::f32::plan_for(M, N, K, gated != 0, nseg, workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0);
+  return plan.tile_rows + (plan.cut ? 1000 : 0);
+}

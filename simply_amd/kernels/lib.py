@@ -157,6 +157,8 @@ def load() -> ctypes.CDLL:
             fn.restype = c_int
         lib.sa_gemm_plan.argtypes = [_I, _I, _I, _I, _I, _L, _P]
         lib.sa_gemm_plan.restype = c_int
+        lib.sa_gemm_f32_plan.argtypes = [_I, _I, _I, _I, _L]
+        lib.sa_gemm_f32_plan.restype = c_int
         lib.sa_expert_tiles_max.argtypes = [_I, _I, _I]
         lib.sa_expert_tiles_max.restype = c_int
         lib.sa_paged_attention_decode_evens.argtypes = [_I, _I, _I]

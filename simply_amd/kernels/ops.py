@@ -532,6 +532,13 @@ def gemm_plan(M: int, N: int, K: int, *, gated: bool = False, soft_cap: bool = F
     return kernel, {"skinny": us[0], "tiled": us[1], "wide": us[2]}
 
 
+def gemm_f32_plan(M: int, N: int, K: int, *, gated: bool = False) -> tuple[int, bool]:
+    """How `gemm` takes M rows of 32-bit operands on the matrix cores: the rows of a tile (16: the kernel for few rows) and
+    whether K is cut over workgroups.  A host function."""
+    plan = _lib.load().sa_gemm_f32_plan(int(M), int(N), int(K), int(gated), WORKSPACE_BYTES)
+    return plan % 1000, plan >= 1000
+
+
 def gemm_normed_takes(M: int, w) -> bool:
     """Whether `gemm_normed` takes M rows against the weight `w`."""
     if not isinstance(w, TiledWeight) or not w.data.is_cuda:

@@ -15,7 +15,7 @@ def draw(shape, seed, std=1.0):
 
 @pytest.mark.parametrize("N,K", [(16, 4), (7, 32), (100, 36), (130, 256), (333, 260), (96, 2304), (2304, 100)])
 def test_products(N, K):
-    """Few rows, tiles and tiles cut over K, plain, gated and soft-capped: each within the bound on a sum of K products in
+    """Few rows and tiles of 64 rows, whole and cut over K, plain, gated and soft-capped: each within the bound on a sum of K products in
     any order, (K + 2) eps sum |a| |w|; and a row's result is the same to the bit whichever of the ways it went."""
     from simply_amd.kernels import ops
 
@@ -41,6 +41,35 @@ def test_products(N, K):
     wide, out = draw((20, K + 24), 4), torch.zeros(20, N + 3, device="cuda")
     got = ops.gemm(wide[:, 8:8 + K], w, out=out[:, :N])
     assert torch.equal(got, ops.gemm(wide[:, 8:8 + K].contiguous(), w)) and not out[:, N:].any()
+
+
+@pytest.mark.parametrize("M,N,K,gated,cut", [(1000, 3135, 260, False, False), (1000, 1570, 260, True, False),
+                                             (333, 1101, 1028, False, True), (333, 1100, 1028, False, True),
+                                             (333, 581, 1028, True, True), (333, 580, 1028, True, True)])
+def test_products_in_tiles_of_128_rows(M, N, K, gated, cut):
+    """Tiles of 128 rows, whole and cut over K, the last rows and columns of their tiles missing, segments that end in the
+    middle of a stage of 32 columns (48 and 144 columns long): bounds as above, and the bits of the kernel for few rows."""
+    from simply_amd.kernels import ops
+
+    assert ops.gemm_f32_plan(M, N, K, gated=gated) == (128, cut) and ops.gemm_f32_plan(5, N, K, gated=gated) == (16, False)
+    a, w, w2 = draw((M, K), 11), draw((N, K), 12, 0.1), draw((N, K), 13, 0.1)
+    kw = dict(w2=w2, activation=ops.ACT_SILU) if gated else {}
+    got = ops.gemm(a, w, **kw)
+    x, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    bound = (K + 2) * EPS * size
+    if gated:
+        up, up_bound = a.double() @ w2.double().T, (K + 2) * EPS * (a.double().abs() @ w2.double().abs().T)
+        want = torch.nn.functional.silu(x) * up
+        bound = 1.1 * bound * up.abs() + x.abs() * up_bound + 8 * EPS * want.abs()
+    else:
+        want = x
+    assert ((got.double() - want).abs() <= bound).all()
+    for rows in (slice(0, 5), slice(126, 131), slice(M - 5, M)):
+        assert torch.equal(ops.gemm(a[rows], w, **kw), got[rows])
+    if not gated:
+        capped = ops.gemm(a, w, soft_cap=2.0)
+        assert ((capped.double() - 2.0 * torch.tanh(want / 2.0)).abs() <= bound + 8 * EPS * 2.0).all()
+        assert torch.equal(ops.gemm(a[M - 5:], w, soft_cap=2.0), capped[M - 5:])
 
 
 def test_products_keep_special_values():
