@@ -175,6 +175,60 @@ def test_errors_no_larger_than_token_by_token(T, H):
     no_larger((one, s1), (ops.linear_chunks(p, *at, 1.0, g, H, d, d, s2, meta, 1, 0, T, bonus=u, out=torch.empty_like(one)), s2), want)
 
 
+def cut_rows(takes, pieces):
+    """The bytes of a workspace for so many pieces, found through the library's own answer (`takes(bytes)`: one piece more than
+    requests at least)."""
+    lo, hi = 1, 1 << 28
+    while lo < hi:
+        lo, hi = (lo, (lo + hi) // 2) if takes((lo + hi) // 2) else ((lo + hi) // 2 + 1, hi)
+    return lo // 6 * pieces   # (five requests)
+
+
+@pytest.mark.parametrize("room", [1, 2, 3])
+def test_rows_in_portions_where_the_workspace_is_small(room):
+    """Room for 64, 128 or 192 rows at a time: portions end within requests, between them and at a remainder, and a request's
+    state goes through memory on the way.  Bounds as for whole steps."""
+    from simply_amd.kernels import lib as _lib, ops
+
+    H, G, dk, dv, before, counts = 2, 1, 40, 24, 3, [1, 63, 64, 30, 141]
+    lib, T = _lib.load(), 3 + sum(counts)
+    meta = [(4 - i, before + sum(counts[:i]), n, 0) for i, n in enumerate(counts)]
+    dev_meta = torch.tensor(meta, dtype=torch.int32).cuda()
+    state = normal((5, H * dk * dv), 121)
+    ptr, stream = ops._ptr, ops._stream
+
+    def check(out, one, want, s2, s1, want_state):
+        assert not out[:before].any()
+        for got, ref, plain in ((out[before:], want[before:], one[before:]), (s2, want_state, s1)):
+            err, base, top = ((x.double().cpu() - ref).abs().max() for x in (got, plain, torch.zeros_like(got)))
+            assert err <= 3 * base and err <= 1e-5 * top, (float(err), float(base), float(top))
+
+    C = 2 * G * dk + H * dv
+    qkv = normal((T, C), 122)
+    heads = qkv[:, :2 * G * dk].reshape(T, 2 * G, dk)
+    qkv[:, :2 * G * dk] = (heads / heads.square().sum(-1, keepdim=True).sqrt()).reshape(T, -1)
+    gates = torch.cat([uniform((T, H), 123), uniform((T, H), 124, 0.9, 1.0)], 1)
+    want, want_state = delta_64(qkv, gates, state, meta, H, G, dk, dv)
+    s1, s2, x, g, out = state.cuda(), state.cuda(), qkv.cuda(), gates.cuda(), torch.zeros(T, H * dv, device="cuda")
+    one = ops.delta_rule(x, g, s1, dev_meta, 5, H, G, dk, dv)
+    size = cut_rows(lambda b: lib.sa_delta_chunks_takes(C, G, H, dk, dv, state.stride(0), 5, b), 5 + room)
+    ws = torch.full((size,), 255, dtype=torch.uint8, device="cuda")
+    _lib.call("sa_delta_chunks", ptr(x), C, G, dk, dv, ptr(g), H, ptr(s2), s2.stride(0), ptr(dev_meta), 5, before, T - before,
+              max(counts), ptr(out), ptr(ws), size, stream())
+    check(out, one, want, s2, s1, want_state)
+
+    at = (0, H * dk, 2 * H * dk)
+    proj, decay, bonus = normal((T, 2 * H * dk + H * dv), 125).bfloat16(), uniform((T, H * dk), 126, 0.5, 1.0), normal((H * dk,), 127)
+    want, want_state = linear_64(proj, at, 1.0, decay, bonus, state, meta, H, dk, dv)
+    s1, s2, p, g, u, out = state.cuda(), state.cuda(), proj.cuda(), decay.cuda(), bonus.cuda(), torch.zeros(T, H * dv, device="cuda")
+    one = ops.linear_state(p, *at, 1.0, g, False, H, dk, dv, False, s1, dev_meta, 5, bonus=u)
+    size = cut_rows(lambda b: lib.sa_linear_chunks_takes(H, dk, dv, at[0], at[1], p.stride(0), g.stride(0), state.stride(0), 5, b), 5 + room)
+    ws = torch.full((size,), 255, dtype=torch.uint8, device="cuda")
+    _lib.call("sa_linear_chunks", ptr(p), p.stride(0), *at, 1.0, ptr(g), g.stride(0), 0, 0, 0.0, ptr(u), 0, H, dk, dv, ptr(s2),
+              s2.stride(0), ptr(dev_meta), 5, before, T - before, max(counts), ptr(out), ptr(ws), size, stream())
+    check(out, one, want, s2, s1, want_state)
+
+
 def special_values(run, T, H, dv, value_at, meta, token, bad):
     """`run(values)` -> (out, state).  A value of head 1, column 2 of `token` that is not finite changes that column of that
     head of its own request from `token` on, where nothing is finite any more, and no other bit."""
