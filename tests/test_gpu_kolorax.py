@@ -99,6 +99,62 @@ def test_long_portions_and_pages_of_sixteen(tmp_path, dtype):
     cases.batches_match_alone(tmp_path / "b", DEV, "aligned", dtype, page_size=16)
 
 
+@pytest.mark.parametrize("length", [150, 301])
+def test_prompts_with_the_choices_that_they_made(tmp_path, monkeypatch, length):
+    """A router that is close moves a token to another expert, and its logits far more than the rounding of everything else,
+    which would hide a mistake of that size.  So the plain implementation takes the engine's own choices, and so does a run of
+    the kernels' plain references with bfloat16 rounding, which says how far off roundings alone are: the engine's median row
+    is off by at most 1.5 times that run's, its worst row by twice that run's.  And the choices are the plain implementation's
+    own but for a few (one in twenty), each between scores within the same distance of one another."""
+    import torch_ops
+
+    d = cases.write_model("aligned", str(tmp_path / "m"), dtype=torch.bfloat16)
+    w, cfg = cases.plain_weights(d, "bfloat16")
+    tokens = cases.random_tokens(length, cfg["vocab"], 7)
+    taken, routed = [], ops.routed_experts
+
+    def run(device):
+        ex = cases.make_executor(d, device, "bfloat16", page_size=16, num_pages=64, max_len=320)
+        ex.add_request("r")
+        return ex.step([StepEntry("r", tokens, list(range(length)))])
+
+    with monkeypatch.context() as mp:
+        mp.setattr(ops, "routed_experts", lambda x, experts, *a, **kw: (taken.append(experts.cpu()), routed(x, experts, *a, **kw))[1])
+        got = run(DEV)
+    with monkeypatch.context() as mp:
+        left = list(taken)
+
+        def route_choice(logits, top, scale, **kw):
+            experts = left.pop(0)
+            s = torch.softmax(logits.float(), -1).gather(1, experts.long())
+            return experts, s / (s.sum(-1, keepdim=True) + 1e-20) * scale
+
+        for name in torch_ops.STAND_INS:
+            mp.setattr(ops, name, getattr(torch_ops, name))
+        mp.setattr(ops, "route_choice", route_choice)
+        rounded = run("cpu")
+        assert not left
+    rows, free, others = [r for e in taken for r in e.tolist()], plain.choose, []
+
+    def choose(z, router):
+        chosen, s = rows.pop(0), torch.softmax(z, -1)
+        own = [e for e, _ in free(z, router)]
+        if set(own) != set(chosen):
+            best = lambda es: max(float(s[e]) for e in es)   # (of what one choice has and the other lacks)
+            others.append(best(set(own) - set(chosen)) / best(set(chosen) - set(own)) - 1.0)
+        total = sum(s[e] for e in chosen) + 1e-20
+        return [(e, s[e] / total) for e in chosen]
+
+    choices = len(rows)
+    monkeypatch.setattr(plain, "choose", choose)
+    want = plain.forward(w, cfg, tokens)
+    assert not rows
+    off, alone = cases.rel_rows(got, want), cases.rel_rows(rounded, want)
+    print(length, *(float(f(x)) for x in (off, alone) for f in (torch.median, torch.max)), choices, len(others), max(others, default=0.0))
+    assert off.median() <= 1.5 * alone.median() and off.max() <= 2.0 * alone.max()
+    assert len(others) <= choices // 20 and all(m <= 2.0 * float(alone.max()) for m in others), (len(others), max(others))
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_drawn_configurations(tmp_path, seed):
     cases.drawn_configuration_runs(tmp_path, DEV, seed)
