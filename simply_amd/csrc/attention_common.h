@@ -10,8 +10,8 @@ typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
 
 constexpr int kTile = 32;         // keys per MFMA tile
-constexpr int kMaxSplits = 256;
-constexpr int kRowExtra = 4;   // key ranges per request at most
+constexpr int kMaxSplits = 256;   // key ranges per request at most
+constexpr int kRowExtra = 4;      // words of a partial result's row behind its values
 
 // A unit of work: `q_len` consecutive tokens of the request in block-table row `slot`; the first is row `q_start`
 // of the step and stands at position `pos0`.
@@ -20,6 +20,15 @@ struct SeqMeta {
 };
 
 __device__ inline __bf16 to_bf16_raw(float f) { return static_cast<__bf16>(f); }
+
+// 16 bytes per lane from global memory (an address per lane) into LDS at byte address lds + 16 * lane (lds is the
+// same for the whole wave).  Written as an instruction: the compiler counts a load into LDS that it knows of as a
+// pending LDS access for as long as the load is under way, and then makes every wait for an operand read a wait for
+// all of them.  It does not know of these loads: the kernel waits for them itself (vmcnt) before the barrier that
+// precedes the first read of what they bring.
+__device__ __forceinline__ void load_to_lds(const bf16* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds) : "memory");
+}
 
 // A value of the lanes l, l ^ 16, l ^ 32 and l ^ 48 combined (the four lanes that share a row of an MFMA result),
 // in every one of them, with gfx950's swaps of 16- and 32-lane rows between two registers: one instruction each

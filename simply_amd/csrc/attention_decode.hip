@@ -338,14 +338,6 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
                     sinks, slopes);
 }
 
-// Ranges of about equal size, whatever the requests' lengths: the workgroups read them and cut the keys of every (request,
-// key head) into as many ranges as it takes for ranges of at most `share` tiles, with the smallest `share` (between bounds,
-// by halving) for which the ranges are no more than the workgroups.  A workgroup takes one range.  A range that is not all
-// of its request's keys leaves its result in slot w of the workspace; first_count[unit] are the workgroup of a unit's first
-// range and how many it has.  Bound by reading the keys, as above.
-// Measured (head size 256, lengths spread evenly over their logarithm): 64 requests of 129 to 8,191 keys over 8 key heads
-// 243 -> 211 us, 24 of them 178 -> 100; 40 over 4 key heads 169 -> 83; 8 34 -> 28.  Lengths that are alike are better off
-// with the kernel above (33 requests of 4,096 keys over 4 key heads: 117 us there, 157 here, two ranges for each).
 // A number per lane combined over the wave, and the sum over the lanes up to each, on the vector unit (shuffles go through
 // LDS: with them the ranges were found 3 to 10 us a launch later).
 template <typename Op>
@@ -367,6 +359,14 @@ __device__ __forceinline__ int sum_up_to(int n, int lane) {
   return n + (lane < 16 ? 0 : lane < 32 ? a : lane < 48 ? b : c);
 }
 
+// Ranges of about equal size, whatever the requests' lengths: the workgroups read them and cut the keys of every (request,
+// key head) into as many ranges as it takes for ranges of at most `share` tiles, with the smallest `share` (between bounds,
+// by halving) for which the ranges are no more than the workgroups.  A workgroup takes one range.  A range that is not all
+// of its request's keys leaves its result in slot w of the workspace; first_count[unit] are the workgroup of a unit's first
+// range and how many it has.  Bound by reading the keys, as above.
+// Measured (head size 256, lengths spread evenly over their logarithm): 64 requests of 129 to 8,191 keys over 8 key heads
+// 243 -> 211 us, 24 of them 178 -> 100; 40 over 4 key heads 169 -> 83; 8 34 -> 28.  Lengths that are alike are better off
+// with the kernel above (33 requests of 4,096 keys over 4 key heads: 117 us there, 157 here, two ranges for each).
 template <int NDC>
 __global__ __launch_bounds__(256) void paged_attention_decode_shares_kernel(
     const bf16* __restrict__ q, int64_t q_stride, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
@@ -607,7 +607,10 @@ int paged_attention_decode(const void* q, int64_t q_stride, const void* k_pages,
     if (workspace != nullptr && index_bytes + slots <= workspace_bytes) {
       int2* first_count = static_cast<int2*>(workspace);
       float* partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + index_bytes);
-#define SA_LAUNCH(NDC)                                                                                                  paged_attention_decode_shares_kernel<NDC><<<workgroups, 256, 0, stream>>>(                                                qp, q_stride, kp, vp, block_table, table_stride, sm, seq_begin, seq_count, op, out_stride, Kh, G, page_size, window,       soft_cap, partial, sinks, slopes, least, first_count)
+#define SA_LAUNCH(NDC)                                                                                                      \
+  paged_attention_decode_shares_kernel<NDC><<<workgroups, 256, 0, stream>>>(                                                \
+      qp, q_stride, kp, vp, block_table, table_stride, sm, seq_begin, seq_count, op, out_stride, Kh, G, page_size, window,  \
+      soft_cap, partial, sinks, slopes, least, first_count)
       if (hd == 64) SA_LAUNCH(2);
       else if (hd == 128) SA_LAUNCH(4);
       else SA_LAUNCH(8);

@@ -1,7 +1,7 @@
 // Paged attention in bfloat16 for prompts whose many query heads share one long key vector (latents: keys of a latent and
 // a rotated part, values of the latent alone).  attention_maps.hip takes one unit of 16 query rows to a workgroup and
 // reads all of the keys and values for it: with 1,088 entries a key that is the bound (16 heads and one token a unit,
-// the L2 caches).  Here a workgroup of four waves takes a group of four units of one request, and the keys and values
+// the L2 caches).  Here a workgroup of eight waves takes a group of four units of one request, and the keys and values
 // of a tile of 32 keys come into LDS once for all of its 64 rows.
 //
 // Two waves go with a unit.  Per tile
@@ -11,14 +11,15 @@
 //     O^T += V^T . P^T      all four units, the wave's own eighth of the value entries: a value block is read once
 // The exchange of P^T costs 4 KiB of LDS a tile and saves reading the values four times.  The second product of a tile
 // follows in the next step, among the scores of the next tile, whose operands it covers, and the last four of it cover
-// the exchange of the maxima; a step has two barriers, of which the first publishes P^T of the tile before and the loads that were asked
-// for during the step before.  Keys and values are both kept in two buffers, 2 * (32 * 1,088) * 2 bytes in all for
+// the exchange of the maxima; a step has two barriers, of which the first publishes P^T of the tile before and the loads
+// that were asked for during the step before.  Keys and values are both kept in two buffers, 2 * (32 * 1,088) * 2 bytes in all for
 // the largest sizes, so one workgroup of eight waves runs on a CU.
 // (Four waves with a SIMD each and twice the accumulators needed more than 256 registers; the compiler then moved all
 // accumulators between the halves of the register file in every step, for the sake of the rare rescaling: 184 us.)
 //
-// Measured, 16 heads over one key of 576 entries and values of 512: a prompt of 2,047 tokens 553 -> 126 us, of 4,095
-// 2,371 -> 441, of 512 90 -> 47; 64 tokens behind 8,000 213 -> 48; keys of 192 and values of 128, 1,000 tokens 70 -> 43.
+// Measured, 16 heads over one key of 576 entries and values of 512: a prompt of 2,047 tokens 553 -> 132 us, of 4,095
+// 2,371 -> 436, of 512 90 -> 49; 64 tokens behind 8,000 213 -> 51; keys of 192 and values of 128, 1,000 tokens 70 -> 46
+// (of which the look for values that are not finite, in tiles that not every unit sees whole, is 1 to 2 %).
 // Without the loads (in a copy) 2,047 tokens took 95 us: LDS is the bound, 208 KiB through it per tile, with the chain
 // score - maximum - exchange - exponential behind it; with the second product after the maxima instead of among the
 // scores it was 135.
@@ -32,26 +33,25 @@ constexpr int kUnits = 4;    // units per workgroup
 constexpr int kWaves = 8;    // two per unit
 constexpr float kLog2e = 1.4426950408889634f;
 
-// Every load into LDS has arrived and every LDS access is done, then the workgroup barrier.  The empty statements keep
-// the compiler from moving memory accesses across it (it does not know of the loads below).
+// Every load into LDS has arrived and every LDS access is done, then the workgroup barrier.  The empty statements and the
+// scheduling barriers keep the compiler from moving memory accesses across it (it does not know of the loads into LDS).
 __device__ inline void publish() {
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_waitcnt((7 << 4));   // vmcnt(0) lgkmcnt(0), expcnt left alone
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
 }
 
 // The barrier alone, behind this wave's LDS accesses; loads may be under way.
 __device__ inline void meet() {
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_waitcnt((7 << 4) | 15 | (3 << 14));   // lgkmcnt(0)
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
-}
-
-// 16 bytes per lane from global memory into LDS at byte address lds + 16 * lane (lds is the same for the whole wave).
-__device__ __forceinline__ void load_to_lds(const bf16* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds) : "memory");
+  asm volatile("" ::: "memory");
 }
 
 struct Shape {
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
   //   value block db, lane (grp, r):       sub-tile grp / 2, keys 8 * (grp % 2) .. + 7 of entry 16 * db + r
   const int row = lane % 16;
   const int k_sub = row / 8, v_sub = lane / 32;   // the sub-tile that this lane's pieces come from
-  // (a wave asks for blocks wave, wave + 4, ...: always the same t, and steps of constant size through the pages)
+  // (a wave asks for blocks wave, wave + 8, ...: always the same t, and steps of constant size through the pages)
   const uint32_t k_lane = ((lane / 16) * 16 + 8 * ((row / 4) % 2) + row % 4 + (wave % 2) * 4) * 8 + (wave / 2) * 512;
   const uint32_t v_lane = (wave * 16 + row) * page_size + ((lane / 16) % 2) * 8;
   const uint32_t v_step = kWaves * 16 * page_size;

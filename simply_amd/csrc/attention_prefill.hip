@@ -20,7 +20,7 @@
 //
 // The two buffers are kept in step by one workgroup barrier per tile.  The barrier is the bare instruction, with the
 // count of outstanding loads given by hand: the usual barrier with its fence would wait for all loads in flight,
-// which is the pipeline.  The loads are written as instructions that the compiler does not know of (load_to_lds below).
+// which is the pipeline.  The loads are written as instructions that the compiler does not know of (load_to_lds).
 //
 // When few workgroups would result (a short portion over a long context), the keys are also cut into ranges over
 // workgroups, and the ranges are merged by the second kernel of the few-rows path.
@@ -37,20 +37,14 @@ constexpr float kLog2e = 1.4426950408889634f;
 // 15:14, expcnt 6:4, lgkmcnt 11:8)
 constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
-// The workgroup barrier alone; the empty statements keep the compiler from moving memory accesses across it.
+// The workgroup barrier alone; the empty statements and the scheduling barriers keep the compiler from moving memory
+// accesses across it.
 __device__ inline void bare_barrier() {
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
-}
-
-// 16 bytes per lane from global memory (an address per lane) into LDS at byte address lds + 16 * lane (lds is the
-// same for the whole wave).  Written as an instruction: the compiler counts a load into LDS that it knows of as a
-// pending LDS access for as long as the load is under way, and then makes every wait for an operand read a wait for
-// all of them.  It does not know of these loads: the kernel waits for them itself (vmcnt) before the barrier that
-// precedes the first read of what they bring.
-__device__ __forceinline__ void load_to_lds(const bf16* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds) : "memory");
+  asm volatile("" ::: "memory");
 }
 
 template <int NDC, int R, bool CAP>

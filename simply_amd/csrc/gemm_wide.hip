@@ -44,11 +44,14 @@ constexpr int kCUs = 256;  // compute units of an MI355X
 // 15:14, expcnt 6:4, lgkmcnt 11:8)
 constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
-// The workgroup barrier alone; the empty statements keep the compiler from moving memory accesses across it.
+// The workgroup barrier alone; the empty statements and the scheduling barriers keep the compiler from moving memory
+// accesses across it.
 __device__ inline void bare_barrier() {
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
 }
 
 // 16 bytes per lane from global memory (base + offset bytes, base the same for the whole wave) into LDS at byte
@@ -455,6 +458,7 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
   // time fitted to measurements at the 2B, 9B and 27B sizes (64 to 2,048 rows, seven tiles, one to fourteen cuts;
   // it is within 6 % of the best measured choice nearly everywhere, and a fifth faster in sum than either the
   // uncut tiles above or the tiled kernel with its cut: the 2B down projection at 512 rows takes 36 us against 55).
+  // Beyond 1,536 rows the uncut tiles above stay; whether the model's choice would be better there has not been measured.
   if (epi == 0 && M <= 1536) {  // (fewer than 17 rows come here only against a very long K)
     struct Tile { int code, rows, wrows; double eff, start; };  // share of the MFMA rate in the loop; us to start
     static const Tile tiles[7] = {{3128128, 128, 128, 0.425, 1.44}, {3128256, 128, 256, 0.535, 2.03},
