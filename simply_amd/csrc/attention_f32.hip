@@ -139,22 +139,25 @@ __global__ __launch_bounds__(256, NB == 8 && !PARTS ? 1 : 2) void attention_f32_
       floatx4 p[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        floatx4 k[NB][2], x{0.f, 0.f, 0.f, 0.f}, y{0.f, 0.f, 0.f, 0.f};
+        floatx4 k[NB][2], x[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
           for (int e = 0; e < 2; ++e) k[b][e] = *reinterpret_cast<const floatx4*>(kp[s] + b * 512 + e * 4);
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
+        for (int b = 0; b < NB; ++b) {   // (a chain for each 32 entries: a long one rounds at its size with every product)
+          x[b] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {   // (two chains)
-            x = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][0][e], q[b][0][e], x, 0, 0, 0);
-            y = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][1][e], q[b][1][e], y, 0, 0, 0);
-          }
+          for (int e = 0; e < 8; ++e) x[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][e / 4][e % 4], q[b][e / 4][e % 4], x[b], 0, 0, 0);
+        }
+#pragma unroll
+        for (int n = NB / 2; n > 0; n /= 2)
+#pragma unroll
+          for (int b = 0; b < n; ++b) x[b] += x[b + n];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = c0 + 16 * s + 4 * g + i;
-          float v = (x[i] + y[i]) * a.scale;
+          float v = x[0][i] * a.scale;
           if (a.cap > 0.f) v = a.cap * tanhf(v / a.cap);
           p[s][i] = key <= pos && key > row_lo ? v : -INFINITY;
           m = fmaxf(m, p[s][i]);
