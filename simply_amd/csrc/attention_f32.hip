@@ -17,6 +17,9 @@
 // Keys that some row of the unit does not see get the weight zero.  Where such keys' values are not finite (a zero weight
 // would spread them), their products are taken one key at a time and left out of the rows that do not see it.
 //
+// Scores are summed in a chain of products for each 32 entries of a head: results are 0.5 to 0.75 times as far from 64 bits as
+// the generic kernel's at heads of 256 (1.06 to 1.3 times with two chains).
+//
 // Bound by the latency of a wave's chunk (loads of keys, scores, exponentials, values, one after the other) at the measured
 // sizes, 2B heads: 4 requests of 257 to 1,023 keys 27.6 us and 4.7 for the merge, where the generic kernel, a workgroup per
 // token and key head that walks through all keys on the vector ALU, took 786; a prompt of 509 tokens 45 us for 498.

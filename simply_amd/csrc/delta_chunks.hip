@@ -28,8 +28,8 @@
 //
 // Long chains of matrix instructions round at the size of the sum with every product, so sums run in several short chains, the
 // state's increment and the entries on the diagonal by themselves.  The error against 64 bits is then that of delta_rule.hip
-// (results 0.6 to 1.05 times, the state 0.4 to 0.7 times, 511 to 2,048 tokens); with one or two chains each results were off
-// by up to twice as much.
+// (results 0.57 to 1.05 times, the state 0.4 to 0.7 times, 150 to 2,048 tokens; results at 96 1.07 times); with one or two
+// chains each results were off by up to twice as much.
 //
 // Measured at 2,048 tokens of 16 heads over 8, sizes 128: 41 us for the pieces and 98 for the walk (38 and 89 with one or two
 // chains), where delta_rule.hip takes 629 token by token.

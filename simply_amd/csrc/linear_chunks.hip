@@ -20,8 +20,9 @@
 // Sums and products are 32-bit (v_mfma_f32_16x16x4_f32).  The first kernel is bound by a wave's vector instructions (16
 // steps of 96 multiplications and the operands' reads from LDS), the second by its matrix instructions one after the other.
 //
-// As in delta_chunks.hip sums run in several short chains: results are 0.9 to 1.0 times as far from 64 bits as those of
-// linear_state.hip, the state 0.8 to 0.95 times (500 to 2,047 tokens; 1.2 to 1.3 times with one or two chains each).
+// As in delta_chunks.hip sums run in several short chains, and a block's decays are multiplied in 64 bits: results are 0.72 to
+// 0.93 times as far from 64 bits as those of linear_state.hip, the state 0.65 to 0.75 times (250 to 2,047 tokens; at 96 1.10 and
+// 0.93; with one or two chains and 32 bits 1.2 to 1.3 times).
 //
 // Measured at 2,048 tokens of 16 heads of 128: 31 us for the pieces and 74 for the walk (30 and 67 with one or two chains and
 // without the look at values that are not finite), where linear_state.hip takes 703 token by token.
@@ -179,13 +180,14 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) to[(g * 4 + e) * 4] = m_c[e];
   }
-  // the block's decays, channel by channel
+  // the block's decays, channel by channel (in 64 bits: 15 roundings of a factor that all of a channel's sums have in common
+  // would be the largest part of their error)
 #pragma unroll
   for (int d = lane; d < NT * 16; d += kWave) {
-    float x = 1.f;
+    double x = 1.0;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) x *= a_s[(wave * 16 + j) * AROW + d];
-    blk_s[wave][d] = x;
+    for (int j = 0; j < 16; ++j) x *= static_cast<double>(a_s[(wave * 16 + j) * AROW + d]);
+    blk_s[wave][d] = static_cast<float>(x);
   }
   __syncthreads();   // (the decays have been read)
   floatx4* key_s = reinterpret_cast<floatx4*>(a_s);
