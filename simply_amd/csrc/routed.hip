@@ -18,6 +18,7 @@ namespace sa {
 constexpr int kRouteSlots = 8;    // experts per lane: up to 512 experts
 constexpr int kTileRowsMax = 64;  // rows of a tile: 16 (one MFMA operand) or 64 (four, which share the weights' operands),
 constexpr int kTileRowsWide = 128;   // or 128, for the wide product kernel alone
+constexpr int kGridMax = 65535;      // a grid's second and third index
 
 // A wave per token.  scores = softmax(logits); `top` times the largest score that is left (of equal ones the lowest
 // index); weight = score * scale.
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(kWave) void expert_product_kernel(
     int N, int K, const int* __restrict__ sorted, const int* __restrict__ plan, int act, float limit,
     void* __restrict__ out, int64_t out_stride, int out_by_pair, int activate) {
   // activate (without a second weight): out[row] = act(a . w1[e]^T) in a's type instead of the 32-bit product
-  const int tile = blockIdx.y;
+  const int tile = blockIdx.z * gridDim.y + blockIdx.y;
   if (tile >= plan[0]) return;
   const int e = plan[1 + 3 * tile], row0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
   const int lane = threadIdx.x, n0 = blockIdx.x * 16;
@@ -603,7 +604,10 @@ extern "C" int sa_expert_tile_rows(int P, int E, int D, int F, int dtype, int64_
   if (P < (wide ? 12 : 32) * static_cast<int64_t>(E)) return 16;
   // Tiles of 128 rows where they fill up and an expert's gate and up are more than the L2s hold (4 MiB an XCD), so that every
   // tile of rows fetches them again (figures: gemm_wide_routed).
-  return wide && P >= 96 * static_cast<int64_t>(E) && 4.0 * D * F > 32.0 * (1 << 20) ? kTileRowsWide : kTileRowsMax;
+  return wide && P >= 96 * static_cast<int64_t>(E) && 4.0 * D * F > 32.0 * (1 << 20) &&
+                 sa_expert_tiles_max(P, E, kTileRowsWide) <= kGridMax
+             ? kTileRowsWide
+             : kTileRowsMax;
 }
 
 extern "C" int sa_expert_sort(const int* experts, int P, int E, int tile_rows, int* sorted, int* plan, int plan_words,
@@ -636,15 +640,15 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
   SA_REQUIRE(tile_rows == 16 || tile_rows == kTileRowsMax || tile_rows == kTileRowsWide,
              "expert_product: tiles of 16, %d or %d rows", kTileRowsMax, kTileRowsWide);
   const int tiles = sa_expert_tiles_max(P, E, tile_rows);
-  SA_REQUIRE(tiles <= 65535, "expert_product: too many tiles");
+  // (the grid's second and third index go to 65,535; tiles of the kernels of 16 and 64 rows here are not limited by that)
+  const int tiles_y = tiles < kGridMax ? tiles : kGridMax, tiles_z = (tiles + tiles_y - 1) / tiles_y;
   const bool gated = w2 != nullptr;
 #define SA_EXPERT(T, G, RT)                                                                                            \
-  expert_product_kernel<T, G, RT><<<dim3((N + 15) / 16, tiles), kWave, 0, stream>>>(static_cast<const T*>(a), a_stride, a_by_token, top,        \
-                                                             static_cast<const T*>(w1), static_cast<const T*>(w2), N,  \
-                                                             K, sorted, plan, act, limit, out, out_stride, out_by_pair, \
-                                                             activate)
+  expert_product_kernel<T, G, RT><<<dim3((N + 15) / 16, tiles_y, tiles_z), kWave, 0, stream>>>(                          \
+      static_cast<const T*>(a), a_stride, a_by_token, top, static_cast<const T*>(w1), static_cast<const T*>(w2), N, K,   \
+      sorted, plan, act, limit, out, out_stride, out_by_pair, activate)
   // Tiles of 64 and 128 rows go to the wide product kernel where it takes the operands; the others to the kernel of 64 rows here.
-  const bool by_wide = dtype == kBF16 && tile_rows != 16 && ((gated || activate) ? !out_by_pair : out_by_pair != 0) &&
+  const bool by_wide = dtype == kBF16 && tile_rows != 16 && tiles <= kGridMax && ((gated || activate) ? !out_by_pair : out_by_pair != 0) &&
                        gemm_wide_routed_takes(N, K, a_stride, a_by_token ? (P + top - 1) / top : P, out_stride, a, w1, w2, out, tile_rows);
   SA_REQUIRE(by_wide || tile_rows != kTileRowsWide, "expert_product: tiles of %d rows need aligned bfloat16 operands, K in multiples of 64",
              kTileRowsWide);

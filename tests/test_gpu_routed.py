@@ -45,3 +45,27 @@ def test_tiles_agree(monkeypatch, T, E, top, D, F, gated):
             want[rows] += weights[rows, k, None] * (h @ ws[2][e].float().T)
             size[rows] += weights[rows, k, None] * (h.abs() @ ws[2][e].float().abs().T)
     assert ((got - want).abs() <= 2.0 ** -6 * size + 1e-5).all()
+
+
+@pytest.mark.parametrize("dtype,tile_rows", [(torch.float32, 16), (torch.float32, 64), (torch.bfloat16, 16), (torch.bfloat16, 64)])
+def test_more_tiles_than_a_grid_s_second_index(dtype, tile_rows):
+    """More than 65,535 tiles of rows; the last rows of the last tiles among them.  Whole numbers that both types hold: exact."""
+    from simply_amd.kernels import lib, ops
+    from simply_amd.kernels.packing import stack_experts
+
+    P, E, N, K = 65536 * tile_rows + 5, 2, 16, 64
+    a = torch.randint(-2, 3, (P, K), generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+    w = [torch.randint(-2, 3, (N, K), generator=torch.Generator().manual_seed(e)).to(dtype).cuda() for e in (2, 3)]
+    stack = stack_experts(w)
+    experts = (torch.arange(P, dtype=torch.int32) % 7 == 0).int().cuda()
+    max_tiles = lib.load().sa_expert_tiles_max(P, E, tile_rows)
+    order = torch.empty(P, dtype=torch.int32, device="cuda")
+    plan = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device="cuda")
+    out = torch.full((P, N), -1.0, device="cuda")
+    lib.call("sa_expert_sort", experts.data_ptr(), P, E, tile_rows, order.data_ptr(), plan.data_ptr(), plan.numel(), ops._stream())
+    lib.call("sa_expert_product", a.data_ptr(), ops._code(a), K, 1, 1, stack.data.data_ptr(), None, N, K, order.data_ptr(),
+             plan.data_ptr(), P, E, tile_rows, 0, 0.0, out.data_ptr(), N, 1, 0, ops._stream())
+    assert int(plan[0]) > 65535
+    a = a.float()
+    want = torch.where(experts[:, None] == 0, a @ w[0].float().T, a @ w[1].float().T)
+    assert torch.equal(out, want)
