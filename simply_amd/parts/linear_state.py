@@ -27,8 +27,8 @@ from ..registry import MIXERS
 from .base import Mixer, ParamSpec, StateNeed, as_product_weight, project
 
 
-#: tokens of a request in a step from which a recurrence with decays per channel is worked through in pieces: one request's 65
-#: tokens take 24 us in pieces and 21 one by one, 96 take 25 and 28 (eight requests': 35 and 30, 36 and 41; 16 heads of 128)
+#: tokens of a request in a step from which a recurrence with decays per channel is worked through in pieces: one request's 80
+#: tokens take 28 us in pieces and 25 one by one, 96 28 and 29 (eight requests' 65 each 46 and 55, 80 47 and 64; 16 heads of 128)
 PIECES_FROM = 80
 
 

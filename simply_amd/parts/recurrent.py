@@ -74,10 +74,9 @@ class GatedDelta(Mixer):
         qkv, gates = ops.delta_inputs(proj[:, :C], self.taps, tails, ab, self.a_log, self.dt_bias, ctx.seq_meta,
                                       ctx.num_seqs, ctx.max_q_len, H, G, dk)
         # Requests with few tokens go through the recurrence token by token, portions of prompts of a bfloat16 run in pieces
-        # on the matrix cores where these take the sizes (2,048 tokens of 16 heads of 128: 629 against 143 us; one token
-        # after the other takes 0.3 us each, the pieces' two kernels 25 us and 0.5 to 3 a piece: even at about 96 tokens of one
-        # request, at 32 to 64 of eight).  A 32-bit run, whose
-        # results do not depend on how the tokens are cut into steps, stays with the rule token by token.
+        # on the matrix cores where these take the sizes (16 heads of 128: 2,048 tokens 589 against 137 us; one request's 96
+        # tokens 32 against 35, 112 36 against 35; eight requests' 65 tokens each 95 against 62, 96 133 against 61).  A 32-bit
+        # run, whose results do not depend on how the tokens are cut into steps, stays with the rule token by token.
         o = torch.empty((x.shape[0], H * dv), dtype=torch.float32, device=x.device)
         short = ctx.num_seqs
         if ctx.dtype == torch.bfloat16 and ctx.max_q_len >= self.PIECES_FROM:
