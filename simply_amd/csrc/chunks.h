@@ -32,6 +32,15 @@ __device__ __forceinline__ floatx4 mul4(floatx4 a, floatx4 b, floatx4 c) {   // 
   return c;
 }
 
+// a . b alone, the four steps' sums by halves: a chain rounds at the size of the sum so far with every product, whose order it
+// cannot choose.
+__device__ __forceinline__ floatx4 halves4(floatx4 a, floatx4 b) {
+  floatx4 x[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) x[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+  return (x[0] + x[1]) + (x[2] + x[3]);
+}
+
 // The chains' sums, by halves.
 template <int N>
 __device__ __forceinline__ floatx4 sum_of(floatx4 (&x)[N]) {
@@ -44,7 +53,8 @@ __device__ __forceinline__ floatx4 sum_of(floatx4 (&x)[N]) {
 
 // acc + m . b for a lower triangular m: the diagonal block of a product over earlier tokens.  A product with a zero carries an
 // entry of b that is not finite into every row; such entries are left out of the product, and added one at a time to the rows
-// at and behind their own.
+// at and behind their own.  IN_TIME: step r of the operands holds tokens 4 r + g instead of 4 g + r.
+template <bool IN_TIME>
 __device__ __forceinline__ floatx4 lower_mul4(floatx4 m, floatx4 b, floatx4 acc, int lane) {
   bool odd = false;
 #pragma unroll
@@ -58,13 +68,13 @@ __device__ __forceinline__ floatx4 lower_mul4(floatx4 m, floatx4 b, floatx4 acc,
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
 #pragma unroll 1
-    for (int of = 0; of < 4; ++of) {   // entry 4 of + r
+    for (int of = 0; of < 4; ++of) {   // entry 4 of + r, or 4 r + of
       const bool mine = of == g && !(fabsf(b[r]) < INFINITY);
       if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
       const floatx4 one = __builtin_amdgcn_mfma_f32_16x16x4f32(of == g ? m[r] : 0.f, mine ? b[r] : 0.f,
                                                                floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] += 4 * g + i >= 4 * of + r ? one[i] : 0.f;
+      for (int i = 0; i < 4; ++i) acc[i] += 4 * g + i >= (IN_TIME ? 4 * r + of : 4 * of + r) ? one[i] : 0.f;
     }
   }
   return acc;

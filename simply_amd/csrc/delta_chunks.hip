@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
         less[e % 2] = mul4(*reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + e * 16 + g * 4]), x[e], less[e % 2]);
       acc -= less[0] + less[1];
       const floatx4 inv = *reinterpret_cast<const floatx4*>(&a_s[(b * 16 + c) * AROW + b * 16 + g * 4]);
-      x[b] = acc + lower_mul4(inv, acc, floatx4{0.f, 0.f, 0.f, 0.f}, lane);
+      x[b] = acc + lower_mul4<false>(inv, acc, floatx4{0.f, 0.f, 0.f, 0.f}, lane);
     }
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) {
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
 #pragma unroll
     for (int b = 0; b < kBlocks - 1; ++b)
       if (b < wave) o2[b] = mul4(p[b], ub[b], o2[b]);   // (uniform over the wave)
-    o2[kBlocks - 1] = lower_mul4(p[kBlocks - 1], u, o2[kBlocks - 1], lane);
+    o2[kBlocks - 1] = lower_mul4<false>(p[kBlocks - 1], u, o2[kBlocks - 1], lane);
     floatx4 result = sum_of(o) + sum_of(o2);
 #pragma unroll
     for (int r = 0; r < 4; ++r) result[r] = fmaf(own[r], u[r], result[r]);

@@ -17,15 +17,21 @@
 //   linear_walk_kernel     the walk through the pieces, a workgroup of four waves per head and 16 value columns, as
 //                          delta_state_kernel does it (delta_chunks.hip), with one barrier a piece
 //
-// Sums and products are 32-bit (v_mfma_f32_16x16x4_f32).  The first kernel is bound by a wave's vector instructions (16
-// steps of 96 multiplications and the operands' reads from LDS), the second by its matrix instructions one after the other.
+// Sums and products are 32-bit (v_mfma_f32_16x16x4_f32).  The first kernel is bound by a wave's vector instructions (two
+// times 16 steps of 32 multiplications in 64 bits with their conversions, of keys and of queries one after the other: with both
+// at once a CU has registers for half the waves, 60 us instead of 46), the second by its matrix instructions one after the other.
 //
-// As in delta_chunks.hip sums run in several short chains, and a block's decays are multiplied in 64 bits: results are 0.72 to
-// 0.93 times as far from 64 bits as those of linear_state.hip, the state 0.65 to 0.75 times (250 to 2,047 tokens; at 96 1.10 and
-// 0.93; with one or two chains and 32 bits 1.2 to 1.3 times).
+// What keeps the error against 64 bits no larger than that of linear_state.hip: decays are multiplied in 64 bits, before they
+// meet a key or query that is rounded once; sums run in chains of 16 products, the state's increment by itself; and over
+// tokens step r of an operand takes tokens 4 r + g, so that a chain adds them in their order, whose last are the largest where
+// decays are fast.  Times the error of linear_state.hip, results and state (80 to 260 tokens, 16 heads of 128):
+//   rates per channel, decays 0.998 to 0.19       0.87 to 0.69   0.65 to 0.51
+//   sigmoid(z)^(1 / 16)                           0.97           0.89 to 0.97
+//   decays drawn anew for each token, 0.69 on     1.00           0.97 to 1.05
+//   the same between 0 and 1                      0.96           1.25 to 1.35
+// (with decays multiplied in 32 bits and two or four chains the second to fourth were 1.04 to 1.19 and 1.16 to 1.8.)
 //
-// Measured at 2,048 tokens of 16 heads of 128: 31 us for the pieces and 74 for the walk (30 and 67 with one or two chains and
-// without the look at values that are not finite), where linear_state.hip takes 703 token by token.
+// Measured at 2,048 tokens of 16 heads of 128: 46 us for the pieces and 76 for the walk, where linear_state.hip takes 704 token by token.
 #include "api.h"
 #include "chunks.h"
 
@@ -110,73 +116,94 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
     *reinterpret_cast<floatx4*>(&a_s[j * AROW + d]) = av;
   }
   __syncthreads();
-  // values of the wave's tokens, as the right operand
+  // values of the wave's tokens, as the right operand: this lane has tokens 4 r + g
   for (int n = 0; n < cb; ++n) {
     const int col = n * 16 + c;
     floatx4 v;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int j = wave * 16 + g * 4 + r;
+      const int j = wave * 16 + r * 4 + g;
       v[r] = j < left && col < a.dv ? to_float(a.proj[static_cast<size_t>(row0 + j) * a.proj_stride + a.v_at + h * a.dv + col]) : 0.f;
     }
     *reinterpret_cast<floatx4*>(dst + lay.v + (n * kBlocks + wave) * kBlock + lane * 4) = v;
   }
-  // the block of 16 tokens on the diagonal: lane c has query c (qp, times the decays in front of it in the block) and key c
-  // (kw, times the decays behind it so far); step i brings token i's decays and its query to all lanes' keys
-  floatx4 qp[NT], kw[NT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    qp[n] = to_float4(*reinterpret_cast<const uint2*>(&q_s[(wave * 16 + c) * QROW + n * 16 + g * 4])) * a.q_mult;
-    kw[n] = to_float4(*reinterpret_cast<const uint2*>(&k_s[(wave * 16 + c) * QROW + n * 16 + g * 4]));
-  }
+  // the block of 16 tokens on the diagonal: lane c has key c, and step i brings token i's decays and its query to all lanes' keys
+  // (kw, times the decays behind the token so far, which are multiplied in 64 bits: a key that has been rounded 15 times over
+  // would be the largest part of the results' error)
+  double kw[NT][4];
   floatx4 own_r{0.f, 0.f, 0.f, 0.f};   // M_cc, by the lane's channels
 #pragma unroll
-  for (int n = 0; n < NT; ++n)
+  for (int n = 0; n < NT; ++n) {
+    const floatx4 q = to_float4(*reinterpret_cast<const uint2*>(&q_s[(wave * 16 + c) * QROW + n * 16 + g * 4])) * a.q_mult;
+    const floatx4 k = to_float4(*reinterpret_cast<const uint2*>(&k_s[(wave * 16 + c) * QROW + n * 16 + g * 4]));
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float x = qp[n][r] * kw[n][r];
+      float x = q[r] * k[r];
       const int d = n * 16 + g * 4 + r;
       if (BONUS) x *= d < a.dk ? load_f(a.bonus, a.bonus_dtype, static_cast<size_t>(h) * a.dk + d) : 0.f;
       own_r[r] += x;
+      kw[n][r] = static_cast<double>(k[r]);
     }
+  }
   const float own = sum_over_row_lanes((own_r[0] + own_r[1]) + (own_r[2] + own_r[3]));
   float m_c[4] = {0.f, 0.f, 0.f, 0.f};   // M[query 4 g + r][key c] of the block
+  auto decay_of = [&](int i, int n) __attribute__((always_inline)) {   // token i's decays of the lane's channels of block n
+    return *reinterpret_cast<const floatx4*>(&a_s[(wave * 16 + i) * AROW + n * 16 + g * 4]);
+  };
 #pragma unroll 1
   for (int i4 = 0; i4 < 4; ++i4) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = i4 * 4 + e;
       floatx4 av[NT], s_r{0.f, 0.f, 0.f, 0.f};
-      const float* ap = &a_s[(wave * 16 + i) * AROW + g * 4];
       const bf16* qi = &q_s[(wave * 16 + i) * QROW + g * 4];
 #pragma unroll
-      for (int n = 0; n < NT; ++n) av[n] = *reinterpret_cast<const floatx4*>(ap + n * 16);
-      if (!BONUS && c < i) {
+      for (int n = 0; n < NT; ++n) av[n] = decay_of(i, n);
+      auto decay_keys = [&]() __attribute__((always_inline)) {
+        if (c < i) {
 #pragma unroll
-        for (int n = 0; n < NT; ++n) kw[n] *= av[n];
-      }
+          for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) kw[n][r] *= static_cast<double>(av[n][r]);
+        }
+      };
+      if (!BONUS) decay_keys();
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const floatx4 q = to_float4(*reinterpret_cast<const uint2*>(qi + n * 16));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s_r[r] = fmaf(q[r], kw[n][r], s_r[r]);
+        for (int r = 0; r < 4; ++r) s_r[r] = fmaf(q[r], static_cast<float>(kw[n][r]), s_r[r]);
       }
-      if (BONUS && c < i) {
-#pragma unroll
-        for (int n = 0; n < NT; ++n) kw[n] *= av[n];
-      }
-      if (BONUS ? i < c : i <= c) {
-#pragma unroll
-        for (int n = 0; n < NT; ++n) qp[n] *= av[n];
-      }
+      if (BONUS) decay_keys();
       float s = sum_over_row_lanes((s_r[0] + s_r[1]) + (s_r[2] + s_r[3])) * a.q_mult;
       s = c < i ? s : c == i ? own : 0.f;
       if (g == i4) m_c[e] = s;
     }
   }
-  // the block's M, turned: as the left operand lane (query c, group g) has keys 4 g .. 4 g + 3
+  floatx4 key[NT], qp[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) key[n][r] = static_cast<float>(kw[n][r]);
+  // query c times the decays in front of it in the block, likewise
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    double x[4] = {1.0, 1.0, 1.0, 1.0};
+#pragma unroll 4
+    for (int i = 0; i < 16; ++i) {
+      const floatx4 av = decay_of(i, n);
+      if (BONUS ? i < c : i <= c) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] *= static_cast<double>(av[r]);
+      }
+    }
+    const floatx4 q = to_float4(*reinterpret_cast<const uint2*>(&q_s[(wave * 16 + c) * QROW + n * 16 + g * 4])) * a.q_mult;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) qp[n][r] = static_cast<float>(x[r] * static_cast<double>(q[r]));
+  }
+  // the block's M, turned: as the left operand lane (query c, group g) has keys 4 r + g
   {
-    float* to = dst + lay.p + (wave * kBlocks + wave) * kBlock + (c / 4) * 64 + c % 4;
+    float* to = dst + lay.p + (wave * kBlocks + wave) * kBlock + (c % 4) * 64 + c / 4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) to[(g * 4 + e) * 4] = m_c[e];
   }
@@ -193,28 +220,29 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
   floatx4* key_s = reinterpret_cast<floatx4*>(a_s);
   static_assert(kBlocks * NT * kWave * 16 <= kTokens * AROW * 4, "the keys lie where the decays lay");
 #pragma unroll
-  for (int n = 0; n < NT; ++n) key_s[(wave * NT + n) * kWave + lane] = kw[n];
+  for (int n = 0; n < NT; ++n) key_s[(wave * NT + n) * kWave + lane] = key[n];
   __syncthreads();
   // keys of earlier blocks, from the nearest on; the queries take a block's decays on the way
 #pragma unroll 1
   for (int b = wave - 1; b >= 0; --b) {
-    floatx4 x[NT];   // (a chain of products for each 16 channels)
+    // (the keys' rows are permuted so that the result's are the left operand's tokens: this lane has keys 4 r + g of query c)
+    floatx4 x[NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) x[n] = mul4(key_s[(b * NT + n) * kWave + lane], qp[n], floatx4{0.f, 0.f, 0.f, 0.f});
-    *reinterpret_cast<floatx4*>(dst + lay.p + (wave * kBlocks + b) * kBlock + lane * 4) = sum_of(x);   // [key 4 g + r][query c]
+    for (int n = 0; n < NT; ++n) x[n] = halves4(key_s[(b * NT + n) * kWave + g * 16 + (c % 4) * 4 + c / 4], qp[n]);
+    *reinterpret_cast<floatx4*>(dst + lay.p + (wave * kBlocks + b) * kBlock + lane * 4) = sum_of(x);
 #pragma unroll
     for (int n = 0; n < NT; ++n) qp[n] *= *reinterpret_cast<const floatx4*>(&blk_s[b][n * 16 + g * 4]);
   }
 #pragma unroll
   for (int n = 0; n < NT; ++n) *reinterpret_cast<floatx4*>(dst + lay.q + (wave * NT + n) * kBlock + lane * 4) = qp[n];
-  // the wave's keys times the decays of the blocks behind, turned: [channel c][tokens 4 g ..]
+  // the wave's keys times the decays of the blocks behind, turned: [channel c][tokens 4 r + g]
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
     float f = 1.f;
     for (int b = wave + 1; b < kBlocks; ++b) f *= blk_s[b][n * 16 + c];
     floatx4 kt;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) kt[r] = a_s[((wave * NT + n) * kWave + (c / 4) * 16 + g * 4 + r) * 4 + c % 4] * f;
+    for (int r = 0; r < 4; ++r) kt[r] = a_s[((wave * NT + n) * kWave + (c / 4) * 16 + r * 4 + g) * 4 + c % 4] * f;
     *reinterpret_cast<floatx4*>(dst + lay.kt + (n * kBlocks + wave) * kBlock + lane * 4) = kt;
   }
   if (tid < NT * 16) dst[lay.all + tid] = blk_s[0][tid] * blk_s[1][tid] * blk_s[2][tid] * blk_s[3][tid];
@@ -274,33 +302,28 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
 #pragma unroll
     for (int n = 0; n < NT; ++n) st[n] = s_s[now][n * kWave + lane];
     // the state behind the piece, for the others to read
-    floatx4 more[NW];   // (summed by itself: 64 products added to the state one by one would round it 64 times)
+    // (summed by itself, a chain for each 16 tokens: 64 products added to the state one by one would round it 64 times)
 #pragma unroll
-    for (int n = 0; n < NW; ++n) more[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < NW; ++n) {
+      floatx4 more[kBlocks];
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b)
+      for (int b = 0; b < kBlocks; ++b) more[b] = mul4(kt[n][b], v[b], floatx4{0.f, 0.f, 0.f, 0.f});
+      const floatx4 added = ((more[0] + more[1]) + more[2]) + more[3];
 #pragma unroll
-      for (int n = 0; n < NW; ++n) more[n] = mul4(kt[n][b], v[b], more[n]);
-#pragma unroll
-    for (int n = 0; n < NW; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[n][r] = fmaf(s[n][r], all[n][r], more[n][r]);
+      for (int r = 0; r < 4; ++r) s[n][r] = fmaf(s[n][r], all[n][r], added[r]);
+    }
 #pragma unroll
     for (int n = 0; n < NW; ++n) s_s[now ^ 1][(wave * NW + n) * kWave + lane] = s[n];
     fetch_state(next);
-    floatx4 o[4], o2[kBlocks];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 o[NT], o2[kBlocks];
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) o2[b] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int n = 0; n < NT; n += 4)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = mul4(q[n + i], st[n + i], o[i]);
+    for (int n = 0; n < NT; ++n) o[n] = mul4(q[n], st[n], floatx4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
     for (int b = 0; b < kBlocks - 1; ++b)
       if (b < wave) o2[b] = mul4(p[b], v[b], o2[b]);   // (uniform over the wave)
-    o2[kBlocks - 1] = lower_mul4(p[kBlocks - 1], v_own, o2[kBlocks - 1], lane);
+    o2[kBlocks - 1] = lower_mul4<true>(p[kBlocks - 1], v_own, o2[kBlocks - 1], lane);
     const floatx4 result = sum_of(o) + sum_of(o2);
     fetch_rest(next);
     if (col_ok) {

@@ -27,9 +27,9 @@ from ..registry import MIXERS
 from .base import Mixer, ParamSpec, StateNeed, as_product_weight, project
 
 
-#: tokens of a request in a step from which a recurrence with decays per channel is worked through in pieces: one request's 80
-#: tokens take 28 us in pieces and 25 one by one, 96 28 and 29 (eight requests' 65 each 46 and 55, 80 47 and 64; 16 heads of 128)
-PIECES_FROM = 80
+#: tokens of a request in a step from which a recurrence with decays per channel is worked through in pieces: one request's 128
+#: tokens take 39 us in pieces and 37 one by one (eight requests' 65 each 57 and 56, 128 58 and 96; 16 heads of 128)
+PIECES_FROM = 128
 
 
 def channel_decay_state(proj, columns, q_mult, gates, H, dk, dv, state, ctx, **kw):
