@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kWave) void expert_product_kernel(
     int N, int K, const int* __restrict__ sorted, const int* __restrict__ plan, int act, float limit,
     void* __restrict__ out, int64_t out_stride, int out_by_pair, int activate) {
   // activate (without a second weight): out[row] = act(a . w1[e]^T) in a's type instead of the 32-bit product
-  const int tile = blockIdx.z * gridDim.y + blockIdx.y;
+  const int tile = blockIdx.z * kGridMax + blockIdx.y;   // (gridDim would be one more load in front of everything)
   if (tile >= plan[0]) return;
   const int e = plan[1 + 3 * tile], row0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
   const int lane = threadIdx.x, n0 = blockIdx.x * 16;
