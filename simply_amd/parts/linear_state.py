@@ -27,9 +27,15 @@ from ..registry import MIXERS
 from .base import Mixer, ParamSpec, StateNeed, as_product_weight, project
 
 
-#: tokens of a request in a step from which a recurrence with decays per channel is worked through in pieces: one request's 128
-#: tokens take 39 us in pieces and 37 one by one (eight requests' 65 each 57 and 56, 128 58 and 96; 16 heads of 128)
+#: Tokens of a step's longest request from which a recurrence with decays per channel is worked through in pieces: one
+#: request's 128 tokens take 39 us in pieces and 37 one by one, 96 39 and 29 (16 heads of 128) ...
 PIECES_FROM = 128
+#: ... and where so many requests bring PIECES_TOO or more: eight requests' 80 tokens each take 57 us in pieces and 63 one by
+#: one, 128 58 and 96.
+MANY, MANY_FROM = 8, 80
+#: Requests of so many tokens go along (the two ways run one behind the other: 0.35 to 0.75 us for a token of the longest
+#: request that stays); 65 tokens of eight requests take 57 and 56.
+PIECES_TOO = 64
 
 
 def channel_decay_state(proj, columns, q_mult, gates, H, dk, dv, state, ctx, **kw):
@@ -37,9 +43,10 @@ def channel_decay_state(proj, columns, q_mult, gates, H, dk, dv, state, ctx, **k
     portions of prompts of a bfloat16 run in pieces on the matrix cores where these take the sizes."""
     out = torch.empty((proj.shape[0], H * dv), dtype=torch.float32, device=proj.device)
     short = ctx.num_seqs
-    if ctx.max_q_len >= PIECES_FROM and proj.dtype == torch.bfloat16:
-        few, rows = ctx.short_requests(PIECES_FROM - 1)
-        if ops.linear_chunks_takes(proj, columns[0], columns[1], gates, state, ctx.num_seqs - few, H, dk, dv):
+    if ctx.max_q_len >= MANY_FROM and proj.dtype == torch.bfloat16:
+        few, rows = ctx.short_requests(PIECES_TOO - 1)
+        long_enough = ctx.max_q_len >= PIECES_FROM or ctx.num_seqs - few >= MANY
+        if long_enough and ops.linear_chunks_takes(proj, columns[0], columns[1], gates, state, ctx.num_seqs - few, H, dk, dv):
             short = few
             ops.linear_chunks(proj, *columns, q_mult, gates, H, dk, dv, state, ctx.seq_meta[short:], ctx.num_seqs - short, rows,
                               ctx.max_q_len, out=out, **kw)
