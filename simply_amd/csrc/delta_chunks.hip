@@ -28,11 +28,12 @@
 //
 // Long chains of matrix instructions round at the size of the sum with every product, so sums run in several short chains, the
 // state's increment and the entries on the diagonal by themselves.  The error against 64 bits is then that of delta_rule.hip
-// (results 0.57 to 1.05 times, the state 0.4 to 0.7 times, 150 to 2,048 tokens; results at 96 1.07 times); with one or two
-// chains each results were off by up to twice as much.
+// (rates and steps as in models of the kind, 64 to 2,048 tokens: results 0.57 to 1.05 times, the state 0.4 to 0.87 times; with
+// decays drawn evenly from 0 to 1, half-lives of a token, 1.2 and 1.2 to 1.4 times, and no less with exponentials in 64 bits);
+// with one or two chains each results were off by up to twice as much.
 //
 // Measured at 2,048 tokens of 16 heads over 8, sizes 128: 41 us for the pieces and 98 for the walk (38 and 89 with one or two
-// chains), where delta_rule.hip takes 629 token by token.
+// chains), where delta_rule.hip takes 589 token by token.
 #include "api.h"
 #include "chunks.h"
 

@@ -28,10 +28,11 @@
 //   rates per channel, decays 0.998 to 0.19       0.87 to 0.69   0.65 to 0.51
 //   sigmoid(z)^(1 / 16)                           0.97           0.89 to 0.97
 //   decays drawn anew for each token, 0.69 on     1.00           0.97 to 1.05
-//   the same between 0 and 1                      0.96           1.25 to 1.35
+//   the same between 0 and 1                      0.96           1.25 to 1.40
 // (with decays multiplied in 32 bits and two or four chains the second to fourth were 1.04 to 1.19 and 1.16 to 1.8.)
 //
-// Measured at 2,048 tokens of 16 heads of 128: 46 us for the pieces and 76 for the walk, where linear_state.hip takes 704 token by token.
+// Measured at 2,048 tokens of 16 heads of 128: 122 us (traced, 48 for the pieces and 81 for the walk), where
+// linear_state.hip takes 704 token by token.
 #include "api.h"
 #include "chunks.h"
 
