@@ -390,6 +390,13 @@ int sa_qk_norm_rope_cache_write(void* proj, int dtype, int64_t row_stride, const
 int sa_residual_add_next_norm(const void* y, int y_dtype, int64_t y_stride, float mult, float* residual, const void* w,
                               const void* b, int w_dtype, float eps, int plus_one, void* out, int out_dtype, int T, int D,
                               hipStream_t stream);
+// sa_residual_add_next_norm of what sa_expert_combine gives from y, weights, shared and gate, out in bfloat16: rows of whole
+// aligned pieces of 8 entries (_takes; y and out are whole tensors).
+int sa_experts_add_next_norm(const float* y, const float* weights, int top, const void* shared, int shared_dtype,
+                             int64_t shared_stride, const float* gate, int64_t gate_stride, float mult, float* residual,
+                             const void* w, const void* b, int w_dtype, float eps, int plus_one, void* out, int T, int D,
+                             hipStream_t stream);
+int sa_experts_add_next_norm_takes(int D, const void* shared, int64_t shared_stride, const void* residual, const void* w, const void* b);
 
 // On fused projection rows [H * dk queries | K * dk keys | K * dv values | ...]: every query and key vector is cut into
 // `sub` equal parts; in each part the first *_norm_dims entries are divided by sqrt(mean of their squares + eps) and
@@ -610,6 +617,21 @@ int sa_expert_sort(const int* experts, int P, int E, int tile_rows, int* sorted,
 int sa_expert_product(const void* a, int dtype, int64_t a_stride, int a_by_token, int top, const void* w1, const void* w2,
                       int N, int K, const int* sorted, const int* plan, int P, int E, int tile_rows, int act, float limit,
                       void* out, int64_t out_stride, int out_by_pair, int activate, hipStream_t stream);
+// A router of a few tokens in one launch: logits [T, rows] (32-bit) = x . w^T with x bfloat16 [T, D] and w tiled, the choice as
+// sa_route (plain) or sa_route_choice make it from the first E logits of a token, sorted and plan as sa_expert_sort with tiles
+// of 16 rows.  _takes: at most 16 tokens, 128 experts (and up to 16 more rows) and 128 pairs, weights of up to 128 K entries.
+int sa_route_few_takes(const void* x, int64_t x_stride, int T, int D, int rows, int E, int top);
+int sa_route_few(const void* x, int64_t x_stride, const void* w, int T, int D, int rows, int E, int top, float scale, int plain,
+                 const void* bias, int bias_dtype, const void* correction, int corr_dtype, int groups, int keep, int softmax,
+                 int group_best, float renorm, float* logits, int* experts, float* weights, int* sorted, int* plan, int plan_words,
+                 hipStream_t stream);
+// sa_expert_product in bfloat16 with tiles of 16 rows, and beside it the same product of all T <= 16 tokens with a dense weight:
+// shared_out[t] = rule(shared_a[t]); shared_w: tiled, with w2 the two factors' tiles in turn.
+int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w1, const void* w2, int N, int K,
+                             const int* sorted, const int* plan, int P, int E, int act, float limit, void* out, int64_t out_stride,
+                             int out_by_pair, int activate, const void* shared_a, int64_t shared_a_stride, const void* shared_w,
+                             int shared_N, int shared_K, int T, float shared_limit, void* shared_out, int64_t shared_out_stride,
+                             hipStream_t stream);
 // out[t] = sum_k weights[t, k] y[t * top + k] + sigmoid(gate[t]) * shared[t]  (shared null: none; gate null: 1).
 int sa_expert_combine(const float* y, const float* weights, int top, const void* shared, int shared_dtype,
                       int64_t shared_stride, const float* gate, int64_t gate_stride, void* out, int out_dtype,

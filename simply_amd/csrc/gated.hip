@@ -270,21 +270,64 @@ __global__ __launch_bounds__(256) void residual_add_next_norm_kernel(
   }
 }
 
-// The same for rows in pieces of eight (ADD: there is a y).
-template <typename YT, typename WT, typename OT, int NP, bool CENTERED, bool ADD>
+// What is added to the residual, eight entries at a time: rows as they are ...
+template <typename YT>
+struct RowsAsTheyAre {
+  const YT* y;
+  int64_t stride;
+  __device__ __forceinline__ Eight at(int row, int d) const { return load_eight(y + static_cast<size_t>(row) * stride + d); }
+};
+// ... or a token's experts' rows [tokens * top, D], weighted and added up in the order of its choices, and its shared row, times
+// sigmoid(gate) if there is one: the sum over experts without a launch and a round trip of its own (8 tokens of
+// 2,048: 4.8 + 4.6 us before, 4.8 now; 2,047 tokens 9.9 + 10.8 and 15.8).
+template <typename ST>
+struct RowsOfExperts {
+  const float *y, *weights;
+  const ST* shared;
+  const float* gate;
+  int64_t shared_stride, gate_stride;
+  int top, D;
+  __device__ __forceinline__ Eight at(int row, int d) const {
+    Eight s;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s.v[e] = 0.f;
+    if (shared != nullptr) s = load_eight(shared + static_cast<size_t>(row) * shared_stride + d);   // (asked for first)
+    const float* from = y + static_cast<size_t>(row) * top * D + d;
+    const float* w = weights + static_cast<size_t>(row) * top;
+    Eight v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v.v[e] = 0.f;
+#pragma unroll 2
+    for (int k = 0; k < top; ++k) {
+      const Eight q = load_eight(from + static_cast<size_t>(k) * D);
+      const float wk = w[k];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v.v[e] = fmaf(wk, q.v[e], v.v[e]);
+    }
+    if (shared != nullptr) {
+      const float f = gate != nullptr ? 1.f + expf(-gate[static_cast<size_t>(row) * gate_stride]) : 1.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v.v[e] += gate != nullptr ? s.v[e] / f : s.v[e];
+    }
+    return v;
+  }
+};
+
+// The same for rows in pieces of eight (ADD: there is something to add).
+template <typename SRC, typename WT, typename OT, int NP, bool CENTERED, bool ADD>
 __global__ __launch_bounds__(256) void residual_add_next_norm_eights_kernel(
-    const YT* __restrict__ y, int64_t y_stride, float mult, float* __restrict__ residual, const WT* __restrict__ w,
-    const WT* __restrict__ b, float eps, float plus_one, OT* __restrict__ out, int D) {
+    SRC y, float mult, float* __restrict__ residual, const WT* __restrict__ w, const WT* __restrict__ b, float eps,
+    float plus_one, OT* __restrict__ out, int D) {
   __shared__ float scratch[16];
   const size_t rb = static_cast<size_t>(blockIdx.x) * D;
   Eight yv[ADD ? NP : 1], hv[NP], wv[NP], bv[CENTERED ? NP : 1];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int at = (p * 256 + threadIdx.x) * 8, d = at < D ? at : D - 8;
-    if constexpr (ADD) yv[p] = load_eight(y + static_cast<size_t>(blockIdx.x) * y_stride + d);
     hv[p] = load_eight(residual + rb + d);
     wv[p] = load_eight(w + d);
     if constexpr (CENTERED) bv[p] = load_eight(b + d);
+    if constexpr (ADD) yv[p] = y.at(blockIdx.x, d);
   }
   float ss = 0.f;
 #pragma unroll
@@ -358,10 +401,10 @@ template <typename YT, typename WT, typename OT, bool CENTERED>
 static void launch_residual_add_next_norm(const void* y, int64_t y_stride, float mult, float* residual, const void* w,
                                           const void* b, float eps, float plus_one, void* out, int T, int D,
                                           hipStream_t stream) {
+  const RowsAsTheyAre<YT> rows{static_cast<const YT*>(y), y_stride};
 #define SA_NEXT_NORM_EIGHTS(NP, ADD)                                                                                    \
-  residual_add_next_norm_eights_kernel<YT, WT, OT, NP, CENTERED, ADD><<<T, 256, 0, stream>>>(                           \
-      static_cast<const YT*>(y), y_stride, mult, residual, static_cast<const WT*>(w), static_cast<const WT*>(b), eps, \
-      plus_one, static_cast<OT*>(out), D)
+  residual_add_next_norm_eights_kernel<RowsAsTheyAre<YT>, WT, OT, NP, CENTERED, ADD><<<T, 256, 0, stream>>>(            \
+      rows, mult, residual, static_cast<const WT*>(w), static_cast<const WT*>(b), eps, plus_one, static_cast<OT*>(out), D)
   if (rows_in_eights(D, y != nullptr ? y_stride : 0, y, w, b, residual, out)) {
     if (y != nullptr) {
       if (D <= 2048) SA_NEXT_NORM_EIGHTS(1, true);
@@ -710,6 +753,51 @@ extern "C" int sa_residual_add_next_norm(const void* y, int y_dtype, int64_t y_s
 #undef SA_NEXT_NORM
 #undef SA_NEXT_NORM_C
   return check_launch("residual_add_next_norm");
+}
+
+extern "C" int sa_experts_add_next_norm_takes(int D, const void* shared, int64_t shared_stride, const void* residual, const void* w,
+                                              const void* b) {
+  return D <= 8192 && rows_in_eights(D, shared != nullptr ? shared_stride : 0, shared, residual, w, b, nullptr);
+}
+
+extern "C" int sa_experts_add_next_norm(const float* y, const float* weights, int top, const void* shared, int shared_dtype,
+                                        int64_t shared_stride, const float* gate, int64_t gate_stride, float mult, float* residual,
+                                        const void* w, const void* b, int w_dtype, float eps, int plus_one, void* out, int T, int D,
+                                        hipStream_t stream) {
+  if (T == 0) return 0;
+  SA_REQUIRE(T > 0 && D > 0 && top > 0 && y != nullptr && weights != nullptr && residual != nullptr && w != nullptr && out != nullptr &&
+                 (shared == nullptr || shared_stride >= D),
+             "experts_add_next_norm: bad sizes T=%d D=%d top=%d, or a null pointer", T, D, top);
+  SA_REQUIRE(sa_experts_add_next_norm_takes(D, shared, shared_stride, residual, w, b) && rows_in_eights(D, 0, y, out, nullptr, nullptr, nullptr),
+             "experts_add_next_norm: rows of %d are not whole aligned pieces of 8 entries (8192 at most)", D);
+  SA_REQUIRE(eps >= 0.f, "experts_add_next_norm: eps must not be negative");
+  SA_REQUIRE((w_dtype == kBF16 || w_dtype == kF32) && (shared == nullptr || shared_dtype == kF32 || shared_dtype == kBF16),
+             "experts_add_next_norm: weights and shared rows are bfloat16 or float32");
+  const float plus = plus_one ? 1.f : 0.f;
+#define SA_EXPERTS_NORM_NP(ST, WT, NP, C)                                                                                  \
+  residual_add_next_norm_eights_kernel<RowsOfExperts<ST>, WT, bf16, NP, C, true><<<T, 256, 0, stream>>>(                   \
+      RowsOfExperts<ST>{y, weights, static_cast<const ST*>(shared), gate, shared_stride, gate_stride, top, D}, mult, residual, \
+      static_cast<const WT*>(w), static_cast<const WT*>(b), eps, plus, static_cast<bf16*>(out), D)
+#define SA_EXPERTS_NORM_C(ST, WT, C)                          \
+  do {                                                        \
+    if (D <= 2048) SA_EXPERTS_NORM_NP(ST, WT, 1, C);          \
+    else if (D <= 4096) SA_EXPERTS_NORM_NP(ST, WT, 2, C);     \
+    else SA_EXPERTS_NORM_NP(ST, WT, 4, C);                    \
+  } while (0)
+#define SA_EXPERTS_NORM(ST, WT)                           \
+  do {                                                    \
+    if (b != nullptr) SA_EXPERTS_NORM_C(ST, WT, true);    \
+    else SA_EXPERTS_NORM_C(ST, WT, false);                \
+  } while (0)
+  const bool s32 = shared == nullptr || shared_dtype == kF32;
+  if (s32 && w_dtype == kBF16) SA_EXPERTS_NORM(float, bf16);
+  else if (s32) SA_EXPERTS_NORM(float, float);
+  else if (w_dtype == kBF16) SA_EXPERTS_NORM(bf16, bf16);
+  else SA_EXPERTS_NORM(bf16, float);
+#undef SA_EXPERTS_NORM
+#undef SA_EXPERTS_NORM_C
+#undef SA_EXPERTS_NORM_NP
+  return check_launch("experts_add_next_norm");
 }
 
 extern "C" int sa_gated_heads(const void* x, int x_dtype, int64_t x_stride, const void* g, int g_dtype, int64_t g_stride,

@@ -1,5 +1,6 @@
 // A feed-forward of routed experts over a ragged batch of tokens.
 //
+//   route_few_kernel      for a handful of tokens: the router's product, its choice and the sort in one launch
 //   route_kernel          softmax of the router's logits, the `top` largest scores and their experts
 //   sort_kernel           the (token, choice) pairs in the order of their experts, cut into tiles of rows of one expert
 //   expert_product_kernel h = act(Wg[e] x) * (Wu[e] x) for every pair, rows in the sorted order; then
@@ -21,23 +22,23 @@ constexpr int kTileRowsWide = 128;   // or 128, for the wide product kernel alon
 constexpr int kGridMax = 65535;      // a grid's second and third index
 
 // A wave per token.  scores = softmax(logits); `top` times the largest score that is left (of equal ones the lowest
-// index); weight = score * scale.
-__global__ __launch_bounds__(kWave) void route_kernel(const float* __restrict__ logits, int64_t stride, int E, int top,
-                                                      float scale, int* __restrict__ experts,
-                                                      float* __restrict__ weights) {
-  const int t = blockIdx.x, lane = threadIdx.x;
-  float z[kRouteSlots];
+// index); weight = score * scale.  SLOTS: experts a lane holds.
+template <int SLOTS>
+__device__ __forceinline__ void choose_plain(const float* __restrict__ logits, int E, int top, float scale, int* experts,
+                                             float* weights) {
+  const int lane = threadIdx.x % kWave;
+  float z[SLOTS];
   float mx = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < kRouteSlots; ++i) {
+  for (int i = 0; i < SLOTS; ++i) {
     const int e = lane + i * kWave;
-    z[i] = e < E ? logits[static_cast<size_t>(t) * stride + e] : -INFINITY;
+    z[i] = e < E ? logits[e] : -INFINITY;
     mx = fmaxf(mx, z[i]);
   }
   mx = wave_max(mx);
   float sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < kRouteSlots; ++i) {
+  for (int i = 0; i < SLOTS; ++i) {
     z[i] = (lane + i * kWave) < E ? expf(z[i] - mx) : -1.f;   // (a score is never negative: -1 marks what is taken or absent)
     sum += z[i] > 0.f ? z[i] : 0.f;
   }
@@ -45,22 +46,29 @@ __global__ __launch_bounds__(kWave) void route_kernel(const float* __restrict__ 
   for (int r = 0; r < top; ++r) {
     float best = -1.f;
 #pragma unroll
-    for (int i = 0; i < kRouteSlots; ++i) best = fmaxf(best, z[i]);
+    for (int i = 0; i < SLOTS; ++i) best = fmaxf(best, z[i]);
     best = wave_max(best);
     float mine = 1e9f;
 #pragma unroll
-    for (int i = kRouteSlots - 1; i >= 0; --i)
+    for (int i = SLOTS - 1; i >= 0; --i)
       if (z[i] == best) mine = static_cast<float>(lane + i * kWave);
     const float first = -wave_max(-mine);
     const int e = first < static_cast<float>(E) ? static_cast<int>(first) : E - 1;   // (logits that are no numbers: some expert)
 #pragma unroll
-    for (int i = 0; i < kRouteSlots; ++i)
+    for (int i = 0; i < SLOTS; ++i)
       if (lane + i * kWave == e) z[i] = -1.f;
     if (lane == 0) {
-      experts[static_cast<size_t>(t) * top + r] = e;
-      weights[static_cast<size_t>(t) * top + r] = best / sum * scale;
+      experts[r] = e;
+      weights[r] = best / sum * scale;
     }
   }
+}
+
+__global__ __launch_bounds__(kWave) void route_kernel(const float* __restrict__ logits, int64_t stride, int E, int top,
+                                                      float scale, int* __restrict__ experts,
+                                                      float* __restrict__ weights) {
+  const size_t t = blockIdx.x;
+  choose_plain<kRouteSlots>(logits + t * stride, E, top, scale, experts + t * top, weights + t * top);
 }
 
 // A wave per token, for routers with options.  bias[e] (or null) is added to the logits first.  Scores are sigmoids of the
@@ -71,49 +79,58 @@ __global__ __launch_bounds__(kWave) void route_kernel(const float* __restrict__ 
 // scores can be chosen (of equal ones the lowest index, for groups and for experts).  weight = score * scale without
 // the correction, with renorm >= 0 divided by the chosen scores' sum + renorm.  Choice scores can be negative: what is
 // taken or shut out is -inf.
-__global__ __launch_bounds__(kWave) void route_choice_kernel(const float* __restrict__ logits, int64_t stride, int E,
-                                                             int top, float scale, const void* __restrict__ bias,
-                                                             int bias_dtype, const void* __restrict__ correction,
-                                                             int corr_dtype, int groups, int keep, int softmax,
-                                                             int group_best, float renorm, int* __restrict__ experts,
-                                                             float* __restrict__ weights) {
-  __shared__ float choice_s[kRouteSlots * kWave];
-  __shared__ float group_s[kRouteSlots * kWave];
-  const int t = blockIdx.x, lane = threadIdx.x;
-  float s[kRouteSlots], c[kRouteSlots];
+struct RouterOptions {
+  const void *bias, *correction;
+  int bias_dtype, corr_dtype, groups, keep, softmax, group_best;
+  float renorm;
+};
+// What a wave wrote to LDS that is its own, its other lanes read from here on (a wave's LDS accesses run in their order: this
+// keeps the compiler to it, and no other wave is waited for).
+__device__ __forceinline__ void wave_ordered() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// choice_s, group_s: SLOTS * 64 words of LDS of the wave's own.
+template <int SLOTS>
+__device__ __forceinline__ void choose_with_options(const float* __restrict__ logits, int E, int top, float scale,
+                                                    const RouterOptions& o, float* choice_s, float* group_s, int* experts,
+                                                    float* weights) {
+  const int lane = threadIdx.x % kWave;
+  float s[SLOTS], c[SLOTS];
   float mx = -INFINITY, sum = 0.f;
 #pragma unroll
-  for (int i = 0; i < kRouteSlots; ++i) {
+  for (int i = 0; i < SLOTS; ++i) {
     const int e = lane + i * kWave;
-    s[i] = e < E ? logits[static_cast<size_t>(t) * stride + e] : -INFINITY;
-    if (bias != nullptr && e < E) s[i] += load_f(bias, bias_dtype, e);
+    s[i] = e < E ? logits[e] : -INFINITY;
+    if (o.bias != nullptr && e < E) s[i] += load_f(o.bias, o.bias_dtype, e);
     mx = fmaxf(mx, s[i]);
   }
-  if (softmax == 1) {
+  if (o.softmax == 1) {
     mx = wave_max(mx);
 #pragma unroll
-    for (int i = 0; i < kRouteSlots; ++i) {
+    for (int i = 0; i < SLOTS; ++i) {
       s[i] = lane + i * kWave < E ? expf(s[i] - mx) : 0.f;
       sum += s[i];
     }
     sum = wave_sum(sum);
   }
 #pragma unroll
-  for (int i = 0; i < kRouteSlots; ++i) {
+  for (int i = 0; i < SLOTS; ++i) {
     const int e = lane + i * kWave;
     c[i] = -INFINITY;
     if (e < E) {
-      if (softmax != 2) s[i] = softmax ? s[i] / sum : 1.f / (1.f + expf(-s[i]));
-      c[i] = correction != nullptr ? s[i] + load_f(correction, corr_dtype, e) : s[i];
+      if (o.softmax != 2) s[i] = o.softmax ? s[i] / sum : 1.f / (1.f + expf(-s[i]));
+      c[i] = o.correction != nullptr ? s[i] + load_f(o.correction, o.corr_dtype, e) : s[i];
       choice_s[e] = c[i];
     } else {
       s[i] = 0.f;
     }
   }
-  if (groups > 1) {
-    __syncthreads();
-    const int per = E / groups;
-    for (int g = lane; g < groups; g += kWave) {
+  if (o.groups > 1) {
+    wave_ordered();
+    const int per = E / o.groups;
+    for (int g = lane; g < o.groups; g += kWave) {
       float a = -INFINITY, b = -INFINITY;   // the two largest of the group
       for (int k = 0; k < per; ++k) {
         const float v = choice_s[g * per + k];
@@ -124,44 +141,44 @@ __global__ __launch_bounds__(kWave) void route_choice_kernel(const float* __rest
           b = v;
         }
       }
-      group_s[g] = per > 1 && group_best > 1 ? a + b : a;
+      group_s[g] = per > 1 && o.group_best > 1 ? a + b : a;
     }
-    __syncthreads();
+    wave_ordered();
     // the `keep` best groups, one after the other; lane 0 marks them by sign in LDS
-    for (int r = 0; r < keep; ++r) {
+    for (int r = 0; r < o.keep; ++r) {
       float best = -INFINITY;
-      for (int g = lane; g < groups; g += kWave) best = fmaxf(best, group_s[g]);
+      for (int g = lane; g < o.groups; g += kWave) best = fmaxf(best, group_s[g]);
       best = wave_max(best);
-      float mine = static_cast<float>(groups - 1);
-      for (int g = lane; g < groups; g += kWave)
+      float mine = static_cast<float>(o.groups - 1);
+      for (int g = lane; g < o.groups; g += kWave)
         if (group_s[g] == best && static_cast<float>(g) < mine) mine = static_cast<float>(g);
       const int g_best = static_cast<int>(-wave_max(-mine));
-      __syncthreads();
+      wave_ordered();
       if (lane == 0) group_s[g_best] = -INFINITY;   // taken: -inf marks a group that stays
-      __syncthreads();
+      wave_ordered();
     }
 #pragma unroll
-    for (int i = 0; i < kRouteSlots; ++i) {
+    for (int i = 0; i < SLOTS; ++i) {
       const int e = lane + i * kWave;
       if (e < E && group_s[e / per] != -INFINITY) c[i] = -INFINITY;
     }
   }
-  __syncthreads();   // the choice scores in LDS have been read: the chosen scores take their place
+  wave_ordered();   // the choice scores in LDS have been read: the chosen scores take their place
   float total = 0.f;
   for (int r = 0; r < top; ++r) {
     float best = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < kRouteSlots; ++i) best = fmaxf(best, c[i]);
+    for (int i = 0; i < SLOTS; ++i) best = fmaxf(best, c[i]);
     best = wave_max(best);
     float mine = 1e9f;
 #pragma unroll
-    for (int i = kRouteSlots - 1; i >= 0; --i)
+    for (int i = SLOTS - 1; i >= 0; --i)
       if (c[i] == best && lane + i * kWave < E) mine = static_cast<float>(lane + i * kWave);
     const float first = -wave_max(-mine);
     const int e = first < static_cast<float>(E) ? static_cast<int>(first) : E - 1;   // (logits that are no numbers: some expert)
     float w = 0.f;
 #pragma unroll
-    for (int i = 0; i < kRouteSlots; ++i)
+    for (int i = 0; i < SLOTS; ++i)
       if (lane + i * kWave == e) {
         c[i] = -INFINITY;
         w = s[i];
@@ -169,21 +186,30 @@ __global__ __launch_bounds__(kWave) void route_choice_kernel(const float* __rest
     w = wave_sum(w);   // (one lane holds it, the others 0)
     total += w;
     if (lane == 0) {
-      experts[static_cast<size_t>(t) * top + r] = e;
+      experts[r] = e;
       choice_s[r] = w;
     }
   }
-  __syncthreads();
-  if (softmax == 2) {
+  wave_ordered();
+  if (o.softmax == 2) {
     float best = -INFINITY, among = 0.f;
     for (int r = 0; r < top; ++r) best = fmaxf(best, choice_s[r]);
     for (int r = 0; r < top; ++r) among += expf(choice_s[r] - best);
-    for (int r = lane; r < top; r += kWave)
-      weights[static_cast<size_t>(t) * top + r] = expf(choice_s[r] - best) / among * scale;
+    for (int r = lane; r < top; r += kWave) weights[r] = expf(choice_s[r] - best) / among * scale;
     return;
   }
-  const float by = renorm >= 0.f ? total + renorm : 1.f;
-  for (int r = lane; r < top; r += kWave) weights[static_cast<size_t>(t) * top + r] = choice_s[r] / by * scale;
+  const float by = o.renorm >= 0.f ? total + o.renorm : 1.f;
+  for (int r = lane; r < top; r += kWave) weights[r] = choice_s[r] / by * scale;
+}
+
+__global__ __launch_bounds__(kWave) void route_choice_kernel(const float* __restrict__ logits, int64_t stride, int E,
+                                                             int top, float scale, RouterOptions options,
+                                                             int* __restrict__ experts, float* __restrict__ weights) {
+  __shared__ float choice_s[kRouteSlots * kWave];
+  __shared__ float group_s[kRouteSlots * kWave];
+  const size_t t = blockIdx.x;
+  choose_with_options<kRouteSlots>(logits + t * stride, E, top, scale, options, choice_s, group_s, experts + t * top,
+                                   weights + t * top);
 }
 
 // One workgroup.  plan: [0] number of tiles; [1 .. 1 + 3 * max_tiles): per tile its expert, its first row in the sorted order
@@ -237,6 +263,117 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 __device__ __forceinline__ bf16x8 load8(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
 
+// The router of a step of at most 16 tokens and 128 experts, from the rows to the plan: logits = x . router^T, every token's
+// choice, and the pairs in the order of their experts, in one workgroup of 16 waves.  Three launches that each have next to
+// nothing to do become one: the product by itself took 4.5 us, the choice 7.0 and the sort 3.6 (8 tokens, 2,048 wide, 16
+// experts), this kernel 10.5.  Bound by its chain of waits: rows and weights from L2, a sum over the waves through LDS, a
+// token's choices one after the other.
+//   product   a wave takes 1 / 16 of K for every tile of 16 experts; the waves' sums are added up in their order
+//   choice    wave t is token t's
+//   sort      lane e counts expert e's pairs; an expert's pairs stay in their order
+// logits [T, stride] (32-bit): the first E are the experts', what follows (a shared expert's score) is only written.
+constexpr int kFewTokens = 16, kFewSlots = 2, kFewPairs = 128;
+struct RouterScratch {
+  float logits[kFewTokens][kFewSlots * kWave + 16];
+  float sums[kFewTokens][16 * 17];   // the waves' tiles of 16 experts x 16 tokens
+  float choice[kFewTokens][kFewSlots * kWave], group[kFewTokens][kFewSlots * kWave];
+  int pairs[kFewPairs];
+};
+__global__ __launch_bounds__(1024) void route_few_kernel(const bf16* __restrict__ x, int64_t x_stride, const bf16* __restrict__ w,
+                                                         int T, int D, int rows, int E, int top, float scale, int plain,
+                                                         RouterOptions options, float* __restrict__ logits,
+                                                         int* __restrict__ experts, float* __restrict__ weights,
+                                                         int* __restrict__ sorted, int* __restrict__ plan) {
+  extern __shared__ __align__(16) char few_lds[];
+  RouterScratch& l = *reinterpret_cast<RouterScratch*>(few_lds);
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r = lane % 16, kq = lane / 16, chunks = D / 32;
+  const int c0 = chunks * wave / 16, c1 = chunks * (wave + 1) / 16;
+  const bf16* row = x + static_cast<size_t>(r < T ? r : T - 1) * x_stride + kq * 8;
+  for (int n0 = 0; n0 < rows; n0 += 16) {
+    const bf16* tile = w + static_cast<size_t>(n0 / 16) * chunks * 512 + lane * 8;
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int kAhead = 4;
+    for (int c = c0; c < c1; c += kAhead) {
+      bf16x8 wv[kAhead], xv[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {   // (a chunk behind the range is read again and not used)
+        const int at = c + i < c1 ? c + i : c1 - 1;
+        wv[i] = load8(tile + static_cast<size_t>(at) * 512);
+        xv[i] = load8(row + at * 32);
+      }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+        if (c + i < c1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i], xv[i], acc, 0, 0, 0);   // (uniform)
+    }
+    if (n0 > 0) __syncthreads();   // the tile before has been added up
+#pragma unroll
+    for (int v = 0; v < 4; ++v) l.sums[wave][(4 * kq + v) * 17 + r] = acc[v];   // [expert][token]
+    __syncthreads();
+    if (tid < 256) {
+      const int n = tid % 16, t = tid / 16;
+      float sum = 0.f;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) sum += l.sums[k][n * 17 + t];
+      l.logits[t][n0 + n] = sum;
+      if (t < T && n0 + n < rows) logits[static_cast<size_t>(t) * rows + n0 + n] = sum;
+    }
+  }
+  __syncthreads();
+  if (wave < T) {
+    const int t = wave;
+    int* chosen = l.pairs + t * top;
+    float* weight = l.sums[wave];   // (the sums have been read)
+    if (plain) choose_plain<kFewSlots>(l.logits[t], E, top, scale, chosen, weight);
+    else choose_with_options<kFewSlots>(l.logits[t], E, top, scale, options, l.choice[wave], l.group[wave], chosen, weight);
+    wave_ordered();
+    for (int k = lane; k < top; k += kWave) {
+      experts[t * top + k] = chosen[k];
+      weights[t * top + k] = weight[k];
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  // A lane has pairs lane, lane + 64 and experts lane, lane + 64; every pair's expert passes by all lanes once (a lane read: no
+  // chain of LDS reads, no prefix sums).
+  const int P = T * top;
+  int mine[kFewSlots], place[kFewSlots] = {}, count[kFewSlots] = {}, below[kFewSlots] = {};
+#pragma unroll
+  for (int i = 0; i < kFewSlots; ++i) mine[i] = lane + i * kWave < P ? l.pairs[lane + i * kWave] : -1;
+#pragma unroll
+  for (int j = 0; j < kFewSlots; ++j)
+    for (int q = 0; q < kWave && j * kWave + q < P; ++q) {
+      const int e = __builtin_amdgcn_readlane(mine[j], q);
+#pragma unroll
+      for (int i = 0; i < kFewSlots; ++i) {
+        place[i] += e < mine[i] || (e == mine[i] && j * kWave + q < lane + i * kWave) ? 1 : 0;
+        count[i] += e == lane + i * kWave ? 1 : 0;
+        below[i] += e < lane + i * kWave ? 1 : 0;
+      }
+    }
+  int before = 0;   // tiles of the experts before
+#pragma unroll
+  for (int i = 0; i < kFewSlots; ++i) {
+    const int tiles = (count[i] + 15) / 16, most = 1 + (kFewPairs - 1) / 16;
+    int n = before;
+    for (int k = 1; k <= most; ++k) {   // (a second tile only where logits that are no numbers gave one expert to a token twice)
+      const uint64_t has = __ballot(tiles >= k);
+      if (has == 0) break;
+      n += __popcll(has & ((uint64_t{1} << lane) - 1));
+      before += __popcll(has);
+    }
+    for (int k = 0; k < tiles; ++k) {
+      const int left = count[i] - k * 16;
+      plan[1 + 3 * (n + k)] = lane + i * kWave;
+      plan[2 + 3 * (n + k)] = below[i] + k * 16;
+      plan[3 + 3 * (n + k)] = left < 16 ? left : 16;
+    }
+    if (lane + i * kWave < P) sorted[place[i]] = lane + i * kWave;
+  }
+  if (lane == 0) plan[0] = before;
+}
+
 // h[row, f] = act(x[token] . Wg[e, f]) * (x[token] . Wu[e, f]); GATED false: y[pair, n] = h[row] . Wd[e, n].
 // A workgroup of one wave takes one tile of rows and 16 columns (for all RT sub-tiles of 16 rows): nothing is shared between
 // waves, and small workgroups even out over the CUs, of which the few experts that a decode step reads would give some two or
@@ -244,16 +381,40 @@ __device__ __forceinline__ bf16x8 load8(const bf16* p) { return *reinterpret_cas
 // bfloat16: the weights are tiled ([E][N / 16][K / 32][64][8], see the product kernels), a wave's operands are one
 // 16-byte load a lane (rows that are not 16-byte aligned are read element by element); 32-bit: row-major weights
 // [E][N][K], a lane per (row, column) of the tile in turn.
-template <typename T, bool GATED, int RT>
+// SHARED (bfloat16, few tokens): the first tile of the grid is the shared feed-forward's, all tokens' rows against its own
+// weights (gate and factor tile by tile in turn, as the dense gated product has them): two launches of 5 to 7 us less a layer,
+// and its 25 MB ride along with the experts' (8 tokens,
+// feed-forwards of 2,048 x 2,048, 16 experts: 34.7 + 7.1 us before and 37.5 now, down 17.5 + 5.5 and 19.3).
+struct SharedExpert {
+  const bf16* a;
+  const bf16* w;
+  void* out;
+  int64_t a_stride, out_stride;
+  int N, K, rows;
+  float limit;
+};
+template <typename T, bool GATED, int RT, bool SHARED = false>
 __global__ __launch_bounds__(kWave) void expert_product_kernel(
     const T* __restrict__ a, int64_t a_stride, int a_by_token, int top, const T* __restrict__ w1, const T* __restrict__ w2,
     int N, int K, const int* __restrict__ sorted, const int* __restrict__ plan, int act, float limit,
-    void* __restrict__ out, int64_t out_stride, int out_by_pair, int activate) {
+    void* __restrict__ out, int64_t out_stride, int out_by_pair, int activate, SharedExpert sh) {
   // activate (without a second weight): out[row] = act(a . w1[e]^T) in a's type instead of the 32-bit product
-  const int tile = blockIdx.z * kGridMax + blockIdx.y;   // (gridDim would be one more load in front of everything)
-  if (tile >= plan[0]) return;
-  const int e = plan[1 + 3 * tile], row0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
+  int tile = blockIdx.z * kGridMax + blockIdx.y;   // (gridDim would be one more load in front of everything)
+  const bool shared = SHARED && tile == 0;
+  if constexpr (SHARED) --tile;
   const int lane = threadIdx.x, n0 = blockIdx.x * 16;
+  int e = 0, row0 = 0, rows;
+  if (shared) {
+    rows = sh.rows;
+    if constexpr (SHARED) {
+      a = sh.a, a_stride = sh.a_stride, out = sh.out, out_stride = sh.out_stride;
+      N = sh.N, K = sh.K, limit = sh.limit, out_by_pair = 0;
+    }
+  } else {
+    if (tile >= plan[0]) return;
+    e = plan[1 + 3 * tile], row0 = plan[2 + 3 * tile], rows = plan[3 + 3 * tile];
+  }
+  if constexpr (SHARED) if (n0 >= N) return;   // (the grid covers the wider of the two)
   if constexpr (sizeof(T) == 2) {
     const int Nt = (N + 15) / 16, Kt = (K + 31) / 32;
     const int r = lane % 16, kq = lane / 16;
@@ -263,12 +424,18 @@ __global__ __launch_bounds__(kWave) void expert_product_kernel(
 #pragma unroll
     for (int s = 0; s < RT; ++s) {
       const int rr = s * 16 + r < rows ? s * 16 + r : rows - 1;
-      pairs[s] = sorted[row0 + rr];
-      arow[s] = a + static_cast<size_t>(a_by_token ? pairs[s] / top : row0 + rr) * a_stride;
+      pairs[s] = shared ? rr : sorted[row0 + rr];
+      arow[s] = a + static_cast<size_t>(a_by_token && !shared ? pairs[s] / top : row0 + rr) * a_stride;
     }
     const size_t wbase = (static_cast<size_t>(e) * Nt + n0 / 16) * Kt;
     const bf16* g = reinterpret_cast<const bf16*>(w1) + wbase * 512 + lane * 8;
     const bf16* u = GATED ? reinterpret_cast<const bf16*>(w2) + wbase * 512 + lane * 8 : nullptr;
+    if constexpr (SHARED) {
+      if (shared) {
+        g = sh.w + (GATED ? 2 : 1) * wbase * 512 + lane * 8;
+        u = g + static_cast<size_t>(Kt) * 512;
+      }
+    }
     floatx4 accg[RT], accu[RT];
 #pragma unroll
     for (int s = 0; s < RT; ++s) accg[s] = accu[s] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -584,9 +751,39 @@ extern "C" int sa_route_choice(const float* logits, int64_t stride, int T, int E
   SA_REQUIRE(bias == nullptr || bias_dtype == kF32 || bias_dtype == kBF16, "route_choice: unknown dtype %d", bias_dtype);
   SA_REQUIRE(softmax >= 0 && softmax <= 2 && (softmax != 2 || renorm < 0.f),
              "route_choice: scores %d (0 sigmoid, 1 softmax, 2 the chosen logits' softmax, which sums to 1 by itself)", softmax);
-  route_choice_kernel<<<T, kWave, 0, stream>>>(logits, stride, E, top, scale, bias, bias_dtype, correction, corr_dtype, groups, keep,
-                                               softmax, group_best, renorm, experts, weights);
+  route_choice_kernel<<<T, kWave, 0, stream>>>(
+      logits, stride, E, top, scale,
+      RouterOptions{bias, correction, bias_dtype, corr_dtype, groups, keep, softmax, group_best, renorm}, experts, weights);
   return check_launch("route_choice");
+}
+
+extern "C" int sa_route_few_takes(const void* x, int64_t x_stride, int T, int D, int rows, int E, int top) {
+  // (the weights all go through one CU: 256 KiB of them take as long as the launch of the product that they save)
+  return T >= 1 && T <= kFewTokens && D >= 32 && D % 32 == 0 && x_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && E >= 1 &&
+         E <= kFewSlots * kWave && rows >= E && rows <= E + 16 && static_cast<int64_t>(rows) * D <= 128 * 1024 && top >= 1 &&
+         top <= E && T * top <= kFewPairs;
+}
+
+extern "C" int sa_route_few(const void* x, int64_t x_stride, const void* w, int T, int D, int rows, int E, int top, float scale,
+                            int plain, const void* bias, int bias_dtype, const void* correction, int corr_dtype, int groups, int keep,
+                            int softmax, int group_best, float renorm, float* logits, int* experts, float* weights, int* sorted,
+                            int* plan, int plan_words, hipStream_t stream) {
+  SA_REQUIRE(sa_route_few_takes(x, x_stride, T, D, rows, E, top) && x_stride >= D, "route_few: T=%d D=%d experts=%d top=%d are not taken", T,
+             D, E, top);
+  SA_REQUIRE(x != nullptr && w != nullptr && logits != nullptr && experts != nullptr && weights != nullptr && sorted != nullptr &&
+                 plan != nullptr && plan_words >= 1 + 3 * sa_expert_tiles_max(T * top, E, 16),
+             "route_few: a null pointer, or a plan too short");
+  SA_REQUIRE(groups >= 1 && E % groups == 0 && keep >= 1 && keep <= groups && (group_best == 1 || group_best == 2) &&
+                 top <= keep * (E / groups) && softmax >= 0 && softmax <= 2 && (softmax != 2 || renorm < 0.f),
+             "route_few: %d experts in %d groups of which %d stay, scores %d", E, groups, keep, softmax);
+  SA_REQUIRE((correction == nullptr || corr_dtype == kF32 || corr_dtype == kBF16) &&
+                 (bias == nullptr || bias_dtype == kF32 || bias_dtype == kBF16),
+             "route_few: unknown dtype");
+  route_few_kernel<<<1, 1024, sizeof(RouterScratch), stream>>>(
+      static_cast<const bf16*>(x), x_stride, static_cast<const bf16*>(w), T, D, rows, E, top, scale, plain,
+      RouterOptions{bias, correction, bias_dtype, corr_dtype, groups, keep, softmax, group_best, renorm}, logits, experts, weights,
+      sorted, plan);
+  return check_launch("route_few");
 }
 
 extern "C" int sa_expert_tiles_max(int P, int E, int tile_rows) {
@@ -646,7 +843,7 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
 #define SA_EXPERT(T, G, RT)                                                                                            \
   expert_product_kernel<T, G, RT><<<dim3((N + 15) / 16, tiles_y, tiles_z), kWave, 0, stream>>>(                          \
       static_cast<const T*>(a), a_stride, a_by_token, top, static_cast<const T*>(w1), static_cast<const T*>(w2), N, K,   \
-      sorted, plan, act, limit, out, out_stride, out_by_pair, activate)
+      sorted, plan, act, limit, out, out_stride, out_by_pair, activate, SharedExpert{})
   // Tiles of 64 and 128 rows go to the wide product kernel where it takes the operands; the others to the kernel of 64 rows here.
   const bool by_wide = dtype == kBF16 && tile_rows != 16 && tiles <= kGridMax && ((gated || activate) ? !out_by_pair : out_by_pair != 0) &&
                        gemm_wide_routed_takes(N, K, a_stride, a_by_token ? (P + top - 1) / top : P, out_stride, a, w1, w2, out, tile_rows);
@@ -677,6 +874,35 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
   }
 #undef SA_EXPERT
   return check_launch("expert_product");
+}
+
+extern "C" int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w1, const void* w2, int N,
+                                        int K, const int* sorted, const int* plan, int P, int E, int act, float limit, void* out,
+                                        int64_t out_stride, int out_by_pair, int activate, const void* shared_a,
+                                        int64_t shared_a_stride, const void* shared_w, int shared_N, int shared_K, int T,
+                                        float shared_limit, void* shared_out, int64_t shared_out_stride, hipStream_t stream) {
+  SA_REQUIRE(!activate || w2 == nullptr, "expert_product: a gated product has its activation already");
+  SA_REQUIRE(P > 0 && E > 0 && N > 0 && K > 0 && top > 0 && a_stride >= K && out_stride >= N && T > 0 && T <= 16 && P == T * top &&
+                 shared_N > 0 && shared_K > 0 && shared_a_stride >= shared_K && shared_out_stride >= shared_N,
+             "expert_product_shared: bad sizes P=%d E=%d N=%d K=%d, %d tokens (at most 16), N=%d K=%d", P, E, N, K, T, shared_N, shared_K);
+  SA_REQUIRE(a != nullptr && w1 != nullptr && sorted != nullptr && plan != nullptr && out != nullptr && shared_a != nullptr &&
+                 shared_w != nullptr && shared_out != nullptr,
+             "expert_product_shared: a null pointer");
+  SA_REQUIRE(act >= 0 && act < (w2 != nullptr ? kNumGatedRules : kNumActivations), "expert_product: unknown activation %d", act);
+  SA_REQUIRE(act != kActClampedGlu || (limit > 0.f && shared_limit > 0.f), "expert_product: the clamped gated product needs a positive limit");
+  const int tiles = 1 + sa_expert_tiles_max(P, E, 16);   // (at most 1 + 16 + P: far from the grid's end)
+  const dim3 grid(((N > shared_N ? N : shared_N) + 15) / 16, tiles);
+  const SharedExpert sh{static_cast<const bf16*>(shared_a), static_cast<const bf16*>(shared_w), shared_out, shared_a_stride,
+                        shared_out_stride, shared_N, shared_K, T, shared_limit};
+  SA_REQUIRE(tiles <= kGridMax, "expert_product_shared: %d tiles", tiles);
+#define SA_EXPERT_SHARED(G)                                                                                            \
+  expert_product_kernel<bf16, G, 1, true><<<grid, kWave, 0, stream>>>(                                                  \
+      static_cast<const bf16*>(a), a_stride, a_by_token, top, static_cast<const bf16*>(w1), static_cast<const bf16*>(w2), N, K, \
+      sorted, plan, act, limit, out, out_stride, out_by_pair, activate, sh)
+  if (w2 != nullptr) SA_EXPERT_SHARED(true);
+  else SA_EXPERT_SHARED(false);
+#undef SA_EXPERT_SHARED
+  return check_launch("expert_product_shared");
 }
 
 extern "C" int sa_expert_combine(const float* y, const float* weights, int top, const void* shared, int shared_dtype,

@@ -1000,13 +1000,17 @@ def residual_add_norm(y: "torch.Tensor | PartialSums | None", residual: torch.Te
     return out
 
 
-def residual_add_next_norm(y: "torch.Tensor | PartialSums | None", residual: torch.Tensor, weight: torch.Tensor, *,
+def residual_add_next_norm(y: "torch.Tensor | PartialSums | ExpertSums | None", residual: torch.Tensor, weight: torch.Tensor, *,
                            eps: float, plus_one: bool = False, mult: float = 1.0, bias: torch.Tensor | None = None,
                            out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """residual += mult * y (y None: nothing is added; a y whose rows are one row expanded adds that row to all);
     returns residual / sqrt(mean(residual^2) + eps) * (weight + plus_one) in out_dtype, or with a bias the layer norm
     (residual - mean) / sqrt(variance + eps) * (weight + plus_one) + bias: one pass over the rows."""
-    if isinstance(y, PartialSums):
+    if isinstance(y, ExpertSums):
+        done = y.add_next_norm(residual, weight, eps=eps, plus_one=plus_one, mult=mult, bias=bias, out_dtype=out_dtype or y.dtype)
+        if done is not None:
+            return done
+    if isinstance(y, (PartialSums, ExpertSums)):
         y = y.materialize()
     _dev(y, residual, weight, bias)
     T, D = residual.shape
@@ -1983,13 +1987,108 @@ def route_choice(logits: torch.Tensor, top: int, scale: float, *, correction: to
     return experts, weights
 
 
+class ExpertSums:
+    """What a token's experts gave, not yet weighted and added up (`expert_sums`): `residual_add_next_norm`
+    takes it in place of y and adds the rows up itself, which saves the sum's kernel and its round trip; anyone else calls
+    `materialize()`.  (The rows are tensors of its own: nothing else writes there.)"""
+
+    def __init__(self, y: torch.Tensor, weights: torch.Tensor, shared: torch.Tensor | None, shared_gate: torch.Tensor | None,
+                 dtype: torch.dtype):
+        self.y, self.weights, self.shared, self.shared_gate = y, weights, shared, shared_gate
+        self.shape, self.dtype, self.device = (weights.shape[0], y.shape[1]), dtype, y.device
+
+    def _rows_args(self):
+        sh, gate = self.shared, self.shared_gate
+        return (_ptr(self.y), _ptr(self.weights), self.weights.shape[1], _ptr(sh), _code(sh) if sh is not None else 0,
+                _rows(sh, "routed_experts: shared") if sh is not None else 0, _ptr(gate), gate.stride(0) if gate is not None else 0)
+
+    def materialize(self) -> torch.Tensor:
+        T, D = self.shape
+        out = torch.empty((T, D), dtype=self.dtype, device=self.device)
+        _lib.call("sa_expert_combine", *self._rows_args(), _ptr(out), _code(out), D, T, D, _stream())
+        return out
+
+    def add_next_norm(self, residual, weight, *, eps, plus_one, mult, bias, out_dtype) -> torch.Tensor | None:
+        """`residual_add_next_norm` with these rows as y, or None where its kernel does not take the sizes."""
+        T, D = self.shape
+        if out_dtype != torch.bfloat16 or tuple(residual.shape) != (T, D) or residual.dtype != torch.float32 \
+                or not residual.is_contiguous() or weight.numel() != D or not weight.is_contiguous() \
+                or (bias is not None and (bias.numel() != D or not bias.is_contiguous() or bias.dtype != weight.dtype)) \
+                or not _lib.load().sa_experts_add_next_norm_takes(
+                    D, _ptr(self.shared), self.shared.stride(0) if self.shared is not None else 0, _ptr(residual), _ptr(weight),
+                    _ptr(bias)):
+            return None
+        _dev(self.y, residual, weight, bias)
+        out = torch.empty((T, D), dtype=out_dtype, device=self.device)
+        _lib.call("sa_experts_add_next_norm", *self._rows_args(), float(mult), _ptr(residual), _ptr(weight), _ptr(bias),
+                  _code(weight), float(eps), int(plus_one), _ptr(out), T, D, _stream())
+        return out
+
+
+def route_few_takes(x: torch.Tensor, router, num_experts: int, top: int) -> bool:
+    """Whether `route_few` takes a step of these rows (bfloat16, a handful of tokens, a tiled router)."""
+    return x.is_cuda and x.dtype == torch.bfloat16 and isinstance(router, TiledWeight) and router.cols == x.shape[1] \
+        and x.stride(1) == 1 and bool(_lib.load().sa_route_few_takes(_ptr(x), x.stride(0), x.shape[0], x.shape[1], router.rows,
+                                                                     int(num_experts), int(top)))
+
+
+def route_few(x: torch.Tensor, router: TiledWeight, num_experts: int, top: int, scale: float, *,
+              options: dict | None = None) -> tuple:
+    """The router of a few tokens in one launch: (logits float32 [T, rows of the router], experts, weights, (sorted, plan)) with
+    the choice as `route` (options None) or `route_choice(**options)` makes it from the first `num_experts` logits, and the order
+    of the pairs as `routed_experts` takes it."""
+    o = options or {}
+    correction, bias, softmax = o.get("correction"), o.get("bias"), o.get("softmax", False)
+    _dev(x, router.data, correction, bias)
+    if not route_few_takes(x, router, num_experts, top):
+        raise KernelError(f"route_few: {tuple(x.shape)} rows and {num_experts} experts are not taken")
+    T, D = x.shape
+    E, dev = int(num_experts), x.device
+    for t, what in ((correction, "correction"), (bias, "bias")):
+        if t is not None and (t.numel() != E or not t.is_contiguous()):
+            raise KernelError(f"route_few: a {what} of {t.numel()} entries for {E} experts")
+    if softmax not in (False, True, "chosen") or (softmax == "chosen" and o.get("renorm") is not None):
+        raise KernelError("route_few: softmax is False, True or 'chosen' (whose weights sum to one: no renorm)")
+    renorm = o.get("renorm")
+    logits = torch.empty((T, router.rows), dtype=torch.float32, device=dev)
+    experts = torch.empty((T, top), dtype=torch.int32, device=dev)
+    weights = torch.empty((T, top), dtype=torch.float32, device=dev)
+    sorted_ = torch.empty(T * top, dtype=torch.int32, device=dev)
+    plan = torch.empty(1 + 3 * _lib.load().sa_expert_tiles_max(T * top, E, 16), dtype=torch.int32, device=dev)
+    _lib.call("sa_route_few", _ptr(x), x.stride(0), _ptr(router.data), T, D, router.rows, E, int(top), float(scale), int(options is None),
+              _ptr(bias), _code(bias) if bias is not None else 0, _ptr(correction), _code(correction) if correction is not None else 0,
+              int(o.get("groups", 1)), int(o.get("keep", 1)), 2 if softmax == "chosen" else int(softmax), int(o.get("group_best", 2)),
+              -1.0 if renorm is None else float(renorm), _ptr(logits), _ptr(experts), _ptr(weights), _ptr(sorted_), _ptr(plan),
+              plan.numel(), _stream())
+    return logits, experts, weights, (sorted_, plan)
+
+
+def few_rows_experts(T: int, top: int, gate_w, up_w, x: torch.Tensor) -> bool:
+    """Whether a step of T tokens goes through the experts in tiles of 16 rows."""
+    return _lib.load().sa_expert_tile_rows(T * top, up_w.experts, up_w.cols, up_w.rows, _code(x), x.stride(0), _ptr(x)) == 16
+
+
 def routed_experts(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, gate_w, up_w, down_w, activation: int,
                    *, shared: torch.Tensor | None = None, shared_gate: torch.Tensor | None = None,
-                   out_dtype: torch.dtype | None = None, limit: float | None = None) -> torch.Tensor:
+                   out_dtype: torch.dtype | None = None, limit: float | None = None,
+                   defer_sum: bool = False) -> "torch.Tensor | ExpertSums":
     """sum_k weights[t, k] * down[e](act(gate[e] x) * (up[e] x)) with e = experts[t, k], plus sigmoid(shared_gate[t]) *
     shared[t] (shared None: nothing; shared_gate None: shared as it is).  gate_w, up_w, down_w: `packing.ExpertStack`s
     (every expert's matrix, tiled if bfloat16).  x [T, D] in the weights' type; shared_gate float32 [T, 1].
-    gate_w None: experts without a gate, down[e](act(up[e] x)).  limit: of the clamped gated rule (ACT_CLAMPED_GLU)."""
+    gate_w None: experts without a gate, down[e](act(up[e] x)).  limit: of the clamped gated rule (ACT_CLAMPED_GLU).
+    defer_sum: leave the sum over k to the caller."""
+    sums = expert_sums(x, experts, weights, gate_w, up_w, down_w, activation, shared=shared, shared_gate=shared_gate,
+                       out_dtype=out_dtype, limit=limit)
+    return sums if defer_sum else sums.materialize()
+
+
+def expert_sums(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, gate_w, up_w, down_w, activation: int, *,
+                shared: torch.Tensor | None = None, shared_gate: torch.Tensor | None = None, out_dtype: torch.dtype | None = None,
+                limit: float | None = None, order: tuple | None = None, dense: tuple | None = None) -> ExpertSums:
+    """`routed_experts` with the sum over k left to the caller.
+    order: (sorted, plan) as `route_few` gives them (at most 16 tokens).  dense, with order: (first, down, limit), the tiled weights
+    of a shared feed-forward of the experts' form (first: paired if they are gated), which runs in the experts' kernels; its rows
+    take `shared`'s place, in 32 bits."""
     _dev(x, experts, weights, gate_w.data if gate_w is not None else None, up_w.data, down_w.data, shared, shared_gate)
     T, D = x.shape
     top, E, F = experts.shape[1], up_w.experts, up_w.rows
@@ -2006,26 +2105,46 @@ def routed_experts(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor
     limit = _gate_limit(activation, limit)
     P = T * top
     dev = x.device
-    # tiles of 64 or 128 rows share the weights' operands between their rows: for steps that bring an expert many
-    tile_rows = _lib.load().sa_expert_tile_rows(P, E, D, F, _code(x), _rows(x, "routed_experts: x"), _ptr(x))
-    max_tiles = _lib.load().sa_expert_tiles_max(P, E, tile_rows)
-    sorted_ = torch.empty(P, dtype=torch.int32, device=dev)
-    plan = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=dev)
-    _lib.call("sa_expert_sort", _ptr(experts), P, E, tile_rows, _ptr(sorted_), _ptr(plan), plan.numel(), _stream())
+    xs = _rows(x, "routed_experts: x")
+    if order is not None:
+        sorted_, plan = order
+        tile_rows = 16
+        if x.dtype != torch.bfloat16 or T > 16 or sorted_.numel() != P or sorted_.dtype != torch.int32 or plan.dtype != torch.int32 \
+                or plan.numel() < 1 + 3 * _lib.load().sa_expert_tiles_max(P, E, 16):
+            raise KernelError("routed_experts: the order does not belong to these tokens")
+    else:
+        # tiles of 64 or 128 rows share the weights' operands between their rows: for steps that bring an expert many
+        tile_rows = _lib.load().sa_expert_tile_rows(P, E, D, F, _code(x), xs, _ptr(x))
+        max_tiles = _lib.load().sa_expert_tiles_max(P, E, tile_rows)
+        sorted_ = torch.empty(P, dtype=torch.int32, device=dev)
+        plan = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=dev)
+        _lib.call("sa_expert_sort", _ptr(experts), P, E, tile_rows, _ptr(sorted_), _ptr(plan), plan.numel(), _stream())
     h = torch.empty((P, F), dtype=x.dtype, device=dev)
     first, second = (gate_w.data, up_w.data) if gate_w is not None else (up_w.data, None)
-    _lib.call("sa_expert_product", _ptr(x), _code(x), _rows(x, "routed_experts: x"), 1, top, _ptr(first),
-              _ptr(second), F, D, _ptr(sorted_), _ptr(plan), P, E, tile_rows, int(activation), limit, _ptr(h), F, 0,
-              int(gate_w is None), _stream())
     y = torch.empty((P, D), dtype=torch.float32, device=dev)
-    _lib.call("sa_expert_product", _ptr(h), _code(h), F, 0, top, _ptr(down_w.data), None, D, F, _ptr(sorted_), _ptr(plan), P,
-              E, tile_rows, 0, 0.0, _ptr(y), D, 1, 0, _stream())
-    out = torch.empty((T, D), dtype=out_dtype or x.dtype, device=dev)
+    if dense is not None:
+        d_first, d_down, d_limit = dense
+        S = d_first.rows
+        if order is None or shared is not None or d_first.paired != (gate_w is not None) or d_first.cols != D or d_down.paired \
+                or tuple(d_down.shape) != (D, S):
+            raise KernelError("routed_experts: the shared feed-forward's weights do not go with the experts'")
+        d_limit = _gate_limit(activation, d_limit)
+        _dev(x, d_first.data, d_down.data)
+        hs = torch.empty((T, S), dtype=x.dtype, device=dev)
+        shared = torch.empty((T, D), dtype=torch.float32, device=dev)
+        _lib.call("sa_expert_product_shared", _ptr(x), xs, 1, top, _ptr(first), _ptr(second), F, D, _ptr(sorted_), _ptr(plan), P, E,
+                  int(activation), limit, _ptr(h), F, 0, int(gate_w is None), _ptr(x), xs, _ptr(d_first.data), S, D, T, d_limit, _ptr(hs),
+                  S, _stream())
+        _lib.call("sa_expert_product_shared", _ptr(h), F, 0, top, _ptr(down_w.data), None, D, F, _ptr(sorted_), _ptr(plan), P, E, 0, 0.0,
+                  _ptr(y), D, 1, 0, _ptr(hs), S, _ptr(d_down.data), D, S, T, 0.0, _ptr(shared), D, _stream())
+    else:
+        _lib.call("sa_expert_product", _ptr(x), _code(x), xs, 1, top, _ptr(first),
+                  _ptr(second), F, D, _ptr(sorted_), _ptr(plan), P, E, tile_rows, int(activation), limit, _ptr(h), F, 0,
+                  int(gate_w is None), _stream())
+        _lib.call("sa_expert_product", _ptr(h), _code(h), F, 0, top, _ptr(down_w.data), None, D, F, _ptr(sorted_), _ptr(plan), P,
+                  E, tile_rows, 0, 0.0, _ptr(y), D, 1, 0, _stream())
     if shared is not None and tuple(shared.shape) != (T, D):
         raise KernelError("routed_experts: the shared expert's rows do not match")
     if shared_gate is not None and (shared_gate.dtype != torch.float32 or shared_gate.shape[0] != T):
         raise KernelError("routed_experts: the shared expert's gate is float32 [T, 1]")
-    _lib.call("sa_expert_combine", _ptr(y), _ptr(weights), top, _ptr(shared), _code(shared) if shared is not None else 0,
-              _rows(shared, "routed_experts: shared") if shared is not None else 0, _ptr(shared_gate),
-              shared_gate.stride(0) if shared_gate is not None else 0, _ptr(out), _code(out), D, T, D, _stream())
-    return out
+    return ExpertSums(y, weights, shared, shared_gate, out_dtype or x.dtype)

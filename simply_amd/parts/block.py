@@ -159,5 +159,7 @@ class PreNormBlock(Block):
         if self.feed_forward is None:
             return h, self._add(h, y, next_norm, ctx.dtype)
         normed = self._add(h, y, n["pre_ffn"], ctx.dtype)
-        y = self.feed_forward.forward(normed, ctx)
+        # (experts' results may be left to the sum in front of the next norm, where both can)
+        both = getattr(self.feed_forward, "defers_experts", False) and next_norm is not None and next_norm.fuses_sum
+        y = self.feed_forward.forward(normed, ctx, **({"defer_experts": True} if both else {}))
         return h, self._add(h, y, next_norm, ctx.dtype)

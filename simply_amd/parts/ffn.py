@@ -112,6 +112,9 @@ class RoutedExperts(FeedForward):
       shared_size one more feed-forward of the experts' form runs for every token and is added, times sigmoid(w . x)
                   (one number per token) if `shared_gate`."""
 
+    #: forward() takes defer_experts=True and may then return an `ops.ExpertSums`
+    defers_experts = True
+
     def __init__(self, hidden_size: int, num_experts: int, top: int, expert_size: int, router_scale: float = 1.0,
                  activation: str = "silu", shared_size: int | None = None, shared_gate: bool = True, gated: bool = True,
                  router: str = "softmax", correction: bool = False, num_groups: int = 1, keep_groups: int = 1,
@@ -178,19 +181,30 @@ class RoutedExperts(FeedForward):
         if self.shared is not None:
             self.shared.load({n: tensors["shared." + n] for n in self.shared.param_specs()})
 
-    def forward(self, x: torch.Tensor, ctx=None) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, ctx=None, defer_experts=False) -> "torch.Tensor | ops.ExpertSums":
         E = self.num_experts
-        logits = ops.gemm(x, self.router, out_dtype=torch.float32)
         plain = self.router_kind == "softmax" and not self.correction and self.num_groups == 1 and self.renormalize is None \
             and not self.router_bias
-        if not plain:
-            experts, weights = ops.route_choice(logits[:, :E], self.top, self.router_scale, correction=self.correction_w,
-                                                groups=self.num_groups, keep=self.keep_groups,
-                                                softmax={"softmax": True, "sigmoid": False}.get(self.router_kind, "chosen"),
-                                                group_best=self.group_best, renorm=self.renormalize,
-                                                bias=self.router_bias_w)
+        options = None if plain else dict(correction=self.correction_w, groups=self.num_groups, keep=self.keep_groups,
+                                          softmax={"softmax": True, "sigmoid": False}.get(self.router_kind, "chosen"),
+                                          group_best=self.group_best, renorm=self.renormalize, bias=self.router_bias_w)
+        order = dense = shared = None
+        # a handful of tokens: the router in one kernel, the shared feed-forward beside the experts
+        if ops.route_few_takes(x, self.router, E, self.top) and ops.few_rows_experts(x.shape[0], self.top, self.gate_w, self.up_w, x):
+            logits, experts, weights, order = ops.route_few(x, self.router, E, self.top, self.router_scale, options=options)
+            if self.shared is not None:
+                dense = (self.shared.gate_up, self.shared.down_proj, self.shared.limit) if self.gated \
+                    else (self.shared.up_proj, self.shared.down_proj, None)
         else:
-            experts, weights = ops.route(logits[:, :E], self.top, self.router_scale)
-        shared = self.shared.forward(x, ctx) if self.shared is not None else None
-        return ops.routed_experts(x, experts, weights, self.gate_w, self.up_w, self.down_w, self.activation_code,
-                                  shared=shared, shared_gate=logits[:, E:E + 1] if self.shared_gate else None, limit=self.limit)
+            logits = ops.gemm(x, self.router, out_dtype=torch.float32)
+            if plain:
+                experts, weights = ops.route(logits[:, :E], self.top, self.router_scale)
+            else:
+                experts, weights = ops.route_choice(logits[:, :E], self.top, self.router_scale, **options)
+            shared = self.shared.forward(x, ctx) if self.shared is not None else None
+        args = (x, experts, weights, self.gate_w, self.up_w, self.down_w, self.activation_code)
+        kw = dict(shared=shared, shared_gate=logits[:, E:E + 1] if self.shared_gate else None, limit=self.limit)
+        if order is None:
+            return ops.routed_experts(*args, **kw, **({"defer_sum": True} if defer_experts and x.is_cuda else {}))
+        sums = ops.expert_sums(*args, **kw, order=order, dense=dense)
+        return sums if defer_experts else sums.materialize()

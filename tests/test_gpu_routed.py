@@ -69,3 +69,58 @@ def test_more_tiles_than_a_grid_s_second_index(dtype, tile_rows):
     a = a.float()
     want = torch.where(experts[:, None] == 0, a @ w[0].float().T, a @ w[1].float().T)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("T,E,top,D,F,S,gated,options", [
+    (1, 1, 1, 32, 16, 16, True, None), (16, 128, 8, 960, 64, 96, True, None), (8, 16, 2, 2048, 128, 128, True, dict(groups=4, keep=2, softmax=True, group_best=1, renorm=1e-20)),
+    (5, 17, 3, 96, 40, 24, False, dict(softmax=False, correction=True, bias=True)), (16, 9, 3, 160, 48, 320, True, dict(softmax="chosen")),
+    (3, 128, 40, 64, 32, 8, False, dict(groups=16, keep=7))])
+def test_few_tokens(T, E, top, D, F, S, gated, options):
+    """The router in one launch and the shared feed-forward beside the experts, against the separate kernels on the same logits: the
+    same experts, weights and order of experts.  The sum over experts with the norm behind it: what the experts and the shared
+    feed-forward give differs by the roundings of a bfloat16 run alone (2^-8 of the shared rows, which the separate kernels round)."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_gate_up, pack_tiles, stack_experts
+
+    x = draw((T, D + 8), 1).bfloat16().cuda()[:, :D]
+    router = pack_tiles(draw((E + 1, D), 2, 3 * D ** -0.5).bfloat16().cuda())
+    o = None if options is None else dict(options)
+    for name in ("correction", "bias"):
+        if o and o.get(name):
+            o[name] = draw((E,), 3).cuda()
+    assert ops.route_few_takes(x, router, E, top)
+    logits, experts, weights, order = ops.route_few(x, router, E, top, 1.5, options=o)
+    # (sums of D products in another order: 2^-24 of their sizes for each of at most D steps)
+    want = ops.gemm(x, router, out_dtype=torch.float32)
+    assert torch.allclose(logits, want, rtol=0, atol=D * 2.0 ** -24 * 3 * D ** 0.5)
+    e, w = ops.route(logits[:, :E], top, 1.5) if o is None else ops.route_choice(logits[:, :E], top, 1.5, **o)
+    assert torch.equal(experts, e) and torch.equal(weights, w)
+    flat, (pairs, plan) = experts.flatten().cpu(), (order[0].cpu().long(), order[1].cpu())
+    assert sorted(pairs.tolist()) == list(range(T * top)) and bool((flat[pairs].diff() >= 0).all())
+    tiles, at = [], 0
+    for n in range(E):
+        rows = int((flat == n).sum())
+        for i in range(0, rows, 16):
+            tiles += [n, at + i, min(16, rows - i)]
+        at += rows
+    assert plan[0] == len(tiles) // 3 and plan[1:1 + len(tiles)].tolist() == tiles
+
+    ws = [[draw((r, c), 10 + 100 * i + n, c ** -0.5).bfloat16().cuda() for n in range(E)] for i, (r, c) in
+          enumerate(((F, D), (F, D), (D, F)))]
+    gate, up, down = (stack_experts(v) for v in ws)
+    sg, su, sd = draw((S, D), 5, D ** -0.5).bfloat16().cuda(), draw((S, D), 6, D ** -0.5).bfloat16().cuda(), draw((D, S), 7, S ** -0.5).bfloat16().cuda()
+    first = pack_gate_up(sg, su) if gated else pack_tiles(su)
+    args = (x, experts, weights, gate if gated else None, up, down, ops.ACT_SILU)
+    hidden = ops.gemm(x, first, activation=ops.ACT_SILU) if gated else ops.gemm(x, first, activate=ops.ACT_SILU)
+    shared = ops.gemm(hidden, pack_tiles(sd), out_dtype=torch.float32)
+    kw = dict(shared_gate=logits[:, E:], out_dtype=torch.float32)
+    got = ops.expert_sums(*args, order=order, dense=(first, pack_tiles(sd), None), **kw).materialize()
+    want = ops.routed_experts(*args, shared=shared, **kw)
+    # (hidden entries of the shared feed-forward may round the other way where their sums are taken in another order)
+    assert torch.allclose(got, want, rtol=0, atol=2.0 ** -8 * float(shared.abs().max()))
+    h = draw((T, D), 8).cuda()
+    h2, scale = h.clone(), draw((D,), 9).bfloat16().cuda()
+    sums = ops.expert_sums(*args, shared=shared, shared_gate=logits[:, E:])
+    a = ops.residual_add_next_norm(sums, h, scale, eps=1e-5, mult=0.7)
+    b = ops.residual_add_next_norm(want, h2, scale, eps=1e-5, mult=0.7, out_dtype=torch.bfloat16)
+    assert torch.equal(h, h2) and torch.equal(a, b)
