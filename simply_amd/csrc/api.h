@@ -642,6 +642,16 @@ int sa_expert_combine(const float* y, const float* weights, int top, const void*
 int sa_token_shift(const void* h, int dtype, int64_t h_stride, const void* mu, int mu_dtype, int streams, float* tails,
                    int64_t tail_stride, const int* seq_meta, int num_seqs, int max_q_len, void* out, int D,
                    hipStream_t stream);
+// A step's tokens, one after the other for each request, through the matrix-state recurrence with decays per key channel from
+// their low-rank factors (sa_low_rank_decay, w tiled), a bonus (sa_linear_state) and the norm per head and silu gate behind it
+// (sa_gated_heads): proj rows hold q, k, v, the gate (H heads of D each) and the decays' factors at the given columns, bfloat16;
+// state [H][D][D] columns first; out [T, H * D] bfloat16.  _takes: heads of 64 or 128, ranks in multiples of 8 up to 128, aligned rows.
+int sa_wkv_token_takes(int D, int rank, int64_t proj_stride, int q_at, int k_at, int low_at, int64_t state_stride, const void* proj,
+                       const void* state);
+int sa_wkv_token(const void* proj, int64_t proj_stride, int q_at, int k_at, int v_at, int g_at, int low_at, int rank,
+                 const void* decay_w, const void* base, int base_dtype, const void* bonus, int bonus_dtype, const void* norm,
+                 int norm_dtype, float eps, int H, int D, float* state, int64_t state_stride, const int* seq_meta, int num_seqs,
+                 void* out, hipStream_t stream);
 // out[t, c] = exp(-exp(sum_r w[c, r] tanh(p[t, r]) + w0[c])), 32-bit; w [C, rank], row-major or (tiled) in the operand
 // tiles of the product kernels.
 int sa_low_rank_decay(const void* p, int p_dtype, int64_t p_stride, const void* w, int w_dtype, int tiled, const void* w0,

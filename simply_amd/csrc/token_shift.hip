@@ -9,6 +9,7 @@
 // Differences, sums, tanh and exponentials are 32-bit whatever the element types are.
 #include "api.h"
 #include "common.h"
+#include "low_rank.h"
 
 namespace sa {
 
@@ -129,11 +130,7 @@ __global__ __launch_bounds__(kWave) void low_rank_decay_kernel(const void* __res
 }
 
 // bfloat16 weights in MFMA operand tiles ([C / 16][rank / 32][64][8], zeros beyond C and rank): a wave takes 16 tokens and
-// `tiles` tiles of 16 channels.  tanh(p) goes in as three bfloat16 numbers (its rounding, the rounding of what that leaves,
-// and the rest: all 24 bits), so that the sum is that of 32-bit factors; a lane computes the eight entries of every 32
-// that its operand holds.
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+// `tiles` tiles of 16 channels; a lane computes tanh (tanh_in_three) of the eight entries of every 32 that its operand holds.
 constexpr int kDecayChunks = 2;   // chunks of 32 factors whose tanh a wave holds at a time
 template <typename PT, typename BT, bool VEC>
 __global__ __launch_bounds__(256) void low_rank_decay_tiled_kernel(const PT* __restrict__ p, int64_t p_stride,
@@ -159,17 +156,7 @@ __global__ __launch_bounds__(256) void low_rank_decay_tiled_kernel(const PT* __r
 #pragma unroll
         for (int j = 0; j < 8; ++j) xs[j] = k0 + j < rank ? to_float(src[j]) : 0.f;
       }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float x = xs[j];
-        // tanh by the hardware's exponential: 1 - 2 / (e^(2x) + 1), and x (1 - x^2 / 3) where that cancels
-        const float y = 1.f - 2.f * __builtin_amdgcn_rcpf(__expf(2.f * x) + 1.f);
-        const float th = fabsf(x) < 0.02f ? x * fmaf(x * x, -1.f / 3.f, 1.f) : y;
-        hi[u][j] = static_cast<__bf16>(th);
-        const float rest = th - static_cast<float>(hi[u][j]);
-        mid[u][j] = static_cast<__bf16>(rest);
-        lo[u][j] = static_cast<__bf16>(rest - static_cast<float>(mid[u][j]));
-      }
+      tanh_in_three(xs, hi[u], mid[u], lo[u]);
     }
   };
   if (chunks <= kDecayChunks) factors(0);   // (held for all of the wave's channels)
@@ -197,11 +184,7 @@ __global__ __launch_bounds__(256) void low_rank_decay_tiled_kernel(const PT* __r
       for (int u = 0; u < kDecayChunks; ++u) {
         if (c0 + u >= chunks) break;   // (uniform)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i][u], hi[u], acc[i], 0, 0, 0);
-          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i][u], mid[u], acc[i], 0, 0, 0);
-          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i][u], lo[u], acc[i], 0, 0, 0);
-        }
+        for (int i = 0; i < 4; ++i) acc[i] = product_in_three(wv[i][u], hi[u], mid[u], lo[u], acc[i]);
       }
     }
     // lane: token r, channels 4 kq .. of every tile

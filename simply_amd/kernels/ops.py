@@ -1838,6 +1838,35 @@ def low_rank_decay(p: torch.Tensor, w: "torch.Tensor | TiledWeight", base: torch
     return out
 
 
+def wkv_token_takes(proj: torch.Tensor, decay_w, head_dim: int, state: torch.Tensor, low_at: int) -> bool:
+    """Whether `wkv_token` takes these sizes (bfloat16; heads of 64 or 128, ranks in multiples of 8 up to 128)."""
+    return proj.is_cuda and proj.dtype == torch.bfloat16 and isinstance(decay_w, TiledWeight) and proj.stride(1) == 1 and bool(
+        _lib.load().sa_wkv_token_takes(int(head_dim), decay_w.cols, proj.stride(0), 0, 0, int(low_at), state.stride(0), _ptr(proj),
+                                       _ptr(state)))
+
+
+def wkv_token(proj: torch.Tensor, columns: tuple, decay_w: TiledWeight, base: torch.Tensor, bonus: torch.Tensor, norm: torch.Tensor,
+              eps: float, num_heads: int, head_dim: int, state: torch.Tensor, seq_meta: torch.Tensor, num_seqs: int) -> torch.Tensor:
+    """`low_rank_decay`, `linear_state` with a bonus and `gated_heads` (norm per head with a weight per entry, silu) in one kernel,
+    for steps that bring a request a token: proj's columns (q, k, v, gate, decay factors), bfloat16 [T, H * d] out."""
+    _dev(proj, decay_w.data, base, bonus, norm, state, seq_meta)
+    T, H, d = proj.shape[0], int(num_heads), int(head_dim)
+    q_at, k_at, v_at, g_at, low_at = (int(c) for c in columns)
+    stride = _rows(proj, "wkv_token: proj")
+    if decay_w.rows != H * d or any(t.numel() != H * d or not t.is_contiguous() for t in (base, bonus, norm)):
+        raise KernelError("wkv_token: decays, bonus and norm have an entry per head and channel")
+    if proj.dtype != torch.bfloat16 or proj.shape[1] < max(q_at + H * d, k_at + H * d, v_at + H * d, g_at + H * d, low_at + decay_w.cols):
+        raise KernelError("wkv_token: the projection rows are too short")
+    if state.dtype != torch.float32 or state.dim() != 2 or state.stride(1) != 1 or state.shape[1] < H * d * d:
+        raise KernelError("wkv_token: the state must be float32 [slots, >= H * d * d]")
+    _seq_meta(seq_meta, num_seqs, "wkv_token")
+    out = torch.empty((T, H * d), dtype=proj.dtype, device=proj.device)
+    _lib.call("sa_wkv_token", _ptr(proj), stride, q_at, k_at, v_at, g_at, low_at, decay_w.cols, _ptr(decay_w.data), _ptr(base),
+              _code(base), _ptr(bonus), _code(bonus), _ptr(norm), _code(norm), float(eps), H, d, _ptr(state), state.stride(0),
+              _ptr(seq_meta), int(num_seqs), _ptr(out), _stream())
+    return out
+
+
 def concat_rows(x: torch.Tensor, y: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     """[x | y] row by row (contiguous float32) in out_dtype."""
     _dev(x, y)

@@ -63,6 +63,10 @@ class WKV(Mixer):
         if self.decay_in is None:
             proj = ops.gemm_sections(mixes, self.in_proj)                             # [T, r | k | v | gate | decay's factor]
             low = proj[:, 4 * C:]
+            if ctx.max_q_len == 1 and ops.wkv_token_takes(proj, self.decay_out, d, cache.state, 4 * C):
+                z = ops.wkv_token(proj, (0, C, 2 * C, 3 * C, 4 * C), self.decay_out, self.decay_base, self.bonus, self.norm,
+                                  self.norm_eps, H, d, cache.state, ctx.seq_meta, ctx.num_seqs)
+                return ops.gemm(z, self.o_proj)
         else:
             proj, low = ops.gemm_sections(mixes[:, :4 * D], self.in_proj), ops.gemm(mixes[:, 4 * D:], self.decay_in)
         decay = ops.low_rank_decay(low, self.decay_out, self.decay_base)

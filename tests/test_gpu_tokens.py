@@ -1,0 +1,40 @@
+"""Kernels that take a decode step's tokens through several operations at once, against the separate kernels."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def draw(shape, seed, std=1.0):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * std
+
+
+@pytest.mark.parametrize("counts,H,d,rank,vectors", [([1], 1, 64, 8, torch.float32), ([1] * 8, 16, 128, 64, torch.bfloat16),
+                                                     ([2, 0, 1, 5], 3, 64, 128, torch.bfloat16), ([1, 1, 3], 2, 128, 40, torch.float32)])
+def test_wkv_token(counts, H, d, rank, vectors):
+    """The same decays (the same products); states and sums over keys differ by the order of sums alone.  A head's o is a sum of d
+    products, off by d roundings of 2^-24 of their sizes at most; the norm and the gate hand that on, rounded to bfloat16."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+
+    C, T, S = H * d, sum(counts), len(counts)
+    proj = draw((T, 4 * C + rank + 8), 1).bfloat16().cuda()[:, :4 * C + rank]
+    w = pack_tiles(draw((C, rank), 2, rank ** -0.5).bfloat16().cuda())
+    base, bonus, norm = (draw((C,), 3 + i, 0.5).to(vectors).cuda() for i in range(3))
+    state = draw((S + 2, C * d + 12), 6).cuda()
+    first, meta = 0, []
+    for i, n in enumerate(counts):
+        meta.append([S + 1 - i, first, n, 7])
+        first += n
+    meta = torch.tensor(meta, dtype=torch.int32).cuda()
+    columns = (0, C, 2 * C, 3 * C, 4 * C)
+    assert ops.wkv_token_takes(proj, w, d, state, 4 * C)
+    mine, theirs = state.clone(), state.clone()
+    got = ops.wkv_token(proj, columns, w, base, bonus, norm, 1e-5, H, d, mine, meta, S)
+    decay = ops.low_rank_decay(proj[:, 4 * C:], w, base)
+    o = ops.linear_state(proj, 0, C, 2 * C, 1.0, decay, False, H, d, d, False, theirs, meta, S, bonus=bonus)
+    want = ops.gated_heads(o, proj[:, 3 * C:4 * C], H, d, kind=ops.GATE_SILU, weight=norm, eps=1e-5, out_dtype=torch.float32)
+    assert torch.allclose(mine, theirs, rtol=2.0 ** -22, atol=2.0 ** -22 * 5)   # (a product and a sum a token)
+    assert torch.equal(mine[:, C * d:], state[:, C * d:]) and torch.equal(mine[0], state[0])
+    # bfloat16: half a step of 2^-8; the sums' roundings lie far below
+    assert ((got.float() - want).abs() <= 2.0 ** -8 * want.abs() + d * 2.0 ** -22).all()
