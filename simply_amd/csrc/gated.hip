@@ -8,6 +8,7 @@
 // correctly rounded ones (no reciprocal-square-root instruction).
 #include "api.h"
 #include "common.h"
+#include "eights.h"
 
 namespace sa {
 
@@ -17,37 +18,6 @@ namespace sa {
 // together.  Layer norm of eight rows of 2,048 with the sum: 10.3 us with an entry at a time behind a test of the row's end, 4.6
 // in pieces (launch and two waits for memory); of 2,047 rows 16.5 and 11.2 us (50 MB: 4.5 TB/s), the sum of normed rows 13.0 and
 // 10.8.
-struct Eight {
-  float v[8];
-};
-__device__ __forceinline__ Eight load_eight(const float* p) {
-  Eight e;
-  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
-  e.v[0] = a.x, e.v[1] = a.y, e.v[2] = a.z, e.v[3] = a.w, e.v[4] = b.x, e.v[5] = b.y, e.v[6] = b.z, e.v[7] = b.w;
-  return e;
-}
-__device__ __forceinline__ Eight load_eight(const bf16* p) {
-  Eight e;
-  const uint4 a = *reinterpret_cast<const uint4*>(p);
-  const uint32_t u[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    e.v[2 * i] = __uint_as_float(u[i] << 16);
-    e.v[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
-  }
-  return e;
-}
-__device__ __forceinline__ void store_eight(float* p, const Eight& e) {
-  reinterpret_cast<float4*>(p)[0] = float4{e.v[0], e.v[1], e.v[2], e.v[3]};
-  reinterpret_cast<float4*>(p)[1] = float4{e.v[4], e.v[5], e.v[6], e.v[7]};
-}
-__device__ __forceinline__ void store_eight(bf16* p, const Eight& e) {
-  uint32_t u[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    u[i] = static_cast<uint32_t>(float_to_bf16(e.v[2 * i]).bits) | (static_cast<uint32_t>(float_to_bf16(e.v[2 * i + 1]).bits) << 16);
-  *reinterpret_cast<uint4*>(p) = uint4{u[0], u[1], u[2], u[3]};
-}
 static bool rows_in_eights(int D, int64_t y_stride, const void* a, const void* b, const void* c, const void* d, const void* e) {
   return D % 8 == 0 && y_stride % 8 == 0 &&
          ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(d) |

@@ -1252,6 +1252,38 @@ def norm_rope_cache_write(proj: torch.Tensor, positions: torch.Tensor, freq: tor
     return proj
 
 
+def latent_rows_takes(q: torch.Tensor, rows: torch.Tensor, weight: torch.Tensor, num_heads: int, latent: int, rot_dims: int,
+                      k_pages: torch.Tensor) -> bool:
+    """Whether `latent_rows` takes these sizes (bfloat16, everything in whole aligned pieces of 8 entries)."""
+    return q.is_cuda and q.dtype == torch.bfloat16 and q.stride(1) == 1 and rows.stride(1) == 1 and bool(
+        _lib.load().sa_latent_rows_takes(int(num_heads), int(latent), rows.shape[1] - int(latent), int(rot_dims), k_pages.shape[2],
+                                         q.stride(0), rows.stride(0), _ptr(q), _ptr(rows), _ptr(weight)))
+
+
+def latent_rows(q: torch.Tensor, rows: torch.Tensor, positions: torch.Tensor, freq: torch.Tensor, rot_dims: int, num_heads: int,
+                latent: int, weight: torch.Tensor, eps: float, slot_mapping: torch.Tensor, k_pages: torch.Tensor,
+                v_pages: torch.Tensor, *, rot_mult: float = 1.0) -> None:
+    """The two `norm_rope_cache_write` of latent attention in one launch: q [T, H * (latent + d)] in place, its heads' entries
+    [latent, latent + rot_dims) turned; rows [T, latent + d] into pages, the latent normed with `weight`, what follows turned."""
+    _dev(q, rows, positions, freq, weight, slot_mapping, k_pages, v_pages)
+    T, H, R = q.shape[0], int(num_heads), int(latent)
+    unit = rows.shape[1]
+    if rows.shape[0] != T or rows.dtype != q.dtype or q.shape[1] < H * unit or weight.numel() != R or not weight.is_contiguous():
+        raise KernelError("latent_rows: queries, rows and weight do not go together")
+    _i32(positions, "latent_rows: positions", T)
+    if freq.dtype != torch.float32 or freq.numel() != rot_dims // 2 or not freq.is_contiguous():
+        raise KernelError("latent_rows: freq must be float32 [rot_dims / 2]")
+    P = k_pages.shape[2]
+    if any(p.dtype != q.dtype or not p.is_contiguous() for p in (k_pages, v_pages)) \
+            or tuple(k_pages.shape[1:]) != (1, P, unit) or tuple(v_pages.shape) != (k_pages.shape[0], 1, R, P):
+        raise KernelError(f"latent_rows: key pages {tuple(k_pages.shape)} and value pages {tuple(v_pages.shape)} do not match")
+    if slot_mapping.dtype != torch.int64 or slot_mapping.numel() < T or not slot_mapping.is_contiguous():
+        raise KernelError("latent_rows: slot_mapping must be int64 [T]")
+    _lib.call("sa_latent_rows", _ptr(q), _rows(q, "latent_rows: q"), _ptr(rows), _rows(rows, "latent_rows: rows"), _ptr(positions),
+              _ptr(freq), int(rot_dims), float(rot_mult), _ptr(weight), _code(weight), float(eps), _ptr(slot_mapping), _ptr(k_pages),
+              _ptr(v_pages), T, H, R, unit - R, P, _stream())
+
+
 def short_conv(x: torch.Tensor, taps: torch.Tensor, tails: torch.Tensor, seq_meta: torch.Tensor, num_seqs: int,
                max_q_len: int, *, in_bias: torch.Tensor | None = None, out_bias: torch.Tensor | None = None,
                silu: bool = False, update_tails: bool = True) -> torch.Tensor:

@@ -102,6 +102,13 @@ class LatentAttention(Mixer):
     def cache_need(self):
         return PagedKVNeed(1, self.kv_rank + self.rot_dim, self.window, self.kv_rank)
 
+    def _write_rows(self, rows, ctx, group, cache, freq, rot_dims, mult):
+        """The tokens' rows [norm(c) | rotated r] into the pages."""
+        R, unit = self.kv_rank, self.kv_rank + self.rot_dim
+        ops.norm_rope_cache_write(rows, ctx.positions, freq, rot_dims, 0, 1, unit, 0, rot_mult=mult, eps=self.norm_eps,
+                                  k_weight=self.dkv_norm, k_norm_dims=R, k_rot_at=R, slot_mapping=group.slot_mapping,
+                                  k_pages=cache.k_pages, v_pages=cache.v_pages, key_values=R)
+
     def forward(self, x, ctx, cache, defer_sum=False):
         H, dk, dr, dv, Rq, R = self.num_heads, self.key_dim, self.rot_dim, self.value_dim, self.q_rank, self.kv_rank
         group = ctx.groups[cache.group_id]
@@ -116,13 +123,14 @@ class LatentAttention(Mixer):
             c_at = H * (dk + dr)
             q = proj[:, :c_at]
         qa = ops.head_product(q, self.uk_t, in_stride=dk + dr, tail=dr)      # [T, H * (R + dr)]: [W_uk^T q | s]
-        ops.norm_rope_cache_write(qa, ctx.positions, freq, rot_dims, H, 0, R + dr, 0, rot_mult=mult, q_rot_at=R)
-        if cache.write:
-            # the token's row [norm(c) | rotated r] into the pages
-            ops.norm_rope_cache_write(proj[:, c_at:c_at + R + dr], ctx.positions, freq, rot_dims, 0, 1, R + dr, 0,
-                                      rot_mult=mult, eps=self.norm_eps, k_weight=self.dkv_norm, k_norm_dims=R,
-                                      k_rot_at=R, slot_mapping=group.slot_mapping, k_pages=cache.k_pages,
-                                      v_pages=cache.v_pages, key_values=R)
+        rows = proj[:, c_at:c_at + R + dr]
+        if cache.write and rot_dims and ops.latent_rows_takes(qa, rows, self.dkv_norm, H, R, rot_dims, cache.k_pages):
+            ops.latent_rows(qa, rows, ctx.positions, freq, rot_dims, H, R, self.dkv_norm, self.norm_eps, group.slot_mapping,
+                            cache.k_pages, cache.v_pages, rot_mult=mult)
+        else:
+            ops.norm_rope_cache_write(qa, ctx.positions, freq, rot_dims, H, 0, R + dr, 0, rot_mult=mult, q_rot_at=R)
+            if cache.write:
+                self._write_rows(rows, ctx, group, cache, freq, rot_dims, mult)
         if ops.attention_maps_units_takes(qa, cache.k_pages, cache.v_pages, H):
             # bfloat16 at sizes that the matrix cores take: units of 16 rows (heads times tokens), keys cut into ranges;
             # a prompt's units come in groups that share the keys

@@ -38,3 +38,34 @@ def test_wkv_token(counts, H, d, rank, vectors):
     assert torch.equal(mine[:, C * d:], state[:, C * d:]) and torch.equal(mine[0], state[0])
     # bfloat16: half a step of 2^-8; the sums' roundings lie far below
     assert ((got.float() - want).abs() <= 2.0 ** -8 * want.abs() + d * 2.0 ** -22).all()
+
+
+@pytest.mark.parametrize("slots,H,R,dr,rot,P,weights", [
+    (list(range(32, 64)), 16, 512, 64, 64, 16, torch.bfloat16), ([5, -1, 7, 40], 3, 64, 32, 32, 16, torch.float32),
+    (list(range(3, 40)), 2, 96, 16, 8, 4, torch.bfloat16), (list(range(64, 96)) + list(range(7, 12)), 5, 1000, 24, 16, 32, torch.float32),
+    ([17], 1, 8, 8, 8, 16, torch.bfloat16)])
+def test_latent_rows(slots, H, R, dr, rot, P, weights):
+    """Queries to the bit (the same products of the same angles); rows to a bfloat16 step: the sum of squares is taken in another
+    order, which can round an entry the other way."""
+    from simply_amd.kernels import ops
+
+    T, unit = len(slots), R + dr
+    q = draw((T, H * unit), 1).bfloat16().cuda()
+    proj = draw((T, unit + 24), 2).bfloat16().cuda()
+    rows, weight = proj[:, 8:8 + unit], draw((R,), 3).to(weights).cuda()
+    positions = torch.arange(T, dtype=torch.int32).cuda() * 37
+    freq = torch.rand(rot // 2, generator=torch.Generator().manual_seed(4)).cuda()
+    slot = torch.tensor(slots, dtype=torch.int64).cuda()
+    pages = 128 // P + 1
+    mine = [torch.full((pages, 1, P, unit), 7.0).bfloat16().cuda(), torch.full((pages, 1, R, P), 7.0).bfloat16().cuda()]
+    theirs = [p.clone() for p in mine]
+    assert ops.latent_rows_takes(q, rows, weight, H, R, rot, mine[0])
+    want = q.clone()
+    ops.latent_rows(q, rows, positions, freq, rot, H, R, weight, 1e-5, slot, *mine, rot_mult=0.9)
+    ops.norm_rope_cache_write(want, positions, freq, rot, H, 0, unit, 0, rot_mult=0.9, q_rot_at=R)
+    ops.norm_rope_cache_write(rows, positions, freq, rot, 0, 1, unit, 0, rot_mult=0.9, eps=1e-5, k_weight=weight, k_norm_dims=R, k_rot_at=R,
+                              slot_mapping=slot, k_pages=theirs[0], v_pages=theirs[1], key_values=R)
+    assert torch.equal(q, want)
+    for a, b in zip(mine, theirs):
+        a, b = a.float(), b.float()
+        assert ((a - b).abs() <= 2.0 ** -7 * b.abs()).all() and float((a != b).float().mean()) < 0.01
