@@ -11,18 +11,18 @@
 //               whole 128-byte pieces of rows, four stages of 32 columns of K ahead in registers; the operand order is made
 //               on the way through LDS (each wave its own part, no barrier in the loop; 16-byte pieces permuted by row, so
 //               that neither side has bank conflicts).
-//   tiles       a workgroup of four waves owns 128 x 128 or 64 x 64 outputs and walks through all segments, adding a
-//               segment's sum to its total at the segment's end: bound by the f32 matrix rate.
+//   tiles       a workgroup of four waves owns 128 x 128, 128 x 96, 128 x 64 or 64 x 64 outputs and walks through all segments,
+//               adding a segment's sum to its total at the segment's end: bound by the f32 matrix rate.
 //   cut tiles   the same tiles, a workgroup per segment (gridDim.z); a sum kernel adds the segments' planes: where the
 //               tiles alone leave CUs idle.
 //
 // Measured, weights from HBM, against the vector-ALU kernel that took these products before (64 x 64 tiles and a thread's
 // 4 x 4 outputs whatever M, so that few rows read W with the workgroups of one row of tiles, one 16-column stage at a time):
 //   (N, K)                4 rows             509 rows
-//   (2304, 9216)          23 us for 959      215 us for 1,450 (100 TFLOP/s of 157)
-//   (2304, 2048)          7.1 for 213        63 for 315
-//   (4096, 2304)          10 for 243         101 for 383
-//   (9216 gated, 2304)    45 for 458         395 for 1,026
+//   (2304, 9216)          23 us for 959      207 us for 1,450; 250 with operands through registers
+//   (2304, 2048)          7.1 for 213        57 for 315; 66
+//   (4096, 2304)          10 for 243         91 for 383; 106
+//   (9216 gated, 2304)    45 for 458         382 for 1,026 (113 TFLOP/s of 157); 470
 //   (256000, 2304)        408 for 1,556 (5.8 TB/s)
 #include "api.h"
 #include "common.h"
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64 * kSegments) void gemm_f32_few_kernel(Args a) {
   if (n0 + 4 * g < a.N) store4(a, c, n0 + 4 * g, y);
 }
 
-// TM: blocks of 16 rows and of 16 weight rows of a wave; four waves, two by two.  With the gated epilogue half of a wave's
+// K that is no multiple of 16 (or rows longer than 16 MB).  TM: blocks of 16 rows and of 16 weight rows of a wave; four waves, two by two.  With the gated epilogue half of a wave's
 // weight rows are the gate's and half the other factor's of the same outputs.  PLANES: this workgroup's segment alone, its
 // sums to planes [segment][M][columns] (gated: all the gate's columns, then the other factor's).
 template <int EPI, int TM, bool PLANES>
@@ -302,6 +302,187 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(Args a, float* __
   }
 }
 
+// A load of 16 bytes a lane from global memory, `offset` bytes behind a base that all lanes share, straight into LDS: lane l's arrive
+// at byte `lds` + 16 l.  The compiler does not know of it: arrived_barrier waits.
+__device__ __forceinline__ void load_to_lds(const float* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const float* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) float*)p));
+}
+// Every wave's loads into LDS have arrived but for its latest PENDING, and its reads of LDS are done.
+template <int PENDING>
+__device__ __forceinline__ void arrived_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(PENDING) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The same for K in multiples of 16, where nothing has to become zero on its way: loads go from global memory straight into LDS,
+// and a wave's matrix instructions never wait for its operands.  TM x TN: blocks of 16 of a wave; WM x (4 / WM) waves.
+// The fragments of a stage's two blocks of 16 columns have registers of their own; the products of the second block are held back
+// behind the next barrier, where they cover the fragment reads of the next stage's first block, and the reads of the second are
+// covered by the products of the first.  Reads and loads go out one by one, each behind some products: a wave issues in order,
+// and more than the 32 cycles of one product between two of them leave the matrix unit idle (4,096 cubed: 117 TFLOP/s through
+// registers, 125 with held-back products, 139.5 with the reads and loads spread; the unit's rate by itself is 155).
+template <int EPI, int TM, int TN, int WM, int STAGES, bool PLANES>
+__global__ __launch_bounds__(256, 2) void gemm_f32_flow_kernel(Args a, float* __restrict__ planes) {
+  constexpr int WAVES = 4, WN = WAVES / WM, AR = WM * TM * 16, WR = WN * TN * 16;   // rows of A and of W of a tile
+  constexpr int LA = AR / 8 / WAVES, LW = WR / 8 / WAVES, LOADS = LA + LW, PRODUCTS = 4 * TM * TN;
+  constexpr int WT = EPI == 1 ? TN / 2 : TN;             // blocks of outputs across of a wave
+  constexpr int STAGE = (AR + WR) * BK;
+  static_assert(EPI != 1 || TN % 2 == 0, "half of a wave's weight rows are the gate's");
+  __shared__ __align__(16) float stages[STAGES * STAGE];
+  const uint32_t lds = lds_address(stages);
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave % WM, wn = wave / WM, c = lane % 16, g = lane / 16;
+  // Which tile: workgroups go to the eight XCDs in turn, each with an L2 of its own; an XCD gets a contiguous share of the tiles, and
+  // neighbours in it are up to eight tiles of rows against the same weights, which it reads from HBM once.
+  int bx = blockIdx.x, by = blockIdx.y;
+  {
+    const int nx = gridDim.x, ny = gridDim.y, total = nx * ny;
+    int l = bx + nx * by;
+    if (total % 8 == 0) l = (l % 8) * (total / 8) + l / 8;
+    const int group = l / (8 * nx) * 8, height = ny - group < 8 ? ny - group : 8;
+    l -= group * nx;
+    by = group + l % height;
+    bx = l / height;
+  }
+  const int m0 = by * AR, n0 = bx * (WN * WT * 16);
+  const int k0 = PLANES ? blockIdx.z * a.seg : 0;
+  const int length = PLANES && k0 + a.seg < a.K ? a.seg : a.K - k0;   // a multiple of 16
+  const int ns = (length + BK - 1) / BK, per_segment = a.seg / 16;
+  // a load brings 8 rows of 128 bytes; lane l's piece arrives at 16 l, so the lane asks for the one that belongs there.  Of its
+  // address the tile's and the stage's part are scalars, `off` is the rest, in bytes.
+  const int r = lane / kPieces, at = ((lane % kPieces) ^ r) * 4;
+  const float* const a_tile = a.A + static_cast<size_t>(m0) * a.lda + k0;
+  const float* const w_tile = a.W + static_cast<size_t>(n0) * a.K + k0;
+  const float* const w2_tile = EPI == 1 ? a.W2 + static_cast<size_t>(n0) * a.K + k0 : w_tile;
+  uint32_t off[LOADS];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const int m = (i * WAVES + wave) * 8 + r, last = a.M - 1 - m0;
+    off[i] = (static_cast<uint32_t>(m < last ? m : last) * static_cast<uint32_t>(a.lda) + at) * 4;
+  }
+  // of a wave's TN * 16 weight rows the first half belongs to the gate (the 8 rows of a load are of one kind)
+  auto of_gate = [&](int i) __attribute__((always_inline)) {
+    return EPI != 1 || (i * WAVES + wave) * 8 % (TN * 16) < WT * 16;
+  };
+#pragma unroll
+  for (int i = 0; i < LW; ++i) {
+    int n = (i * WAVES + wave) * 8 + r;
+    const int last = a.N - 1 - n0;
+    if (EPI == 1) n = n / (TN * 16) * (WT * 16) + n % (TN * 16) % (WT * 16);
+    off[LA + i] = (static_cast<uint32_t>(n < last ? n : last) * static_cast<uint32_t>(a.K) + at) * 4;
+  }
+  // load i of stage s into a buffer (behind the last stage: that one again; columns behind the end: some of its own, not used)
+  auto ask = [&](int i, int s, int buf) __attribute__((always_inline)) {
+    const int k = (s < ns ? s : ns - 1) * BK;
+    const uint32_t back = k + at < length ? 0u : 64u;
+    const int row = i < LA ? i * WAVES * 8 : AR + (i - LA) * WAVES * 8;
+    load_to_lds((i < LA ? a_tile : of_gate(i - LA) ? w_tile : w2_tile) + k, off[i] - back, lds + (buf * STAGE + (row + wave * 8) * BK) * 4);
+  };
+  floatx4 x[2][TM], w[2][TN];
+  auto read = [&](int buf, int b, int i) __attribute__((always_inline)) {
+    const float* stage = stages + buf * STAGE;
+    if (i < TN) w[b][i] = *reinterpret_cast<const floatx4*>(stage + AR * BK + piece_at((wn * TN + i) * 16 + c, b * 4 + g));
+    else x[b][i - TN] = *reinterpret_cast<const floatx4*>(stage + piece_at((wm * TM + i - TN) * 16 + c, b * 4 + g));
+  };
+  floatx4 acc[TM][TN], total[PLANES ? 1 : TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (!PLANES) total[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+  auto end_of_segment = [&]() __attribute__((always_inline)) {
+    if constexpr (!PLANES) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+          total[i][t] += acc[i][t];
+          acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
+  int left = per_segment;
+  // The products of block b; meanwhile (next) block `to` of the stage in buffer `buf` is read, and (load) stage `stage` goes into
+  // buffer `into`.
+  auto multiply = [&](int b, bool next, int to, int buf, bool load, int stage, int into) __attribute__((always_inline)) {
+    constexpr int READ_EVERY = PRODUCTS * 3 / 4 / (TM + TN), LOAD_EVERY = PRODUCTS / LOADS;
+    static_assert(READ_EVERY >= 1 && LOAD_EVERY >= 1, "a product for each read and load");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+          acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[b][t][j], x[b][i][j], acc[i][t], 0, 0, 0);
+          const int q = (j * TM + i) * TN + t + 1;
+          __builtin_amdgcn_sched_barrier(0);
+          if (next && q % READ_EVERY == 0 && q / READ_EVERY <= TM + TN) read(buf, to, q / READ_EVERY - 1);
+          if (load && q % LOAD_EVERY == 0 && q / LOAD_EVERY <= LOADS) ask(q / LOAD_EVERY - 1, stage, into);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    if (!PLANES && --left == 0) {
+      left = per_segment;
+      end_of_segment();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) ask(i, s, s);
+  arrived_barrier<(STAGES - 1) * LOADS>();
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int i = 0; i < TM + TN; ++i) read(0, b, i);
+  multiply(0, false, 0, 0, false, 0, 0);
+  int buf = 1, into = 0;
+  for (int s = 1; s < ns; ++s) {
+    arrived_barrier<(STAGES - 2) * LOADS>();   // everyone's loads of this stage; and everyone has read the stage before
+    multiply(1, true, 0, buf, true, s + STAGES - 1, into);
+    multiply(0, true, 1, buf, false, 0, 0);
+    into = buf;
+    buf = buf + 1 == STAGES ? 0 : buf + 1;
+  }
+  if (length % BK == 0) multiply(1, false, 0, 0, false, 0, 0);   // (uniform)
+  if (!PLANES && left != per_segment) end_of_segment();
+  asm volatile("s_waitcnt vmcnt(0)" : : : "memory");   // the loads asked for behind the last stage
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + (wm * TM + i) * 16 + c;
+    if (m >= a.M) continue;
+    if (PLANES) {
+      const int64_t width = EPI == 1 ? 2 * static_cast<int64_t>(a.N) : a.N;
+      Args b = a;
+      b.C = planes + static_cast<size_t>(blockIdx.z) * a.M * width;
+      b.ldc = width;
+#pragma unroll
+      for (int t = 0; t < TN; ++t) {
+        const int n = n0 + (wn * WT + t % WT) * 16 + 4 * g;
+        Args to = b;
+        if (EPI == 1 && t >= WT) to.C += a.N;
+        if (n < a.N) store4(to, m, n, acc[i][t]);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < WT; ++t) {
+        const int n = n0 + (wn * WT + t) * 16 + 4 * g;
+        floatx4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = finish<EPI>(a, total[PLANES ? 0 : i][t][e], total[PLANES ? 0 : i][EPI == 1 ? t + WT : t][e]);
+        if (n < a.N) store4(a, m, n, y);
+      }
+    }
+  }
+}
+
 // C = epilogue(sum of the segments' planes, in order), V columns a thread.
 template <int EPI, int V>
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(Args a, const float* __restrict__ planes, int nseg) {
@@ -343,17 +524,37 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(Args a, const float* 
   }
 }
 
-template <int EPI>
-static void launch_tiles(const Args& a, int tm, int nseg, float* planes, hipStream_t stream) {
-  const int rows = 32 * tm, cols = EPI == 1 ? rows / 2 : rows;
-  const dim3 grid((a.N + cols - 1) / cols, (a.M + rows - 1) / rows, planes != nullptr ? nseg : 1);
-  if (planes == nullptr) {
-    if (tm == 4) gemm_f32_tile_kernel<EPI, 4, false><<<grid, 256, 0, stream>>>(a, nullptr);
-    else gemm_f32_tile_kernel<EPI, 2, false><<<grid, 256, 0, stream>>>(a, nullptr);
+// Whether the products are gemm_f32_flow_kernel's: whole blocks of 16, and 128 rows' bytes in 32 bits.
+static bool flows(int K, int64_t lda) { return K % 16 == 0 && K < (1 << 22) && lda < (1 << 22); }
+
+struct Plan {
+  int rows, cols;   // a tile's rows of A and of W; rows 16: few rows
+  bool cut;
+};
+
+template <int EPI, bool PLANES>
+static void launch_tile(const Args& a, const Plan& plan, int nseg, float* planes, hipStream_t stream) {
+  const int cols = EPI == 1 ? plan.cols / 2 : plan.cols;
+  const dim3 grid((a.N + cols - 1) / cols, (a.M + plan.rows - 1) / plan.rows, PLANES ? nseg : 1);
+  if (!flows(a.K, a.lda)) {
+    if (plan.rows == 128) gemm_f32_tile_kernel<EPI, 4, PLANES><<<grid, 256, 0, stream>>>(a, planes);
+    else gemm_f32_tile_kernel<EPI, 2, PLANES><<<grid, 256, 0, stream>>>(a, planes);
     return;
   }
-  if (tm == 4) gemm_f32_tile_kernel<EPI, 4, true><<<grid, 256, 0, stream>>>(a, planes);
-  else gemm_f32_tile_kernel<EPI, 2, true><<<grid, 256, 0, stream>>>(a, planes);
+  if (plan.rows == 64) gemm_f32_flow_kernel<EPI, 2, 2, 2, 3, PLANES><<<grid, 256, 0, stream>>>(a, planes);
+  else if (plan.cols == 64) gemm_f32_flow_kernel<EPI, 4, 2, 2, 2, PLANES><<<grid, 256, 0, stream>>>(a, planes);
+  else if (plan.cols == 128) gemm_f32_flow_kernel<EPI, 4, 4, 2, 2, PLANES><<<grid, 256, 0, stream>>>(a, planes);
+  else if constexpr (EPI == 1) gemm_f32_flow_kernel<EPI, 2, 6, 4, 2, PLANES><<<grid, 256, 0, stream>>>(a, planes);
+  else gemm_f32_flow_kernel<EPI, 4, 3, 2, 2, PLANES><<<grid, 256, 0, stream>>>(a, planes);
+}
+
+template <int EPI>
+static void launch_tiles(const Args& a, const Plan& plan, int nseg, float* planes, hipStream_t stream) {
+  if (planes == nullptr) {
+    launch_tile<EPI, false>(a, plan, nseg, nullptr, stream);
+    return;
+  }
+  launch_tile<EPI, true>(a, plan, nseg, planes, stream);
   const bool by_four = a.N % 4 == 0 && a.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15u) == 0;
   const size_t all = static_cast<size_t>(a.M) * (a.N / (by_four ? 4 : 1));
   const int blocks = static_cast<int>((all + 255) / 256 > 4096 ? 4096 : (all + 255) / 256);
@@ -361,26 +562,32 @@ static void launch_tiles(const Args& a, int tm, int nseg, float* planes, hipStre
   else gemm_f32_sum_kernel<EPI, 1><<<blocks, 256, 0, stream>>>(a, planes, nseg);
 }
 
-struct Plan {
-  int tile_rows;   // 64 or 128; 16: few rows
-  bool cut;
-};
-// The tile and whether K is cut over workgroups: rounds over the 256 CUs times a tile's products at the share of a CU's
-// 614 GFLOP/s that the tile reaches, and for cut tiles the planes written and read at 4 TB/s and one launch more.
-static Plan plan_for(int M, int N, int K, bool gated, int nseg, size_t workspace_bytes) {
-  Plan best{16, false};
+// The tile and whether K is cut over workgroups: the workgroups that the busiest of 256 CUs gets, times a tile's products at the
+// share of a CU's 614 GFLOP/s that the tile reaches, and for cut tiles the planes written and read at 4 TB/s and one launch more.
+// The shares are what products of 512 rows and of 4,096 measured, with a start of 6 us; those of K that is no multiple of 16 the
+// older kernel's.
+static Plan plan_for(int M, int N, int K, int64_t lda, bool gated, int nseg, size_t workspace_bytes) {
+  Plan best{16, 16, false};
   if (M <= 16) return best;
+  struct Tile {
+    int rows, cols;
+    double share;
+  };
+  static const Tile flowing[4] = {{128, 128, 0.88}, {128, 96, 0.83}, {128, 64, 0.83}, {64, 64, 0.73}};
+  static const Tile older[2] = {{128, 128, 0.85}, {64, 64, 0.7}};
+  const bool flow = flows(K, lda);
   const double NW = gated ? 2.0 * N : N;
   const size_t plane_bytes = static_cast<size_t>(nseg) * M * static_cast<size_t>(NW) * sizeof(float);
   double best_us = 1e30;
-  for (int tile_rows = 128; tile_rows >= 64; tile_rows /= 2) {
-    const double rows = tile_rows, tiles = ceil(M / rows) * ceil(NW / rows);
-    const double tile_us = 2.0 * rows * rows * K / (0.614e6 * (tile_rows == 128 ? 0.85 : 0.7));
+  for (int i = 0; i < (flow ? 4 : 2); ++i) {
+    const Tile& t = flow ? flowing[i] : older[i];
+    const double tiles = ceil(M / static_cast<double>(t.rows)) * ceil(NW / t.cols);
+    const double tile_us = 2.0 * t.rows * t.cols * K / (0.614e6 * t.share);
     for (int cut = 0; cut < 2; ++cut) {
       if (cut && (nseg == 1 || plane_bytes > workspace_bytes)) continue;
-      const double us = cut ? ceil(tiles * nseg / 256.0) * tile_us / nseg + 2.0 * plane_bytes / 4e6 + 5.0
-                            : ceil(tiles / 256.0) * tile_us;
-      if (us < best_us) best_us = us, best = Plan{tile_rows, cut != 0};
+      const double us = cut ? ceil(tiles * nseg / 256.0) * tile_us / nseg + 2.0 * plane_bytes / 4e6 + 7.0
+                            : ceil(tiles / 256.0) * tile_us + 6.0;
+      if (us < best_us) best_us = us, best = Plan{t.rows, t.cols, cut != 0};
     }
   }
   return best;
@@ -394,14 +601,14 @@ static int segments(int K, int* length) {
 
 template <int EPI>
 static void launch(const Args& a, int nseg, float* workspace, size_t workspace_bytes, hipStream_t stream) {
-  const Plan plan = plan_for(a.M, a.N, a.K, EPI == 1, nseg, workspace != nullptr ? workspace_bytes : 0);
-  if (plan.tile_rows == 16) {
+  const Plan plan = plan_for(a.M, a.N, a.K, a.lda, EPI == 1, nseg, workspace != nullptr ? workspace_bytes : 0);
+  if (plan.rows == 16) {
     const int blocks = (a.N + 15) / 16;
     if (a.M <= 8) gemm_f32_few_kernel<EPI, 8><<<blocks, 64 * nseg, 0, stream>>>(a);
     else gemm_f32_few_kernel<EPI, 16><<<blocks, 64 * nseg, 0, stream>>>(a);
     return;
   }
-  launch_tiles<EPI>(a, plan.tile_rows / 32, nseg, plan.cut ? workspace : nullptr, stream);
+  launch_tiles<EPI>(a, plan, nseg, plan.cut ? workspace : nullptr, stream);
 }
 
 }  // namespace f32
@@ -426,11 +633,12 @@ int gemm_f32(const float* A, int64_t lda, const float* W, const float* W2, float
 
 }  // namespace sa
 
-// Which way M rows go: 16 (few rows), or a tile's rows (64 or 128), plus 1000 where K is cut over workgroups.
+// Which way M rows go: 16 (few rows), or a tile's rows (64 or 128), plus 1000 where K is cut over workgroups, plus 10000 times the
+// weight rows of a tile.
 extern "C" int sa_gemm_f32_plan(int M, int N, int K, int gated, int64_t workspace_bytes) {
   if (M < 1 || N < 1 || K < 1) return 0;
   int length;
   const int nseg = sa::f32::segments(K, &length);
-  const sa::f32::Plan plan = sa::f32::plan_for(M, N, K, gated != 0, nseg, workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0);
-  return plan.tile_rows + (plan.cut ? 1000 : 0);
+  const sa::f32::Plan plan = sa::f32::plan_for(M, N, K, K, gated != 0, nseg, workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0);
+  return plan.rows + (plan.cut ? 1000 : 0) + 10000 * plan.cols;
 }

@@ -535,8 +535,14 @@ def gemm_plan(M: int, N: int, K: int, *, gated: bool = False, soft_cap: bool = F
 def gemm_f32_plan(M: int, N: int, K: int, *, gated: bool = False) -> tuple[int, bool]:
     """How `gemm` takes M rows of 32-bit operands on the matrix cores: the rows of a tile (16: the kernel for few rows) and
     whether K is cut over workgroups.  A host function."""
-    plan = _lib.load().sa_gemm_f32_plan(int(M), int(N), int(K), int(gated), WORKSPACE_BYTES)
+    plan = _lib.load().sa_gemm_f32_plan(int(M), int(N), int(K), int(gated), WORKSPACE_BYTES) % 10000
     return plan % 1000, plan >= 1000
+
+
+def gemm_f32_tile(M: int, N: int, K: int, *, gated: bool = False) -> tuple[int, int]:
+    """Rows of the operands that a tile of `gemm` takes in 32 bits: of the first and of the weights (gated: of both together)."""
+    plan = _lib.load().sa_gemm_f32_plan(int(M), int(N), int(K), int(gated), WORKSPACE_BYTES)
+    return plan % 1000, plan // 10000
 
 
 def gemm_normed_takes(M: int, w) -> bool:

@@ -72,6 +72,36 @@ def test_products_in_tiles_of_128_rows(M, N, K, gated, cut):
         assert torch.equal(ops.gemm(a[M - 5:], w, soft_cap=2.0), capped[M - 5:])
 
 
+@pytest.mark.parametrize("M,N,K,gated,tile,cut", [
+    (70, 130, 48, False, (64, 64), False), (333, 581, 272, True, (64, 64), False), (130, 300, 1040, False, (64, 64), True),
+    (700, 1500, 272, False, (128, 64), False), (700, 760, 272, True, (128, 64), False), (200, 701, 528, False, (128, 64), True),
+    (1500, 2000, 16, False, (128, 96), False), (300, 8003, 80, False, (128, 96), False), (300, 4010, 80, True, (128, 96), False),
+    (509, 2300, 2064, False, (128, 96), True), (1000, 3135, 272, False, (128, 128), False), (1000, 1570, 272, True, (128, 128), False)])
+def test_products_of_whole_blocks(M, N, K, gated, tile, cut):
+    """K in blocks of 16, through the tiles that hold their operands ahead of the products: the last rows and columns missing, a
+    last stage of one block, one block in all, segments that end inside a stage.  Bounds as above, the bits of the kernel for few
+    rows, and the same from rows of a wider buffer."""
+    from simply_amd.kernels import ops
+
+    assert ops.gemm_f32_tile(M, N, K, gated=gated) == tile and ops.gemm_f32_plan(M, N, K, gated=gated) == (tile[0], cut)
+    wide, w, w2 = draw((M, K + 12), 21), draw((N, K), 22, 0.1), draw((N, K), 23, 0.1)
+    a = wide[:, 8:8 + K]
+    kw = dict(w2=w2, activation=ops.ACT_SILU) if gated else {}
+    got = ops.gemm(a, w, **kw)
+    x, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    bound = (K + 2) * EPS * size
+    if gated:
+        up, up_bound = a.double() @ w2.double().T, (K + 2) * EPS * (a.double().abs() @ w2.double().abs().T)
+        want = torch.nn.functional.silu(x) * up
+        bound = 1.1 * bound * up.abs() + x.abs() * up_bound + 8 * EPS * want.abs()
+    else:
+        want = x
+    assert ((got.double() - want).abs() <= bound).all()
+    assert torch.equal(ops.gemm(a.contiguous(), w, **kw), got)
+    for rows in (slice(0, 5), slice(62, 67), slice(M - 5, M)):
+        assert torch.equal(ops.gemm(a[rows], w, **kw), got[rows])
+
+
 def test_products_keep_special_values():
     """An infinite or undefined entry reaches its own row and column only."""
     from simply_amd.kernels import ops
