@@ -261,6 +261,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
   for (int p = 0; p < NSTAGE; ++p)
 #pragma unroll
     for (int n = 0; n < LOADS; ++n) request_one(n, p < slabs ? p : slabs - 1, p);
+  // (routed) A wave none of whose rows exist copies its share of every slab and leaves the matrix units to the others.
+  if (ROUTED && wm * WM * 16 >= tile_rows) {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm((NSTAGE - 1) * LOADS));
+    bare_barrier();
+    int into = 0;
+    for (int s = 1; s < slabs; ++s) {
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm((NSTAGE - 2) * LOADS));
+      bare_barrier();
+      const int ahead = s + NSTAGE - 1 < slabs ? s + NSTAGE - 1 : slabs - 1;
+#pragma unroll
+      for (int n = 0; n < LOADS; ++n) request_one(n, ahead, into);
+      into = into + 1 == NSTAGE ? 0 : into + 1;
+    }
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    return;
+  }
   // slab 0: nothing held back yet, and its loads for later are already asked for
   __builtin_amdgcn_s_waitcnt(waitcnt_vm((NSTAGE - 1) * LOADS));
   bare_barrier();
@@ -382,12 +398,16 @@ static void launch_routed(const bf16* A, int64_t lda, const bf16* W, const Route
 
 }  // namespace wide
 
-// Products of routed experts on this kernel's tiles: 64 rows of an expert x 128 weight rows with three buffers, or 128 x 192
-// with two (tile_rows); workgroups of four waves, two a CU.  Gate and up together with down of 16 experts, in microseconds:
-//   2,048 x 2,048, rows an expert   16: 72   32: 75   96: 103 / 94   128: 117 / 148   256: 184 / 199   512: 332 / 339 (64 / 128)
-//   4,096 x 3,584                   16: 271  32: 270  96: 352 / 342  128: 420 / 396   256: 636 / 586   512: 1,107 / 1,035
-// (the kernel of routed.hip for 64 rows, which took these products before: 327 at 256 rows of 2,048 x 2,048).  Also tried for
-// 64 rows: eight waves with six buffers (212 at 256 rows), 64 x 256 (199), four waves across (184).
+// Products of routed experts on this kernel's tiles: 64 rows of an expert x 128 weight rows with three buffers, two workgroups of four
+// waves a CU, or (tile_rows) 128 x 256 with three, one of eight waves, 64 x 64 outputs each: a tile's upper 64 rows, which an expert's
+// last tile often lacks, are the business of four waves of their own, that then leave the matrix units to the others.  Gate and up
+// together with down of 16 experts, in microseconds:
+//   2,048 x 2,048, rows an expert   37: 89 / 100   64: 106 / 100   125: 130 / 126   256: 192 / 179   500: 334 / 269 (64 / 128)
+//   4,096 x 3,584                   64: 300 / 270  125: 391 / 367  256: 620 / 534
+//   1,024 x 1,024                   256: 65 / 72   500: 98 / 108
+// (128 x 192 of four waves, two a CU, which the 128 rows were before: 209 at 256 rows of 2,048 x 2,048, 626 of 4,096 x 3,584.)  Also
+// tried for 64 rows: eight waves with six buffers, 64 x 256, four waves across; for 128: 128 x 128 (191 and 546), waves of 128 x 64 and
+// 64 x 128 (237 and 233).
 bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t ldc, const void* A, const void* W, const void* W2,
                             const void* C, int tile_rows) {
   auto aligned = [](const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
@@ -405,7 +425,7 @@ int gemm_wide_routed(const void* A, int64_t lda, const void* W, const void* W2, 
   const bf16* a = static_cast<const bf16*>(A);
   const bf16* w = static_cast<const bf16*>(W);
   bf16* c = static_cast<bf16*>(C);
-  if (tile_rows == 128) wide::launch_routed<4, 6, 2, 2, 4>(a, lda, w, rt, c, y, ldc, tiles, tile_rows, N, K, act, limit, stream);
+  if (tile_rows == 128) wide::launch_routed<4, 4, 2, 3, 8>(a, lda, w, rt, c, y, ldc, tiles, tile_rows, N, K, act, limit, stream);
   else wide::launch_routed<2, 4, 2, 3, 4>(a, lda, w, rt, c, y, ldc, tiles, tile_rows, N, K, act, limit, stream);
   return check_launch("gemm_wide_routed");
 }

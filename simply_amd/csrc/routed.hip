@@ -799,9 +799,9 @@ extern "C" int sa_expert_tile_rows(int P, int E, int D, int F, int dtype, int64_
   // 2,048, 16 experts: 8 rows 63 us with tiles of 16 and 72 with the wide kernel's 64; 16 rows 105 and 72); the kernel of 64
   // rows here is ahead from 32 on.
   if (P < (wide ? 12 : 32) * static_cast<int64_t>(E)) return 16;
-  // Tiles of 128 rows where they fill up and an expert's gate and up are more than the L2s hold (4 MiB an XCD), so that every
-  // tile of rows fetches them again (figures: gemm_wide_routed).
-  return wide && P >= 96 * static_cast<int64_t>(E) && 4.0 * D * F > 32.0 * (1 << 20) &&
+  // Tiles of 128 rows where an expert has more than 64 on average or nearly, and its gate and up are 16 MiB, more than an XCD's L2
+  // holds, so that every tile of rows fetches them again (figures: gemm_wide_routed).
+  return wide && P >= 60 * static_cast<int64_t>(E) && 4.0 * D * F >= 16.0 * (1 << 20) &&
                  sa_expert_tiles_max(P, E, kTileRowsWide) <= kGridMax
              ? kTileRowsWide
              : kTileRowsMax;
