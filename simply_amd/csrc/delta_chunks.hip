@@ -16,7 +16,8 @@
 //                         queries, the solution W, U0 by blocks of 16 rows (the blocks on the diagonal inverted by
 //                         substitution, the others by products), and all operands of the second kernel, scaled, in the
 //                         order in which its matrix instructions take them, into the workspace
-//   delta_state_kernel    the walk through the pieces, a workgroup of four waves per head and 16 value columns
+//   delta_state_kernel    the walk through the pieces, a workgroup of four waves per head and 16 value columns; or, for long
+//                         requests of few heads (keeps_states), delta_walk_kernel for the state alone and piece_outputs_kernel
 //
 // Everything is 32-bit: products are v_mfma_f32_16x16x4_f32, sums of logarithms 64-bit.  A 16 x 16 result holds rows
 // 4 g + r (g = lane / 16) and column lane % 16; an operand of step r holds k = 4 g + r, so that a result is the next
@@ -32,8 +33,8 @@
 // decays drawn evenly from 0 to 1, half-lives of a token, 1.2 and 1.2 to 1.4 times, and no less with exponentials in 64 bits);
 // with one or two chains each results were off by up to twice as much.
 //
-// Measured at 2,048 tokens of 16 heads over 8, sizes 128: 41 us for the pieces and 98 for the walk (38 and 89 with one or two
-// chains), where delta_rule.hip takes 589 token by token.
+// Measured at 2,048 tokens of 16 heads over 8, sizes 128: 121 us (traced, 50 for the pieces, 60 for the walk of the state, 29 for the
+// outputs; 137 with delta_state_kernel's 106 instead), where delta_rule.hip takes 589 token by token.
 #include "api.h"
 #include "chunks.h"
 
@@ -44,18 +45,19 @@ using namespace chunks;
 
 // A piece's operands in the workspace (floats), for NT blocks of 16 key channels and CB blocks of 16 value columns.
 struct Layout {
-  int w, q, kt, p, u0, decay, own, words;
+  int w, q, kt, p, u0, decay, own, states, words;   // states: in front of the pieces, where they are kept
 };
-__host__ __device__ constexpr Layout layout(int nt, int cb) {
+__host__ __device__ constexpr Layout layout(int nt, int cb, bool keep) {
   Layout l{};
   l.w = 0;                             // [token block][channel block]
   l.q = l.w + kBlocks * nt * kBlock;   // likewise
   l.kt = l.q + kBlocks * nt * kBlock;  // [channel block][token block]
   l.p = l.kt + kBlocks * nt * kBlock;  // [token block][token block], without the diagonal
-  l.u0 = l.p + kBlocks * kBlocks * kBlock;   // [column block][token block]
+  l.u0 = l.p + kBlocks * kBlocks * kBlock;   // [column block][token block]; where states are kept, then U
   l.decay = l.u0 + cb * kBlocks * kBlock;    // exp(L_64)
   l.own = l.decay + 64;                      // the diagonal of P
-  l.words = l.own + kTokens;
+  l.states = l.own + kTokens;                // [column block][channel block]
+  l.words = l.states + (keep ? cb * nt * kBlock : 0);
   return l;
 }
 
@@ -68,6 +70,7 @@ struct Args {
   const int* seq_meta;
   int64_t state_stride;
   int C, G, H, dk, dv, row0, row1;   // the rows of the step that this launch is about
+  bool keep;            // the states in front of the pieces
 };
 
 // exp(x) for x <= 0; what 32 bits do not hold of x goes in as a factor (a rounding of x alone would be |x| of them of exp(x)).
@@ -85,14 +88,14 @@ __global__ __launch_bounds__(256) void delta_pieces_kernel(Args a) {
   __shared__ float beta_s[kTokens], in_s[kTokens], out_s[kTokens];   // beta, exp(L_i), exp(L_64 - L_i)
   static_assert(kTokens * ROW >= kTokens * AROW || NT < 4, "A lies where q lay");
   const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
-  const int t0 = blockIdx.x * kTokens;
+  const int t0 = blockIdx.y * kTokens;
   if (t0 >= sp.count) return;   // (uniform)
   const int left = sp.count - t0 < kTokens ? sp.count - t0 : kTokens;
-  const int h = blockIdx.y, tid = threadIdx.x, lane = tid % kWave;
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
   const int qk = h / (a.H / a.G), row0 = sp.first + t0;
-  const Layout lay = layout(NT, (a.dv + 15) / 16);
-  float* dst = a.pieces + (static_cast<size_t>(sp.piece0 + blockIdx.x) * a.H + h) * lay.words;
+  const Layout lay = layout(NT, (a.dv + 15) / 16, a.keep);
+  float* dst = a.pieces + (static_cast<size_t>(sp.piece0 + blockIdx.y) * a.H + h) * lay.words;
 
   // rows of q and k (tokens behind the last, channels behind the last: zeros)
 #pragma unroll
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
   const int col = blockIdx.y * 16 + c;
   const bool col_ok = col < a.dv;
-  const Layout lay = layout(NT, (a.dv + 15) / 16);
+  const Layout lay = layout(NT, (a.dv + 15) / 16, a.keep);
   const float* src = a.pieces + (static_cast<size_t>(sp.piece0) * a.H + h) * lay.words;
   const size_t step = static_cast<size_t>(a.H) * lay.words;
   float* S = a.state + static_cast<size_t>(sp.slot) * a.state_stride + static_cast<size_t>(h) * a.dk * a.dv;
@@ -275,26 +278,27 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
     u0 = *reinterpret_cast<const floatx4*>(from + lay.u0 + (blockIdx.y * kBlocks + wave) * kBlock + lane * 4);
   };
   auto fetch_rest = [&](const float* from) __attribute__((always_inline)) {
-#pragma unroll
-    for (int n = 0; n < NT; ++n) q[n] = *reinterpret_cast<const floatx4*>(from + lay.q + (wave * NT + n) * kBlock + lane * 4);
+    all = from[lay.decay];
 #pragma unroll
     for (int n = 0; n < NW; ++n)
 #pragma unroll
       for (int b = 0; b < kBlocks; ++b)
         kt[n][b] = *reinterpret_cast<const floatx4*>(from + lay.kt + ((wave * NW + n) * kBlocks + b) * kBlock + lane * 4);
 #pragma unroll
+    for (int n = 0; n < NT; ++n) q[n] = *reinterpret_cast<const floatx4*>(from + lay.q + (wave * NT + n) * kBlock + lane * 4);
+#pragma unroll
     for (int b = 0; b < kBlocks; ++b) {   // (the last: the wave's own; others behind it: that again, not used)
       const int at = b < wave ? b : wave;
       p[b] = *reinterpret_cast<const floatx4*>(from + lay.p + (wave * kBlocks + at) * kBlock + lane * 4);
     }
     own = *reinterpret_cast<const floatx4*>(from + lay.own + wave * 16 + g * 4);
-    all = from[lay.decay];
   };
   fetch_state(src);
   fetch_rest(src);
   int now = 0;
   for (int t0 = 0; t0 < sp.count; t0 += kTokens, now ^= 1) {
-    const float* next = t0 + kTokens < sp.count ? src + step : src;   // (behind the last piece: that one again, for nothing)
+    // (behind the last piece: that one again, for nothing)
+    const float* next = t0 + kTokens < sp.count ? src + step : src;
     __syncthreads();   // the state in front of the piece is there
     floatx4 st[NT];
 #pragma unroll
@@ -340,7 +344,6 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
     floatx4 result = sum_of(o) + sum_of(o2);
 #pragma unroll
     for (int r = 0; r < 4; ++r) result[r] = fmaf(own[r], u[r], result[r]);
-    fetch_rest(next);
     if (col_ok) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -348,7 +351,128 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
         if (t < sp.count) a.out[static_cast<size_t>(sp.first + t) * (static_cast<size_t>(a.H) * a.dv) + static_cast<size_t>(h) * a.dv + col] = result[r];
       }
     }
+    fetch_rest(next);
     src = next;
+  }
+#pragma unroll
+  for (int n = 0; n < NW; ++n) {
+    const int d = (wave * NW + n) * 16 + g * 4;
+    if (col_ok && d < a.dk) *reinterpret_cast<floatx4*>(S + static_cast<size_t>(col) * a.dk + d) = s[n];
+  }
+}
+
+// The walk for the state alone: the same sums, and U and the state in front of each piece are kept for piece_outputs_kernel.  Of 110
+// matrix instructions a wave issues 64 a piece; the next piece's operands are asked for, and what is kept is written, among the
+// products of the state's increment.  (Operands of two pieces ahead, in twice the registers, were slower: 66 us instead of 60.)
+template <int NT>
+__global__ __launch_bounds__(256) void delta_walk_kernel(Args a) {
+  constexpr int NW = NT / 4;   // blocks of key channels whose state a wave holds
+  __shared__ __align__(16) floatx4 s_s[2][NT * kWave];
+  __shared__ __align__(16) floatx4 u_s[kBlocks * kWave];
+  const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
+  if (sp.count <= 0) return;
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
+  const int col = blockIdx.y * 16 + c, count = (sp.count + kTokens - 1) / kTokens;
+  const bool col_ok = col < a.dv;
+  const Layout lay = layout(NT, (a.dv + 15) / 16, true);
+  float* first = a.pieces + (static_cast<size_t>(sp.piece0) * a.H + h) * lay.words;
+  const size_t step = static_cast<size_t>(a.H) * lay.words;
+  float* S = a.state + static_cast<size_t>(sp.slot) * a.state_stride + static_cast<size_t>(h) * a.dk * a.dv;
+  floatx4 s[NW];
+#pragma unroll
+  for (int n = 0; n < NW; ++n) {
+    const int d = (wave * NW + n) * 16 + g * 4;
+    s[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (col_ok && d < a.dk) s[n] = *reinterpret_cast<const floatx4*>(S + static_cast<size_t>(col) * a.dk + d);
+    s_s[0][(wave * NW + n) * kWave + lane] = s[n];
+  }
+  floatx4 w[NT], kt[NW][kBlocks], u0;
+  float all;
+  // a piece's operands, asked for a piece ahead
+  auto fetch_w = [&](const float* from, int n) __attribute__((always_inline)) {
+    w[n] = *reinterpret_cast<const floatx4*>(from + lay.w + (wave * NT + n) * kBlock + lane * 4);
+  };
+  auto fetch_kt = [&](const float* from, int n, int b) __attribute__((always_inline)) {
+    kt[n][b] = *reinterpret_cast<const floatx4*>(from + lay.kt + ((wave * NW + n) * kBlocks + b) * kBlock + lane * 4);
+  };
+  auto fetch_rest = [&](const float* from) __attribute__((always_inline)) {
+    u0 = *reinterpret_cast<const floatx4*>(from + lay.u0 + (blockIdx.y * kBlocks + wave) * kBlock + lane * 4);
+    all = from[lay.decay];
+  };
+#pragma unroll
+  for (int n = 0; n < NT; ++n) fetch_w(first, n);
+#pragma unroll
+  for (int n = 0; n < NW; ++n)
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) fetch_kt(first, n, b);
+  fetch_rest(first);
+  for (int at = 0; at < count; at += 2) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (at + i >= count) break;   // (uniform)
+      float* piece = first + (at + i) * step;
+      // (behind the last piece: that one again, for nothing; its U0 may have become U)
+      const float* from = at + i + 1 < count ? piece + step : piece;
+      __syncthreads();   // the state in front of the piece is there
+      floatx4 st[NT], x[4], more[2][NW];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) st[n] = s_s[i][n * kWave + lane];
+      __builtin_amdgcn_sched_barrier(0);   // (all reads are under way before the first product)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int n = 0; n < NT; n += 4)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)   // (the four chains in turn)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            x[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[n + e][r], st[n + e][r], x[e], 0, 0, 0);
+      const floatx4 u = u0 - sum_of(x);
+      u_s[wave * kWave + lane] = u;
+      __syncthreads();
+      floatx4 ub[kBlocks];
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b) ub[b] = u_s[b * kWave + lane];
+#pragma unroll
+      for (int n = 0; n < NW; ++n) more[0][n] = more[1][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+      const float decay = all;
+      // memory is asked for among these products, one access after every few: nothing but LDS stands between the others' u and x
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < kBlocks; b += 2) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int n = 0; n < NW; ++n)
+              more[e][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[n][b + e][r], ub[b + e][r], more[e][n], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (b / 2 * 4 + r < NT) fetch_w(from, b / 2 * 4 + r);
+          if (b == 0 && r < NW)
+            *reinterpret_cast<floatx4*>(piece + lay.states + (blockIdx.y * NT + wave * NW + r) * kBlock + lane * 4) = s[r];
+          if (b == 0 && r == 3) *reinterpret_cast<floatx4*>(piece + lay.u0 + (blockIdx.y * kBlocks + wave) * kBlock + lane * 4) = u;
+          if (b == 2 && r < NW) {
+            fetch_kt(from, r, 0);
+            fetch_kt(from, r, 1);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < NW; ++n) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[n][r] = fmaf(s[n][r], decay, more[0][n][r] + more[1][n][r]);
+        s_s[i ^ 1][(wave * NW + n) * kWave + lane] = s[n];
+      }
+#pragma unroll
+      for (int n = 0; n < NW; ++n) {
+        fetch_kt(from, n, 2);
+        fetch_kt(from, n, 3);
+      }
+      fetch_rest(from);
+    }
   }
 #pragma unroll
   for (int n = 0; n < NW; ++n) {
@@ -362,8 +486,8 @@ __global__ __launch_bounds__(256) void delta_state_kernel(Args a) {
 
 using namespace sa;
 
-static int64_t delta_piece_bytes(int H, int dk, int dv) {
-  return static_cast<int64_t>(H) * delta::layout(dk <= 64 ? 4 : 8, (dv + 15) / 16).words * static_cast<int64_t>(sizeof(float));
+static int64_t delta_piece_bytes(int H, int dk, int dv, bool keep = false) {
+  return static_cast<int64_t>(H) * delta::layout(dk <= 64 ? 4 : 8, (dv + 15) / 16, keep).words * static_cast<int64_t>(sizeof(float));
 }
 
 extern "C" int sa_delta_chunks_takes(int C, int G, int H, int dk, int dv, int64_t state_stride, int num_seqs, int64_t workspace_bytes) {
@@ -389,21 +513,31 @@ extern "C" int sa_delta_chunks(const float* qkv, int C, int G, int dk, int dv, c
   delta::Args a;
   a.qkv = qkv, a.gates = gates, a.state = state, a.out = out, a.pieces = static_cast<float*>(workspace), a.seq_meta = seq_meta;
   a.state_stride = state_stride, a.C = C, a.G = G, a.H = H, a.dk = dk, a.dv = dv;
+  a.keep = chunks::keeps_states(max_q_len, static_cast<int64_t>(H) * ((dv + 15) / 16) * num_seqs) &&
+           rows / chunks::kTokens + num_seqs < workspace_bytes / delta_piece_bytes(H, dk, dv, true);
   // as many rows at a time as the workspace has room for: R rows are at most R / 64 + num_seqs pieces
-  const int64_t room = (workspace_bytes / delta_piece_bytes(H, dk, dv) - num_seqs) * chunks::kTokens;
+  const int64_t room = (workspace_bytes / delta_piece_bytes(H, dk, dv, a.keep) - num_seqs) * chunks::kTokens;
   const int span = static_cast<int>(room < rows ? room : rows);
   for (int r = 0; r < rows; r += span) {
     a.row0 = first_row + r;
     a.row1 = first_row + (r + span < rows ? r + span : rows);
     const int longest = a.row1 - a.row0 < max_q_len ? a.row1 - a.row0 : max_q_len;
-    const dim3 pieces((longest + chunks::kTokens - 1) / chunks::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
-    if (dk <= 64) {
-      delta::delta_pieces_kernel<4><<<pieces, 256, 0, stream>>>(a);
-      delta::delta_state_kernel<4><<<walk, 256, 0, stream>>>(a);
-    } else {
-      delta::delta_pieces_kernel<8><<<pieces, 256, 0, stream>>>(a);
-      delta::delta_state_kernel<8><<<walk, 256, 0, stream>>>(a);
-    }
+    const dim3 pieces(H, (longest + chunks::kTokens - 1) / chunks::kTokens, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
+#define SA_DELTA(NT)                                                                               \
+  do {                                                                                             \
+    delta::delta_pieces_kernel<NT><<<pieces, 256, 0, stream>>>(a);                                 \
+    if (a.keep) {                                                                                  \
+      const delta::Layout lay = delta::layout(NT, (dv + 15) / 16, true);                           \
+      const chunks::OutputsAt at{lay.q, lay.p, lay.u0, lay.states, lay.own, lay.words};            \
+      delta::delta_walk_kernel<NT><<<walk, 256, 0, stream>>>(a);                            \
+      chunks::piece_outputs_kernel<NT, true><<<pieces, 256, 0, stream>>>(a.pieces, at, seq_meta, a.row0, a.row1, H, dv, out); \
+    } else {                                                                                       \
+      delta::delta_state_kernel<NT><<<walk, 256, 0, stream>>>(a);                           \
+    }                                                                                              \
+  } while (0)
+    if (dk <= 64) SA_DELTA(4);
+    else SA_DELTA(8);
+#undef SA_DELTA
   }
   return check_launch("delta_chunks");
 }

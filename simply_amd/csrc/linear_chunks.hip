@@ -15,7 +15,8 @@
 //   linear_pieces_kernel   everything that does not need the state, a workgroup per piece and head: M and the scaled queries,
 //                          keys and values, in the order in which the second kernel's instructions take them
 //   linear_walk_kernel     the walk through the pieces, a workgroup of four waves per head and 16 value columns, as
-//                          delta_state_kernel does it (delta_chunks.hip), with one barrier a piece
+//                          delta_state_kernel does it (delta_chunks.hip), with one barrier a piece; or, for long requests of few
+//                          heads (keeps_states), linear_scan_kernel for the state alone and piece_outputs_kernel, the same sums
 //
 // Sums and products are 32-bit (v_mfma_f32_16x16x4_f32).  The first kernel is bound by a wave's vector instructions (two
 // times 16 steps of 32 multiplications in 64 bits with their conversions, of keys and of queries one after the other: with both
@@ -31,7 +32,8 @@
 //   the same between 0 and 1                      0.96           1.25 to 1.40
 // (with decays multiplied in 32 bits and two or four chains the second to fourth were 1.04 to 1.19 and 1.16 to 1.8.)
 //
-// Measured at 2,048 tokens of 16 heads of 128: 122 us (traced, 48 for the pieces and 81 for the walk), where
+// Measured at 2,048 tokens of 16 heads of 128: 91 us (traced, 48 for the pieces, 22 for the scan and 25 for the outputs; 126 with the
+// walk's 81 instead), where
 // linear_state.hip takes 704 token by token.
 #include "api.h"
 #include "chunks.h"
@@ -43,16 +45,17 @@ using namespace chunks;
 
 // A piece's operands in the workspace (floats), for NT blocks of 16 key channels and CB blocks of 16 value columns.
 struct Layout {
-  int q, kt, p, v, all, words;
+  int q, kt, p, v, all, states, words;   // states: in front of the pieces, where they are kept
 };
-__host__ __device__ constexpr Layout layout(int nt, int cb) {
+__host__ __device__ constexpr Layout layout(int nt, int cb, bool keep) {
   Layout l{};
   l.q = 0;                              // [token block][channel block]
   l.kt = l.q + kBlocks * nt * kBlock;   // [channel block][token block]
   l.p = l.kt + kBlocks * nt * kBlock;   // [token block][token block]
   l.v = l.p + kBlocks * kBlocks * kBlock;   // [column block][token block]
   l.all = l.v + cb * kBlocks * kBlock;      // [16 nt] the decays of the whole piece
-  l.words = l.all + 16 * nt;
+  l.states = l.all + 16 * nt;               // [column block][channel block]
+  l.words = l.states + (keep ? cb * nt * kBlock : 0);
   return l;
 }
 
@@ -68,6 +71,7 @@ struct Args {
   int64_t proj_stride, gates_stride, state_stride;
   float q_mult, inv_tau;
   int q_at, k_at, v_at, H, dk, dv, bias_dtype, bonus_dtype, row0, row1;
+  bool keep;            // the states in front of the pieces
 };
 
 __device__ __forceinline__ floatx4 to_float4(uint2 v) {   // four bfloat16
@@ -83,14 +87,14 @@ __global__ __launch_bounds__(256) void linear_pieces_kernel(Args a) {
   __shared__ __align__(16) bf16 k_s[kTokens * QROW];
   __shared__ __align__(16) float blk_s[kBlocks][NT * 16];   // a block's decays, multiplied
   const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
-  const int t0 = blockIdx.x * kTokens;
+  const int t0 = blockIdx.y * kTokens;
   if (t0 >= sp.count) return;   // (uniform)
   const int left = sp.count - t0 < kTokens ? sp.count - t0 : kTokens;
-  const int h = blockIdx.y, tid = threadIdx.x, lane = tid % kWave;
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
   const int row0 = sp.first + t0, cb = (a.dv + 15) / 16;
-  const Layout lay = layout(NT, cb);
-  float* dst = a.pieces + (static_cast<size_t>(sp.piece0 + blockIdx.x) * a.H + h) * lay.words;
+  const Layout lay = layout(NT, cb, a.keep);
+  float* dst = a.pieces + (static_cast<size_t>(sp.piece0 + blockIdx.y) * a.H + h) * lay.words;
 
   // rows of q, k and the decays (tokens behind the last: nothing, decays of one; channels behind the last: zeros)
 #pragma unroll
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), c = lane % 16, g = lane / 16;
   const int col = blockIdx.y * 16 + c;
   const bool col_ok = col < a.dv;
-  const Layout lay = layout(NT, (a.dv + 15) / 16);
+  const Layout lay = layout(NT, (a.dv + 15) / 16, a.keep);
   const float* src = a.pieces + (static_cast<size_t>(sp.piece0) * a.H + h) * lay.words;
   const size_t step = static_cast<size_t>(a.H) * lay.words;
   float* S = a.state + static_cast<size_t>(sp.slot) * a.state_stride + static_cast<size_t>(h) * a.dk * a.dv;
@@ -343,13 +347,60 @@ __global__ __launch_bounds__(256) void linear_walk_kernel(Args a) {
   }
 }
 
+// The walk for the state alone, which keeps the state in front of each piece for piece_outputs_kernel: a wave per head and block of 16
+// channels x 16 columns, and no barriers, as no wave needs another's part.  What a piece adds does not need the state, so that its
+// products run ahead of the chain, which is one multiply-add a piece.
+template <int NT>
+__global__ __launch_bounds__(256, 2) void linear_scan_kernel(Args a) {
+  constexpr int AHEAD = 3;   // pieces whose operands are asked for
+  const Span sp = span_of(a.seq_meta, a.row0, a.row1, blockIdx.z);
+  if (sp.count <= 0) return;
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
+  const int job = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(tid / kWave), n = job % NT, cbk = job / NT;
+  const int c = lane % 16, g = lane / 16, col = cbk * 16 + c, d = n * 16 + g * 4, count = (sp.count + kTokens - 1) / kTokens;
+  const bool ok = col < a.dv && d < a.dk;
+  const Layout lay = layout(NT, (a.dv + 15) / 16, true);
+  float* piece = a.pieces + (static_cast<size_t>(sp.piece0) * a.H + h) * lay.words;
+  const size_t step = static_cast<size_t>(a.H) * lay.words;
+  float* S = a.state + static_cast<size_t>(sp.slot) * a.state_stride + static_cast<size_t>(h) * a.dk * a.dv + static_cast<size_t>(col) * a.dk + d;
+  floatx4 s{0.f, 0.f, 0.f, 0.f};
+  if (ok) s = *reinterpret_cast<const floatx4*>(S);
+  floatx4 kt[AHEAD][kBlocks], v[AHEAD][kBlocks], all[AHEAD];
+  auto fetch = [&](int i, int of) __attribute__((always_inline)) {   // (behind the last piece: that one again, for nothing)
+    const float* from = piece + (of < count ? of : count - 1) * step;
+    all[i] = *reinterpret_cast<const floatx4*>(from + lay.all + d);
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+      kt[i][b] = *reinterpret_cast<const floatx4*>(from + lay.kt + (n * kBlocks + b) * kBlock + lane * 4);
+      v[i][b] = *reinterpret_cast<const floatx4*>(from + lay.v + (cbk * kBlocks + b) * kBlock + lane * 4);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) fetch(i, i);
+  for (int at = 0; at < count; at += AHEAD) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      if (at + i >= count) break;   // (uniform)
+      floatx4 more[kBlocks];
+#pragma unroll
+      for (int b = 0; b < kBlocks; ++b) more[b] = mul4(kt[i][b], v[i][b], floatx4{0.f, 0.f, 0.f, 0.f});
+      const floatx4 added = ((more[0] + more[1]) + more[2]) + more[3], decays = all[i];
+      *reinterpret_cast<floatx4*>(piece + (at + i) * step + lay.states + (cbk * NT + n) * kBlock + lane * 4) = s;
+      fetch(i, at + i + AHEAD);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[r] = fmaf(s[r], decays[r], added[r]);
+    }
+  }
+  if (ok) *reinterpret_cast<floatx4*>(S) = s;
+}
+
 }  // namespace linear
 }  // namespace sa
 
 using namespace sa;
 
-static int64_t linear_piece_bytes(int H, int dk, int dv) {
-  return static_cast<int64_t>(H) * linear::layout(dk <= 64 ? 4 : 8, (dv + 15) / 16).words * static_cast<int64_t>(sizeof(float));
+static int64_t linear_piece_bytes(int H, int dk, int dv, bool keep = false) {
+  return static_cast<int64_t>(H) * linear::layout(dk <= 64 ? 4 : 8, (dv + 15) / 16, keep).words * static_cast<int64_t>(sizeof(float));
 }
 
 extern "C" int sa_linear_chunks_takes(int H, int dk, int dv, int q_at, int k_at, int64_t proj_stride, int64_t gates_stride,
@@ -385,19 +436,28 @@ extern "C" int sa_linear_chunks(const void* proj, int64_t proj_stride, int q_at,
   a.pieces = static_cast<float*>(workspace), a.seq_meta = seq_meta, a.proj_stride = proj_stride, a.gates_stride = gates_stride;
   a.state_stride = state_stride, a.q_mult = q_mult, a.inv_tau = tau > 0.f ? 1.f / tau : 0.f, a.q_at = q_at, a.k_at = k_at;
   a.v_at = v_at, a.H = H, a.dk = dk, a.dv = dv, a.bias_dtype = bias_dtype, a.bonus_dtype = bonus_dtype;
+  a.keep = chunks::keeps_states(max_q_len, static_cast<int64_t>(H) * ((dv + 15) / 16) * num_seqs) &&
+           rows / chunks::kTokens + num_seqs < workspace_bytes / linear_piece_bytes(H, dk, dv, true);
   // as many rows at a time as the workspace has room for: R rows are at most R / 64 + num_seqs pieces
-  const int64_t room = (workspace_bytes / linear_piece_bytes(H, dk, dv) - num_seqs) * chunks::kTokens;
+  const int64_t room = (workspace_bytes / linear_piece_bytes(H, dk, dv, a.keep) - num_seqs) * chunks::kTokens;
   const int span = static_cast<int>(room < rows ? room : rows);
   for (int r = 0; r < rows; r += span) {
     a.row0 = first_row + r;
     a.row1 = first_row + (r + span < rows ? r + span : rows);
     const int longest = a.row1 - a.row0 < max_q_len ? a.row1 - a.row0 : max_q_len;
-    const dim3 pieces((longest + chunks::kTokens - 1) / chunks::kTokens, H, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
+    const dim3 pieces(H, (longest + chunks::kTokens - 1) / chunks::kTokens, num_seqs), walk(H, (dv + 15) / 16, num_seqs);
 #define SA_LINEAR(NT)                                                                              \
   do {                                                                                             \
     if (bonus != nullptr) linear::linear_pieces_kernel<NT, true><<<pieces, 256, 0, stream>>>(a);   \
     else linear::linear_pieces_kernel<NT, false><<<pieces, 256, 0, stream>>>(a);                   \
-    linear::linear_walk_kernel<NT><<<walk, 256, 0, stream>>>(a);                                   \
+    if (a.keep) {                                                                                  \
+      const linear::Layout lay = linear::layout(NT, (dv + 15) / 16, true);                         \
+      const chunks::OutputsAt at{lay.q, lay.p, lay.v, lay.states, 0, lay.words};                   \
+      linear::linear_scan_kernel<NT><<<dim3(H, (dv + 15) / 16 * (NT / 4), num_seqs), 256, 0, stream>>>(a); \
+      chunks::piece_outputs_kernel<NT, false><<<pieces, 256, 0, stream>>>(a.pieces, at, seq_meta, a.row0, a.row1, H, dv, out); \
+    } else {                                                                                       \
+      linear::linear_walk_kernel<NT><<<walk, 256, 0, stream>>>(a);                                 \
+    }                                                                                              \
   } while (0)
     if (dk <= 64) SA_LINEAR(4);
     else SA_LINEAR(8);

@@ -313,3 +313,41 @@ def test_delta_rule_keeps_special_values(bad, token):
     hit[token:first + count, 1] = True
     got, want = got.view(T, H, dv), want.view(T, H, dv)
     assert not torch.isfinite(got[hit]).any() and torch.equal(got[~hit], want[~hit])
+
+
+@pytest.mark.parametrize("H,dk,dv,T", [(2, 128, 128, 768), (3, 40, 24, 1025), (1, 64, 130, 831), (2, 100, 3, 900)])
+@pytest.mark.parametrize("bad", [None, float("inf"), float("nan")])
+def test_outputs_behind_the_walk(H, dk, dv, T, bad):
+    """A long request by itself, whose states are kept and whose outputs are made behind the walk, and the same request among so many
+    that its outputs are made on the way: the same sums in the same order, so the same bits, also where a value is not finite."""
+    from simply_amd.kernels import ops
+
+    n = 128 // (H * -(-dv // 16)) + 1   # one more than half of the CUs have walkers for
+    G, counts = H, [T] + [1] * n
+    rows = sum(counts)
+    meta = torch.tensor([[len(counts) - 1 - i, sum(counts[:i]), c, 0] for i, c in enumerate(counts)], dtype=torch.int32).cuda()
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(1.0), b.nan_to_num(1.0))
+
+    def both(run, width):
+        got = []
+        for k in (1, len(counts)):
+            state, out = normal((len(counts), H * dk * dv), 131).cuda(), torch.zeros(rows, width, device="cuda")
+            run(state, k, out)
+            got.append((out[:T], state[len(counts) - 1]))
+        assert same(got[0][0], got[1][0]) and same(got[0][1], got[1][1]) and got[0][0][:100].isfinite().all()
+
+    C = 2 * G * dk + H * dv
+    C += -C % 4
+    qkv = normal((rows, C), 132) * dk ** -0.5
+    gates = torch.cat([uniform((rows, H), 133), uniform((rows, H), 134, 0.9, 1.0)], 1)
+    proj = normal((rows, 2 * H * dk + H * dv), 135).bfloat16()
+    proj = torch.cat([proj, torch.zeros(rows, -proj.shape[1] % 4, dtype=proj.dtype)], 1)
+    if bad is not None:
+        qkv[T - 70, 2 * G * dk + 1] = bad
+        proj[T - 70, 2 * H * dk + 1] = bad
+    x, g, p, decay, bonus = qkv.cuda(), gates.cuda(), proj.cuda(), uniform((rows, H * dk), 136, 0.5, 1.0).cuda(), normal((H * dk,), 137).cuda()
+    of = lambda t, k: t[:T] if k == 1 else t
+    both(lambda s, k, out: ops.delta_chunks(of(x, k), of(g, k), s, meta, k, 0, T, H, G, dk, dv, out=of(out, k)), H * dv)
+    for u in (None, bonus):
+        both(lambda s, k, out: ops.linear_chunks(of(p, k), 0, H * dk, 2 * H * dk, 1.0, of(decay, k), H, dk, dv, s, meta, k, 0, T, bonus=u,
+                                                 out=of(out, k)), H * dv)
