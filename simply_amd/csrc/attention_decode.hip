@@ -623,6 +623,10 @@ int paged_attention_decode(const void* q, int64_t q_stride, const void* k_pages,
     }
   }
   int KS = paged_attention_decode_ranges(seq_count, Kh, window, max_kv_len, num_splits);
+  // Few keys: one range, and no second kernel.  Microseconds with one range / as cut above, keys in HBM: heads of 256, 64 keys
+  // 9.3 / 12.4, 128 11.6 / 13.3, 192 14.3 / 13.5; of 128, 64 7.2 / 11.1, 256 10.4 / 11.7, 512 13.8 / 12.1 (one request, 4 and 16 key
+  // heads; 8 requests: 9.9 / 12.7, 12.5 / 14.2, 15.7 / 14.4 and 7.8 / 11.9, 11.8 / 15.4, 14.4 / 17.0).
+  if (num_splits <= 0 && decode_max_tiles(window, max_kv_len) <= (hd > 128 ? 5 : 9)) KS = 1;
   const size_t per_split = static_cast<size_t>(units) * 16 * (hd + kRowExtra) * sizeof(float);
   while (KS > 1 && (workspace == nullptr || per_split * KS > workspace_bytes)) --KS;
   // (ranges of more than kMaxRangeSubTiles sub-tiles, which a small workspace or a caller's own num_splits may
