@@ -628,19 +628,19 @@ int sa_expert_product(const void* a, int dtype, int64_t a_stride, int a_by_token
                       void* out, int64_t out_stride, int out_by_pair, int activate, hipStream_t stream);
 // A router of a few tokens in one launch: logits [T, rows] (32-bit) = x . w^T with x bfloat16 [T, D] and w tiled, the choice as
 // sa_route (plain) or sa_route_choice make it from the first E logits of a token, sorted and plan as sa_expert_sort with tiles
-// of 16 rows.  _takes: at most 16 tokens, 128 experts (and up to 16 more rows) and 128 pairs, weights of up to 128 K entries.
+// of 16 rows; and, with dense_w (tiled, gated: the two factors' tiles in turn), dense_out [T, dense_N] bfloat16 = rule(x . dense_w^T).
+// _takes: at most 16 tokens, 128 experts (and up to 16 more rows) and 128 pairs, weights of up to 128 K entries.
 int sa_route_few_takes(const void* x, int64_t x_stride, int T, int D, int rows, int E, int top);
 int sa_route_few(const void* x, int64_t x_stride, const void* w, int T, int D, int rows, int E, int top, float scale, int plain,
                  const void* bias, int bias_dtype, const void* correction, int corr_dtype, int groups, int keep, int softmax,
                  int group_best, float renorm, float* logits, int* experts, float* weights, int* sorted, int* plan, int plan_words,
-                 hipStream_t stream);
-// sa_expert_product in bfloat16 with tiles of 16 rows, and beside it the same product of all T <= 16 tokens with a dense weight:
-// shared_out[t] = rule(shared_a[t]); shared_w: tiled, with w2 the two factors' tiles in turn.
-int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w1, const void* w2, int N, int K,
-                             const int* sorted, const int* plan, int P, int E, int act, float limit, void* out, int64_t out_stride,
-                             int out_by_pair, int activate, const void* shared_a, int64_t shared_a_stride, const void* shared_w,
-                             int shared_N, int shared_K, int T, float shared_limit, void* shared_out, int64_t shared_out_stride,
-                             hipStream_t stream);
+                 const void* dense_w, int dense_N, int dense_gated, int dense_act, float dense_limit, void* dense_out, hipStream_t stream);
+// sa_expert_product in bfloat16 with tiles of 16 rows and one weight, and beside it all T <= 16 tokens' product with a dense one:
+// shared_out[t] = shared_a[t] . shared_w^T, 32-bit.
+int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w, int N, int K, const int* sorted,
+                             const int* plan, int P, int E, void* out, int64_t out_stride, int out_by_pair, const void* shared_a,
+                             int64_t shared_a_stride, const void* shared_w, int shared_N, int shared_K, int T, void* shared_out,
+                             int64_t shared_out_stride, hipStream_t stream);
 // out[t] = sum_k weights[t, k] y[t * top + k] + sigmoid(gate[t]) * shared[t]  (shared null: none; gate null: 1).
 int sa_expert_combine(const float* y, const float* weights, int top, const void* shared, int shared_dtype,
                       int64_t shared_stride, const float* gate, int64_t gate_stride, void* out, int out_dtype,

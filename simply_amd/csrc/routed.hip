@@ -267,30 +267,83 @@ __device__ __forceinline__ bf16x8 load8(const bf16* p) { return *reinterpret_cas
 // choice, and the pairs in the order of their experts, in one workgroup of 16 waves.  Three launches that each have next to
 // nothing to do become one: the product by itself took 4.5 us, the choice 7.0 and the sort 3.6 (8 tokens, 2,048 wide, 16
 // experts), this kernel 10.5.  Bound by its chain of waits: rows and weights from L2, a sum over the waves through LDS, a
-// token's choices one after the other.
+// token's choices one after the other, in code that the CU has to fetch (for up to 64 experts and pairs: a variant of half the size,
+// SLOTS 1).  Meanwhile the other workgroups of the launch (DENSE) make the hidden rows of a shared feed-forward, which need no
+// router: a workgroup per 16 columns, whose waves share K as in the product here.  Beside the experts' first product they cost 2.8 us
+// (2,048 x 2,048), here nothing.
 //   product   a wave takes 1 / 16 of K for every tile of 16 experts; the waves' sums are added up in their order
 //   choice    wave t is token t's
 //   sort      lane e counts expert e's pairs; an expert's pairs stay in their order
 // logits [T, stride] (32-bit): the first E are the experts', what follows (a shared expert's score) is only written.
 constexpr int kFewTokens = 16, kFewSlots = 2, kFewPairs = 128;
-struct RouterScratch {
-  float logits[kFewTokens][kFewSlots * kWave + 16];
-  float sums[kFewTokens][16 * 17];   // the waves' tiles of 16 experts x 16 tokens
-  float choice[kFewTokens][kFewSlots * kWave], group[kFewTokens][kFewSlots * kWave];
-  int pairs[kFewPairs];
+struct DenseHidden {
+  const bf16* w;   // tiled; gated: the two factors' tiles in turn
+  bf16* out;       // [T, N]
+  int N, gated, act;
+  float limit;
 };
+template <int SLOTS>
+struct RouterScratch {
+  float logits[kFewTokens][SLOTS * kWave + 16];
+  float sums[kFewTokens][16 * 17];   // the waves' tiles of 16 experts x 16 tokens
+  float choice[kFewTokens][SLOTS * kWave], group[kFewTokens][SLOTS * kWave];
+  int pairs[SLOTS * kWave];
+};
+constexpr int kDenseLds = 2 * kFewTokens * 16 * 17 * sizeof(float);   // the waves' sums of two tiles
+template <int SLOTS>
 __global__ __launch_bounds__(1024) void route_few_kernel(const bf16* __restrict__ x, int64_t x_stride, const bf16* __restrict__ w,
                                                          int T, int D, int rows, int E, int top, float scale, int plain,
                                                          RouterOptions options, float* __restrict__ logits,
                                                          int* __restrict__ experts, float* __restrict__ weights,
-                                                         int* __restrict__ sorted, int* __restrict__ plan) {
+                                                         int* __restrict__ sorted, int* __restrict__ plan, DenseHidden dense) {
   extern __shared__ __align__(16) char few_lds[];
-  RouterScratch& l = *reinterpret_cast<RouterScratch*>(few_lds);
+  RouterScratch<SLOTS>& l = *reinterpret_cast<RouterScratch<SLOTS>*>(few_lds);
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int r = lane % 16, kq = lane / 16, chunks = D / 32;
   const int c0 = chunks * wave / 16, c1 = chunks * (wave + 1) / 16;
   const bf16* row = x + static_cast<size_t>(r < T ? r : T - 1) * x_stride + kq * 8;
+  if (blockIdx.x > 0) {   // a tile of the shared feed-forward's hidden columns
+    float (*sums)[kFewTokens][16 * 17] = reinterpret_cast<float (*)[kFewTokens][16 * 17]>(few_lds);
+    const int n0 = (blockIdx.x - 1) * 16;
+    const bf16* g = dense.w + static_cast<size_t>((blockIdx.x - 1) * (dense.gated ? 2 : 1)) * chunks * 512 + lane * 8;
+    const bf16* u = dense.gated ? g + static_cast<size_t>(chunks) * 512 : g;
+    floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    constexpr int kAhead = 4;
+    for (int c = c0; c < c1; c += kAhead) {
+      bf16x8 gv[kAhead], uv[kAhead], xv[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const int at = c + i < c1 ? c + i : c1 - 1;
+        gv[i] = load8(g + static_cast<size_t>(at) * 512);
+        uv[i] = load8(u + static_cast<size_t>(at) * 512);
+        xv[i] = load8(row + at * 32);
+      }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        if (c + i >= c1) break;   // (uniform)
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gv[i], xv[i], acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(uv[i], xv[i], acc[1], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sums[f][wave][(4 * kq + v) * 17 + r] = acc[f][v];   // [column][token]
+    __syncthreads();
+    const int n = tid % 16, t = tid / 16;
+    if (tid >= 256 || t >= T || n0 + n >= dense.N) return;
+    float s[2] = {0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      s[0] += sums[0][k][n * 17 + t];
+      s[1] += sums[1][k][n * 17 + t];
+    }
+    const float first = to_float(float_to_bf16(s[0])), second = to_float(float_to_bf16(s[1]));
+    const float h = dense.gated ? gated_product(dense.act, dense.limit, first, second) : gated_activation(dense.act, first);
+    dense.out[static_cast<size_t>(t) * dense.N + n0 + n] = float_to_bf16(h);
+    return;
+  }
   for (int n0 = 0; n0 < rows; n0 += 16) {
     const bf16* tile = w + static_cast<size_t>(n0 / 16) * chunks * 512 + lane * 8;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -325,8 +378,8 @@ __global__ __launch_bounds__(1024) void route_few_kernel(const bf16* __restrict_
     const int t = wave;
     int* chosen = l.pairs + t * top;
     float* weight = l.sums[wave];   // (the sums have been read)
-    if (plain) choose_plain<kFewSlots>(l.logits[t], E, top, scale, chosen, weight);
-    else choose_with_options<kFewSlots>(l.logits[t], E, top, scale, options, l.choice[wave], l.group[wave], chosen, weight);
+    if (plain) choose_plain<SLOTS>(l.logits[t], E, top, scale, chosen, weight);
+    else choose_with_options<SLOTS>(l.logits[t], E, top, scale, options, l.choice[wave], l.group[wave], chosen, weight);
     wave_ordered();
     for (int k = lane; k < top; k += kWave) {
       experts[t * top + k] = chosen[k];
@@ -338,15 +391,15 @@ __global__ __launch_bounds__(1024) void route_few_kernel(const bf16* __restrict_
   // A lane has pairs lane, lane + 64 and experts lane, lane + 64; every pair's expert passes by all lanes once (a lane read: no
   // chain of LDS reads, no prefix sums).
   const int P = T * top;
-  int mine[kFewSlots], place[kFewSlots] = {}, count[kFewSlots] = {}, below[kFewSlots] = {};
+  int mine[SLOTS], place[SLOTS] = {}, count[SLOTS] = {}, below[SLOTS] = {};
 #pragma unroll
-  for (int i = 0; i < kFewSlots; ++i) mine[i] = lane + i * kWave < P ? l.pairs[lane + i * kWave] : -1;
+  for (int i = 0; i < SLOTS; ++i) mine[i] = lane + i * kWave < P ? l.pairs[lane + i * kWave] : -1;
 #pragma unroll
-  for (int j = 0; j < kFewSlots; ++j)
+  for (int j = 0; j < SLOTS; ++j)
     for (int q = 0; q < kWave && j * kWave + q < P; ++q) {
       const int e = __builtin_amdgcn_readlane(mine[j], q);
 #pragma unroll
-      for (int i = 0; i < kFewSlots; ++i) {
+      for (int i = 0; i < SLOTS; ++i) {
         place[i] += e < mine[i] || (e == mine[i] && j * kWave + q < lane + i * kWave) ? 1 : 0;
         count[i] += e == lane + i * kWave ? 1 : 0;
         below[i] += e < lane + i * kWave ? 1 : 0;
@@ -354,8 +407,8 @@ __global__ __launch_bounds__(1024) void route_few_kernel(const bf16* __restrict_
     }
   int before = 0;   // tiles of the experts before
 #pragma unroll
-  for (int i = 0; i < kFewSlots; ++i) {
-    const int tiles = (count[i] + 15) / 16, most = 1 + (kFewPairs - 1) / 16;
+  for (int i = 0; i < SLOTS; ++i) {
+    const int tiles = (count[i] + 15) / 16, most = 1 + (SLOTS * kWave - 1) / 16;
     int n = before;
     for (int k = 1; k <= most; ++k) {   // (a second tile only where logits that are no numbers gave one expert to a token twice)
       const uint64_t has = __ballot(tiles >= k);
@@ -381,17 +434,15 @@ __global__ __launch_bounds__(1024) void route_few_kernel(const bf16* __restrict_
 // bfloat16: the weights are tiled ([E][N / 16][K / 32][64][8], see the product kernels), a wave's operands are one
 // 16-byte load a lane (rows that are not 16-byte aligned are read element by element); 32-bit: row-major weights
 // [E][N][K], a lane per (row, column) of the tile in turn.
-// SHARED (bfloat16, few tokens): the first tile of the grid is the shared feed-forward's, all tokens' rows against its own
-// weights (gate and factor tile by tile in turn, as the dense gated product has them): two launches of 5 to 7 us less a layer,
-// and its 25 MB ride along with the experts' (8 tokens,
-// feed-forwards of 2,048 x 2,048, 16 experts: 34.7 + 7.1 us before and 37.5 now, down 17.5 + 5.5 and 19.3).
+// SHARED (bfloat16, few tokens, products without a gate): the first tile of the grid is the shared feed-forward's, all tokens' rows
+// against its own weights: a launch less a layer, and its 8 MB ride along with the experts' (8 tokens, feed-forwards of 2,048 x
+// 2,048, 16 experts: 17.5 + 5.5 us before and 19.3 now).
 struct SharedExpert {
   const bf16* a;
   const bf16* w;
   void* out;
   int64_t a_stride, out_stride;
   int N, K, rows;
-  float limit;
 };
 template <typename T, bool GATED, int RT, bool SHARED = false>
 __global__ __launch_bounds__(kWave) void expert_product_kernel(
@@ -408,7 +459,7 @@ __global__ __launch_bounds__(kWave) void expert_product_kernel(
     rows = sh.rows;
     if constexpr (SHARED) {
       a = sh.a, a_stride = sh.a_stride, out = sh.out, out_stride = sh.out_stride;
-      N = sh.N, K = sh.K, limit = sh.limit, out_by_pair = 0;
+      N = sh.N, K = sh.K, out_by_pair = 0;
     }
   } else {
     if (tile >= plan[0]) return;
@@ -432,8 +483,8 @@ __global__ __launch_bounds__(kWave) void expert_product_kernel(
     const bf16* u = GATED ? reinterpret_cast<const bf16*>(w2) + wbase * 512 + lane * 8 : nullptr;
     if constexpr (SHARED) {
       if (shared) {
-        g = sh.w + (GATED ? 2 : 1) * wbase * 512 + lane * 8;
-        u = g + static_cast<size_t>(Kt) * 512;
+        static_assert(!GATED, "the shared rows of gated products are the router's launch's");
+        g = sh.w + wbase * 512 + lane * 8;
       }
     }
     floatx4 accg[RT], accu[RT];
@@ -767,7 +818,8 @@ extern "C" int sa_route_few_takes(const void* x, int64_t x_stride, int T, int D,
 extern "C" int sa_route_few(const void* x, int64_t x_stride, const void* w, int T, int D, int rows, int E, int top, float scale,
                             int plain, const void* bias, int bias_dtype, const void* correction, int corr_dtype, int groups, int keep,
                             int softmax, int group_best, float renorm, float* logits, int* experts, float* weights, int* sorted,
-                            int* plan, int plan_words, hipStream_t stream) {
+                            int* plan, int plan_words, const void* dense_w, int dense_N, int dense_gated, int dense_act, float dense_limit,
+                            void* dense_out, hipStream_t stream) {
   SA_REQUIRE(sa_route_few_takes(x, x_stride, T, D, rows, E, top) && x_stride >= D, "route_few: T=%d D=%d experts=%d top=%d are not taken", T,
              D, E, top);
   SA_REQUIRE(x != nullptr && w != nullptr && logits != nullptr && experts != nullptr && weights != nullptr && sorted != nullptr &&
@@ -779,10 +831,20 @@ extern "C" int sa_route_few(const void* x, int64_t x_stride, const void* w, int 
   SA_REQUIRE((correction == nullptr || corr_dtype == kF32 || corr_dtype == kBF16) &&
                  (bias == nullptr || bias_dtype == kF32 || bias_dtype == kBF16),
              "route_few: unknown dtype");
-  route_few_kernel<<<1, 1024, sizeof(RouterScratch), stream>>>(
-      static_cast<const bf16*>(x), x_stride, static_cast<const bf16*>(w), T, D, rows, E, top, scale, plain,
-      RouterOptions{bias, correction, bias_dtype, corr_dtype, groups, keep, softmax, group_best, renorm}, logits, experts, weights,
-      sorted, plan);
+  SA_REQUIRE(dense_w == nullptr || (dense_out != nullptr && dense_N > 0 && dense_act >= 0 &&
+                                    dense_act < (dense_gated ? kNumGatedRules : kNumActivations) &&
+                                    (dense_act != kActClampedGlu || dense_limit > 0.f)),
+             "route_few: a shared feed-forward of %d columns, activation %d", dense_N, dense_act);
+  const DenseHidden dense{static_cast<const bf16*>(dense_w), static_cast<bf16*>(dense_out), dense_N, dense_gated, dense_act, dense_limit};
+  const int blocks = 1 + (dense_w != nullptr ? (dense_N + 15) / 16 : 0);
+#define SA_ROUTE_FEW(SLOTS)                                                                                                          \
+  route_few_kernel<SLOTS><<<blocks, 1024, sizeof(RouterScratch<SLOTS>) > kDenseLds ? sizeof(RouterScratch<SLOTS>) : kDenseLds, stream>>>( \
+      static_cast<const bf16*>(x), x_stride, static_cast<const bf16*>(w), T, D, rows, E, top, scale, plain,                            \
+      RouterOptions{bias, correction, bias_dtype, corr_dtype, groups, keep, softmax, group_best, renorm}, logits, experts, weights,    \
+      sorted, plan, dense)
+  if (E <= kWave && T * top <= kWave) SA_ROUTE_FEW(1);
+  else SA_ROUTE_FEW(2);
+#undef SA_ROUTE_FEW
   return check_launch("route_few");
 }
 
@@ -876,32 +938,24 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
   return check_launch("expert_product");
 }
 
-extern "C" int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w1, const void* w2, int N,
-                                        int K, const int* sorted, const int* plan, int P, int E, int act, float limit, void* out,
-                                        int64_t out_stride, int out_by_pair, int activate, const void* shared_a,
-                                        int64_t shared_a_stride, const void* shared_w, int shared_N, int shared_K, int T,
-                                        float shared_limit, void* shared_out, int64_t shared_out_stride, hipStream_t stream) {
-  SA_REQUIRE(!activate || w2 == nullptr, "expert_product: a gated product has its activation already");
+extern "C" int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w, int N, int K,
+                                        const int* sorted, const int* plan, int P, int E, void* out, int64_t out_stride, int out_by_pair,
+                                        const void* shared_a, int64_t shared_a_stride, const void* shared_w, int shared_N, int shared_K,
+                                        int T, void* shared_out, int64_t shared_out_stride, hipStream_t stream) {
   SA_REQUIRE(P > 0 && E > 0 && N > 0 && K > 0 && top > 0 && a_stride >= K && out_stride >= N && T > 0 && T <= 16 && P == T * top &&
                  shared_N > 0 && shared_K > 0 && shared_a_stride >= shared_K && shared_out_stride >= shared_N,
              "expert_product_shared: bad sizes P=%d E=%d N=%d K=%d, %d tokens (at most 16), N=%d K=%d", P, E, N, K, T, shared_N, shared_K);
-  SA_REQUIRE(a != nullptr && w1 != nullptr && sorted != nullptr && plan != nullptr && out != nullptr && shared_a != nullptr &&
+  SA_REQUIRE(a != nullptr && w != nullptr && sorted != nullptr && plan != nullptr && out != nullptr && shared_a != nullptr &&
                  shared_w != nullptr && shared_out != nullptr,
              "expert_product_shared: a null pointer");
-  SA_REQUIRE(act >= 0 && act < (w2 != nullptr ? kNumGatedRules : kNumActivations), "expert_product: unknown activation %d", act);
-  SA_REQUIRE(act != kActClampedGlu || (limit > 0.f && shared_limit > 0.f), "expert_product: the clamped gated product needs a positive limit");
   const int tiles = 1 + sa_expert_tiles_max(P, E, 16);   // (at most 1 + 16 + P: far from the grid's end)
   const dim3 grid(((N > shared_N ? N : shared_N) + 15) / 16, tiles);
   const SharedExpert sh{static_cast<const bf16*>(shared_a), static_cast<const bf16*>(shared_w), shared_out, shared_a_stride,
-                        shared_out_stride, shared_N, shared_K, T, shared_limit};
+                        shared_out_stride, shared_N, shared_K, T};
   SA_REQUIRE(tiles <= kGridMax, "expert_product_shared: %d tiles", tiles);
-#define SA_EXPERT_SHARED(G)                                                                                            \
-  expert_product_kernel<bf16, G, 1, true><<<grid, kWave, 0, stream>>>(                                                  \
-      static_cast<const bf16*>(a), a_stride, a_by_token, top, static_cast<const bf16*>(w1), static_cast<const bf16*>(w2), N, K, \
-      sorted, plan, act, limit, out, out_stride, out_by_pair, activate, sh)
-  if (w2 != nullptr) SA_EXPERT_SHARED(true);
-  else SA_EXPERT_SHARED(false);
-#undef SA_EXPERT_SHARED
+  expert_product_kernel<bf16, false, 1, true><<<grid, kWave, 0, stream>>>(
+      static_cast<const bf16*>(a), a_stride, a_by_token, top, static_cast<const bf16*>(w), nullptr, N, K, sorted, plan, 0, 0.f, out,
+      out_stride, out_by_pair, 0, sh);
   return check_launch("expert_product_shared");
 }
 

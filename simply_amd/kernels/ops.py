@@ -2100,10 +2100,11 @@ def route_few_takes(x: torch.Tensor, router, num_experts: int, top: int) -> bool
 
 
 def route_few(x: torch.Tensor, router: TiledWeight, num_experts: int, top: int, scale: float, *,
-              options: dict | None = None) -> tuple:
+              options: dict | None = None, dense: tuple | None = None) -> tuple:
     """The router of a few tokens in one launch: (logits float32 [T, rows of the router], experts, weights, (sorted, plan)) with
     the choice as `route` (options None) or `route_choice(**options)` makes it from the first `num_experts` logits, and the order
-    of the pairs as `routed_experts` takes it."""
+    of the pairs as `routed_experts` takes it.  dense: (weight, activation, limit) of a feed-forward that takes every token
+    (tiled; paired if it is gated); its hidden rows [T, weight.rows] then come as a fifth result."""
     o = options or {}
     correction, bias, softmax = o.get("correction"), o.get("bias"), o.get("softmax", False)
     _dev(x, router.data, correction, bias)
@@ -2122,11 +2123,21 @@ def route_few(x: torch.Tensor, router: TiledWeight, num_experts: int, top: int, 
     weights = torch.empty((T, top), dtype=torch.float32, device=dev)
     sorted_ = torch.empty(T * top, dtype=torch.int32, device=dev)
     plan = torch.empty(1 + 3 * _lib.load().sa_expert_tiles_max(T * top, E, 16), dtype=torch.int32, device=dev)
+    d_args, hidden = (None, 0, 0, 0, 0.0, None), None
+    if dense is not None:
+        first, activation, limit = dense
+        _dev(x, first.data)
+        if not isinstance(first, TiledWeight) or first.cols != D or (activation == ACT_CLAMPED_GLU and not first.paired):
+            raise KernelError("route_few: the feed-forward's weight does not go with the rows")
+        hidden = torch.empty((T, first.rows), dtype=x.dtype, device=dev)
+        d_args = (_ptr(first.data), first.rows, int(first.paired), int(activation), _gate_limit(activation, limit), _ptr(hidden))
     _lib.call("sa_route_few", _ptr(x), x.stride(0), _ptr(router.data), T, D, router.rows, E, int(top), float(scale), int(options is None),
               _ptr(bias), _code(bias) if bias is not None else 0, _ptr(correction), _code(correction) if correction is not None else 0,
               int(o.get("groups", 1)), int(o.get("keep", 1)), 2 if softmax == "chosen" else int(softmax), int(o.get("group_best", 2)),
               -1.0 if renorm is None else float(renorm), _ptr(logits), _ptr(experts), _ptr(weights), _ptr(sorted_), _ptr(plan),
-              plan.numel(), _stream())
+              plan.numel(), *d_args, _stream())
+    if hidden is not None:
+        return logits, experts, weights, (sorted_, plan), hidden
     return logits, experts, weights, (sorted_, plan)
 
 
@@ -2153,9 +2164,8 @@ def expert_sums(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, g
                 shared: torch.Tensor | None = None, shared_gate: torch.Tensor | None = None, out_dtype: torch.dtype | None = None,
                 limit: float | None = None, order: tuple | None = None, dense: tuple | None = None) -> ExpertSums:
     """`routed_experts` with the sum over k left to the caller.
-    order: (sorted, plan) as `route_few` gives them (at most 16 tokens).  dense, with order: (first, down, limit), the tiled weights
-    of a shared feed-forward of the experts' form (first: paired if they are gated), which runs in the experts' kernels; its rows
-    take `shared`'s place, in 32 bits."""
+    order: (sorted, plan) as `route_few` gives them (at most 16 tokens).  dense, with order: (hidden rows, down) of a shared
+    feed-forward, whose product with the tiled weight `down` runs beside the experts'; its rows take `shared`'s place, in 32 bits."""
     _dev(x, experts, weights, gate_w.data if gate_w is not None else None, up_w.data, down_w.data, shared, shared_gate)
     T, D = x.shape
     top, E, F = experts.shape[1], up_w.experts, up_w.rows
@@ -2189,25 +2199,20 @@ def expert_sums(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, g
     h = torch.empty((P, F), dtype=x.dtype, device=dev)
     first, second = (gate_w.data, up_w.data) if gate_w is not None else (up_w.data, None)
     y = torch.empty((P, D), dtype=torch.float32, device=dev)
+    _lib.call("sa_expert_product", _ptr(x), _code(x), xs, 1, top, _ptr(first),
+              _ptr(second), F, D, _ptr(sorted_), _ptr(plan), P, E, tile_rows, int(activation), limit, _ptr(h), F, 0,
+              int(gate_w is None), _stream())
     if dense is not None:
-        d_first, d_down, d_limit = dense
-        S = d_first.rows
-        if order is None or shared is not None or d_first.paired != (gate_w is not None) or d_first.cols != D or d_down.paired \
-                or tuple(d_down.shape) != (D, S):
-            raise KernelError("routed_experts: the shared feed-forward's weights do not go with the experts'")
-        d_limit = _gate_limit(activation, d_limit)
-        _dev(x, d_first.data, d_down.data)
-        hs = torch.empty((T, S), dtype=x.dtype, device=dev)
+        hidden, d_down = dense
+        if order is None or shared is not None or not isinstance(d_down, TiledWeight) or d_down.paired \
+                or tuple(d_down.shape) != (D, hidden.shape[1]) or hidden.shape[0] != T or hidden.dtype != x.dtype:
+            raise KernelError("routed_experts: the shared feed-forward does not go with the experts")
+        _dev(x, hidden, d_down.data)
         shared = torch.empty((T, D), dtype=torch.float32, device=dev)
-        _lib.call("sa_expert_product_shared", _ptr(x), xs, 1, top, _ptr(first), _ptr(second), F, D, _ptr(sorted_), _ptr(plan), P, E,
-                  int(activation), limit, _ptr(h), F, 0, int(gate_w is None), _ptr(x), xs, _ptr(d_first.data), S, D, T, d_limit, _ptr(hs),
-                  S, _stream())
-        _lib.call("sa_expert_product_shared", _ptr(h), F, 0, top, _ptr(down_w.data), None, D, F, _ptr(sorted_), _ptr(plan), P, E, 0, 0.0,
-                  _ptr(y), D, 1, 0, _ptr(hs), S, _ptr(d_down.data), D, S, T, 0.0, _ptr(shared), D, _stream())
+        _lib.call("sa_expert_product_shared", _ptr(h), F, 0, top, _ptr(down_w.data), D, F, _ptr(sorted_), _ptr(plan), P, E, _ptr(y), D, 1,
+                  _ptr(hidden), _rows(hidden, "routed_experts: hidden rows"), _ptr(d_down.data), D, hidden.shape[1], T, _ptr(shared), D,
+                  _stream())
     else:
-        _lib.call("sa_expert_product", _ptr(x), _code(x), xs, 1, top, _ptr(first),
-                  _ptr(second), F, D, _ptr(sorted_), _ptr(plan), P, E, tile_rows, int(activation), limit, _ptr(h), F, 0,
-                  int(gate_w is None), _stream())
         _lib.call("sa_expert_product", _ptr(h), _code(h), F, 0, top, _ptr(down_w.data), None, D, F, _ptr(sorted_), _ptr(plan), P,
                   E, tile_rows, 0, 0.0, _ptr(y), D, 1, 0, _stream())
     if shared is not None and tuple(shared.shape) != (T, D):

@@ -189,12 +189,16 @@ class RoutedExperts(FeedForward):
                                           softmax={"softmax": True, "sigmoid": False}.get(self.router_kind, "chosen"),
                                           group_best=self.group_best, renorm=self.renormalize, bias=self.router_bias_w)
         order = dense = shared = None
-        # a handful of tokens: the router in one kernel, the shared feed-forward beside the experts
+        # a handful of tokens: the router in one kernel, the shared feed-forward beside it and the experts
         if ops.route_few_takes(x, self.router, E, self.top) and ops.few_rows_experts(x.shape[0], self.top, self.gate_w, self.up_w, x):
-            logits, experts, weights, order = ops.route_few(x, self.router, E, self.top, self.router_scale, options=options)
-            if self.shared is not None:
-                dense = (self.shared.gate_up, self.shared.down_proj, self.shared.limit) if self.gated \
-                    else (self.shared.up_proj, self.shared.down_proj, None)
+            args = (x, self.router, E, self.top, self.router_scale)
+            if self.shared is None:
+                logits, experts, weights, order = ops.route_few(*args, options=options)
+            else:
+                first = (self.shared.gate_up, self.activation_code, self.shared.limit) if self.gated \
+                    else (self.shared.up_proj, self.activation_code, None)
+                logits, experts, weights, order, hidden = ops.route_few(*args, options=options, dense=first)
+                dense = (hidden, self.shared.down_proj)
         else:
             logits = ops.gemm(x, self.router, out_dtype=torch.float32)
             if plain:

@@ -114,7 +114,12 @@ def test_few_tokens(T, E, top, D, F, S, gated, options):
     hidden = ops.gemm(x, first, activation=ops.ACT_SILU) if gated else ops.gemm(x, first, activate=ops.ACT_SILU)
     shared = ops.gemm(hidden, pack_tiles(sd), out_dtype=torch.float32)
     kw = dict(shared_gate=logits[:, E:], out_dtype=torch.float32)
-    got = ops.expert_sums(*args, order=order, dense=(first, pack_tiles(sd), None), **kw).materialize()
+    beside = ops.route_few(x, router, E, top, 1.5, options=o, dense=(first, ops.ACT_SILU, None))
+    assert all(torch.equal(a, b) for a, b in zip(beside, (logits, experts, weights)))
+    assert torch.equal(beside[3][0], order[0]) and torch.equal(beside[3][1][:1 + len(tiles)], order[1][:1 + len(tiles)])
+    # (a bfloat16 step where a sum of D products in another order rounds the other way)
+    assert torch.allclose(beside[4].float(), hidden.float(), rtol=2.0 ** -7, atol=2.0 ** -12)
+    got = ops.expert_sums(*args, order=order, dense=(beside[4], pack_tiles(sd)), **kw).materialize()
     want = ops.routed_experts(*args, shared=shared, **kw)
     # (hidden entries of the shared feed-forward may round the other way where their sums are taken in another order)
     assert torch.allclose(got, want, rtol=0, atol=2.0 ** -8 * float(shared.abs().max()))
