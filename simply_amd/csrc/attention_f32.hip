@@ -10,8 +10,8 @@
 // query's position, so a token's result does not depend on how the tokens were cut into steps, on its unit, on what else is
 // in the batch or on which pages hold the keys.  Two ways of running the ranges, with the same arithmetic:
 //
-//   a workgroup per unit, key head and range, partial results to the workspace, a merge kernel: few units (decoding), whose
-//   ranges are all there is to fill the chip with;
+//   a workgroup per unit, key head and chunk, four waves to it, partial results to the workspace, a merge kernel: few units
+//   (decoding), whose chunks are all there is to fill the chip with;
 //   a workgroup per unit and key head that walks through the ranges: prompts, or where the workspace is too small.
 //
 // Keys that some row of the unit does not see get the weight zero.  Where such keys' values are not finite (a zero weight
@@ -21,7 +21,7 @@
 // the generic kernel's at heads of 256 (1.06 to 1.3 times with two chains).
 //
 // Bound by the latency of a wave's chunk (loads of keys, scores, exponentials, values, one after the other) at the measured
-// sizes, 2B heads: 4 requests of 257 to 1,023 keys 27.6 us and 4.7 for the merge, where the generic kernel, a workgroup per
+// sizes, 2B heads: 4 requests of 257 to 1,023 keys 10.4 us and 5.4 for the merge, where the generic kernel, a workgroup per
 // token and key head that walks through all keys on the vector ALU, took 786; a prompt of 509 tokens 45 us for 498.
 #include "api.h"
 #include "attention_common.h"
@@ -85,10 +85,180 @@ struct Running {
   }
 };
 
-// NB: head size / 32.  PARTS: this workgroup's range alone, its partial result to parts
-// [unit * Kh + kh][range of the grid][16][hd + kExtra].
-template <int NB, bool PARTS>
-__global__ __launch_bounds__(256, NB == 8 && !PARTS ? 1 : 2) void attention_f32_kernel(Args a, int unit_begin, float* __restrict__ parts) {
+// Adds a range's chunks up under their common maximum: chunk(w, ..) gives chunk w's maximum, sum and V values of a row.
+template <int V, typename Chunk>
+__device__ __forceinline__ void add_chunks(Chunk chunk, float* top_out, float* sum_out, floatx4 (&po)[V / 4]) {
+  float m[kWaves], l[kWaves], top = -INFINITY, sum = 0.f;
+  floatx4 x[kWaves][V / 4];
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) chunk(w, &m[w], &l[w], x[w]);
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) top = fmaxf(top, m[w]);
+#pragma unroll
+  for (int i = 0; i < V / 4; ++i) po[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const float f = part_weight(m[w], top);
+    sum = fmaf(l[w], f, sum);
+#pragma unroll
+    for (int i = 0; i < V / 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) po[i][e] = fmaf(x[w][i][e], f, po[i][e]);
+  }
+  *top_out = top, *sum_out = sum;
+}
+
+// A workgroup per unit, key head and chunk, its partial result to parts [unit * Kh + kh][chunk of the grid][16][hd + kExtra].  Each of
+// the four waves scores a quarter of the chunk's keys, hands the weights to the others through LDS, and multiplies all of them with
+// a quarter of the values' entries: a wave issues 128 matrix instructions where the chunk has 512 and waits for memory twice, on four
+// times as many CUs as ranges would have.  Every sum is that of attention_f32_kernel, in its order.  NB: head size / 32.
+// 4 requests of 257 to 1,023 keys, 2B heads: 10.4 us and 5.4 for the merge; with a wave a chunk and a workgroup a range 27.6, with four waves a chunk and a
+// workgroup a range 25.5.  Bound by the chain of waits.
+template <int NB>
+__global__ __launch_bounds__(256, 2) void attention_f32_parts_kernel(Args a, int unit_begin, float* __restrict__ parts) {
+  constexpr int HD = NB * 32, NT = HD / 16, MINE = NT / 4, ROW = HD + 4;
+  __shared__ __align__(16) float q_s[16 * ROW];
+  __shared__ __align__(16) floatx4 p_s[4][kWave];
+  __shared__ float m_p[4][16];
+  __shared__ int odd_s;   // pieces with values that are not finite at keys that some row does not see
+  const int tid = threadIdx.x, lane = tid % kWave, part = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int c = lane % 16, g = lane / 16, kh = blockIdx.y;
+  const SeqMeta u = a.units[unit_begin + blockIdx.x];
+  if (u.q_len <= 0) return;
+  int lo, hi;
+  unit_keys(u, a.window, &lo, &hi);
+  const int c0 = lo / kRangeKeys * kRangeKeys + static_cast<int>(blockIdx.z) * kChunkKeys;
+  if (c0 >= hi || c0 + kChunkKeys <= lo) return;
+  const int* table = a.table + static_cast<size_t>(u.slot) * a.table_stride;
+  if (tid == 0) odd_s = 0;
+  const float* kp = nullptr;
+  const float* vp[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {   // (a piece that no row sees stands for the nearest one that is seen)
+    int key = c0 + 16 * s;
+    key = key + 15 < lo ? lo / 16 * 16 : key >= hi ? (hi - 1) / 16 * 16 : key;
+    const size_t page = static_cast<size_t>(table[key / a.page_size]) * a.Kh + kh;
+    const int in_page = key % a.page_size;
+    if (s == part) kp = a.k_pages + (page * a.page_size + in_page) * HD + lane * 8;   // (keys in blocks of 16 x 32, see common.h)
+    vp[s] = a.v_pages + (page * HD + part * MINE * 16 + c) * a.page_size + in_page + 4 * g;
+  }
+  floatx4 k[NB][2], v[4][MINE];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) k[b][e] = *reinterpret_cast<const floatx4*>(kp + b * 512 + e * 4);
+  // the unit's rows of queries (rows that are not there: the first)
+  for (int i = tid; i < 16 * HD / 4; i += 256) {
+    const int row = i / (HD / 4), d = i % (HD / 4) * 4;
+    const bool there = row < u.q_len * a.G;
+    const float* from = a.q + static_cast<size_t>(u.q_start + (there ? row / a.G : 0)) * a.q_stride +
+                        static_cast<size_t>(kh * a.G + (there ? row % a.G : 0)) * HD + d;
+    *reinterpret_cast<floatx4*>(&q_s[row * ROW + d]) = *reinterpret_cast<const floatx4*>(from);
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int t = 0; t < MINE; ++t) v[s][t] = *reinterpret_cast<const floatx4*>(vp[s] + static_cast<size_t>(t) * 16 * a.page_size);
+  const bool live = c < u.q_len * a.G;
+  const int pos = u.pos0 + (live ? c / a.G : 0);
+  const int row_lo = a.window > 0 ? pos - a.window : -1;   // keys behind this one are seen
+  __syncthreads();
+  floatx4 x[NB], p;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {   // (a chain for each 32 entries: a long one rounds at its size with every product)
+    x[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 q[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) q[e] = *reinterpret_cast<const floatx4*>(&q_s[c * ROW + b * 32 + g * 8 + e * 4]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][e / 4][e % 4], q[e / 4][e % 4], x[b], 0, 0, 0);
+  }
+#pragma unroll
+  for (int n = NB / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int b = 0; b < n; ++b) x[b] += x[b + n];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int key = c0 + 16 * part + 4 * g + i;
+    float y = x[0][i] * a.scale;
+    if (a.cap > 0.f) y = a.cap * tanhf(y / a.cap);
+    p[i] = key <= pos && key > row_lo ? y : -INFINITY;
+  }
+  const float mine = max_over_row_lanes(fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3])));
+  if (g == 0) m_p[part][c] = mine;
+  __syncthreads();
+  const float m = fmaxf(fmaxf(m_p[0][c], m_p[1][c]), fmaxf(m_p[2][c], m_p[3][c]));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p[i] = p[i] == -INFINITY ? 0.f : expf(p[i] - m);   // (a row that sees nothing here: all zero)
+  p_s[part][lane] = p;
+  // values of keys that some row does not see
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int key = c0 + 16 * s;
+    // every row of the unit sees the keys from its last row's first key to its first row's position
+    const bool whole = key > u.pos0 + u.q_len - 1 - (a.window > 0 ? a.window : 0x3fffffff) && key + 15 <= u.pos0;
+    if (key >= hi || key + 15 < lo || whole) continue;   // (uniform)
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = key + 4 * g + i;
+      const bool held = at >= lo && at < hi;   // (what lies beyond has not been written, or is another's by now)
+#pragma unroll
+      for (int t = 0; t < MINE; ++t) {
+        v[s][t][i] = held ? v[s][t][i] : 0.f;
+        odd |= !(fabsf(v[s][t][i]) < INFINITY);
+      }
+    }
+    if (__any(odd) && lane == 0) atomicOr(&odd_s, 1 << s);
+  }
+  __syncthreads();
+  float l = 0.f;
+  floatx4 o[MINE];
+#pragma unroll
+  for (int t = 0; t < MINE; ++t) o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int odd = __builtin_amdgcn_readfirstlane(odd_s);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const floatx4 w = p_s[s][lane];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l += w[i];
+    const int key = c0 + 16 * s;
+    if (key >= hi || key + 15 < lo) continue;   // (uniform)
+    if ((odd >> s & 1) == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < MINE; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[s][t][i], w[i], o[t], 0, 0, 0);
+    } else {
+      for (int j = 0; j < 16; ++j) {
+        const bool seen = key + j <= pos && key + j > row_lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (j % 4 != i) continue;
+          const bool of_lane = j / 4 == g;
+#pragma unroll
+          for (int t = 0; t < MINE; ++t) {
+            const floatx4 one = __builtin_amdgcn_mfma_f32_16x16x4f32(of_lane ? v[s][t][i] : 0.f, of_lane ? w[i] : 0.f,
+                                                                     floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[t][e] += seen ? one[e] : 0.f;
+          }
+        }
+      }
+    }
+  }
+  l = sum_over_row_lanes(l);
+  if (!live) return;
+  float* dst = parts + ((static_cast<size_t>(blockIdx.x) * a.Kh + kh) * gridDim.z + blockIdx.z) * (16 * (HD + kExtra)) +
+               static_cast<size_t>(c) * (HD + kExtra);
+#pragma unroll
+  for (int t = 0; t < MINE; ++t) *reinterpret_cast<floatx4*>(dst + (part * MINE + t) * 16 + g * 4) = o[t];
+  if (g == 0 && part == 0) *reinterpret_cast<floatx4*>(dst + HD) = floatx4{m, l, 0.f, 0.f};
+}
+
+// A workgroup per unit and key head that walks through the ranges.  NB: head size / 32.
+template <int NB>
+__global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void attention_f32_kernel(Args a, int unit_begin) {
   constexpr int HD = NB * 32, NT = HD / 16, V = HD / 16, ROW = HD + 4;
   __shared__ __align__(16) float o_s[kWaves][16 * ROW];
   __shared__ float m_s[kWaves][16], l_s[kWaves][16];
@@ -98,9 +268,7 @@ __global__ __launch_bounds__(256, NB == 8 && !PARTS ? 1 : 2) void attention_f32_
   if (u.q_len <= 0) return;
   int lo, hi;
   unit_keys(u, a.window, &lo, &hi);
-  const int r0 = lo / kRangeKeys + (PARTS ? static_cast<int>(blockIdx.z) : 0);
-  const int r1 = PARTS ? r0 + 1 : (hi + kRangeKeys - 1) / kRangeKeys;
-  if (r0 * kRangeKeys >= hi) return;
+  const int r0 = lo / kRangeKeys, r1 = (hi + kRangeKeys - 1) / kRangeKeys;
   const int* table = a.table + static_cast<size_t>(u.slot) * a.table_stride;
 
   // the lane's row of queries: entries 32 b + 8 g .. + 7
@@ -230,66 +398,56 @@ __global__ __launch_bounds__(256, NB == 8 && !PARTS ? 1 : 2) void attention_f32_
       l_s[wave][c] = l;
     }
     __syncthreads();
-    // the range's four chunks, under their common maximum
-    float top = m_s[0][row], sum = 0.f;
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) top = fmaxf(top, m_s[w][row]);
+    float top, sum;
     floatx4 po[V / 4];
+    add_chunks<V>([&](int w, float* cm, float* cl, floatx4 (&x)[V / 4]) __attribute__((always_inline)) {
+      *cm = m_s[w][row], *cl = l_s[w][row];
 #pragma unroll
-    for (int i = 0; i < V / 4; ++i) po[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-      const float f = part_weight(m_s[w][row], top);
-      sum = fmaf(l_s[w][row], f, sum);
-#pragma unroll
-      for (int i = 0; i < V / 4; ++i) {
-        const floatx4 x = *reinterpret_cast<const floatx4*>(&o_s[w][row * ROW + d0 + 4 * i]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) po[i][e] = fmaf(x[e], f, po[i][e]);
-      }
-    }
-    if (PARTS) {
-      float* dst = parts + ((static_cast<size_t>(blockIdx.x) * a.Kh + kh) * gridDim.z + blockIdx.z) * (16 * (HD + kExtra)) +
-                   static_cast<size_t>(row) * (HD + kExtra);
-#pragma unroll
-      for (int i = 0; i < V / 4; ++i) *reinterpret_cast<floatx4*>(dst + d0 + 4 * i) = po[i];
-      if (tid % 16 == 0) *reinterpret_cast<floatx4*>(dst + HD) = floatx4{top, sum, 0.f, 0.f};
-    } else {
-      run.add(top, sum, po);
-    }
+      for (int i = 0; i < V / 4; ++i) x[i] = *reinterpret_cast<const floatx4*>(&o_s[w][row * ROW + d0 + 4 * i]);
+    }, &top, &sum, po);
+    run.add(top, sum, po);
   }
-  if (!PARTS) run.write(a, u, kh, row, HD, d0);
+  run.write(a, u, kh, row, HD, d0);
 }
 
+// A unit's chunks, by ranges: four neighbouring values of a row in a thread, threads for the rows of the longest unit.
 template <int NB>
-__global__ __launch_bounds__(256) void attention_f32_merge_kernel(Args a, int unit_begin, const float* __restrict__ parts, int ranges) {
-  constexpr int HD = NB * 32, V = HD / 16;
+__global__ __launch_bounds__(4 * NB * 32) void attention_f32_merge_kernel(Args a, int unit_begin, const float* __restrict__ parts, int ranges) {
+  constexpr int HD = NB * 32;
   const SeqMeta u = a.units[unit_begin + blockIdx.x];
-  if (u.q_len <= 0) return;
+  const int kh = blockIdx.y, row = threadIdx.x / (HD / 4), d0 = threadIdx.x % (HD / 4) * 4;
+  if (row >= u.q_len * a.G) return;
   int lo, hi;
   unit_keys(u, a.window, &lo, &hi);
-  const int kh = blockIdx.y, tid = threadIdx.x, row = tid / 16, d0 = tid % 16 * V;
-  const int n = (hi + kRangeKeys - 1) / kRangeKeys - lo / kRangeKeys;
-  const float* src = parts + (static_cast<size_t>(blockIdx.x) * a.Kh + kh) * ranges * (16 * (HD + kExtra)) +
+  const int first = lo / kRangeKeys, n = (hi + kRangeKeys - 1) / kRangeKeys - first;
+  const float* src = parts + (static_cast<size_t>(blockIdx.x) * a.Kh + kh) * ranges * kWaves * (16 * (HD + kExtra)) +
                      static_cast<size_t>(row) * (HD + kExtra);
-  Running<V> run;
+  Running<4> run;
   run.clear();
-  for (int z = 0; z < n && z < ranges; ++z, src += 16 * (HD + kExtra)) {
-    floatx4 po[V / 4];
+  for (int z = 0; z < n && z < ranges; ++z) {
+    float top, sum;
+    floatx4 po[1];
+    add_chunks<4>([&](int w, float* cm, float* cl, floatx4 (&x)[1]) __attribute__((always_inline)) {
+      const int c0 = (first + z) * kRangeKeys + w * kChunkKeys;
+      const float* from = src + static_cast<size_t>(z * kWaves + w) * (16 * (HD + kExtra));
+      const bool there = c0 < hi && c0 + kChunkKeys > lo;   // (others have written nothing: what lies there is read and not used)
+      const floatx4 ml = *reinterpret_cast<const floatx4*>(from + HD), y = *reinterpret_cast<const floatx4*>(from + d0);
+      *cm = there ? ml[0] : -INFINITY, *cl = there ? ml[1] : 0.f;
 #pragma unroll
-    for (int i = 0; i < V / 4; ++i) po[i] = *reinterpret_cast<const floatx4*>(src + d0 + 4 * i);
-    run.add(src[HD], src[HD + 1], po);
+      for (int e = 0; e < 4; ++e) x[0][e] = there ? y[e] : 0.f;
+    }, &top, &sum, po);
+    run.add(top, sum, po);
   }
   run.write(a, u, kh, row, HD, d0);
 }
 
 template <int NB>
-static void launch(const Args& a, int unit_begin, int units, int ranges, float* parts, hipStream_t stream) {
+static void launch(const Args& a, int unit_begin, int units, int rows, int ranges, float* parts, hipStream_t stream) {
   if (parts != nullptr) {
-    attention_f32_kernel<NB, true><<<dim3(units, a.Kh, ranges), 256, 0, stream>>>(a, unit_begin, parts);
-    attention_f32_merge_kernel<NB><<<dim3(units, a.Kh), 256, 0, stream>>>(a, unit_begin, parts, ranges);
+    attention_f32_parts_kernel<NB><<<dim3(units, a.Kh, ranges * kWaves), 256, 0, stream>>>(a, unit_begin, parts);
+    attention_f32_merge_kernel<NB><<<dim3(units, a.Kh), rows * NB * 8, 0, stream>>>(a, unit_begin, parts, ranges);
   } else {
-    attention_f32_kernel<NB, false><<<dim3(units, a.Kh), 256, 0, stream>>>(a, unit_begin, nullptr);
+    attention_f32_kernel<NB><<<dim3(units, a.Kh), 256, 0, stream>>>(a, unit_begin);
   }
 }
 
@@ -328,14 +486,14 @@ extern "C" int sa_paged_attention_f32(const float* q, int64_t q_stride, const fl
   const int64_t seen = window > 0 && static_cast<int64_t>(window) + max_q_len - 1 < max_kv_len ? static_cast<int64_t>(window) + max_q_len - 1 : max_kv_len;
   const int ranges = static_cast<int>(seen < max_kv_len ? (seen + f32att::kRangeKeys - 2) / f32att::kRangeKeys + 1
                                                         : (seen + f32att::kRangeKeys - 1) / f32att::kRangeKeys);
-  // A workgroup per range while the units alone do not fill the 256 CUs.
-  const int64_t bytes = static_cast<int64_t>(unit_count) * Kh * ranges * 16 * (hd + f32att::kExtra) * static_cast<int64_t>(sizeof(float));
-  float* parts = ranges > 1 && ranges <= 65535 && static_cast<int64_t>(unit_count) * Kh < 256 && workspace != nullptr &&
+  // A workgroup per chunk while the units alone do not fill the 256 CUs.
+  const int64_t bytes = static_cast<int64_t>(unit_count) * Kh * ranges * f32att::kWaves * 16 * (hd + f32att::kExtra) * static_cast<int64_t>(sizeof(float));
+  float* parts = ranges > 1 && ranges <= 65535 / f32att::kWaves && static_cast<int64_t>(unit_count) * Kh < 256 && workspace != nullptr &&
                          bytes <= workspace_bytes
                      ? static_cast<float*>(workspace)
                      : nullptr;
-  if (hd == 64) f32att::launch<2>(a, unit_begin, unit_count, ranges, parts, stream);
-  else if (hd == 128) f32att::launch<4>(a, unit_begin, unit_count, ranges, parts, stream);
-  else f32att::launch<8>(a, unit_begin, unit_count, ranges, parts, stream);
+  if (hd == 64) f32att::launch<2>(a, unit_begin, unit_count, max_q_len * a.G, ranges, parts, stream);
+  else if (hd == 128) f32att::launch<4>(a, unit_begin, unit_count, max_q_len * a.G, ranges, parts, stream);
+  else f32att::launch<8>(a, unit_begin, unit_count, max_q_len * a.G, ranges, parts, stream);
   return check_launch("paged_attention_f32");
 }
