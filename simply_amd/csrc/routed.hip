@@ -266,7 +266,7 @@ __device__ __forceinline__ bf16x8 load8(const bf16* p) { return *reinterpret_cas
 // The router of a step of at most 16 tokens and 128 experts, from the rows to the plan: logits = x . router^T, every token's
 // choice, and the pairs in the order of their experts, in one workgroup of 16 waves.  Three launches that each have next to
 // nothing to do become one: the product by itself took 4.5 us, the choice 7.0 and the sort 3.6 (8 tokens, 2,048 wide, 16
-// experts), this kernel 10.5.  Bound by its chain of waits: rows and weights from L2, a sum over the waves through LDS, a
+// experts), this kernel 9.6.  Bound by its chain of waits: rows and weights from L2, a sum over the waves through LDS, a
 // token's choices one after the other, in code that the CU has to fetch (for up to 64 experts and pairs: a variant of half the size,
 // SLOTS 1).  Meanwhile the other workgroups of the launch (DENSE) make the hidden rows of a shared feed-forward, which need no
 // router: a workgroup per 16 columns, whose waves share K as in the product here.  Beside the experts' first product they cost 2.8 us
