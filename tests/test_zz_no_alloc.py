@@ -89,6 +89,23 @@ def test_static_scratch_equals_workspace(window):
             assert ((got.float() - plain).abs() <= bound).all(), (num_splits, max_len)
 
 
+@pytest.mark.parametrize("H,Kh,hd,window,lens", [
+    (8, 4, 256, 0, [16, 1]), (8, 4, 256, 0, [128, 33, 65]), (8, 4, 256, 0, [129, 100]), (8, 4, 256, 0, [256]),
+    (6, 2, 128, 0, [64]), (6, 2, 128, 0, [256, 200, 17]), (6, 2, 128, 0, [257, 5]), (4, 4, 64, 0, [250, 256]), (4, 4, 64, 0, [288]),
+    (8, 4, 256, 100, [700, 90]), (8, 4, 256, 120, [700]), (16, 1, 64, 240, [900, 31]), (16, 1, 64, 250, [900])])
+def test_static_scratch_equals_workspace_at_few_keys(H, Kh, hd, window, lens):
+    """Where the number of ranges falls to one (128 keys for heads of 256, 256 for smaller ones, a window that holds no more) and
+    right behind it: both entry points cut alike."""
+    lib = load_library()
+    device = torch.device("cuda:0")
+    workspace = torch.empty(64 << 20, dtype=torch.uint8, device=device)
+    case = make_case(lens, H, Kh, hd, 16, 4, device)
+    for num_splits in (0, -1, 3):
+        want, got = run_both(lib, case, H, Kh, hd, 16, window, max(lens), num_splits, workspace)
+        assert torch.isfinite(want.float()).all() and want.float().abs().max() > 0
+        assert torch.equal(want, got), (num_splits, (want.float() - got.float()).abs().max().item())
+
+
 def test_static_scratch_refuses_what_does_not_fit():
     lib = load_library()
     device = torch.device("cuda:0")
