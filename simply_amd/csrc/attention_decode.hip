@@ -582,12 +582,14 @@ int paged_attention_decode_ranges(int seq_count, int Kh, int window, int max_kv_
   return KS;
 }
 
-// The ranges of a launch of the kernels here, with a workspace or without: as above, but for few keys, unless the caller asks for a
+// The ranges of a launch of the kernels here, with a workspace or without: as above, but up to 128 keys, unless the caller asks for a
 // number, one range and no second kernel.  Microseconds with one range / as cut above, keys in HBM: heads of 256, 64 keys
-// 9.3 / 12.4, 128 11.6 / 13.3, 192 14.3 / 13.5; of 128, 64 7.2 / 11.1, 256 10.4 / 11.7, 512 13.8 / 12.1 (one request, 4 and 16 key
-// heads; 8 requests: 9.9 / 12.7, 12.5 / 14.2, 15.7 / 14.4 and 7.8 / 11.9, 11.8 / 15.4, 14.4 / 17.0).
-static int decode_launch_ranges(int seq_count, int Kh, int hd, int window, int max_kv_len, int num_splits) {
-  if (num_splits <= 0 && decode_max_tiles(window, max_kv_len) <= (hd > 128 ? 5 : 9)) return 1;
+// 9.3 / 12.4, 128 11.6 / 13.3, 192 14.3 / 13.5; of 128, 64 7.2 / 11.1 (one request, 4 and 16 key heads; 8 requests: 9.9 / 12.7,
+// 12.5 / 14.2, 15.7 / 14.4 and 7.8 / 11.9).  Heads of 128 and 64 would gain up to 256 keys (10.4 / 11.7, 8 requests 11.8 / 15.4), but a
+// wave then has two tiles of 32 keys, and with fewer maxima fewer weights are exactly one: errors against 32 bits are 1.004 to 1.012
+// times as large from 160 keys on, and the same up to 128.
+static int decode_launch_ranges(int seq_count, int Kh, int window, int max_kv_len, int num_splits) {
+  if (num_splits <= 0 && decode_max_tiles(window, max_kv_len) <= 5) return 1;
   return paged_attention_decode_ranges(seq_count, Kh, window, max_kv_len, num_splits);
 }
 
@@ -631,7 +633,7 @@ int paged_attention_decode(const void* q, int64_t q_stride, const void* k_pages,
       return check_launch("paged_attention_merge");
     }
   }
-  int KS = decode_launch_ranges(seq_count, Kh, hd, window, max_kv_len, num_splits);
+  int KS = decode_launch_ranges(seq_count, Kh, window, max_kv_len, num_splits);
   const size_t per_split = static_cast<size_t>(units) * 16 * (hd + kRowExtra) * sizeof(float);
   while (KS > 1 && (workspace == nullptr || per_split * KS > workspace_bytes)) --KS;
   // (ranges of more than kMaxRangeSubTiles sub-tiles, which a small workspace or a caller's own num_splits may
@@ -695,7 +697,7 @@ int paged_attention_decode_static(const void* q, int64_t q_stride, const void* k
                                   hipStream_t stream) {
   if (seq_count == 0) return 0;
   // the ranges that the entry point with a workspace chooses when it has room for all of them; here they must fit
-  const int KS = decode_launch_ranges(seq_count, Kh, hd, window, max_kv_len, num_splits);
+  const int KS = decode_launch_ranges(seq_count, Kh, window, max_kv_len, num_splits);
   const size_t need = KS > 1 ? static_cast<size_t>(seq_count) * Kh * KS * 16 * (hd + kRowExtra) * sizeof(float) : 0;
   if (need > kStaticScratchBytes) {
     set_error("paged_attention_decode_static: %d requests x %d key heads x %d key ranges of head size %d need %zu bytes "

@@ -103,3 +103,27 @@ def test_recorded_steps_follow_the_lengths(tmp_path, monkeypatch):
     got, ex = decode(True)
     assert torch.equal(got, want) and torch.isfinite(want).all()
     assert len(ex._graphs) == 2 and {k[-1] for k in ex._graphs} == {(-1, 0), (0, 0)}, list(ex._graphs)
+
+
+@pytest.mark.parametrize("H,K,hd,S,keys", [(8, 4, 256, 4, 128), (32, 16, 128, 1, 128), (32, 16, 128, 1, 160), (32, 16, 128, 8, 256),
+                                           (16, 8, 128, 2, 224), (8, 4, 64, 4, 256)])
+def test_few_keys_errors_no_larger_than_in_ranges(H, K, hd, S, keys):
+    """Relative errors against attention in 32 bits, mean of twelve drawings: with the number of ranges that is chosen no larger than
+    with a range for every 64 keys.  (Drawing by drawing the two share nearly all roundings: the means are alike to 0.0001 where the
+    waves' tiles are, and 0.004 to 0.012 apart where a wave has two tiles; 0.002 lies between.)"""
+    from simply_amd.kernels import ops
+
+    P, means = 16, [0.0, 0.0]
+    per = -(-keys // P)
+    table = torch.arange(S * per, dtype=torch.int32, device="cuda").view(S, per)
+    meta = torch.tensor([[i, i, 1, keys - 1] for i in range(S)], dtype=torch.int32, device="cuda")
+    kw = dict(window=None, soft_cap=50.0, max_kv_len=keys, max_q_len=1)
+    for seed in range(12):
+        g = torch.Generator().manual_seed(100 * keys + seed)
+        k, v = torch.randn(S * per, K, P, hd, generator=g).bfloat16().cuda(), torch.randn(S * per, K, hd, P, generator=g).bfloat16().cuda()
+        q = (torch.randn(S, H * hd, generator=g) * (0.05, 0.1, 0.3)[seed % 3]).bfloat16().cuda()
+        want = ops.paged_attention_f32(q.float(), k.float(), v.float(), table, meta, 0, S, H, out=torch.empty(S, H * hd, device="cuda"), **kw).double()
+        for i, n in enumerate((0, max(1, min(256 // (S * K), (keys + 63) // 64)))):
+            got = ops.paged_attention_decode(q, k, v, table, meta, 0, S, H, num_splits=n, out=torch.empty_like(q), **kw)
+            means[i] += float((got.double() - want).norm() / want.norm()) / 12
+    assert 1e-4 < means[0] <= 1.002 * means[1] < 1e-2, means

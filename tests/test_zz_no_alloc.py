@@ -94,8 +94,8 @@ def test_static_scratch_equals_workspace(window):
     (6, 2, 128, 0, [64]), (6, 2, 128, 0, [256, 200, 17]), (6, 2, 128, 0, [257, 5]), (4, 4, 64, 0, [250, 256]), (4, 4, 64, 0, [288]),
     (8, 4, 256, 100, [700, 90]), (8, 4, 256, 120, [700]), (16, 1, 64, 240, [900, 31]), (16, 1, 64, 250, [900])])
 def test_static_scratch_equals_workspace_at_few_keys(H, Kh, hd, window, lens):
-    """Where the number of ranges falls to one (128 keys for heads of 256, 256 for smaller ones, a window that holds no more) and
-    right behind it: both entry points cut alike."""
+    """Where the number of ranges falls to one (128 keys, a window that holds no more), right behind it and up to 288 keys: both entry
+    points cut alike."""
     lib = load_library()
     device = torch.device("cuda:0")
     workspace = torch.empty(64 << 20, dtype=torch.uint8, device=device)
