@@ -165,6 +165,9 @@ int sa_paged_attention(const void* q, int dtype, int64_t q_stride, const void* k
 // Attention of units (seq_meta's layout; at most 16 rows, heads of a key head times tokens, each) in 32 bits on the matrix
 // cores; sinks (float [H]) may be null.  sa_paged_attention_f32_takes: which sizes.
 int sa_paged_attention_f32_takes(int H, int Kh, int hd, int page_size, int64_t q_stride, const void* q);
+// Partial results of a range of 256 keys that a launch leaves in the workspace: 4 (its chunks), 1, or 0, where a workgroup walks
+// through a unit's ranges.  A host function.
+int sa_paged_attention_f32_parts(int unit_count, int Kh, int hd, int window, int max_kv_len, int max_q_len, int64_t workspace_bytes);
 int sa_paged_attention_f32(const float* q, int64_t q_stride, const float* k_pages, const float* v_pages, const int* block_table,
                            int table_stride, const int* units, int unit_begin, int unit_count, float* out, int64_t out_stride,
                            int H, int Kh, int hd, int page_size, int window, float soft_cap, float scale, const float* sinks,

@@ -8,10 +8,12 @@
 // the products of a sum over k may take k in any order, so step r of the value product takes keys 4 g + r of both operands).
 // A range's four chunks are added up through LDS, ranges one after the other.  The order of every sum is fixed by the
 // query's position, so a token's result does not depend on how the tokens were cut into steps, on its unit, on what else is
-// in the batch or on which pages hold the keys.  Two ways of running the ranges, with the same arithmetic:
+// in the batch or on which pages hold the keys.  Three ways of running the ranges, with the same arithmetic (sa_paged_attention_f32_parts
+// says which, and why):
 //
-//   a workgroup per unit, key head and chunk, four waves to it, partial results to the workspace, a merge kernel: few units
+//   a workgroup per unit, key head and chunk, four waves to it, partial results to the workspace, a merge kernel: few units and ranges
 //   (decoding), whose chunks are all there is to fill the chip with;
+//   a workgroup per unit, key head and range, partial results and a merge likewise: few units with more ranges;
 //   a workgroup per unit and key head that walks through the ranges: prompts, or where the workspace is too small.
 //
 // Keys that some row of the unit does not see get the weight zero.  Where such keys' values are not finite (a zero weight
@@ -112,8 +114,8 @@ __device__ __forceinline__ void add_chunks(Chunk chunk, float* top_out, float* s
 // the four waves scores a quarter of the chunk's keys, hands the weights to the others through LDS, and multiplies all of them with
 // a quarter of the values' entries: a wave issues 128 matrix instructions where the chunk has 512 and waits for memory twice, on four
 // times as many CUs as ranges would have.  Every sum is that of attention_f32_kernel, in its order.  NB: head size / 32.
-// 4 requests of 257 to 1,023 keys, 2B heads: 10.4 us and 5.4 for the merge; with a wave a chunk and a workgroup a range 27.6, with four waves a chunk and a
-// workgroup a range 25.5.  Bound by the chain of waits.
+// 4 requests of 257 to 1,023 keys, 2B heads: 10.4 us and 5.4 for the merge; with a wave a chunk and a workgroup a range 27.6, with four
+// waves a chunk and a workgroup a range 25.5.  Bound by the chain of waits.
 template <int NB>
 __global__ __launch_bounds__(256, 2) void attention_f32_parts_kernel(Args a, int unit_begin, float* __restrict__ parts) {
   constexpr int HD = NB * 32, NT = HD / 16, MINE = NT / 4, ROW = HD + 4;
@@ -256,9 +258,10 @@ __global__ __launch_bounds__(256, 2) void attention_f32_parts_kernel(Args a, int
   if (g == 0 && part == 0) *reinterpret_cast<floatx4*>(dst + HD) = floatx4{m, l, 0.f, 0.f};
 }
 
-// A workgroup per unit and key head that walks through the ranges.  NB: head size / 32.
-template <int NB>
-__global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void attention_f32_kernel(Args a, int unit_begin) {
+// A workgroup per unit and key head that walks through the ranges, a wave a chunk; or (PARTS) one for each range, its partial result
+// to parts [unit * Kh + kh][range of the grid][16][hd + kExtra].  NB: head size / 32.
+template <int NB, bool PARTS>
+__global__ __launch_bounds__(256, NB == 8 && !PARTS ? 1 : 2) void attention_f32_kernel(Args a, int unit_begin, float* __restrict__ parts) {
   constexpr int HD = NB * 32, NT = HD / 16, V = HD / 16, ROW = HD + 4;
   __shared__ __align__(16) float o_s[kWaves][16 * ROW];
   __shared__ float m_s[kWaves][16], l_s[kWaves][16];
@@ -268,7 +271,9 @@ __global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void attention_f32_kernel(Arg
   if (u.q_len <= 0) return;
   int lo, hi;
   unit_keys(u, a.window, &lo, &hi);
-  const int r0 = lo / kRangeKeys, r1 = (hi + kRangeKeys - 1) / kRangeKeys;
+  const int r0 = lo / kRangeKeys + (PARTS ? static_cast<int>(blockIdx.z) : 0);
+  const int r1 = PARTS ? r0 + 1 : (hi + kRangeKeys - 1) / kRangeKeys;
+  if (r0 * kRangeKeys >= hi) return;
   const int* table = a.table + static_cast<size_t>(u.slot) * a.table_stride;
 
   // the lane's row of queries: entries 32 b + 8 g .. + 7
@@ -405,14 +410,46 @@ __global__ __launch_bounds__(256, NB == 8 ? 1 : 2) void attention_f32_kernel(Arg
 #pragma unroll
       for (int i = 0; i < V / 4; ++i) x[i] = *reinterpret_cast<const floatx4*>(&o_s[w][row * ROW + d0 + 4 * i]);
     }, &top, &sum, po);
-    run.add(top, sum, po);
+    if constexpr (PARTS) {
+      float* dst = parts + ((static_cast<size_t>(blockIdx.x) * a.Kh + kh) * gridDim.z + blockIdx.z) * (16 * (HD + kExtra)) +
+                   static_cast<size_t>(row) * (HD + kExtra);
+#pragma unroll
+      for (int i = 0; i < V / 4; ++i) *reinterpret_cast<floatx4*>(dst + d0 + 4 * i) = po[i];
+      if (tid % 16 == 0) *reinterpret_cast<floatx4*>(dst + HD) = floatx4{top, sum, 0.f, 0.f};
+    } else {
+      run.add(top, sum, po);
+    }
+  }
+  if constexpr (!PARTS) run.write(a, u, kh, row, HD, d0);
+}
+
+// A unit's ranges: sixteen threads for a row, with V values each on their way at once (one request of 65,536 keys, 2B heads, 221 us with
+// its attention; 242 with four values a thread, as below).
+template <int NB>
+__global__ __launch_bounds__(256) void attention_f32_merge_kernel(Args a, int unit_begin, const float* __restrict__ parts, int ranges) {
+  constexpr int HD = NB * 32, V = HD / 16;
+  const SeqMeta u = a.units[unit_begin + blockIdx.x];
+  if (u.q_len <= 0) return;
+  int lo, hi;
+  unit_keys(u, a.window, &lo, &hi);
+  const int kh = blockIdx.y, row = threadIdx.x / 16, d0 = threadIdx.x % 16 * V;
+  const int n = (hi + kRangeKeys - 1) / kRangeKeys - lo / kRangeKeys;
+  const float* src = parts + (static_cast<size_t>(blockIdx.x) * a.Kh + kh) * ranges * (16 * (HD + kExtra)) +
+                     static_cast<size_t>(row) * (HD + kExtra);
+  Running<V> run;
+  run.clear();
+  for (int z = 0; z < n && z < ranges; ++z, src += 16 * (HD + kExtra)) {
+    floatx4 po[V / 4];
+#pragma unroll
+    for (int i = 0; i < V / 4; ++i) po[i] = *reinterpret_cast<const floatx4*>(src + d0 + 4 * i);
+    run.add(src[HD], src[HD + 1], po);
   }
   run.write(a, u, kh, row, HD, d0);
 }
 
 // A unit's chunks, by ranges: four neighbouring values of a row in a thread, threads for the rows of the longest unit.
 template <int NB>
-__global__ __launch_bounds__(4 * NB * 32) void attention_f32_merge_kernel(Args a, int unit_begin, const float* __restrict__ parts, int ranges) {
+__global__ __launch_bounds__(4 * NB * 32) void attention_f32_merge_chunks_kernel(Args a, int unit_begin, const float* __restrict__ parts, int ranges) {
   constexpr int HD = NB * 32;
   const SeqMeta u = a.units[unit_begin + blockIdx.x];
   const int kh = blockIdx.y, row = threadIdx.x / (HD / 4), d0 = threadIdx.x % (HD / 4) * 4;
@@ -442,12 +479,15 @@ __global__ __launch_bounds__(4 * NB * 32) void attention_f32_merge_kernel(Args a
 }
 
 template <int NB>
-static void launch(const Args& a, int unit_begin, int units, int rows, int ranges, float* parts, hipStream_t stream) {
-  if (parts != nullptr) {
+static void launch(const Args& a, int unit_begin, int units, int rows, int ranges, int per, float* parts, hipStream_t stream) {
+  if (per == kWaves) {
     attention_f32_parts_kernel<NB><<<dim3(units, a.Kh, ranges * kWaves), 256, 0, stream>>>(a, unit_begin, parts);
-    attention_f32_merge_kernel<NB><<<dim3(units, a.Kh), rows * NB * 8, 0, stream>>>(a, unit_begin, parts, ranges);
+    attention_f32_merge_chunks_kernel<NB><<<dim3(units, a.Kh), rows * NB * 8, 0, stream>>>(a, unit_begin, parts, ranges);
+  } else if (per == 1) {
+    attention_f32_kernel<NB, true><<<dim3(units, a.Kh, ranges), 256, 0, stream>>>(a, unit_begin, parts);
+    attention_f32_merge_kernel<NB><<<dim3(units, a.Kh), 256, 0, stream>>>(a, unit_begin, parts, ranges);
   } else {
-    attention_f32_kernel<NB><<<dim3(units, a.Kh), 256, 0, stream>>>(a, unit_begin);
+    attention_f32_kernel<NB, false><<<dim3(units, a.Kh), 256, 0, stream>>>(a, unit_begin, nullptr);
   }
 }
 
@@ -459,6 +499,26 @@ using namespace sa;
 extern "C" int sa_paged_attention_f32_takes(int H, int Kh, int hd, int page_size, int64_t q_stride, const void* q) {
   return Kh > 0 && Kh <= 65535 && H % Kh == 0 && H / Kh <= 16 && (hd == 64 || hd == 128 || hd == 256) && page_size > 0 &&
          page_size % 16 == 0 && q_stride % 4 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0;
+}
+
+// Ranges that a unit's keys can touch.
+static int f32_ranges(int window, int max_kv_len, int max_q_len) {
+  const int64_t seen = window > 0 && static_cast<int64_t>(window) + max_q_len - 1 < max_kv_len ? static_cast<int64_t>(window) + max_q_len - 1 : max_kv_len;
+  return static_cast<int>(seen < max_kv_len ? (seen + f32att::kRangeKeys - 2) / f32att::kRangeKeys + 1
+                                            : (seen + f32att::kRangeKeys - 1) / f32att::kRangeKeys);
+}
+
+extern "C" int sa_paged_attention_f32_parts(int unit_count, int Kh, int hd, int window, int max_kv_len, int max_q_len, int64_t workspace_bytes) {
+  const int ranges = f32_ranges(window, max_kv_len, max_q_len);
+  const int64_t heads = static_cast<int64_t>(unit_count) * Kh;
+  const int64_t bytes = heads * ranges * 16 * (hd + f32att::kExtra) * static_cast<int64_t>(sizeof(float));   // a part a range
+  // Parts while the units alone do not fill the 256 CUs.
+  if (ranges <= 1 || ranges > 65535 || heads >= 256 || bytes > workspace_bytes) return 0;
+  // A workgroup per chunk while the ranges leave half of the CUs idle: beyond that, four times the parts cost the merge more than four
+  // times the workgroups give.  Chunks / ranges in us, heads of 256, 4 key heads, by (unit, key head, range) triples: 64 (one request of
+  // 4,096 keys) 21 / 30, 128 (one of 8,192) 38.5 / 39.8, (8 of 1,024) 21 / 28, 256 (one of 16,384) 66 / 58, (8 of 2,048) 34 / 34.5,
+  // 512 (one of 32,768) 146 / 104, (16 of 2,048) 55 / 55; 16 key heads of 128: 64 (one of 1,024) 9.4 / 13.6, 256 (one of 4,096) 28 / 25.
+  return heads * ranges <= 128 && bytes * f32att::kWaves <= workspace_bytes ? f32att::kWaves : 1;
 }
 
 extern "C" int sa_paged_attention_f32(const float* q, int64_t q_stride, const float* k_pages, const float* v_pages,
@@ -482,18 +542,11 @@ extern "C" int sa_paged_attention_f32(const float* q, int64_t q_stride, const fl
   a.q = q, a.k_pages = k_pages, a.v_pages = v_pages, a.table = block_table, a.units = reinterpret_cast<const SeqMeta*>(units);
   a.out = out, a.sinks = sinks, a.q_stride = q_stride, a.out_stride = out_stride, a.table_stride = table_stride, a.Kh = Kh;
   a.G = H / Kh, a.page_size = page_size, a.window = window, a.cap = soft_cap, a.scale = scale;
-  // ranges that a unit's keys can touch
-  const int64_t seen = window > 0 && static_cast<int64_t>(window) + max_q_len - 1 < max_kv_len ? static_cast<int64_t>(window) + max_q_len - 1 : max_kv_len;
-  const int ranges = static_cast<int>(seen < max_kv_len ? (seen + f32att::kRangeKeys - 2) / f32att::kRangeKeys + 1
-                                                        : (seen + f32att::kRangeKeys - 1) / f32att::kRangeKeys);
-  // A workgroup per chunk while the units alone do not fill the 256 CUs.
-  const int64_t bytes = static_cast<int64_t>(unit_count) * Kh * ranges * f32att::kWaves * 16 * (hd + f32att::kExtra) * static_cast<int64_t>(sizeof(float));
-  float* parts = ranges > 1 && ranges <= 65535 / f32att::kWaves && static_cast<int64_t>(unit_count) * Kh < 256 && workspace != nullptr &&
-                         bytes <= workspace_bytes
-                     ? static_cast<float*>(workspace)
-                     : nullptr;
-  if (hd == 64) f32att::launch<2>(a, unit_begin, unit_count, max_q_len * a.G, ranges, parts, stream);
-  else if (hd == 128) f32att::launch<4>(a, unit_begin, unit_count, max_q_len * a.G, ranges, parts, stream);
-  else f32att::launch<8>(a, unit_begin, unit_count, max_q_len * a.G, ranges, parts, stream);
+  const int ranges = f32_ranges(window, max_kv_len, max_q_len);
+  const int per = workspace != nullptr ? sa_paged_attention_f32_parts(unit_count, Kh, hd, window, max_kv_len, max_q_len, workspace_bytes) : 0;
+  float* parts = static_cast<float*>(workspace);
+  if (hd == 64) f32att::launch<2>(a, unit_begin, unit_count, max_q_len * a.G, ranges, per, parts, stream);
+  else if (hd == 128) f32att::launch<4>(a, unit_begin, unit_count, max_q_len * a.G, ranges, per, parts, stream);
+  else f32att::launch<8>(a, unit_begin, unit_count, max_q_len * a.G, ranges, per, parts, stream);
   return check_launch("paged_attention_f32");
 }

@@ -41,6 +41,7 @@ _SIGNATURES = {
     "sa_add_rmsnorm_planes": [_P, _I, _P, _I, _F, _I, _P, _P, _I, _F, _I, _P, _I, _I, _I, _P],
     "sa_paged_attention": [_P, _I, _L, _P, _P, _P, _I, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "sa_paged_attention_f32_takes": [_I, _I, _I, _I, _L, _P],
+    "sa_paged_attention_f32_parts": [_I, _I, _I, _I, _I, _I, _L],
     "sa_paged_attention_f32": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _P, _L, _I, _I, _I, _I, _I, _F, _F, _P, _I, _I, _P, _L, _P],
     "sa_paged_attention_decode": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _P, _L, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _L,
                                   _P],

@@ -703,6 +703,14 @@ def attention_f32_takes(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
         _lib.load().sa_paged_attention_f32_takes(int(num_heads), int(Kh), int(hd), int(page_size), q.stride(0), _ptr(q)))
 
 
+def attention_f32_parts(unit_count: int, num_kv_heads: int, head_dim: int, window: int | None, max_kv_len: int, max_q_len: int,
+                        workspace_bytes: int | None = None) -> int:
+    """Partial results of a range of 256 keys that `paged_attention_f32` leaves in the workspace: 4 (a workgroup for each chunk of
+    64 keys), 1 (for each range), or 0: a workgroup walks through a unit's ranges.  A host function."""
+    return _lib.load().sa_paged_attention_f32_parts(int(unit_count), int(num_kv_heads), int(head_dim), int(window or 0), int(max_kv_len),
+                                                    int(max_q_len), WORKSPACE_BYTES if workspace_bytes is None else int(workspace_bytes))
+
+
 def paged_attention_f32(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,
                         units: torch.Tensor, unit_begin: int, unit_count: int, num_heads: int, *, window: int | None,
                         soft_cap: float | None, max_kv_len: int, max_q_len: int, out: torch.Tensor, scale: float = 1.0,

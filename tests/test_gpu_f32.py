@@ -184,6 +184,38 @@ def test_attention(H, Kh, hd, P, window, cap, sink):
     assert torch.equal(one, out)
 
 
+@pytest.mark.parametrize("H,Kh,hd,window,per", [(8, 4, 256, None, 1), (8, 4, 256, 300, 3), (6, 2, 128, None, 5), (16, 1, 64, 700, 1)])
+def test_attention_in_chunks_ranges_and_walks(H, Kh, hd, window, per):
+    """The same units with a workgroup for each chunk, for each range, and one that walks through the ranges (a workspace of nothing):
+    the same bits, within the bound above, and nothing written behind the rows that there are."""
+    from simply_amd.kernels import lib, ops
+    from test_gpu_kernels import paged_setup
+
+    P, lens = 16, [per, 64, 255, 256, 257, 513, 1100]
+    kp, vp, table = paged_setup(torch.float32, len(lens), H, Kh, hd, P, lens, 71)
+    q = draw((per * len(lens), H * hd), 72, 0.5)
+    units = torch.tensor([(s, per * s, per, n - per) for s, n in enumerate(lens)], dtype=torch.int32).cuda()
+    outs = []
+    for parts, count, planned, room in ((4, 1, 1100, None), (1, len(lens), 60000 if window is None else 1100, None), (0, len(lens), 1100, 0)):
+        if parts == 1 and window is not None:   # (a window bounds the ranges: more units then, each several times)
+            count = 1 + 128 // (Kh * 3)
+        assert ops.attention_f32_parts(count, Kh, hd, window, planned, per, room) == parts
+        out = torch.full((len(q) + 1, H * hd), 7.0, device="cuda")
+        more = units.repeat(-(-count // len(lens)) + 1, 1).contiguous()
+        ws = torch.full((64 << 20,), 255, dtype=torch.uint8, device="cuda")   # (undefined numbers)
+        for i in range(0, len(lens), count):
+            lib.call("sa_paged_attention_f32", q.data_ptr(), q.stride(0), kp.data_ptr(), vp.data_ptr(), table.data_ptr(), table.stride(0),
+                     more.data_ptr(), i, count, out.data_ptr(), out.stride(0), H, Kh, hd, P, window or 0, 30.0, 0.7, None, planned, per,
+                     ws.data_ptr(), ws.numel() if room is None else room, torch.cuda.current_stream().cuda_stream)
+        assert (out[-1] == 7).all()
+        outs.append(out[:-1])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    for s, n in enumerate(lens):
+        want = attention_64(q[per * s:per * s + per].reshape(-1, H, hd), kp, vp, table, s, torch.arange(n - per, n, device="cuda"), H, window, 30.0,
+                            0.7, None)
+        assert (outs[0][per * s:per * s + per].double().reshape(want.shape) - want).abs().max() <= 1e-5 * want.abs().max()
+
+
 @pytest.mark.parametrize("H,Kh,hd", [(8, 4, 256), (6, 2, 128), (4, 4, 64)])
 def test_attention_errors_no_larger_than_row_by_row(H, Kh, hd):
     """Root mean square errors against 64 bits over a prompt of 300 tokens behind 200: no larger than those of the kernel that
