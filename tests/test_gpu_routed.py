@@ -129,3 +129,20 @@ def test_few_tokens(T, E, top, D, F, S, gated, options):
     a = ops.residual_add_next_norm(sums, h, scale, eps=1e-5, mult=0.7)
     b = ops.residual_add_next_norm(want, h2, scale, eps=1e-5, mult=0.7, out_dtype=torch.bfloat16)
     assert torch.equal(h, h2) and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,D,E", [(1, 1024, 16), (1, 4096, 16), (3, 992, 16), (16, 1024, 16), (8, 2048, 64), (5, 7168, 16), (16, 96, 16)])
+def test_router_of_few_tokens_errors_no_larger_than_the_product_kernel_s(T, D, E):
+    """Logits against 64 bits, root mean squares over 24 drawings: no larger than those of the product kernel that takes more tokens (a
+    twentieth for the difference of the two sets of roundings)."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+
+    here = there = 0.0
+    for seed in range(24):
+        x, w = draw((T, D), 50 + seed).bfloat16().cuda(), draw((E, D), 90 + seed, D ** -0.5).bfloat16().cuda()
+        tiled, want = pack_tiles(w), x.double() @ w.double().T
+        assert ops.route_few_takes(x, tiled, E, 2)
+        here += float((ops.route_few(x, tiled, E, 2, 1.0)[0].double() - want).square().mean())
+        there += float((ops.gemm(x, tiled, out_dtype=torch.float32).double() - want).square().mean())
+    assert 0 < here <= 1.05 ** 2 * there, (here / there) ** 0.5
