@@ -2149,6 +2149,15 @@ def route_few(x: torch.Tensor, router: TiledWeight, num_experts: int, top: int, 
     return logits, experts, weights, (sorted_, plan)
 
 
+#: The widest shared feed-forward whose products run beside the router and the experts.  Its second product is then a wave per 16
+#: columns that walks all of the hidden entries by itself, while the product kernels cut them over waves.  The whole feed-forward of
+#: 1, 8 and 16 tokens in us, beside / in launches of its own (16 experts, top 2): of 2,048 x 2,048 with 2,048 hidden entries 26 / 36,
+#: 65 / 75, 87 / 105; 4,096 34 / 39, 74 / 83, 82 / 94; 6,144 43 / 44, 82 / 88, 98 / 113; 8,192 54 / 51, 88 / 89, 104 / 109; 16,384
+#: 88 / 73, 124 / 109, 142 / 127; of 1,024 x 1,024 with 5,120 33 / 34, 42 / 45, 49 / 55; 6,144 36 / 36, 46 / 47, 52 / 53; 8,192 42 / 38,
+#: 52 / 48, 59 / 55.
+SHARED_BESIDE_MAX = 5120
+
+
 def few_rows_experts(T: int, top: int, gate_w, up_w, x: torch.Tensor) -> bool:
     """Whether a step of T tokens goes through the experts in tiles of 16 rows."""
     return _lib.load().sa_expert_tile_rows(T * top, up_w.experts, up_w.cols, up_w.rows, _code(x), x.stride(0), _ptr(x)) == 16

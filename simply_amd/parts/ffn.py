@@ -192,8 +192,9 @@ class RoutedExperts(FeedForward):
         # a handful of tokens: the router in one kernel, the shared feed-forward beside it and the experts
         if ops.route_few_takes(x, self.router, E, self.top) and ops.few_rows_experts(x.shape[0], self.top, self.gate_w, self.up_w, x):
             args = (x, self.router, E, self.top, self.router_scale)
-            if self.shared is None:
+            if self.shared is None or self.shared.intermediate_size > ops.SHARED_BESIDE_MAX:
                 logits, experts, weights, order = ops.route_few(*args, options=options)
+                shared = self.shared.forward(x, ctx) if self.shared is not None else None
             else:
                 first = (self.shared.gate_up, self.activation_code, self.shared.limit) if self.gated \
                     else (self.shared.up_proj, self.activation_code, None)

@@ -146,3 +146,26 @@ def test_router_of_few_tokens_errors_no_larger_than_the_product_kernel_s(T, D, E
         here += float((ops.route_few(x, tiled, E, 2, 1.0)[0].double() - want).square().mean())
         there += float((ops.gemm(x, tiled, out_dtype=torch.float32).double() - want).square().mean())
     assert 0 < here <= 1.05 ** 2 * there, (here / there) ** 0.5
+
+
+@pytest.mark.parametrize("shared", [16, 5120, 5136])
+def test_shared_feed_forwards_beside_the_experts_and_apart(shared):
+    """Up to and beyond the widest that runs beside the router and the experts, against 64 bits: half a bfloat16 step of 2^-8 for the
+    hidden entries and for the result, and another for the shared rows where they come by themselves."""
+    from simply_amd.parts.ffn import RoutedExperts
+
+    T, D, E, F = 5, 64, 4, 48
+    part = RoutedExperts(D, E, 2, F, shared_size=shared, shared_gate=False)
+    tensors = {n: draw(s.shape, 200 + i, s.shape[1] ** -0.5).bfloat16().cuda() for i, (n, s) in enumerate(part.param_specs().items())}
+    part.load(tensors)
+    x = draw((T, D), 199).bfloat16().cuda()
+    got = part.forward(x).double()
+    w = {n: t.double() for n, t in tensors.items()}
+    ff = lambda p, up: (torch.nn.functional.silu(x.double() @ w[p + "gate" + up].T) * (x.double() @ w[p + "up" + up].T)) @ w[p + "down" + up].T
+    scores = torch.softmax(x.double() @ w["router"].T, -1)
+    best = scores.topk(2, -1)
+    want = ff("shared.", "_proj")
+    for k in range(2):
+        every = torch.stack([ff(f"e{e}.", "") for e in range(E)])
+        want += best.values[:, k:k + 1] * every[best.indices[:, k], torch.arange(T, device="cuda")]
+    assert float((got - want).norm() / want.norm()) <= 1.5 * 2.0 ** -8
