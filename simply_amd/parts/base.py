@@ -22,6 +22,11 @@ residual sum before it) that has not been computed yet, which `project` folds in
 One that sets `defers_sum` takes `forward(..., defer_sum=True)` and may then return its last product with the
 cuts of K not yet added up (`ops.PartialSums`); a block asks for that only when the norm that receives the result
 says `adds_partial_sums`, and hands the result to that norm's `add_into` before anything else runs.
+
+Results of routed experts may be handed on as `ops.ExpertSums`, the experts' rows not yet weighted and added up.  The methods that know
+of it say so (`knows_expert_sums`): a feed-forward's `forward`, which then takes `defer_experts=True` and may return one; a norm's
+`after_sum`, which then takes one in place of y; and whatever a block arrangement puts between the two.  A block asks for it only where
+all of them do.  What says so is the method, not the class: one that overrides it is not taken to know.
 """
 from __future__ import annotations
 
@@ -29,6 +34,12 @@ import dataclasses
 from typing import Any, Mapping
 
 import torch
+
+
+def knows_expert_sums(method):
+    """Marks a method that takes or returns `ops.ExpertSums` (see above)."""
+    method.knows_expert_sums = True
+    return method
 
 
 @dataclasses.dataclass(frozen=True)

@@ -11,7 +11,7 @@ import torch
 
 from ..kernels import ops
 from ..registry import BLOCKS
-from .base import Block, PendingNorm
+from .base import Block, PendingNorm, knows_expert_sums
 from .norm import NoNorm
 
 #: stands for "no norm follows": the kernel of the last residual sum then hands the stream on in the activation type
@@ -142,6 +142,7 @@ class PreNormBlock(Block):
     def first_norm(self):
         return self.norms["pre_mixer"]
 
+    @knows_expert_sums
     def _add(self, h, y, norm, dtype):
         """h += mult * y; returns norm(h), or None without a norm."""
         if norm is not None and norm.fuses_sum:
@@ -159,7 +160,8 @@ class PreNormBlock(Block):
         if self.feed_forward is None:
             return h, self._add(h, y, next_norm, ctx.dtype)
         normed = self._add(h, y, n["pre_ffn"], ctx.dtype)
-        # (experts' results may be left to the sum in front of the next norm, where both can)
-        both = getattr(self.feed_forward, "defers_experts", False) and next_norm is not None and next_norm.fuses_sum
-        y = self.feed_forward.forward(normed, ctx, **({"defer_experts": True} if both else {}))
+        # (experts' results may be left to the sum in front of the next norm, where all that stands between can)
+        defer = next_norm is not None and next_norm.fuses_sum and all(
+            getattr(method, "knows_expert_sums", False) for method in (self.feed_forward.forward, self._add, next_norm.after_sum))
+        y = self.feed_forward.forward(normed, ctx, **({"defer_experts": True} if defer else {}))
         return h, self._add(h, y, next_norm, ctx.dtype)

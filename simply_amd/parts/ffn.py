@@ -7,7 +7,7 @@ import torch
 
 from ..kernels import ops
 from ..registry import ACTIVATIONS, FEED_FORWARDS
-from .base import FeedForward, ParamSpec, PendingNorm, as_product_weight, project
+from .base import FeedForward, ParamSpec, PendingNorm, as_product_weight, knows_expert_sums, project
 
 # activation name -> its code in the gated product's epilogue (simply/model_lib.py:93-104 registers these three)
 ACTIVATIONS.register("gelu_tanh", ops.ACT_GELU_TANH)
@@ -112,9 +112,6 @@ class RoutedExperts(FeedForward):
       shared_size one more feed-forward of the experts' form runs for every token and is added, times sigmoid(w . x)
                   (one number per token) if `shared_gate`."""
 
-    #: forward() takes defer_experts=True and may then return an `ops.ExpertSums`
-    defers_experts = True
-
     def __init__(self, hidden_size: int, num_experts: int, top: int, expert_size: int, router_scale: float = 1.0,
                  activation: str = "silu", shared_size: int | None = None, shared_gate: bool = True, gated: bool = True,
                  router: str = "softmax", correction: bool = False, num_groups: int = 1, keep_groups: int = 1,
@@ -181,6 +178,7 @@ class RoutedExperts(FeedForward):
         if self.shared is not None:
             self.shared.load({n: tensors["shared." + n] for n in self.shared.param_specs()})
 
+    @knows_expert_sums
     def forward(self, x: torch.Tensor, ctx=None, defer_experts=False) -> "torch.Tensor | ops.ExpertSums":
         E = self.num_experts
         plain = self.router_kind == "softmax" and not self.correction and self.num_groups == 1 and self.renormalize is None \

@@ -7,7 +7,7 @@ import torch
 
 from ..kernels import ops
 from ..registry import NORMS
-from .base import Norm, ParamSpec
+from .base import Norm, ParamSpec, knows_expert_sums
 
 
 @NORMS.register("none")
@@ -51,6 +51,7 @@ class RMSNorm(Norm):
             raise NotImplementedError("rmsnorm: a norm with a factor is applied through add_into only")
         return ops.rmsnorm(x, self.scale, self.eps, self.scale_plus_one, out_dtype)
 
+    @knows_expert_sums
     def after_sum(self, residual, y, mult, out_dtype):
         return ops.residual_add_next_norm(y, residual, self.scale, eps=self.eps, plus_one=self.scale_plus_one, mult=mult,
                                           out_dtype=out_dtype)
@@ -92,6 +93,7 @@ class LayerNorm(Norm):
     def load(self, tensors):
         self.scale, self.bias = tensors["scale"].contiguous(), tensors["bias"].to(tensors["scale"].dtype).contiguous()
 
+    @knows_expert_sums
     def after_sum(self, residual, y, mult, out_dtype):
         return ops.residual_add_next_norm(y, residual, self.scale, bias=self.bias, eps=self.eps, mult=mult,
                                           out_dtype=out_dtype)

@@ -1,9 +1,14 @@
 """Which way a feed-forward of routed experts goes, and what a block hands on from it: the decisions alone, on the CPU."""
+import types
+
 import pytest
 import torch
 
 from simply_amd.kernels import ops
+from simply_amd.parts.base import Mixer, knows_expert_sums
+from simply_amd.parts.block import PreNormBlock
 from simply_amd.parts.ffn import RoutedExperts
+from simply_amd.parts.norm import LayerNorm, RMSNorm
 
 
 class Routed(Exception):
@@ -29,3 +34,64 @@ def test_a_wide_shared_feed_forward_has_launches_of_its_own(few, size, way, gate
     part = RoutedExperts(32, 4, 2, 16, shared_size=size, shared_gate=False, gated=gated)
     with pytest.raises(Routed, match=way):
         part.forward(torch.zeros(2, 32))
+
+
+class Plain(RoutedExperts):
+    """One that overrides forward() as it was before anything was left to the next norm."""
+
+    def __init__(self):
+        super().__init__(32, 4, 2, 16)
+
+    def forward(self, x, ctx):
+        return x + 1
+
+
+class Deferring(RoutedExperts):
+    def __init__(self):
+        super().__init__(32, 4, 2, 16)
+
+    @knows_expert_sums
+    def forward(self, x, ctx, defer_experts=False):
+        return "sums" if defer_experts else x + 1
+
+
+class Adds(RMSNorm):
+    @knows_expert_sums
+    def after_sum(self, residual, y, mult, out_dtype):
+        return y
+
+
+class AddsTensors(RMSNorm):
+    def after_sum(self, residual, y, mult, out_dtype):
+        assert isinstance(y, torch.Tensor)
+        return y
+
+
+class OwnSum(PreNormBlock):
+    def _add(self, h, y, norm, dtype):
+        assert isinstance(y, torch.Tensor)
+        return y
+
+
+class Same(Mixer):
+    def forward(self, x, ctx, cache):
+        return x
+
+
+def run(block, part, norm):
+    norms = {n: norm(32, 1e-6) for n in ("pre_mixer", "pre_ffn")}
+    x = torch.zeros(2, 32)
+    return block(Same(), part, norms).forward(x, types.SimpleNamespace(dtype=torch.float32), None, x, norm(32, 1e-6))[1]
+
+
+def test_experts_sums_are_handed_on_where_all_know_of_them():
+    assert run(PreNormBlock, Deferring(), Adds) == "sums"
+    for block, part, norm in ((PreNormBlock, Plain(), Adds), (PreNormBlock, Deferring(), AddsTensors), (OwnSum, Deferring(), Adds),
+                              (OwnSum, Plain(), AddsTensors)):
+        assert torch.equal(run(block, part, norm), torch.ones(2, 32))
+    patched = Deferring()   # a program's own function in the place of a part's forward
+    patched.forward = lambda x, ctx: x + 1
+    assert torch.equal(run(PreNormBlock, patched, Adds), torch.ones(2, 32))
+    # the parts here do
+    for method in (RoutedExperts.forward, RMSNorm.after_sum, LayerNorm.after_sum, PreNormBlock._add):
+        assert method.knows_expert_sums
