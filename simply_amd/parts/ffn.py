@@ -178,6 +178,12 @@ class RoutedExperts(FeedForward):
         if self.shared is not None:
             self.shared.load({n: tensors["shared." + n] for n in self.shared.param_specs()})
 
+    def _shared_beside(self) -> bool:
+        """Whether a few tokens' products of the shared feed-forward run beside the router and the experts: one of the parts here, not
+        too wide (what stands in its place, or overrides its forward(), is called as ever)."""
+        return getattr(getattr(self.shared, "forward", None), "__func__", None) in (GatedDense.forward, Dense.forward) \
+            and self.shared.intermediate_size <= ops.SHARED_BESIDE_MAX
+
     @knows_expert_sums
     def forward(self, x: torch.Tensor, ctx=None, defer_experts=False) -> "torch.Tensor | ops.ExpertSums":
         E = self.num_experts
@@ -190,12 +196,12 @@ class RoutedExperts(FeedForward):
         # a handful of tokens: the router in one kernel, the shared feed-forward beside it and the experts
         if ops.route_few_takes(x, self.router, E, self.top) and ops.few_rows_experts(x.shape[0], self.top, self.gate_w, self.up_w, x):
             args = (x, self.router, E, self.top, self.router_scale)
-            if self.shared is None or self.shared.intermediate_size > ops.SHARED_BESIDE_MAX:
+            if not self._shared_beside():
                 logits, experts, weights, order = ops.route_few(*args, options=options)
                 shared = self.shared.forward(x, ctx) if self.shared is not None else None
             else:
-                first = (self.shared.gate_up, self.activation_code, self.shared.limit) if self.gated \
-                    else (self.shared.up_proj, self.activation_code, None)
+                first = (self.shared.gate_up, self.shared.activation_code, self.shared.limit) if isinstance(self.shared, GatedDense) \
+                    else (self.shared.up_proj, self.shared.activation_code, None)
                 logits, experts, weights, order, hidden = ops.route_few(*args, options=options, dense=first)
                 dense = (hidden, self.shared.down_proj)
         else:

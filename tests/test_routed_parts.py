@@ -5,9 +5,9 @@ import pytest
 import torch
 
 from simply_amd.kernels import ops
-from simply_amd.parts.base import Mixer, knows_expert_sums
+from simply_amd.parts.base import FeedForward, Mixer, knows_expert_sums
 from simply_amd.parts.block import PreNormBlock
-from simply_amd.parts.ffn import RoutedExperts
+from simply_amd.parts.ffn import GatedDense, RoutedExperts
 from simply_amd.parts.norm import LayerNorm, RMSNorm
 
 
@@ -34,6 +34,26 @@ def test_a_wide_shared_feed_forward_has_launches_of_its_own(few, size, way, gate
     part = RoutedExperts(32, 4, 2, 16, shared_size=size, shared_gate=False, gated=gated)
     with pytest.raises(Routed, match=way):
         part.forward(torch.zeros(2, 32))
+
+
+def test_a_shared_feed_forward_of_another_kind_is_called(few, monkeypatch):
+    """One in the place of the part's own, one whose forward() is overridden, one that a program has patched."""
+
+    class Own(GatedDense):
+        def forward(self, x, ctx=None, defer_sum=False):
+            return super().forward(x, ctx)
+
+    class Other(FeedForward):
+        def forward(self, x, ctx):
+            return x
+
+    patched = GatedDense(32, 16)
+    patched.forward = lambda x, ctx: x
+    for shared in (Own(32, 16), Other(), patched):
+        part = RoutedExperts(32, 4, 2, 16, shared_size=16, shared_gate=False)
+        part.shared = shared
+        with pytest.raises(Routed, match="apart"):
+            part.forward(torch.zeros(2, 32))
 
 
 class Plain(RoutedExperts):
