@@ -30,6 +30,12 @@ struct LatentRows {
   float mult, eps;
 };
 
+// Heads that a workgroup's threads turn at a time, and how many times one after the other; further heads are other workgroups'.
+// (One token, 64 entries turned, us, this kernel / the wave-per-vector kernel in two launches: 16 heads 4.5 / 11.2, 64 7.6 / 11.2,
+// 128 8.2 / 11.3, 512 9.0 / 11.5; one workgroup for all heads took 11.8 at 128 and 38 at 512.)
+constexpr int kHeadsInTurn = 8;
+__host__ __device__ constexpr int query_groups(int rot_dims) { return 1024 / (rot_dims / 8 * kRowsTokens); }
+
 struct Turn {
   float c[4], s[4];
 };
@@ -58,14 +64,15 @@ template <int NP>
 __global__ __launch_bounds__(1024) void latent_rows_kernel(LatentRows a) {
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, t0 = blockIdx.x * kRowsTokens;
   const int unit = a.R + a.dr;
-  if (blockIdx.y == 1) {
-    const int pieces = a.rot_dims / 8, groups = 1024 / (pieces * kRowsTokens);
+  if (blockIdx.y > 0) {
+    const int pieces = a.rot_dims / 8, groups = query_groups(a.rot_dims), first = (blockIdx.y - 1) * groups * kHeadsInTurn;
+    const int end = first + groups * kHeadsInTurn < a.H ? first + groups * kHeadsInTurn : a.H;
     const int piece = tid % pieces, t = t0 + (tid / pieces) % kRowsTokens, group = tid / (pieces * kRowsTokens);
     if (t >= a.T || group >= groups) return;
     const Turn turn = turn_of(static_cast<float>(a.positions[t]), a.freq + piece * 4, a.mult);
     bf16* at = a.q + static_cast<size_t>(t) * a.q_stride + a.R + piece * 8;
 #pragma unroll 2
-    for (int h = group; h < a.H; h += groups) {
+    for (int h = first + group; h < end; h += groups) {
       bf16* p = at + static_cast<size_t>(h) * unit;
       store_eight(p, turned(load_eight(p), turn));
     }
@@ -144,7 +151,7 @@ using namespace sa;
 extern "C" int sa_latent_rows_takes(int H, int R, int dr, int rot_dims, int page_size, int64_t q_stride, int64_t row_stride,
                                     const void* q, const void* rows, const void* weight) {
   const int pieces = rot_dims / 8;
-  return H >= 1 && R >= 8 && R % 8 == 0 && R <= 1024 && dr >= 8 && dr % 8 == 0 && dr <= 8 * kWave && rot_dims >= 8 && rot_dims % 8 == 0 &&
+  return H >= 1 && H <= 65535 && R >= 8 && R % 8 == 0 && R <= 1024 && dr >= 8 && dr % 8 == 0 && dr <= 8 * kWave && rot_dims >= 8 && rot_dims % 8 == 0 &&
          rot_dims <= dr && pieces * kRowsTokens <= 1024 && page_size >= 1 && q_stride % 8 == 0 && row_stride % 8 == 0 &&
          ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(rows) | reinterpret_cast<uintptr_t>(weight)) & 15u) == 0;
 }
@@ -162,7 +169,8 @@ extern "C" int sa_latent_rows(void* q, int64_t q_stride, const void* rows, int64
              "latent_rows: rows too short, or an unknown dtype");
   const LatentRows a{static_cast<bf16*>(q), static_cast<const bf16*>(rows), q_stride, row_stride, positions, freq, weight, slots,
                      static_cast<bf16*>(k_pages), static_cast<bf16*>(v_pages), T, H, R, dr, rot_dims, page_size, w_dtype, mult, eps};
-  const dim3 grid((T + kRowsTokens - 1) / kRowsTokens, 2);
+  const int heads = query_groups(rot_dims) * kHeadsInTurn;
+  const dim3 grid((T + kRowsTokens - 1) / kRowsTokens, 1 + (H + heads - 1) / heads);
   const size_t lds = static_cast<size_t>(kRowsTokens) * R * sizeof(bf16);
   if (R <= 512) latent_rows_kernel<1><<<grid, 1024, lds, stream>>>(a);
   else latent_rows_kernel<2><<<grid, 1024, lds, stream>>>(a);

@@ -69,3 +69,9 @@ def test_latent_rows(slots, H, R, dr, rot, P, weights):
     for a, b in zip(mine, theirs):
         a, b = a.float(), b.float()
         assert ((a - b).abs() <= 2.0 ** -7 * b.abs()).all() and float((a != b).float().mean()) < 0.01
+
+
+@pytest.mark.parametrize("T,H,dr,rot", [(1, 64, 64, 64), (1, 65, 64, 64), (3, 200, 64, 64), (17, 129, 16, 16), (2, 9, 512, 512), (5, 19, 264, 256)])
+def test_latent_rows_of_many_heads(T, H, dr, rot):
+    """Heads that more than one workgroup turns: eight times what its 1,024 threads hold of 16 tokens."""
+    test_latent_rows(list(range(48, 48 + T)), H, 16, dr, rot, 16, torch.bfloat16)
