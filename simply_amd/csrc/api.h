@@ -403,9 +403,9 @@ int sa_experts_add_next_norm_takes(int D, const void* shared, int64_t shared_str
 
 // Queries [T, H (R + dr)] turned in place (the rot_dims entries behind a head's R) and key rows [T, R + dr] = [latent | shared part]
 // written into pages, the latent normed and weighted, the shared part turned: sa_norm_rope_cache_write of the queries and of the
-// keys (one key head, key_values = R) in one launch, bfloat16.  _takes: sizes in multiples of 8, R <= 1024, aligned rows.
+// keys (one key head, key_values = R) in one launch, bfloat16.  _takes: sizes in multiples of 8, R <= 1024, aligned rows and pages.
 int sa_latent_rows_takes(int H, int R, int dr, int rot_dims, int page_size, int64_t q_stride, int64_t row_stride, const void* q,
-                         const void* rows, const void* weight);
+                         const void* rows, const void* weight, const void* k_pages, const void* v_pages);
 int sa_latent_rows(void* q, int64_t q_stride, const void* rows, int64_t row_stride, const int* positions, const float* freq,
                    int rot_dims, float mult, const void* weight, int w_dtype, float eps, const int64_t* slots, void* k_pages,
                    void* v_pages, int T, int H, int R, int dr, int page_size, hipStream_t stream);

@@ -149,18 +149,19 @@ __global__ __launch_bounds__(1024) void latent_rows_kernel(LatentRows a) {
 using namespace sa;
 
 extern "C" int sa_latent_rows_takes(int H, int R, int dr, int rot_dims, int page_size, int64_t q_stride, int64_t row_stride,
-                                    const void* q, const void* rows, const void* weight) {
+                                    const void* q, const void* rows, const void* weight, const void* k_pages, const void* v_pages) {
   const int pieces = rot_dims / 8;
   return H >= 1 && H <= 65535 && R >= 8 && R % 8 == 0 && R <= 1024 && dr >= 8 && dr % 8 == 0 && dr <= 8 * kWave && rot_dims >= 8 && rot_dims % 8 == 0 &&
          rot_dims <= dr && pieces * kRowsTokens <= 1024 && page_size >= 1 && q_stride % 8 == 0 && row_stride % 8 == 0 &&
-         ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(rows) | reinterpret_cast<uintptr_t>(weight)) & 15u) == 0;
+         ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(rows) | reinterpret_cast<uintptr_t>(weight) |
+           reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) & 15u) == 0;
 }
 
 extern "C" int sa_latent_rows(void* q, int64_t q_stride, const void* rows, int64_t row_stride, const int* positions, const float* freq,
                               int rot_dims, float mult, const void* weight, int w_dtype, float eps, const int64_t* slots, void* k_pages,
                               void* v_pages, int T, int H, int R, int dr, int page_size, hipStream_t stream) {
   if (T == 0) return 0;
-  SA_REQUIRE(T > 0 && sa_latent_rows_takes(H, R, dr, rot_dims, page_size, q_stride, row_stride, q, rows, weight),
+  SA_REQUIRE(T > 0 && sa_latent_rows_takes(H, R, dr, rot_dims, page_size, q_stride, row_stride, q, rows, weight, k_pages, v_pages),
              "latent_rows: %d heads, latents of %d, %d shared entries of which %d turn are not taken", H, R, dr, rot_dims);
   SA_REQUIRE(q != nullptr && rows != nullptr && positions != nullptr && freq != nullptr && weight != nullptr && slots != nullptr &&
                  k_pages != nullptr && v_pages != nullptr,

@@ -118,7 +118,7 @@ _SIGNATURES = {
     "sa_concat_rows": [_P, _P, _P, _I, _I, _I, _I, _P],
     "sa_attention_inputs": [_P, _I, _L, _I, _I, _I, _I, _I, _I, _I, _P, _I, _I, _P, _L, _I, _P, _P, _I, _F, _P, _I, _F, _F, _I,
                             _F, _P, _I, _I, _P, _P, _L, _P, _P, _I, _P, _P, _I, _P],
-    "sa_latent_rows_takes": [_I, _I, _I, _I, _I, _L, _L, _P, _P, _P],
+    "sa_latent_rows_takes": [_I, _I, _I, _I, _I, _L, _L, _P, _P, _P, _P, _P],
     "sa_latent_rows": [_P, _L, _P, _L, _P, _P, _I, _F, _P, _I, _F, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "sa_wkv_token_takes": [_I, _I, _L, _I, _I, _I, _L, _P, _P],
     "sa_wkv_token": [_P, _L, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _I, _F, _I, _I, _P, _L, _P, _I, _P, _P],

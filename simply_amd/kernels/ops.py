@@ -1267,11 +1267,11 @@ def norm_rope_cache_write(proj: torch.Tensor, positions: torch.Tensor, freq: tor
 
 
 def latent_rows_takes(q: torch.Tensor, rows: torch.Tensor, weight: torch.Tensor, num_heads: int, latent: int, rot_dims: int,
-                      k_pages: torch.Tensor) -> bool:
+                      k_pages: torch.Tensor, v_pages: torch.Tensor | None = None) -> bool:
     """Whether `latent_rows` takes these sizes (bfloat16, everything in whole aligned pieces of 8 entries)."""
     return q.is_cuda and q.dtype == torch.bfloat16 and q.stride(1) == 1 and rows.stride(1) == 1 and bool(
         _lib.load().sa_latent_rows_takes(int(num_heads), int(latent), rows.shape[1] - int(latent), int(rot_dims), k_pages.shape[2],
-                                         q.stride(0), rows.stride(0), _ptr(q), _ptr(rows), _ptr(weight)))
+                                         q.stride(0), rows.stride(0), _ptr(q), _ptr(rows), _ptr(weight), _ptr(k_pages), _ptr(v_pages)))
 
 
 def latent_rows(q: torch.Tensor, rows: torch.Tensor, positions: torch.Tensor, freq: torch.Tensor, rot_dims: int, num_heads: int,

@@ -124,7 +124,7 @@ class LatentAttention(Mixer):
             q = proj[:, :c_at]
         qa = ops.head_product(q, self.uk_t, in_stride=dk + dr, tail=dr)      # [T, H * (R + dr)]: [W_uk^T q | s]
         rows = proj[:, c_at:c_at + R + dr]
-        if cache.write and rot_dims and ops.latent_rows_takes(qa, rows, self.dkv_norm, H, R, rot_dims, cache.k_pages):
+        if cache.write and rot_dims and ops.latent_rows_takes(qa, rows, self.dkv_norm, H, R, rot_dims, cache.k_pages, cache.v_pages):
             ops.latent_rows(qa, rows, ctx.positions, freq, rot_dims, H, R, self.dkv_norm, self.norm_eps, group.slot_mapping,
                             cache.k_pages, cache.v_pages, rot_mult=mult)
         else:

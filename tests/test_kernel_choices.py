@@ -1,0 +1,38 @@
+"""Which kernel of the library takes a call: its host functions, which need the built library and no GPU."""
+import pytest
+
+from simply_amd.kernels import build
+
+
+@pytest.fixture(scope="module")
+def lib():
+    if build.find_library() is None:
+        pytest.skip("the kernel library has not been built here")
+    from simply_amd.kernels import lib
+    return lib.load()
+
+
+def test_32_bit_attention_of_long_contexts_keeps_its_ranges(lib):
+    """Partial results of a range: its chunks' where there are few, the range's own where those are many or the workspace does not hold
+    the chunks', and none only where the units fill the chip or the workspace does not hold a part for every range."""
+    from simply_amd.kernels import ops
+
+    parts = ops.attention_f32_parts
+    assert parts(4, 4, 256, None, 1023, 1) == 4 and parts(1, 4, 256, None, 8192, 1) == 4 and parts(8, 4, 256, None, 1024, 1) == 4
+    assert parts(1, 4, 256, None, 8193, 1) == 1 and parts(16, 4, 256, None, 2048, 1) == 1 and parts(1, 16, 128, None, 4096, 1) == 1
+    # 4,097 keys and more of 32 requests, planned for 8,192; two of 131,072 (14.6 ms a launch walked, 0.7 in ranges); a long portion
+    assert parts(32, 4, 256, None, 8192, 1) == 1 and parts(2, 4, 256, None, 131072, 1) == 1 and parts(32, 4, 256, None, 16640, 8) == 1
+    # a window bounds them
+    assert parts(4, 4, 256, 1024, 100000, 1) == 4 and parts(16, 4, 256, 1024, 100000, 1) == 1
+    assert parts(64, 4, 256, None, 4096, 1) == 0 and parts(4, 4, 256, None, 256, 1) == 0
+    row = 16 * (256 + 4) * 4
+    assert [parts(2, 4, 256, None, 2048, 1, n * 8 * 8 * row) for n in (0, 1, 3, 4)] == [0, 1, 1, 4]
+    assert parts(2, 4, 256, None, 2048, 1, 8 * 8 * row - 1) == 0
+
+
+@pytest.mark.parametrize("which", ["q", "rows", "weight", "k_pages", "v_pages"])
+def test_latent_rows_look_at_every_buffer_s_alignment(lib, which):
+    """Pieces of 16 bytes are read and written at all five: a view that begins elsewhere goes the way of single entries."""
+    base = dict(q=4096, rows=8192, weight=12288, k_pages=16384, v_pages=20480)
+    takes = lambda **at: lib.sa_latent_rows_takes(16, 512, 64, 64, 16, 16 * 576, 576, *{**base, **at}.values())
+    assert takes() and takes(**{which: base[which] + 16}) and not takes(**{which: base[which] + 2}) and not takes(**{which: base[which] + 8})

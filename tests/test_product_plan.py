@@ -57,19 +57,3 @@ def test_expected_times_grow_with_the_work(ops):
     # what no fast kernel takes (K that is no multiple of 8) is left to the kernel that takes every size
     kernel, us = ops.gemm_plan(4, 100, 100)
     assert kernel == ops.ALGO_GENERIC and all(v < 0 for v in us.values())
-
-
-def test_32_bit_attention_of_long_contexts_keeps_its_ranges(ops):
-    """Partial results of a range: its chunks' where there are few, the range's own where those are many or the workspace does not hold
-    the chunks', and none only where the units fill the chip or the workspace does not hold a part for every range."""
-    parts = ops.attention_f32_parts
-    assert parts(4, 4, 256, None, 1023, 1) == 4 and parts(1, 4, 256, None, 8192, 1) == 4 and parts(8, 4, 256, None, 1024, 1) == 4
-    assert parts(1, 4, 256, None, 8193, 1) == 1 and parts(16, 4, 256, None, 2048, 1) == 1 and parts(1, 16, 128, None, 4096, 1) == 1
-    # 4,097 keys and more of 32 requests, planned for 8,192; two of 131,072 (14.6 ms a launch walked, 0.7 in ranges); a long portion
-    assert parts(32, 4, 256, None, 8192, 1) == 1 and parts(2, 4, 256, None, 131072, 1) == 1 and parts(32, 4, 256, None, 16640, 8) == 1
-    # a window bounds them
-    assert parts(4, 4, 256, 1024, 100000, 1) == 4 and parts(16, 4, 256, 1024, 100000, 1) == 1
-    assert parts(64, 4, 256, None, 4096, 1) == 0 and parts(4, 4, 256, None, 256, 1) == 0
-    row = 16 * (256 + 4) * 4
-    assert [parts(2, 4, 256, None, 2048, 1, n * 8 * 8 * row) for n in (0, 1, 3, 4)] == [0, 1, 1, 4]
-    assert parts(2, 4, 256, None, 2048, 1, 8 * 8 * row - 1) == 0
