@@ -402,9 +402,19 @@ static void launch_routed(const bf16* A, int64_t lda, const bf16* W, const Route
 // waves a CU, or (tile_rows) 128 x 256 with three, one of eight waves, 64 x 64 outputs each: a tile's upper 64 rows, which an expert's
 // last tile often lacks, are the business of four waves of their own, that then leave the matrix units to the others.  Gate and up
 // together with down of 16 experts, in microseconds:
-//   2,048 x 2,048, rows an expert   37: 89 / 100   64: 106 / 100   125: 130 / 126   256: 192 / 179   500: 334 / 269 (64 / 128)
-//   4,096 x 3,584                   64: 300 / 270  125: 391 / 367  256: 620 / 534
-//   1,024 x 1,024                   256: 65 / 72   500: 98 / 108
+//   2,048 x 2,048, rows an expert   37: 89 / 100   64: 105 / 95    96: 106 / 99    128: 127 / 120   256: 186 / 173   400: 254 / 206 (64 / 128)
+//   4,096 x 3,584                   64: 304 / 275  96: 339 / 283   136: 431 / 437  256: 600 / 534   400: 907 / 711
+//   3,072 x 2,048                   68: 149 / 130  96: 157 / 137   136: 199 / 207  256: 275 / 248   512: 492 / 388
+//   2,048 x 3,072                   68: 143 / 147  96: 151 / 154   136: 192 / 185  256: 274 / 243   512: 477 / 392
+//   2,560 x 2,560                   68: 168 / 159  96: 187 / 168   136: 223 / 243  256: 298 / 287   512: 508 / 436
+//   3,072 x 1,536                   68: 110 / 101  136: 157 / 187  272: 226 / 251  336: 263 / 253   512: 362 / 317
+//   1,024 x 4,096                   60: 94 / 116   96: 110 / 128   136: 145 / 149  208: 172 / 167   336: 239 / 214
+//   4,096 x 1,024                   60: 111 / 106  96: 109 / 115   136: 138 / 146  240: 188 / 195   336: 237 / 199
+//   1,024 x 8,192                   60: 180 / 235  128: 265 / 271  192: 318 / 298  256: 413 / 354
+//   2,048 x 1,536                   60: 79 / 79    128: 99 / 106   256: 146 / 152  400: 200 / 170
+//   1,792 x 1,792                   60: 73 / 78    128: 129 / 115  256: 178 / 178  400: 232 / 242
+//   1,536 x 1,536                   60: 59 / 63    128: 83 / 88    256: 122 / 115  400: 159 / 162
+//   1,024 x 1,024                   60: 37 / 43    128: 48 / 48    256: 67 / 68    400: 88 / 73
 // (128 x 192 of four waves, two a CU, which the 128 rows were before: 209 at 256 rows of 2,048 x 2,048, 626 of 4,096 x 3,584.)  Also
 // tried for 64 rows: eight waves with six buffers, 64 x 256, four waves across; for 128: 128 x 128 (191 and 546), waves of 128 x 64 and
 // 64 x 128 (237 and 233).

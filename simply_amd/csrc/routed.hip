@@ -11,6 +11,8 @@
 // kernels is sized for the most tiles that the pairs can make.  Every pair's row is computed by itself, with sums
 // in an order that depends on the sizes alone, so a token's result does not depend on the batch.  Scores are
 // 32-bit; the products are bfloat16 on the matrix cores (32-bit accumulation) or 32-bit on the vector unit.
+#include <climits>
+
 #include "api.h"
 #include "common.h"
 
@@ -867,12 +869,13 @@ extern "C" int sa_expert_tile_rows(int P, int E, int D, int F, int dtype, int64_
   // 2,048, 16 experts: 8 rows 63 us with tiles of 16 and 72 with the wide kernel's 64; 16 rows 105 and 72); the kernel of 64
   // rows here is ahead from 32 on.
   if (P < (wide ? 12 : 32) * static_cast<int64_t>(E)) return 16;
-  // Tiles of 128 rows where an expert has more than 64 on average or nearly, and its gate and up are 16 MiB, more than an XCD's L2
-  // holds, so that every tile of rows fetches them again (figures: gemm_wide_routed).
-  return wide && P >= 60 * static_cast<int64_t>(E) && 4.0 * D * F >= 16.0 * (1 << 20) &&
-                 sa_expert_tiles_max(P, E, kTileRowsWide) <= kGridMax
-             ? kTileRowsWide
-             : kTileRowsMax;
+  // Tiles of 128 x 256, one a CU, instead of 64 x 128, two a CU, halve what a CU fetches; what they cost is rounds: half as many
+  // columns of tiles, and a last round that may be nearly empty.  With 2,048 columns or more in both products they are ahead from
+  // nearly 64 rows an expert on; with fewer in one of them that product does not fill the CUs until there are many tiles of rows, and
+  // only an expert so large that its products are long makes up for it (figures: gemm_wide_routed).
+  const double mib = 4.0 * D * F / (1 << 20);   // of gate and up
+  const int from = D >= 2048 && F >= 2048 ? 60 : mib >= 32 ? 128 : mib >= 16 ? 320 : INT_MAX;
+  return wide && P >= from * static_cast<int64_t>(E) && sa_expert_tiles_max(P, E, kTileRowsWide) <= kGridMax ? kTileRowsWide : kTileRowsMax;
 }
 
 extern "C" int sa_expert_sort(const int* experts, int P, int E, int tile_rows, int* sorted, int* plan, int plan_words,

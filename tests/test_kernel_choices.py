@@ -36,3 +36,12 @@ def test_latent_rows_look_at_every_buffer_s_alignment(lib, which):
     base = dict(q=4096, rows=8192, weight=12288, k_pages=16384, v_pages=20480)
     takes = lambda **at: lib.sa_latent_rows_takes(16, 512, 64, 64, 16, 16 * 576, 576, *{**base, **at}.values())
     assert takes() and takes(**{which: base[which] + 16}) and not takes(**{which: base[which] + 2}) and not takes(**{which: base[which] + 8})
+
+
+@pytest.mark.parametrize("D,F,per,rows", [
+    (2048, 2048, 11, 16), (2048, 2048, 59, 64), (2048, 2048, 60, 128), (4096, 3584, 64, 128), (3072, 2048, 96, 128),
+    # one product of fewer columns than fill the CUs: 64 rows were ahead by up to a third (1,024 x 8,192: 180 us for 235)
+    (1024, 4096, 60, 64), (1024, 4096, 128, 64), (4096, 1024, 96, 64), (3072, 1536, 136, 64), (3072, 1536, 272, 64), (1024, 8192, 60, 64),
+    (1024, 4096, 336, 128), (3072, 1536, 336, 128), (1024, 8192, 192, 128), (1024, 1024, 400, 64), (2048, 1536, 256, 64)])
+def test_rows_of_a_tile_of_routed_experts(lib, D, F, per, rows):
+    assert lib.sa_expert_tile_rows(16 * per, 16, D, F, 1, D, 4096) == rows
