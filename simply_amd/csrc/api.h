@@ -638,12 +638,12 @@ int sa_route_few(const void* x, int64_t x_stride, const void* w, int T, int D, i
                  const void* bias, int bias_dtype, const void* correction, int corr_dtype, int groups, int keep, int softmax,
                  int group_best, float renorm, float* logits, int* experts, float* weights, int* sorted, int* plan, int plan_words,
                  const void* dense_w, int dense_N, int dense_gated, int dense_act, float dense_limit, void* dense_out, hipStream_t stream);
-// sa_expert_product in bfloat16 with tiles of 16 rows and one weight, and beside it all T <= 16 tokens' product with a dense one:
-// shared_out[t] = shared_a[t] . shared_w^T, 32-bit.
-int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w, int N, int K, const int* sorted,
-                             const int* plan, int P, int E, void* out, int64_t out_stride, int out_by_pair, const void* shared_a,
-                             int64_t shared_a_stride, const void* shared_w, int shared_N, int shared_K, int T, void* shared_out,
-                             int64_t shared_out_stride, hipStream_t stream);
+// The experts' second product as sa_expert_product makes it in bfloat16 with tiles of 16 rows, y[pair] = h[row] . w[e]^T (32-bit),
+// and beside it all T <= 16 tokens' product with a dense weight: shared_y[t] = shared_h[t] . shared_w^T, 32-bit.
+int sa_expert_product_shared(const void* h, int64_t h_stride, int top, const void* w, int N, int K, const int* sorted,
+                             const int* plan, int P, int E, void* y, int64_t y_stride, const void* shared_h,
+                             int64_t shared_h_stride, const void* shared_w, int shared_N, int shared_K, int T, void* shared_y,
+                             int64_t shared_y_stride, hipStream_t stream);
 // out[t] = sum_k weights[t, k] y[t * top + k] + sigmoid(gate[t]) * shared[t]  (shared null: none; gate null: 1).
 int sa_expert_combine(const float* y, const float* weights, int top, const void* shared, int shared_dtype,
                       int64_t shared_stride, const float* gate, int64_t gate_stride, void* out, int out_dtype,

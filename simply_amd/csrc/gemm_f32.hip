@@ -174,9 +174,10 @@ __global__ __launch_bounds__(64 * kSegments) void gemm_f32_few_kernel(Args a) {
   if (n0 + 4 * g < a.N) store4(a, c, n0 + 4 * g, y);
 }
 
-// K that is no multiple of 16 (or rows longer than 16 MB).  TM: blocks of 16 rows and of 16 weight rows of a wave; four waves, two by two.  With the gated epilogue half of a wave's
-// weight rows are the gate's and half the other factor's of the same outputs.  PLANES: this workgroup's segment alone, its
-// sums to planes [segment][M][columns] (gated: all the gate's columns, then the other factor's).
+// Tiles for K that is no multiple of 16 (or rows longer than 16 MB).  TM: blocks of 16 rows and of 16 weight rows of a wave; four
+// waves, two by two.  With the gated epilogue half of a wave's weight rows are the gate's and half the other factor's of the same
+// outputs.  PLANES: this workgroup's segment alone, its sums to planes [segment][M][columns] (gated: all the gate's columns, then
+// the other factor's).
 template <int EPI, int TM, bool PLANES>
 __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(Args a, float* __restrict__ planes) {
   constexpr int ROWS = 2 * TM * 16;                 // rows of A, and rows of W, of a tile

@@ -947,24 +947,23 @@ extern "C" int sa_expert_product(const void* a, int dtype, int64_t a_stride, int
   return check_launch("expert_product");
 }
 
-extern "C" int sa_expert_product_shared(const void* a, int64_t a_stride, int a_by_token, int top, const void* w, int N, int K,
-                                        const int* sorted, const int* plan, int P, int E, void* out, int64_t out_stride, int out_by_pair,
-                                        const void* shared_a, int64_t shared_a_stride, const void* shared_w, int shared_N, int shared_K,
-                                        int T, void* shared_out, int64_t shared_out_stride, hipStream_t stream) {
-  SA_REQUIRE(P > 0 && E > 0 && N > 0 && K > 0 && top > 0 && a_stride >= K && out_stride >= N && T > 0 && T <= 16 && P == T * top &&
-                 shared_N > 0 && shared_K > 0 && shared_a_stride >= shared_K && shared_out_stride >= shared_N,
+extern "C" int sa_expert_product_shared(const void* h, int64_t h_stride, int top, const void* w, int N, int K, const int* sorted,
+                                        const int* plan, int P, int E, void* y, int64_t y_stride, const void* shared_h,
+                                        int64_t shared_h_stride, const void* shared_w, int shared_N, int shared_K, int T, void* shared_y,
+                                        int64_t shared_y_stride, hipStream_t stream) {
+  SA_REQUIRE(P > 0 && E > 0 && N > 0 && K > 0 && top > 0 && h_stride >= K && y_stride >= N && T > 0 && T <= 16 && P == T * top &&
+                 shared_N > 0 && shared_K > 0 && shared_h_stride >= shared_K && shared_y_stride >= shared_N,
              "expert_product_shared: bad sizes P=%d E=%d N=%d K=%d, %d tokens (at most 16), N=%d K=%d", P, E, N, K, T, shared_N, shared_K);
-  SA_REQUIRE(a != nullptr && w != nullptr && sorted != nullptr && plan != nullptr && out != nullptr && shared_a != nullptr &&
-                 shared_w != nullptr && shared_out != nullptr,
+  SA_REQUIRE(h != nullptr && w != nullptr && sorted != nullptr && plan != nullptr && y != nullptr && shared_h != nullptr &&
+                 shared_w != nullptr && shared_y != nullptr,
              "expert_product_shared: a null pointer");
-  const int tiles = 1 + sa_expert_tiles_max(P, E, 16);   // (at most 1 + 16 + P: far from the grid's end)
-  const dim3 grid(((N > shared_N ? N : shared_N) + 15) / 16, tiles);
-  const SharedExpert sh{static_cast<const bf16*>(shared_a), static_cast<const bf16*>(shared_w), shared_out, shared_a_stride,
-                        shared_out_stride, shared_N, shared_K, T};
+  const int tiles = 1 + sa_expert_tiles_max(P, E, 16);   // (1 + ceil(P / 16) + min(E, P): as many experts as asked for)
   SA_REQUIRE(tiles <= kGridMax, "expert_product_shared: %d tiles", tiles);
+  const dim3 grid(((N > shared_N ? N : shared_N) + 15) / 16, tiles);
+  const SharedExpert sh{static_cast<const bf16*>(shared_h), static_cast<const bf16*>(shared_w), shared_y, shared_h_stride,
+                        shared_y_stride, shared_N, shared_K, T};
   expert_product_kernel<bf16, false, 1, true><<<grid, kWave, 0, stream>>>(
-      static_cast<const bf16*>(a), a_stride, a_by_token, top, static_cast<const bf16*>(w), nullptr, N, K, sorted, plan, 0, 0.f, out,
-      out_stride, out_by_pair, 0, sh);
+      static_cast<const bf16*>(h), h_stride, 0, top, static_cast<const bf16*>(w), nullptr, N, K, sorted, plan, 0, 0.f, y, y_stride, 1, 0, sh);
   return check_launch("expert_product_shared");
 }
 

@@ -2226,7 +2226,7 @@ def expert_sums(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, g
             raise KernelError("routed_experts: the shared feed-forward does not go with the experts")
         _dev(x, hidden, d_down.data)
         shared = torch.empty((T, D), dtype=torch.float32, device=dev)
-        _lib.call("sa_expert_product_shared", _ptr(h), F, 0, top, _ptr(down_w.data), D, F, _ptr(sorted_), _ptr(plan), P, E, _ptr(y), D, 1,
+        _lib.call("sa_expert_product_shared", _ptr(h), F, top, _ptr(down_w.data), D, F, _ptr(sorted_), _ptr(plan), P, E, _ptr(y), D,
                   _ptr(hidden), _rows(hidden, "routed_experts: hidden rows"), _ptr(d_down.data), D, hidden.shape[1], T, _ptr(shared), D,
                   _stream())
     else:
