@@ -351,3 +351,64 @@ def test_outputs_behind_the_walk(H, dk, dv, T, bad):
     for u in (None, bonus):
         both(lambda s, k, out: ops.linear_chunks(of(p, k), 0, H * dk, 2 * H * dk, 1.0, of(decay, k), H, dk, dv, s, meta, k, 0, T, bonus=u,
                                                  out=of(out, k)), H * dv)
+
+
+@pytest.mark.parametrize("H,G,dk,dv,counts", [(2, 1, 128, 128, [1, 65, 900, 0]), (3, 3, 40, 24, [768, 63, 0, 1030]), (1, 1, 64, 130, [832, 64, 800])])
+def test_outputs_behind_the_walk_of_several_requests(H, G, dk, dv, counts):
+    """Short, long and empty requests in slots of any order behind rows of others, few enough that the states are kept: among empty
+    requests, so many that they are not, with a workspace just too small for the states, and with one just large enough: the same
+    bits, and nothing written elsewhere.  The definition in 64 bits beside them, bounds as above."""
+    from simply_amd.kernels import lib as _lib, ops
+
+    before, S = 3, len(counts)
+    lib, T, ptr, stream = _lib.load(), 3 + sum(counts), ops._ptr, ops._stream
+    meta = [(3 * i % S if S % 3 else S - 1 - i, before + sum(counts[:i]), n, 0) for i, n in enumerate(counts)]
+    assert sorted(m[0] for m in meta) == list(range(S))
+    blocks, nt = -(-dv // 16), 4 if dk <= 64 else 8
+    many = 128 // (H * blocks) + 1
+    every = meta + [(S, T, 0, 0)] * many
+    dev = torch.tensor(every, dtype=torch.int32).cuda()
+    state = normal((S + 1, H * dk * dv), 141)
+    pieces = sum(counts) // 64 + S
+
+    def check(takes, launch, plain, exact):
+        least = cut_rows(lambda b: takes(5, b), 1)   # a piece without its state
+        kept = least + H * blocks * nt * 1024
+        got = []
+        for n, size in ((S, 256 << 20), (len(every), 256 << 20), (S, pieces * kept), (S, (pieces + 1) * kept)):
+            s, out = state.cuda(), torch.full((T + 1, H * dv), 7.0, device="cuda")
+            ws = torch.full((size,), 255, dtype=torch.uint8, device="cuda")
+            launch(s, n, out, ws)
+            assert (out[:before] == 7).all() and (out[T:] == 7).all() and torch.equal(s[S].cpu(), state[S])
+            got.append((out[before:T], s))
+        for out, s in got[1:]:
+            assert torch.equal(out, got[0][0]) and torch.equal(s, got[0][1])
+        s1 = state.cuda()
+        one = plain(s1)
+        want, want_state = exact()
+        for a, b, ref in ((got[0][0], one[before:], want[before:]), (got[0][1], s1, want_state)):
+            err, base, top = ((x.double().cpu() - ref).abs().max() for x in (a, b, torch.zeros_like(a)))
+            assert err <= 3 * base and err <= 1e-5 * top, (float(err), float(base), float(top))
+
+    C = 2 * G * dk + H * dv
+    C += -C % 4
+    qkv = normal((T, C), 142)
+    heads = qkv[:, :2 * G * dk].reshape(T, 2 * G, dk)
+    qkv[:, :2 * G * dk] = (heads / heads.square().sum(-1, keepdim=True).sqrt()).reshape(T, -1)
+    gates = torch.cat([uniform((T, H), 143), uniform((T, H), 144, 0.9, 1.0)], 1)
+    x, g = qkv.cuda(), gates.cuda()
+    check(lambda n, b: lib.sa_delta_chunks_takes(C, G, H, dk, dv, state.stride(0), n, b),
+          lambda s, n, out, ws: _lib.call("sa_delta_chunks", ptr(x), C, G, dk, dv, ptr(g), H, ptr(s), s.stride(0), ptr(dev), n, before,
+                                          T - before, max(counts), ptr(out), ptr(ws), ws.numel(), stream()),
+          lambda s: ops.delta_rule(x, g, s, dev, S, H, G, dk, dv), lambda: delta_64(qkv, gates, state, meta, H, G, dk, dv))
+
+    at = (0, H * dk, 2 * H * dk)
+    proj, decay, bonus = normal((T, 2 * H * dk + H * dv), 145).bfloat16(), uniform((T, H * dk), 146, 0.5, 1.0), normal((H * dk,), 147)
+    proj = torch.cat([proj, torch.zeros(T, -proj.shape[1] % 4, dtype=proj.dtype)], 1)
+    p, d, u = proj.cuda(), decay.cuda(), bonus.cuda()
+    check(lambda n, b: lib.sa_linear_chunks_takes(H, dk, dv, at[0], at[1], p.stride(0), d.stride(0), state.stride(0), n, b),
+          lambda s, n, out, ws: _lib.call("sa_linear_chunks", ptr(p), p.stride(0), *at, 1.0, ptr(d), d.stride(0), 0, 0, 0.0, ptr(u), 0, H, dk,
+                                          dv, ptr(s), s.stride(0), ptr(dev), n, before, T - before, max(counts), ptr(out), ptr(ws), ws.numel(),
+                                          stream()),
+          lambda s: ops.linear_state(p, *at, 1.0, d, False, H, dk, dv, False, s, dev, S, bonus=u),
+          lambda: linear_64(proj, at, 1.0, decay, bonus, state, meta, H, dk, dv))
