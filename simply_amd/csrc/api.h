@@ -633,7 +633,9 @@ int sa_expert_product(const void* a, int dtype, int64_t a_stride, int a_by_token
 // sa_route (plain) or sa_route_choice make it from the first E logits of a token, sorted and plan as sa_expert_sort with tiles
 // of 16 rows; and, with dense_w (tiled, gated: the two factors' tiles in turn), dense_out [T, dense_N] bfloat16 = rule(x . dense_w^T).
 // _takes: at most 16 tokens, 128 experts (and up to 16 more rows) and 128 pairs, weights of up to 128 K entries.
+// _pays: whether it is expected to be faster than sa_gemm, sa_route(_choice) and sa_expert_sort (host functions, both).
 int sa_route_few_takes(const void* x, int64_t x_stride, int T, int D, int rows, int E, int top);
+int sa_route_few_pays(int T, int D, int rows, int E, int top);
 int sa_route_few(const void* x, int64_t x_stride, const void* w, int T, int D, int rows, int E, int top, float scale, int plain,
                  const void* bias, int bias_dtype, const void* correction, int corr_dtype, int groups, int keep, int softmax,
                  int group_best, float renorm, float* logits, int* experts, float* weights, int* sorted, int* plan, int plan_words,

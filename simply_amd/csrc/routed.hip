@@ -823,6 +823,17 @@ extern "C" int sa_route_few_takes(const void* x, int64_t x_stride, int T, int D,
          top <= E && T * top <= kFewPairs;
 }
 
+// One CU against a product on many and two launches more.  What it costs above them in us, fitted to 300 sizes (logits on 1 to 9 tiles
+// of 16 experts, 1 to 16 tokens, 1 to 128 pairs): a wave adds up and chooses for each token, tiles come one after the other, pairs pass
+// by the sorting wave, the weights come through one CU, and more than 64 experts or pairs take the larger variant.  Few / three launches
+// in us: 16 experts, top 2, 2,048 wide, 1 token 5.9 / 9.7, 8 7.8 / 11.1, 16 10.2 / 12.0; 32, top 4, 1,024 wide, 8 tokens 11.5 / 12.5, 12
+// 13.5 / 12.7, 16 15.8 / 12.9; 64, top 6, 1,024 wide, 4 14.3 / 15.4, 8 17.4 / 15.7, 16 27.6 / 16.2; 128, top 8, 960 wide, 1 19.3 / 21.2,
+// 8 30.0 / 21.9, 16 42.8 / 22.2.  (The line lies a little below the fit: of the sizes it takes none is more than 2 % behind.)
+extern "C" int sa_route_few_pays(int T, int D, int rows, int E, int top) {
+  const int tiles = (rows + 15) / 16;
+  return 0.08 * T * tiles + 0.07 * T * top + 0.12 * tiles * D / 1024 + (E > kWave || T * top > kWave ? 1.3 : 0.0) < 4.4;
+}
+
 extern "C" int sa_route_few(const void* x, int64_t x_stride, const void* w, int T, int D, int rows, int E, int top, float scale,
                             int plain, const void* bias, int bias_dtype, const void* correction, int corr_dtype, int groups, int keep,
                             int softmax, int group_best, float renorm, float* logits, int* experts, float* weights, int* sorted,

@@ -123,6 +123,7 @@ _SIGNATURES = {
     "sa_wkv_token_takes": [_I, _I, _L, _I, _I, _I, _L, _P, _P],
     "sa_wkv_token": [_P, _L, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _I, _P, _I, _F, _I, _I, _P, _L, _P, _I, _P, _P],
     "sa_route_few_takes": [_P, _L, _I, _I, _I, _I, _I],
+    "sa_route_few_pays": [_I, _I, _I, _I, _I],
     "sa_route_few": [_P, _L, _P, _I, _I, _I, _I, _I, _F, _I, _P, _I, _P, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P, _I,
                      _I, _I, _F, _P, _P],
     "sa_expert_product_shared": [_P, _L, _I, _P, _I, _I, _P, _P, _I, _I, _P, _L, _P, _L, _P, _I, _I, _I, _P, _L, _P],

@@ -2107,6 +2107,11 @@ def route_few_takes(x: torch.Tensor, router, num_experts: int, top: int) -> bool
                                                                      int(num_experts), int(top)))
 
 
+def route_few_pays(T: int, router, num_experts: int, top: int) -> bool:
+    """Whether `route_few`, where it takes the rows, is expected to be faster than the product, the choice and the sort by themselves."""
+    return bool(_lib.load().sa_route_few_pays(int(T), router.cols, router.rows, int(num_experts), int(top)))
+
+
 def route_few(x: torch.Tensor, router: TiledWeight, num_experts: int, top: int, scale: float, *,
               options: dict | None = None, dense: tuple | None = None) -> tuple:
     """The router of a few tokens in one launch: (logits float32 [T, rows of the router], experts, weights, (sorted, plan)) with

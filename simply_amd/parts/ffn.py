@@ -194,7 +194,8 @@ class RoutedExperts(FeedForward):
                                           group_best=self.group_best, renorm=self.renormalize, bias=self.router_bias_w)
         order = dense = shared = None
         # a handful of tokens: the router in one kernel, the shared feed-forward beside it and the experts
-        if ops.route_few_takes(x, self.router, E, self.top) and ops.few_rows_experts(x.shape[0], self.top, self.gate_w, self.up_w, x):
+        if ops.route_few_takes(x, self.router, E, self.top) and ops.route_few_pays(x.shape[0], self.router, E, self.top) \
+                and ops.few_rows_experts(x.shape[0], self.top, self.gate_w, self.up_w, x):
             args = (x, self.router, E, self.top, self.router_scale)
             if not self._shared_beside():
                 logits, experts, weights, order = ops.route_few(*args, options=options)

@@ -45,3 +45,35 @@ def test_latent_rows_look_at_every_buffer_s_alignment(lib, which):
     (1024, 4096, 336, 128), (3072, 1536, 336, 128), (1024, 8192, 192, 128), (1024, 1024, 400, 64), (2048, 1536, 256, 64)])
 def test_rows_of_a_tile_of_routed_experts(lib, D, F, per, rows):
     assert lib.sa_expert_tile_rows(16 * per, 16, D, F, 1, D, 4096) == rows
+
+
+@pytest.mark.parametrize("T,D,E,top,pays", [
+    (1, 2048, 16, 2, True), (16, 2048, 16, 2, True), (16, 4096, 16, 2, True), (16, 512, 8, 2, True), (4, 2048, 16, 8, True),
+    (16, 1024, 16, 4, False), (16, 2048, 16, 8, False), (4, 4096, 32, 4, True), (12, 1024, 32, 4, False), (16, 4096, 32, 8, False),
+    (4, 1024, 64, 6, True), (8, 1024, 64, 6, False), (16, 2048, 64, 8, False), (1, 960, 128, 8, True), (8, 960, 128, 8, False)])
+def test_router_of_few_tokens_where_it_pays(lib, T, D, E, top, pays):
+    """Sizes at which one workgroup or three launches were clearly ahead (128 experts, top 8, 16 tokens: 43 us for 22)."""
+    assert bool(lib.sa_route_few_pays(T, D, E, E, top)) == pays
+
+
+def test_routers_that_do_not_pay_go_the_way_of_many_tokens(lib, monkeypatch):
+    """With 128 experts a step of 8 tokens is routed by the product, the choice and the sort."""
+    import types
+
+    import torch
+
+    from simply_amd.kernels import ops
+    from simply_amd.parts.ffn import RoutedExperts
+
+    part, seen = RoutedExperts(960, 128, 8, 16), []
+    part.router = types.SimpleNamespace(rows=128, cols=960)
+    monkeypatch.setattr(ops, "route_few_takes", lambda *a: True)
+    monkeypatch.setattr(ops, "few_rows_experts", lambda *a: True)
+    monkeypatch.setattr(ops, "route_few", lambda *a, **k: seen.append("few") or (torch.zeros(1, 128), None, None, ()))
+    monkeypatch.setattr(ops, "gemm", lambda x, w, **k: seen.append("product") or torch.zeros(x.shape[0], 128))
+    monkeypatch.setattr(ops, "route", lambda *a: (None, None))
+    monkeypatch.setattr(ops, "routed_experts", lambda *a, **k: None)
+    monkeypatch.setattr(ops, "expert_sums", lambda *a, **k: types.SimpleNamespace(materialize=lambda: None))
+    for tokens in (1, 8):
+        part.forward(torch.zeros(tokens, 960))
+    assert seen == ["few", "product"]

@@ -23,6 +23,7 @@ def few(monkeypatch):
         raise Routed("beside" if dense is not None else "apart")
 
     monkeypatch.setattr(ops, "route_few_takes", lambda *a: True)
+    monkeypatch.setattr(ops, "route_few_pays", lambda *a: True)
     monkeypatch.setattr(ops, "few_rows_experts", lambda *a: True)
     monkeypatch.setattr(ops, "route_few", route_few)
 
