@@ -399,6 +399,8 @@ int sa_experts_add_next_norm(const float* y, const float* weights, int top, cons
                              int64_t shared_stride, const float* gate, int64_t gate_stride, float mult, float* residual,
                              const void* w, const void* b, int w_dtype, float eps, int plus_one, void* out, int T, int D,
                              hipStream_t stream);
+// _pays: whether it is expected to be faster than the two (host functions, both).
+int sa_experts_add_next_norm_pays(int D, int top);
 int sa_experts_add_next_norm_takes(int D, const void* shared, int64_t shared_stride, const void* residual, const void* w, const void* b);
 
 // Queries [T, H (R + dr)] turned in place (the rot_dims entries behind a head's R) and key rows [T, R + dr] = [latent | shared part]

@@ -725,6 +725,12 @@ extern "C" int sa_residual_add_next_norm(const void* y, int y_dtype, int64_t y_s
   return check_launch("residual_add_next_norm");
 }
 
+// A workgroup adds a token's rows up one after the other, four pieces of 2,048 entries with their own sums each; the sum's kernel has a
+// workgroup per piece.  Fused / sum and norm in us, 1, 64 and 2,047 tokens: 2,048 wide, top 16 3.8 / 4.9, 6.0 / 6.9, 59 / 63; 4,096,
+// top 8 4.6 / 5.2, 6.8 / 7.3, 69 / 72, top 16 5.8 / 5.6, 9.3 / 8.3, 125 / 130; 8,192, top 2 5.8 / 6.2, 7.9 / 8.2, 61 / 66, top 4
+// 6.5 / 6.1, 9.0 / 8.7, 89 / 98, top 16 15.8 / 6.6, 27.9 / 15.2, 249 / 249.
+extern "C" int sa_experts_add_next_norm_pays(int D, int top) { return top <= (D <= 2048 ? 16 : D <= 4096 ? 8 : 2); }
+
 extern "C" int sa_experts_add_next_norm_takes(int D, const void* shared, int64_t shared_stride, const void* residual, const void* w,
                                               const void* b) {
   return D <= 8192 && rows_in_eights(D, shared != nullptr ? shared_stride : 0, shared, residual, w, b, nullptr);

@@ -2163,6 +2163,11 @@ def route_few(x: torch.Tensor, router: TiledWeight, num_experts: int, top: int, 
 SHARED_BESIDE_MAX = 5120
 
 
+def expert_sums_pay(D: int, top: int) -> bool:
+    """Whether the sum over `top` experts' rows of D entries is expected to be faster in the next norm than by itself."""
+    return bool(_lib.load().sa_experts_add_next_norm_pays(int(D), int(top)))
+
+
 def few_rows_experts(T: int, top: int, gate_w, up_w, x: torch.Tensor) -> bool:
     """Whether a step of T tokens goes through the experts in tiles of 16 rows."""
     return _lib.load().sa_expert_tile_rows(T * top, up_w.experts, up_w.cols, up_w.rows, _code(x), x.stride(0), _ptr(x)) == 16

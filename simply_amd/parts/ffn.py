@@ -187,6 +187,7 @@ class RoutedExperts(FeedForward):
     @knows_expert_sums
     def forward(self, x: torch.Tensor, ctx=None, defer_experts=False) -> "torch.Tensor | ops.ExpertSums":
         E = self.num_experts
+        defer = defer_experts and x.is_cuda and ops.expert_sums_pay(self.hidden_size, self.top)
         plain = self.router_kind == "softmax" and not self.correction and self.num_groups == 1 and self.renormalize is None \
             and not self.router_bias
         options = None if plain else dict(correction=self.correction_w, groups=self.num_groups, keep=self.keep_groups,
@@ -215,6 +216,6 @@ class RoutedExperts(FeedForward):
         args = (x, experts, weights, self.gate_w, self.up_w, self.down_w, self.activation_code)
         kw = dict(shared=shared, shared_gate=logits[:, E:E + 1] if self.shared_gate else None, limit=self.limit)
         if order is None:
-            return ops.routed_experts(*args, **kw, **({"defer_sum": True} if defer_experts and x.is_cuda else {}))
+            return ops.routed_experts(*args, **kw, **({"defer_sum": True} if defer else {}))
         sums = ops.expert_sums(*args, **kw, order=order, dense=dense)
-        return sums if defer_experts else sums.materialize()
+        return sums if defer else sums.materialize()
