@@ -102,6 +102,70 @@ def test_products_of_whole_blocks(M, N, K, gated, tile, cut):
         assert torch.equal(ops.gemm(a[rows], w, **kw), got[rows])
 
 
+@pytest.mark.parametrize("M,N,K,gated,tile,cut", [
+    (17, 1570, 256, False, (64, 128), True), (17, 18433, 160, False, (64, 128), False), (130, 4100, 160, True, (64, 128), False),
+    (65, 18433, 160, False, (128, 64), True), (17, 3135, 160, True, (128, 64), False), (257, 8003, 160, False, (128, 128), False),
+    (65, 18433, 992, True, (128, 128), True), (200, 18433, 160, False, (128, 192), False), (65, 4100, 992, False, (128, 192), True),
+    (130, 3135, 992, False, (128, 256), True), (257, 18433, 160, False, (128, 256), False), (1000, 4100, 160, True, (128, 256), True)])
+def test_products_of_parts(M, N, K, gated, tile, cut):
+    """K in segments of whole stages of 32 columns (the last one shorter at 992), the products those of bfloat16 parts: every tile, whole,
+    cut, and cut behind 256 whole ones, the last rows and columns missing.  Rows and weights of very different sizes: the parts hold
+    all of a number's 24 bits, so the bounds are those of a sum in 32 bits; the bits are those of the kernel for few rows."""
+    from simply_amd.kernels import ops
+
+    assert ops.gemm_f32_tile(M, N, K, gated=gated) == tile and ops.gemm_f32_plan(M, N, K, gated=gated) == (tile[0], cut)
+    wide, w, w2 = draw((M, K + 12), 31), draw((N, K), 32, 0.1), draw((N, K), 33, 0.1)
+    a = wide[:, 8:8 + K]
+    a[::3] *= 2.0 ** 40
+    a[1::3, ::2] *= 2.0 ** -30
+    w[::5] *= 2.0 ** -45
+    kw = dict(w2=w2, activation=ops.ACT_SILU) if gated else {}
+    got = ops.gemm(a, w, **kw)
+    x, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    bound = (K + 2) * EPS * size
+    if gated:
+        up, up_bound = a.double() @ w2.double().T, (K + 2) * EPS * (a.double().abs() @ w2.double().abs().T)
+        want = torch.nn.functional.silu(x) * up
+        bound = 1.1 * bound * up.abs() + x.abs() * up_bound + 8 * EPS * want.abs()
+    else:
+        want = x
+    assert ((got.double() - want).abs() <= bound).all()
+    assert torch.equal(ops.gemm(a.contiguous(), w, **kw), got)
+    for rows in (slice(0, 5), slice(0, 16), slice(M // 2, M // 2 + 5), slice(M - 5, M)):
+        assert torch.equal(ops.gemm(a[rows], w, **kw), got[rows])
+    if not gated:
+        capped = ops.gemm(a, w, soft_cap=2.0)
+        assert ((capped.double() - 2.0 * torch.tanh(want / 2.0)).abs() <= bound + 8 * EPS * 2.0).all()
+        assert torch.equal(ops.gemm(a[M - 5:], w, soft_cap=2.0), capped[M - 5:])
+
+
+@pytest.mark.parametrize("N", [50, 4100])
+def test_products_of_parts_keep_special_values(N):
+    """An infinite or undefined entry reaches its own row and column only, as in plain 32-bit arithmetic, and entries next to the
+    largest number, whose first part is rounded to an infinite one, give the finite sums that they have."""
+    from simply_amd.kernels import ops
+
+    K, largest = 256, torch.finfo(torch.float32).max
+    for M in (3, 16, 40, 200):
+        a, w, up = draw((M, K), 5), draw((N, K), 6), draw((N, K), 7)
+        a[1, 70], a[0, 9], w[7, 3], w[20, 9], up[9, 200] = float("inf"), largest, float("nan"), 0.0, float("-inf")
+        a[2, 11], w[20, 11] = -largest, 2.0 ** -20
+        got, gated = ops.gemm(a, w), ops.gemm(a, w, w2=up, activation=ops.ACT_SILU)
+        assert torch.isnan(got[:, 7]).all() and torch.isnan(gated[:, 7]).all()
+        keep = torch.arange(N, device="cuda") != 7
+        assert torch.isinf(got[1, keep]).all() and (got[1, keep].sign() == w[keep, 70].sign()).all()
+        rest = torch.arange(M, device="cuda") != 1
+        want = a[rest].double() @ w[keep].double().T
+        size = a[rest].double().abs() @ w[keep].double().abs().T
+        y = got[rest][:, keep].double()
+        ok = want.abs() < largest / 2
+        assert ((y - want).abs()[ok] <= ((K + 2) * EPS * size)[ok]).all()
+        assert torch.isfinite(got[0, 20]) and torch.isfinite(got[2, 20])
+        # the other factor's column: infinite or, where the gate's factor is zero, undefined
+        assert not torch.isfinite(gated[rest][:, 9]).any()
+        assert torch.equal(ops.gemm(a[-2:], w)[:, keep], got[-2:, keep])
+
+
 def test_products_keep_special_values():
     """An infinite or undefined entry reaches its own row and column only."""
     from simply_amd.kernels import ops
