@@ -461,10 +461,13 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
   // Workgroups of four waves run two to a CU, where one's epilogue and first loads overlap the other's
   // products (measured: 7-9 % faster than one workgroup of twice the tile once every CU has two of them;
   // slower when it has one; from one and a half per CU on it is also the best for few rows of very many weight
-  // rows, which are bound by streaming them).
+  // rows, which are bound by streaming them).  A tile of 128 x 128, whose waves read more of LDS for a product, takes
+  // 1.38 times as long for its size: it pays where it gives every CU work (2,048 rows, us, against 192 x 128:
+  // 2,048 outputs of K = 2,048 22 for 25, of 8,192 74 for 77; 1,024 outputs 18.5 for 22 and 62 for 72; 4,096 rows
+  // against 1,024 outputs of K = 4,096 38 for 41), and not with a second round (2,304 outputs: 35 for 25).
   const int NW = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N;
-  const int shapes[5][4] = {{2128192, 128, 192, 93}, {2256192, 256, 192, 100}, {3256128, 256, 128, 100},
-                            {3128256, 128, 256, 100}, {3192128, 192, 128, 100}};
+  const int shapes[6][4] = {{2128192, 128, 192, 93}, {2256192, 256, 192, 100}, {3256128, 256, 128, 100},
+                            {3128256, 128, 256, 100}, {3192128, 192, 128, 100}, {4128128, 128, 128, 138}};
   int64_t best = -1;
   for (const auto& sh : shapes) {
     const int64_t tiles = static_cast<int64_t>((M + sh[1] - 1) / sh[1]) * ((NW + sh[2] - 1) / sh[2]);
