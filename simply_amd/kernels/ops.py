@@ -1867,6 +1867,39 @@ def token_shift(h: torch.Tensor, mu: torch.Tensor, tails: torch.Tensor, seq_meta
     return out
 
 
+def add_next_norm_shift(y: "torch.Tensor | ExpertSums | None", residual: torch.Tensor, weight: torch.Tensor, *, eps: float,
+                        plus_one: bool, mult: float, bias: torch.Tensor | None, mu: torch.Tensor, tails: torch.Tensor,
+                        seq_meta: torch.Tensor, num_seqs: int) -> torch.Tensor | None:
+    """`residual_add_next_norm` in bfloat16 and `token_shift` of its result in one kernel, for a step with one token of every
+    request: the mixes [T, S * D]; or None where the kernel does not take these (nothing has been done then)."""
+    sums = isinstance(y, ExpertSums)
+    if isinstance(y, PartialSums):
+        return None
+    T, D = residual.shape
+    rows = y.y if sums else y
+    if residual.dtype != torch.float32 or not residual.is_cuda or not residual.is_contiguous() or T != num_seqs \
+            or any(v is not None and (v.dtype != weight.dtype or not v.is_contiguous()) for v in (weight, bias, mu)) \
+            or weight.numel() != D or (bias is not None and bias.numel() != D) or mu.dim() != 2 or mu.shape[1] != D \
+            or tails.dtype != torch.float32 or tails.dim() != 2 or tails.stride(1) != 1 or tails.shape[1] < D \
+            or (y is not None and tuple(y.shape) != (T, D)) \
+            or (rows is not None and not sums and (rows.dtype != torch.bfloat16 or rows.stride(1) != 1)):
+        return None
+    shared = y.shared if sums else None
+    stride = rows.stride(0) if rows is not None and not sums else 0
+    if not _lib.load().sa_add_next_norm_shift_takes(D, mu.shape[0], _ptr(rows), stride, _ptr(shared),
+                                                    shared.stride(0) if shared is not None else 0, _ptr(residual), _ptr(weight),
+                                                    _ptr(bias), _ptr(mu), _ptr(tails), tails.stride(0)):
+        return None
+    _dev(rows, residual, weight, bias, mu, tails, seq_meta)
+    _seq_meta(seq_meta, num_seqs, "add_next_norm_shift")
+    experts = y._rows_args()[1:] if sums else (None, 0, None, 0, 0, None, 0)
+    out = torch.empty((T, mu.shape[0] * D), dtype=torch.bfloat16, device=residual.device)
+    _lib.call("sa_add_next_norm_shift", _ptr(rows), stride, *experts, float(mult), _ptr(residual), _ptr(weight), _ptr(bias),
+              _code(weight), float(eps), int(plus_one), _ptr(mu), mu.shape[0], _ptr(tails), tails.stride(0), _ptr(seq_meta), _ptr(out),
+              T, D, _stream())
+    return out
+
+
 def low_rank_decay(p: torch.Tensor, w: "torch.Tensor | TiledWeight", base: torch.Tensor) -> torch.Tensor:
     """float32 [T, C]: exp(-exp(w tanh(p) + base)) with p [T, rank], w [C, rank] (tiled if bfloat16 on the GPU), base [C].
     All of it is 32-bit: where the matrix cores take bfloat16 operands, tanh is three of them."""

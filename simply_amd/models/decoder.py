@@ -138,6 +138,12 @@ class DecoderModel:
         if self.stream_sum is not None:
             h = begin_streams(h, self.spec.streams)
         normed = None
+
+        def norm_in_front(i):
+            block = self.layers[schedule[i].layer]
+            offer = getattr(block, "norm_of_step", None)
+            return offer(ctx, cache_views[i]) if offer is not None else block.first_norm()
+
         for i, entry in enumerate(schedule):
             block = self.layers[entry.layer]
             if entry.add_embedding:
@@ -148,10 +154,10 @@ class DecoderModel:
             if entry.begins_pass is not None:
                 if isinstance(normed, PendingNorm):
                     h = normed.settle()
-                h, normed = self.pass_input.forward(h, again, entry.begins_pass, ctx, block.first_norm())
+                h, normed = self.pass_input.forward(h, again, entry.begins_pass, ctx, norm_in_front(i))
             nxt = None
             if i + 1 < len(schedule) and not schedule[i + 1].add_embedding and schedule[i + 1].begins_pass is None:
-                nxt = self.layers[schedule[i + 1].layer].first_norm()
+                nxt = norm_in_front(i + 1)
             h, normed = block.forward(h, ctx, cache_views[i], normed, nxt)
             if after_layer is not None:
                 if isinstance(normed, PendingNorm):

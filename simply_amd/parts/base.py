@@ -27,6 +27,9 @@ Results of routed experts may be handed on as `ops.ExpertSums`, the experts' row
 of it say so (`knows_expert_sums`): a feed-forward's `forward`, which then takes `defer_experts=True` and may return one; a norm's
 `after_sum`, which then takes one in place of y; and whatever a block arrangement puts between the two.  A block asks for it only where
 all of them do.  What says so is the method, not the class: one that overrides it is not taken to know.
+A block may offer, for a step, another norm than `first_norm()` to what comes before it (`norm_of_step(ctx, cache)`): one whose `after_sum`
+may return what the block's mixer makes of the normed rows first (`MixedRows`), in the same kernel.  The block then finds that in place
+of the normed rows.
 """
 from __future__ import annotations
 
@@ -40,6 +43,13 @@ def knows_expert_sums(method):
     """Marks a method that takes or returns `ops.ExpertSums` (see above)."""
     method.knows_expert_sums = True
     return method
+
+
+@dataclasses.dataclass(frozen=True)
+class MixedRows:
+    """In place of normed rows: what the mixer behind the norm has made of them (see above)."""
+
+    rows: torch.Tensor
 
 
 @dataclasses.dataclass(frozen=True)

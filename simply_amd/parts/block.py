@@ -142,6 +142,12 @@ class PreNormBlock(Block):
     def first_norm(self):
         return self.norms["pre_mixer"]
 
+    def norm_of_step(self, ctx, cache):
+        """The first norm as the mixer has it in this step, for whoever computes it ahead of `forward`."""
+        offer = getattr(self.mixer, "norm_of_step", None)
+        norm = self.first_norm()
+        return offer(norm, ctx, cache) if offer is not None and type(self).forward is PreNormBlock.forward else norm
+
     @knows_expert_sums
     def _add(self, h, y, norm, dtype):
         """h += mult * y; returns norm(h), or None without a norm."""
@@ -155,7 +161,8 @@ class PreNormBlock(Block):
         if isinstance(normed, PendingNorm):
             normed, h = normed.materialize(), normed.residual
         if normed is None:
-            normed = n["pre_mixer"].forward(h, ctx.dtype)
+            norm = self.norm_of_step(ctx, cache)
+            normed = norm.after_sum(h, None, 1.0, ctx.dtype) if norm is not self.first_norm() else n["pre_mixer"].forward(h, ctx.dtype)
         y = self.mixer.forward(normed, ctx, cache)
         if self.feed_forward is None:
             return h, self._add(h, y, next_norm, ctx.dtype)

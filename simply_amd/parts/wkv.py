@@ -15,8 +15,31 @@ import torch
 
 from ..kernels import ops
 from ..registry import MIXERS
-from .base import Mixer, ParamSpec, StateNeed, as_product_weight
+from .base import MixedRows, Mixer, Norm, ParamSpec, StateNeed, as_product_weight, knows_expert_sums
 from .linear_state import channel_decay_state
+from .norm import LayerNorm, RMSNorm
+
+
+class ShiftedNorm(Norm):
+    """The norm in front of the mixer, together with the mixer's token shift: for a step with one token of every request."""
+
+    fuses_sum = True
+
+    def __init__(self, norm, mixer, ctx, cache):
+        self.norm, self.mixer, self.ctx, self.cache = norm, mixer, ctx, cache
+
+    def forward(self, x, out_dtype):
+        return self.norm.forward(x, out_dtype)
+
+    @knows_expert_sums
+    def after_sum(self, residual, y, mult, out_dtype):
+        n, m = self.norm, self.mixer
+        rows = None
+        if out_dtype == torch.bfloat16:
+            rows = ops.add_next_norm_shift(y, residual, n.scale, eps=n.eps, plus_one=getattr(n, "scale_plus_one", False), mult=mult,
+                                           bias=getattr(n, "bias", None), mu=m.mu, tails=self.cache.state[:, m.state_words:],
+                                           seq_meta=self.ctx.seq_meta, num_seqs=self.ctx.num_seqs)
+        return MixedRows(rows) if rows is not None else n.after_sum(residual, y, mult, out_dtype)
 
 
 @MIXERS.register("wkv")
@@ -54,12 +77,23 @@ class WKV(Mixer):
     def cache_need(self):
         return StateNeed((self.state_words + self.hidden_size,), torch.float32)   # S, then the last token's h
 
+    def norm_of_step(self, norm, ctx, cache):
+        """`norm`, or in a step with one token of every request that norm with the token shift in its kernel."""
+        known = type(norm).after_sum in (RMSNorm.after_sum, LayerNorm.after_sum) and norm.fuses_sum
+        if known and type(self).forward is WKV.forward and cache.write and ctx.dtype == torch.bfloat16 and ctx.max_q_len == 1 \
+                and ctx.num_tokens == ctx.num_seqs and ctx.positions.is_cuda:
+            return ShiftedNorm(norm, self, ctx, cache)
+        return norm
+
     def forward(self, x, ctx, cache):
         if not cache.write:
             raise RuntimeError("wkv: a recurrent state cannot be read through another entry's cache")
         D, H, d = self.hidden_size, self.num_heads, self.head_dim
         C = H * d
-        mixes = ops.token_shift(x, self.mu, cache.state[:, self.state_words:], ctx.seq_meta, ctx.num_seqs, ctx.max_q_len)
+        if isinstance(x, MixedRows):
+            mixes = x.rows
+        else:
+            mixes = ops.token_shift(x, self.mu, cache.state[:, self.state_words:], ctx.seq_meta, ctx.num_seqs, ctx.max_q_len)
         if self.decay_in is None:
             proj = ops.gemm_sections(mixes, self.in_proj)                             # [T, r | k | v | gate | decay's factor]
             low = proj[:, 4 * C:]

@@ -75,3 +75,32 @@ def test_latent_rows(slots, H, R, dr, rot, P, weights):
 def test_latent_rows_of_many_heads(T, H, dr, rot):
     """Heads that more than one workgroup turns: eight times what its 1,024 threads hold of 16 tokens."""
     test_latent_rows(list(range(48, 48 + T)), H, 16, dr, rot, 16, torch.bfloat16)
+
+
+@pytest.mark.parametrize("T,D,vectors,centered,add", [
+    (1, 8, torch.bfloat16, True, "rows"), (3, 2048, torch.bfloat16, True, "row"), (8, 2048, torch.float32, False, "none"),
+    (5, 2056, torch.bfloat16, True, "experts"), (64, 4096, torch.float32, False, "experts32"), (7, 1000, torch.bfloat16, False, "experts"),
+    (2, 4096, torch.bfloat16, True, "none")])
+def test_norm_and_token_shift(T, D, vectors, centered, add):
+    """The same sums, norms, mixes and last rows as the norm's kernel and the token shift's, to the bit; requests in other slots, other
+    rows and the columns behind the last rows stay as they are.  Rows that are not whole pieces of eight are left to those two."""
+    from simply_amd.kernels import ops
+
+    h = draw((T, D), 1).cuda()
+    w, b = (draw((D,), 2 + i, 0.3).to(vectors).cuda() for i in range(2))
+    mu = torch.rand((5, D), generator=torch.Generator().manual_seed(4)).to(vectors).cuda()
+    state = draw((T + 2, D + 24), 5).cuda()
+    meta = torch.tensor([[T + 1 - j, j, 1, 9] for j in range(T)], dtype=torch.int32).cuda()
+    shared = draw((T, D), 6).to(torch.float32 if add == "experts32" else torch.bfloat16).cuda()
+    y = {"rows": lambda: draw((T, D + 8), 7).bfloat16().cuda()[:, :D], "row": lambda: draw((1, D), 7).bfloat16().cuda().expand(T, -1),
+         "none": lambda: None}.get(add, lambda: ops.ExpertSums(draw((T * 2, D), 8).cuda(), torch.rand((T, 2)).cuda(), shared, None, torch.bfloat16))()
+    kw = dict(eps=1e-5, mult=0.7, bias=b if centered else None)
+    mine, theirs, one, two = h.clone(), h.clone(), state.clone(), state.clone()
+    got = ops.add_next_norm_shift(y, mine, w, plus_one=False, mu=mu, tails=one[:, 16:], seq_meta=meta, num_seqs=T, **kw)
+    normed = ops.residual_add_next_norm(y, theirs, w, out_dtype=torch.bfloat16, **kw)
+    want = ops.token_shift(normed, mu, two[:, 16:], meta, T, 1)
+    assert torch.equal(got, want) and torch.equal(mine, theirs) and torch.equal(one, two)
+    args = dict(plus_one=False, seq_meta=meta, num_seqs=T, **kw)
+    assert ops.add_next_norm_shift(y, mine, w, mu=mu, tails=one[:, 15:], **args) is None      # not aligned
+    assert ops.add_next_norm_shift(y, mine, w, mu=mu[:4], tails=one[:, 16:], **args) is None  # not five streams
+    assert torch.equal(mine, theirs) and torch.equal(one, two)
