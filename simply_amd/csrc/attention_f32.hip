@@ -11,10 +11,10 @@
 // in the batch or on which pages hold the keys.  Three ways of running the ranges, with the same arithmetic (sa_paged_attention_f32_parts
 // says which, and why):
 //
-//   a workgroup per unit, key head and chunk, four waves to it, partial results to the workspace, a merge kernel: few units and ranges
-//   (decoding), whose chunks are all there is to fill the chip with;
-//   a workgroup per unit, key head and range, partial results and a merge likewise: few units with more ranges;
-//   a workgroup per unit and key head that walks through the ranges: prompts, or where the workspace is too small.
+//   a workgroup per unit, key head and chunk, four waves to it, partial results to the workspace, a merge kernel: few units and ranges,
+//   whose chunks are all there is to fill the chip with;
+//   a workgroup per unit, key head and range, partial results and a merge likewise: more of them, longer prompts;
+//   a workgroup per unit and key head that walks through the ranges: many decoding requests, or where the workspace is too small.
 //
 // Keys that some row of the unit does not see get the weight zero.  Where such keys' values are not finite (a zero weight
 // would spread them), their products are taken one key at a time and left out of the rows that do not see it.
@@ -24,7 +24,7 @@
 //
 // Bound by the latency of a wave's chunk (loads of keys, scores, exponentials, values, one after the other) at the measured
 // sizes, 2B heads: 4 requests of 257 to 1,023 keys 10.4 us and 5.4 for the merge, where the generic kernel, a workgroup per
-// token and key head that walks through all keys on the vector ALU, took 786; a prompt of 509 tokens 45 us for 498.
+// token and key head that walks through all keys on the vector ALU, took 786; a prompt of 509 tokens 35 us for 498 (42 walked).
 #include "api.h"
 #include "attention_common.h"
 
@@ -512,6 +512,17 @@ extern "C" int sa_paged_attention_f32_parts(int unit_count, int Kh, int hd, int 
   const int ranges = f32_ranges(window, max_kv_len, max_q_len);
   const int64_t heads = static_cast<int64_t>(unit_count) * Kh;
   const int64_t bytes = heads * ranges * 16 * (hd + f32att::kExtra) * static_cast<int64_t>(sizeof(float));   // a part a range
+  // Prompts (units of four tokens and more; up to four heads a key head have such): a unit sees what lies before it, so units that walk are as slow as the last one's ranges one
+  // after the other, and a chunk is a chain of waits of 10 us that more workgroups cover.  Walked / ranges / chunks in us, heads of 256,
+  // 4 key heads, by triples (see below): 64 tokens (32) 20 / 20 / 12, behind 2,048 others (288) 186 / 43 / 44; 509 (512) 42 / 38 / 35; 700
+  // (1,056) 83 / 62 / 51; behind 512 (1,760) 163 / 97 / 96; 384 behind 2,048 (1,920) 198 / 125 / 124; 1,024 (2,048) 137 / 94 / 95; 509
+  // behind 2,048 (2,560) 198 / 154 / 166; 2,048 (8,192) 397 / 274.  16 key heads of 128: 256 (512, one range) 20 / 23 / 25, 512 (2,048)
+  // 62 / 52 / 59; 4 of 64: 128 (32) 8.6 / 10.5 / 7.3, 512 (256) 15.3 / 11.3 / 11.4, 16 heads over 4, 1,024 (4,096) 64 / 48 / 58.
+  if (max_q_len >= 4) {
+    if (heads * ranges * 36 <= static_cast<int64_t>(hd) * hd && ranges * f32att::kWaves <= 65535 && bytes * f32att::kWaves <= workspace_bytes)
+      return f32att::kWaves;
+    return ranges > 1 && ranges <= 65535 && bytes <= workspace_bytes ? 1 : 0;
+  }
   // Parts while the units alone do not fill the 256 CUs.
   if (ranges <= 1 || ranges > 65535 || heads >= 256 || bytes > workspace_bytes) return 0;
   // A workgroup per chunk while the ranges leave half of the CUs idle: beyond that, four times the parts cost the merge more than four

@@ -30,6 +30,19 @@ def test_32_bit_attention_of_long_contexts_keeps_its_ranges(lib):
     assert parts(2, 4, 256, None, 2048, 1, 8 * 8 * row - 1) == 0
 
 
+def test_32_bit_attention_of_prompts_fills_the_chip(lib):
+    """Units of several tokens: a part for each chunk of short prompts, for each range of longer ones; walked where one range is all there
+    is of many units, or the workspace holds no part for every range."""
+    from simply_amd.kernels import ops
+
+    parts = ops.attention_f32_parts
+    assert parts(8, 4, 256, None, 64, 8) == 4 and parts(64, 4, 256, None, 509, 8) == 4 and parts(88, 4, 256, None, 700, 8) == 4
+    assert parts(128, 4, 256, None, 1024, 8) == 1 and parts(64, 4, 256, None, 2557, 8) == 1 and parts(256, 4, 256, None, 2048, 8) == 1
+    assert parts(32, 16, 128, None, 256, 8) == 0 and parts(64, 16, 128, None, 512, 8) == 1 and parts(8, 4, 64, None, 128, 8) == 4
+    row = 16 * (256 + 4) * 4
+    assert [parts(64, 4, 256, None, 509, 8, n * 512 * row) for n in (0, 1, 3, 4)] == [0, 1, 1, 4]
+
+
 @pytest.mark.parametrize("which", ["q", "rows", "weight", "k_pages", "v_pages"])
 def test_latent_rows_look_at_every_buffer_s_alignment(lib, which):
     """Pieces of 16 bytes are read and written at all five: a view that begins elsewhere goes the way of single entries."""
