@@ -24,10 +24,10 @@
 //
 // Measured, weights from HBM; "unit" with the 32-bit matrix unit throughout:
 //   (N, K)                4 rows, unit   61 rows, unit    509 rows, unit    1,024 rows, unit
-//   (2304, 9216)          21.8, 21.7     40, 46           143, 176          219, 333
-//   (2304, 2048)          10.6, 10.3     15.6, 19.7       46, 54            62, 104
-//   (4096, 2304)          10.6, 10.7     18.0, 19.0       65, 87            99, 156
-//   (9216 gated, 2304)    36, 43         61, 64           206, 329          405, 635 (215 TFLOP/s)
+//   (2304, 9216)          21.8, 21.7     40, 46           114, 176          227, 333
+//   (2304, 2048)          10.6, 10.3     15.6, 19.7       39, 54            68, 104
+//   (4096, 2304)          10.6, 10.7     18.0, 19.0       67, 87            104, 156
+//   (9216 gated, 2304)    36, 43         61, 64           210, 329          435, 635 (200 TFLOP/s)
 //   (256000, 2304)        378, 392 (6.2 TB/s)
 #include "api.h"
 #include "common.h"
@@ -643,8 +643,11 @@ template <int EPI, int TM, int TN, int WM, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a, Share share) {
   constexpr int THREADS = WAVES * kWave, WN = WAVES / WM, AB = WM * TM, WB = WN * TN;   // blocks of 16 rows of A and of W
   constexpr int BLOCKS = AB + WB, LOADS = (BLOCKS + WAVES - 1) / WAVES, BUF = BLOCKS * 3 * 512;
-  constexpr int WT = EPI == 1 ? TN / 2 : TN;             // blocks of outputs across of a wave
-  static_assert(EPI != 1 || TN % 2 == 0, "half of a wave's weight rows are the gate's");
+  // Gated: half of a wave's weight rows are the gate's; with an odd number of blocks a wave beside another has the gate's rows or the
+  // other factor's, and the two exchange half of their sums at the end.  Such tiles' weight parts are read block by block.
+  constexpr bool APART = TN % 2 == 1 && TN > 4, GATE_APART = EPI == 1 && APART;
+  constexpr int WT = EPI == 1 && !APART ? TN / 2 : TN;   // blocks of outputs across of a wave
+  static_assert(EPI != 1 || TN % 2 == 0 || (APART && WN == 2 && TM == 2), "gate and factor in one wave, or in two beside each other");
   static_assert(AB % WAVES == 0, "a wave's first blocks are A's");
   __shared__ __align__(16) __bf16 lds[2 * BUF];
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -658,28 +661,33 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
     l = share.full + (l - share.full) / share.nseg;
   }
   const Tile tile = tile_at(share, l);
-  const int m0 = tile.y * AB * 16, n0 = tile.x * (WN * WT * 16);
+  const int m0 = tile.y * AB * 16, n0 = tile.x * ((GATE_APART ? 1 : WN) * WT * 16);
   const int k0 = segment < 0 ? 0 : segment * a.seg;
   const int length = segment >= 0 && k0 + a.seg < a.K ? a.seg : a.K - k0;   // a multiple of 32
   const int ns = length / BK, per_segment = a.seg / BK;
   const int r = lane / 4, p = lane % 4;
-  const float* from[LOADS];
+  // a load's address: the tile's part is the same for all lanes, the rest is an offset in elements (32 bits: K < 4 Mi, 288 rows)
+  const float* const a_tile = a.A + static_cast<size_t>(m0) * a.lda + k0;
+  const float* const w_tile = a.W + static_cast<size_t>(n0) * a.K + k0;
+  const float* const w2_tile = EPI == 1 ? a.W2 + static_cast<size_t>(n0) * a.K + k0 : w_tile;
+  uint32_t from[LOADS];
   auto mine = [&](int i) __attribute__((always_inline)) { return BLOCKS % WAVES == 0 || i * WAVES + wave < BLOCKS; };
+  auto of_gate = [&](int i) __attribute__((always_inline)) {   // (the rows of a block are of one kind)
+    const int n = i * WAVES + wave - AB;
+    return EPI != 1 || (GATE_APART ? n < TN : n % TN < WT);
+  };
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
     const int b = mine(i) ? i * WAVES + wave : 0;
-    if (b < AB) {
-      const int m = m0 + b * 16 + r;
-      from[i] = a.A + static_cast<size_t>(m < a.M ? m : a.M - 1) * a.lda + k0 + p * 4;
+    if (i < AB / WAVES) {
+      const int m = b * 16 + r, last = a.M - 1 - m0;
+      from[i] = static_cast<uint32_t>(m < last ? m : last) * static_cast<uint32_t>(a.lda) + p * 4;
     } else {
       int n = b - AB;
-      const float* w = a.W;
-      if (EPI == 1) {   // of a wave's TN blocks the first half is the gate's
-        if (n % TN >= WT) w = a.W2;
-        n = n / TN * WT + n % TN % WT;
-      }
-      n = n0 + n * 16 + r;
-      from[i] = w + static_cast<size_t>(n < a.N ? n : a.N - 1) * a.K + k0 + p * 4;
+      if (GATE_APART) n %= TN;
+      else if (EPI == 1) n = n / TN * WT + n % TN % WT;   // of a wave's TN blocks the first half is the gate's
+      const int row = (n < 0 ? 0 : n) * 16 + r, last = a.N - 1 - n0;
+      from[i] = static_cast<uint32_t>(row < last ? row : last) * static_cast<uint32_t>(a.K) + p * 4;
     }
   }
   // signs of the segments being summed and being made parts of, and stages that are left of each
@@ -688,8 +696,9 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
   floatx4 v[LOADS][2];
   auto load = [&](int i, int s) __attribute__((always_inline)) {   // (behind the last stage: that one again)
     const int k = (s < ns ? s : ns - 1) * BK;
-    v[i][0] = *reinterpret_cast<const floatx4*>(from[i] + k);
-    v[i][1] = *reinterpret_cast<const floatx4*>(from[i] + k + 16);
+    const float* at = (i < AB / WAVES ? a_tile : of_gate(i) ? w_tile : w2_tile) + k;
+    v[i][0] = *reinterpret_cast<const floatx4*>(at + from[i]);
+    v[i][1] = *reinterpret_cast<const floatx4*>(at + from[i] + 16);
   };
   auto to_lds = [&](int i, int buf) __attribute__((always_inline)) {
     const Parts x = i < AB / WAVES ? parts(prepared * v[i][0], prepared * v[i][1]) : parts(v[i][0], v[i][1]);
@@ -722,30 +731,58 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
     // this stage's parts are there and the other buffer's have been read; loads into registers stay under way
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
     __builtin_amdgcn_sched_barrier(0);
-    bf16x8 w[TN][3], x[2][3];
+    if constexpr (APART) {
+      bf16x8 w[2][3], x[TM][3];
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int q = 0; q < 3; ++q) w[t][q] = read(buf, AB + wn * TN + t, q);
+        for (int q = 0; q < 3; ++q) x[i][q] = read(buf, wm * TM + i, q);
 #pragma unroll
-    for (int q = 0; q < 3; ++q) x[0][q] = read(buf, wm * TM, q);
+      for (int q = 0; q < 3; ++q) w[0][q] = read(buf, AB + wn * TN, q);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      if (i + 1 < TM) {
+      for (int t = 0; t < TN; ++t) {
+        if (t + 1 < TN) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) x[(i + 1) & 1][q] = read(buf, wm * TM + i + 1, q);
-      }
-#pragma unroll
-      for (int j = i * LOADS / TM; j < (i + 1) * LOADS / TM; ++j)
-        if (mine(j)) {
-          to_lds(j, buf ^ 1);
-          load(j, s + 2);
+          for (int q = 0; q < 3; ++q) w[(t + 1) & 1][q] = read(buf, AB + wn * TN + t + 1, q);
         }
 #pragma unroll
-      for (int q = 0; q < kProducts; ++q)
+        for (int j = t * LOADS / TN; j < (t + 1) * LOADS / TN; ++j)
+          if (mine(j)) {
+            to_lds(j, buf ^ 1);
+            load(j, s + 2);
+          }
 #pragma unroll
-        for (int t = 0; t < TN; ++t)
-          acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][kPartOfW[q]], x[i & 1][kPartOfX[q]], acc[i][t], 0, 0, 0);
+        for (int q = 0; q < kProducts; ++q)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t & 1][kPartOfW[q]], x[i][kPartOfX[q]], acc[i][t], 0, 0, 0);
+      }
+    } else {
+      bf16x8 w[TN][3], x[2][3];
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) w[t][q] = read(buf, AB + wn * TN + t, q);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) x[0][q] = read(buf, wm * TM, q);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        if (i + 1 < TM) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) x[(i + 1) & 1][q] = read(buf, wm * TM + i + 1, q);
+        }
+#pragma unroll
+        for (int j = i * LOADS / TM; j < (i + 1) * LOADS / TM; ++j)
+          if (mine(j)) {
+            to_lds(j, buf ^ 1);
+            load(j, s + 2);
+          }
+#pragma unroll
+        for (int q = 0; q < kProducts; ++q)
+#pragma unroll
+          for (int t = 0; t < TN; ++t)
+            acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][kPartOfW[q]], x[i & 1][kPartOfX[q]], acc[i][t], 0, 0, 0);
+      }
     }
     end_of_preparing();
     if (--left == 0) end_of_segment();
@@ -777,27 +814,55 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
       for (int t = 0; t < TN; ++t) to[(i * TN + t) * THREADS] = total[i][t];
     return;
   }
-  uint64_t again = 0;   // outputs whose sums are not finite: TM x WT x 4 bits
+  if constexpr (GATE_APART) {   // the gate's wave keeps the first block of rows and gets the factor's sums of it, the other the second
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");   // the last stage's parts have been read
+    floatx4* sums = reinterpret_cast<floatx4*>(lds);
+#pragma unroll
+    for (int t = 0; t < TN; ++t) sums[(wave * TN + t) * kWave + lane] = wn ? total[0][t] : total[1][t];
+    __syncthreads();
+    const int m = m0 + (wm * TM + wn) * 16 + c;
+    if (m >= a.M) return;
+    uint64_t again = 0;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      const int n = n0 + t * 16 + 4 * g;
+      const floatx4 other = sums[((wm + WM * (1 - wn)) * TN + t) * kWave + lane];
+      const floatx4 x = wn ? other : total[0][t], y = wn ? total[1][t] : other;
+      floatx4 z;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (!(finite(x[e]) && finite(y[e]))) again |= 1ull << (t * 4 + e);
+        z[e] = finish<EPI>(a, x[e], y[e]);
+      }
+      if (n < a.N) store4(a, m, n, z);
+    }
+    for (int e = 0; again != 0; ++e, again >>= 1) {
+      const int n = n0 + e / 4 * 16 + 4 * g + e % 4;
+      if ((again & 1) && n < a.N) redo<EPI>(a, m, n);
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int m = m0 + (wm * TM + i) * 16 + c;
     if (m >= a.M) continue;
+    uint64_t again = 0;   // outputs whose sums are not finite: WT x 4 bits
 #pragma unroll
     for (int t = 0; t < WT; ++t) {
       const int n = n0 + (wn * WT + t) * 16 + 4 * g;
       floatx4 y;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float v0 = total[i][t][e], v1 = total[i][EPI == 1 ? t + WT : t][e];
-        if (!(finite(v0) && finite(v1))) again |= 1ull << ((i * WT + t) * 4 + e);
+        const float v0 = total[i][t][e], v1 = total[i][EPI == 1 && !APART ? t + WT : t][e];
+        if (!(finite(v0) && finite(v1))) again |= 1ull << (t * 4 + e);
         y[e] = finish<EPI>(a, v0, v1);
       }
       if (n < a.N) store4(a, m, n, y);
     }
-  }
-  for (int e = 0; again != 0; ++e, again >>= 1) {
-    const int m = m0 + (wm * TM + e / (4 * WT)) * 16 + c, n = n0 + (wn * WT + e / 4 % WT) * 16 + 4 * g + e % 4;
-    if ((again & 1) && n < a.N) redo<EPI>(a, m, n);
+    for (int e = 0; again != 0; ++e, again >>= 1) {
+      const int n = n0 + (wn * WT + e / 4) * 16 + 4 * g + e % 4;
+      if ((again & 1) && n < a.N) redo<EPI>(a, m, n);
+    }
   }
 }
 
@@ -888,8 +953,9 @@ struct Plan {
   bool cut;         // products of parts: the tiles behind the last 256 whole ones
 };
 
-// Whether the products are those of parts: segments of whole stages (a matter of K alone).
-static bool by_parts(int K, int seg) { return K % BK == 0 && seg % BK == 0; }
+// Whether the products are those of parts: segments of whole stages (a matter of K alone but for rows of 64 MB and more apart, whose
+// offsets in a tile take more than 32 bits).
+static bool by_parts(int K, int seg, int64_t lda) { return K % BK == 0 && seg % BK == 0 && K < (1 << 22) && lda < (1 << 24); }
 
 template <int EPI, bool PLANES>
 static void launch_tile(const Args& a, const Plan& plan, int nseg, float* planes, hipStream_t stream) {
@@ -909,14 +975,15 @@ static void launch_tile(const Args& a, const Plan& plan, int nseg, float* planes
 
 template <int EPI, int TM, int TN, int WM, int WAVES>
 static void launch_parts(const Args& a, const Plan& plan, int nseg, float* planes, hipStream_t stream) {
-  constexpr int ROWS = WM * TM * 16, COLS = WAVES / WM * (EPI == 1 ? TN / 2 : TN) * 16, THREADS = WAVES * kWave;
+  constexpr int ROWS = WM * TM * 16, COLS = EPI == 1 ? WAVES / WM * TN * 8 : WAVES / WM * TN * 16, THREADS = WAVES * kWave;
   Share s;
   s.nx = (a.N + COLS - 1) / COLS, s.ny = (a.M + ROWS - 1) / ROWS, s.nseg = nseg, s.planes = planes;
   const int tiles = s.nx * s.ny;
   s.full = plan.cut ? tiles / 256 * 256 : tiles;
   gemm_f32_parts_kernel<EPI, TM, TN, WM, WAVES><<<s.full + (tiles - s.full) * nseg, THREADS, 0, stream>>>(a, s);
-  if (s.full < tiles)
-    gemm_f32_parts_sum_kernel<EPI, TM, TN, WM, WAVES><<<dim3(TM * (EPI == 1 ? TN / 2 : TN), tiles - s.full), THREADS, 0, stream>>>(a, s);
+  if constexpr (EPI != 1 || TN % 2 == 0)
+    if (s.full < tiles)
+      gemm_f32_parts_sum_kernel<EPI, TM, TN, WM, WAVES><<<dim3(TM * (EPI == 1 ? TN / 2 : TN), tiles - s.full), THREADS, 0, stream>>>(a, s);
 }
 
 template <int EPI>
@@ -965,9 +1032,10 @@ static Plan plan_for(int M, int N, int K, int64_t lda, bool gated, int nseg, siz
 }
 
 // The same for products of parts: a round's start, its tiles at the rate that a CU reaches with them, the planes, the weights read
-// once.  The figures are fitted to 18 to 20 ways of each of 17 to 1,024 rows against (9,216 gated, 2,304), (2,304, 9,216),
-// (2,304, 2,048) and (4,096, 2,304) (314 times, 7 % off in the mean square); what is chosen takes 0.6 % more than the best way of
-// each size, 9 % at worst (121.5 us for 114.6 at 180 rows of the gated one).
+// once.  The figures are fitted to 4 to 11 ways of each of 61 to 1,024 rows against (9,216 gated, 2,304), (2,304, 9,216), (2,304, 2,048)
+// and (4,096, 2,304) (346 times, 7 % off in the mean square); what is chosen takes about 1 % more than the best way of each size, 8 % at
+// worst (55.1 us for 51.2 at 300 rows against (4,096, 2,304)).  128 x 288 is there for widths of whole such tiles where rounds of the
+// others are half empty: 509 rows against (2,304, 9,216) 114 us for 144, against (2,304, 2,048) 39 for 47.
 static Plan plan_for_parts(int M, int N, int K, bool gated, int nseg, size_t workspace_bytes) {
   Plan best{16, 16, false};
   if (M <= 16) return best;
@@ -975,8 +1043,8 @@ static Plan plan_for_parts(int M, int N, int K, bool gated, int nseg, size_t wor
     int rows, cols, at_once;   // workgroups of a CU at a time
     double rate, start;        // FLOP a us of a CU, us
   };
-  static const Tile tiles_of[5] = {{64, 128, 2, 0.69e6, 1.2}, {128, 64, 2, 0.73e6, 0.4}, {128, 128, 1, 0.885e6, 1.1}, {128, 192, 1, 0.99e6, 1.5},
-                                   {128, 256, 1, 1.07e6, 1.2}};
+  static const Tile tiles_of[6] = {{64, 128, 2, 0.65e6, 2.0}, {128, 64, 2, 0.66e6, 0.0}, {128, 128, 1, 0.84e6, 1.6}, {128, 192, 1, 0.98e6, 2.3},
+                                   {128, 256, 1, 1.0e6, 1.9}, {128, 288, 1, 0.92e6, 1.6}};
   const double NW = gated ? 2.0 * N : N;
   double best_us = 1e30;
   for (const Tile& t : tiles_of) {
@@ -988,8 +1056,8 @@ static Plan plan_for_parts(int M, int N, int K, bool gated, int nseg, size_t wor
     };
     for (int cut = 0; cut < 2; ++cut) {
       const double rest = cut ? fmod(tiles, 256.0) : 0.0, plane_bytes = rest * nseg * t.rows * t.cols * sizeof(float);
-      if (cut && (rest == 0 || nseg == 1 || plane_bytes > workspace_bytes)) continue;
-      double us = rounds(tiles - rest, tile_us) + rounds(rest * nseg, tile_us / nseg) + 2.0 * plane_bytes / 6.9e6;
+      if (cut && (rest == 0 || nseg == 1 || plane_bytes > workspace_bytes || (gated && t.cols == 288))) continue;   // (no planes of those)
+      double us = rounds(tiles - rest, tile_us) + rounds(rest * nseg, tile_us / nseg) + 2.0 * plane_bytes / 7.9e6 + (cut ? 0.5 : 0.0);
       if (us < NW * K * sizeof(float) / 4.5e6) us = NW * K * sizeof(float) / 4.5e6;
       if (us < best_us) best_us = us, best = Plan{t.rows, t.cols, cut != 0};
     }
@@ -1025,6 +1093,7 @@ static void launch(const Args& a, int nseg, float* workspace, size_t workspace_b
     else if (plan.cols == 64) launch_parts<EPI, 4, 2, 2, 4>(a, plan, nseg, workspace, stream);
     else if (plan.cols == 128) launch_parts<EPI, 4, 2, 2, 8>(a, plan, nseg, workspace, stream);
     else if (plan.cols == 256) launch_parts<EPI, 4, 4, 2, 8>(a, plan, nseg, workspace, stream);
+    else if (plan.cols == 288) launch_parts<EPI, 2, 9, 4, 8>(a, plan, nseg, workspace, stream);
     else if constexpr (EPI != 1) launch_parts<EPI, 4, 3, 2, 8>(a, plan, nseg, workspace, stream);
     return;
   }
@@ -1044,7 +1113,7 @@ int gemm_f32(const float* A, int64_t lda, const float* W, const float* W2, float
   f32::Args a;
   a.A = A, a.W = W, a.W2 = W2, a.C = C, a.lda = lda, a.ldc = ldc, a.M = M, a.N = N, a.K = K, a.act = act, a.cap = cap;
   const int nseg = f32::segments(K, &a.seg);
-  a.parts = f32::by_parts(K, a.seg);
+  a.parts = f32::by_parts(K, a.seg, lda);
   float* ws = static_cast<float*>(workspace);
   if (epi == kEpilogueGated) f32::launch<1>(a, nseg, ws, workspace_bytes, stream);
   else if (epi == kEpilogueSoftCap) f32::launch<2>(a, nseg, ws, workspace_bytes, stream);
@@ -1061,7 +1130,7 @@ extern "C" int sa_gemm_f32_plan(int M, int N, int K, int gated, int64_t workspac
   int length;
   const int nseg = sa::f32::segments(K, &length);
   const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
-  const sa::f32::Plan plan = sa::f32::by_parts(K, length) ? sa::f32::plan_for_parts(M, N, K, gated != 0, nseg, bytes)
+  const sa::f32::Plan plan = sa::f32::by_parts(K, length, K) ? sa::f32::plan_for_parts(M, N, K, gated != 0, nseg, bytes)
                                                           : sa::f32::plan_for(M, N, K, K, gated != 0, nseg, bytes);
   return plan.rows + (plan.cut ? 1000 : 0) + 10000 * plan.cols;
 }

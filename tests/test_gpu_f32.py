@@ -103,10 +103,11 @@ def test_products_of_whole_blocks(M, N, K, gated, tile, cut):
 
 
 @pytest.mark.parametrize("M,N,K,gated,tile,cut", [
-    (17, 1570, 256, False, (64, 128), True), (17, 18433, 160, False, (64, 128), False), (130, 4100, 160, True, (64, 128), False),
-    (65, 18433, 160, False, (128, 64), True), (17, 3135, 160, True, (128, 64), False), (257, 8003, 160, False, (128, 128), False),
+    (17, 1570, 256, True, (64, 128), True), (17, 18433, 160, False, (64, 128), False), (17, 9200, 160, True, (64, 128), False),
+    (65, 18433, 160, False, (128, 64), True), (17, 2300, 160, True, (128, 64), False), (257, 8003, 160, False, (128, 128), False),
     (65, 18433, 992, True, (128, 128), True), (200, 18433, 160, False, (128, 192), False), (65, 4100, 992, False, (128, 192), True),
-    (130, 3135, 992, False, (128, 256), True), (257, 18433, 160, False, (128, 256), False), (1000, 4100, 160, True, (128, 256), True)])
+    (130, 3135, 992, False, (128, 256), True), (257, 18433, 160, False, (128, 256), False), (130, 18433, 992, True, (128, 256), True),
+    (130, 4100, 992, False, (128, 288), True), (1000, 9200, 160, False, (128, 288), False), (1000, 4100, 160, True, (128, 288), False)])
 def test_products_of_parts(M, N, K, gated, tile, cut):
     """K in segments of whole stages of 32 columns (the last one shorter at 992), the products those of bfloat16 parts: every tile, whole,
     cut, and cut behind 256 whole ones, the last rows and columns missing.  Rows and weights of very different sizes: the parts hold
@@ -139,14 +140,14 @@ def test_products_of_parts(M, N, K, gated, tile, cut):
         assert torch.equal(ops.gemm(a[M - 5:], w, soft_cap=2.0), capped[M - 5:])
 
 
-@pytest.mark.parametrize("N", [50, 4100])
-def test_products_of_parts_keep_special_values(N):
+@pytest.mark.parametrize("N,rows", [(50, (3, 16, 40, 200)), (4100, (3, 40, 200, 1000))])
+def test_products_of_parts_keep_special_values(N, rows):
     """An infinite or undefined entry reaches its own row and column only, as in plain 32-bit arithmetic, and entries next to the
     largest number, whose first part is rounded to an infinite one, give the finite sums that they have."""
     from simply_amd.kernels import ops
 
     K, largest = 256, torch.finfo(torch.float32).max
-    for M in (3, 16, 40, 200):
+    for M in rows:
         a, w, up = draw((M, K), 5), draw((N, K), 6), draw((N, K), 7)
         a[1, 70], a[0, 9], w[7, 3], w[20, 9], up[9, 200] = float("inf"), largest, float("nan"), 0.0, float("-inf")
         a[2, 11], w[20, 11] = -largest, 2.0 ** -20
