@@ -569,7 +569,7 @@ class CacheManager:
                                                             torch.from_numpy(g.table[rows]))
         elif dirty:
             if self._stage_host is None:
-                ints = sum(self.num_slots * (g.max_blocks + 3) for g in self.groups)
+                ints = sum(self.num_slots * (g.max_blocks + 1) for g in self.groups)
                 self._stage_host = torch.empty(ints, dtype=torch.int32, pin_memory=True)
                 self._stage_dev = torch.empty(ints, dtype=torch.int32, device=self.device)
                 self._stage_done = torch.cuda.Event()
@@ -578,17 +578,16 @@ class CacheManager:
             at, parts = 0, []
             for g in dirty:
                 rows = sorted(g.dirty_slots)
-                n, body = len(rows), at + 2 * len(rows)  # the rows' numbers as 64-bit integers, then the rows
-                host[at:body].view(np.int64)[:] = rows
+                n, body = len(rows), at + len(rows)   # the rows' numbers, then the rows
+                host[at:body] = rows
                 host[body:body + n * g.max_blocks].reshape(n, g.max_blocks)[:] = g.table[rows]
-                parts.append((g, at, n, body))
+                parts.append((self._device_tables[g.group_id], at, n))
                 at = body + n * g.max_blocks
-                at += at & 1
+            from ..kernels import ops
+
             dev[:at].copy_(self._stage_host[:at], non_blocking=True)
             self._stage_done.record()
-            for g, first, n, body in parts:
-                self._device_tables[g.group_id].index_copy_(0, dev[first:body].view(torch.int64),
-                                                            dev[body:body + n * g.max_blocks].view(n, g.max_blocks))
+            ops.table_rows(dev, parts)
         for g in self.groups:
             g.dirty_slots.clear()
         return self._device_tables

@@ -78,6 +78,10 @@ int sa_decode_advance_slots(int B, int* step_counter, const int* sampled_tokens,
                             float* out_logprobs, int max_steps, const int* token_seq, int num_groups,
                             const int* const* block_tables, const int* table_strides, int64_t* const* slot_mappings,
                             int page_size, hipStream_t stream);
+// Rows of num_groups (at most 4) block tables [heights, widths] from one array on the device: from words[firsts[g]] on, rows[g] row
+// numbers and behind them the rows.  tables, heights, widths, rows and firsts are host arrays of num_groups entries.
+int sa_table_rows(const int* words, int num_words, int num_groups, int* const* tables, const int* heights, const int* widths,
+                  const int* rows, const int* firsts, hipStream_t stream);
 // slot_mapping[b] = block_table[token_seq[b], positions[b] / page_size] * page_size + positions[b] % page_size
 int sa_decode_slots(int B, const int* positions, const int* token_seq, const int* block_table, int table_stride,
                     int page_size, int64_t* slot_mapping, hipStream_t stream);

@@ -10,6 +10,7 @@ import dataclasses
 import time
 from typing import Sequence
 
+import numpy as np
 import torch
 
 from ..config import EngineConfig, load_config
@@ -239,7 +240,7 @@ class LMInterface:
             return []
         if n > self.engine_config.max_seq_len:
             raise ValueError(f"score_tokens: {n} tokens to run, max_seq_len is {self.engine_config.max_seq_len}")
-        ex, dev = self.executor, self.executor.device
+        ex = self.executor
         # logits of a portion: float32 [rows, vocab], 256 MiB at most
         rows = max(1, min(self.engine_config.issue_budget, (64 << 20) // vocab))
         self._num_scored += 1
@@ -250,13 +251,15 @@ class LMInterface:
             for i in range(0, n, rows):
                 part = ids[i:min(i + rows, n)]
                 logits = ex.step([StepEntry(rid, part, list(range(len(part))))])
-                given = torch.tensor(ids[i + 1:i + 1 + len(part)], dtype=torch.int32, device=dev)
-                full = lambda v, dt: torch.full((len(part),), v, dtype=dt, device=dev)
-                out.append(ops.score(logits, full(sp.temperature, torch.float32), full(sp.top_k, torch.int32),
-                                     full(sp.top_p, torch.float32), given))
+                # (what the rows ask for goes over in one copy that does not wait for the model's kernels)
+                asked = np.empty((4, len(part)), dtype=np.int32)
+                asked[0], asked[1].view(np.float32)[:], asked[2].view(np.float32)[:] = sp.top_k, sp.temperature, sp.top_p
+                asked[3] = ids[i + 1:i + 1 + len(part)]
+                top_k, temperature, top_p, given = ex._to_device(asked).unbind(0)
+                out.append(ops.score(logits, temperature.view(torch.float32), top_k, top_p.view(torch.float32), given))
         finally:
             ex.finish_request(rid)
-        return torch.cat(out).tolist()
+        return [score for part in out for score in part.tolist()]
 
 
 LLM = LMInterface

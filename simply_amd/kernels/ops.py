@@ -371,6 +371,22 @@ def decode_slots(positions: torch.Tensor, token_seq: torch.Tensor, block_table: 
               int(page_size), _ptr(slot_mapping), _stream())
 
 
+def table_rows(words: torch.Tensor, parts: "list[tuple[torch.Tensor, int, int]]") -> None:
+    """Puts rows into block tables.  words: int32 on the device; parts: (table, first, n) of each table: from words[first] on, the
+    numbers of n rows and behind them the rows."""
+    _i32(words, "table_rows: words")
+    for table, first, n in parts:
+        _dev(table)
+        if table.dim() != 2 or table.dtype != torch.int32 or not table.is_contiguous():
+            raise KernelError("table_rows: a block table must be contiguous int32 [sequences, blocks]")
+    for i in range(0, len(parts), 4):
+        some = parts[i:i + 4]
+        ints = lambda values: (ctypes.c_int * len(some))(*values)
+        _lib.call("sa_table_rows", _ptr(words), words.numel(), len(some), (ctypes.c_void_p * len(some))(*[t.data_ptr() for t, _, _ in some]),
+                  ints([t.shape[0] for t, _, _ in some]), ints([t.shape[1] for t, _, _ in some]), ints([n for _, _, n in some]),
+                  ints([first for _, first, _ in some]), _stream())
+
+
 # --------------------------------------------------------------------------- matrix products
 
 EPILOGUE_NONE, EPILOGUE_GATED, EPILOGUE_SOFT_CAP, EPILOGUE_ACTIVATED = 0, 1, 2, 3

@@ -104,3 +104,26 @@ def test_norm_and_token_shift(T, D, vectors, centered, add):
     assert ops.add_next_norm_shift(y, mine, w, mu=mu, tails=one[:, 15:], **args) is None      # not aligned
     assert ops.add_next_norm_shift(y, mine, w, mu=mu[:4], tails=one[:, 16:], **args) is None  # not five streams
     assert torch.equal(mine, theirs) and torch.equal(one, two)
+
+
+@pytest.mark.parametrize("widths, rows", [((1,), (1,)), ((512, 3), (4, 0)), ((300, 257, 1, 64, 7), (5, 8, 1, 2, 3))])
+def test_rows_of_block_tables(widths, rows):
+    """Rows of one to five block tables from one array: each in its place, all others as they were."""
+    from simply_amd.kernels import lib, ops
+
+    g = torch.Generator().manual_seed(sum(widths))
+    tables = [torch.randint(-1, 1000, (8, w), generator=g, dtype=torch.int32) for w in widths]
+    words, parts, want, at = [], [], [t.clone() for t in tables], 0
+    for k, (t, n) in enumerate(zip(tables, rows)):
+        places = torch.randperm(8, generator=g, dtype=torch.int32)[:n]
+        new = torch.randint(-1, 1000, (n, t.shape[1]), generator=g, dtype=torch.int32)
+        want[k][places.long()] = new
+        words += [places, new.reshape(-1)]
+        parts.append((t.cuda(), at, n))
+        at += n * (1 + t.shape[1])
+    words = torch.cat(words).cuda()
+    ops.table_rows(words, parts)
+    for (table, _, _), w in zip(parts, want):
+        assert torch.equal(table.cpu(), w)
+    with pytest.raises(lib.KernelError):
+        ops.table_rows(words[:-1], parts[-1:])
