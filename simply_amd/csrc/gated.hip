@@ -290,7 +290,7 @@ struct RowItself {
 };
 // ... or, in a step with one token of every request, only the mixes with the row before it that token_shift_kernel makes (the row
 // rounded to bfloat16 first, as that kernel reads it), and the row becomes the request's last: a launch and a round trip less
-// (8 tokens of 2,048 wide, five mixes: 4.7 + 5.1 us before, 5.2 now).
+// (8 tokens of 2,048 wide, five mixes: 4.7 + 5.1 us before, 4.8 now).
 // Workgroup j has request j.
 template <typename MT>
 struct RowMixed {
