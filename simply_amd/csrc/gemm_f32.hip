@@ -58,8 +58,8 @@ struct Args {
 // Where the 16-byte piece p of row r lies in a tile of rows of 128 bytes (in floats).
 __device__ __forceinline__ int piece_at(int r, int p) { return r * BK + ((p ^ (r & 7)) * 4); }
 
-// Eight numbers, each as the sum of three bfloat16 ones, which hold its 24 bits exactly: the first is the number rounded, the second
-// what that leaves rounded, the third what both leave.
+// Eight numbers, each as the sum of three bfloat16 ones, which hold its 24 bits exactly (see kScale): the first is the number rounded,
+// the second what that leaves rounded, the third what both leave.
 struct Parts {
   bf16x8 p[3];
 };
@@ -107,6 +107,10 @@ constexpr int kPartOfW[kProducts] = {2, 0, 1, 1, 0, 0}, kPartOfX[kProducts] = {0
 // The bfloat16 unit drops what lies below a sum's last bits, towards minus infinity: 0.3 of the root mean square error of a sum of
 // 9,216 products, the same way in every sum.  Every other segment is therefore summed with its sign turned.
 __device__ __forceinline__ float segment_sign(int segment) { return segment % 2 ? -1.f : 1.f; }
+// A bfloat16 ends at 2^-133, and below 2^-126 the unit drops more of a sum's bits: with parts as they come, a sum of numbers around 2^-116
+// would be 2e-6 off, around 2^-126 2e-3.  Both factors are therefore taken 2^24 times as large, which leaves no bit of a 32-bit number,
+// subnormal ones included, below 2^-126; sums are scaled back.  Numbers of 2^104 and more, and sums of 2^80 and more, become infinite.
+constexpr float kScale = 16777216.f, kUnscale = 1.f / kScale / kScale;
 
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
 // Element (m, n) of A . W^T summed in plain 32-bit arithmetic, in segments: where products of parts gave no finite number (parts of
@@ -206,7 +210,8 @@ __global__ __launch_bounds__(64 * kSegments, PARTS ? 4 : 1) void gemm_f32_few_ke
 #pragma unroll
     for (int i = 0; i < AP; ++i) {
       if constexpr (PARTS) {   // a lane's four columns of a row, part by part: [part][column group][row][8]
-        float v[4] = {sign * x[i][0], sign * x[i][1], sign * x[i][2], sign * x[i][3]};
+        const float by = sign * kScale;
+        float v[4] = {by * x[i][0], by * x[i][1], by * x[i][2], by * x[i][3]};
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
           typedef __attribute__((ext_vector_type(2))) uint32_t uint32x2;
@@ -233,8 +238,8 @@ __global__ __launch_bounds__(64 * kSegments, PARTS ? 4 : 1) void gemm_f32_few_ke
       for (int q = 0; q < 3; ++q) x.p[q] = *reinterpret_cast<const bf16x8*>(a_s + q * (AROWS * 16) + (g * AROWS + c % AROWS) * 4);
 #pragma unroll
       for (int v = 0; v < NW; ++v) {
-        const Parts w = parts<true>(*reinterpret_cast<const floatx4*>(w_s + v * 16 * BK + piece_at(c, g)),
-                              *reinterpret_cast<const floatx4*>(w_s + v * 16 * BK + piece_at(c, 4 + g)));
+        const Parts w = parts<true>(kScale * *reinterpret_cast<const floatx4*>(w_s + v * 16 * BK + piece_at(c, g)),
+                                    kScale * *reinterpret_cast<const floatx4*>(w_s + v * 16 * BK + piece_at(c, 4 + g)));
 #pragma unroll
         for (int q = 0; q < kProducts; ++q)
           acc[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.p[kPartOfW[q]], x.p[kPartOfX[q]], acc[v], 0, 0, 0);
@@ -279,7 +284,7 @@ __global__ __launch_bounds__(64 * kSegments, PARTS ? 4 : 1) void gemm_f32_few_ke
   __syncthreads();
   floatx4* sums = reinterpret_cast<floatx4*>(lds);
 #pragma unroll
-  for (int v = 0; v < NW; ++v) sums[(wave * NW + v) * kWave + lane] = PARTS ? sign * acc[v] : acc[v];
+  for (int v = 0; v < NW; ++v) sums[(wave * NW + v) * kWave + lane] = PARTS ? sign * kUnscale * acc[v] : acc[v];
   __syncthreads();
   if (wave != 0) return;
   const int nseg = blockDim.x / kWave;
@@ -690,8 +695,9 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
       from[i] = static_cast<uint32_t>(row < last ? row : last) * static_cast<uint32_t>(a.K) + p * 4;
     }
   }
-  // signs of the segments being summed and being made parts of, and stages that are left of each
-  float summed = segment_sign(segment < 0 ? 0 : segment), prepared = summed;
+  // signs and scales of the segments being summed and being made parts of, and stages that are left of each
+  const float first = segment_sign(segment < 0 ? 0 : segment);
+  float summed = first * kUnscale, prepared = first * kScale;
   int left = per_segment, to_prepare = per_segment;
   floatx4 v[LOADS][2];
   auto load = [&](int i, int s) __attribute__((always_inline)) {   // (behind the last stage: that one again)
@@ -701,7 +707,8 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
     v[i][1] = *reinterpret_cast<const floatx4*>(at + from[i] + 16);
   };
   auto to_lds = [&](int i, int buf) __attribute__((always_inline)) {
-    const Parts x = i < AB / WAVES ? parts(prepared * v[i][0], prepared * v[i][1]) : parts(v[i][0], v[i][1]);
+    const float by = i < AB / WAVES ? prepared : kScale;
+    const Parts x = parts(by * v[i][0], by * v[i][1]);
 #pragma unroll
     for (int q = 0; q < 3; ++q)
       *reinterpret_cast<bf16x8*>(lds + buf * BUF + ((i * WAVES + wave) * 3 + q) * 512 + part_at(r, p)) = x.p[q];

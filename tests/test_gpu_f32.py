@@ -140,6 +140,42 @@ def test_products_of_parts(M, N, K, gated, tile, cut):
         assert torch.equal(ops.gemm(a[M - 5:], w, soft_cap=2.0), capped[M - 5:])
 
 
+@pytest.mark.parametrize("a_exp,w_exp", [(0, 0), (-60, 70), (-112, 60), (-126, 60), (-140, 100), (60, -116), (90, -126)])
+@pytest.mark.parametrize("M,N", [(5, 100), (12, 100), (40, 100), (200, 1000), (300, 4100)])
+def test_products_of_parts_keep_every_bit(M, N, a_exp, w_exp):
+    """One product for each output, of numbers down to the smallest of 32 bits: all bits of both factors count.  The unit drops what lies
+    below the sum's bits (2^-23 of it at most, in the last of the six additions; the others add numbers of 2^-8 and less), the three
+    products of parts that are left out are 2^-25 together: 2^-22.  Two parts of three would miss by up to 2^-16, five products of six by
+    2^-17 and more.  Rows' bits do not depend on how many there are."""
+    from simply_amd.kernels import ops
+
+    K = 256
+    columns = torch.randint(0, K, (M,), generator=torch.Generator().manual_seed(41)).cuda()
+    scaled = lambda x, e: x * 2.0 ** (e // 2) * 2.0 ** (e - e // 2)
+    a, w = torch.zeros((M, K), device="cuda"), scaled(draw((N, K), 42), w_exp)
+    a[torch.arange(M, device="cuda"), columns] = scaled(draw((M,), 43), a_exp)
+    got = ops.gemm(a, w)
+    want = a.double().sum(1)[:, None] * w.double()[:, columns].T
+    assert ((got.double() - want).abs() <= 2.0 ** -22 * want.abs() + 2.0 ** -149).all()
+    for rows in (slice(0, 5), slice(M - 5, M), slice(0, min(M, 16))):
+        assert torch.equal(ops.gemm(a[rows], w), got[rows])
+
+
+@pytest.mark.parametrize("K", [2304, 9216])
+@pytest.mark.parametrize("a_exp,w_exp", [(0, 0), (-120, 60), (60, -120)])
+def test_errors_of_products_of_parts(K, a_exp, w_exp):
+    """Errors against 64 bits are no larger than the 32-bit unit's, which takes the same rows with 16 columns of zeros behind them."""
+    from simply_amd.kernels import ops
+
+    a, w = draw((300, K), 51) * 2.0 ** a_exp, draw((500, K), 52, 0.1) * 2.0 ** w_exp
+    want = a.double() @ w.double().T
+    error = lambda y, of: (((y.double() - of) ** 2).sum() / (of ** 2).sum()).sqrt().item()
+    pad = lambda x: torch.nn.functional.pad(x, (0, 16))
+    for M in (4, 12, 300):
+        parts, unit = ops.gemm(a[:M], w), ops.gemm(pad(a[:M]), pad(w))
+        assert error(parts, want[:M]) <= error(unit, want[:M]), M
+
+
 @pytest.mark.parametrize("N,rows", [(50, (3, 16, 40, 200)), (4100, (3, 40, 200, 1000))])
 def test_products_of_parts_keep_special_values(N, rows):
     """An infinite or undefined entry reaches its own row and column only, as in plain 32-bit arithmetic, and entries next to the
