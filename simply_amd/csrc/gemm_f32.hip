@@ -22,6 +22,10 @@
 //   cut tiles   a workgroup per segment; a sum kernel adds the segments' planes: where the tiles alone leave CUs idle.  With parts
 //               only the tiles behind the last 256 whole ones are cut.
 //
+// Products of parts whose sums are no finite numbers are done again on the 32-bit unit, in the workgroup that has them (see redo).  That
+// takes, in us, without / one row / all rows of such: 4 rows against (9,216 gated, 2,304) 37 / 67 / 69, 509 rows 230 / 430 / 1,000, against
+// (2,304, 9,216) 114 / 310 / 860; 4 rows against (256,000, 2,304) 390 / 850 / 820.
+//
 // Measured, weights from HBM; "unit" with the 32-bit matrix unit throughout:
 //   (N, K)                4 rows, unit   61 rows, unit    509 rows, unit    1,024 rows, unit
 //   (2304, 9216)          21.8, 21.7     40, 46           114, 176          227, 333
@@ -29,6 +33,8 @@
 //   (4096, 2304)          10.6, 10.7     18.0, 19.0       67, 87            104, 156
 //   (9216 gated, 2304)    36, 43         61, 64           210, 329          435, 635 (200 TFLOP/s)
 //   (256000, 2304)        378, 392 (6.2 TB/s)
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -113,20 +119,6 @@ __device__ __forceinline__ float segment_sign(int segment) { return segment % 2 
 constexpr float kScale = 16777216.f, kUnscale = 1.f / kScale / kScale;
 
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
-// Element (m, n) of A . W^T summed in plain 32-bit arithmetic, in segments: where products of parts gave no finite number (parts of
-// an infinite entry have opposite signs, and an entry next to the largest number is rounded to an infinite part).
-__device__ __forceinline__ float plain_sum(const Args& a, const float* W, int m, int n) {
-  const float* x = a.A + static_cast<size_t>(m) * a.lda;
-  const float* w = W + static_cast<size_t>(n) * a.K;
-  float total = 0.f;
-  for (int k = 0; k < a.K; k += a.seg) {
-    float sum = 0.f;
-    for (int i = k; i < a.K && i < k + a.seg; ++i) sum = fmaf(x[i], w[i], sum);
-    total += sum;
-  }
-  return total;
-}
-
 template <int EPI>
 __device__ __forceinline__ float finish(const Args& a, float x, float y) {
   if (EPI == 1) return gated_product_exact(a.act, a.cap, x, y);
@@ -145,11 +137,55 @@ __device__ __forceinline__ void store4(const Args& a, int m, int n, floatx4 v) {
   }
 }
 
-// An output whose products of parts gave no finite number.
-template <int EPI>
-__device__ __forceinline__ void redo(const Args& a, int m, int n) {
-  const float x = plain_sum(a, a.W, m, n);
-  a.C[static_cast<size_t>(m) * a.ldc + n] = finish<EPI>(a, x, EPI == 1 ? plain_sum(a, a.W2, m, n) : x);
+// Sums of NB blocks of 16 weight rows (w: lane c's row of each, from its columns 4 g on) with 16 rows (x likewise), over the columns from
+// k0 to k1, on the 32-bit matrix unit and in this file's order for it, added to `total`.
+template <int NB>
+__device__ __forceinline__ void plain_segment(const float* x, const float* const (&w)[NB], int k0, int k1, floatx4 (&total)[NB]) {
+  floatx4 acc[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int k = k0; k < k1; k += 16) {
+    const floatx4 xv = *reinterpret_cast<const floatx4*>(x + k);
+    floatx4 wv[NB];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) wv[t] = *reinterpret_cast<const floatx4*>(w[t] + k);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < NB; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[t][j], xv[j], acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < NB; ++t) total[t] += acc[t];
+}
+// Where the numbers of row m of A (of output n's weights) begin that lane group g multiplies; behind the last: the last.
+__device__ __forceinline__ const float* row_of(const float* rows, int64_t stride, int i, int count, int g) {
+  return rows + static_cast<size_t>(i < count ? i : count - 1) * stride + 4 * g;
+}
+
+// Products of parts give no finite number where a part is infinite (an infinite entry's have opposite signs, and entries of 2^104 and
+// more, scaled, are) or a sum is.  A wave that has such outputs does its NB blocks of 16 x 16 from row m0 and output n0 on once more on the
+// 32-bit unit and stores those outputs: `again` has the bit 4 t + e for output 4 g + e of block t.  (The whole wave comes here.)
+template <int EPI, int NB>
+__device__ __forceinline__ void redo(const Args& a, int m0, int n0, uint64_t again) {
+  constexpr int SUMS = EPI == 1 ? 2 * NB : NB;
+  if (__ballot(again != 0) == 0) return;
+  const int lane = threadIdx.x % kWave, c = lane % 16, g = lane / 16;
+  const float* const x = row_of(a.A, a.lda, m0 + c, a.M, g);
+  const float* w[SUMS];
+  floatx4 total[SUMS];
+#pragma unroll
+  for (int t = 0; t < SUMS; ++t) {
+    w[t] = row_of(t < NB ? a.W : a.W2, a.K, n0 + t % NB * 16 + c, a.N, g);
+    total[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int k = 0; k < a.K; k += a.seg) plain_segment<SUMS>(x, w, k, a.K - k < a.seg ? a.K : k + a.seg, total);
+  float* const out = a.C + static_cast<size_t>(m0 + c) * a.ldc + n0 + 4 * g;   // (lanes without a bit: not used)
+#pragma unroll
+  for (int t = 0; t < NB; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if ((again >> (4 * t + e)) & 1) out[t * 16 + e] = finish<EPI>(a, total[t][e], total[EPI == 1 ? NB + t : t][e]);
 }
 
 // blockDim: a wave per segment.  AROWS: rows of A that are read (8 or 16).
@@ -160,6 +196,7 @@ template <int EPI, int AROWS, bool PARTS>
 __global__ __launch_bounds__(64 * kSegments, PARTS ? 4 : 1) void gemm_f32_few_kernel(Args a) {
   constexpr int NW = EPI == 1 ? 2 : 1, AP = AROWS / 8, D = PARTS && (EPI == 1 || AROWS == 16) ? 2 : 4;   // stages ahead
   constexpr int TOGETHER = PARTS && EPI != 1 && AROWS == 8 ? 2 : 1;   // stages whose products run side by side
+  constexpr bool BUFFERS = TOGETHER == 2;
   constexpr int kAFloats = PARTS ? AROWS * BK * 3 / 2 : AROWS * BK;
   constexpr int kStageFloats = NW * 16 * BK + kAFloats, kWaveFloats = TOGETHER * kStageFloats;
   __shared__ __align__(16) float lds[kSegments * kWaveFloats];
@@ -169,31 +206,51 @@ __global__ __launch_bounds__(64 * kSegments, PARTS ? 4 : 1) void gemm_f32_few_ke
   const int k0 = wave * a.seg;
   const int k1 = a.K - k0 < a.seg ? a.K : k0 + a.seg;
   const int ns = (k1 - k0 + BK - 1) / BK;
-  const float* wp[NW][2];
-  const float* ap[AP];
+  // Where a lane's rows begin.  BUFFERS (K < 4 Mi, rows less than 16 Mi apart): in bytes behind what all lanes share, for loads that add
+  // the stage's columns, a scalar, themselves, where the vector unit has enough to do (256,000 outputs of 4 rows 387 us for 450; with 9 to
+  // 16 rows the other kind is the faster one, 26 us for 30 against (2,304, 9,216)).
+  using Rows = std::conditional_t<BUFFERS, int, const float*>;
+  Rows wp[NW][2], ap[AP];
+  const int here = a.N - n0 < 16 ? a.N - n0 : 16;
+  const size_t tile = static_cast<size_t>(n0) * a.K;
+  auto buffer = [](const float* p, int rows, int64_t stride, int K) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, static_cast<int>(((rows - 1) * stride + K) * 4), 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t w_buffer = buffer(a.W + tile, BUFFERS ? here : 1, a.K, a.K), a_buffer = buffer(a.A, BUFFERS ? a.M : 1, a.lda, a.K);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int n = n0 + 8 * i + r;
-    const size_t at = static_cast<size_t>(n < a.N ? n : a.N - 1) * a.K;
-    wp[0][i] = a.W + at;
-    if (NW == 2) wp[NW - 1][i] = a.W2 + at;
+    const int n = 8 * i + r < here ? 8 * i + r : here - 1;
+    if constexpr (BUFFERS) {
+      wp[0][i] = (n * a.K + p * 4) * 4;
+    } else {
+      wp[0][i] = a.W + tile + static_cast<size_t>(n) * a.K;
+      if (NW == 2) wp[NW - 1][i] = a.W2 + tile + static_cast<size_t>(n) * a.K;
+    }
   }
 #pragma unroll
   for (int i = 0; i < AP; ++i) {
-    const int m = 8 * i + r;
-    ap[i] = a.A + static_cast<size_t>(m < a.M ? m : a.M - 1) * a.lda;
+    const int m = 8 * i + r < a.M ? 8 * i + r : a.M - 1;
+    if constexpr (BUFFERS) ap[i] = (m * static_cast<int>(a.lda) + p * 4) * 4;
+    else ap[i] = a.A + static_cast<size_t>(m) * a.lda;
   }
   floatx4 wv[D][NW][2], av[D][AP];
   auto load = [&](floatx4 (&w)[NW][2], floatx4 (&x)[AP], int s) __attribute__((always_inline)) {
     // (behind the segment's last stage: that one again; columns behind its end: its first ones, replaced by zeros below)
-    int k = k0 + (s < ns ? s : ns - 1) * BK + p * 4;
-    if (!PARTS) k = k < k1 ? k : k0;
+    const int at = k0 + (s < ns ? s : ns - 1) * BK;
+    if constexpr (BUFFERS) {
 #pragma unroll
-    for (int v = 0; v < NW; ++v)
+      for (int i = 0; i < 2; ++i) w[0][i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(w_buffer, wp[0][i], at * 4, 0));
 #pragma unroll
-      for (int i = 0; i < 2; ++i) w[v][i] = *reinterpret_cast<const floatx4*>(wp[v][i] + k);
+      for (int i = 0; i < AP; ++i) x[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(a_buffer, ap[i], at * 4, 0));
+    } else {
+      const int k = PARTS || at + p * 4 < k1 ? at + p * 4 : k0;
 #pragma unroll
-    for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const floatx4*>(ap[i] + k);
+      for (int v = 0; v < NW; ++v)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) w[v][i] = *reinterpret_cast<const floatx4*>(wp[v][i] + k);
+#pragma unroll
+      for (int i = 0; i < AP; ++i) x[i] = *reinterpret_cast<const floatx4*>(ap[i] + k);
+    }
   };
   floatx4 acc[NW];
 #pragma unroll
@@ -283,29 +340,68 @@ __global__ __launch_bounds__(64 * kSegments, PARTS ? 4 : 1) void gemm_f32_few_ke
     }
   __syncthreads();
   floatx4* sums = reinterpret_cast<floatx4*>(lds);
-#pragma unroll
-  for (int v = 0; v < NW; ++v) sums[(wave * NW + v) * kWave + lane] = PARTS ? sign * kUnscale * acc[v] : acc[v];
-  __syncthreads();
-  if (wave != 0) return;
+  int* const infinite = reinterpret_cast<int*>(sums + kSegments * NW * kWave);   // of each segment: whether some sum of it is no finite number
   const int nseg = blockDim.x / kWave;
-  floatx4 t[NW];
+  auto put = [&](const floatx4 (&t)[NW]) __attribute__((always_inline)) {
 #pragma unroll
-  for (int v = 0; v < NW; ++v) t[v] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int z = 0; z < nseg; ++z)
+    for (int v = 0; v < NW; ++v) sums[(wave * NW + v) * kWave + lane] = t[v];
+  };
+  auto added = [&](floatx4 (&t)[NW]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int v = 0; v < NW; ++v) t[v] += sums[(z * NW + v) * kWave + lane];
-  if (c >= a.M || n0 + 4 * g >= a.N) return;
-  floatx4 y;
+    for (int v = 0; v < NW; ++v) t[v] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < nseg; ++z)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) y[i] = finish<EPI>(a, t[0][i], t[NW - 1][i]);
-  store4(a, c, n0 + 4 * g, y);
+      for (int v = 0; v < NW; ++v) t[v] += sums[(z * NW + v) * kWave + lane];
+  };
   if constexpr (PARTS) {
-    int again = 0;
+    bool all = true;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) {
+      acc[v] = sign * kUnscale * acc[v];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) all = all && finite(acc[v][i]);
+    }
+    const bool some = __ballot(!all) != 0;
+    if (lane == 0) infinite[wave] = some;
+  }
+  put(acc);
+  __syncthreads();
+  const bool stores = wave == 0 && c < a.M && n0 + 4 * g < a.N;
+  floatx4 t[NW], y;
+  int again = 0;
+  if (wave == 0) {
+    added(t);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      y[i] = finish<EPI>(a, t[0][i], t[NW - 1][i]);
+      if (!(finite(t[0][i]) && finite(t[NW - 1][i]))) again |= 1 << i;
+    }
+    if (stores) store4(a, c, n0 + 4 * g, y);
+  }
+  if constexpr (PARTS) {   // (see redo; here a wave has its segment)
+    int some = 0;
+    for (int z = 0; z < nseg; ++z) some |= infinite[z];
+    if (some == 0) return;
+    int at = tid;
+    asm("" : "+v"(at));
+    const int cc = at % 16, gg = at % kWave / 16;
+    const float* const x = row_of(a.A, a.lda, cc, a.M, gg);
+    const float* w[NW];
+#pragma unroll
+    for (int v = 0; v < NW; ++v) {
+      w[v] = row_of(v == 0 ? a.W : a.W2, a.K, n0 + cc, a.N, gg);
+      t[v] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    plain_segment<NW>(x, w, k0, k1, t);
+    __syncthreads();   // (the sums of parts have been read)
+    put(t);
+    __syncthreads();
+    if (!stores) return;
+    added(t);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (!(finite(t[0][i]) && finite(t[NW - 1][i]))) again |= 1 << i;
-    for (int i = 0; again != 0; ++i, again >>= 1)
-      if ((again & 1) && n0 + 4 * g + i < a.N) redo<EPI>(a, c, n0 + 4 * g + i);
+      if (((again >> i) & 1) && n0 + 4 * g + i < a.N)
+        a.C[static_cast<size_t>(c) * a.ldc + n0 + 4 * g + i] = finish<EPI>(a, t[0][i], t[NW - 1][i]);
   }
 }
 
@@ -652,8 +748,9 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
   // other factor's, and the two exchange half of their sums at the end.  Such tiles' weight parts are read block by block.
   constexpr bool APART = TN % 2 == 1 && TN > 4, GATE_APART = EPI == 1 && APART;
   constexpr int WT = EPI == 1 && !APART ? TN / 2 : TN;   // blocks of outputs across of a wave
+  constexpr int AGAIN = APART ? 3 : WT;                  // of them done again at a time
   static_assert(EPI != 1 || TN % 2 == 0 || (APART && WN == 2 && TM == 2), "gate and factor in one wave, or in two beside each other");
-  static_assert(AB % WAVES == 0, "a wave's first blocks are A's");
+  static_assert(AB % WAVES == 0 && WT % AGAIN == 0, "a wave's first blocks are A's");
   __shared__ __align__(16) __bf16 lds[2 * BUF];
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave % WM, wn = wave / WM, c = lane % 16, g = lane / 16;
@@ -828,7 +925,6 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
     for (int t = 0; t < TN; ++t) sums[(wave * TN + t) * kWave + lane] = wn ? total[0][t] : total[1][t];
     __syncthreads();
     const int m = m0 + (wm * TM + wn) * 16 + c;
-    if (m >= a.M) return;
     uint64_t again = 0;
 #pragma unroll
     for (int t = 0; t < TN; ++t) {
@@ -838,22 +934,20 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
       floatx4 z;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        if (!(finite(x[e]) && finite(y[e]))) again |= 1ull << (t * 4 + e);
+        if (m < a.M && n + e < a.N && !(finite(x[e]) && finite(y[e]))) again |= 1ull << (t * 4 + e);
         z[e] = finish<EPI>(a, x[e], y[e]);
       }
-      if (n < a.N) store4(a, m, n, z);
+      if (m < a.M && n < a.N) store4(a, m, n, z);
     }
-    for (int e = 0; again != 0; ++e, again >>= 1) {
-      const int n = n0 + e / 4 * 16 + 4 * g + e % 4;
-      if ((again & 1) && n < a.N) redo<EPI>(a, m, n);
-    }
+    for (int t = 0; t < TN; t += AGAIN) redo<EPI, AGAIN>(a, m0 + (wm * TM + wn) * 16, n0 + t * 16, again >> (4 * t) & ((1ull << (4 * AGAIN)) - 1));
     return;
   }
+  uint64_t again[TM];   // outputs whose sums are not finite: WT x 4 bits
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
     const int m = m0 + (wm * TM + i) * 16 + c;
+    again[i] = 0;
     if (m >= a.M) continue;
-    uint64_t again = 0;   // outputs whose sums are not finite: WT x 4 bits
 #pragma unroll
     for (int t = 0; t < WT; ++t) {
       const int n = n0 + (wn * WT + t) * 16 + 4 * g;
@@ -861,15 +955,19 @@ __global__ __launch_bounds__(WAVES * kWave, 2) void gemm_f32_parts_kernel(Args a
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float v0 = total[i][t][e], v1 = total[i][EPI == 1 && !APART ? t + WT : t][e];
-        if (!(finite(v0) && finite(v1))) again |= 1ull << (t * 4 + e);
+        if (n + e < a.N && !(finite(v0) && finite(v1))) again[i] |= 1ull << (t * 4 + e);
         y[e] = finish<EPI>(a, v0, v1);
       }
       if (n < a.N) store4(a, m, n, y);
     }
-    for (int e = 0; again != 0; ++e, again >>= 1) {
-      const int n = n0 + (wn * WT + e / 4) * 16 + 4 * g + e % 4;
-      if ((again & 1) && n < a.N) redo<EPI>(a, m, n);
-    }
+  }
+#pragma unroll 1
+  for (int i = 0; i < TM; ++i) {
+    uint64_t of_row = 0;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) of_row = j == i ? again[j] : of_row;
+    for (int t = 0; t < WT; t += AGAIN)
+      redo<EPI, AGAIN>(a, m0 + (wm * TM + i) * 16, n0 + (wn * WT + t) * 16, of_row >> (4 * t) & ((1ull << (4 * AGAIN)) - 1));
   }
 }
 
@@ -883,7 +981,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_f32_parts_sum_kernel(Args 
   const int i = blockIdx.x / WT, t = blockIdx.x % WT;
   const Tile tile = tile_at(share, share.full + blockIdx.y);
   const int m = tile.y * (WM * TM * 16) + (wm * TM + i) * 16 + c, n = tile.x * (WN * WT * 16) + (wn * WT + t) * 16 + 4 * g;
-  if (m >= a.M || n >= a.N) return;
+  const bool stores = m < a.M && n < a.N;
   const floatx4* from = reinterpret_cast<const floatx4*>(share.planes) +
                         (static_cast<size_t>(blockIdx.y) * share.nseg * (TM * TN) + i * TN + t) * THREADS + tid;
   floatx4 v[kSegments][EPI == 1 ? 2 : 1];
@@ -900,15 +998,14 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_f32_parts_sum_kernel(Args 
       x += v[z][0];
       if constexpr (EPI == 1) y += v[z][1];
     }
-  int again = 0;
+  uint64_t again = 0;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    if (!(finite(x[e]) && finite(y[e]))) again |= 1 << e;
+    if (stores && n + e < a.N && !(finite(x[e]) && finite(y[e]))) again |= 1ull << e;
     to[e] = finish<EPI>(a, x[e], y[e]);
   }
-  store4(a, m, n, to);
-  for (int e = 0; again != 0; ++e, again >>= 1)
-    if ((again & 1) && n + e < a.N) redo<EPI>(a, m, n + e);
+  if (stores) store4(a, m, n, to);
+  redo<EPI, 1>(a, m - c, n - 4 * g, again);
 }
 
 // C = epilogue(sum of the segments' planes, in order), V columns a thread.

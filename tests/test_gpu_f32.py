@@ -203,6 +203,60 @@ def test_products_of_parts_keep_special_values(N, rows):
         assert torch.equal(ops.gemm(a[-2:], w)[:, keep], got[-2:, keep])
 
 
+@pytest.mark.parametrize("M,N,gated", [(5, 100, False), (12, 100, True), (60, 100, True), (200, 4100, False), (300, 4100, True), (600, 2300, False)])
+def test_products_of_parts_of_large_numbers(M, N, gated):
+    """Entries and sums beyond what scaled parts hold, in some rows, weights and segments: the bound on a sum of K 32-bit products, and
+    the bits of rows that are few."""
+    from simply_amd.kernels import ops
+
+    K = 992
+    a, w, w2 = draw((M, K), 61), draw((N, K), 62, 0.1), draw((N, K), 63, 0.1) * 2.0 ** -100
+    a[0] *= 2.0 ** 81
+    a[M // 2, 5:9] *= 2.0 ** 110
+    a[M - 1, 700] = 2.0 ** 126
+    w[N - 2] *= 2.0 ** 30
+    w[3, 980:] *= 2.0 ** 100
+    a[:, 980:] *= 2.0 ** -20
+    kw = dict(w2=w2, activation=ops.ACT_SILU) if gated else {}
+    got, largest = ops.gemm(a, w, **kw), torch.finfo(torch.float32).max
+    x, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    want, bound = x, (K + 2) * EPS * size
+    if gated:
+        up, up_bound = a.double() @ w2.double().T, (K + 2) * EPS * (a.double().abs() @ w2.double().abs().T)
+        want = torch.nn.functional.silu(x) * up
+        bound = 1.1 * bound * up.abs() + x.abs() * up_bound + 8 * EPS * want.abs()
+        size = torch.maximum(size, torch.maximum(want.abs(), a.double().abs() @ w2.double().abs().T))
+    held = size < largest / 2   # (no partial sum on the way can overflow)
+    assert held.any(1).all() and (x.abs() > 2.0 ** 82)[held].any()
+    assert ((got.double() - want).abs()[held] <= bound[held]).all()
+    for rows in (slice(0, 5), slice(M // 2 - 2, M // 2 + 3), slice(M - 5, M), slice(0, min(16, M))):
+        assert torch.equal(ops.gemm(a[rows], w, **kw).nan_to_num(), got[rows].nan_to_num())
+
+
+@pytest.mark.parametrize("M", [4, 16, 509])
+def test_products_of_undefined_rows_take_bounded_time(M):
+    """Rows that are not finite are done again by the matrix unit: less than 20 times as long as others (2 to 8 times are measured; by
+    single lanes it was 110 to 210)."""
+    from simply_amd.kernels import ops
+
+    w, a = draw((2304, 9216), 71, 0.1), draw((M, 9216), 72)
+    b = a.clone()
+    b[:, 5] = float("nan")
+    assert torch.isnan(ops.gemm(b, w)).all()
+
+    def time(x):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for _ in range(10):
+            ops.gemm(x, w)
+        end.record()
+        end.synchronize()
+        return begin.elapsed_time(end)
+
+    time(a)
+    assert time(b) < 20 * max(time(a), time(a))
+
+
 def test_products_keep_special_values():
     """An infinite or undefined entry reaches its own row and column only."""
     from simply_amd.kernels import ops
