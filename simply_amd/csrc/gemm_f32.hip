@@ -1136,10 +1136,15 @@ static Plan plan_for(int M, int N, int K, int64_t lda, bool gated, int nseg, siz
 }
 
 // The same for products of parts: a round's start, its tiles at the rate that a CU reaches with them, the planes, the weights read
-// once.  The figures are fitted to 4 to 11 ways of each of 61 to 1,024 rows against (9,216 gated, 2,304), (2,304, 9,216), (2,304, 2,048)
-// and (4,096, 2,304) (346 times, 7 % off in the mean square); what is chosen takes about 1 % more than the best way of each size, 8 % at
-// worst (55.1 us for 51.2 at 300 rows against (4,096, 2,304)).  128 x 288 is there for widths of whole such tiles where rounds of the
-// others are half empty: 509 rows against (2,304, 9,216) 114 us for 144, against (2,304, 2,048) 39 for 47.
+// once.  The figures of tiles of 64 x 128 and more are fitted to 4 to 11 ways of each of 61 to 1,024 rows against (9,216 gated, 2,304),
+// (2,304, 9,216), (2,304, 2,048) and (4,096, 2,304), those of the small tiles to 17 to 4,096 rows against these and 27 other weights of
+// 256 to 18,433 rows and K of 160 to 14,336.  128 x 288 is there for widths of whole such tiles where rounds of the others are half empty:
+// 509 rows against (2,304, 9,216) 114 us for 144, against (2,304, 2,048) 39 for 47.
+// Small tiles: of 64 x 64 for narrow weights (up to 3,072 rows), where larger ones leave CUs idle (17 rows against (1,024, 4,096) 16 us
+// for 22, 1,024 against (512, 256) 9 for 17, 1,024 against (1,024, 1,024) 25 for 31), of 32 rows, cut, for what fills no more (17 rows
+// against (9,216 gated, 2,304) 50 us for 59, (14,336 gated, 3,584) 98 for 118, (8,192, 3,584) 30 for 37).  What is chosen takes
+// about 2 % more than the best way of each of these sizes.  Not for wide weights with K of 256 and less, whose tiles are
+// chosen as before, though smaller ones would be ahead there (100 rows against (1,570 gated, 256): 10.5 us for 16).
 static Plan plan_for_parts(int M, int N, int K, bool gated, int nseg, size_t workspace_bytes) {
   Plan best{16, 16, false};
   if (M <= 16) return best;
@@ -1147,20 +1152,26 @@ static Plan plan_for_parts(int M, int N, int K, bool gated, int nseg, size_t wor
     int rows, cols, at_once;   // workgroups of a CU at a time
     double rate, start;        // FLOP a us of a CU, us
   };
-  static const Tile tiles_of[6] = {{64, 128, 2, 0.65e6, 2.0}, {128, 64, 2, 0.66e6, 0.0}, {128, 128, 1, 0.84e6, 1.6}, {128, 192, 1, 0.98e6, 2.3},
-                                   {128, 256, 1, 1.0e6, 1.9}, {128, 288, 1, 0.92e6, 1.6}};
+  static const Tile tiles_of[9] = {{64, 128, 2, 0.65e6, 2.0}, {128, 64, 2, 0.66e6, 0.0}, {128, 128, 1, 0.84e6, 1.6}, {128, 192, 1, 0.98e6, 2.3},
+                                   {128, 256, 1, 1.0e6, 1.9}, {128, 288, 1, 0.92e6, 1.6}, {64, 64, 3, 0.59e6, 0.5},  {32, 64, 4, 0.38e6, 0.15},
+                                   {32, 128, 2, 0.38e6, 2.2}};
   const double NW = gated ? 2.0 * N : N;
+  const bool narrow = NW <= 3072, one_stage = K <= kSegments * BK;   // (segments of one stage)
+  const bool few_tiles = narrow && one_stage && ceil(M / 64.0) * ceil(NW / 64.0) <= 512;
   double best_us = 1e30;
   for (const Tile& t : tiles_of) {
+    const bool rows_of_32 = t.rows == 32, of_64 = t.rows == 64 && t.cols == 64;
     if (gated && t.cols == 192) continue;   // (three blocks of a wave)
+    if (rows_of_32 ? M > 32 || (one_stage && !narrow) || NW > 255.0 * t.cols : of_64 ? !narrow : few_tiles) continue;
     const double tiles = ceil(M / static_cast<double>(t.rows)) * ceil(NW / t.cols), tile_us = 2.0 * t.rows * t.cols * K / t.rate;
     auto rounds = [&](double workgroups, double us) {
       const double of_a_cu = ceil(workgroups / 256.0);
       return of_a_cu * us + ceil(of_a_cu / t.at_once) * t.start;
     };
-    for (int cut = 0; cut < 2; ++cut) {
+    for (int cut = rows_of_32; cut < 2; ++cut) {   // (whole, they have too little of the weights under way)
       const double rest = cut ? fmod(tiles, 256.0) : 0.0, plane_bytes = rest * nseg * t.rows * t.cols * sizeof(float);
       if (cut && (rest == 0 || nseg == 1 || plane_bytes > workspace_bytes || (gated && t.cols == 288))) continue;   // (no planes of those)
+      if (one_stage && rest * nseg > 256.0) continue;   // (not worth a second workgroup of a CU: 509 rows against (512, 256) 8.7 us for 11)
       double us = rounds(tiles - rest, tile_us) + rounds(rest * nseg, tile_us / nseg) + 2.0 * plane_bytes / 7.9e6 + (cut ? 0.5 : 0.0);
       if (us < NW * K * sizeof(float) / 4.5e6) us = NW * K * sizeof(float) / 4.5e6;
       if (us < best_us) best_us = us, best = Plan{t.rows, t.cols, cut != 0};
@@ -1193,7 +1204,10 @@ static void launch(const Args& a, int nseg, float* workspace, size_t workspace_b
     return;
   }
   if (a.parts) {
-    if (plan.rows == 64) launch_parts<EPI, 2, 4, 2, 4>(a, plan, nseg, workspace, stream);
+    if (plan.rows == 32 && plan.cols == 64) launch_parts<EPI, 2, 2, 1, 2>(a, plan, nseg, workspace, stream);
+    else if (plan.rows == 32) launch_parts<EPI, 2, 4, 1, 2>(a, plan, nseg, workspace, stream);
+    else if (plan.rows == 64 && plan.cols == 64) launch_parts<EPI, 2, 2, 2, 4>(a, plan, nseg, workspace, stream);
+    else if (plan.rows == 64) launch_parts<EPI, 2, 4, 2, 4>(a, plan, nseg, workspace, stream);
     else if (plan.cols == 64) launch_parts<EPI, 4, 2, 2, 4>(a, plan, nseg, workspace, stream);
     else if (plan.cols == 128) launch_parts<EPI, 4, 2, 2, 8>(a, plan, nseg, workspace, stream);
     else if (plan.cols == 256) launch_parts<EPI, 4, 4, 2, 8>(a, plan, nseg, workspace, stream);

@@ -140,6 +140,25 @@ def test_products_of_parts(M, N, K, gated, tile, cut):
         assert torch.equal(ops.gemm(a[M - 5:], w, soft_cap=2.0), capped[M - 5:])
 
 
+@pytest.mark.parametrize("M,N,K,gated,tile,cut", [
+    (33, 1001, 992, False, (64, 64), True), (130, 1000, 160, False, (64, 64), True), (40, 520, 992, True, (64, 64), True),
+    (700, 1003, 992, False, (64, 64), False), (300, 1003, 992, True, (64, 64), False), (500, 1530, 160, True, (64, 64), False),
+    (17, 1001, 992, False, (32, 64), True), (20, 4100, 992, True, (32, 64), True), (20, 500, 160, False, (32, 64), True),
+    (31, 18433, 992, False, (32, 128), True), (20, 9200, 992, True, (32, 128), True)])
+def test_products_of_parts_in_small_tiles(M, N, K, gated, tile, cut):
+    """Narrow weights and few rows.  A row that holds an infinite entry is done again by such tiles too."""
+    from simply_amd.kernels import ops
+
+    test_products_of_parts(M, N, K, gated, tile, cut)
+    a, w, w2 = draw((M, K), 34), draw((N, K), 35, 0.1), draw((N, K), 36, 0.1)
+    kw = dict(w2=w2, activation=ops.ACT_SILU) if gated else {}
+    before = ops.gemm(a, w, **kw)
+    a[M - 2, 3] = float("inf")
+    got, others = ops.gemm(a, w, **kw), torch.arange(M, device="cuda") != M - 2
+    assert torch.equal(got[others], before[others]) and not torch.isfinite(ops.gemm(a, w)[M - 2]).any()
+    assert torch.equal(ops.gemm(a[M - 5:], w, **kw).nan_to_num(), got[M - 5:].nan_to_num())
+
+
 @pytest.mark.parametrize("a_exp,w_exp", [(0, 0), (-60, 70), (-112, 60), (-126, 60), (-140, 100), (60, -116), (90, -126)])
 @pytest.mark.parametrize("M,N", [(5, 100), (12, 100), (40, 100), (200, 1000), (300, 4100)])
 def test_products_of_parts_keep_every_bit(M, N, a_exp, w_exp):

@@ -43,6 +43,21 @@ def test_32_bit_attention_of_prompts_fills_the_chip(lib):
     assert [parts(64, 4, 256, None, 509, 8, n * 512 * row) for n in (0, 1, 3, 4)] == [0, 1, 1, 4]
 
 
+def test_32_bit_products_of_narrow_weights_and_few_rows_take_small_tiles(lib):
+    """(M, N, K, gated): where larger tiles took up to twice as long, and the sizes beside them that stay with those."""
+    from simply_amd.kernels import ops
+
+    def tile(M, N, K, gated=False):
+        return (*ops.gemm_f32_tile(M, N, K, gated=gated), ops.gemm_f32_plan(M, N, K, gated=gated)[1])
+
+    assert tile(1024, 512, 256) == tile(509, 512, 256) == tile(300, 1024, 256, True) == tile(1024, 1024, 1024) == (64, 64, False)
+    assert tile(61, 1024, 4096) == tile(100, 512, 256) == tile(61, 1152, 6912) == (64, 64, True)
+    assert tile(17, 9216, 2304, True) == tile(32, 14336, 3584, True) == (32, 128, True)
+    assert tile(17, 2048, 1024) == tile(32, 8192, 3584) == (32, 64, True)
+    assert tile(33, 9216, 2304, True) == (64, 128, True) and tile(509, 2304, 9216) == (128, 288, True)
+    assert tile(509, 9216, 2304, True) == (128, 256, True) and tile(17, 36864, 4608, True)[:2] == (64, 128)
+
+
 @pytest.mark.parametrize("which", ["q", "rows", "weight", "k_pages", "v_pages"])
 def test_latent_rows_look_at_every_buffer_s_alignment(lib, which):
     """Pieces of 16 bytes are read and written at all five: a view that begins elsewhere goes the way of single entries."""
