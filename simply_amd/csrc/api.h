@@ -121,7 +121,9 @@ int sa_gemm_sections(const void* A, int64_t lda, const void* W, void* C, int c_d
 // expects of the three (negative: not eligible).  c_dtype is the output's element type (the wide kernel writes
 // 32-bit results of large products without an epilogue only).  A host function: nothing is launched.
 int sa_gemm_plan(int M, int N, int K, int epilogue, int c_dtype, int64_t workspace_bytes, double* us);
-// Which way the 32-bit matrix-core kernels take M rows: 16 (few rows), or the rows of a tile (64 or 128), plus 1000 where K
+// The wide kernel's tile for them (epilogue 0 or 1): stages * 1000000 + rows * 1000 + weight rows.  A host function.
+int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t workspace_bytes);
+// Which way the 32-bit matrix-core kernels take M rows: 16 (few rows), or the rows of a tile (32, 64 or 128), plus 1000 where K
 // is cut over workgroups, plus 10000 times the weight rows of a tile.  A host function.
 int sa_gemm_f32_plan(int M, int N, int K, int gated, int64_t workspace_bytes);
 int sa_sum_planes(const float* planes, int count, void* C, int c_dtype, int64_t ldc, int M, int N, hipStream_t stream);

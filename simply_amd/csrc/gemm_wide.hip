@@ -462,9 +462,12 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
   // products (measured: 7-9 % faster than one workgroup of twice the tile once every CU has two of them;
   // slower when it has one; from one and a half per CU on it is also the best for few rows of very many weight
   // rows, which are bound by streaming them).  A tile of 128 x 128, whose waves read more of LDS for a product, takes
-  // 1.38 times as long for its size: it pays where it gives every CU work (2,048 rows, us, against 192 x 128:
-  // 2,048 outputs of K = 2,048 22 for 25, of 8,192 74 for 77; 1,024 outputs 18.5 for 22 and 62 for 72; 4,096 rows
-  // against 1,024 outputs of K = 4,096 38 for 41), and not with a second round (2,304 outputs: 35 for 25).
+  // 1.38 times as long for its size, so it is taken in two cases alone.  One round of it is cheaper than one of 192 x 128, however few
+  // tiles that is; measured, us, at 16 to 256 tiles of gated products of 129 to 4,096 rows and 104 to 256 of plain ones of 1,537 to
+  // 4,096: ahead in all 96, by 3 to 38 % (2,048 rows against 2,048 outputs of K = 2,048 20.8 for 23.7, of 8,192 75.5 for 78.5; 1,024 of
+  // 4,096 28.3 for 35.0; gated, 129 rows against 512 of 1,024 11.8 for 14.5, 256 against 1,024 of 4,096 37.5 for 38.9, 256
+  // against 8,192 of 2,048 27.2 for 30.1).  And two rounds of it than one of 256 x 192 (1,664 rows against 4,992 outputs 44.5 for
+  // 46.4); a second round costs more than one of 192 x 128 (2,048 rows against 2,304 outputs: 35 for 25).
   const int NW = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N;
   const int shapes[6][4] = {{2128192, 128, 192, 93}, {2256192, 256, 192, 100}, {3256128, 256, 128, 100},
                             {3128256, 128, 256, 100}, {3192128, 192, 128, 100}, {4128128, 128, 128, 138}};
@@ -588,3 +591,11 @@ double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, s
 }
 
 }  // namespace sa
+
+extern "C" int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t workspace_bytes) {
+  if (M < 1 || N < 1 || K < 1 || epilogue < 0 || epilogue > 1) return 0;
+  int shape = 0, ks = 1;
+  const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
+  sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks);
+  return shape;
+}

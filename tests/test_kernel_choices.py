@@ -58,6 +58,16 @@ def test_32_bit_products_of_narrow_weights_and_few_rows_take_small_tiles(lib):
     assert tile(509, 9216, 2304, True) == (128, 256, True) and tile(17, 36864, 4608, True)[:2] == (64, 128)
 
 
+@pytest.mark.parametrize("M,N,K,gated,shape", [
+    (2048, 1024, 4096, 0, 4128128), (2048, 2048, 2048, 0, 4128128), (1537, 2048, 8192, 0, 4128128), (4096, 1024, 1024, 0, 4128128),
+    (2048, 2304, 2304, 0, 3192128), (1664, 4992, 2048, 0, 4128128), (1664, 5120, 2048, 0, 2256192),
+    (129, 512, 1024, 1, 4128128), (300, 2048, 2048, 1, 4128128), (256, 8192, 2048, 1, 4128128), (384, 8192, 2048, 1, 3192128),
+    (1025, 2048, 1024, 1, 3192128), (2048, 9216, 2304, 1, 2128192), (128, 8192, 2048, 1, 3128128)])
+def test_wide_tiles_of_128_by_128_where_one_round_is_enough(lib, M, N, K, gated, shape):
+    """One round of them in place of one of 192 x 128, or two for one of 256 x 192."""
+    assert lib.sa_gemm_wide_shape(M, N, K, gated, 256 << 20) == shape
+
+
 @pytest.mark.parametrize("which", ["q", "rows", "weight", "k_pages", "v_pages"])
 def test_latent_rows_look_at_every_buffer_s_alignment(lib, which):
     """Pieces of 16 bytes are read and written at all five: a view that begins elsewhere goes the way of single entries."""
