@@ -272,6 +272,11 @@ class Norm(Part):
     #: True if after_sum() exists: a residual sum and this norm of its result in one kernel
     fuses_sum = False
 
+    @property
+    def by_itself(self) -> "Norm":
+        """The norm without what a mixer may have put into its `after_sum` for a step, for kernels that know norms alone."""
+        return self
+
     def after_sum(self, residual: torch.Tensor, y: "torch.Tensor | None", mult: float,
                   out_dtype: torch.dtype) -> torch.Tensor:
         """residual += mult * y (y None: nothing is added; rows may be one row expanded); returns self(residual)."""

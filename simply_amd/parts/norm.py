@@ -58,6 +58,7 @@ class RMSNorm(Norm):
 
     def add_into(self, residual, y, next_norm, out_dtype):
         """residual += self(y) and, fused when the next norm is an RMSNorm too, next_norm(residual)."""
+        next_norm = getattr(next_norm, "by_itself", next_norm)
         if self.mult != 1.0 or isinstance(next_norm, NoNorm):
             # one kernel: the sum, and the residual handed on in the activation type where no norm follows
             hand_on = isinstance(next_norm, NoNorm) and out_dtype != torch.float32

@@ -28,6 +28,10 @@ class ShiftedNorm(Norm):
     def __init__(self, norm, mixer, ctx, cache):
         self.norm, self.mixer, self.ctx, self.cache = norm, mixer, ctx, cache
 
+    @property
+    def by_itself(self):
+        return self.norm
+
     def forward(self, x, out_dtype):
         return self.norm.forward(x, out_dtype)
 
