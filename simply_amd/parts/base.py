@@ -45,6 +45,11 @@ def knows_expert_sums(method):
     return method
 
 
+def is_method(bound, *functions) -> bool:
+    """Whether an object's method is one of these functions: not one of a subclass, nor one that a program put into the object."""
+    return getattr(bound, "__func__", None) in functions
+
+
 @dataclasses.dataclass(frozen=True)
 class MixedRows:
     """In place of normed rows: what the mixer behind the norm has made of them (see above)."""

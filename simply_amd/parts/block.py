@@ -11,7 +11,7 @@ import torch
 
 from ..kernels import ops
 from ..registry import BLOCKS
-from .base import Block, PendingNorm, knows_expert_sums
+from .base import Block, PendingNorm, is_method, knows_expert_sums
 from .norm import NoNorm
 
 #: stands for "no norm follows": the kernel of the last residual sum then hands the stream on in the activation type
@@ -146,7 +146,7 @@ class PreNormBlock(Block):
         """The first norm as the mixer has it in this step, for whoever computes it ahead of `forward`."""
         offer = getattr(self.mixer, "norm_of_step", None)
         norm = self.first_norm()
-        return offer(norm, ctx, cache) if offer is not None and type(self).forward is PreNormBlock.forward else norm
+        return offer(norm, ctx, cache) if offer is not None and is_method(self.forward, PreNormBlock.forward) else norm
 
     @knows_expert_sums
     def _add(self, h, y, norm, dtype):

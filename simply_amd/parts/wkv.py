@@ -15,7 +15,7 @@ import torch
 
 from ..kernels import ops
 from ..registry import MIXERS
-from .base import MixedRows, Mixer, Norm, ParamSpec, StateNeed, as_product_weight, knows_expert_sums
+from .base import MixedRows, Mixer, Norm, ParamSpec, StateNeed, as_product_weight, is_method, knows_expert_sums
 from .linear_state import channel_decay_state
 from .norm import LayerNorm, RMSNorm
 
@@ -82,9 +82,11 @@ class WKV(Mixer):
         return StateNeed((self.state_words + self.hidden_size,), torch.float32)   # S, then the last token's h
 
     def norm_of_step(self, norm, ctx, cache):
-        """`norm`, or in a step with one token of every request that norm with the token shift in its kernel."""
-        known = type(norm).after_sum in (RMSNorm.after_sum, LayerNorm.after_sum) and norm.fuses_sum
-        if known and type(self).forward is WKV.forward and cache.write and ctx.dtype == torch.bfloat16 and ctx.max_q_len == 1 \
+        """`norm`, or in a step with one token of every request that norm with the token shift in its kernel.  (A norm or a mixer
+        whose methods are others than the ones here is left alone, be it by its class or by what a program put in their place.)"""
+        known = norm.fuses_sum and is_method(norm.after_sum, RMSNorm.after_sum, LayerNorm.after_sum) \
+            and is_method(norm.forward, RMSNorm.forward, LayerNorm.forward)
+        if known and is_method(self.forward, WKV.forward) and cache.write and ctx.dtype == torch.bfloat16 and ctx.max_q_len == 1 \
                 and ctx.num_tokens == ctx.num_seqs and ctx.positions.is_cuda:
             return ShiftedNorm(norm, self, ctx, cache)
         return norm
