@@ -405,7 +405,6 @@ int sa_experts_add_next_norm(const float* y, const float* weights, int top, cons
                              int64_t shared_stride, const float* gate, int64_t gate_stride, float mult, float* residual,
                              const void* w, const void* b, int w_dtype, float eps, int plus_one, void* out, int T, int D,
                              hipStream_t stream);
-// _pays: whether it is expected to be faster than the two (host functions, both).
 // What sa_residual_add_next_norm (y bfloat16 rows or null, weights null) or sa_experts_add_next_norm (weights given) followed by
 // sa_token_shift give in a step with one token of every request, w, b and mu of one type: out [T, streams * D] bfloat16 holds the
 // mixes, the normed rows become the requests' tails.
@@ -415,6 +414,7 @@ int sa_add_next_norm_shift(const void* y, int64_t y_stride, const float* weights
                            int64_t tail_stride, const int* seq_meta, void* out, int T, int D, hipStream_t stream);
 int sa_add_next_norm_shift_takes(int D, int streams, const void* y, int64_t y_stride, const void* shared, int64_t shared_stride,
                                  const void* residual, const void* w, const void* b, const void* mu, const void* tails, int64_t tail_stride);
+// sa_experts_add_next_norm_pays: whether it is expected to be faster than the two (host functions, both).
 int sa_experts_add_next_norm_pays(int D, int top);
 int sa_experts_add_next_norm_takes(int D, const void* shared, int64_t shared_stride, const void* residual, const void* w, const void* b);
 

@@ -110,8 +110,9 @@ def test_products_of_whole_blocks(M, N, K, gated, tile, cut):
     (130, 4100, 992, False, (128, 288), True), (1000, 9200, 160, False, (128, 288), False), (1000, 4100, 160, True, (128, 288), False)])
 def test_products_of_parts(M, N, K, gated, tile, cut):
     """K in segments of whole stages of 32 columns (the last one shorter at 992), the products those of bfloat16 parts: every tile, whole,
-    cut, and cut behind 256 whole ones, the last rows and columns missing.  Rows and weights of very different sizes: the parts hold
-    all of a number's 24 bits, so the bounds are those of a sum in 32 bits; the bits are those of the kernel for few rows."""
+    cut, and cut behind 256 whole ones, the last rows and columns missing, rows and weights of very different sizes: the bounds of a sum
+    in 32 bits, and the bits of the kernel for few rows.  (That all 24 bits of every number count is the next tests' matter: two of three
+    parts would stay within these bounds.)"""
     from simply_amd.kernels import ops
 
     assert ops.gemm_f32_tile(M, N, K, gated=gated) == tile and ops.gemm_f32_plan(M, N, K, gated=gated) == (tile[0], cut)

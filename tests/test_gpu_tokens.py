@@ -106,6 +106,31 @@ def test_norm_and_token_shift(T, D, vectors, centered, add):
     assert torch.equal(mine, theirs) and torch.equal(one, two)
 
 
+@pytest.mark.parametrize("add", ["rows", "none", "experts", "gated experts"])
+@pytest.mark.parametrize("T,D,centered,plus_one", [(5, 2048, False, True), (8, 2056, True, False), (3, 4096, False, True), (16, 1000, True, True)])
+def test_norm_and_token_shift_of_requests_in_another_order(T, D, centered, plus_one, add):
+    """Requests whose tokens stand elsewhere in the step than the requests do: sums, norms, mixes and last rows to the bit as the two
+    kernels have them, with a gain of 1 + w, and with a shared feed-forward that a gate weights."""
+    from simply_amd.kernels import ops
+
+    h = draw((T, D), 1).cuda()
+    w, b = (draw((D,), 2 + i, 0.3).bfloat16().cuda() for i in range(2))
+    mu = torch.rand((5, D), generator=torch.Generator().manual_seed(4)).bfloat16().cuda()
+    state = draw((T + 2, D + 24), 5).cuda()
+    row = [(5 * j + 2) % T for j in range(T)] if T % 5 else [(3 * j + 2) % T for j in range(T)]
+    meta = torch.tensor([[(j + 3) % (T + 2), row[j], 1, 9] for j in range(T)], dtype=torch.int32).cuda()
+    assert sorted(row) == list(range(T)) and row != sorted(row)
+    gate = torch.randn((T, 3), generator=torch.Generator().manual_seed(9)).cuda()[:, :1] if add == "gated experts" else None
+    y = {"rows": lambda: draw((T, D), 7).bfloat16().cuda(), "none": lambda: None}.get(
+        add, lambda: ops.ExpertSums(draw((T * 3, D), 8).cuda(), torch.rand((T, 3)).cuda(), draw((T, D), 6).bfloat16().cuda(), gate, torch.bfloat16))()
+    kw = dict(eps=1e-5, mult=0.7, plus_one=plus_one, bias=b if centered else None)
+    mine, theirs, one, two = h.clone(), h.clone(), state.clone(), state.clone()
+    got = ops.add_next_norm_shift(y, mine, w, mu=mu, tails=one[:, 16:], seq_meta=meta, num_seqs=T, **kw)
+    want = ops.token_shift(ops.residual_add_next_norm(y, theirs, w, out_dtype=torch.bfloat16, **kw), mu, two[:, 16:], meta, T, 1)
+    assert torch.equal(got, want) and torch.equal(mine, theirs) and torch.equal(one, two)
+    assert not torch.equal(one, state) and not any(torch.equal(got[0], got[i]) for i in range(1, T))
+
+
 @pytest.mark.parametrize("widths, rows", [((1,), (1,)), ((512, 3), (4, 0)), ((300, 257, 1, 64, 7), (5, 8, 1, 2, 3))])
 def test_rows_of_block_tables(widths, rows):
     """Rows of one to five block tables from one array: each in its place, all others as they were."""
