@@ -14,7 +14,9 @@
 //   a workgroup per unit, key head and chunk, four waves to it, partial results to the workspace, a merge kernel: few units and ranges,
 //   whose chunks are all there is to fill the chip with;
 //   a workgroup per unit, key head and range, partial results and a merge likewise: more of them, longer prompts;
-//   a workgroup per unit and key head that walks through the ranges: many decoding requests, or where the workspace is too small.
+//   a workgroup per unit and key head that walks through the ranges: many decoding requests, units of one or two tokens (more than four
+//   heads a key head), and where the workspace holds no part for every range: an engine's 256 MiB hold those of a portion of 2,048
+//   tokens of 8 heads over 4 key heads of 256, or of 1,024 tokens of 32 heads over 16 of 128, up to 3,840 keys.
 //
 // Keys that some row of the unit does not see get the weight zero.  Where such keys' values are not finite (a zero weight
 // would spread them), their products are taken one key at a time and left out of the rows that do not see it.
@@ -512,8 +514,9 @@ extern "C" int sa_paged_attention_f32_parts(int unit_count, int Kh, int hd, int 
   const int ranges = f32_ranges(window, max_kv_len, max_q_len);
   const int64_t heads = static_cast<int64_t>(unit_count) * Kh;
   const int64_t bytes = heads * ranges * 16 * (hd + f32att::kExtra) * static_cast<int64_t>(sizeof(float));   // a part a range
-  // Prompts (units of four tokens and more; up to four heads a key head have such): a unit sees what lies before it, so units that walk are as slow as the last one's ranges one
-  // after the other, and a chunk is a chain of waits of 10 us that more workgroups cover.  Walked / ranges / chunks in us, heads of 256,
+  // Prompts (units of four tokens and more; up to four heads a key head have such, prompts of more walk as before): a unit sees what lies
+  // before it, so units that walk are as slow as the last one's ranges one after the other, and a chunk is a chain of waits of 10 us that
+  // more workgroups cover.  What the workspace does not hold walks.  Walked / ranges / chunks in us, heads of 256,
   // 4 key heads, by triples (see below): 64 tokens (32) 20 / 20 / 12, behind 2,048 others (288) 186 / 43 / 44; 509 (512) 42 / 38 / 35; 700
   // (1,056) 83 / 62 / 51; behind 512 (1,760) 163 / 97 / 96; 384 behind 2,048 (1,920) 198 / 125 / 124; 1,024 (2,048) 137 / 94 / 95; 509
   // behind 2,048 (2,560) 198 / 154 / 166; 2,048 (8,192) 397 / 274.  16 key heads of 128: 256 (512, one range) 20 / 23 / 25, 512 (2,048)

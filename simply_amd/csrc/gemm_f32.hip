@@ -5,8 +5,9 @@
 // multiples of 32), every number is taken as the sum of three bfloat16 ones, which hold its 24 bits exactly, and a product as the six
 // of them that matter, on v_mfma_f32_16x16x32_bf16: 417 TFLOP/s of whole products at the unit's nominal rate where the 32-bit unit
 // has 157.  Sums are 32-bit in either case, and with the bfloat16 unit's fewer roundings (six for 32 columns where the 32-bit unit
-// has eight) errors against 64 bits are smaller, at every one of the sizes below (root mean square over the result's: 3.7e-7 for 4.5e-7
-// gated, 5.2e-7 for 6.1e-7 at K = 9,216, 2.4e-7 for 2.9e-7 at 2,048).  Elsewhere v_mfma_f32_16x16x4_f32.
+// has eight) errors of a product against 64 bits are smaller, at every one of the sizes below (root mean square over the result's: 3.7e-7
+// for 4.5e-7 gated, 5.2e-7 for 6.1e-7 at K = 9,216, 2.4e-7 for 2.9e-7 at 2,048), down to the smallest 32-bit numbers (see kScale).
+// Elsewhere v_mfma_f32_16x16x4_f32.
 //
 // Every output element is summed in one order whatever M is, so a row's result does not depend on which other rows are in
 // the batch: K is cut into at most eight segments of the same length, a multiple of 16 (the length depends on K alone); a
@@ -17,7 +18,7 @@
 //               whole 128-byte pieces of rows, two to four stages of 32 columns of K ahead in registers; the operand order is made
 //               on the way through LDS (each wave its own part, no barrier in the loop; 16-byte pieces permuted by row, so
 //               that neither side has bank conflicts).
-//   tiles       a workgroup of four or eight waves owns a tile of outputs and walks through all segments, adding a segment's sum to
+//   tiles       a workgroup of two to eight waves owns a tile of outputs and walks through all segments, adding a segment's sum to
 //               its total at the segment's end: bound by the matrix unit and, with parts, the power that it draws.
 //   cut tiles   a workgroup per segment; a sum kernel adds the segments' planes: where the tiles alone leave CUs idle.  With parts
 //               only the tiles behind the last 256 whole ones are cut.
@@ -26,13 +27,18 @@
 // takes, in us, without / one row / all rows of such: 4 rows against (9,216 gated, 2,304) 37 / 67 / 69, 509 rows 230 / 430 / 1,000, against
 // (2,304, 9,216) 114 / 310 / 860; 4 rows against (256,000, 2,304) 390 / 850 / 820.
 //
-// Measured, weights from HBM; "unit" with the 32-bit matrix unit throughout:
-//   (N, K)                4 rows, unit   61 rows, unit    509 rows, unit    1,024 rows, unit
-//   (2304, 9216)          21.8, 21.7     40, 46           114, 176          227, 333
-//   (2304, 2048)          10.6, 10.3     15.6, 19.7       39, 54            68, 104
-//   (4096, 2304)          10.6, 10.7     18.0, 19.0       67, 87            104, 156
-//   (9216 gated, 2304)    36, 43         61, 64           210, 329          435, 635 (200 TFLOP/s)
-//   (256000, 2304)        378, 392 (6.2 TB/s)
+// Measured, us, weights from HBM; "unit" with the 32-bit matrix unit throughout (many launches in a row; clocks differ by 5 to 8 % from one
+// run to the next):
+//   (N, K)                 4 rows, unit   12, unit    17, unit    61, unit    509, unit      1,024, unit
+//   (2304, 2048)           8.6, 8.3       9.2, 9.2    14.7, 15.0  15.6, 16.8  41, 54         73, 104
+//   (2304, 9216)           24.2, 23.9     26.9, 26.0  41, 45      39, 45      122, 175       223, 333
+//   (4096, 2304)           10.2, 9.6      10.2, 10.8  16.1, 17.0  17.4, 18.9  75, 86         107, 155
+//   (9216 gated, 2304)     36.9, 43.7     39.5, 45.2  51, 58      57, 64      218, 329       405, 637 (215 TFLOP/s)
+//   (3584, 14336)          39.4, 39.1     43.6, 43.4  61, 65      61, 67      265, 397       535, 873
+//   (14336 gated, 3584)    79, 87         83, 88      95, 123     117, 127    496, 770       1,014, 1,528
+//   (4608, 36864)          170, 166       195, 189    163, 222    203, 224    863, 1,244     1,702, 2,737
+//   (36864 gated, 4608)    234, 242       241, 250    305, 381    316, 395    1,590, 2,502   3,047, 4,948
+//   (256000, 2304)         393, 400 (6.0 TB/s)  478, 508  541, 650  555, 661  2,830, 4,390   5,490, 8,626
 #include <type_traits>
 
 #include "api.h"
@@ -1139,7 +1145,9 @@ static Plan plan_for(int M, int N, int K, int64_t lda, bool gated, int nseg, siz
 // once.  The figures of tiles of 64 x 128 and more are fitted to 4 to 11 ways of each of 61 to 1,024 rows against (9,216 gated, 2,304),
 // (2,304, 9,216), (2,304, 2,048) and (4,096, 2,304), those of the small tiles to 17 to 4,096 rows against these and 27 other weights of
 // 256 to 18,433 rows and K of 160 to 14,336.  128 x 288 is there for widths of whole such tiles where rounds of the others are half empty:
-// 509 rows against (2,304, 9,216) 114 us for 144, against (2,304, 2,048) 39 for 47.
+// 509 rows against (2,304, 9,216) 114 us for 144, against (2,304, 2,048) 39 for 47.  Gated ones are
+// chosen for odd widths alone: at 24 such sizes, 1,300 to 2,048 rows of 2,064 to 3,283 outputs with K of 512 to 1,536, they are 0.98 to
+// 1.19 times as fast as the best of the others, 1.09 in the mean (2,048 rows of 2,285 outputs, K = 512: 58 us for 70).
 // Small tiles: of 64 x 64 for narrow weights (up to 3,072 rows), where larger ones leave CUs idle (17 rows against (1,024, 4,096) 16 us
 // for 22, 1,024 against (512, 256) 9 for 17, 1,024 against (1,024, 1,024) 25 for 31), of 32 rows, cut, for what fills no more (17 rows
 // against (9,216 gated, 2,304) 50 us for 59, (14,336 gated, 3,584) 98 for 118, (8,192, 3,584) 30 for 37).  What is chosen takes
