@@ -1145,7 +1145,7 @@ static Plan plan_for(int M, int N, int K, int64_t lda, bool gated, int nseg, siz
 // once.  The figures of tiles of 64 x 128 and more are fitted to 4 to 11 ways of each of 61 to 1,024 rows against (9,216 gated, 2,304),
 // (2,304, 9,216), (2,304, 2,048) and (4,096, 2,304), those of the small tiles to 17 to 4,096 rows against these and 27 other weights of
 // 256 to 18,433 rows and K of 160 to 14,336.  128 x 288 is there for widths of whole such tiles where rounds of the others are half empty:
-// 509 rows against (2,304, 9,216) 114 us for 144, against (2,304, 2,048) 39 for 47.  Gated ones are
+// 509 rows against (2,304, 9,216) 136 us for 152, against (2,304, 2,048) 40 for 47.  Gated ones are
 // chosen for odd widths alone: at 24 such sizes, 1,300 to 2,048 rows of 2,064 to 3,283 outputs with K of 512 to 1,536, they are 0.98 to
 // 1.19 times as fast as the best of the others, 1.09 in the mean (2,048 rows of 2,285 outputs, K = 512: 58 us for 70).
 // Small tiles: of 64 x 64 for narrow weights (up to 3,072 rows), where larger ones leave CUs idle (17 rows against (1,024, 4,096) 16 us
