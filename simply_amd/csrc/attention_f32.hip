@@ -521,8 +521,14 @@ extern "C" int sa_paged_attention_f32_parts(int unit_count, int Kh, int hd, int 
   // (1,056) 83 / 62 / 51; behind 512 (1,760) 163 / 97 / 96; 384 behind 2,048 (1,920) 198 / 125 / 124; 1,024 (2,048) 137 / 94 / 95; 509
   // behind 2,048 (2,560) 198 / 154 / 166; 2,048 (8,192) 397 / 274.  16 key heads of 128: 256 (512, one range) 20 / 23 / 25, 512 (2,048)
   // 62 / 52 / 59; 4 of 64: 128 (32) 8.6 / 10.5 / 7.3, 512 (256) 15.3 / 11.3 / 11.4, 16 heads over 4, 1,024 (4,096) 64 / 48 / 58.
+  // A chunk's part is one more for the merge to walk through, so chunks end at six ranges (ranges / chunks: 17 tokens behind 8,000 (384)
+  // 56 / 78, 5 behind 30,000 (472) 96 / 161, 100 behind 2,000 (468) 45 / 52; 64 behind 700 (96) 29 / 23), but where the ranges leave half
+  // of the CUs idle (as below; up to 24 ranges: 118 of 2 tokens over one key head 74 / 150).  Over 1,528 sizes what is chosen takes
+  // 1.5 % more than the best way, 20 % at worst: walking, of heads of 64 and 128 whose units all see two ranges and make whole rounds.
   if (max_q_len >= 4) {
-    if (heads * ranges * 36 <= static_cast<int64_t>(hd) * hd && ranges * f32att::kWaves <= 65535 && bytes * f32att::kWaves <= workspace_bytes)
+    const int64_t triples = heads * ranges;
+    if (((triples * 36 <= static_cast<int64_t>(hd) * hd && ranges <= 6) || (triples <= 128 && ranges <= 24)) &&
+        bytes * f32att::kWaves <= workspace_bytes)
       return f32att::kWaves;
     return ranges > 1 && ranges <= 65535 && bytes <= workspace_bytes ? 1 : 0;
   }

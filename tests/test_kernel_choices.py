@@ -43,6 +43,16 @@ def test_32_bit_attention_of_prompts_fills_the_chip(lib):
     assert [parts(64, 4, 256, None, 509, 8, n * 512 * row) for n in (0, 1, 3, 4)] == [0, 1, 1, 4]
 
 
+def test_32_bit_attention_of_few_tokens_behind_many_goes_by_ranges(lib):
+    """A few units that see many ranges: a part for each chunk would leave the merge four times as many to walk through."""
+    from simply_amd.kernels import ops
+
+    parts = ops.attention_f32_parts
+    assert parts(3, 4, 256, None, 8017, 8) == 1 and parts(1, 4, 256, None, 30005, 5) == 1 and parts(13, 4, 256, None, 2100, 8) == 1
+    assert parts(1, 8, 128, None, 8005, 5) == 1 and parts(1, 1, 128, None, 30005, 5) == 1
+    assert parts(8, 4, 256, None, 1088, 8) == 4 and parts(1, 4, 256, None, 4000, 5) == 4 and parts(16, 4, 64, None, 305, 5) == 4
+
+
 def test_32_bit_products_of_narrow_weights_and_few_rows_take_small_tiles(lib):
     """(M, N, K, gated): where larger tiles took up to twice as long, and the sizes beside them that stay with those."""
     from simply_amd.kernels import ops
