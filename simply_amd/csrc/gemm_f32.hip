@@ -1143,16 +1143,17 @@ static Plan plan_for(int M, int N, int K, int64_t lda, bool gated, int nseg, siz
 
 // The same for products of parts: a round's start, its tiles at the rate that a CU reaches with them, the planes, the weights read
 // once.  The figures of tiles of 64 x 128 and more are fitted to 4 to 11 ways of each of 61 to 1,024 rows against (9,216 gated, 2,304),
-// (2,304, 9,216), (2,304, 2,048) and (4,096, 2,304), those of the small tiles to 17 to 4,096 rows against these and 27 other weights of
+// (2,304, 9,216), (2,304, 2,048) and (4,096, 2,304), those of the small tiles to 17 to 4,096 rows against these and 39 other weights of
 // 256 to 18,433 rows and K of 160 to 14,336.  128 x 288 is there for widths of whole such tiles where rounds of the others are half empty:
 // 509 rows against (2,304, 9,216) 136 us for 152, against (2,304, 2,048) 40 for 47.  Gated ones are
 // chosen for odd widths alone: at 24 such sizes, 1,300 to 2,048 rows of 2,064 to 3,283 outputs with K of 512 to 1,536, they are 0.98 to
 // 1.19 times as fast as the best of the others, 1.09 in the mean (2,048 rows of 2,285 outputs, K = 512: 58 us for 70).
 // Small tiles: of 64 x 64 for narrow weights (up to 3,072 rows), where larger ones leave CUs idle (17 rows against (1,024, 4,096) 16 us
-// for 22, 1,024 against (512, 256) 9 for 17, 1,024 against (1,024, 1,024) 25 for 31), of 32 rows, cut, for what fills no more (17 rows
-// against (9,216 gated, 2,304) 50 us for 59, (14,336 gated, 3,584) 98 for 118, (8,192, 3,584) 30 for 37).  What is chosen takes
-// about 2 % more than the best way of each of these sizes.  Not for wide weights with K of 256 and less, whose tiles are
-// chosen as before, though smaller ones would be ahead there (100 rows against (1,570 gated, 256): 10.5 us for 16).
+// for 22, 1,024 against (512, 256) 9 for 17, 1,024 against (1,024, 1,024) 25 for 31) and for K up to 768 while they make two rounds at
+// most (130 rows against (4,096, 512) 14 us for 20, (3,584, 736) 18 for 26, 100 against (1,570 gated, 256) 10.7 for 15.4), of 32 rows,
+// cut, for what fills no more (17 rows against (9,216 gated, 2,304) 50 us for 59, (14,336 gated, 3,584) 98 for 118, (8,192, 3,584) 30
+// for 37).  Over 436 sizes what is chosen takes 2 % more than the best way.  Not for up to 32 rows of wide weights with K of 256 and
+// less, whose tiles are chosen as before, though smaller ones would be ahead (17 rows against (2,300 gated, 160): 8 us for 10).
 static Plan plan_for_parts(int M, int N, int K, bool gated, int nseg, size_t workspace_bytes) {
   Plan best{16, 16, false};
   if (M <= 16) return best;
@@ -1165,12 +1166,12 @@ static Plan plan_for_parts(int M, int N, int K, bool gated, int nseg, size_t wor
                                    {32, 128, 2, 0.38e6, 2.2}};
   const double NW = gated ? 2.0 * N : N;
   const bool narrow = NW <= 3072, one_stage = K <= kSegments * BK;   // (segments of one stage)
-  const bool few_tiles = narrow && one_stage && ceil(M / 64.0) * ceil(NW / 64.0) <= 512;
+  const bool two_rounds = ceil(M / 64.0) * ceil(NW / 64.0) <= 512;   // of tiles of 64 x 64
   double best_us = 1e30;
   for (const Tile& t : tiles_of) {
     const bool rows_of_32 = t.rows == 32, of_64 = t.rows == 64 && t.cols == 64;
     if (gated && t.cols == 192) continue;   // (three blocks of a wave)
-    if (rows_of_32 ? M > 32 || (one_stage && !narrow) || NW > 255.0 * t.cols : of_64 ? !narrow : few_tiles) continue;
+    if (rows_of_32 ? M > 32 || (one_stage && !narrow) || NW > 255.0 * t.cols : of_64 ? !narrow && !(M > 32 && K <= 768 && two_rounds) : narrow && one_stage && two_rounds) continue;
     const double tiles = ceil(M / static_cast<double>(t.rows)) * ceil(NW / t.cols), tile_us = 2.0 * t.rows * t.cols * K / t.rate;
     auto rounds = [&](double workgroups, double us) {
       const double of_a_cu = ceil(workgroups / 256.0);

@@ -62,6 +62,8 @@ def test_32_bit_products_of_narrow_weights_and_few_rows_take_small_tiles(lib):
 
     assert tile(1024, 512, 256) == tile(509, 512, 256) == tile(300, 1024, 256, True) == tile(1024, 1024, 1024) == (64, 64, False)
     assert tile(61, 1024, 4096) == tile(100, 512, 256) == tile(61, 1152, 6912) == (64, 64, True)
+    assert tile(130, 4096, 512) == tile(256, 2048, 512, True) == tile(130, 3584, 736) == tile(100, 1570, 256, True) == (64, 64, False)
+    assert tile(700, 4096, 512) == (128, 128, False) and tile(130, 3840, 1024)[:2] == (128, 256)
     assert tile(17, 9216, 2304, True) == tile(32, 14336, 3584, True) == (32, 128, True)
     assert tile(17, 2048, 1024) == tile(32, 8192, 3584) == (32, 64, True)
     assert tile(33, 9216, 2304, True) == (64, 128, True) and tile(509, 2304, 9216) == (128, 288, True)
