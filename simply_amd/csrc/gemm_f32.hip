@@ -988,6 +988,7 @@ __global__ __launch_bounds__(WAVES * kWave) void gemm_f32_parts_sum_kernel(Args 
   const Tile tile = tile_at(share, share.full + blockIdx.y);
   const int m = tile.y * (WM * TM * 16) + (wm * TM + i) * 16 + c, n = tile.x * (WN * WT * 16) + (wn * WT + t) * 16 + 4 * g;
   const bool stores = m < a.M && n < a.N;
+  if (__ballot(stores) == 0) return;   // (17 rows gated against (1,570, 256): 10.0 us for 11.6 with the planes of such waves read)
   const floatx4* from = reinterpret_cast<const floatx4*>(share.planes) +
                         (static_cast<size_t>(blockIdx.y) * share.nseg * (TM * TN) + i * TN + t) * THREADS + tid;
   floatx4 v[kSegments][EPI == 1 ? 2 : 1];
