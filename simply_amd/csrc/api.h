@@ -123,6 +123,9 @@ int sa_gemm_sections(const void* A, int64_t lda, const void* W, void* C, int c_d
 int sa_gemm_plan(int M, int N, int K, int epilogue, int c_dtype, int64_t workspace_bytes, double* us);
 // The wide kernel's tile for them (epilogue 0 or 1): stages * 1000000 + rows * 1000 + weight rows.  A host function.
 int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t workspace_bytes);
+// Where the broad kernel takes its place (output rows of whole 16-byte pieces): cuts of K * 1000000 + rows * 1000 + weight rows of
+// a tile, else 0.  A host function.
+int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t workspace_bytes);
 // Which way the 32-bit matrix-core kernels take M rows: 16 (few rows), or the rows of a tile (32, 64 or 128), plus 1000 where K
 // is cut over workgroups, plus 10000 times the weight rows of a tile.  A host function.
 int sa_gemm_f32_plan(int M, int N, int K, int gated, int64_t workspace_bytes);
@@ -275,6 +278,9 @@ bool gemm_skinny_takes(int M, int N, int K, int64_t lda, const void* A, const vo
 // the arguments.
 double gemm_skinny_predict_us(int M, int N, int K, int epi);
 double gemm_tiled_predict_us(int M, int N, int K, int epi);
+double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks);
+void gemm_broad(int tile, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int epi,
+                int act, float limit, int ks, float* partials, bool raw, hipStream_t stream);
 double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes);
 // The experts' products on the wide kernel (plan, sorted: of the sort kernel with tiles of tile_rows rows, 64 or 128).
 bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t ldc, const void* A, const void* W, const void* W2,

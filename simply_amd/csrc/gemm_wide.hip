@@ -28,7 +28,7 @@
 // 256 CUs otherwise): each writes its 32-bit partial tile to `partials` [z][M][N], and the tiled kernel's sum kernel
 // adds them up.
 #include "api.h"
-#include "common.h"
+#include "slabs.h"
 
 namespace sa {
 
@@ -40,19 +40,8 @@ namespace wide {
 constexpr int BK = 64;
 constexpr int kCUs = 256;  // compute units of an MI355X
 
-// s_waitcnt for "at most n vector-memory loads outstanding" and nothing else (gfx9 encoding: vmcnt in bits 3:0 and
-// 15:14, expcnt 6:4, lgkmcnt 11:8)
-constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-
-// The workgroup barrier alone; the empty statements and the scheduling barriers keep the compiler from moving memory
-// accesses across it.
-__device__ inline void bare_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-}
+using slabs::bare_barrier;
+using slabs::waitcnt_vm;
 
 // 16 bytes per lane from global memory (base + offset bytes, base the same for the whole wave) into LDS at byte
 // address lds + 16 * lane (the same for the whole wave).  Written as an instruction: the compiler counts a load
@@ -451,7 +440,7 @@ bool gemm_wide_takes(int M, int N, int K, int64_t lda, int64_t ldc, const void* 
 
 // The tile and the cut of K for a product whose caller fixes neither, and the time that this kernel is expected to
 // take with them in microseconds (the figure by which the library chooses between its product kernels).
-static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& shape, int& ks) {
+static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& shape, int& ks, bool broad = true) {
   const int NW_all = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N;
   // without a fitted model below: the weights streamed once at the rate this kernel reaches for few rows, or the
   // products at its rate for many, whichever takes longer, after its start
@@ -528,6 +517,24 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     // (the model of the tiles knows nothing of memory: the weights streamed once from HBM are a floor under it)
     if (best_us >= 0) us = fmax(best_us, 5.0 + 0.02 * (M < 64 ? M : 64) + 2.0 * NW_all * K / 5.8e6);
   }
+  // The tiles of the broad kernel against all of these.  What the others take beyond 1,536 rows or gated, where no model above
+  // says it: their rounds of slabs at what 128 outputs of 256 rows (or as many of another tile) take, fitted like the broad ones.
+  if (broad && M >= 96) {
+    double other = us;
+    if (epi == 1 || M > 1536) {
+      const int rows = shape / 1000 % 1000, wrows = shape % 1000;
+      const int64_t tiles = static_cast<int64_t>((M + rows - 1) / rows) * ((NW + wrows - 1) / wrows);
+      const int64_t rounds = (tiles + wide::kCUs - 1) / wide::kCUs;
+      other = fmax(5.0 + 2.0 * NW_all * K / 5.8e6, 3.0 + rounds * ((epi == 1 ? 0.88 : 0.78) * (K / wide::BK) * rows * wrows / 32768.0 + 2.8));
+    }
+    int broad_tile = 0, cut = ks;
+    const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, broad_tile, cut);
+    if (broad_us < 0.98 * other) {
+      shape = 1000000 + broad_tile;
+      ks = cut;
+      us = broad_us;
+    }
+  }
   return us;
 }
 
@@ -548,7 +555,14 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
   const bf16* a = static_cast<const bf16*>(A);
   const bf16* w = static_cast<const bf16*>(W);
   bf16* c = static_cast<bf16*>(C);
-  if (shape == 0) plan_shape(M, N, K, epi, ws != nullptr, workspace_bytes, shape, ks);
+  // (the broad kernel stores pieces of eight columns, and knows no sections)
+  const bool whole_pieces = N % 8 == 0 && ldc % 8 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+  const bool broad = whole_pieces && sec.n_step == 0;
+  if (shape == 0) plan_shape(M, N, K, epi, ws != nullptr, workspace_bytes, shape, ks, broad);
+  if (shape / 1000000 == 1 && !broad) {
+    set_error("gemm: the broad tiles want widths and rows of whole pieces of eight columns, and no sections");
+    return 1;
+  }
   // 32-bit results: the cuts' partial sums as they are, of one cut straight into C (whose rows are contiguous)
   const bool raw = ks > 1 || c_dtype == kF32;
   float* to = ks > 1 ? ws : static_cast<float*>(C);
@@ -567,6 +581,9 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
     case 6064064: wide::launch<1, 2, 4, 6>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream); break;
     case 5128064: wide::launch<2, 2, 4, 5>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream); break;
     case 4128128: wide::launch<2, 4, 4, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream); break;
+    case 1256256: case 1256288: case 1192256: case 1192288:
+      gemm_broad(shape % 1000000, a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, stream);
+      break;
     case 6064128: wide::launch<1, 4, 4, 6>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream); break;
     default:
       set_error("gemm: unknown wide tile %d", shape);
@@ -596,6 +613,14 @@ extern "C" int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t wor
   if (M < 1 || N < 1 || K < 1 || epilogue < 0 || epilogue > 1) return 0;
   int shape = 0, ks = 1;
   const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
-  sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks);
+  sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks, false);
   return shape;
+}
+
+extern "C" int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t workspace_bytes) {
+  if (M < 1 || N < 1 || K < 1 || epilogue < 0 || epilogue > 1) return 0;
+  int shape = 0, ks = 1;
+  const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
+  sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks);
+  return shape / 1000000 == 1 ? (ks - 1) * 1000000 + shape : 0;
 }

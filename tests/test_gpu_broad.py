@@ -1,0 +1,67 @@
+"""The broad product kernel (tiles of 256 x 288 to 192 x 256 outputs, four waves) at the edges of its tiles, rings and cuts."""
+import pytest
+import torch
+
+import torch_ops as ref
+from test_gpu_kernels import check, gated, rand
+
+TILES = [256288, 256256, 192288, 192256]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (191, 256, 128), (193, 264, 192), (257, 296, 320), (255, 1000, 448), (300, 584, 1088),
+                                   (513, 2304, 2304)])
+def test_gemm_broad(gpu_lib, M, N, K):
+    """Against the 32-bit reference, one bfloat16 step (gated: three, its two products are rounded first); uncut to the bit what the
+    wide kernel gives, whose sums run along K in the same order; strided rows in and out; fewer slabs than the rings hold."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.lib import KernelError
+    from simply_amd.kernels.packing import pack_gate_up, pack_tiles
+    a, w, w2 = rand((M, K), torch.bfloat16, 1), rand((N, K), torch.bfloat16, 2, 0.05), rand((N, K), torch.bfloat16, 3, 0.05)
+    tw, tw2 = pack_tiles(w), pack_gate_up(w, w2)
+    t = dict(bf16_steps=1.0)
+    big = rand((M, K + 16), torch.bfloat16, 4)
+    for tile in TILES:
+        kw = dict(algo=ops.ALGO_WIDE, shape=1000000 + tile)
+        check(ops.gemm(a, tw, **kw), ref.gemm(a, w), **t)
+        assert torch.equal(ops.gemm(a, tw, **kw), ops.gemm(a, tw, algo=ops.ALGO_WIDE, shape=3128128))
+        assert torch.equal(ops.gemm(a, tw2, **kw), ops.gemm(a, tw2, algo=ops.ALGO_WIDE, shape=3128128))
+        for act in range(5):
+            opt = {"activation": act, **({"limit": 0.9} if act == 4 else {})}
+            check(ops.gemm(a, tw2, **kw, **opt), ref.gemm(a, w, w2=w2, **opt), bf16_steps=4.0 if act == 2 else 3.0)
+            if act < 4:
+                assert torch.equal(ops.gemm(a, tw, activate=act, **kw), ops.gemm(a, tw, activate=act, algo=ops.ALGO_WIDE, shape=3128128))
+        out = torch.full((M, N + 16), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.gemm(big[:, 8:8 + K], tw, out=out[:, 8:8 + N], **kw)
+        check(out[:, 8:8 + N], ref.gemm(big[:, 8:8 + K], w), **t)
+        assert (out[:, :8] == 7.0).all() and (out[:, 8 + N:] == 7.0).all()
+        for cuts in (2, 3):   # (more than K has slabs shrinks to what it has)
+            check(ops.gemm(a, tw, algo=ops.ALGO_WIDE, shape=cuts * 10000000 + 1000000 + tile), ref.gemm(a, w), **t)
+        # rows that are not of whole 16-byte pieces are refused where the tile is asked for, and go another way by themselves
+        odd = torch.empty((M, N + 4), dtype=torch.bfloat16, device="cuda")
+        with pytest.raises(KernelError, match="broad"):
+            ops.gemm(a, tw, out=odd[:, :N], **kw)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,is_gated", [(1024, 9216, 2304, True), (2048, 8192, 2048, False), (1056, 4096, 14336, False)])
+def test_gemm_takes_broad_tiles_by_itself(gpu_lib, M, N, K, is_gated):
+    """The dispatcher's choice with the broad kernel, and beside it what that kernel does not take: rows 8 bytes off."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_gate_up, pack_tiles
+    assert gpu_lib.load().sa_gemm_broad_tile(M, N, K, int(is_gated), 256 << 20) > 0
+    a, w, w2 = rand((M, K), torch.bfloat16, 5), rand((N, K), torch.bfloat16, 6, 0.03), rand((N, K), torch.bfloat16, 7, 0.03)
+    tw, want = (pack_gate_up(w, w2), ref.gemm(a, w, w2=w2)) if is_gated else (pack_tiles(w), ref.gemm(a, w))
+    t = gated(dict(bf16_steps=1.0)) if is_gated else dict(bf16_steps=1.0)
+    check(ops.gemm(a, tw), want, **t)
+    off = torch.empty((M, N + 8), dtype=torch.bfloat16, device="cuda")
+    check(ops.gemm(a, tw, out=off[:, 4:4 + N]), want, **t)
+
+
+def test_broad_tiles_where_they_are_ahead():
+    """(M, N, K, gated): cuts * 1000000 + rows * 1000 + weight rows, or 0 where the wide kernel's tiles are taken."""
+    from simply_amd.kernels import lib
+    tile = lambda *at: lib.load().sa_gemm_broad_tile(*at, 256 << 20)
+    assert tile(2048, 9216, 2304, 1) == 1256288 and tile(2048, 8192, 2048, 0) == 1256256 and tile(1056, 36864, 4608, 1) == 1192288
+    assert tile(2048, 4096, 2304, 0) == tile(2048, 2048, 2048, 0) == tile(512, 2304, 9216, 0) == tile(64, 9216, 2304, 1) == 0
+    assert tile(1056, 4608, 36864, 0) // 1000000 > 1 and lib.load().sa_gemm_broad_tile(1056, 4608, 36864, 0, 0) // 1000000 <= 1
