@@ -278,9 +278,9 @@ bool gemm_skinny_takes(int M, int N, int K, int64_t lda, const void* A, const vo
 // the arguments.
 double gemm_skinny_predict_us(int M, int N, int K, int epi);
 double gemm_tiled_predict_us(int M, int N, int K, int epi);
-double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks);
+double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks, int n_step = 0);
 void gemm_broad(int tile, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int epi,
-                int act, float limit, int ks, float* partials, bool raw, hipStream_t stream);
+                int act, float limit, int ks, float* partials, bool raw, Sections sec, hipStream_t stream);
 double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes);
 // The experts' products on the wide kernel (plan, sorted: of the sort kernel with tiles of tile_rows rows, 64 or 128).
 bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t ldc, const void* A, const void* W, const void* W2,

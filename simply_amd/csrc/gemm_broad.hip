@@ -59,7 +59,7 @@ template <int WM, int WN, int RA, int RW, int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_broad_kernel(const bf16* __restrict__ A, int64_t lda,
                                                          const bf16* __restrict__ W, bf16* __restrict__ C, int64_t ldc,
                                                          int M, int N, int K, int chunks, int act, float limit,
-                                                         float* __restrict__ partials) {
+                                                         float* __restrict__ partials, Sections sec) {
   constexpr int MT = 2 * WM, NT = 2 * WN;
   constexpr int BM = MT * 16;
   constexpr int A_SLAB = MT * 1024, W_HALF = NT * 512;         // elements
@@ -94,9 +94,19 @@ __global__ __launch_bounds__(256, 1) void gemm_broad_kernel(const bf16* __restri
   const int slabs_all = K / BK;
   const int slab0 = blockIdx.z * slabs_all / gridDim.z;
   const int slabs = (blockIdx.z + 1) * slabs_all / gridDim.z - slab0;
-  const int m_base = by * BM, nt_base = bx * NT;
+  const int m_base = by * BM;
   const int NW = EPI == 1 ? 2 * ((N + 15) / 16) * 16 : N;
-  const int ntiles = (NW + 15) / 16;
+  // several products at once: which section this workgroup is in, its columns of A, its rows of W
+  int first_tile = 0, NL = NW;   // the section's first 16-row tile of W and the end of its rows
+  if (EPI == 0 && sec.n_step > 0) {
+    const int per = (sec.n_step + NT * 16 - 1) / (NT * 16), s = bx / per;
+    bx -= s * per;
+    first_tile = s * (sec.n_step / 16);
+    A += static_cast<size_t>(s) * sec.a_step;
+    NL = (s + 1) * sec.n_step < NW ? (s + 1) * sec.n_step : NW;
+  }
+  const int ntiles = (NL + 15) / 16;
+  const int nt_base = first_tile + bx * NT;
 
   // ---- what this wave copies: of a slab of A the KiB blocks (tile tile_mine + 2 i, its rows 8 half_mine ..), half of them in each
   // half; of a half of W the tiles wave + 4 i.  Rows beyond M read row M - 1, tiles beyond the last the last one (never stored).
@@ -260,7 +270,7 @@ __global__ __launch_bounds__(256, 1) void gemm_broad_kernel(const bf16* __restri
 #pragma unroll 2
     for (int p = threadIdx.x; p < rows_here * PIECES; p += 256) {
       const int r = p / PIECES, c = p % PIECES, n = n_first + c * 8;
-      if (n >= N) continue;
+      if (n >= (EPI == 1 ? N : NL)) continue;
       union Eight { uint4 q; uint16_t h[8]; } a, b, out;
       const __bf16* from = lds + r * PITCH + (EPI == 1 ? (c / 2) * 32 + c % 2 * 8 : c * 8);
       a.q = *reinterpret_cast<const uint4*>(from);
@@ -288,16 +298,17 @@ __global__ __launch_bounds__(256, 1) void gemm_broad_kernel(const bf16* __restri
 
 template <int WM, int WN, int RA, int RW>
 static void launch(const bf16* A, int64_t lda, const bf16* W, bf16* C, int64_t ldc, int M, int N, int K, int epi,
-                   int act, float limit, int ks, float* partials, bool raw, hipStream_t stream) {
+                   int act, float limit, int ks, float* partials, bool raw, Sections sec, hipStream_t stream) {
   constexpr int BM = 2 * WM * 16, BNW = 2 * WN * 16;
   const int NW = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N;
-  const dim3 grid((NW + BNW - 1) / BNW, (M + BM - 1) / BM, ks);
+  const int whole = sec.n_step > 0 ? (NW - 1) / sec.n_step : 0;   // sections before the last one
+  const dim3 grid(whole * ((sec.n_step + BNW - 1) / BNW) + (NW - whole * sec.n_step + BNW - 1) / BNW, (M + BM - 1) / BM, ks);
   if (epi == 1)
-    gemm_broad_kernel<WM, WN, RA, RW, 1><<<grid, 256, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32, act, limit, nullptr);
+    gemm_broad_kernel<WM, WN, RA, RW, 1><<<grid, 256, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32, act, limit, nullptr, sec);
   else if (raw)
-    gemm_broad_kernel<WM, WN, RA, RW, 3><<<grid, 256, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32, act, limit, partials);
+    gemm_broad_kernel<WM, WN, RA, RW, 3><<<grid, 256, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32, act, limit, partials, sec);
   else
-    gemm_broad_kernel<WM, WN, RA, RW, 0><<<grid, 256, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32, act, limit, nullptr);
+    gemm_broad_kernel<WM, WN, RA, RW, 0><<<grid, 256, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32, act, limit, nullptr, sec);
 }
 
 }  // namespace broad
@@ -305,14 +316,15 @@ static void launch(const bf16* A, int64_t lda, const bf16* W, bf16* C, int64_t l
 // The tile (rows * 1000 + weight rows) and cut of K that this kernel is expected to be fastest with, and its microseconds: full
 // rounds of 256 workgroups, and a last one whose slabs take the less time the fewer CUs have one (the clock rises), fitted to 27
 // sizes of weights from 1,024 x 1,024 to 73,728 x 4,608 at 256 to 3,072 rows (3 to 6 % root mean square).
-double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks) {
+double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks, int n_step) {
   struct Tile { int rows, wrows; double alone, full, start; };   // us a slab alone and with every CU at work; us a round
   static const Tile tiles[4] = {{256, 288, 0.99, 1.45, 7.6}, {256, 256, 0.89, 1.35, 6.4}, {192, 288, 0.80, 1.19, 5.2}, {192, 256, 0.76, 1.05, 4.0}};
   const int NW = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N, slabs = K / broad::BK;
   double best = -1.0;
   int cut_out = 1;
   for (const Tile& t : tiles) {
-    const int64_t count = static_cast<int64_t>((M + t.rows - 1) / t.rows) * ((NW + t.wrows - 1) / t.wrows);
+    const int columns = n_step > 0 ? NW / n_step * ((n_step + t.wrows - 1) / t.wrows) : (NW + t.wrows - 1) / t.wrows;   // (whole sections)
+    const int64_t count = static_cast<int64_t>((M + t.rows - 1) / t.rows) * columns;
     const int cuts[3] = {ks > 1 ? ks : 1, static_cast<int>(broad::kCUs / count), static_cast<int>(2 * broad::kCUs / count)};
     for (int c = 0; c < 3; ++c) {
       const int cut = cuts[c];
@@ -333,15 +345,15 @@ double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t
 }
 
 void gemm_broad(int tile, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int epi,
-                int act, float limit, int ks, float* partials, bool raw, hipStream_t stream) {
+                int act, float limit, int ks, float* partials, bool raw, Sections sec, hipStream_t stream) {
   const bf16* a = static_cast<const bf16*>(A);
   const bf16* w = static_cast<const bf16*>(W);
   bf16* c = static_cast<bf16*>(C);
   switch (tile) {
-    case 256288: broad::launch<8, 9, 3, 3>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, stream); break;
-    case 192288: broad::launch<6, 9, 3, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, stream); break;
-    case 256256: broad::launch<8, 8, 3, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, stream); break;
-    default: broad::launch<6, 8, 3, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, stream); break;
+    case 256288: broad::launch<8, 9, 3, 3>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, sec, stream); break;
+    case 192288: broad::launch<6, 9, 3, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, sec, stream); break;
+    case 256256: broad::launch<8, 8, 3, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, sec, stream); break;
+    default: broad::launch<6, 8, 3, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, partials, raw, sec, stream); break;
   }
 }
 

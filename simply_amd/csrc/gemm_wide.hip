@@ -477,14 +477,16 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     const int rows = M <= 64 ? 64 : 128;
     if (static_cast<int64_t>((M + rows - 1) / rows) * ((NW + 127) / 128) <= wide::kCUs) shape = M <= 64 ? 6064128 : 3128128;
   }
+  // More rows against few outputs (64 tiles of 128 x 128 at most) too: 2,048 rows of K = 4,096 against 512 outputs 27.6 / 15.2 us, of K =
+  // 2,048 against 256 16.5 / 10.9 and against 64 15.5 / 13.4, 3,000 of 2,304 against 160 17.2 / 11.1 (uncut / with the cut).
   // 17 to 1,536 rows without an epilogue (portions of prompts, many decoding requests): the tiles above are too few
   // for 256 CUs, and every workgroup walks all of K at the pace of its own slabs.  Smaller tiles with deeper
   // pipelines, and K cut over workgroups so that about one round of them covers the GPU, chosen by a model of the
   // time fitted to measurements at the 2B, 9B and 27B sizes (64 to 2,048 rows, seven tiles, one to fourteen cuts;
   // it is within 6 % of the best measured choice nearly everywhere, and a fifth faster in sum than either the
   // uncut tiles above or the tiled kernel with its cut: the 2B down projection at 512 rows takes 36 us against 55).
-  // Beyond 1,536 rows the uncut tiles above stay; whether the model's choice would be better there has not been measured.
-  if (epi == 0 && M <= 1536) {  // (fewer than 17 rows come here only against a very long K)
+  const bool few_tiles = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128) <= 64;
+  if (epi == 0 && (M <= 1536 || few_tiles)) {  // (fewer than 17 rows come here only against a very long K)
     struct Tile { int code, rows, wrows; double eff, start; };  // share of the MFMA rate in the loop; us to start
     static const Tile tiles[7] = {{3128128, 128, 128, 0.425, 1.44}, {3128256, 128, 256, 0.535, 2.03},
                                   {3192128, 192, 128, 0.535, 1.25}, {3256128, 256, 128, 0.615, 1.58},
@@ -521,7 +523,7 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
   // says it: their rounds of slabs at what 128 outputs of 256 rows (or as many of another tile) take, fitted like the broad ones.
   if (broad && M >= 96) {
     double other = us;
-    if (epi == 1 || M > 1536) {
+    if (epi == 1 || (M > 1536 && !few_tiles)) {
       const int rows = shape / 1000 % 1000, wrows = shape % 1000;
       const int64_t tiles = static_cast<int64_t>((M + rows - 1) / rows) * ((NW + wrows - 1) / wrows);
       const int64_t rounds = (tiles + wide::kCUs - 1) / wide::kCUs;
@@ -555,13 +557,31 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
   const bf16* a = static_cast<const bf16*>(A);
   const bf16* w = static_cast<const bf16*>(W);
   bf16* c = static_cast<bf16*>(C);
-  // (the broad kernel stores pieces of eight columns, and knows no sections)
-  const bool whole_pieces = N % 8 == 0 && ldc % 8 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
-  const bool broad = whole_pieces && sec.n_step == 0;
-  if (shape == 0) plan_shape(M, N, K, epi, ws != nullptr, workspace_bytes, shape, ks, broad);
+  // (the broad kernel stores pieces of eight columns)
+  const bool broad = N % 8 == 0 && ldc % 8 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+  const bool planned = shape == 0;
+  double planned_us = 0.0;
+  if (planned) planned_us = plan_shape(M, N, K, epi, ws != nullptr, workspace_bytes, shape, ks, broad && sec.n_step == 0);
   if (shape / 1000000 == 1 && !broad) {
-    set_error("gemm: the broad tiles want widths and rows of whole pieces of eight columns, and no sections");
+    set_error("gemm: the broad tiles want widths and rows of whole pieces of eight columns");
     return 1;
+  }
+  // Several products at once: where the broad kernel's tiles are ahead for the whole sections, they run on it and a shorter last one
+  // by itself (at 2,047 rows of four sections of 2,048 outputs it would be eight more tiles behind a full round).  Measured, us,
+  // wide / broad and the rest: 2,047 rows of four sections of 2,048 and 64 outputs 74 / 65, 4,096 rows 138 / 120; sections of 4,096, 1,024
+  // rows 163 / 115, 2,047 275 / 218, 512 92 / 96; of 1,024, 2,047 rows 27 / 35, 4,096 53 / 41.
+  if (planned && broad && sec.n_step > 0 && c_dtype == kBF16) {
+    const int whole = N / sec.n_step, rest = N % sec.n_step;
+    int tile = 0, one = 1;
+    const double whole_us = gemm_broad_plan(M, whole * sec.n_step, K, 0, false, 0, tile, one, sec.n_step);
+    const double rest_us = rest > 0 ? gemm_wide_predict_us(M, rest, K, 0, ws != nullptr, workspace_bytes) : 0.0;
+    if (whole > 0 && M >= 96 && whole_us + rest_us < 0.98 * planned_us) {
+      gemm_broad(tile, a, lda, w, c, ldc, M, whole * sec.n_step, K, 0, 0, 0.f, 1, nullptr, false, sec, stream);
+      if (check_launch("gemm_broad")) return 1;
+      const size_t at = static_cast<size_t>(whole) * sec.n_step;
+      return rest == 0 ? 0 : sa_gemm(a + static_cast<size_t>(whole) * sec.a_step, kBF16, lda, w + at * K, nullptr, kBF16, c + at, kBF16, ldc,
+                                     M, rest, K, 0, 0.f, 0, 1, 0, workspace, static_cast<int64_t>(workspace_bytes), stream);
+    }
   }
   // 32-bit results: the cuts' partial sums as they are, of one cut straight into C (whose rows are contiguous)
   const bool raw = ks > 1 || c_dtype == kF32;
@@ -582,7 +602,7 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
     case 5128064: wide::launch<2, 2, 4, 5>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream); break;
     case 4128128: wide::launch<2, 4, 4, 4>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream); break;
     case 1256256: case 1256288: case 1192256: case 1192288:
-      gemm_broad(shape % 1000000, a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, stream);
+      gemm_broad(shape % 1000000, a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream);
       break;
     case 6064128: wide::launch<1, 4, 4, 6>(a, lda, w, c, ldc, M, N, K, epi, act, limit, ks, to, raw, sec, stream); break;
     default:

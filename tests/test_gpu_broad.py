@@ -65,3 +65,26 @@ def test_broad_tiles_where_they_are_ahead():
     assert tile(2048, 9216, 2304, 1) == 1256288 and tile(2048, 8192, 2048, 0) == 1256256 and tile(1056, 36864, 4608, 1) == 1192288
     assert tile(2048, 4096, 2304, 0) == tile(2048, 2048, 2048, 0) == tile(512, 2304, 9216, 0) == tile(64, 9216, 2304, 1) == 0
     assert tile(1056, 4608, 36864, 0) // 1000000 > 1 and lib.load().sa_gemm_broad_tile(1056, 4608, 36864, 0, 0) // 1000000 <= 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,n,last,K", [(4096, 1024, 64, 1024), (1031, 2048, 2048, 1088), (2047, 2048, 16, 2048)])
+def test_sections_on_broad_tiles(gpu_lib, M, n, last, K):
+    """Several products at once of so many rows that the whole sections go to the broad kernel, a shorter last one by itself."""
+    from simply_amd.kernels import ops
+    ws = [rand((last if s == 3 else n, K), torch.bfloat16, 20 + s, 0.05) for s in range(4)]
+    a = rand((M, 4 * K), torch.bfloat16, 30)
+    got = ops.gemm_sections(a, ops.SectionedWeight(ws))
+    for s, w in enumerate(ws):
+        check(got[:, s * n:s * n + w.shape[0]], ref.gemm(a[:, s * K:(s + 1) * K], w), bf16_steps=1.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1537, 4, 512), (2047, 64, 2048), (2048, 512, 4096), (4096, 132, 1088), (1600, 640, 2304)])
+def test_many_rows_against_few_outputs(gpu_lib, M, N, K):
+    """Beyond 1,536 rows: tiles and a cut of K as for fewer rows, up to 64 tiles of 128 x 128 (and the first size with more)."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+    a, w = rand((M, K), torch.bfloat16, 40), rand((N, K), torch.bfloat16, 41, 0.05)
+    check(ops.gemm(a, pack_tiles(w)), ref.gemm(a, w), bf16_steps=1.0)
+    check(ops.gemm(a, pack_tiles(w), out_dtype=torch.float32), ref.gemm(a, w, out_dtype=torch.float32), rtol=2e-3, atol=2e-3)
