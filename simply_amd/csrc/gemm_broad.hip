@@ -336,7 +336,7 @@ double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t
       const int per = (slabs + cut - 1) / cut;
       double us = 3.0 + full * (per * t.full + t.start);
       if (rest > 0) us += per * (t.alone + (t.full - t.alone) * rest) + t.start;
-      if (cut > 1) us += partial_bytes / 5.5e6 + partial_bytes / 1e7 + 2.5;   // written, read again, the sum kernel
+      if (cut > 1) us += partial_bytes / 8e6 + partial_bytes / 5.5e6;   // written, and read again by whoever adds them up
       if (best < 0 || us < best) best = us, tile = t.rows * 1000 + t.wrows, cut_out = cut;
     }
   }

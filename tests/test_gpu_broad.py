@@ -88,3 +88,20 @@ def test_many_rows_against_few_outputs(gpu_lib, M, N, K):
     a, w = rand((M, K), torch.bfloat16, 40), rand((N, K), torch.bfloat16, 41, 0.05)
     check(ops.gemm(a, pack_tiles(w)), ref.gemm(a, w), bf16_steps=1.0)
     check(ops.gemm(a, pack_tiles(w), out_dtype=torch.float32), ref.gemm(a, w, out_dtype=torch.float32), rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [8, 1028, 2304, 3588, 4608, 5120])
+def test_norm_of_any_number_of_planes(gpu_lib, D):
+    """A product's planes added up in the norm behind it: to the bit what the sum kernel and the norm of its result give."""
+    from simply_amd.kernels import ops
+    T = 70
+    kw = dict(post_weight=rand((D,), torch.bfloat16, 50, 0.3), post_eps=1e-6, post_plus_one=True, next_weight=rand((D,), torch.bfloat16, 51, 0.3),
+              next_eps=1e-6, next_plus_one=True, out_dtype=torch.bfloat16)
+    for count in (1, 2, 3, 4, 5, 6, 7, 8, 11):
+        planes, h = rand((count, T, D), torch.float32, 60 + count), rand((T, D), torch.float32, 52)
+        h2 = h.clone()
+        y = torch.empty((T, D), dtype=torch.bfloat16, device="cuda")
+        whole = ops.PartialSums(planes, y.clone()).materialize()
+        got, want = ops.add_rmsnorm(ops.PartialSums(planes, y), h, **kw), ops.add_rmsnorm(whole, h2, **kw)
+        assert torch.equal(got, want) and torch.equal(h, h2)
