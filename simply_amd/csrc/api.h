@@ -277,6 +277,10 @@ bool gemm_skinny_takes(int M, int N, int K, int64_t lda, const void* A, const vo
 // the kernel is not made for them.  The dispatcher runs the kernel with the smallest figure among those that take
 // the arguments.
 double gemm_skinny_predict_us(int M, int N, int K, int epi);
+// Many rows against at most 64 outputs, no epilogue (what the tiled kernel is asked for there, unless the caller fixes its cuts).
+bool gemm_narrow_takes(int M, int N, int K);
+double gemm_narrow_predict_us(int M, int N, int K);
+int gemm_narrow(const void* A, int64_t lda, const void* W, void* C, int c_dtype, int64_t ldc, int M, int N, int K, hipStream_t stream);
 double gemm_tiled_predict_us(int M, int N, int K, int epi);
 double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks, int n_step = 0);
 void gemm_broad(int tile, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int epi,

@@ -348,6 +348,7 @@ bool gemm_streams_weights(int M, int NW, int K) {
 // once, or the products at this kernel's rate, whichever takes longer, after a start that includes the sum of the
 // cuts of K.  Fitted to the same sweep (within 0.86 to 1.38 of the measured time up to 64 rows).
 double gemm_tiled_predict_us(int M, int N, int K, int epi) {
+  if (epi == 0 && gemm_narrow_takes(M, N, K)) return gemm_narrow_predict_us(M, N, K);
   const double NW = epi == 1 ? 2.0 * ((N + 15) / 16) * 16 : N;
   return 9.0 + 0.08 * (M < 64 ? M : 64) + fmax(2.0 * NW * K / 5.7e6, static_cast<double>(M) * NW * K / (0.6e9 / 2));
 }
@@ -361,6 +362,8 @@ bool gemm_tiled_takes(int M, int N, int K, int64_t lda, const void* A, const voi
 // ksplit > 0 fixes the number of cuts of K.
 int gemm_tiled(const void* A, int64_t lda, const void* W, void* C, int c_dtype, int64_t ldc, int M, int N, int K,
                int epi, int act, float cap, int ksplit, void* workspace, size_t workspace_bytes, hipStream_t stream, Sections sec) {
+  if (ksplit == 0 && epi == 0 && sec.n_step == 0 && gemm_narrow_takes(M, N, K))
+    return gemm_narrow(A, lda, W, C, c_dtype, ldc, M, N, K, stream);
   const bf16* a = static_cast<const bf16*>(A);
   const bf16* w = static_cast<const bf16*>(W);
   float* ws = static_cast<float*>(workspace);

@@ -574,7 +574,7 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
     const int whole = N / sec.n_step, rest = N % sec.n_step;
     int tile = 0, one = 1;
     const double whole_us = gemm_broad_plan(M, whole * sec.n_step, K, 0, false, 0, tile, one, sec.n_step);
-    const double rest_us = rest > 0 ? gemm_wide_predict_us(M, rest, K, 0, ws != nullptr, workspace_bytes) : 0.0;
+    const double rest_us = rest > 0 ? fmin(gemm_tiled_predict_us(M, rest, K, 0), gemm_wide_predict_us(M, rest, K, 0, ws != nullptr, workspace_bytes)) : 0.0;
     if (whole > 0 && M >= 96 && whole_us + rest_us < 0.98 * planned_us) {
       gemm_broad(tile, a, lda, w, c, ldc, M, whole * sec.n_step, K, 0, 0, 0.f, 1, nullptr, false, sec, stream);
       if (check_launch("gemm_broad")) return 1;

@@ -105,3 +105,22 @@ def test_norm_of_any_number_of_planes(gpu_lib, D):
         whole = ops.PartialSums(planes, y.clone()).materialize()
         got, want = ops.add_rmsnorm(ops.PartialSums(planes, y), h, **kw), ops.add_rmsnorm(whole, h2, **kw)
         assert torch.equal(got, want) and torch.equal(h, h2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 1, 32), (64, 16, 64), (100, 20, 96), (129, 33, 1056), (257, 48, 2080), (2047, 64, 2048), (1000, 64, 4096)])
+def test_many_rows_against_a_handful_of_outputs(gpu_lib, M, N, K):
+    """A workgroup for 16 rows and all outputs: fewer chunks of K than waves, remainders, one to four tiles, both types of result; and a
+    row's bits do not depend on the rows beside it."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+    big, w = rand((M, K + 16), torch.bfloat16, 70), rand((N, K), torch.bfloat16, 71, 0.05)
+    a, tw = big[:, 8:8 + K], pack_tiles(w)
+    assert ops.gemm_plan(M, N, K)[0] == ops.ALGO_TILED
+    check(ops.gemm(a, tw), ref.gemm(a, w), bf16_steps=1.0)
+    got = ops.gemm(a, tw, out_dtype=torch.float32)
+    torch.testing.assert_close(got, (a.double() @ w.double().T).float(), rtol=1e-5, atol=2e-6 * K ** 0.5)
+    assert torch.equal(got[-33:], ops.gemm(a[-33:], tw, out_dtype=torch.float32))
+    out = torch.full((M, N + 3), 7.0, device="cuda")
+    ops.gemm(a, tw, out=out[:, 2:2 + N])
+    assert torch.equal(out[:, 2:2 + N], got) and (out[:, :2] == 7.0).all() and (out[:, 2 + N:] == 7.0).all()
