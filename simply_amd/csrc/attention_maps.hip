@@ -502,6 +502,10 @@ extern "C" int sa_paged_attention_maps_units(const void* q, int64_t q_stride, co
   const int KhV = Kh * maps * sh.chunks;
   SA_REQUIRE(KhV <= 65535 && unit_count <= 65535, "paged_attention_maps_units: too many heads or units");
   int KS = paged_attention_decode_ranges(unit_count, KhV, window, max_kv_len, 0);
+  // few units with few keys: a workgroup for each tile of 32 keys, as far as there are CUs (every wave reads all of a tile's keys, 36 KiB of
+  // a latent's: two tiles are two trips to memory one behind the other)
+  const int most = paged_attention_decode_ranges(unit_count, KhV, window, max_kv_len, 1 << 20);   // (one for each tile)
+  if (KS < most && static_cast<int64_t>(unit_count) * KhV * most <= 256) KS = most;
   const size_t per_split = static_cast<size_t>(unit_count) * KhV * 16 * (hd_v + kRowExtra) * sizeof(float);
   while (KS > 1 && (workspace == nullptr || per_split * KS > workspace_bytes)) --KS;
   const bool partial = differential != 0;

@@ -521,6 +521,9 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
   }
   // The tiles of the broad kernel against all of these.  What the others take beyond 1,536 rows or gated, where no model above
   // says it: their rounds of slabs at what 128 outputs of 256 rows (or as many of another tile) take, fitted like the broad ones.
+  // (Behind other kernels, weights in HBM, the broad tiles keep their time better than in a loop of the one product, by which both are
+  // fitted: 2,048 rows against 6,144 outputs of K = 2,048 49 and 49 us there, 60 and 49 in a prompt.  Hence the line at 1.03; at 1.12
+  // prompts are 0.3 to 1 % slower again.)
   if (broad && M >= 96) {
     double other = us;
     if (epi == 1 || (M > 1536 && !few_tiles)) {
@@ -531,7 +534,7 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     }
     int broad_tile = 0, cut = ks;
     const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, broad_tile, cut);
-    if (broad_us < 0.98 * other) {
+    if (broad_us < 1.03 * other) {
       shape = 1000000 + broad_tile;
       ks = cut;
       us = broad_us;
