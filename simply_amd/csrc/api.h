@@ -291,7 +291,9 @@ bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t l
                             const void* C, int tile_rows);
 int gemm_wide_routed(const void* A, int64_t lda, const void* W, const void* W2, void* C, float* y, int64_t ldc, int tiles, int N,
                      int K, int tile_rows, const int* plan, const int* sorted, int by_token, int top, int act, float limit,
-                     hipStream_t stream);
+                     hipStream_t stream, const void* beside_a = nullptr,
+                     int64_t beside_lda = 0, const void* beside_w = nullptr, void* beside_y = nullptr, int64_t beside_ldc = 0,
+                     int beside_k = 0, int beside_rows = 0);
 int gemm_skinny(const void* A, int64_t lda, const void* W, const void* W2, void* C, int c_dtype, int64_t ldc, int M,
                 int N, int K, int epi, int act, float cap, int packed, int shape, hipStream_t stream, Sections sec = {});
 bool paged_attention_decode_takes(int H, int Kh, int hd, int page_size, int max_q_len, int64_t q_stride, const void* q);
@@ -656,6 +658,13 @@ int sa_expert_sort(const int* experts, int P, int E, int tile_rows, int* sorted,
 int sa_expert_product(const void* a, int dtype, int64_t a_stride, int a_by_token, int top, const void* w1, const void* w2,
                       int N, int K, const int* sorted, const int* plan, int P, int E, int tile_rows, int act, float limit,
                       void* out, int64_t out_stride, int out_by_pair, int activate, hipStream_t stream);
+// The experts' second product (no activation, out by pair, 32-bit) and beside it, in the same launch, shared_y [T, N] (bfloat16) =
+// shared_h [T, shared_K] . shared_w^T of a feed-forward that takes every token: bfloat16, tiles of 64 or 128 rows, aligned operands.
+int sa_expert_product_beside_takes(int N, int K, int64_t h_stride, int P, int tile_rows, const void* shared_h, int64_t shared_h_stride,
+                                   const void* shared_w, int shared_K, int T);
+int sa_expert_product_beside(const void* h, int64_t h_stride, int top, const void* w, int N, int K, const int* sorted, const int* plan,
+                             int P, int E, int tile_rows, void* y, int64_t y_stride, const void* shared_h, int64_t shared_h_stride,
+                             const void* shared_w, int shared_K, int T, void* shared_y, int64_t shared_y_stride, hipStream_t stream);
 // A router of a few tokens in one launch: logits [T, rows] (32-bit) = x . w^T with x bfloat16 [T, D] and w tiled, the choice as
 // sa_route (plain) or sa_route_choice make it from the first E logits of a token, sorted and plan as sa_expert_sort with tiles
 // of 16 rows; and, with dense_w (tiled, gated: the two factors' tiles in turn), dense_out [T, dense_N] bfloat16 = rule(x . dense_w^T).

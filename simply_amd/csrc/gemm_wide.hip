@@ -64,6 +64,14 @@ struct Routed {
   const int* sorted;
   const bf16* w2;
   int by_token, top;
+  // EPI 4: row tiles from `tiles` on are those of a product beside the experts', rows of its own times one weight of as many outputs
+  // (the second product of a feed-forward that takes every token), bfloat16 results in the rows' order
+  int tiles;
+  const bf16* beside_a;
+  const bf16* beside_w;
+  bf16* beside_y;
+  int64_t beside_lda, beside_ldc;
+  int beside_k, beside_rows;
 };
 
 // WM x WN: 16 x 16 tiles of a wave (rows of A x rows of W); WAVES_M x (WAVES / WAVES_M) waves.
@@ -94,11 +102,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
   if (ROUTED) {
     // (no turning round: how many tiles there are is known on the device only, and a tile's neighbours in x, which share
     // its rows, go to the XCDs in turn, so that an XCD meets the same weights again in the expert's next tile)
-    if (by >= rt.plan[0]) return;
-    row_first = rt.plan[2 + 3 * by], tile_rows = rt.plan[3 + 3 * by];
-    const size_t expert = static_cast<size_t>(rt.plan[1 + 3 * by]) * ((N + 15) / 16) * chunks * 512;
-    W += expert;
-    if (EPI == 1) rt.w2 += expert;
+    if (EPI == 4 && by >= rt.tiles) {
+      row_first = (by - rt.tiles) * BM, tile_rows = rt.beside_rows - row_first < BM ? rt.beside_rows - row_first : BM;
+      A = rt.beside_a, lda = rt.beside_lda, W = rt.beside_w, K = rt.beside_k, chunks = K / 32;
+      ldc = rt.beside_ldc;
+    } else {
+      if (by >= rt.plan[0]) return;
+      row_first = rt.plan[2 + 3 * by], tile_rows = rt.plan[3 + 3 * by];
+      const size_t expert = static_cast<size_t>(rt.plan[1 + 3 * by]) * ((N + 15) / 16) * chunks * 512;
+      W += expert;
+      if (EPI == 1) rt.w2 += expert;
+    }
   } else {
     const int nx = gridDim.x, ny = gridDim.y, total = nx * ny;
     int l = bx + nx * by;
@@ -307,6 +321,18 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
     const int m = m_base + (wm * WM + i) * 16 + row;
     if (m >= tile_rows) continue;
     if (EPI == 4) {
+      if (by >= rt.tiles) {   // (beside the experts: rounded, in the rows' order)
+        bf16* c_row = rt.beside_y + static_cast<size_t>(row_first + m) * ldc;
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+          const int n = (nt_base + wn * WN + j) * 16 + quad * 4;
+          uint2 packed;
+          packed.x = static_cast<uint32_t>(float_to_bf16(acc[i][j][0]).bits) | (static_cast<uint32_t>(float_to_bf16(acc[i][j][1]).bits) << 16);
+          packed.y = static_cast<uint32_t>(float_to_bf16(acc[i][j][2]).bits) | (static_cast<uint32_t>(float_to_bf16(acc[i][j][3]).bits) << 16);
+          if (n < NL) *reinterpret_cast<uint2*>(c_row + n) = packed;
+        }
+        continue;
+      }
       float* y_row = partials + static_cast<size_t>(rt.sorted[row_first + m]) * ldc;
 #pragma unroll
       for (int j = 0; j < WN; ++j) {
@@ -373,7 +399,8 @@ static void launch_routed(const bf16* A, int64_t lda, const bf16* W, const Route
                           int rows, int N, int K, int act, float limit, hipStream_t stream) {
   constexpr int BNW = (WAVES / WAVES_M) * WN * 16;
   const int NW = rt.w2 != nullptr ? 2 * ((N + 15) / 16) * 16 : N;
-  const dim3 grid((NW + BNW - 1) / BNW, tiles);
+  constexpr int BM = WAVES_M * WM * 16;
+  const dim3 grid((NW + BNW - 1) / BNW, tiles + (rt.beside_rows + BM - 1) / BM);
   if (rt.w2 != nullptr)
     gemm_wide_kernel<WM, WN, WAVES_M, 1, NSTAGE, WAVES, true><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, rows, N, K, K / 32,
                                                                                                act, limit, nullptr, Sections{}, rt);
@@ -418,9 +445,12 @@ bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t l
 // per pair.
 int gemm_wide_routed(const void* A, int64_t lda, const void* W, const void* W2, void* C, float* y, int64_t ldc, int tiles, int N,
                      int K, int tile_rows, const int* plan, const int* sorted, int by_token, int top, int act, float limit,
-                     hipStream_t stream) {
+                     hipStream_t stream, const void* beside_a, int64_t beside_lda, const void* beside_w, void* beside_y,
+                     int64_t beside_ldc, int beside_k, int beside_rows) {
   wide::Routed rt;
   rt.plan = plan, rt.sorted = sorted, rt.w2 = static_cast<const bf16*>(W2), rt.by_token = by_token, rt.top = top;
+  rt.tiles = tiles, rt.beside_a = static_cast<const bf16*>(beside_a), rt.beside_w = static_cast<const bf16*>(beside_w);
+  rt.beside_y = static_cast<bf16*>(beside_y), rt.beside_lda = beside_lda, rt.beside_ldc = beside_ldc, rt.beside_k = beside_k, rt.beside_rows = beside_rows;
   const bf16* a = static_cast<const bf16*>(A);
   const bf16* w = static_cast<const bf16*>(W);
   bf16* c = static_cast<bf16*>(C);

@@ -978,6 +978,35 @@ extern "C" int sa_expert_product_shared(const void* h, int64_t h_stride, int top
   return check_launch("expert_product_shared");
 }
 
+extern "C" int sa_expert_product_beside_takes(int N, int K, int64_t h_stride, int P, int tile_rows, const void* shared_h,
+                                              int64_t shared_h_stride, const void* shared_w, int shared_K, int T) {
+  alignas(16) static const char aligned_stand_in[16] = {};   // (the experts' operands and the results are whole tensors)
+  const void* p = aligned_stand_in;
+  return N > 0 && K > 0 && P > 0 && T > 0 && shared_K > 0 && shared_h_stride >= shared_K &&
+         gemm_wide_routed_takes(N, K, h_stride, P, N, p, p, nullptr, p, tile_rows) &&
+         gemm_wide_routed_takes(N, shared_K, shared_h_stride, T, N, shared_h, shared_w, nullptr, p, tile_rows);
+}
+
+extern "C" int sa_expert_product_beside(const void* h, int64_t h_stride, int top, const void* w, int N, int K, const int* sorted,
+                                        const int* plan, int P, int E, int tile_rows, void* y, int64_t y_stride, const void* shared_h,
+                                        int64_t shared_h_stride, const void* shared_w, int shared_K, int T, void* shared_y,
+                                        int64_t shared_y_stride, hipStream_t stream) {
+  SA_REQUIRE(P > 0 && E > 0 && N > 0 && K > 0 && top > 0 && T > 0 && shared_K > 0 && h_stride >= K && y_stride >= N &&
+                 shared_h_stride >= shared_K && shared_y_stride >= N,
+             "expert_product_beside: bad sizes P=%d E=%d N=%d K=%d T=%d K=%d", P, E, N, K, T, shared_K);
+  SA_REQUIRE(h != nullptr && w != nullptr && sorted != nullptr && plan != nullptr && y != nullptr && shared_h != nullptr &&
+                 shared_w != nullptr && shared_y != nullptr,
+             "expert_product_beside: a null pointer");
+  SA_REQUIRE(tile_rows == kTileRowsMax || tile_rows == kTileRowsWide, "expert_product_beside: tiles of %d or %d rows", kTileRowsMax, kTileRowsWide);
+  const int tiles = sa_expert_tiles_max(P, E, tile_rows);
+  SA_REQUIRE(static_cast<int64_t>(tiles) + (T + tile_rows - 1) / tile_rows <= kGridMax &&
+                 gemm_wide_routed_takes(N, K, h_stride, P, y_stride, h, w, nullptr, y, tile_rows) &&
+                 gemm_wide_routed_takes(N, shared_K, shared_h_stride, T, shared_y_stride, shared_h, shared_w, nullptr, shared_y, tile_rows),
+             "expert_product_beside: aligned bfloat16 operands, K in multiples of 64; got N=%d K=%d and K=%d", N, K, shared_K);
+  return gemm_wide_routed(h, h_stride, w, nullptr, nullptr, static_cast<float*>(y), y_stride, tiles, N, K, tile_rows, plan, sorted, 0, top, 0,
+                          0.f, stream, shared_h, shared_h_stride, shared_w, shared_y, shared_y_stride, shared_K, T);
+}
+
 extern "C" int sa_expert_combine(const float* y, const float* weights, int top, const void* shared, int shared_dtype,
                                  int64_t shared_stride, const float* gate, int64_t gate_stride, void* out, int out_dtype,
                                  int64_t out_stride, int T, int D, hipStream_t stream) {

@@ -2222,6 +2222,22 @@ def few_rows_experts(T: int, top: int, gate_w, up_w, x: torch.Tensor) -> bool:
     return _lib.load().sa_expert_tile_rows(T * top, up_w.experts, up_w.cols, up_w.rows, _code(x), x.stride(0), _ptr(x)) == 16
 
 
+def experts_beside(T: int, top: int, up_w, down_w, x: torch.Tensor, dense) -> bool:
+    """Whether a step of T tokens takes the second product of a shared feed-forward (a tiled weight `dense`) beside its experts': with
+    tiles of 128 rows, whose last round of workgroups it fills.  A wide one makes tiles that walk longer than the experts' and is ahead
+    only with many tokens.  Both second products and the experts' first, us, apart / beside, 16 experts, top 2, shared of the
+    experts' size: of 2,048 x 2,048 500 tokens 115 / 104, 1,024 152 / 136, 1,500 160 / 165, 2,047 221 / 190, 4,096 339 / 324; of 4,096 x
+    3,584 500 310 / 321, 1,024 438 / 398, 2,047 631 / 603; of 2,560 x 2,560 774 211 / 181, 3,000 428 / 391; shared of 3,072 beside 2,048:
+    1,024 158 / 164, 1,500 170 / 180, 2,047 238 / 207; of 8,192 1,500 199 / 240, 2,047 272 / 264, 4,096 424 / 397."""
+    if not isinstance(dense, TiledWeight) or dense.paired or x.dtype != torch.bfloat16 or not x.is_cuda or not up_w.tiled \
+            or dense.shape[0] != down_w.rows or (dense.cols > up_w.rows and T < 1800):
+        return False
+    lib, P = _lib.load(), T * top
+    rows = lib.sa_expert_tile_rows(P, up_w.experts, up_w.cols, up_w.rows, _code(x), x.stride(0), _ptr(x))
+    return rows == 128 and bool(lib.sa_expert_product_beside_takes(down_w.rows, up_w.rows, up_w.rows, P, rows, _ptr(dense.data), dense.cols,
+                                                                   _ptr(dense.data), dense.cols, T))
+
+
 def routed_experts(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, gate_w, up_w, down_w, activation: int,
                    *, shared: torch.Tensor | None = None, shared_gate: torch.Tensor | None = None,
                    out_dtype: torch.dtype | None = None, limit: float | None = None,
@@ -2240,8 +2256,9 @@ def expert_sums(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, g
                 shared: torch.Tensor | None = None, shared_gate: torch.Tensor | None = None, out_dtype: torch.dtype | None = None,
                 limit: float | None = None, order: tuple | None = None, dense: tuple | None = None) -> ExpertSums:
     """`routed_experts` with the sum over k left to the caller.
-    order: (sorted, plan) as `route_few` gives them (at most 16 tokens).  dense, with order: (hidden rows, down) of a shared
-    feed-forward, whose product with the tiled weight `down` runs beside the experts'; its rows take `shared`'s place, in 32 bits."""
+    order: (sorted, plan) as `route_few` gives them (at most 16 tokens).  dense, with order or where `experts_beside` says so: (hidden
+    rows, down) of a shared feed-forward, whose product with the tiled weight `down` runs beside the experts'; its rows take `shared`'s
+    place, with order in 32 bits."""
     _dev(x, experts, weights, gate_w.data if gate_w is not None else None, up_w.data, down_w.data, shared, shared_gate)
     T, D = x.shape
     top, E, F = experts.shape[1], up_w.experts, up_w.rows
@@ -2280,14 +2297,19 @@ def expert_sums(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, g
               int(gate_w is None), _stream())
     if dense is not None:
         hidden, d_down = dense
-        if order is None or shared is not None or not isinstance(d_down, TiledWeight) or d_down.paired \
+        if shared is not None or not isinstance(d_down, TiledWeight) or d_down.paired \
                 or tuple(d_down.shape) != (D, hidden.shape[1]) or hidden.shape[0] != T or hidden.dtype != x.dtype:
             raise KernelError("routed_experts: the shared feed-forward does not go with the experts")
         _dev(x, hidden, d_down.data)
-        shared = torch.empty((T, D), dtype=torch.float32, device=dev)
-        _lib.call("sa_expert_product_shared", _ptr(h), F, top, _ptr(down_w.data), D, F, _ptr(sorted_), _ptr(plan), P, E, _ptr(y), D,
-                  _ptr(hidden), _rows(hidden, "routed_experts: hidden rows"), _ptr(d_down.data), D, hidden.shape[1], T, _ptr(shared), D,
-                  _stream())
+        shared = torch.empty((T, D), dtype=x.dtype if order is None else torch.float32, device=dev)
+        if order is None:
+            _lib.call("sa_expert_product_beside", _ptr(h), F, top, _ptr(down_w.data), D, F, _ptr(sorted_), _ptr(plan), P, E, tile_rows,
+                      _ptr(y), D, _ptr(hidden), _rows(hidden, "routed_experts: hidden rows"), _ptr(d_down.data), hidden.shape[1], T,
+                      _ptr(shared), D, _stream())
+        else:
+            _lib.call("sa_expert_product_shared", _ptr(h), F, top, _ptr(down_w.data), D, F, _ptr(sorted_), _ptr(plan), P, E, _ptr(y), D,
+                      _ptr(hidden), _rows(hidden, "routed_experts: hidden rows"), _ptr(d_down.data), D, hidden.shape[1], T, _ptr(shared), D,
+                      _stream())
     else:
         _lib.call("sa_expert_product", _ptr(h), _code(h), F, 0, top, _ptr(down_w.data), None, D, F, _ptr(sorted_), _ptr(plan), P,
                   E, tile_rows, 0, 0.0, _ptr(y), D, 1, 0, _stream())

@@ -48,9 +48,11 @@ class Dense(FeedForward):
         self.up_proj = as_product_weight(tensors["up_proj"])
         self.down_proj = as_product_weight(tensors["down_proj"])
 
+    def first(self, x: torch.Tensor) -> torch.Tensor:
+        return ops.gemm(x, self.up_proj, activate=self.activation_code)   # (the activation is the product's epilogue)
+
     def forward(self, x: torch.Tensor, ctx=None, defer_sum=False) -> torch.Tensor:
-        z = ops.gemm(x, self.up_proj, activate=self.activation_code)   # (the activation is the product's epilogue)
-        return ops.gemm(z, self.down_proj, defer_sum=defer_sum)
+        return ops.gemm(self.first(x), self.down_proj, defer_sum=defer_sum)
 
 
 @FEED_FORWARDS.register("gated_dense")
@@ -83,15 +85,16 @@ class GatedDense(FeedForward):
             self.gate_up, self.gate_proj, self.up_proj = None, gate, up
         self.down_proj = as_product_weight(tensors["down_proj"])
 
-    def forward(self, x: torch.Tensor, ctx=None, defer_sum=False) -> torch.Tensor:
+    def first(self, x: torch.Tensor) -> torch.Tensor:
         # gelu(x.Wg^T) * (x.Wu^T), one kernel
         if self.gate_up is not None:
-            z = project(x, self.gate_up, activation=self.activation_code, limit=self.limit)
-        else:
-            if isinstance(x, PendingNorm):
-                x = x.materialize()
-            z = ops.gemm(x, self.gate_proj, w2=self.up_proj, activation=self.activation_code, limit=self.limit)
-        return ops.gemm(z, self.down_proj, defer_sum=defer_sum)
+            return project(x, self.gate_up, activation=self.activation_code, limit=self.limit)
+        if isinstance(x, PendingNorm):
+            x = x.materialize()
+        return ops.gemm(x, self.gate_proj, w2=self.up_proj, activation=self.activation_code, limit=self.limit)
+
+    def forward(self, x: torch.Tensor, ctx=None, defer_sum=False) -> torch.Tensor:
+        return ops.gemm(self.first(x), self.down_proj, defer_sum=defer_sum)
 
 
 @FEED_FORWARDS.register("routed_experts")
@@ -178,11 +181,14 @@ class RoutedExperts(FeedForward):
         if self.shared is not None:
             self.shared.load({n: tensors["shared." + n] for n in self.shared.param_specs()})
 
+    def _shared_is_known(self) -> bool:
+        """Whether the shared feed-forward is one of the parts here (what stands in its place, or overrides its forward(), is called as
+        ever)."""
+        return getattr(getattr(self.shared, "forward", None), "__func__", None) in (GatedDense.forward, Dense.forward)
+
     def _shared_beside(self) -> bool:
-        """Whether a few tokens' products of the shared feed-forward run beside the router and the experts: one of the parts here, not
-        too wide (what stands in its place, or overrides its forward(), is called as ever)."""
-        return getattr(getattr(self.shared, "forward", None), "__func__", None) in (GatedDense.forward, Dense.forward) \
-            and self.shared.intermediate_size <= ops.SHARED_BESIDE_MAX
+        """Whether a few tokens' products of the shared feed-forward run beside the router and the experts: known, and not too wide."""
+        return self._shared_is_known() and self.shared.intermediate_size <= ops.SHARED_BESIDE_MAX
 
     @knows_expert_sums
     def forward(self, x: torch.Tensor, ctx=None, defer_experts=False) -> "torch.Tensor | ops.ExpertSums":
@@ -212,10 +218,14 @@ class RoutedExperts(FeedForward):
                 experts, weights = ops.route(logits[:, :E], self.top, self.router_scale)
             else:
                 experts, weights = ops.route_choice(logits[:, :E], self.top, self.router_scale, **options)
-            shared = self.shared.forward(x, ctx) if self.shared is not None else None
+            # (many tokens: its second product in the last round of the experts')
+            if self._shared_is_known() and ops.experts_beside(x.shape[0], self.top, self.up_w, self.down_w, x, self.shared.down_proj):
+                dense = (self.shared.first(x), self.shared.down_proj)
+            elif self.shared is not None:
+                shared = self.shared.forward(x, ctx)
         args = (x, experts, weights, self.gate_w, self.up_w, self.down_w, self.activation_code)
         kw = dict(shared=shared, shared_gate=logits[:, E:E + 1] if self.shared_gate else None, limit=self.limit)
-        if order is None:
+        if order is None and dense is None:
             return ops.routed_experts(*args, **kw, **({"defer_sum": True} if defer else {}))
         sums = ops.expert_sums(*args, **kw, order=order, dense=dense)
         return sums if defer else sums.materialize()

@@ -169,3 +169,23 @@ def test_shared_feed_forwards_beside_the_experts_and_apart(shared):
         every = torch.stack([ff(f"e{e}.", "") for e in range(E)])
         want += best.values[:, k:k + 1] * every[best.indices[:, k], torch.arange(T, device="cuda")]
     assert float((got - want).norm() / want.norm()) <= 1.5 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("T,F,shared_F", [(600, 2048, 64), (1031, 2112, 2048), (1801, 2048, 4160)])
+def test_shared_product_beside_the_experts_of_many_tokens(gpu_lib, T, F, shared_F):
+    """The second product of a shared feed-forward in the launch of the experts' second products: the experts' rows to the bit those of the
+    launch without it, its own those of the wide kernel by itself with K uncut (the same order of sums)."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles, stack_experts
+    D, E, top = 2048, 16, 2
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    draw = lambda *shape: (torch.randn(shape, generator=gen, device="cuda") * 0.05).to(torch.bfloat16)
+    gate, up, down = (stack_experts([draw(r, c) for _ in range(E)]) for r, c in ((F, D), (F, D), (D, F)))
+    x, hidden, w = draw(T, D), draw(T, shared_F + 8)[:, :shared_F], draw(D, shared_F)
+    experts = torch.stack([torch.randperm(E, generator=gen, device="cuda")[:top] for _ in range(T)]).int().contiguous()
+    weights = torch.rand((T, top), generator=gen, device="cuda")
+    assert ops.experts_beside(T, top, up, down, x, pack_tiles(w))
+    args = (x, experts, weights, gate, up, down, ops.ACT_SILU)
+    apart, beside = ops.expert_sums(*args), ops.expert_sums(*args, dense=(hidden, pack_tiles(w)))
+    assert torch.equal(apart.y, beside.y)
+    assert torch.equal(beside.shared, ops.gemm(hidden, pack_tiles(w), algo=ops.ALGO_WIDE, shape=3128128))
