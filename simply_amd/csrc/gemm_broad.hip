@@ -43,6 +43,13 @@ __device__ __forceinline__ void each(F&& f) {
   }
 }
 
+// Two values rounded to bfloat16, the first in the lower half: one instruction (one by one they take a shift and an or besides).
+__device__ __forceinline__ uint32_t two_bf16(float a, float b) {
+  typedef __attribute__((ext_vector_type(2))) float floatx2;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{a, b}), bf16x2));
+}
+
 // 16 bytes per lane from base + offset + FROM bytes into LDS at byte address lds + TO + 16 * lane
 template <int FROM, int TO>
 __device__ __forceinline__ void load_block(const bf16* base, uint32_t offset, uint32_t lds) {
@@ -258,9 +265,7 @@ __global__ __launch_bounds__(256, 1) void gemm_broad_kernel(const bf16* __restri
   for (int i = 0; i < WM; ++i)
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
-      uint2 packed;
-      packed.x = static_cast<uint32_t>(float_to_bf16(acc[i][j][0]).bits) | (static_cast<uint32_t>(float_to_bf16(acc[i][j][1]).bits) << 16);
-      packed.y = static_cast<uint32_t>(float_to_bf16(acc[i][j][2]).bits) | (static_cast<uint32_t>(float_to_bf16(acc[i][j][3]).bits) << 16);
+      const uint2 packed{two_bf16(acc[i][j][0], acc[i][j][1]), two_bf16(acc[i][j][2], acc[i][j][3])};
       *reinterpret_cast<uint2*>(lds + ((wm * WM + i) * 16 + row) * PITCH + tile_of(j) * 16 + quad * 4) = packed;
     }
   __syncthreads();
@@ -271,15 +276,15 @@ __global__ __launch_bounds__(256, 1) void gemm_broad_kernel(const bf16* __restri
     for (int p = threadIdx.x; p < rows_here * PIECES; p += 256) {
       const int r = p / PIECES, c = p % PIECES, n = n_first + c * 8;
       if (n >= (EPI == 1 ? N : NL)) continue;
-      union Eight { uint4 q; uint16_t h[8]; } a, b, out;
+      union Eight { uint4 q; uint32_t w[4]; } a, b, out;   // (pairs of bfloat16)
       const __bf16* from = lds + r * PITCH + (EPI == 1 ? (c / 2) * 32 + c % 2 * 8 : c * 8);
       a.q = *reinterpret_cast<const uint4*>(from);
       if (EPI == 1) b.q = *reinterpret_cast<const uint4*>(from + 16);
       else b = a;
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        out.h[e] = float_to_bf16(value(__builtin_bit_cast(float, static_cast<uint32_t>(a.h[e]) << 16),
-                                       __builtin_bit_cast(float, static_cast<uint32_t>(b.h[e]) << 16))).bits;
+      for (int e = 0; e < 4; ++e)
+        out.w[e] = two_bf16(value(__uint_as_float(a.w[e] << 16), __uint_as_float(b.w[e] << 16)),
+                            value(__uint_as_float(a.w[e] & 0xffff0000u), __uint_as_float(b.w[e] & 0xffff0000u)));
       *reinterpret_cast<uint4*>(C + static_cast<size_t>(m_base + r) * ldc + n) = out.q;
     }
   };
