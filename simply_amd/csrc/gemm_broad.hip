@@ -1,10 +1,10 @@
 // C[M, N] = epilogue(A[M, K] . W[N, K]^T) in bfloat16 for many rows, on the largest tiles that a CU's registers hold: a workgroup of
 // four waves, one to a SIMD, has 256 x 288, 256 x 256, 192 x 288 or 192 x 256 outputs, a wave a quarter of them.
 //   * What bounds it: the matrix units' power.  With every CU at work they are busy 72 % of the cycles at 1.93 GHz (2,048 rows, 8,192
-//     outputs, K = 8,192: 188 us, 1.46 PFLOP/s; the wide kernel 250); loads left out the same loop takes 25 % less time, half of
-//     that by the clock.  A wave's 128 x 144 outputs need 17 fragment reads for 72 products where the wide kernel's 64 x 96 need 10
-//     for 24, and a tile of 256 x 288 brings 34 KiB into LDS for 144 products a SIMD where two of 128 x 192 bring 40 for 96: what is
-//     moved for a product is what the power can be saved on.
+//     outputs, K = 8,192: 188 us, 1.46 PFLOP/s); with the loads left out the same loop takes 25 % less time, in part by the clock.
+//     A wave's 128 x 144 outputs need 17 fragment reads for 72 products where the wide kernel's 64 x 96 need 10 for 24, and a tile of
+//     256 x 288 brings 34 KiB into LDS for 72 products a SIMD where two of 128 x 192 bring 40 for 48: what is moved for a product
+//     is what power can be saved on.
 //   * Layout in LDS: W as KiB blocks in MFMA operand order, which is how it lies in global memory, in a ring of halves (32 columns
 //     of K); A as rows of 128 bytes (whole lines), their 16-byte pieces permuted by the row's number against bank conflicts, in a
 //     ring of slabs (64 columns).  The rings are as deep as 160 KiB allow: three slabs of A, three or four halves of W, so that a
@@ -18,7 +18,6 @@
 // Before (the wide kernel) and now, us: gated, 2,048 rows of the 2B feed-forward 159 / 134, 8,192 rows 578 / 511, 1,056
 // rows of the 27B one 649 / 593; 2,048 rows against 8,192 outputs of K = 2,048 66 / 56, 4,096 cubed 110 / 95.
 #include "api.h"
-
 #include "slabs.h"
 
 namespace sa {
