@@ -126,6 +126,8 @@ int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t workspace_byte
 // Where the broad kernel takes its place (output rows of whole 16-byte pieces): cuts of K * 1000000 + rows * 1000 + weight rows of
 // a tile, else 0.  A host function.
 int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t workspace_bytes);
+// Where it takes the whole sections of n_step outputs of sa_gemm_sections: rows * 1000 + weight rows of a tile, else 0.  A host function.
+int sa_gemm_sections_tile(int M, int N, int K, int n_step, int64_t workspace_bytes);
 // Which way the 32-bit matrix-core kernels take M rows: 16 (few rows), or the rows of a tile (32, 64 or 128), plus 1000 where K
 // is cut over workgroups, plus 10000 times the weight rows of a tile.  A host function.
 int sa_gemm_f32_plan(int M, int N, int K, int gated, int64_t workspace_bytes);

@@ -573,6 +573,20 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
   return us;
 }
 
+// Several products at once (sections of n_step outputs, 0: one product): the broad kernel's tile for the whole sections where they on it and
+// a shorter last one by itself (at 2,047 rows of four sections of 2,048 outputs it would be eight more tiles behind a full round) are
+// ahead of planned_us, the wide kernel's time; else 0, as where no section is whole.  Measured, us, wide / broad and the rest: 2,047 rows of
+// four sections of 2,048 and 64 outputs 74 / 65, 4,096 rows 138 / 120; sections of 4,096, 1,024 rows 163 / 115, 2,047 275 / 218, 512
+// 92 / 96; of 1,024, 2,047 rows 27 / 35, 4,096 53 / 41.
+static int sections_broad_tile(int M, int N, int K, int n_step, bool have_workspace, size_t workspace_bytes, double planned_us) {
+  if (n_step <= 0 || N < n_step || M < 96) return 0;
+  const int whole = N / n_step, rest = N % n_step;
+  int tile = 0, one = 1;
+  double us = gemm_broad_plan(M, whole * n_step, K, 0, false, 0, tile, one, n_step);
+  if (rest > 0) us += fmin(gemm_tiled_predict_us(M, rest, K, 0), gemm_wide_predict_us(M, rest, K, 0, have_workspace, workspace_bytes));
+  return us < 0.98 * planned_us ? tile : 0;
+}
+
 // shape: 0: chosen here; else stages * 1000000 + rows * 1000 + weight rows of a workgroup's tile (2256192, 3256128,
 // 3128256, 3192128; 2128192: workgroups of four waves, two to a CU).
 // ks > 1 cuts K over that many workgroups per tile (no epilogue only; the partial tiles go through `workspace`,
@@ -599,22 +613,15 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
     set_error("gemm: the broad tiles want widths and rows of whole pieces of eight columns");
     return 1;
   }
-  // Several products at once: where the broad kernel's tiles are ahead for the whole sections, they run on it and a shorter last one
-  // by itself (at 2,047 rows of four sections of 2,048 outputs it would be eight more tiles behind a full round).  Measured, us,
-  // wide / broad and the rest: 2,047 rows of four sections of 2,048 and 64 outputs 74 / 65, 4,096 rows 138 / 120; sections of 4,096, 1,024
-  // rows 163 / 115, 2,047 275 / 218, 512 92 / 96; of 1,024, 2,047 rows 27 / 35, 4,096 53 / 41.
-  if (planned && broad && sec.n_step > 0 && c_dtype == kBF16) {
+  // Several products at once: where the broad kernel's tiles are ahead, the whole sections run on it and a shorter last one by itself.
+  const int broad_tile = planned && broad && c_dtype == kBF16 ? sections_broad_tile(M, N, K, sec.n_step, ws != nullptr, workspace_bytes, planned_us) : 0;
+  if (broad_tile > 0) {
     const int whole = N / sec.n_step, rest = N % sec.n_step;
-    int tile = 0, one = 1;
-    const double whole_us = gemm_broad_plan(M, whole * sec.n_step, K, 0, false, 0, tile, one, sec.n_step);
-    const double rest_us = rest > 0 ? fmin(gemm_tiled_predict_us(M, rest, K, 0), gemm_wide_predict_us(M, rest, K, 0, ws != nullptr, workspace_bytes)) : 0.0;
-    if (whole > 0 && M >= 96 && whole_us + rest_us < 0.98 * planned_us) {
-      gemm_broad(tile, a, lda, w, c, ldc, M, whole * sec.n_step, K, 0, 0, 0.f, 1, nullptr, false, sec, stream);
-      if (check_launch("gemm_broad")) return 1;
-      const size_t at = static_cast<size_t>(whole) * sec.n_step;
-      return rest == 0 ? 0 : sa_gemm(a + static_cast<size_t>(whole) * sec.a_step, kBF16, lda, w + at * K, nullptr, kBF16, c + at, kBF16, ldc,
-                                     M, rest, K, 0, 0.f, 0, 1, 0, workspace, static_cast<int64_t>(workspace_bytes), stream);
-    }
+    gemm_broad(broad_tile, a, lda, w, c, ldc, M, whole * sec.n_step, K, 0, 0, 0.f, 1, nullptr, false, sec, stream);
+    if (check_launch("gemm_broad")) return 1;
+    const size_t at = static_cast<size_t>(whole) * sec.n_step;
+    return rest == 0 ? 0 : sa_gemm(a + static_cast<size_t>(whole) * sec.a_step, kBF16, lda, w + at * K, nullptr, kBF16, c + at, kBF16, ldc,
+                                   M, rest, K, 0, 0.f, 0, 1, 0, workspace, static_cast<int64_t>(workspace_bytes), stream);
   }
   // 32-bit results: the cuts' partial sums as they are, of one cut straight into C (whose rows are contiguous)
   const bool raw = ks > 1 || c_dtype == kF32;
@@ -676,4 +683,12 @@ extern "C" int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t wor
   const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
   sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks);
   return shape / 1000000 == 1 ? (ks - 1) * 1000000 + shape : 0;
+}
+
+extern "C" int sa_gemm_sections_tile(int M, int N, int K, int n_step, int64_t workspace_bytes) {
+  if (M < 1 || N < 1 || K < 1 || n_step < 1) return 0;
+  int shape = 0, ks = 1;
+  const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
+  const double us = sa::plan_shape(M, N, K, 0, bytes > 0, bytes, shape, ks, false);
+  return sa::sections_broad_tile(M, N, K, n_step, bytes > 0, bytes, us);
 }

@@ -124,3 +124,23 @@ def test_many_rows_against_a_handful_of_outputs(gpu_lib, M, N, K):
     out = torch.full((M, N + 3), 7.0, device="cuda")
     ops.gemm(a, tw, out=out[:, 2:2 + N])
     assert torch.equal(out[:, 2:2 + N], got) and (out[:, :2] == 7.0).all() and (out[:, 2 + N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("M", [1, 96, 512, 4096])
+def test_plan_of_a_lone_section_shorter_than_a_step(M):
+    """No whole section: nothing for the broad kernel (its plan of no outputs divided by their tiles)."""
+    from simply_amd.kernels import lib
+    for N in (16, 1024, 2047):
+        assert lib.load().sa_gemm_sections_tile(M, N, 2048, 2048, 256 << 20) == 0
+
+
+@pytest.mark.gpu
+def test_a_lone_section_shorter_than_a_step(gpu_lib):
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+    M, N, K = 512, 1024, 2048
+    a, w = rand((M, K), torch.bfloat16, 80), rand((N, K), torch.bfloat16, 81, 0.05)
+    tw, out, ws = pack_tiles(w), torch.empty((M, N), dtype=torch.bfloat16, device="cuda"), ops._workspace(a.device)
+    gpu_lib.call("sa_gemm_sections", a.data_ptr(), K, tw.data.data_ptr(), out.data_ptr(), 1, N, M, N, K, 2048, K, ws.data_ptr(), ws.numel(),
+                 ops._stream())
+    check(out, ref.gemm(a, w), bf16_steps=1.0)
