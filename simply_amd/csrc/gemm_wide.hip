@@ -468,6 +468,14 @@ bool gemm_wide_takes(int M, int N, int K, int64_t lda, int64_t ldc, const void* 
          static_cast<int64_t>(M) * lda < (int64_t{1} << 31);  // byte offsets of rows are kept in 32 bits
 }
 
+// The time of an uncut product on tiles of `shape`, `columns` of them side by side: their rounds of slabs at what 128 outputs of 256 rows (or
+// as many of another tile) take, fitted like the broad kernel's.
+static double rounds_us(int shape, int M, int64_t columns, int NW, int K, int epi) {
+  const int rows = shape / 1000 % 1000, wrows = shape % 1000;
+  const int64_t rounds = ((M + rows - 1) / rows * columns + wide::kCUs - 1) / wide::kCUs;
+  return fmax(5.0 + 2.0 * NW * K / 5.8e6, 3.0 + rounds * ((epi == 1 ? 0.88 : 0.78) * (K / wide::BK) * rows * wrows / 32768.0 + 2.8));
+}
+
 // The tile and the cut of K for a product whose caller fixes neither, and the time that this kernel is expected to
 // take with them in microseconds (the figure by which the library chooses between its product kernels).
 static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& shape, int& ks, bool broad = true) {
@@ -550,18 +558,13 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     if (best_us >= 0) us = fmax(best_us, 5.0 + 0.02 * (M < 64 ? M : 64) + 2.0 * NW_all * K / 5.8e6);
   }
   // The tiles of the broad kernel against all of these.  What the others take beyond 1,536 rows or gated, where no model above
-  // says it: their rounds of slabs at what 128 outputs of 256 rows (or as many of another tile) take, fitted like the broad ones.
+  // says it: rounds_us.
   // (Behind other kernels, weights in HBM, the broad tiles keep their time better than in a loop of the one product, by which both are
   // fitted: 2,048 rows against 6,144 outputs of K = 2,048 49 and 49 us there, 60 and 49 in a prompt.  Hence the line at 1.03; at 1.12
   // prompts are 0.3 to 1 % slower again.)
   if (broad && M >= 96) {
     double other = us;
-    if (epi == 1 || (M > 1536 && !few_tiles)) {
-      const int rows = shape / 1000 % 1000, wrows = shape % 1000;
-      const int64_t tiles = static_cast<int64_t>((M + rows - 1) / rows) * ((NW + wrows - 1) / wrows);
-      const int64_t rounds = (tiles + wide::kCUs - 1) / wide::kCUs;
-      other = fmax(5.0 + 2.0 * NW_all * K / 5.8e6, 3.0 + rounds * ((epi == 1 ? 0.88 : 0.78) * (K / wide::BK) * rows * wrows / 32768.0 + 2.8));
-    }
+    if (epi == 1 || (M > 1536 && !few_tiles)) other = rounds_us(shape, M, (NW + shape % 1000 - 1) / (shape % 1000), NW_all, K, epi);
     int broad_tile = 0, cut = ks;
     const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, broad_tile, cut);
     if (broad_us < 1.03 * other) {
@@ -575,15 +578,19 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
 
 // Several products at once (sections of n_step outputs, 0: one product): the broad kernel's tile for the whole sections where they on it and
 // a shorter last one by itself (at 2,047 rows of four sections of 2,048 outputs it would be eight more tiles behind a full round) are
-// ahead of planned_us, the wide kernel's time; else 0, as where no section is whole.  Measured, us, wide / broad and the rest: 2,047 rows of
-// four sections of 2,048 and 64 outputs 74 / 65, 4,096 rows 138 / 120; sections of 4,096, 1,024 rows 163 / 115, 2,047 275 / 218, 512
-// 92 / 96; of 1,024, 2,047 rows 27 / 35, 4,096 53 / 41.
-static int sections_broad_tile(int M, int N, int K, int n_step, bool have_workspace, size_t workspace_bytes, double planned_us) {
+// ahead of the wide kernel's `shape` and cut of K, whose time is planned_us; else 0, as where no section is whole.  Measured, us, wide / broad
+// and the rest: 2,047 rows of four sections of 2,048 and 64 outputs 78 / 63, of three and 16 55 / 56, 1,031 rows of four 49 / 46, 4,096
+// 140 / 120; sections of 4,096, 700 rows 108 / 89, 1,024 without a rest 125 / 112, 2,500 334 / 284; of 1,024, 3,000 rows 45 / 31, 4,096
+// without a rest 42 / 34.
+static int sections_broad_tile(int M, int N, int K, int n_step, bool have_workspace, size_t workspace_bytes, int shape, int ks, double planned_us) {
   if (n_step <= 0 || N < n_step || M < 96) return 0;
   const int whole = N / n_step, rest = N % n_step;
   int tile = 0, one = 1;
   double us = gemm_broad_plan(M, whole * n_step, K, 0, false, 0, tile, one, n_step);
   if (rest > 0) us += fmin(gemm_tiled_predict_us(M, rest, K, 0), gemm_wide_predict_us(M, rest, K, 0, have_workspace, workspace_bytes));
+  const int wrows = shape % 1000;
+  const int64_t columns = static_cast<int64_t>(whole) * ((n_step + wrows - 1) / wrows) + (rest + wrows - 1) / wrows;
+  if (ks == 1) planned_us = rounds_us(shape, M, columns, N, K, 0);   // (the plan of one product knows no sections)
   return us < 0.98 * planned_us ? tile : 0;
 }
 
@@ -614,7 +621,7 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
     return 1;
   }
   // Several products at once: where the broad kernel's tiles are ahead, the whole sections run on it and a shorter last one by itself.
-  const int broad_tile = planned && broad && c_dtype == kBF16 ? sections_broad_tile(M, N, K, sec.n_step, ws != nullptr, workspace_bytes, planned_us) : 0;
+  const int broad_tile = planned && broad && c_dtype == kBF16 ? sections_broad_tile(M, N, K, sec.n_step, ws != nullptr, workspace_bytes, shape, ks, planned_us) : 0;
   if (broad_tile > 0) {
     const int whole = N / sec.n_step, rest = N % sec.n_step;
     gemm_broad(broad_tile, a, lda, w, c, ldc, M, whole * sec.n_step, K, 0, 0, 0.f, 1, nullptr, false, sec, stream);
@@ -690,5 +697,5 @@ extern "C" int sa_gemm_sections_tile(int M, int N, int K, int n_step, int64_t wo
   int shape = 0, ks = 1;
   const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
   const double us = sa::plan_shape(M, N, K, 0, bytes > 0, bytes, shape, ks, false);
-  return sa::sections_broad_tile(M, N, K, n_step, bytes > 0, bytes, us);
+  return sa::sections_broad_tile(M, N, K, n_step, bytes > 0, bytes, shape, ks, us);
 }

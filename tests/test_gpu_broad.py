@@ -70,7 +70,7 @@ def test_broad_tiles_where_they_are_ahead():
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,n,last,K", [(4096, 1024, 64, 1024), (1031, 2048, 2048, 1088), (2047, 2048, 16, 2048)])
 def test_sections_on_broad_tiles(gpu_lib, M, n, last, K):
-    """Several products at once of so many rows that the whole sections go to the broad kernel, a shorter last one by itself."""
+    """Several products at once of many rows, with a last section that is shorter (on the wide kernel) or whole (on the broad one)."""
     from simply_amd.kernels import ops
     ws = [rand((last if s == 3 else n, K), torch.bfloat16, 20 + s, 0.05) for s in range(4)]
     a = rand((M, 4 * K), torch.bfloat16, 30)
@@ -144,3 +144,26 @@ def test_a_lone_section_shorter_than_a_step(gpu_lib):
     gpu_lib.call("sa_gemm_sections", a.data_ptr(), K, tw.data.data_ptr(), out.data_ptr(), 1, N, M, N, K, 2048, K, ws.data_ptr(), ws.numel(),
                  ops._stream())
     check(out, ref.gemm(a, w), bf16_steps=1.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,n,sections,last,K", [(2047, 2048, 4, 64, 2048), (2047, 2048, 4, 16, 2048), (700, 4096, 4, 64, 4096), (3000, 1024, 4, 64, 1024),
+                                                 (1500, 2048, 4, 304, 2048)])
+def test_whole_sections_on_broad_tiles_and_a_shorter_last_one(gpu_lib, M, n, sections, last, K):
+    """The whole sections in the broad kernel's launch, the last one by itself from where they end: its rows of W, its columns of A and C."""
+    from simply_amd.kernels import ops
+    assert gpu_lib.load().sa_gemm_sections_tile(M, sections * n + last, K, n, ops.WORKSPACE_BYTES) > 0
+    ws = [rand((last if s == sections else n, K), torch.bfloat16, 90 + s, 0.05) for s in range(sections + 1)]
+    big = rand((M, (sections + 1) * K + 16), torch.bfloat16, 99)
+    a = big[:, 8:8 + (sections + 1) * K]
+    got = ops.gemm_sections(a, ops.SectionedWeight(ws))
+    for s, w in enumerate(ws):
+        check(got[:, s * n:s * n + w.shape[0]], ref.gemm(a[:, s * K:(s + 1) * K], w), bf16_steps=1.0)
+
+
+def test_sections_where_the_broad_tiles_are_ahead():
+    """(M, outputs, K, n_step): by the rounds of the wide kernel's tiles against those of the broad one's, for prompts and shorter portions."""
+    from simply_amd.kernels import lib
+    tile = lambda *at: lib.load().sa_gemm_sections_tile(*at, 256 << 20)
+    assert tile(2047, 8256, 2048, 2048) == 256256 and tile(1024, 16384, 4096, 4096) == 256256 and tile(3000, 4160, 1024, 1024) == 192256
+    assert tile(512, 16384, 4096, 4096) == tile(2047, 4096, 1024, 1024) == tile(774, 8256, 2048, 2048) == tile(64, 8256, 2048, 2048) == 0
