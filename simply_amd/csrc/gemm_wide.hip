@@ -480,6 +480,7 @@ static double rounds_us(int shape, int M, int64_t columns, int NW, int K, int ep
 // take with them in microseconds (the figure by which the library chooses between its product kernels).
 static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& shape, int& ks, bool broad = true) {
   const int NW_all = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N;
+  const int asked = ks;   // the caller's cut of K, 1: none
   // without a fitted model below: the weights streamed once at the rate this kernel reaches for few rows, or the
   // products at its rate for many, whichever takes longer, after its start
   double us = 5.0 + 0.02 * (M < 64 ? M : 64) +
@@ -563,14 +564,29 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
   // fitted: 2,048 rows against 6,144 outputs of K = 2,048 49 and 49 us there, 60 and 49 in a prompt.  Hence the line at 1.03; at 1.12
   // prompts are 0.3 to 1 % slower again.)
   if (broad && M >= 96) {
-    double other = us;
-    if (epi == 1 || (M > 1536 && !few_tiles)) other = rounds_us(shape, M, (NW + shape % 1000 - 1) / (shape % 1000), NW_all, K, epi);
-    int broad_tile = 0, cut = ks;
-    const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, broad_tile, cut);
-    if (broad_us < 1.03 * other) {
-      shape = 1000000 + broad_tile;
+    const bool fitted = epi == 0 && (M <= 1536 || few_tiles);
+    double best_us = fitted ? us : rounds_us(shape, M, (NW + shape % 1000 - 1) / (shape % 1000), NW_all, K, epi);
+    // With the cut that the tiles above take, or where they take none any.  (More than three cuts of few rows cost more than the broad
+    // kernel's model says: 160 rows of 9,216 against 2,304 outputs with 14 cuts 23 and 28 us, 896 with four 49 and 56, 129 of 8,192
+    // against 2,048 with 16 20 and 24, all expected at about the same.)
+    int tile = 0, cut = ks;
+    const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, tile, cut);
+    if (broad_us < (fitted && cut > 3 ? 0.94 : 1.03) * best_us) {
+      shape = 1000000 + tile;
       ks = cut;
-      us = broad_us;
+      us = best_us = broad_us;
+    }
+    // With a cut of their own beside tiles that are cut too, which was found for tiles of another size, only well ahead: 544 rows of 36,864
+    // against 4,608 outputs 216 / 178 us, 640 261 / 217, of 14,336 against 6,144 320 rows 87 / 76, against 4,096 544 rows 85 / 76.  Of 80
+    // sizes that the model has up to 8 % ahead or behind 61 were slower (129 rows of 4,096 against 12,288, by the model 7 % ahead, by 14 %).
+    if (asked == 1 && cut > 1) {
+      int own_tile = 0, own_cut = 1;
+      const double own_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, own_tile, own_cut);
+      if (own_cut > 1 && own_us < 0.92 * best_us) {
+        shape = 1000000 + own_tile;
+        ks = own_cut;
+        us = own_us;
+      }
     }
   }
   return us;

@@ -167,3 +167,30 @@ def test_sections_where_the_broad_tiles_are_ahead():
     tile = lambda *at: lib.load().sa_gemm_sections_tile(*at, 256 << 20)
     assert tile(2047, 8256, 2048, 2048) == 256256 and tile(1024, 16384, 4096, 4096) == 256256 and tile(3000, 4160, 1024, 1024) == 192256
     assert tile(512, 16384, 4096, 4096) == tile(2047, 4096, 1024, 1024) == tile(774, 8256, 2048, 2048) == tile(64, 8256, 2048, 2048) == 0
+
+
+def test_broad_tiles_with_a_cut_of_their_own():
+    """Beside tiles whose K is cut too: a cut for the broad tiles' size well ahead, the other tiles' cut where it serves both, else the others."""
+    from simply_amd.kernels import lib
+    tile = lambda *at: lib.load().sa_gemm_broad_tile(*at, 0, 256 << 20)
+    assert tile(544, 4608, 36864) == 5192288 and tile(320, 6144, 14336) == 5192256 and tile(1024, 4608, 36864) == 4256288
+    assert tile(1056, 4608, 36864) == 3256288
+    assert tile(160, 2304, 9216) == tile(896, 2304, 9216) == tile(129, 2048, 8192) == tile(129, 12288, 4096) == 0
+    # a workspace that holds two of the five planes, or none
+    two = 2 * 544 * 4608 * 4
+    assert lib.load().sa_gemm_broad_tile(544, 4608, 36864, 0, two) // 1000000 <= 2
+    assert lib.load().sa_gemm_broad_tile(544, 4608, 36864, 0, 0) // 1000000 <= 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(544, 4096, 14336), (320, 6144, 14336)])
+def test_gemm_takes_broad_tiles_with_a_cut_of_their_own(gpu_lib, M, N, K):
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+    assert gpu_lib.load().sa_gemm_broad_tile(M, N, K, 0, ops.WORKSPACE_BYTES) // 1000000 > 1
+    a, w = rand((M, K), torch.bfloat16, 110), rand((N, K), torch.bfloat16, 111, 0.02)
+    tw, want = pack_tiles(w), ref.gemm(a, w)
+    check(ops.gemm(a, tw), want, bf16_steps=1.0)
+    left = ops.gemm(a, tw, defer_sum=True)
+    assert isinstance(left, ops.PartialSums)
+    check(left.materialize(), want, bf16_steps=1.0)
