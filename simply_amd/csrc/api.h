@@ -124,8 +124,9 @@ int sa_gemm_plan(int M, int N, int K, int epilogue, int c_dtype, int64_t workspa
 // The wide kernel's tile for them (epilogue 0 or 1): stages * 1000000 + rows * 1000 + weight rows.  A host function.
 int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t workspace_bytes);
 // Where the broad kernel takes its place (output rows of whole 16-byte pieces): cuts of K * 1000000 + rows * 1000 + weight rows of
-// a tile, else 0.  A host function.
+// a tile, else 0.  _planes_: for sa_gemm_planes, whose caller adds the cuts up.  Host functions.
 int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t workspace_bytes);
+int sa_gemm_planes_broad_tile(int M, int N, int K, int64_t workspace_bytes);
 // Where it takes the whole sections of n_step outputs of sa_gemm_sections: rows * 1000 + weight rows of a tile, else 0.  A host function.
 int sa_gemm_sections_tile(int M, int N, int K, int n_step, int64_t workspace_bytes);
 // Which way the 32-bit matrix-core kernels take M rows: 16 (few rows), or the rows of a tile (32, 64 or 128), plus 1000 where K
@@ -284,10 +285,12 @@ bool gemm_narrow_takes(int M, int N, int K);
 double gemm_narrow_predict_us(int M, int N, int K);
 int gemm_narrow(const void* A, int64_t lda, const void* W, void* C, int c_dtype, int64_t ldc, int M, int N, int K, hipStream_t stream);
 double gemm_tiled_predict_us(int M, int N, int K, int epi);
-double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks, int n_step = 0);
+double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks, double behind_us,
+                       int n_step = 0);
 void gemm_broad(int tile, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int epi,
                 int act, float limit, int ks, float* partials, bool raw, Sections sec, hipStream_t stream);
-double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes);
+// planes: where K is cut the caller adds the planes up (no sum kernel behind the product).
+double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, bool planes);
 // The experts' products on the wide kernel (plan, sorted: of the sort kernel with tiles of tile_rows rows, 64 or 128).
 bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t ldc, const void* A, const void* W, const void* W2,
                             const void* C, int tile_rows);

@@ -319,8 +319,10 @@ static void launch(const bf16* A, int64_t lda, const bf16* W, bf16* C, int64_t l
 
 // The tile (rows * 1000 + weight rows) and cut of K that this kernel is expected to be fastest with, and its microseconds: full
 // rounds of 256 workgroups, and a last one whose slabs take the less time the fewer CUs have one (the clock rises), fitted to 27
-// sizes of weights from 1,024 x 1,024 to 73,728 x 4,608 at 256 to 3,072 rows (3 to 6 % root mean square).
-double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks, int n_step) {
+// sizes of weights from 1,024 x 1,024 to 73,728 x 4,608 at 256 to 3,072 rows (3 to 6 % root mean square).  behind_us: what a cut costs the
+// caller behind the product, beside the planes' bytes.
+double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& tile, int& ks, double behind_us,
+                       int n_step) {
   struct Tile { int rows, wrows; double alone, full, start; };   // us a slab alone and with every CU at work; us a round
   static const Tile tiles[4] = {{256, 288, 0.99, 1.45, 7.6}, {256, 256, 0.89, 1.35, 6.4}, {192, 288, 0.80, 1.19, 5.2}, {192, 256, 0.76, 1.05, 4.0}};
   const int NW = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N, slabs = K / broad::BK;
@@ -340,7 +342,7 @@ double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t
       const int per = (slabs + cut - 1) / cut;
       double us = 3.0 + full * (per * t.full + t.start);
       if (rest > 0) us += per * (t.alone + (t.full - t.alone) * rest) + t.start;
-      if (cut > 1) us += partial_bytes / 8e6 + partial_bytes / 5.5e6;   // written, and read again by whoever adds them up
+      if (cut > 1) us += partial_bytes / 8e6 + partial_bytes / 5.5e6 + behind_us;   // written, and read again by whoever adds them up
       if (best < 0 || us < best) best = us, tile = t.rows * 1000 + t.wrows, cut_out = cut;
     }
   }

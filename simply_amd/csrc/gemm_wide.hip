@@ -478,7 +478,7 @@ static double rounds_us(int shape, int M, int64_t columns, int NW, int K, int ep
 
 // The tile and the cut of K for a product whose caller fixes neither, and the time that this kernel is expected to
 // take with them in microseconds (the figure by which the library chooses between its product kernels).
-static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& shape, int& ks, bool broad = true) {
+static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, int& shape, int& ks, bool planes, bool broad = true) {
   const int NW_all = epi == 1 ? 2 * ((N + 15) / 16) * 16 : N;
   const int asked = ks;   // the caller's cut of K, 1: none
   // without a fitted model below: the weights streamed once at the rate this kernel reaches for few rows, or the
@@ -569,9 +569,15 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     // With the cut that the tiles above take, or where they take none any.  (More than three cuts of few rows cost more than the broad
     // kernel's model says: 160 rows of 9,216 against 2,304 outputs with 14 cuts 23 and 28 us, 896 with four 49 and 56, 129 of 8,192
     // against 2,048 with 16 20 and 24, all expected at about the same.)
+    // Beyond 1,536 rows the tiles above are not cut: where the sum is a kernel of its own, it counts, and cuts are taken only ahead (3,072 rows of
+    // 9,216 against 2,304 outputs in two cuts 112 / 115 us with the sum, 132 / 127 with a norm that adds them up, 4,096 of 16,384 against
+    // 2,048 207 / 219 and 230 / 229, 1,600 of 4,096 against 1,024 in seven 28 / 32).  The pass for an activation behind a cut does not: it takes
+    // what the code in an uncut product's epilogue takes (2,304 outputs of 9,216, erf GELU, 4,096 rows: 18 us and 19).
+    const double behind_us = fitted || planes ? 0.0 : 3.7;
     int tile = 0, cut = ks;
-    const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, tile, cut);
-    if (broad_us < (fitted && cut > 3 ? 0.94 : 1.03) * best_us) {
+    const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, tile, cut, behind_us);
+    const double line = cut == 1 ? 1.03 : fitted ? (cut > 3 ? 0.94 : 1.03) : planes ? 1.03 : 0.96;
+    if (broad_us < line * best_us) {
       shape = 1000000 + tile;
       ks = cut;
       us = best_us = broad_us;
@@ -581,7 +587,7 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     // sizes that the model has up to 8 % ahead or behind 61 were slower (129 rows of 4,096 against 12,288, by the model 7 % ahead, by 14 %).
     if (asked == 1 && cut > 1) {
       int own_tile = 0, own_cut = 1;
-      const double own_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, own_tile, own_cut);
+      const double own_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, own_tile, own_cut, behind_us);
       if (own_cut > 1 && own_us < 0.92 * best_us) {
         shape = 1000000 + own_tile;
         ks = own_cut;
@@ -602,8 +608,8 @@ static int sections_broad_tile(int M, int N, int K, int n_step, bool have_worksp
   if (n_step <= 0 || N < n_step || M < 96) return 0;
   const int whole = N / n_step, rest = N % n_step;
   int tile = 0, one = 1;
-  double us = gemm_broad_plan(M, whole * n_step, K, 0, false, 0, tile, one, n_step);
-  if (rest > 0) us += fmin(gemm_tiled_predict_us(M, rest, K, 0), gemm_wide_predict_us(M, rest, K, 0, have_workspace, workspace_bytes));
+  double us = gemm_broad_plan(M, whole * n_step, K, 0, false, 0, tile, one, 0.0, n_step);
+  if (rest > 0) us += fmin(gemm_tiled_predict_us(M, rest, K, 0), gemm_wide_predict_us(M, rest, K, 0, have_workspace, workspace_bytes, false));
   const int wrows = shape % 1000;
   const int64_t columns = static_cast<int64_t>(whole) * ((n_step + wrows - 1) / wrows) + (rest + wrows - 1) / wrows;
   if (ks == 1) planned_us = rounds_us(shape, M, columns, N, K, 0);   // (the plan of one product knows no sections)
@@ -631,7 +637,7 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
   const bool broad = N % 8 == 0 && ldc % 8 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
   const bool planned = shape == 0;
   double planned_us = 0.0;
-  if (planned) planned_us = plan_shape(M, N, K, epi, ws != nullptr, workspace_bytes, shape, ks, broad && sec.n_step == 0);
+  if (planned) planned_us = plan_shape(M, N, K, epi, ws != nullptr, workspace_bytes, shape, ks, planes_left != nullptr, broad && sec.n_step == 0);
   if (shape / 1000000 == 1 && !broad) {
     set_error("gemm: the broad tiles want widths and rows of whole pieces of eight columns");
     return 1;
@@ -685,9 +691,9 @@ int gemm_wide(const void* A, int64_t lda, const void* W, void* C, int64_t ldc, i
 }
 
 
-double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes) {
+double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, bool planes) {
   int shape = 0, ks = 1;
-  return plan_shape(M, N, K, epi, have_workspace, workspace_bytes, shape, ks);
+  return plan_shape(M, N, K, epi, have_workspace, workspace_bytes, shape, ks, planes);
 }
 
 }  // namespace sa
@@ -696,22 +702,30 @@ extern "C" int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t wor
   if (M < 1 || N < 1 || K < 1 || epilogue < 0 || epilogue > 1) return 0;
   int shape = 0, ks = 1;
   const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
-  sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks, false);
+  sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks, false, false);
   return shape;
 }
 
-extern "C" int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t workspace_bytes) {
-  if (M < 1 || N < 1 || K < 1 || epilogue < 0 || epilogue > 1) return 0;
+static int broad_tile(int M, int N, int K, int epi, int64_t workspace_bytes, bool planes) {
+  if (M < 1 || N < 1 || K < 1 || epi < 0 || epi > 1) return 0;
   int shape = 0, ks = 1;
   const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
-  sa::plan_shape(M, N, K, epilogue, bytes > 0, bytes, shape, ks);
+  sa::plan_shape(M, N, K, epi, bytes > 0, bytes, shape, ks, planes);
   return shape / 1000000 == 1 ? (ks - 1) * 1000000 + shape : 0;
+}
+
+extern "C" int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t workspace_bytes) {
+  return broad_tile(M, N, K, epilogue, workspace_bytes, false);
+}
+
+extern "C" int sa_gemm_planes_broad_tile(int M, int N, int K, int64_t workspace_bytes) {
+  return broad_tile(M, N, K, 0, workspace_bytes, true);
 }
 
 extern "C" int sa_gemm_sections_tile(int M, int N, int K, int n_step, int64_t workspace_bytes) {
   if (M < 1 || N < 1 || K < 1 || n_step < 1) return 0;
   int shape = 0, ks = 1;
   const size_t bytes = workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0;
-  const double us = sa::plan_shape(M, N, K, 0, bytes > 0, bytes, shape, ks, false);
+  const double us = sa::plan_shape(M, N, K, 0, bytes > 0, bytes, shape, ks, false, false);
   return sa::sections_broad_tile(M, N, K, n_step, bytes > 0, bytes, shape, ks, us);
 }

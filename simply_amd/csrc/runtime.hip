@@ -86,7 +86,7 @@ static int gemm_routed(const void* A, int a_dtype, int64_t lda, const void* W, c
     double best = -1.0;
     const double us[3] = {skinny_ok ? gemm_skinny_predict_us(M, N, K, epilogue) : -1.0,
                           tiled_ok ? gemm_tiled_predict_us(M, N, K, epilogue) : -1.0,
-                          wide_ok ? gemm_wide_predict_us(M, N, K, epilogue, workspace != nullptr, ws_bytes) : -1.0};
+                          wide_ok ? gemm_wide_predict_us(M, N, K, epilogue, workspace != nullptr, ws_bytes, planes_left != nullptr) : -1.0};
     for (int i = 0; i < 3; ++i)
       if (us[i] >= 0.0 && (best < 0.0 || us[i] < best)) {
         best = us[i];
@@ -150,7 +150,7 @@ extern "C" int sa_gemm_plan(int M, int N, int K, int epilogue, int c_dtype, int6
   const bool tiled_ok = gemm_tiled_takes(M, N, K, lda, p, p, nullptr, 1);
   const double us[3] = {skinny_ok ? gemm_skinny_predict_us(M, N, K, epi) : -1.0,
                         tiled_ok ? gemm_tiled_predict_us(M, N, K, epi) : -1.0,
-                        wide_ok ? gemm_wide_predict_us(M, N, K, epi, ws_bytes > 0, ws_bytes) : -1.0};
+                        wide_ok ? gemm_wide_predict_us(M, N, K, epi, ws_bytes > 0, ws_bytes, false) : -1.0};
   int kernel = 1;
   double best = -1.0;
   for (int i = 0; i < 3; ++i) {

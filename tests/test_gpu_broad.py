@@ -194,3 +194,29 @@ def test_gemm_takes_broad_tiles_with_a_cut_of_their_own(gpu_lib, M, N, K):
     left = ops.gemm(a, tw, defer_sum=True)
     assert isinstance(left, ops.PartialSums)
     check(left.materialize(), want, bf16_steps=1.0)
+
+
+def test_cuts_where_the_sum_is_a_kernel_of_its_own():
+    """Beyond 1,536 rows: cuts that pay where a norm adds the planes up are not taken where a kernel has to."""
+    from simply_amd.kernels import lib
+    planes = lambda *at: lib.load().sa_gemm_planes_broad_tile(*at, 256 << 20)
+    summed = lambda *at: lib.load().sa_gemm_broad_tile(*at, 0, 256 << 20)
+    assert planes(2047, 2304, 9216) == 4256288 and planes(4096, 2048, 16384) == 2256256 and planes(1056, 4608, 36864) == 3256288
+    assert summed(2047, 2304, 9216) == summed(4096, 2048, 16384) == summed(1600, 1024, 4096) == 0
+    assert summed(4096, 2304, 9216) == 2256288 and summed(1056, 4608, 36864) == 3256288
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,shape", [(300, 584, 1088, 31192256), (257, 296, 320, 21256288), (544, 4096, 14336, 0)])
+def test_activated_products_with_a_cut_on_broad_tiles(gpu_lib, M, N, K, shape):
+    """The activation of the summed product rounded to bfloat16, by a pass behind the sum: within one step of it on what the product gives."""
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+    if shape == 0:
+        assert gpu_lib.load().sa_gemm_broad_tile(M, N, K, 0, ops.WORKSPACE_BYTES) // 1000000 > 1
+    a, w = rand((M, K), torch.bfloat16, 120), rand((N, K), torch.bfloat16, 121, 0.03)
+    tw, kw = pack_tiles(w), dict(algo=ops.ALGO_WIDE, shape=shape) if shape else {}
+    plain = ops.gemm(a, tw, **kw)
+    check(plain, ref.gemm(a, w), bf16_steps=1.0)
+    for act in range(4):
+        check(ops.gemm(a, tw, activate=act, **kw), ref.ACTIVATIONS[act](plain.float()).to(torch.bfloat16), bf16_steps=1.0)
