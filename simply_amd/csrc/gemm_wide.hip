@@ -64,8 +64,10 @@ struct Routed {
   const int* sorted;
   const bf16* w2;
   int by_token, top;
-  // EPI 4: row tiles from `tiles` on are those of a product beside the experts', rows of its own times one weight of as many outputs
-  // (the second product of a feed-forward that takes every token), bfloat16 results in the rows' order
+};
+// EPI 4: row tiles from `tiles` on are those of a product beside the experts', rows of its own times one weight of as many outputs
+// (the second product of a feed-forward that takes every token), bfloat16 results in the rows' order.
+struct RoutedBeside : Routed {
   int tiles;
   const bf16* beside_a;
   const bf16* beside_w;
@@ -74,12 +76,19 @@ struct Routed {
   int beside_k, beside_rows;
 };
 
+// (A launch's arguments hold what it reads and no more: 56 bytes of others in front of the grid's size cost 0.1 to 0.4 us a launch,
+// 512 rows of 2,048 against 2,048 outputs 11.0 for 10.7.)
+struct OneProduct {};
+template <bool ROUTED, int EPI>
+using Rows = std::conditional_t<!ROUTED, OneProduct, std::conditional_t<EPI == 4, RoutedBeside, Routed>>;
+static_assert(std::is_empty_v<Rows<false, 0>> && sizeof(Rows<true, 1>) == 32, "what only some kernels read is an argument of those alone");
+
 // WM x WN: 16 x 16 tiles of a wave (rows of A x rows of W); WAVES_M x (WAVES / WAVES_M) waves.
 template <int WM, int WN, int WAVES_M, int EPI, int NSTAGE, int WAVES, bool ROUTED = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __restrict__ A, int64_t lda,
                                                         const bf16* __restrict__ W, bf16* __restrict__ C, int64_t ldc,
                                                         int M, int N, int K, int chunks, int act, float limit,
-                                                        float* __restrict__ partials, Sections sec, Routed rt) {
+                                                        float* __restrict__ partials, Sections sec, Rows<ROUTED, EPI> rt) {
   constexpr int WAVES_N = WAVES / WAVES_M;
   constexpr int MT = WAVES_M * WM, NT = WAVES_N * WN;  // 16-row tiles of A and of W per workgroup
   constexpr int BM = MT * 16;
@@ -99,14 +108,19 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
   // so that an XCD gets a contiguous share of the tiles, and within it tiles go in columns eight wide, rows first.
   int bx = blockIdx.x, by = blockIdx.y;
   int row_first = 0, tile_rows = M;   // (ROUTED: the tile's rows)
-  if (ROUTED) {
+  bool beside = false;
+  if constexpr (ROUTED) {
     // (no turning round: how many tiles there are is known on the device only, and a tile's neighbours in x, which share
     // its rows, go to the XCDs in turn, so that an XCD meets the same weights again in the expert's next tile)
-    if (EPI == 4 && by >= rt.tiles) {
-      row_first = (by - rt.tiles) * BM, tile_rows = rt.beside_rows - row_first < BM ? rt.beside_rows - row_first : BM;
-      A = rt.beside_a, lda = rt.beside_lda, W = rt.beside_w, K = rt.beside_k, chunks = K / 32;
-      ldc = rt.beside_ldc;
-    } else {
+    if constexpr (EPI == 4) {
+      beside = by >= rt.tiles;
+      if (beside) {
+        row_first = (by - rt.tiles) * BM, tile_rows = rt.beside_rows - row_first < BM ? rt.beside_rows - row_first : BM;
+        A = rt.beside_a, lda = rt.beside_lda, W = rt.beside_w, K = rt.beside_k, chunks = K / 32;
+        ldc = rt.beside_ldc;
+      }
+    }
+    if (!beside) {
       if (by >= rt.plan[0]) return;
       row_first = rt.plan[2 + 3 * by], tile_rows = rt.plan[3 + 3 * by];
       const size_t expert = static_cast<size_t>(rt.plan[1 + 3 * by]) * ((N + 15) / 16) * chunks * 512;
@@ -162,7 +176,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
     const int r = half_mine * 8 + lane / 8;  // row of the tile
     const int m = m_base + (tile_mine + (WAVES / 2) * i) * 16 + r;
     int from = m < tile_rows ? m : tile_rows - 1;
-    if (ROUTED) from = rt.by_token ? rt.sorted[row_first + from] / rt.top : row_first + from;
+    if constexpr (ROUTED) from = rt.by_token ? rt.sorted[row_first + from] / rt.top : row_first + from;
     a_off[i] = (static_cast<uint32_t>(from) * static_cast<uint32_t>(lda) + ((lane % 8) ^ (r / 2)) * 8) * 2;
   }
   const bf16* w_from[WPW];  // the same for the whole wave
@@ -171,7 +185,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
     const int nt = nt_base + tile_mine + (WAVES / 2) * i;
     const int clamped = __builtin_amdgcn_readfirstlane(nt < ntiles ? nt : ntiles - 1);
     // (routed gated products: the two factors' tiles alternate here, but lie in weights of their own)
-    const bf16* from = ROUTED && EPI == 1 && clamped % 2 ? rt.w2 : W;
+    const bf16* from = W;
+    if constexpr (ROUTED && EPI == 1) from = clamped % 2 ? rt.w2 : W;
     const int at = ROUTED && EPI == 1 ? clamped / 2 : clamped;
     w_from[i] = from + (static_cast<size_t>(at) * chunks + half_mine) * 512 + static_cast<size_t>(slab0) * 1024;
   }
@@ -320,8 +335,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wide_kernel(const bf16* __res
   for (int i = 0; i < WM; ++i) {
     const int m = m_base + (wm * WM + i) * 16 + row;
     if (m >= tile_rows) continue;
-    if (EPI == 4) {
-      if (by >= rt.tiles) {   // (beside the experts: rounded, in the rows' order)
+    if constexpr (EPI == 4) {
+      if (beside) {   // (rounded, in the rows' order)
         bf16* c_row = rt.beside_y + static_cast<size_t>(row_first + m) * ldc;
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
@@ -385,17 +400,17 @@ static void launch(const bf16* A, int64_t lda, const bf16* W, bf16* C, int64_t l
   const dim3 grid(whole * ((sec.n_step + BNW - 1) / BNW) + (NW - whole * sec.n_step + BNW - 1) / BNW, (M + BM - 1) / BM, ks);
   if (epi == 1)
     gemm_wide_kernel<WM, WN, WAVES_M, 1, NSTAGE, WAVES><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32,
-                                                                                         act, limit, nullptr, sec, Routed{});
+                                                                                         act, limit, nullptr, sec, {});
   else if (raw)
     gemm_wide_kernel<WM, WN, WAVES_M, 3, NSTAGE, WAVES><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32,
-                                                                                         act, limit, partials, sec, Routed{});
+                                                                                         act, limit, partials, sec, {});
   else
     gemm_wide_kernel<WM, WN, WAVES_M, 0, NSTAGE, WAVES><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, C, ldc, M, N, K, K / 32,
-                                                                                         act, limit, nullptr, sec, Routed{});
+                                                                                         act, limit, nullptr, sec, {});
 }
 
 template <int WM, int WN, int WAVES_M, int NSTAGE, int WAVES>
-static void launch_routed(const bf16* A, int64_t lda, const bf16* W, const Routed& rt, bf16* C, float* y, int64_t ldc, int tiles,
+static void launch_routed(const bf16* A, int64_t lda, const bf16* W, const RoutedBeside& rt, bf16* C, float* y, int64_t ldc, int tiles,
                           int rows, int N, int K, int act, float limit, hipStream_t stream) {
   constexpr int BNW = (WAVES / WAVES_M) * WN * 16;
   const int NW = rt.w2 != nullptr ? 2 * ((N + 15) / 16) * 16 : N;
@@ -447,7 +462,7 @@ int gemm_wide_routed(const void* A, int64_t lda, const void* W, const void* W2, 
                      int K, int tile_rows, const int* plan, const int* sorted, int by_token, int top, int act, float limit,
                      hipStream_t stream, const void* beside_a, int64_t beside_lda, const void* beside_w, void* beside_y,
                      int64_t beside_ldc, int beside_k, int beside_rows) {
-  wide::Routed rt;
+  wide::RoutedBeside rt;
   rt.plan = plan, rt.sorted = sorted, rt.w2 = static_cast<const bf16*>(W2), rt.by_token = by_token, rt.top = top;
   rt.tiles = tiles, rt.beside_a = static_cast<const bf16*>(beside_a), rt.beside_w = static_cast<const bf16*>(beside_w);
   rt.beside_y = static_cast<bf16*>(beside_y), rt.beside_lda = beside_lda, rt.beside_ldc = beside_ldc, rt.beside_k = beside_k, rt.beside_rows = beside_rows;
