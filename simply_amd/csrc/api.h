@@ -362,6 +362,8 @@ int sa_paged_attention_maps(const void* q, int dtype, int64_t q_stride, const vo
 
 // sa_paged_attention_maps in bfloat16 on the matrix cores, over units of few rows (csrc/attention_maps.hip).
 int sa_attention_maps_heads_per_unit(int H, int Kh);
+// Into how many ranges of keys sa_paged_attention_maps_units cuts each unit's, given room for them.  A host function.
+int sa_paged_attention_maps_ranges(int unit_count, int H, int Kh, int maps, int hd_v, int window, int max_kv_len, int max_q_len);
 int sa_paged_attention_maps_units_takes(int H, int Kh, int maps, int hd, int hd_v, int page_size, int64_t q_stride,
                                         const void* q);
 int sa_paged_attention_maps_units(const void* q, int64_t q_stride, const void* k_pages, const void* v_pages,

@@ -454,9 +454,33 @@ static int heads_per_unit(int G) {
   return 1;
 }
 
+// Into how many ranges a unit's keys are cut: as paged_attention_decode cuts them, or, with few units of one map, a workgroup for each
+// tile of 32 keys, as far as there are CUs (every wave reads all of a tile's keys, 36 KiB of a latent's: two tiles are two trips to memory
+// one behind the other).  That many ranges want the merge of a workgroup a row, which takes units of up to four rows, values of more than
+// 256 entries and more than 64 ranges; the other one, and the combination of two maps, walk a row's ranges one by one.  Measured, us, as
+// before / a tile each, keys in HBM:
+//   16 heads, keys of 576, values of 512: 1 request 4 tiles 15.2 / 11.7, 8 16.1 / 12.0, 33 16.7 / 13.8, 48 17.2 / 16.3, 65 17.4 / 18.6,
+//     129 22 / 28; 3 requests 33 tiles 17.2 / 15.0, 48 17.8 / 18.3; 16 requests 14 19.3 / 17.0.  3 tiles: 11.9 / 12.1.
+//   4 heads, 320 and 256: 1 request 33 tiles 13.2 / 10.5, 65 14.6 / 11.8, 95 15.0 / 14.0, 129 15.1 / 16.2; 64 and 64: 65 8.9 / 7.8.
+//   16 heads, 320 and 256 (16 rows): 8 tiles 17 / 20, 33 38 / 59, 65 63 / 13, 129 112 / 17, 255 118 / 27.
+//   two maps, 8 heads of 64, values of 128: 5 tiles 10.9 / 11.9, 33 29 / 46, 95 64 / 121.
+static int maps_ranges(int unit_count, int KhV, int maps, int hd_v, int window, int max_kv_len, int max_rows) {
+  const int ranges = paged_attention_decode_ranges(unit_count, KhV, window, max_kv_len, 0);
+  const int tiles = paged_attention_decode_ranges(unit_count, KhV, window, max_kv_len, 1 << 20);   // (one for each, up to 256)
+  const bool serial_merge = max_rows > 4 && hd_v <= 256;
+  const bool ahead = serial_merge ? tiles > 64 : tiles >= 4 && tiles <= (hd_v <= 256 ? 64 : 33);
+  return maps == 1 && ahead && ranges < tiles && static_cast<int64_t>(unit_count) * KhV * tiles <= 256 ? tiles : ranges;
+}
+
 }  // namespace sa
 
 using namespace sa;
+
+extern "C" int sa_paged_attention_maps_ranges(int unit_count, int H, int Kh, int maps, int hd_v, int window, int max_kv_len, int max_q_len) {
+  if (unit_count < 1 || H < 1 || Kh < 1 || H % Kh != 0 || maps < 1 || maps > 2 || hd_v < 1 || window < 0 || max_kv_len < 1 || max_q_len < 1) return 0;
+  const int Gc = heads_per_unit(H / Kh), max_rows = Gc * max_q_len < 16 ? Gc * max_q_len : 16;
+  return maps_ranges(unit_count, Kh * maps * (H / Kh / Gc), maps, hd_v, window, max_kv_len, max_rows);
+}
 
 extern "C" int sa_attention_maps_heads_per_unit(int H, int Kh) {
   return (H > 0 && Kh > 0 && H % Kh == 0) ? heads_per_unit(H / Kh) : 0;
@@ -501,11 +525,8 @@ extern "C" int sa_paged_attention_maps_units(const void* q, int64_t q_stride, co
   sh.page_size = page_size, sh.window = window, sh.scale = scale;
   const int KhV = Kh * maps * sh.chunks;
   SA_REQUIRE(KhV <= 65535 && unit_count <= 65535, "paged_attention_maps_units: too many heads or units");
-  int KS = paged_attention_decode_ranges(unit_count, KhV, window, max_kv_len, 0);
-  // few units with few keys: a workgroup for each tile of 32 keys, as far as there are CUs (every wave reads all of a tile's keys, 36 KiB of
-  // a latent's: two tiles are two trips to memory one behind the other)
-  const int most = paged_attention_decode_ranges(unit_count, KhV, window, max_kv_len, 1 << 20);   // (one for each tile)
-  if (KS < most && static_cast<int64_t>(unit_count) * KhV * most <= 256) KS = most;
+  const int max_rows = Gc * max_q_len < 16 ? Gc * max_q_len : 16;
+  int KS = maps_ranges(unit_count, KhV, maps, hd_v, window, max_kv_len, max_rows);
   const size_t per_split = static_cast<size_t>(unit_count) * KhV * 16 * (hd_v + kRowExtra) * sizeof(float);
   while (KS > 1 && (workspace == nullptr || per_split * KS > workspace_bytes)) --KS;
   const bool partial = differential != 0;
@@ -561,7 +582,6 @@ extern "C" int sa_paged_attention_maps_units(const void* q, int64_t q_stride, co
 #undef SA_LAUNCH
   }
   if (check_launch("paged_attention_maps_units")) return 1;
-  const int max_rows = Gc * max_q_len < 16 ? Gc * max_q_len : 16;
   if (partial) {
     attention_maps_combine_kernel<<<dim3(Kh * sh.chunks, unit_count, max_rows), 256, 0, stream>>>(
         ws, KS, um, unit_begin, op, out_stride, KhV, sh.chunks, Gc, G, hd_v, lambda, eps, mult);

@@ -78,6 +78,7 @@ _SIGNATURES = {
     "sa_norm_rope_cache_write": [_P, _I, _L, _P, _P, _I, _F, _P, _I, _I, _P, _I, _I, _I, _F, _I, _P, _P, _P, _I, _I, _I,
                                  _I, _I, _I, _I, _P],
     "sa_attention_maps_heads_per_unit": [_I, _I],
+    "sa_paged_attention_maps_ranges": [_I, _I, _I, _I, _I, _I, _I, _I],
     "sa_paged_attention_maps_units_takes": [_I, _I, _I, _I, _I, _I, _L, _P],
     "sa_paged_attention_maps_units": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _P, _L, _I, _I, _I, _I, _I, _I, _F, _I, _I, _F,
                                       _F, _F, _I, _I, _P, _L, _P],
