@@ -127,6 +127,8 @@ int sa_gemm_wide_shape(int M, int N, int K, int epilogue, int64_t workspace_byte
 // a tile, else 0.  _planes_: for sa_gemm_planes, whose caller adds the cuts up.  Host functions.
 int sa_gemm_broad_tile(int M, int N, int K, int epilogue, int64_t workspace_bytes);
 int sa_gemm_planes_broad_tile(int M, int N, int K, int64_t workspace_bytes);
+// Whether many rows against so few outputs go to the kernel that is made for them, in the tiled kernel's place.  A host function.
+int sa_gemm_narrow_takes(int M, int N, int K);
 // Where it takes the whole sections of n_step outputs of sa_gemm_sections: rows * 1000 + weight rows of a tile, else 0.  A host function.
 int sa_gemm_sections_tile(int M, int N, int K, int n_step, int64_t workspace_bytes);
 // Which way the 32-bit matrix-core kernels take M rows: 16 (few rows), or the rows of a tile (32, 64 or 128), plus 1000 where K

@@ -6,9 +6,11 @@
 // eight waves' sums, which are added in the waves' order: a row's sums run the same way whatever rows are beside it.
 // K a multiple of 32, W tiled.
 //
-// us, 32-bit results, before (the tiled kernel, mostly with K cut and a sum kernel) / now, K = 2,048: 16 outputs 33 rows 8.4 / 4.1, 774
-// 10.0 / 4.5, 2,047 11.4 / 4.7, 8,192 20.5 / 8.1; 64 outputs 8.6 / 5.8, 10.7 / 6.4, 13.0 / 6.7, 21.6 / 12.6; K = 4,096, 64 outputs, 33 rows
-// 9.4 / 9.2, 2,047 16.1 / 10.8.  For 17 to 32 rows the few-rows kernel takes as long (16 outputs 4.7 / 4.0, 64 4.9 / 5.7) and keeps them.
+// us in a graph of launches, 32-bit results, before (the tiled kernel, mostly with K cut and a sum kernel) / now, K = 2,048: 16 outputs 33
+// rows 8.4 / 4.2, 774 9.9 / 4.3, 2,047 11 / 4.4, 8,192 20.5 / 7.2; 64 outputs 8.7 / 6.3, 11.8 / 6.5, 13.0 / 6.6, 22.2 / 12.0; K = 4,096, 64
+// outputs, 33 rows 9.5 / 9.8, 2,047 16.1 / 10.6.  A CU's loads are what it then waits for: sixteen waves take as long (10.6 there), the
+// loads left to the compiler's order, a few at a time, up to 9 % longer.  For 17 to 32 rows the few-rows kernel takes as long (16
+// outputs 4.7 / 4.0, 64 4.9 / 5.7) and keeps them.
 #include "api.h"
 #include "common.h"
 
@@ -45,6 +47,7 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_narrow_kernel(const bf16*
 #pragma unroll
       for (int j = 0; j < NT; ++j) fw[u][j] = *reinterpret_cast<const bf16x8*>(w + j * tile + static_cast<size_t>(c + u) * 512);
     }
+    __builtin_amdgcn_sched_barrier(0);   // all of them under way before the first is waited for
 #pragma unroll
     for (int u = 0; u < COUNT; ++u)
 #pragma unroll
@@ -71,11 +74,27 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_narrow_kernel(const bf16*
 
 }  // namespace narrow
 
-bool gemm_narrow_takes(int M, int N, int K) { return M > 32 && N <= 64 && K % 32 == 0; }
-
-double gemm_narrow_predict_us(int M, int N, int K) {
-  return 4.5 + static_cast<double>(M) * K * 2 / 4e6 + 0.3 * (K / 2048.0) * ((N + 15) / 16);
+// Microseconds of a launch among others: the loads of 16 rows and all weights by every CU, as many times as it gets 16 rows, or all rows
+// once (within 14 % of the measured time of 8 to 64 outputs up to 2,047 rows of K = 512 to 36,864 and up to 8,192 of 4,096; beyond, where
+// this kernel is far ahead, it takes up to 1.8 times as long).
+static double narrow_us(int M, int N, int K) {
+  const double times = fmax(1.0, (M + 15) / 16 / 256.0);
+  return 2.1 + fmax(times * K / 1024.0 * (0.79 + 0.27 * ((N + 15) / 16)), static_cast<double>(M) * K * 2 / 6e6);
 }
+
+// Up to K = 4,096 always (which kernel a row meets does not depend on its neighbours there; the one size that loses is 33 rows against 64
+// outputs, 9.5 / 9.8 us).  A longer K, of which a workgroup walks all by itself, is left to the tiled kernel with its cuts of K, whose time
+// for so few outputs is the second figure, until there are rows for many workgroups; us, tiled / this, 32-bit results: K = 8,192, 16
+// outputs 33 rows 10.2 / 10.8, 200 12.0 / 11.0, 64 outputs 200 13.5 / 17.3, 2,047 22 / 18; 16,384, 16 outputs 200 15 / 20, 1,031 23 / 20, 64
+// outputs 1,031 24 / 32, 4,096 60 / 36; 36,864, 16 outputs 33 rows 19 / 41, 1,031 39 / 41, 2,047 64 / 42, 64 outputs 33 rows 21 / 70, 2,047
+// 72 / 74, 4,096 158 / 115.
+bool gemm_narrow_takes(int M, int N, int K) {
+  return M > 32 && N <= 64 && K % 32 == 0 &&
+         (K <= 4096 || narrow_us(M, N, K) <= 7.0 + 0.03 * (M < 64 ? M : 64) + 0.28 * K / 1024 + static_cast<double>(M) * K * 2 / 3.6e6);
+}
+
+// (the wide kernel's small tiles are 1 to 3 us below their figure at these sizes)
+double gemm_narrow_predict_us(int M, int N, int K) { return 0.5 + narrow_us(M, N, K); }
 
 int gemm_narrow(const void* A, int64_t lda, const void* W, void* C, int c_dtype, int64_t ldc, int M, int N, int K, hipStream_t stream) {
   const bf16* a = static_cast<const bf16*>(A);
@@ -91,3 +110,5 @@ int gemm_narrow(const void* A, int64_t lda, const void* W, void* C, int c_dtype,
 }
 
 }  // namespace sa
+
+extern "C" int sa_gemm_narrow_takes(int M, int N, int K) { return M > 0 && N > 0 && K > 0 && sa::gemm_narrow_takes(M, N, K); }

@@ -392,7 +392,7 @@ int gemm_tiled(const void* A, int64_t lda, const void* W, void* C, int c_dtype, 
       const int row_tiles = (M + 63) / 64 * tiles;
       const int by_rows = static_cast<int>((static_cast<int64_t>(NW) + M) * K * 2 / (2 * static_cast<int64_t>(M) * NW * 4));
       const int cuts = min(min(256 / row_tiles, stages / 4), by_rows);
-      // (K = 2,048: 2,047 rows of 16 outputs 17.7 -> 10.5 us, of 64 18.2 -> 12.2, of 128 18.7 -> 14.7; 513 rows of 16 17.2 -> 9.7)
+      // (K = 2,048: 2,047 rows of 128 outputs 18.7 -> 14.7 us; up to 64 outputs only the longer K that gemm_narrow leaves come here)
       if (cuts > ks) ks = cuts;
     }
   }

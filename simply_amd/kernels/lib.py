@@ -37,6 +37,7 @@ _SIGNATURES = {
     "sa_gemm_wide_shape": [_I, _I, _I, _I, _L],
     "sa_gemm_broad_tile": [_I, _I, _I, _I, _L],
     "sa_gemm_planes_broad_tile": [_I, _I, _I, _L],
+    "sa_gemm_narrow_takes": [_I, _I, _I],
     "sa_gemm_sections_tile": [_I, _I, _I, _I, _L],
     "sa_table_rows": [_P, _I, _I, _P, _P, _P, _P, _P, _P],
     "sa_decode_slots": [_I, _P, _P, _P, _I, _I, _P, _P],

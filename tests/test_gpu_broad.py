@@ -220,3 +220,25 @@ def test_activated_products_with_a_cut_on_broad_tiles(gpu_lib, M, N, K, shape):
     check(plain, ref.gemm(a, w), bf16_steps=1.0)
     for act in range(4):
         check(ops.gemm(a, tw, activate=act, **kw), ref.ACTIVATIONS[act](plain.float()).to(torch.bfloat16), bf16_steps=1.0)
+
+
+def test_few_outputs_of_a_long_k_keep_their_cuts():
+    """(rows, outputs, K): up to K = 4,096 the narrow kernel whatever the rows; beyond only with rows for many workgroups."""
+    from simply_amd.kernels import lib, ops
+    takes = lib.load().sa_gemm_narrow_takes
+    assert all(takes(M, N, K) for M in (33, 100, 2047, 8192) for N in (1, 16, 64) for K in (32, 2048, 4096))
+    assert takes(200, 16, 8192) and takes(2047, 64, 8192) and takes(1031, 16, 16384) and takes(4096, 64, 16384) and takes(2047, 16, 36864)
+    assert not any(takes(*at) for at in ((33, 16, 8192), (200, 64, 8192), (200, 16, 16384), (1031, 64, 16384), (33, 16, 36864), (2047, 64, 36864),
+                                         (32, 16, 2048), (100, 65, 2048), (100, 16, 2056)))
+    assert ops.gemm_plan(33, 16, 36864)[1]["tiled"] < 16   # (not the 41 us of 16 rows' workgroups that walk it all)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 16, 8192), (200, 16, 8192), (40, 64, 16416), (100, 48, 36864)])
+def test_few_outputs_on_both_sides_of_the_line(gpu_lib, M, N, K):
+    from simply_amd.kernels import ops
+    from simply_amd.kernels.packing import pack_tiles
+    a, w = rand((M, K), torch.bfloat16, 130), rand((N, K), torch.bfloat16, 131, 0.05)
+    tw = pack_tiles(w)
+    check(ops.gemm(a, tw), ref.gemm(a, w), bf16_steps=1.0)
+    torch.testing.assert_close(ops.gemm(a, tw, out_dtype=torch.float32), (a.double() @ w.double().T).float(), rtol=1e-5, atol=2e-6 * K ** 0.5)
