@@ -292,6 +292,7 @@ double gemm_broad_plan(int M, int N, int K, int epi, bool have_workspace, size_t
 void gemm_broad(int tile, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, int epi,
                 int act, float limit, int ks, float* partials, bool raw, Sections sec, hipStream_t stream);
 // planes: where K is cut the caller adds the planes up (no sum kernel behind the product).
+double gemm_wide_tile_us(int K);
 double gemm_wide_predict_us(int M, int N, int K, int epi, bool have_workspace, size_t workspace_bytes, bool planes);
 // The experts' products on the wide kernel (plan, sorted: of the sort kernel with tiles of tile_rows rows, 64 or 128).
 bool gemm_wide_routed_takes(int N, int K, int64_t lda, int64_t a_rows, int64_t ldc, const void* A, const void* W, const void* W2,
@@ -671,6 +672,8 @@ int sa_expert_product(const void* a, int dtype, int64_t a_stride, int a_by_token
 // shared_h [T, shared_K] . shared_w^T of a feed-forward that takes every token: bfloat16, tiles of 64 or 128 rows, aligned operands.
 int sa_expert_product_beside_takes(int N, int K, int64_t h_stride, int P, int tile_rows, const void* shared_h, int64_t shared_h_stride,
                                    const void* shared_w, int shared_K, int T);
+// Whether it is expected to be ahead of two launches, with tiles of 128 rows.  Host functions, both.
+int sa_expert_product_beside_pays(int N, int K, int P, int E, int shared_K, int T);
 int sa_expert_product_beside(const void* h, int64_t h_stride, int top, const void* w, int N, int K, const int* sorted, const int* plan,
                              int P, int E, int tile_rows, void* y, int64_t y_stride, const void* shared_h, int64_t shared_h_stride,
                              const void* shared_w, int shared_K, int T, void* shared_y, int64_t shared_y_stride, hipStream_t stream);

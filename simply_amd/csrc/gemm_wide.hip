@@ -483,6 +483,9 @@ bool gemm_wide_takes(int M, int N, int K, int64_t lda, int64_t ldc, const void* 
          static_cast<int64_t>(M) * lda < (int64_t{1} << 31);  // byte offsets of rows are kept in 32 bits
 }
 
+// Of a tile of 32,768 outputs with every CU at work.
+double gemm_wide_tile_us(int K) { return 0.78 * K / wide::BK + 2.8; }
+
 // The time of an uncut product on tiles of `shape`, `columns` of them side by side: their rounds of slabs at what 128 outputs of 256 rows (or
 // as many of another tile) take, fitted like the broad kernel's.
 static double rounds_us(int shape, int M, int64_t columns, int NW, int K, int epi) {

@@ -987,6 +987,43 @@ extern "C" int sa_expert_product_beside_takes(int N, int K, int64_t h_stride, in
          gemm_wide_routed_takes(N, shared_K, shared_h_stride, T, N, shared_h, shared_w, nullptr, p, tile_rows);
 }
 
+// Whether that launch is expected to be ahead of the experts' second products and a launch of the shared one's, with tiles of 128 rows.  The
+// host counts what the CUs get: an expert's tokens as even routing deals them out, tile after tile to the CU that is free first, the
+// shared product's behind the experts' (an XCD's workgroups start in the grid's order).  Rounds do not end as sharply as counted, so that it
+// is taken up to 8 us behind.  Both second products and the experts' first, us, apart / beside, at expected gains in us: 16 experts of 2,048
+// x 2,048, 2 chosen, shared of 2,048: 640 tokens 127 / 109 (15), 1,500 162 / 162 (-7), 2,047 209 / 185 (23); shared of 3,072: 774 132 / 118
+// (7), 1,280 168 / 172 (-11), 2,047 218 / 196 (18); of 8,192: 774 166 / 177 (-34), 2,047 264 / 258 (-3), 4,096 401 / 382 (35); 4,096 x 3,584: 500
+// 307 / 315 (-24), 1,024 409 / 378 (33); 64 experts, 8 chosen, 500 400 / 412 (-16); 8 experts of 4,096 x 3,584, one chosen, shared of
+// 7,168: 774 239 / 207 (14), 3,000 471 / 514 (-56).  Of 116 sizes none is taken that is slower by 1.5 %.
+extern "C" int sa_expert_product_beside_pays(int N, int K, int P, int E, int shared_K, int T) {
+  if (N < 1 || K < 1 || P < 1 || E < 1 || shared_K < 1 || T < 1) return 0;
+  constexpr int kRows = kTileRowsWide, kCUs = 256;
+  const double mean = static_cast<double>(P) / E, deviation = sqrt(mean * (1.0 - 1.0 / E)) + 1e-9;
+  double tiles = 0.0;   // of an expert: the sum over k of the chance that it has more than 128 k tokens
+  for (int k = 0; k * kRows <= P; ++k) {
+    const double more = 0.5 * erfc((k * kRows + 0.5 - mean) / (deviation * sqrt(2.0)));
+    tiles += more;
+    if (more < 1e-6 && k * kRows > mean) break;
+  }
+  const int columns = (N + 255) / 256;
+  const int64_t own = llround(E * tiles * columns);
+  int64_t left = static_cast<int64_t>((T + kRows - 1) / kRows) * columns;
+  const double own_us = gemm_wide_tile_us(K), shared_us = gemm_wide_tile_us(shared_K);
+  const double apart = (own + kCUs - 1) / kCUs * own_us +
+                       fmin(gemm_wide_predict_us(T, N, shared_K, 0, true, size_t{256} << 20, false), gemm_tiled_predict_us(T, N, shared_K, 0));
+  // the CUs that are free before the experts' last round and those behind it, each with the time from which they are
+  double early = own / kCUs * own_us, late = early + own_us, beside = own % kCUs ? late : early;
+  int64_t early_cus = kCUs - own % kCUs, late_cus = own % kCUs;
+  while (left > 0) {
+    const bool first = late_cus == 0 || early <= late;
+    double& from = first ? early : late;
+    left -= first ? early_cus : late_cus;
+    from += shared_us;
+    beside = fmax(beside, from);
+  }
+  return beside <= apart + 8.0;
+}
+
 extern "C" int sa_expert_product_beside(const void* h, int64_t h_stride, int top, const void* w, int N, int K, const int* sorted,
                                         const int* plan, int P, int E, int tile_rows, void* y, int64_t y_stride, const void* shared_h,
                                         int64_t shared_h_stride, const void* shared_w, int shared_K, int T, void* shared_y,

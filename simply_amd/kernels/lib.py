@@ -134,6 +134,7 @@ _SIGNATURES = {
     "sa_route_few": [_P, _L, _P, _I, _I, _I, _I, _I, _F, _I, _P, _I, _P, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P, _I,
                      _I, _I, _F, _P, _P],
     "sa_expert_product_beside_takes": [_I, _I, _L, _I, _I, _P, _L, _P, _I, _I],
+    "sa_expert_product_beside_pays": [_I, _I, _I, _I, _I, _I],
     "sa_expert_product_beside": [_P, _L, _I, _P, _I, _I, _P, _P, _I, _I, _I, _P, _L, _P, _L, _P, _I, _I, _P, _L, _P],
     "sa_expert_product_shared": [_P, _L, _I, _P, _I, _I, _P, _P, _I, _I, _P, _L, _P, _L, _P, _I, _I, _I, _P, _L, _P],
     "sa_experts_add_next_norm_pays": [_I, _I],

@@ -2224,18 +2224,15 @@ def few_rows_experts(T: int, top: int, gate_w, up_w, x: torch.Tensor) -> bool:
 
 def experts_beside(T: int, top: int, up_w, down_w, x: torch.Tensor, dense) -> bool:
     """Whether a step of T tokens takes the second product of a shared feed-forward (a tiled weight `dense`) beside its experts': with
-    tiles of 128 rows, whose last round of workgroups it fills.  A wide one makes tiles that walk longer than the experts' and is ahead
-    only with many tokens.  Both second products and the experts' first, us, apart / beside, 16 experts, top 2, shared of the
-    experts' size: of 2,048 x 2,048 500 tokens 115 / 104, 1,024 152 / 136, 1,500 160 / 165, 2,047 221 / 190, 4,096 339 / 324; of 4,096 x
-    3,584 500 310 / 321, 1,024 438 / 398, 2,047 631 / 603; of 2,560 x 2,560 774 211 / 181, 3,000 428 / 391; shared of 3,072 beside 2,048:
-    1,024 158 / 164, 1,500 170 / 180, 2,047 238 / 207; of 8,192 1,500 199 / 240, 2,047 272 / 264, 4,096 424 / 397."""
+    tiles of 128 rows, whose last round of workgroups it fills, where that is expected to be ahead of a launch of its own."""
     if not isinstance(dense, TiledWeight) or dense.paired or x.dtype != torch.bfloat16 or not x.is_cuda or not up_w.tiled \
-            or dense.shape[0] != down_w.rows or (dense.cols > up_w.rows and T < 1800):
+            or dense.shape[0] != down_w.rows:
         return False
     lib, P = _lib.load(), T * top
     rows = lib.sa_expert_tile_rows(P, up_w.experts, up_w.cols, up_w.rows, _code(x), x.stride(0), _ptr(x))
     return rows == 128 and bool(lib.sa_expert_product_beside_takes(down_w.rows, up_w.rows, up_w.rows, P, rows, _ptr(dense.data), dense.cols,
-                                                                   _ptr(dense.data), dense.cols, T))
+                                                                   _ptr(dense.data), dense.cols, T)) \
+        and bool(lib.sa_expert_product_beside_pays(down_w.rows, up_w.rows, P, up_w.experts, dense.cols, T))
 
 
 def routed_experts(x: torch.Tensor, experts: torch.Tensor, weights: torch.Tensor, gate_w, up_w, down_w, activation: int,

@@ -57,3 +57,15 @@ def test_expected_times_grow_with_the_work(ops):
     # what no fast kernel takes (K that is no multiple of 8) is left to the kernel that takes every size
     kernel, us = ops.gemm_plan(4, 100, 100)
     assert kernel == ops.ALGO_GENERIC and all(v < 0 for v in us.values())
+
+
+@pytest.mark.parametrize("sizes,pays", [
+    # (outputs, experts' K, pairs, experts, shared K, tokens): a last round that the shared tiles fill, or one round more for them
+    ((2048, 2048, 1280, 16, 2048, 640), True), ((2048, 2048, 4094, 16, 2048, 2047), True), ((2048, 2048, 1548, 16, 3072, 774), True),
+    ((2048, 2048, 2560, 16, 3072, 1280), False), ((2048, 2048, 1548, 16, 8192, 774), False), ((2048, 2048, 8192, 16, 8192, 4096), True),
+    ((4096, 3584, 1000, 16, 3584, 500), False), ((4096, 3584, 2048, 16, 3584, 1024), True), ((2048, 2048, 4000, 64, 2048, 500), False),
+    ((4096, 3584, 774, 8, 7168, 774), True), ((4096, 3584, 3000, 8, 7168, 3000), False),
+    ((0, 2048, 1280, 16, 2048, 640), False), ((16, 64, 2, 1, 64, 1), True)])
+def test_a_shared_product_beside_the_experts(ops, sizes, pays):
+    from simply_amd.kernels import lib
+    assert bool(lib.load().sa_expert_product_beside_pays(*sizes)) == pays
