@@ -587,29 +587,34 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     // With the cut that the tiles above take, or where they take none any.  (More than three cuts of few rows cost more than the broad
     // kernel's model says: 160 rows of 9,216 against 2,304 outputs with 14 cuts 23 and 28 us, 896 with four 49 and 56, 129 of 8,192
     // against 2,048 with 16 20 and 24, all expected at about the same.)
-    // Beyond 1,536 rows the tiles above are not cut: where the sum is a kernel of its own, it counts, and cuts are taken only ahead (3,072 rows of
-    // 9,216 against 2,304 outputs in two cuts 112 / 115 us with the sum, 132 / 127 with a norm that adds them up, 4,096 of 16,384 against
-    // 2,048 207 / 219 and 230 / 229, 1,600 of 4,096 against 1,024 in seven 28 / 32).  The pass for an activation behind a cut does not: it takes
-    // what the code in an uncut product's epilogue takes (2,304 outputs of 9,216, erf GELU, 4,096 rows: 18 us and 19).
+    // Beyond 1,536 rows the tiles above are not cut: where the sum is a kernel of its own, it counts, and two to four cuts are taken only
+    // ahead, more not (3,072 rows of 9,216 against 2,304 outputs in two cuts 112 / 115 us with the sum, 132 / 127 with a norm that adds them
+    // up, 4,096 of 16,384 against 2,048 207 / 219 and 230 / 229, 1,600 of 4,096 against 1,024 in seven 28 / 32, of 4,608 against 640 in nine
+    // 31 / 33).  The pass for an activation behind a cut does not count: it takes what the code in an uncut product's epilogue takes (2,304
+    // outputs of 9,216, erf GELU, 4,096 rows: 18 us and 19).
     const double behind_us = fitted || planes ? 0.0 : 3.7;
-    int tile = 0, cut = ks;
+    const int others = ks;
+    int tile = 0, cut = others;
     const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, tile, cut, behind_us);
-    const double line = cut == 1 ? 1.03 : fitted ? (cut > 3 ? 0.94 : 1.03) : planes ? 1.03 : 0.96;
+    const double line = cut == 1 ? 1.03 : fitted ? (cut > 3 ? 0.94 : 1.03) : planes ? 1.03 : cut > 4 ? 0.0 : 0.96;
     if (broad_us < line * best_us) {
       shape = 1000000 + tile;
       ks = cut;
-      us = best_us = broad_us;
+      best_us = broad_us;
+      // (the figure that the other kernels' are compared with, crude as theirs, never grows by a better tile: 4,096 rows of K = 64 against
+      // 14,336 gated outputs would go to the tiled kernel, 125 us for 72)
+      us = fmin(us, broad_us);
     }
     // With a cut of their own beside tiles that are cut too, which was found for tiles of another size, only well ahead: 544 rows of 36,864
     // against 4,608 outputs 216 / 178 us, 640 261 / 217, of 14,336 against 6,144 320 rows 87 / 76, against 4,096 544 rows 85 / 76.  Of 80
     // sizes that the model has up to 8 % ahead or behind 61 were slower (129 rows of 4,096 against 12,288, by the model 7 % ahead, by 14 %).
-    if (asked == 1 && cut > 1) {
+    if (asked == 1 && others > 1) {
       int own_tile = 0, own_cut = 1;
       const double own_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, own_tile, own_cut, behind_us);
       if (own_cut > 1 && own_us < 0.92 * best_us) {
         shape = 1000000 + own_tile;
         ks = own_cut;
-        us = own_us;
+        us = fmin(us, own_us);
       }
     }
   }

@@ -202,7 +202,7 @@ def test_cuts_where_the_sum_is_a_kernel_of_its_own():
     planes = lambda *at: lib.load().sa_gemm_planes_broad_tile(*at, 256 << 20)
     summed = lambda *at: lib.load().sa_gemm_broad_tile(*at, 0, 256 << 20)
     assert planes(2047, 2304, 9216) == 4256288 and planes(4096, 2048, 16384) == 2256256 and planes(1056, 4608, 36864) == 3256288
-    assert summed(2047, 2304, 9216) == summed(4096, 2048, 16384) == summed(1600, 1024, 4096) == 0
+    assert summed(2047, 2304, 9216) == summed(4096, 2048, 16384) == summed(1600, 1024, 4096) == summed(1600, 640, 4608) == 0
     assert summed(4096, 2304, 9216) == 2256288 and summed(1056, 4608, 36864) == 3256288
 
 

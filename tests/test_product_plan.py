@@ -69,3 +69,10 @@ def test_expected_times_grow_with_the_work(ops):
 def test_a_shared_product_beside_the_experts(ops, sizes, pays):
     from simply_amd.kernels import lib
     assert bool(lib.load().sa_expert_product_beside_pays(*sizes)) == pays
+
+
+def test_a_short_k_against_many_outputs_stays_with_the_large_tiles(ops):
+    """The broad kernel's figure counts the start of every round; the tiled kernel's does not, and is not ahead for it."""
+    for M, N, K, gated in ((4096, 14336, 64, True), (2048, 14336, 64, True), (8192, 18432, 128, True), (8192, 18432, 128, False),
+                           (4096, 14336, 64, False), (1600, 36864, 64, False), (4096, 8192, 64, True)):
+        assert ops.gemm_plan(M, N, K, gated=gated)[0] == ops.ALGO_WIDE, (M, N, K, gated)
