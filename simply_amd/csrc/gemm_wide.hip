@@ -487,11 +487,16 @@ bool gemm_wide_takes(int M, int N, int K, int64_t lda, int64_t ldc, const void* 
 double gemm_wide_tile_us(int K) { return 0.78 * K / wide::BK + 2.8; }
 
 // The time of an uncut product on tiles of `shape`, `columns` of them side by side: their rounds of slabs at what 128 outputs of 256 rows (or
-// as many of another tile) take, fitted like the broad kernel's.
+// as many of another tile) take, fitted like the broad kernel's.  One round that leaves more than half of the CUs idle is faster, the clock
+// rises: 45 to 80 tiles of 192 x 128, K = 4,608, 31 us where a full round takes 48.  (128 x 128, which take longer for their size, come out
+// even: K = 8,192, 104 tiles 58 us, 160 60.)
 static double rounds_us(int shape, int M, int64_t columns, int NW, int K, int epi) {
   const int rows = shape / 1000 % 1000, wrows = shape % 1000;
-  const int64_t rounds = ((M + rows - 1) / rows * columns + wide::kCUs - 1) / wide::kCUs;
-  return fmax(5.0 + 2.0 * NW * K / 5.8e6, 3.0 + rounds * ((epi == 1 ? 0.88 : 0.78) * (K / wide::BK) * rows * wrows / 32768.0 + 2.8));
+  const int64_t tiles = (M + rows - 1) / rows * columns, rounds = (tiles + wide::kCUs - 1) / wide::kCUs;
+  double slab_us = (epi == 1 ? 0.88 : 0.78) * rows * wrows / 32768.0;
+  const double half_full = tiles / (wide::kCUs / 2.0);
+  if (epi == 0 && rows * wrows > 128 * 128 && half_full < 1.0) slab_us *= 0.6 + 0.4 * fmax(0.0, 2.0 * half_full - 1.0);
+  return fmax(5.0 + 2.0 * NW * K / 5.8e6, 3.0 + rounds * (slab_us * (K / wide::BK) + 2.8));
 }
 
 // The tile and the cut of K for a product whose caller fixes neither, and the time that this kernel is expected to
@@ -587,16 +592,18 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     // With the cut that the tiles above take, or where they take none any.  (More than three cuts of few rows cost more than the broad
     // kernel's model says: 160 rows of 9,216 against 2,304 outputs with 14 cuts 23 and 28 us, 896 with four 49 and 56, 129 of 8,192
     // against 2,048 with 16 20 and 24, all expected at about the same.)
-    // Beyond 1,536 rows the tiles above are not cut: where the sum is a kernel of its own, it counts, and two to four cuts are taken only
-    // ahead, more not (3,072 rows of 9,216 against 2,304 outputs in two cuts 112 / 115 us with the sum, 132 / 127 with a norm that adds them
-    // up, 4,096 of 16,384 against 2,048 207 / 219 and 230 / 229, 1,600 of 4,096 against 1,024 in seven 28 / 32, of 4,608 against 640 in nine
-    // 31 / 33).  The pass for an activation behind a cut does not count: it takes what the code in an uncut product's epilogue takes (2,304
-    // outputs of 9,216, erf GELU, 4,096 rows: 18 us and 19).
+    // Beyond 1,536 rows the tiles above are not cut: where the sum is a kernel of its own, it counts, and cuts are taken only ahead (3,072 rows
+    // of 9,216 against 2,304 outputs in two cuts 112 / 115 us with the sum, 132 / 127 with a norm that adds them up, 4,096 of 16,384 against
+    // 2,048 207 / 219 and 230 / 229); five and more only well ahead and of 13 slabs or more each, either way (1,600 of 4,096 against 1,024 in
+    // seven 28 / 32, of 4,608 against 640 in nine 31 / 33, 1,800 of 6,144 against 1,280 in five 42 / 53 and 52 / 59; of 8,192 against 1,024 in
+    // six 52 / 46, 2,500 against 512 in nine 50 / 38, 2,047 of 36,864 against 640 in ten 282 / 103).  The
+    // pass for an activation behind a cut does not count: it takes what the code in an uncut product's epilogue takes (2,304 outputs of
+    // 9,216, erf GELU, 4,096 rows: 18 us and 19).
     const double behind_us = fitted || planes ? 0.0 : 3.7;
     const int others = ks;
     int tile = 0, cut = others;
     const double broad_us = gemm_broad_plan(M, N, K, epi, have_workspace, workspace_bytes, tile, cut, behind_us);
-    const double line = cut == 1 ? 1.03 : fitted ? (cut > 3 ? 0.94 : 1.03) : planes ? 1.03 : cut > 4 ? 0.0 : 0.96;
+    const double line = cut == 1 ? 1.03 : fitted ? (cut > 3 ? 0.94 : 1.03) : cut > 4 ? (K / wide::BK / cut >= 13 ? 0.93 : 0.0) : planes ? 1.03 : 0.96;
     if (broad_us < line * best_us) {
       shape = 1000000 + tile;
       ks = cut;
