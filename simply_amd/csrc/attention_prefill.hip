@@ -26,6 +26,7 @@
 // workgroups, and the ranges are merged by the second kernel of the few-rows path.
 #include "api.h"
 #include "attention_common.h"
+#include "slabs.h"
 
 namespace sa {
 namespace prefill {
@@ -33,19 +34,8 @@ namespace prefill {
 constexpr int kWaves = 4;
 constexpr float kLog2e = 1.4426950408889634f;
 
-// s_waitcnt for "at most n vector-memory loads outstanding" and nothing else (gfx9 encoding: vmcnt in bits 3:0 and
-// 15:14, expcnt 6:4, lgkmcnt 11:8)
-constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-
-// The workgroup barrier alone; the empty statements and the scheduling barriers keep the compiler from moving memory
-// accesses across it.
-__device__ inline void bare_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-}
+using slabs::bare_barrier;
+using slabs::waitcnt_vm;
 
 template <int NDC, int R, bool CAP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1 ? 2 : 1, R == 1 ? 2 : 1))) void paged_attention_prefill_kernel(

@@ -1,7 +1,7 @@
 // C[M, N] = epilogue(A[M, K] . W[N, K]^T) in bfloat16 for many rows, on the largest tiles that a CU's registers hold: a workgroup of
 // four waves, one to a SIMD, has 256 x 288, 256 x 256, 192 x 288 or 192 x 256 outputs, a wave a quarter of them.
 //   * What bounds it: the matrix units' power.  With every CU at work they are busy 72 % of the cycles at 1.93 GHz (2,048 rows, 8,192
-//     outputs, K = 8,192: 188 us, 1.46 PFLOP/s); with the loads left out the same loop takes 25 % less time, in part by the clock.
+//     outputs, K = 8,192: 188 us, 1.46 PFLOP/s); with the loads left out the same loop takes 22 % less time, in part by the clock.
 //     A wave's 128 x 144 outputs need 17 fragment reads for 72 products where the wide kernel's 64 x 96 need 10 for 24, and a tile of
 //     256 x 288 brings 34 KiB into LDS for 72 products a SIMD where two of 128 x 192 bring 40 for 48: what is moved for a product
 //     is what power can be saved on.

@@ -539,14 +539,14 @@ static double plan_shape(int M, int N, int K, int epi, bool have_workspace, size
     const int rows = M <= 64 ? 64 : 128;
     if (static_cast<int64_t>((M + rows - 1) / rows) * ((NW + 127) / 128) <= wide::kCUs) shape = M <= 64 ? 6064128 : 3128128;
   }
-  // More rows against few outputs (64 tiles of 128 x 128 at most) too: 2,048 rows of K = 4,096 against 512 outputs 27.6 / 15.2 us, of K =
-  // 2,048 against 256 16.5 / 10.9 and against 64 15.5 / 13.4, 3,000 of 2,304 against 160 17.2 / 11.1 (uncut / with the cut).
   // 17 to 1,536 rows without an epilogue (portions of prompts, many decoding requests): the tiles above are too few
   // for 256 CUs, and every workgroup walks all of K at the pace of its own slabs.  Smaller tiles with deeper
   // pipelines, and K cut over workgroups so that about one round of them covers the GPU, chosen by a model of the
   // time fitted to measurements at the 2B, 9B and 27B sizes (64 to 2,048 rows, seven tiles, one to fourteen cuts;
   // it is within 6 % of the best measured choice nearly everywhere, and a fifth faster in sum than either the
   // uncut tiles above or the tiled kernel with its cut: the 2B down projection at 512 rows takes 36 us against 55).
+  // More rows against few outputs (64 tiles of 128 x 128 at most) too: 2,048 rows of K = 4,096 against 512 outputs 27.6 / 15.2 us, of K =
+  // 2,048 against 256 16.5 / 10.9 and against 64 15.5 / 13.4, 3,000 of 2,304 against 160 17.2 / 11.1 (uncut / with the cut).
   const bool few_tiles = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128) <= 64;
   if (epi == 0 && (M <= 1536 || few_tiles)) {  // (fewer than 17 rows come here only against a very long K)
     struct Tile { int code, rows, wrows; double eff, start; };  // share of the MFMA rate in the loop; us to start

@@ -1,5 +1,5 @@
-// What the kernels that take both operands of a bfloat16 product through LDS share: waits that count the loads under way, and a
-// barrier that waits for nothing else.
+// What the kernels share that bring operands into LDS by loads of their own count: waits for the loads under way, and a barrier that
+// waits for nothing else.
 #pragma once
 #include "common.h"
 
