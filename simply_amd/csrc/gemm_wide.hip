@@ -487,16 +487,12 @@ bool gemm_wide_takes(int M, int N, int K, int64_t lda, int64_t ldc, const void* 
 double gemm_wide_tile_us(int K) { return 0.78 * K / wide::BK + 2.8; }
 
 // The time of an uncut product on tiles of `shape`, `columns` of them side by side: their rounds of slabs at what 128 outputs of 256 rows (or
-// as many of another tile) take, fitted like the broad kernel's.  One round that leaves more than half of the CUs idle is faster, the clock
-// rises: 45 to 80 tiles of 192 x 128, K = 4,608, 31 us where a full round takes 48.  (128 x 128, which take longer for their size, come out
-// even: K = 8,192, 104 tiles 58 us, 160 60.)
+// as many of another tile) take, fitted like the broad kernel's.  (128 x 128, which take longer for their size, are taken for few tiles, at
+// which the clock is higher: 0.69 to 0.98 us there.)
 static double rounds_us(int shape, int M, int64_t columns, int NW, int K, int epi) {
   const int rows = shape / 1000 % 1000, wrows = shape % 1000;
-  const int64_t tiles = (M + rows - 1) / rows * columns, rounds = (tiles + wide::kCUs - 1) / wide::kCUs;
-  double slab_us = (epi == 1 ? 0.88 : 0.78) * rows * wrows / 32768.0;
-  const double half_full = tiles / (wide::kCUs / 2.0);
-  if (epi == 0 && rows * wrows > 128 * 128 && half_full < 1.0) slab_us *= 0.6 + 0.4 * fmax(0.0, 2.0 * half_full - 1.0);
-  return fmax(5.0 + 2.0 * NW * K / 5.8e6, 3.0 + rounds * (slab_us * (K / wide::BK) + 2.8));
+  const int64_t rounds = ((M + rows - 1) / rows * columns + wide::kCUs - 1) / wide::kCUs;
+  return fmax(5.0 + 2.0 * NW * K / 5.8e6, 3.0 + rounds * ((epi == 1 ? 0.88 : 0.78) * (K / wide::BK) * rows * wrows / 32768.0 + 2.8));
 }
 
 // The tile and the cut of K for a product whose caller fixes neither, and the time that this kernel is expected to
