@@ -462,7 +462,8 @@ static int heads_per_unit(int G) {
 //   16 heads, keys of 576, values of 512: 1 request 4 tiles 15.2 / 11.7, 8 16.1 / 12.0, 33 16.7 / 13.8, 48 17.2 / 16.3, 65 17.4 / 18.6,
 //     129 22 / 28; 3 requests 33 tiles 17.2 / 15.0, 48 17.8 / 18.3; 16 requests 14 19.3 / 17.0.  3 tiles: 11.9 / 12.1.
 //   4 heads, 320 and 256: 1 request 33 tiles 13.2 / 10.5, 65 14.6 / 11.8, 95 15.0 / 14.0, 129 15.1 / 16.2; 64 and 64: 65 8.9 / 7.8.
-//   16 heads, 320 and 256 (16 rows): 8 tiles 17 / 20, 33 38 / 59, 65 63 / 13, 129 112 / 17, 255 118 / 27.
+//   16 heads, 320 and 256 (16 rows): 8 tiles 17 / 20, 33 38 / 59, 65 63 / 13, 129 112 / 17, 255 118 / 27; in 256 ranges 376 128 / 31,
+//     939 169 / 40.
 //   two maps, 8 heads of 64, values of 128: 5 tiles 10.9 / 11.9, 33 29 / 46, 95 64 / 121.
 static int maps_ranges(int unit_count, int KhV, int maps, int hd_v, int window, int max_kv_len, int max_rows) {
   const int ranges = paged_attention_decode_ranges(unit_count, KhV, window, max_kv_len, 0);
